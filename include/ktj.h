@@ -473,11 +473,12 @@ typedef struct ktj_engine ktj_engine;
  * records is finished a tenth sooner.
  *
  * ktj_destroy leaves what every engine needs before its first record (its stream and events, the
- * small page-locked buffers, 1 MiB of device memory for the inputs of small traces), the 64 MiB of
- * page-locked staging for large submissions if the engine made one, and, while they are small
- * (64 MiB together), the working memory and the document buffer of its last pass behind
+ * small page-locked buffers, 1 to 64 MiB of device memory for inputs), the 16 or 64 MiB of
+ * page-locked staging for larger submissions and documents if the engine made one, and, up to
+ * 512 MiB together, the working memory and the document buffer of its last pass behind
  * for the next ktj_create on the same device, which starts from them instead of allocating: one
- * such set per device, held until the process ends.  A trace of a few records otherwise spends
+ * such set per device, held until the process ends (working memory and document buffer only until
+ * sixteen engines in a row have needed less than an eighth of them, or an allocation fails).  A trace of a few records otherwise spends
  * more time creating and destroying these than on the GPU.  Nothing is kept of an engine that saw
  * a HIP error.
  * ---------------------------------------------------------------------------------------- */
@@ -565,6 +566,13 @@ int ktj_submit_records_device(ktj_engine* e, int rec_class, const void* device_p
  * submitted after it goes behind. */
 int ktj_submit_info(ktj_engine* e, int info_kind, const void* info);
 
+/* A whole input in one call: everything of the bundle of include/ktj_stream.h, in the order of the calls
+ * that it stands for (trace start, strings, schemas, collectives, args, API table, clock, window, device,
+ * resource and overhead infos, records, spans).  The bundle may be released when the call returns.
+ * Status of the first of those calls that failed, KTJ_OK otherwise. */
+struct ktj_stream;
+int ktj_submit_stream(ktj_engine* e, const struct ktj_stream* stream);
+
 /* Tells the engine that the first activity has arrived (see ktj_submit_info).  Every record
  * submission of an activity class does so by itself; a caller that batches its records and
  * submits them later (like the ActivityLogger shim) calls this when it receives the first one. */
@@ -598,6 +606,10 @@ int ktj_process_noalloc(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
 /* Device / host views of the finished document (valid until the next ktj_process/destroy). */
 int ktj_output_device(ktj_engine* e, const void** device_ptr, uint64_t* n_bytes);
 int ktj_output_host(ktj_engine* e, const char** host_ptr, uint64_t* n_bytes); /* pinned; D2H on first call */
+
+/* The document into memory of the caller (any host memory, `capacity` bytes), without a page-locked copy
+ * of it in the engine.  *n_bytes receives its length; KTJ_ERR_ARG if it does not fit. */
+int ktj_output_copy(ktj_engine* e, void* dst, uint64_t capacity, uint64_t* n_bytes);
 
 /* ChromeTraceLogger::finalizeTrace (output_json.cpp:1023-1028, 1066-1108): ktj_process if not
  * done, D2H, write "<path>.tmp", remove + rename. */

@@ -200,8 +200,8 @@ def load_synth():
 ENGINE_SYMBOLS = [
     "ktj_create", "ktj_destroy", "ktj_last_error", "ktj_trace_start", "ktj_intern_strings",
     "ktj_register_schema", "ktj_add_collective", "ktj_submit_args", "ktj_set_api_table", "ktj_set_clock_model",
-    "ktj_set_window", "ktj_submit_records", "ktj_submit_records_device", "ktj_host_alloc", "ktj_host_free", "ktj_submit_info", "ktj_begin_activities",
-    "ktj_process", "ktj_process_noalloc", "ktj_output_device", "ktj_output_host", "ktj_finalize", "ktj_get_stats",
+    "ktj_set_window", "ktj_submit_records", "ktj_submit_records_device", "ktj_host_alloc", "ktj_host_free", "ktj_submit_info", "ktj_submit_stream", "ktj_begin_activities",
+    "ktj_process", "ktj_process_noalloc", "ktj_output_device", "ktj_output_host", "ktj_output_copy", "ktj_finalize", "ktj_get_stats",
     "ktj_version",
     # include/ktj_rocprofiler.h
     "ktj_set_sdk_agents", "ktj_set_sdk_kernel_names", "ktj_submit_sdk_buffer", "ktj_submit_sdk_api_record", "ktj_flush",
@@ -272,6 +272,10 @@ def load_engine():
         lib.ktj_output_device.argtypes = [vp, C.POINTER(C.c_void_p), C.POINTER(C.c_uint64)]
         lib.ktj_output_host.restype = C.c_int
         lib.ktj_output_host.argtypes = [vp, C.POINTER(C.c_void_p), C.POINTER(C.c_uint64)]
+        lib.ktj_output_copy.restype = C.c_int
+        lib.ktj_output_copy.argtypes = [vp, vp, C.c_uint64, C.POINTER(C.c_uint64)]
+        lib.ktj_submit_stream.restype = C.c_int
+        lib.ktj_submit_stream.argtypes = [vp, C.POINTER(Stream)]
         lib.ktj_finalize.restype = C.c_int
         lib.ktj_finalize.argtypes = [vp, C.c_int64, C.POINTER(C.c_uint64)]
         lib.ktj_get_stats.restype = C.c_int

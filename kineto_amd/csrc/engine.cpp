@@ -35,8 +35,8 @@ using namespace ktj::gpu;
 
 namespace {
 
-#define KTJ_INPUT_ARENA_BYTES (1u << 20)   /* device memory for the inputs of small traces */
-#define KTJ_INPUT_PIECE_MAX (128u << 10)   /* largest array that takes a piece of it */
+#define KTJ_INPUT_ARENA_BYTES (1ull << 20)     /* device memory for the inputs of an engine, to begin with */
+#define KTJ_INPUT_ARENA_MAX (64ull << 20)      /* what it may grow to for the engines that follow */
 #define KTJ_STAGE_SMALL_BYTES (256u << 10) /* pinned ring that small submissions pass through */
 #define KTJ_STAGE_SMALL_MAX (64u << 10)    /* largest submission that does */
 /* large submissions: pinned chunks, two per copying thread.  Measured for 1.9 GB of records from
@@ -46,8 +46,22 @@ namespace {
 #define KTJ_STAGE_CHUNK (8ull << 20)
 #define KTJ_STAGE_BIG_MIN (16ull << 20)    /* smallest submission that is spread over threads */
 #define KTJ_STAGE_THREADS_MAX 4
-#define KTJ_KIT_DEVICE_BYTES_MAX (64ull << 20) /* working and document memory that waits for the next engine */
-#define KTJ_KIT_PINNED_BYTES_MAX (1ull << 20)  /* same, per pinned buffer sized by a document */
+#define KTJ_STAGE_SLOTS (2 * KTJ_STAGE_THREADS_MAX)
+/* Submissions between the ring and KTJ_STAGE_BIG_MIN, and documents on their way to the host, pass
+ * through eight pinned slots of this size (the first part of the memory that large submissions use
+ * whole): the copy engine works on some while the host fills or empties the others. */
+#define KTJ_STAGE_SLOT (2ull << 20)
+#define KTJ_STAGE_PART (1ull << 20)        /* an upload through them is handed to the copy engine in parts of this size */
+/* Working and document memory that waits for the next engine, per device: a thousandth of the card's
+ * memory, enough for traces of a few hundred thousand records, which otherwise spend more time in
+ * hipMalloc and hipFree than on the GPU.  What KTJ_KIT_LEAN engines in a row could have done with an
+ * eighth of is given back (above KTJ_KIT_SMALL_BYTES), and all of it when an allocation fails. */
+#define KTJ_KIT_DEVICE_BYTES_MAX (512ull << 20)
+#define KTJ_KIT_SMALL_BYTES (64ull << 20)
+#define KTJ_KIT_LEAN 16u
+#define KTJ_KIT_PINNED_BYTES_MAX (1ull << 20)  /* same, for the pinned copy of a document (ktj_output_host) */
+
+bool drop_waiting_memory(); /* gives back what the current device's kit holds; true if that was anything */
 
 /* One working buffer in device memory.  `p` is what the kernels use: either the buffer's own
  * allocation (freed with the engine; the engine's device is current then) or, for the entry point
@@ -72,28 +86,35 @@ struct DevBuf {
     if (own) { hipError_t e = hipFree(own); p = own = nullptr; cap = own_cap = 0; if (e != hipSuccess) return e; }
     size_t want = bytes + (with_slack ? bytes / 8 : 0) + 256;
     hipError_t e = hipMalloc(&own, want);
+    if (e == hipErrorOutOfMemory && drop_waiting_memory()) { (void)hipGetLastError(); e = hipMalloc(&own, want); }
     if (e != hipSuccess) { p = own = nullptr; return e; }
     p = own;
     cap = own_cap = want;
     return hipSuccess;
   }
   void borrow(void* ptr, size_t bytes) { p = ptr; cap = bytes; }
+  void unborrow() { p = own; cap = own_cap; }
   void release() { if (own) (void)hipFree(own); p = own = nullptr; cap = own_cap = 0; }
   template <typename T> T* as() const { return reinterpret_cast<T*>(p); }
 };
 
-/* Device memory for the inputs of a small trace: one allocation that the engine's small arrays are
- * carved out of (a trace of a few records otherwise spends more time in hipMalloc than on the GPU).
- * Pieces are never given back; a new engine that inherits the arena starts at its beginning. */
+/* Device memory for an engine's inputs: one allocation that its arrays are carved out of (a trace of
+ * a few records otherwise spends more time in hipMalloc than on the GPU, a session of a few
+ * megabytes as much as on its copies).  Pieces are never given back; a new engine that inherits the
+ * arena starts at its beginning, and finds it large enough for what its predecessor asked for. */
 struct InputArena {
   DevBuf mem;
-  size_t used = 0;
+  size_t used = 0, missed = 0; /* missed: what it had no room for */
   void* take(size_t bytes) {
     const size_t off = (used + 255) & ~(size_t)255;
-    if (bytes > KTJ_INPUT_PIECE_MAX || !mem.p || off > mem.cap || bytes > mem.cap - off) return nullptr;
+    if (!mem.p || off > mem.cap || bytes > mem.cap - off) {
+      if (bytes <= KTJ_INPUT_ARENA_MAX) missed += bytes + 256;
+      return nullptr;
+    }
     used = off + bytes;
     return static_cast<char*>(mem.p) + off;
   }
+  size_t wanted() const { const size_t w = used + missed; return missed && w <= KTJ_INPUT_ARENA_MAX && w > mem.cap ? w : 0; }
 };
 
 /* append-only device array fed from host memory */
@@ -111,9 +132,11 @@ struct DevVec {
       if (piece) nb.borrow(piece, want);
       else e = nb.ensure(want);
       if (e != hipSuccess) return e;
-      if (bytes) { e = hipMemcpyAsync(nb.p, buf.p, bytes, hipMemcpyDeviceToDevice, st); if (e != hipSuccess) return e; }
-      e = hipStreamSynchronize(st);
-      if (e != hipSuccess) return e;
+      if (bytes) {
+        e = hipMemcpyAsync(nb.p, buf.p, bytes, hipMemcpyDeviceToDevice, st);
+        if (e == hipSuccess) e = hipStreamSynchronize(st);
+        if (e != hipSuccess) return e;
+      }
       buf = std::move(nb);
     }
     return hipSuccess;
@@ -211,9 +234,6 @@ struct ktj_engine {
   size_t pool_used = 0, pool_need = 0;
   bool measuring = false;
   char* pinned_out = nullptr; size_t pinned_out_cap = 0;
-  char* file_stage[2] = {nullptr, nullptr};   /* pinned staging of the file sink, at most KTJ_FILE_STAGE_BYTES each */
-  size_t file_stage_cap[2] = {0, 0};
-  hipEvent_t ev_file_stage[2] = {};
   bool host_copy_valid = false;
   /* submissions from ordinary host memory: small ones pass through a pinned ring and are not waited
    * for (the stream orders them before the pass), large ones through pinned chunks that several
@@ -221,8 +241,11 @@ struct ktj_engine {
   InputArena input_arena;
   char* stage_small = nullptr; char* stage_small_dev = nullptr; size_t stage_small_used = 0;
   PieceJobs pieces{}; /* small submissions in the ring that no kernel has moved yet */
-  char* stage_big = nullptr; size_t stage_big_chunks = 0;
-  hipEvent_t ev_stage_big[2 * KTJ_STAGE_THREADS_MAX] = {};
+  char* stage_big = nullptr; size_t stage_big_bytes = 0;
+  size_t stage_big_used = 0; /* of the slots' memory: uploads that the stream may not have passed yet */
+  hipEvent_t ev_stage_big[KTJ_STAGE_SLOTS] = {};
+  size_t most_needed = 0;    /* the largest pass's working memory and document */
+  uint32_t kit_lean = 0; /* engines in a row, this kit's, that needed little of what it holds */
   bool hip_failed = false; /* a HIP call failed at some point: nothing of this engine is handed on */
 
   /* results */
@@ -308,26 +331,6 @@ int need(ktj_engine* e, DevBuf& b, size_t bytes) {
     if (_rc != KTJ_OK) return _rc;                        \
   } while (0)
 
-/* A small host table to the device.  A pass that may not allocate stages it through the pinned
- * buffer of the engine (allocated with the engine) instead of the runtime's own staging. */
-int upload_small(ktj_engine* e, DevBuf& dst, const void* src, size_t bytes) {
-  /* these tables outlive the pass (they are uploaded only when they change), so outside a pass that
-   * may not allocate they keep allocations of their own rather than a piece of the pass's pool */
-  if (e->noalloc) NEED(dst, bytes ? bytes : 16);
-  else HIPCHK(dst.ensure(bytes ? bytes : 16));
-  if (bytes && e->noalloc) {
-    if (bytes > e->pinned_small_cap) {
-      e->last_error = "ktj_process_noalloc: a table of " + std::to_string(bytes) + " bytes exceeds the pinned staging buffer";
-      return KTJ_ERR_LIMIT;
-    }
-    memcpy(e->pinned_small, src, bytes);
-    src = e->pinned_small;
-  }
-  if (bytes) HIPCHK(hipMemcpyAsync(dst.p, src, bytes, hipMemcpyHostToDevice, e->stream));
-  HIPCHK(hipStreamSynchronize(e->stream));
-  return KTJ_OK;
-}
-
 /* The small submissions gathered in the pinned ring go to their places on the device: one launch for
  * all of them, ordered on the engine's stream like everything else.  Before a pass, before an array
  * they belong to moves, and when the ring or the list is full. */
@@ -347,15 +350,82 @@ bool is_pinned_host(const void* p) {
   return a.type == hipMemoryTypeHost;
 }
 
+/* n bytes into the pinned ring of small submissions, to be moved to dst by the next put_pending_pieces;
+ * n <= KTJ_STAGE_SMALL_MAX */
+int stage_piece(ktj_engine* e, void* dst, const void* src, size_t n) {
+  /* the piece sits in the ring where its place on the device does, modulo 16 */
+  size_t off = ((e->stage_small_used + 63) & ~(size_t)63) + ((uintptr_t)dst & 15u);
+  if (off + n > KTJ_STAGE_SMALL_BYTES || e->pieces.count == KTJ_MAX_PIECES) {
+    const int rc = put_pending_pieces(e);
+    if (rc != KTJ_OK) return rc;
+  }
+  if (off + n > KTJ_STAGE_SMALL_BYTES) { /* the ring is full: what is in it has to be on the device first */
+    HIPCHK(hipStreamSynchronize(e->stream));
+    off = (uintptr_t)dst & 15u;
+  }
+  memcpy(e->stage_small + off, src, n);
+  const uint32_t k = e->pieces.count++;
+  e->pieces.src[k] = e->stage_small_dev + off;
+  e->pieces.dst[k] = static_cast<char*>(dst);
+  e->pieces.n[k] = n;
+  e->stage_small_used = off + n;
+  return KTJ_OK;
+}
+
+/* The pinned slots: KTJ_STAGE_SLOTS of `slot_bytes` each (kept with the kit). */
+int ensure_stage(ktj_engine* e, size_t slot_bytes) {
+  const size_t bytes = KTJ_STAGE_SLOTS * slot_bytes;
+  if (e->stage_big_bytes < bytes) {
+    if (e->stage_big) { HIPCHK(hipStreamSynchronize(e->stream)); HIPCHK(hipHostFree(e->stage_big)); }
+    e->stage_big = nullptr; e->stage_big_bytes = 0; e->stage_big_used = 0;
+    void* p = nullptr;
+    HIPCHK(hipHostMalloc(&p, bytes, hipHostMallocDefault));
+    e->stage_big = static_cast<char*>(p);
+    e->stage_big_bytes = bytes;
+  }
+  for (auto& ev : e->ev_stage_big)
+    if (!ev) HIPCHK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+  return KTJ_OK;
+}
+
+/* uploads out of the slots are on their way: everything else that uses the slots waits for them */
+int drain_stage(ktj_engine* e) {
+  if (e->stage_big_used) { HIPCHK(hipStreamSynchronize(e->stream)); e->stage_big_used = 0; }
+  return KTJ_OK;
+}
+
+/* Runs worker(0 .. n_threads - 1), worker 0 on the calling thread; a thread that cannot be started
+ * has its share done by the caller. */
+template <typename Worker> void run_workers(unsigned n_threads, Worker worker) {
+  std::vector<std::thread> pool;
+  unsigned started = 1;
+  try {
+    pool.reserve(n_threads);
+    for (; started < n_threads; ++started) pool.emplace_back(worker, started);
+  } catch (...) {}
+  worker(0);
+  for (unsigned t = started; t < n_threads; ++t) worker(t);
+  for (auto& th : pool) th.join();
+}
+unsigned copy_threads(size_t bytes, size_t per_thread) {
+  unsigned n = std::thread::hardware_concurrency() / 2;
+  if (n > KTJ_STAGE_THREADS_MAX) n = KTJ_STAGE_THREADS_MAX;
+  if (n > bytes / per_thread) n = (unsigned)(bytes / per_thread);
+  return n ? n : 1;
+}
+
 /* n bytes of host memory behind a device array.  The caller may free or reuse src when this
  * returns; the copy itself is only ordered on the engine's stream, in front of the next pass.
  *   - up to KTJ_STAGE_SMALL_MAX bytes: into the pinned ring, from where one kernel launch takes all
  *     such pieces to their places (put_pending_pieces; a trace of a few records pays a dozen copies
  *     and stream synchronisations otherwise);
- *   - from KTJ_STAGE_BIG_MIN bytes of ordinary memory: threads copy chunks into pinned buffers, two
- *     per thread, and hand each to the copy engine as soon as it is full (one thread's copy through
- *     the runtime's own staging reaches about half of what the link carries);
- *   - everything else, and page-locked sources: one copy, waited for. */
+ *   - below KTJ_STAGE_BIG_MIN bytes of ordinary memory: part by part into the pinned slots and on to
+ *     the copy engine, not waited for (a copy from ordinary memory is waited for by the runtime, with
+ *     nothing overlapped: a session of 30 000 records, 2.8 MB in five arrays, submits in 262 us that way);
+ *   - above: threads copy chunks into pinned buffers, two per thread, and hand each to the copy
+ *     engine as soon as it is full (one thread's copy through the runtime's own staging reaches about
+ *     half of what the link carries);
+ *   - page-locked sources: one copy, waited for. */
 int append_from_host(ktj_engine* e, DevVec& v, const void* src, size_t n) {
   if (n == 0) return KTJ_OK;
   hipStream_t st = e->stream;
@@ -366,42 +436,26 @@ int append_from_host(ktj_engine* e, DevVec& v, const void* src, size_t n) {
   HIPCHK(v.reserve(n, st, &e->input_arena));
   char* dst = v.end();
   if (n <= KTJ_STAGE_SMALL_MAX && e->stage_small) {
-    /* the piece sits in the ring where its place on the device does, modulo 16 */
-    size_t off = ((e->stage_small_used + 63) & ~(size_t)63) + ((uintptr_t)dst & 15u);
-    if (off + n > KTJ_STAGE_SMALL_BYTES || e->pieces.count == KTJ_MAX_PIECES) {
-      const int rc = put_pending_pieces(e);
-      if (rc != KTJ_OK) return rc;
-    }
-    if (off + n > KTJ_STAGE_SMALL_BYTES) { /* the ring is full: what is in it has to be on the device first */
-      HIPCHK(hipStreamSynchronize(st));
-      off = (uintptr_t)dst & 15u;
-    }
-    memcpy(e->stage_small + off, src, n);
-    const uint32_t k = e->pieces.count++;
-    e->pieces.src[k] = e->stage_small_dev + off;
-    e->pieces.dst[k] = dst;
-    e->pieces.n[k] = n;
-    e->stage_small_used = off + n;
+    const int rc = stage_piece(e, dst, src, n);
+    if (rc != KTJ_OK) return rc;
     v.bytes += n;
     return KTJ_OK;
   }
-  unsigned n_threads = std::thread::hardware_concurrency() / 2;
-  if (n_threads > KTJ_STAGE_THREADS_MAX) n_threads = KTJ_STAGE_THREADS_MAX;
-  if (n >= KTJ_STAGE_BIG_MIN && n_threads >= 2 && !is_pinned_host(src)) {
-    const size_t slots = 2 * (size_t)n_threads;
-    if (e->stage_big_chunks < slots) {
-      if (e->stage_big) HIPCHK(hipHostFree(e->stage_big));
-      e->stage_big = nullptr; e->stage_big_chunks = 0;
-      void* p = nullptr;
-      HIPCHK(hipHostMalloc(&p, slots * KTJ_STAGE_CHUNK, hipHostMallocDefault));
-      e->stage_big = static_cast<char*>(p);
-      e->stage_big_chunks = slots;
-    }
-    for (size_t k = 0; k < slots; ++k)
-      if (!e->ev_stage_big[k]) HIPCHK(hipEventCreateWithFlags(&e->ev_stage_big[k], hipEventDisableTiming));
+  if (is_pinned_host(src)) {
+    HIPCHK(hipMemcpyAsync(dst, src, n, hipMemcpyHostToDevice, st));
+    HIPCHK(hipStreamSynchronize(st)); /* the caller may free src when we return */
+    v.bytes += n;
+    return KTJ_OK;
+  }
+  const unsigned n_threads = copy_threads(n, KTJ_STAGE_CHUNK);
+  if (n >= KTJ_STAGE_BIG_MIN && n_threads >= 2) {
+    int rc = drain_stage(e);
+    if (rc == KTJ_OK) rc = ensure_stage(e, KTJ_STAGE_CHUNK);
+    if (rc != KTJ_OK) return rc;
     const size_t n_chunks = (n + KTJ_STAGE_CHUNK - 1) / KTJ_STAGE_CHUNK;
     hipError_t err[KTJ_STAGE_THREADS_MAX];
-    auto worker = [&](unsigned t) {
+    for (auto& x : err) x = hipSuccess;
+    run_workers(n_threads, [&](unsigned t) {
       err[t] = hipSetDevice(e->device);
       /* thread t takes chunks t, t + T, ...; its two pinned slots alternate */
       for (size_t c = t, turn = 0; c < n_chunks && err[t] == hipSuccess; c += n_threads, ++turn) {
@@ -413,17 +467,7 @@ int append_from_host(ktj_engine* e, DevVec& v, const void* src, size_t n) {
         err[t] = hipMemcpyAsync(dst + off, stage, len, hipMemcpyHostToDevice, st);
         if (err[t] == hipSuccess) err[t] = hipEventRecord(e->ev_stage_big[slot], st);
       }
-    };
-    for (auto& x : err) x = hipSuccess;
-    std::vector<std::thread> pool;
-    unsigned started = 1; /* thread 0 is this one; a thread that cannot be started has its chunks copied here */
-    try {
-      pool.reserve(n_threads);
-      for (; started < n_threads; ++started) pool.emplace_back(worker, started);
-    } catch (...) {}
-    worker(0);
-    for (unsigned t = started; t < n_threads; ++t) worker(t);
-    for (auto& th : pool) th.join();
+    });
     /* the slots are free for the next call once the stream has passed them */
     const hipError_t done = hipStreamSynchronize(st);
     for (unsigned t = 0; t < n_threads; ++t) HIPCHK(err[t]);
@@ -431,9 +475,47 @@ int append_from_host(ktj_engine* e, DevVec& v, const void* src, size_t n) {
     v.bytes += n;
     return KTJ_OK;
   }
-  HIPCHK(hipMemcpyAsync(dst, src, n, hipMemcpyHostToDevice, st));
-  HIPCHK(hipStreamSynchronize(st)); /* the caller may free src when we return */
+  {
+    const int rc = ensure_stage(e, KTJ_STAGE_SLOT);
+    if (rc != KTJ_OK) return rc;
+  }
+  for (size_t done = 0; done < n;) {
+    if (e->stage_big_used == e->stage_big_bytes) { /* all slots are full: wait until the stream has passed them */
+      const int rc = drain_stage(e);
+      if (rc != KTJ_OK) return rc;
+    }
+    const size_t len = std::min(std::min<size_t>(n - done, KTJ_STAGE_PART), e->stage_big_bytes - e->stage_big_used);
+    char* stage = e->stage_big + e->stage_big_used;
+    memcpy(stage, static_cast<const char*>(src) + done, len);
+    HIPCHK(hipMemcpyAsync(dst + done, stage, len, hipMemcpyHostToDevice, st));
+    e->stage_big_used = std::min((e->stage_big_used + len + 255) & ~(size_t)255, e->stage_big_bytes);
+    done += len;
+  }
   v.bytes += n;
+  return KTJ_OK;
+}
+
+/* A small host table to the device, in front of the pass that is about to start. */
+int upload_small(ktj_engine* e, DevBuf& dst, const void* src, size_t bytes) {
+  const size_t room = bytes ? bytes : 16;
+  if (e->noalloc) {
+    NEED(dst, room);
+    if (bytes > e->pinned_small_cap) {
+      e->last_error = "ktj_process_noalloc: a table of " + std::to_string(bytes) + " bytes exceeds the pinned staging buffer";
+      return KTJ_ERR_LIMIT;
+    }
+  } else if (!dst.p || dst.cap < room) {
+    /* these tables outlive the pass (they are uploaded only when they change), so they are pieces of
+     * the engine's input memory and not of the pass's pool */
+    void* piece = e->input_arena.take(room + room / 2);
+    if (piece) dst.borrow(piece, room + room / 2);
+    else HIPCHK(dst.ensure(room));
+  }
+  if (bytes == 0) return KTJ_OK;
+  if (bytes <= KTJ_STAGE_SMALL_MAX) return stage_piece(e, dst.p, src, bytes);
+  if (e->noalloc) { memcpy(e->pinned_small, src, bytes); src = e->pinned_small; } /* not the runtime's own staging */
+  HIPCHK(hipMemcpyAsync(dst.p, src, bytes, hipMemcpyHostToDevice, e->stream));
+  HIPCHK(hipStreamSynchronize(e->stream));
   return KTJ_OK;
 }
 
@@ -553,18 +635,30 @@ struct Kit {
   hipStream_t stream = nullptr;
   hipEvent_t ev[EV_COUNT] = {};
   hipEvent_t ev_d2h[2] = {};
-  hipEvent_t ev_file_stage[2] = {};
-  hipEvent_t ev_stage_big[2 * KTJ_STAGE_THREADS_MAX] = {};
+  hipEvent_t ev_stage_big[KTJ_STAGE_SLOTS] = {};
+  uint32_t lean = 0;
   void* pinned_small = nullptr; size_t pinned_small_cap = 0; char* pinned_small_dev = nullptr;
   HostCtl* h_ctl = nullptr; HostCtl* h_ctl_dev = nullptr;
   char* pinned_out = nullptr; size_t pinned_out_cap = 0;
-  char* file_stage[2] = {nullptr, nullptr}; size_t file_stage_cap[2] = {0, 0};
   char* stage_small = nullptr; char* stage_small_dev = nullptr;
-  char* stage_big = nullptr; size_t stage_big_chunks = 0;
+  char* stage_big = nullptr; size_t stage_big_bytes = 0;
   DevBuf d_scalars, pool, out, arena_mem;
 };
 std::mutex g_kit_mutex;
 std::map<int, Kit*>& kits() { static auto* m = new std::map<int, Kit*>(); return *m; } /* never destroyed: the runtime may be gone by then */
+
+bool drop_waiting_memory() {
+  int device = 0;
+  if (hipGetDevice(&device) != hipSuccess) return false;
+  std::lock_guard<std::mutex> lock(g_kit_mutex);
+  auto it = kits().find(device);
+  if (it == kits().end() || !it->second->full) return false;
+  Kit& k = *it->second;
+  const bool any = k.pool.own_cap + k.out.own_cap != 0;
+  k.pool.release();
+  k.out.release();
+  return any;
+}
 
 /* the engine's device is current */
 bool take_kit(ktj_engine* e) {
@@ -574,14 +668,13 @@ bool take_kit(ktj_engine* e) {
   Kit& k = *it->second;
   e->stream = k.stream;
   memcpy(e->ev, k.ev, sizeof k.ev); memcpy(e->ev_d2h, k.ev_d2h, sizeof k.ev_d2h);
-  memcpy(e->ev_file_stage, k.ev_file_stage, sizeof k.ev_file_stage);
   memcpy(e->ev_stage_big, k.ev_stage_big, sizeof k.ev_stage_big);
+  e->kit_lean = k.lean;
   e->pinned_small = k.pinned_small; e->pinned_small_cap = k.pinned_small_cap; e->pinned_small_dev = k.pinned_small_dev;
   e->h_ctl = k.h_ctl; e->h_ctl_dev = k.h_ctl_dev;
   e->pinned_out = k.pinned_out; e->pinned_out_cap = k.pinned_out_cap;
-  for (int i = 0; i < 2; ++i) { e->file_stage[i] = k.file_stage[i]; e->file_stage_cap[i] = k.file_stage_cap[i]; }
   e->stage_small = k.stage_small; e->stage_small_dev = k.stage_small_dev;
-  e->stage_big = k.stage_big; e->stage_big_chunks = k.stage_big_chunks;
+  e->stage_big = k.stage_big; e->stage_big_bytes = k.stage_big_bytes;
   e->d_scalars = std::move(k.d_scalars); e->pool = std::move(k.pool); e->out = std::move(k.out);
   e->input_arena.mem = std::move(k.arena_mem);
   k = Kit();
@@ -594,6 +687,17 @@ void give_kit(ktj_engine* e) {
   if (e->pinned_small_cap > KTJ_KIT_PINNED_BYTES_MAX) return; /* grown for an unusually long header: not worth holding */
   for (auto& ev : e->ev) if (!ev) return;
   for (auto& ev : e->ev_d2h) if (!ev) return;
+  /* back from whatever they were lent (the pool never is; the document may sit in a caller's buffer) */
+  e->pool.unborrow();
+  e->out.unborrow();
+  const size_t held = e->pool.own_cap + e->out.own_cap;
+  if (held > KTJ_KIT_SMALL_BYTES && (e->most_needed < held / 8)) {
+    if (++e->kit_lean >= KTJ_KIT_LEAN) { e->pool.release(); e->out.release(); e->kit_lean = 0; }
+  } else e->kit_lean = 0;
+  if (const size_t want = e->input_arena.wanted()) { /* room for the inputs of another engine like this one */
+    e->input_arena.mem.release();
+    if (e->input_arena.mem.ensure(want + want / 4, false) != hipSuccess) (void)hipGetLastError();
+  }
   std::lock_guard<std::mutex> lock(g_kit_mutex);
   Kit* slot = nullptr;
   try {
@@ -606,21 +710,16 @@ void give_kit(ktj_engine* e) {
   k.stream = e->stream; e->stream = nullptr;
   memcpy(k.ev, e->ev, sizeof k.ev); memset(e->ev, 0, sizeof e->ev);
   memcpy(k.ev_d2h, e->ev_d2h, sizeof k.ev_d2h); memset(e->ev_d2h, 0, sizeof e->ev_d2h);
-  memcpy(k.ev_file_stage, e->ev_file_stage, sizeof k.ev_file_stage); memset(e->ev_file_stage, 0, sizeof e->ev_file_stage);
+  k.lean = e->kit_lean;
   memcpy(k.ev_stage_big, e->ev_stage_big, sizeof k.ev_stage_big); memset(e->ev_stage_big, 0, sizeof e->ev_stage_big);
   k.pinned_small = e->pinned_small; k.pinned_small_cap = e->pinned_small_cap; k.pinned_small_dev = e->pinned_small_dev;
   e->pinned_small = nullptr;
   k.h_ctl = e->h_ctl; k.h_ctl_dev = e->h_ctl_dev; e->h_ctl = nullptr;
   if (e->pinned_out_cap <= KTJ_KIT_PINNED_BYTES_MAX) { k.pinned_out = e->pinned_out; k.pinned_out_cap = e->pinned_out_cap; e->pinned_out = nullptr; }
-  for (int i = 0; i < 2; ++i)
-    if (e->file_stage_cap[i] <= KTJ_KIT_PINNED_BYTES_MAX) { k.file_stage[i] = e->file_stage[i]; k.file_stage_cap[i] = e->file_stage_cap[i]; e->file_stage[i] = nullptr; }
   k.stage_small = e->stage_small; k.stage_small_dev = e->stage_small_dev; e->stage_small = nullptr;
-  k.stage_big = e->stage_big; k.stage_big_chunks = e->stage_big_chunks; e->stage_big = nullptr;
+  k.stage_big = e->stage_big; k.stage_big_bytes = e->stage_big_bytes; e->stage_big = nullptr;
   k.d_scalars = std::move(e->d_scalars);
   if (e->pool.own_cap + e->out.own_cap <= KTJ_KIT_DEVICE_BYTES_MAX) {
-    /* back from whatever they were lent (the pool never is; the document may sit in a caller's buffer) */
-    e->pool.p = e->pool.own; e->pool.cap = e->pool.own_cap;
-    e->out.p = e->out.own; e->out.cap = e->out.own_cap;
     k.pool = std::move(e->pool);
     k.out = std::move(e->out);
   }
@@ -696,8 +795,6 @@ void ktj_destroy(ktj_engine* e) {
   if (e->pinned_out) (void)hipHostFree(e->pinned_out);
   if (e->stage_small) (void)hipHostFree(e->stage_small);
   if (e->stage_big) (void)hipHostFree(e->stage_big);
-  for (auto& p : e->file_stage) if (p) (void)hipHostFree(p);
-  for (auto& ev : e->ev_file_stage) if (ev) (void)hipEventDestroy(ev);
   for (auto& ev : e->ev_stage_big) if (ev) (void)hipEventDestroy(ev);
   for (auto& ev : e->ev) if (ev) (void)hipEventDestroy(ev);
   for (auto& ev : e->ev_d2h) if (ev) (void)hipEventDestroy(ev);
@@ -1020,6 +1117,34 @@ int ktj_submit_info(ktj_engine* e, int info_kind, const void* info) {
   return KTJ_OK;
 }
 
+/* A complete stream in one call (include/ktj_stream.h), in the call order of the buffering logger's
+ * replay (libkineto/src/output_membuf.h:91-107): device and resource infos, the activities, the spans. */
+int ktj_submit_stream(ktj_engine* e, const ktj_stream* s) {
+  if (!e || !s) return KTJ_ERR_ARG;
+  int rc = ktj_trace_start(e, s->meta_kv, s->n_meta, s->device_properties);
+  uint32_t id;
+  uint64_t slot;
+  if (rc == KTJ_OK) rc = ktj_intern_strings(e, s->str_blob, s->str_off, s->n_strings, &id);
+  for (uint64_t i = 0; i < s->n_schemas && rc == KTJ_OK; ++i)
+    rc = ktj_register_schema(e, s->fields + s->schemas[i].first_field, s->schemas[i].n_fields, &id);
+  for (uint64_t i = 0; i < s->n_collectives && rc == KTJ_OK; ++i) rc = ktj_add_collective(e, &s->collectives[i], nullptr);
+  if (rc == KTJ_OK) rc = ktj_submit_args(e, s->args, s->n_args, &slot);
+  if (rc == KTJ_OK) rc = ktj_set_api_table(e, s->cid_name_ids, s->n_cids, s->flow_start_cids, s->n_flow_start, s->malloc_cid);
+  if (rc == KTJ_OK) rc = ktj_set_clock_model(e, &s->clock);
+  if (rc == KTJ_OK) rc = ktj_set_window(e, s->window_start_ns, s->window_end_ns);
+  for (uint64_t i = 0; i < s->n_device_infos && rc == KTJ_OK; ++i) rc = ktj_submit_info(e, KTJ_INFO_DEVICE, &s->device_infos[i]);
+  for (uint64_t i = 0; i < s->n_resource_infos && rc == KTJ_OK; ++i) rc = ktj_submit_info(e, KTJ_INFO_RESOURCE, &s->resource_infos[i]);
+  for (uint64_t i = 0; i < s->n_overhead_infos && rc == KTJ_OK; ++i) rc = ktj_submit_info(e, KTJ_INFO_OVERHEAD, &s->overhead_infos[i]);
+  if (rc == KTJ_OK) rc = ktj_begin_activities(e);
+  if (rc == KTJ_OK) rc = ktj_submit_records(e, KTJ_REC_GENERIC, s->generic, s->n_generic);
+  if (rc == KTJ_OK) rc = ktj_submit_records(e, KTJ_REC_RUNTIME, s->runtime, s->n_runtime);
+  if (rc == KTJ_OK) rc = ktj_submit_records(e, KTJ_REC_DEVICE, s->device, s->n_device);
+  if (rc == KTJ_OK) rc = ktj_submit_records(e, KTJ_REC_EXTCORR, s->extcorr, s->n_extcorr);
+  if (rc == KTJ_OK) rc = ktj_submit_records(e, KTJ_REC_USERCORR, s->usercorr, s->n_usercorr);
+  for (uint64_t i = 0; i < s->n_spans && rc == KTJ_OK; ++i) rc = ktj_submit_info(e, KTJ_INFO_SPAN, &s->spans[i]);
+  return rc;
+}
+
 /* One pass of the whole path.  out_device == nullptr: the document goes into the engine's own
  * buffer and working memory is allocated as needed (ktj_process).  Otherwise (ktj_process_noalloc,
  * e->noalloc set by the caller): the document goes into the caller's buffer of out_cap bytes and
@@ -1027,7 +1152,6 @@ int ktj_submit_info(ktj_engine* e, int info_kind, const void* info) {
 static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, uint64_t out_cap) {
   HIPCHK(hipSetDevice(e->device));
   hipStream_t st = e->stream;
-  { const int rc = put_pending_pieces(e); if (rc != KTJ_OK) return rc; }
   e->arena_used = 0;
   e->processed = false;
   e->total_bytes = 0;
@@ -1058,6 +1182,20 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
     e->api_dirty = false;
   }
 
+  /* collective metadata is looked at only if both entries and a schema that refers to them exist */
+  const uint32_t n_coll = e->coll_schemas ? (uint32_t)e->collectives.size() : 0u;
+  if (n_coll && e->coll_dirty) {
+    std::string blob;
+    std::vector<uint64_t> off(e->collectives.size() + 1, 0);
+    for (size_t k = 0; k < e->collectives.size(); ++k) { blob += e->collectives[k].args; off[k + 1] = blob.size(); }
+    blob.append(16, '\0'); /* string copies load whole aligned words */
+    int rc = upload_small(e, e->d_coll_blob, blob.data(), blob.size());
+    if (rc == KTJ_OK) rc = upload_small(e, e->d_coll_off, off.data(), off.size() * 8);
+    if (rc != KTJ_OK) return rc;
+    e->coll_dirty = false;
+  }
+  { const int rc = put_pending_pieces(e); if (rc != KTJ_OK) return rc; }
+
   /* working memory */
   const uint32_t ns = (uint32_t)e->n_strings;
   if (nx >= 0x7FFFFFFFull || nr >= 0x7FFFFFFFull) { e->last_error = "more than 2^31 - 2 records of one class"; return KTJ_ERR_LIMIT; }
@@ -1065,6 +1203,7 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
   const uint32_t cap_full = pow2_at_least((nr + nd) + (nr + nd) / 2);
   const uint32_t cap_narrow = pow2_at_least((nx + nr) + (nx + nr) / 2), cap_cpu = pow2_at_least(2 * ng);
   e->pool_used = 0;
+  size_t pass_bytes = 0;
   for (int phase = e->noalloc ? 1 : 0; phase < 2; ++phase) { /* 0: add the sizes up and size the pool; 1: hand the buffers out */
   e->measuring = phase == 0;
   e->pool_need = 0;
@@ -1108,6 +1247,7 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
   if (e->measuring) {
     e->measuring = false;
     if (e->pool.cap < e->pool_need + 4096) HIPCHK(e->pool.ensure(e->pool_need + 4096));
+    pass_bytes = e->pool_need;
   }
   }
 
@@ -1138,18 +1278,6 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
   ctx.args = e->args.buf.as<uint64_t>(); ctx.n_args = e->n_args;
   ctx.base_time_ns = e->base_time_ns;
   ctx.create_flags = e->flags;
-  /* collective metadata is looked at only if both entries and a schema that refers to them exist */
-  const uint32_t n_coll = e->coll_schemas ? (uint32_t)e->collectives.size() : 0u;
-  if (n_coll && e->coll_dirty) {
-    std::string blob;
-    std::vector<uint64_t> off(e->collectives.size() + 1, 0);
-    for (size_t k = 0; k < e->collectives.size(); ++k) { blob += e->collectives[k].args; off[k + 1] = blob.size(); }
-    blob.append(16, '\0'); /* string copies load whole aligned words */
-    int rc = upload_small(e, e->d_coll_blob, blob.data(), blob.size());
-    if (rc == KTJ_OK) rc = upload_small(e, e->d_coll_off, off.data(), off.size() * 8);
-    if (rc != KTJ_OK) return rc;
-    e->coll_dirty = false;
-  }
   ctx.coll_blob = e->d_coll_blob.as<char>(); ctx.coll_off = e->d_coll_off.as<uint64_t>(); ctx.n_coll = n_coll;
   uint32_t* cpu_row = nullptr; /* last CPU op per id: only where something is read from that op */
   if (n_coll || max_spans) {
@@ -1395,6 +1523,9 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
   }
   HIPCHK(hipEventRecord(e->ev[EV_EMIT], st));
   HIPCHK(hipStreamSynchronize(st));
+  e->stage_small_used = 0; /* the stream has passed every upload: ring and slots are free from their beginning */
+  e->stage_big_used = 0;
+  if (!out_device) e->most_needed = std::max(e->most_needed, pass_bytes + (size_t)e->total_bytes);
 
   /* ---- statistics ---- */
   ktj_stats& s = e->stats;
@@ -1476,6 +1607,7 @@ int ktj_process_noalloc(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
   /* The small tables of this pass sit in the scratch array, which every engine on this GPU shares:
    * whatever the pass returned, the next allocating pass must upload them into its own buffers again. */
   e->schemas_dirty = e->api_dirty = e->coll_dirty = true;
+  for (DevBuf* b : {&e->d_fields, &e->d_schemas, &e->d_cid_names, &e->d_flow_bits, &e->d_coll_blob, &e->d_coll_off}) b->unborrow();
   if (n_bytes) *n_bytes = e->total_bytes; /* on KTJ_ERR_LIMIT for a short output buffer: the size that is needed */
   return rc;
 }
@@ -1516,44 +1648,104 @@ int ktj_output_host(ktj_engine* e, const char** host_ptr, uint64_t* n_bytes) {
   return KTJ_OK;
 }
 
-/* The file sink streams the document from HBM through two small pinned buffers: the copy of one
- * chunk runs while the previous one is written.  One pinned buffer for the whole document would
- * cost more than the copy and the write together: its pages are mapped for the CPU one fault at a
- * time when write() first reads them (0.9 s for 1.6 GB, against 0.03 s for the copy and 0.15 s for
- * the write into the page cache). */
-#define KTJ_FILE_STAGE_BYTES (16ull << 20)
+/* A document on its way to the host goes through the pinned slots, never through a pinned buffer of its
+ * own size: pinning and unpinning such a buffer, and the faults of its pages, cost more than the copy
+ * (60 MB: 15 ms of the 15.7 ms that a session took). */
+
+/* into a caller's memory: every thread has two slots, one being filled by the copy engine while the
+ * other is copied out of.  The destination's pages are often new, so the threads share its faults too. */
+#define KTJ_COPY_OUT_PER_THREAD (4ull << 20) /* a thread costs some 20 us to start: not worth it for less */
+static int copy_document_out(ktj_engine* e, char* dst) {
+  const uint64_t n = e->total_bytes;
+  int rc = drain_stage(e);
+  if (rc != KTJ_OK) return rc;
+  if (n <= KTJ_STAGE_SMALL_BYTES) { /* one short kernel writes it into the ring: a copy engine transfer takes twice as long */
+    PieceJobs job{};
+    const size_t at = (size_t)((uintptr_t)e->out.p & 15u);
+    if (at + n <= KTJ_STAGE_SMALL_BYTES) {
+      job.src[0] = e->out.as<char>(); job.dst[0] = e->stage_small_dev + at; job.n[0] = n; job.count = 1;
+      HIPCHK(put_pieces(job, e->stream));
+      HIPCHK(hipStreamSynchronize(e->stream));
+      memcpy(dst, e->stage_small + at, n);
+      return KTJ_OK;
+    }
+  }
+  rc = ensure_stage(e, KTJ_STAGE_SLOT);
+  if (rc != KTJ_OK) return rc;
+  const size_t part = n < 4 * KTJ_STAGE_SLOT ? KTJ_STAGE_SLOT / 4 : KTJ_STAGE_SLOT; /* short documents: the first part is there sooner */
+  const uint64_t n_parts = (n + part - 1) / part;
+  const unsigned n_threads = copy_threads(n, KTJ_COPY_OUT_PER_THREAD), slots = KTJ_STAGE_SLOTS / n_threads;
+  hipError_t err[KTJ_STAGE_THREADS_MAX];
+  for (auto& x : err) x = hipSuccess;
+  run_workers(n_threads, [&](unsigned t) {
+    err[t] = hipSetDevice(e->device);
+    auto len_of = [&](uint64_t c) { return (size_t)std::min<uint64_t>(part, n - c * part); };
+    auto start = [&](uint64_t turn) { /* thread t takes parts t, t + T, ... */
+      const uint64_t c = t + turn * n_threads;
+      const size_t slot = (size_t)t * slots + turn % slots;
+      if (c >= n_parts || err[t] != hipSuccess) return;
+      err[t] = hipMemcpyAsync(e->stage_big + slot * KTJ_STAGE_SLOT, e->out.as<char>() + c * part, len_of(c), hipMemcpyDeviceToHost, e->stream);
+      if (err[t] == hipSuccess) err[t] = hipEventRecord(e->ev_stage_big[slot], e->stream);
+    };
+    for (unsigned k = 0; k + 1 < slots; ++k) start(k);
+    for (uint64_t turn = 0; t + turn * n_threads < n_parts && err[t] == hipSuccess; ++turn) {
+      start(turn + slots - 1);
+      const uint64_t c = t + turn * n_threads;
+      const size_t slot = (size_t)t * slots + turn % slots;
+      if (err[t] == hipSuccess) err[t] = hipEventSynchronize(e->ev_stage_big[slot]);
+      if (err[t] == hipSuccess) memcpy(dst + c * part, e->stage_big + slot * KTJ_STAGE_SLOT, len_of(c));
+    }
+  });
+  const hipError_t done = hipStreamSynchronize(e->stream);
+  for (unsigned t = 0; t < n_threads; ++t) HIPCHK(err[t]);
+  HIPCHK(done);
+  return KTJ_OK;
+}
+
+int ktj_output_copy(ktj_engine* e, void* dst, uint64_t capacity, uint64_t* n_bytes) {
+  if (!e || !n_bytes) return KTJ_ERR_ARG;
+  if (!e->processed) return KTJ_ERR_STATE;
+  *n_bytes = e->total_bytes;
+  if (!dst || capacity < e->total_bytes) return KTJ_ERR_ARG;
+  HIPCHK(hipSetDevice(e->device));
+  if (e->host_copy_valid) { memcpy(dst, e->pinned_out, e->total_bytes); return KTJ_OK; }
+  struct timespec t0, t1;
+  clock_gettime(CLOCK_MONOTONIC, &t0);
+  const int rc = copy_document_out(e, static_cast<char*>(dst));
+  if (rc != KTJ_OK) return rc;
+  clock_gettime(CLOCK_MONOTONIC, &t1);
+  e->stats.stage_ms[KTJ_STAGE_D2H] = (float)((t1.tv_sec - t0.tv_sec) * 1e3 + (t1.tv_nsec - t0.tv_nsec) * 1e-6);
+  e->stats.stage_bytes[KTJ_STAGE_D2H] = e->total_bytes;
+  return KTJ_OK;
+}
+
+/* into the file: one writer (writers of one file wait for each other on its inode), the copies of the
+ * next slots running meanwhile */
 static int stream_document_to_file(ktj_engine* e, int fd, float* copy_wait_ms) {
   const uint64_t n = e->total_bytes;
-  const uint64_t n_chunks = (n + KTJ_FILE_STAGE_BYTES - 1) / KTJ_FILE_STAGE_BYTES;
-  for (uint64_t k = 0; k < 2 && k < n_chunks; ++k) { /* small documents take one small buffer */
-    const size_t need = (size_t)((std::min<uint64_t>(KTJ_FILE_STAGE_BYTES, n) + 65535) & ~65535ull);
-    if (e->file_stage_cap[k] < need) {
-      if (e->file_stage[k]) HIPCHK(hipHostFree(e->file_stage[k]));
-      e->file_stage[k] = nullptr; e->file_stage_cap[k] = 0;
-      void* p = nullptr;
-      HIPCHK(hipHostMalloc(&p, need, hipHostMallocDefault));
-      e->file_stage[k] = static_cast<char*>(p);
-      e->file_stage_cap[k] = need;
-    }
-    if (!e->ev_file_stage[k]) HIPCHK(hipEventCreateWithFlags(&e->ev_file_stage[k], hipEventDisableTiming));
-  }
-  auto chunk_len = [n](uint64_t c) { return std::min<uint64_t>(KTJ_FILE_STAGE_BYTES, n - c * KTJ_FILE_STAGE_BYTES); };
-  auto start_copy = [e, &chunk_len](uint64_t c) -> hipError_t {
-    hipError_t rc = hipMemcpyAsync(e->file_stage[c & 1], static_cast<const char*>(e->out.p) + c * KTJ_FILE_STAGE_BYTES,
-                                   chunk_len(c), hipMemcpyDeviceToHost, e->stream);
-    return rc != hipSuccess ? rc : hipEventRecord(e->ev_file_stage[c & 1], e->stream);
+  int rc = drain_stage(e);
+  if (rc == KTJ_OK) rc = ensure_stage(e, KTJ_STAGE_SLOT);
+  if (rc != KTJ_OK) return rc;
+  const uint64_t part = n < 4 * KTJ_STAGE_SLOT ? KTJ_STAGE_SLOT / 4 : KTJ_STAGE_SLOT;
+  const uint64_t n_chunks = (n + part - 1) / part;
+  auto chunk_len = [n, part](uint64_t c) { return std::min<uint64_t>(part, n - c * part); };
+  auto start_copy = [&](uint64_t c) -> hipError_t {
+    if (c >= n_chunks) return hipSuccess;
+    const size_t slot = c % KTJ_STAGE_SLOTS;
+    hipError_t err = hipMemcpyAsync(e->stage_big + slot * KTJ_STAGE_SLOT, static_cast<const char*>(e->out.p) + c * part, chunk_len(c),
+                                    hipMemcpyDeviceToHost, e->stream);
+    return err != hipSuccess ? err : hipEventRecord(e->ev_stage_big[slot], e->stream);
   };
   double waited = 0;
-  if (n_chunks) HIPCHK(start_copy(0));
+  for (uint64_t c = 0; c + 1 < KTJ_STAGE_SLOTS; ++c) HIPCHK(start_copy(c));
   for (uint64_t c = 0; c < n_chunks; ++c) {
-    /* the other buffer is free: its chunk (c - 1) has been written */
-    if (c + 1 < n_chunks) HIPCHK(start_copy(c + 1));
+    HIPCHK(start_copy(c + KTJ_STAGE_SLOTS - 1)); /* its slot is free: chunk c - 1 has been written */
     struct timespec t0, t1;
     clock_gettime(CLOCK_MONOTONIC, &t0);
-    HIPCHK(hipEventSynchronize(e->ev_file_stage[c & 1]));
+    HIPCHK(hipEventSynchronize(e->ev_stage_big[c % KTJ_STAGE_SLOTS]));
     clock_gettime(CLOCK_MONOTONIC, &t1);
     waited += (t1.tv_sec - t0.tv_sec) * 1e3 + (t1.tv_nsec - t0.tv_nsec) * 1e-6;
-    const char* src = e->file_stage[c & 1];
+    const char* src = e->stage_big + (c % KTJ_STAGE_SLOTS) * KTJ_STAGE_SLOT;
     uint64_t left = chunk_len(c);
     while (left) {
       const ssize_t w = write(fd, src, left);

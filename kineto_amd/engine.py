@@ -17,6 +17,13 @@ _DBG_DTYPE = dict(ts=np.int64, dur=np.int64, dev=np.int64, res=np.int64, meta=np
                   name_view=np.uint8, name_off=np.uint64, arg_view=np.uint8, arg_off=np.uint64)
 
 
+_new_bytes = C.pythonapi.PyBytes_FromStringAndSize
+_new_bytes.restype, _new_bytes.argtypes = C.py_object, [C.c_void_p, C.c_ssize_t]
+_madvise = C.CDLL(None).madvise
+_madvise.restype, _madvise.argtypes = C.c_int, [C.c_size_t, C.c_size_t, C.c_int]
+_MADV_HUGEPAGE, _PAGE, _FRESH_PAGES_BYTES = 14, 4096, 32 << 20
+
+
 class EngineError(RuntimeError):
     pass
 
@@ -39,41 +46,9 @@ class TraceEngine:
             raise EngineError(f"{what} rc={rc}: {self.lib.ktj_last_error(self.h).decode()}")
 
     def submit_stream(self, sp):
-        """Feeds one ktj_stream through the C ABI, call by call."""
-        s = sp.contents
-        lib, h = self.lib, self.h
-        self._chk(lib.ktj_trace_start(h, s.meta_kv, s.n_meta, s.device_properties), "ktj_trace_start")
-        first = C.c_uint32()
-        self._chk(lib.ktj_intern_strings(h, s.str_blob, s.str_off, s.n_strings, C.byref(first)), "ktj_intern_strings")
-        for i in range(s.n_schemas):
-            d = s.schemas[i]
-            sid = C.c_uint32()
-            fptr = C.cast(C.addressof(s.fields.contents) + d.first_field * C.sizeof(abi.Field), C.POINTER(abi.Field))
-            self._chk(lib.ktj_register_schema(h, fptr, d.n_fields, C.byref(sid)), "ktj_register_schema")
-        for i in range(s.n_collectives):
-            self._chk(lib.ktj_add_collective(h, C.byref(s.collectives[i]), None), "ktj_add_collective")
-        slot0 = C.c_uint64()
-        self._chk(lib.ktj_submit_args(h, s.args, s.n_args, C.byref(slot0)), "ktj_submit_args")
-        self._chk(lib.ktj_set_api_table(h, s.cid_name_ids, s.n_cids, s.flow_start_cids, s.n_flow_start, s.malloc_cid),
-                  "ktj_set_api_table")
-        self._chk(lib.ktj_set_clock_model(h, C.byref(s.clock)), "ktj_set_clock_model")
-        self._chk(lib.ktj_set_window(h, s.window_start_ns, s.window_end_ns), "ktj_set_window")
-        # call order of the buffering logger's replay (libkineto/src/output_membuf.h:91-107): device
-        # and resource infos, the activities, then the spans
-        for kind, ptr, n in ((abi.INFO_DEVICE, s.device_infos, s.n_device_infos),
-                             (abi.INFO_RESOURCE, s.resource_infos, s.n_resource_infos),
-                             (abi.INFO_OVERHEAD, s.overhead_infos, s.n_overhead_infos)):
-            for i in range(n):
-                self._chk(lib.ktj_submit_info(h, kind, C.byref(ptr[i])), "ktj_submit_info")
-        self._chk(lib.ktj_begin_activities(h), "ktj_begin_activities")
-        for cls, ptr, n in ((abi.REC_GENERIC, s.generic, s.n_generic), (abi.REC_RUNTIME, s.runtime, s.n_runtime),
-                            (abi.REC_DEVICE, s.device, s.n_device), (abi.REC_EXTCORR, s.extcorr, s.n_extcorr),
-                            (abi.REC_USERCORR, s.usercorr, s.n_usercorr)):
-            if n:
-                self._chk(lib.ktj_submit_records(h, cls, C.cast(ptr, C.c_void_p), n), "ktj_submit_records")
-        for i in range(s.n_spans):
-            self._chk(lib.ktj_submit_info(h, abi.INFO_SPAN, C.byref(s.spans[i])), "ktj_submit_info")
-        self.end_time_ns = s.end_time_ns
+        """Feeds one ktj_stream through the C ABI."""
+        self._chk(self.lib.ktj_submit_stream(self.h, sp), "ktj_submit_stream")
+        self.end_time_ns = sp.contents.end_time_ns
 
     def process(self, end_time_ns=None):
         self._chk(self.lib.ktj_process(self.h, self.end_time_ns if end_time_ns is None else end_time_ns), "ktj_process")
@@ -85,9 +60,16 @@ class TraceEngine:
         return n.value
 
     def output(self):
-        p, n = C.c_void_p(), C.c_uint64()
-        self._chk(self.lib.ktj_output_host(self.h, C.byref(p), C.byref(n)), "ktj_output_host")
-        return C.string_at(p, n.value)
+        """The finished document as bytes, copied by the library straight into the new object."""
+        n = C.c_uint64(self.output_size())
+        doc = _new_bytes(None, n.value)
+        at = C.cast(C.c_char_p(doc), C.c_void_p).value
+        if n.value >= _FRESH_PAGES_BYTES:
+            # malloc hands out new pages for an object of this size, and a fault for each 4 KiB of them
+            # costs more than the copy (60 MB: 15 000 faults, 14 ms): ask for large pages first
+            _madvise((at + _PAGE - 1) & -_PAGE, (n.value - _PAGE) & -_PAGE, _MADV_HUGEPAGE)
+        self._chk(self.lib.ktj_output_copy(self.h, at, n, C.byref(n)), "ktj_output_copy")
+        return doc
 
     def output_view(self):
         """The finished document as a uint8 numpy view of the engine's pinned host copy (no copy;
