@@ -9,6 +9,7 @@
 #include <hip/hip_runtime_api.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cerrno>
 #include <cstdio>
 #include <cstdlib>
@@ -46,12 +47,12 @@ namespace {
 #define KTJ_STAGE_CHUNK (8ull << 20)
 #define KTJ_STAGE_BIG_MIN (16ull << 20)    /* smallest submission that is spread over threads */
 #define KTJ_STAGE_THREADS_MAX 4
-#define KTJ_STAGE_SLOTS (2 * KTJ_STAGE_THREADS_MAX)
+#define KTJ_STAGE_SLOTS 16
+static_assert(KTJ_STAGE_SLOTS >= 2 * KTJ_STAGE_THREADS_MAX, "two per copying thread");
 /* Submissions between the ring and KTJ_STAGE_BIG_MIN, and documents on their way to the host, pass
- * through eight pinned slots of this size (the first part of the memory that large submissions use
+ * through sixteen pinned slots of this size (the first part of the memory that large submissions use
  * whole): the copy engine works on some while the host fills or empties the others. */
-#define KTJ_STAGE_SLOT (2ull << 20)
-#define KTJ_STAGE_PART (1ull << 20)        /* an upload through them is handed to the copy engine in parts of this size */
+#define KTJ_STAGE_SLOT (1ull << 20)
 /* Working and document memory that waits for the next engine, per device: a thousandth of the card's
  * memory, enough for traces of a few hundred thousand records, which otherwise spend more time in
  * hipMalloc and hipFree than on the GPU.  What KTJ_KIT_LEAN engines in a row could have done with an
@@ -158,6 +159,7 @@ struct HostCtl {
   uint64_t act_bytes;
   uint32_t n_out;
   uint32_t pad;
+  alignas(128) uint64_t part_flag[KTJ_PART_SLOTS]; /* copy_parts: what the slots hold */
 };
 #define KTJ_GUESS_BYTES_PER_ROW 480u /* the fixed text of an event with its flow event */
 #define KTJ_PINNED_SMALL_BYTES (256u << 10) /* header/footer text and small tables of a pass that may not allocate */
@@ -241,7 +243,8 @@ struct ktj_engine {
   InputArena input_arena;
   char* stage_small = nullptr; char* stage_small_dev = nullptr; size_t stage_small_used = 0;
   PieceJobs pieces{}; /* small submissions in the ring that no kernel has moved yet */
-  char* stage_big = nullptr; size_t stage_big_bytes = 0;
+  char* stage_big = nullptr; char* stage_big_dev = nullptr; size_t stage_big_bytes = 0;
+  uint64_t part_seq = 1; /* what the flags of the next document's parts count from */
   size_t stage_big_used = 0; /* of the slots' memory: uploads that the stream may not have passed yet */
   hipEvent_t ev_stage_big[KTJ_STAGE_SLOTS] = {};
   size_t most_needed = 0;    /* the largest pass's working memory and document */
@@ -372,9 +375,8 @@ int stage_piece(ktj_engine* e, void* dst, const void* src, size_t n) {
   return KTJ_OK;
 }
 
-/* The pinned slots: KTJ_STAGE_SLOTS of `slot_bytes` each (kept with the kit). */
-int ensure_stage(ktj_engine* e, size_t slot_bytes) {
-  const size_t bytes = KTJ_STAGE_SLOTS * slot_bytes;
+/* The pinned slots: at least `bytes` of memory (kept with the kit). */
+int ensure_stage(ktj_engine* e, size_t bytes) {
   if (e->stage_big_bytes < bytes) {
     if (e->stage_big) { HIPCHK(hipStreamSynchronize(e->stream)); HIPCHK(hipHostFree(e->stage_big)); }
     e->stage_big = nullptr; e->stage_big_bytes = 0; e->stage_big_used = 0;
@@ -382,6 +384,8 @@ int ensure_stage(ktj_engine* e, size_t slot_bytes) {
     HIPCHK(hipHostMalloc(&p, bytes, hipHostMallocDefault));
     e->stage_big = static_cast<char*>(p);
     e->stage_big_bytes = bytes;
+    HIPCHK(hipHostGetDevicePointer(&p, e->stage_big, 0));
+    e->stage_big_dev = static_cast<char*>(p);
   }
   for (auto& ev : e->ev_stage_big)
     if (!ev) HIPCHK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
@@ -407,9 +411,9 @@ template <typename Worker> void run_workers(unsigned n_threads, Worker worker) {
   for (unsigned t = started; t < n_threads; ++t) worker(t);
   for (auto& th : pool) th.join();
 }
-unsigned copy_threads(size_t bytes, size_t per_thread) {
+unsigned copy_threads(size_t bytes, size_t per_thread, unsigned most) {
   unsigned n = std::thread::hardware_concurrency() / 2;
-  if (n > KTJ_STAGE_THREADS_MAX) n = KTJ_STAGE_THREADS_MAX;
+  if (n > most) n = most;
   if (n > bytes / per_thread) n = (unsigned)(bytes / per_thread);
   return n ? n : 1;
 }
@@ -447,10 +451,10 @@ int append_from_host(ktj_engine* e, DevVec& v, const void* src, size_t n) {
     v.bytes += n;
     return KTJ_OK;
   }
-  const unsigned n_threads = copy_threads(n, KTJ_STAGE_CHUNK);
+  const unsigned n_threads = copy_threads(n, KTJ_STAGE_CHUNK, KTJ_STAGE_THREADS_MAX);
   if (n >= KTJ_STAGE_BIG_MIN && n_threads >= 2) {
     int rc = drain_stage(e);
-    if (rc == KTJ_OK) rc = ensure_stage(e, KTJ_STAGE_CHUNK);
+    if (rc == KTJ_OK) rc = ensure_stage(e, 2 * KTJ_STAGE_THREADS_MAX * KTJ_STAGE_CHUNK);
     if (rc != KTJ_OK) return rc;
     const size_t n_chunks = (n + KTJ_STAGE_CHUNK - 1) / KTJ_STAGE_CHUNK;
     hipError_t err[KTJ_STAGE_THREADS_MAX];
@@ -476,7 +480,7 @@ int append_from_host(ktj_engine* e, DevVec& v, const void* src, size_t n) {
     return KTJ_OK;
   }
   {
-    const int rc = ensure_stage(e, KTJ_STAGE_SLOT);
+    const int rc = ensure_stage(e, KTJ_STAGE_SLOTS * KTJ_STAGE_SLOT);
     if (rc != KTJ_OK) return rc;
   }
   for (size_t done = 0; done < n;) {
@@ -484,7 +488,7 @@ int append_from_host(ktj_engine* e, DevVec& v, const void* src, size_t n) {
       const int rc = drain_stage(e);
       if (rc != KTJ_OK) return rc;
     }
-    const size_t len = std::min(std::min<size_t>(n - done, KTJ_STAGE_PART), e->stage_big_bytes - e->stage_big_used);
+    const size_t len = std::min(std::min<size_t>(n - done, KTJ_STAGE_SLOT), e->stage_big_bytes - e->stage_big_used);
     char* stage = e->stage_big + e->stage_big_used;
     memcpy(stage, static_cast<const char*>(src) + done, len);
     HIPCHK(hipMemcpyAsync(dst + done, stage, len, hipMemcpyHostToDevice, st));
@@ -641,7 +645,7 @@ struct Kit {
   HostCtl* h_ctl = nullptr; HostCtl* h_ctl_dev = nullptr;
   char* pinned_out = nullptr; size_t pinned_out_cap = 0;
   char* stage_small = nullptr; char* stage_small_dev = nullptr;
-  char* stage_big = nullptr; size_t stage_big_bytes = 0;
+  char* stage_big = nullptr; char* stage_big_dev = nullptr; size_t stage_big_bytes = 0;
   DevBuf d_scalars, pool, out, arena_mem;
 };
 std::mutex g_kit_mutex;
@@ -674,7 +678,7 @@ bool take_kit(ktj_engine* e) {
   e->h_ctl = k.h_ctl; e->h_ctl_dev = k.h_ctl_dev;
   e->pinned_out = k.pinned_out; e->pinned_out_cap = k.pinned_out_cap;
   e->stage_small = k.stage_small; e->stage_small_dev = k.stage_small_dev;
-  e->stage_big = k.stage_big; e->stage_big_bytes = k.stage_big_bytes;
+  e->stage_big = k.stage_big; e->stage_big_dev = k.stage_big_dev; e->stage_big_bytes = k.stage_big_bytes;
   e->d_scalars = std::move(k.d_scalars); e->pool = std::move(k.pool); e->out = std::move(k.out);
   e->input_arena.mem = std::move(k.arena_mem);
   k = Kit();
@@ -717,7 +721,7 @@ void give_kit(ktj_engine* e) {
   k.h_ctl = e->h_ctl; k.h_ctl_dev = e->h_ctl_dev; e->h_ctl = nullptr;
   if (e->pinned_out_cap <= KTJ_KIT_PINNED_BYTES_MAX) { k.pinned_out = e->pinned_out; k.pinned_out_cap = e->pinned_out_cap; e->pinned_out = nullptr; }
   k.stage_small = e->stage_small; k.stage_small_dev = e->stage_small_dev; e->stage_small = nullptr;
-  k.stage_big = e->stage_big; k.stage_big_bytes = e->stage_big_bytes; e->stage_big = nullptr;
+  k.stage_big = e->stage_big; k.stage_big_dev = e->stage_big_dev; k.stage_big_bytes = e->stage_big_bytes; e->stage_big = nullptr;
   k.d_scalars = std::move(e->d_scalars);
   if (e->pool.own_cap + e->out.own_cap <= KTJ_KIT_DEVICE_BYTES_MAX) {
     k.pool = std::move(e->pool);
@@ -1652,52 +1656,98 @@ int ktj_output_host(ktj_engine* e, const char** host_ptr, uint64_t* n_bytes) {
  * own size: pinning and unpinning such a buffer, and the faults of its pages, cost more than the copy
  * (60 MB: 15 ms of the 15.7 ms that a session took). */
 
-/* into a caller's memory: every thread has two slots, one being filled by the copy engine while the
- * other is copied out of.  The destination's pages are often new, so the threads share its faults too. */
-#define KTJ_COPY_OUT_PER_THREAD (4ull << 20) /* a thread costs some 20 us to start: not worth it for less */
-static int copy_document_out(ktj_engine* e, char* dst) {
-  const uint64_t n = e->total_bytes;
-  int rc = drain_stage(e);
-  if (rc != KTJ_OK) return rc;
-  if (n <= KTJ_STAGE_SMALL_BYTES) { /* one short kernel writes it into the ring: a copy engine transfer takes twice as long */
-    PieceJobs job{};
-    const size_t at = (size_t)((uintptr_t)e->out.p & 15u);
-    if (at + n <= KTJ_STAGE_SMALL_BYTES) {
-      job.src[0] = e->out.as<char>(); job.dst[0] = e->stage_small_dev + at; job.n[0] = n; job.count = 1;
-      HIPCHK(put_pieces(job, e->stream));
-      HIPCHK(hipStreamSynchronize(e->stream));
-      memcpy(dst, e->stage_small + at, n);
-      return KTJ_OK;
-    }
+/* The parts of a document crossing the link: copy_parts is launched for half of the slots at a time,
+ * whenever the half's previous parts have been taken. */
+struct DocumentParts {
+  ktj_engine* e;
+  uint64_t n, part, n_parts, seq, launched = 0;
+  uint32_t slots;
+  explicit DocumentParts(ktj_engine* e_) : e(e_), n(e_->total_bytes) {
+    /* short documents in short parts: the first is there sooner, and the last is soon taken */
+    part = n < (2ull << 20) ? 128u << 10 : n < (8ull << 20) ? 256u << 10 : 512u << 10;
+    slots = (uint32_t)std::min<uint64_t>(KTJ_PART_SLOTS, KTJ_STAGE_SLOTS * KTJ_STAGE_SLOT / part);
+    n_parts = (n + part - 1) / part;
+    seq = e->part_seq;
+    e->part_seq += n_parts;
   }
-  rc = ensure_stage(e, KTJ_STAGE_SLOT);
+  size_t len(uint64_t c) const { return (size_t)std::min<uint64_t>(part, n - c * part); }
+  const char* data(uint64_t c) const { return e->stage_big + (c % slots) * part; }
+  bool here(uint64_t c) const { return __atomic_load_n(&e->h_ctl->part_flag[c % slots], __ATOMIC_ACQUIRE) == seq + c; }
+  /* may the next parts be launched once `taken` parts have left their slots? */
+  bool room(uint64_t taken) const { return launched < n_parts && launched + slots / 2 <= taken + slots; }
+  hipError_t launch() {
+    const uint64_t last = std::min<uint64_t>(launched + slots / 2, n_parts);
+    const hipError_t err = copy_parts(e->out.as<char>(), n, launched, last, part, slots, e->stage_big_dev, e->h_ctl_dev->part_flag, seq,
+                                      e->d_scalars.as<Scalars>()->part_done, e->stream);
+    launched = last;
+    return err;
+  }
+  /* part c is waited for: a launch that failed must not be waited for forever */
+  hipError_t wait(uint64_t c) const {
+    for (unsigned spins = 1; !here(c); ++spins)
+      if (spins % 65536 == 0) {
+        const hipError_t q = hipStreamQuery(e->stream);
+        if (q != hipErrorNotReady && !here(c)) return q == hipSuccess ? hipErrorUnknown : q;
+      }
+    return hipSuccess;
+  }
+};
+
+/* into a caller's memory: this thread has the parts sent and sees them arrive, the others copy them out of
+ * their slots (one thread's copy is slower than the link, and the destination's pages are often new:
+ * the threads share its faults) */
+#define KTJ_COPY_OUT_PER_THREAD (3ull << 20) /* a thread costs some 10 us to start: not worth it for less */
+#define KTJ_COPY_OUT_THREADS 6
+#define KTJ_COPY_OUT_ONE (512u << 10)
+static int copy_document_out(ktj_engine* e, char* dst) {
+  int rc = drain_stage(e);
+  if (rc == KTJ_OK) rc = ensure_stage(e, KTJ_STAGE_SLOTS * KTJ_STAGE_SLOT);
   if (rc != KTJ_OK) return rc;
-  const size_t part = n < 4 * KTJ_STAGE_SLOT ? KTJ_STAGE_SLOT / 4 : KTJ_STAGE_SLOT; /* short documents: the first part is there sooner */
-  const uint64_t n_parts = (n + part - 1) / part;
-  const unsigned n_threads = copy_threads(n, KTJ_COPY_OUT_PER_THREAD), slots = KTJ_STAGE_SLOTS / n_threads;
-  hipError_t err[KTJ_STAGE_THREADS_MAX];
-  for (auto& x : err) x = hipSuccess;
+  if (e->total_bytes <= KTJ_COPY_OUT_ONE) { /* one transfer and one copy: 8 us for 64 KiB, 20 us in parts */
+    HIPCHK(hipMemcpyAsync(e->stage_big, e->out.p, e->total_bytes, hipMemcpyDeviceToHost, e->stream));
+    HIPCHK(hipStreamSynchronize(e->stream));
+    memcpy(dst, e->stage_big, e->total_bytes);
+    return KTJ_OK;
+  }
+  DocumentParts doc(e);
+  hipError_t err = hipSuccess;
+  while (doc.room(0) && err == hipSuccess) err = doc.launch();
+  HIPCHK(err);
+  const unsigned n_threads = copy_threads(doc.n, KTJ_COPY_OUT_PER_THREAD, KTJ_COPY_OUT_THREADS);
+  std::atomic<uint64_t> arrived{0}, next{0};
+  std::atomic<bool> failed{false};
+  std::atomic<uint64_t> left[KTJ_PART_SLOTS]; /* 1 + the last part that was copied out of the slot */
+  for (auto& x : left) x.store(0, std::memory_order_relaxed);
+  auto copy_one = [&](uint64_t c) {
+    memcpy(dst + c * doc.part, doc.data(c), doc.len(c));
+    left[c % doc.slots].store(c + 1, std::memory_order_release);
+  };
   run_workers(n_threads, [&](unsigned t) {
-    err[t] = hipSetDevice(e->device);
-    auto len_of = [&](uint64_t c) { return (size_t)std::min<uint64_t>(part, n - c * part); };
-    auto start = [&](uint64_t turn) { /* thread t takes parts t, t + T, ... */
-      const uint64_t c = t + turn * n_threads;
-      const size_t slot = (size_t)t * slots + turn % slots;
-      if (c >= n_parts || err[t] != hipSuccess) return;
-      err[t] = hipMemcpyAsync(e->stage_big + slot * KTJ_STAGE_SLOT, e->out.as<char>() + c * part, len_of(c), hipMemcpyDeviceToHost, e->stream);
-      if (err[t] == hipSuccess) err[t] = hipEventRecord(e->ev_stage_big[slot], e->stream);
-    };
-    for (unsigned k = 0; k + 1 < slots; ++k) start(k);
-    for (uint64_t turn = 0; t + turn * n_threads < n_parts && err[t] == hipSuccess; ++turn) {
-      start(turn + slots - 1);
-      const uint64_t c = t + turn * n_threads;
-      const size_t slot = (size_t)t * slots + turn % slots;
-      if (err[t] == hipSuccess) err[t] = hipEventSynchronize(e->ev_stage_big[slot]);
-      if (err[t] == hipSuccess) memcpy(dst + c * part, e->stage_big + slot * KTJ_STAGE_SLOT, len_of(c));
+    if (t != 0) {
+      for (uint64_t c; (c = next.fetch_add(1, std::memory_order_relaxed)) < doc.n_parts;) {
+        for (unsigned spins = 1; arrived.load(std::memory_order_acquire) <= c; ++spins) {
+          if (failed.load(std::memory_order_relaxed)) return;
+          if (spins % 4096 == 0) std::this_thread::yield();
+        }
+        copy_one(c);
+      }
+      return;
     }
+    uint64_t taken = 0; /* parts 0 .. taken - 1 have left their slots */
+    for (uint64_t c = 0; taken < doc.n_parts && err == hipSuccess;) {
+      while (taken < c && left[taken % doc.slots].load(std::memory_order_acquire) > taken) ++taken;
+      if (doc.room(taken)) err = doc.launch();
+      else if (c < doc.launched && doc.here(c)) arrived.store(++c, std::memory_order_release);
+      else {
+        uint64_t k = next.load(std::memory_order_relaxed); /* nothing new: help with what is here */
+        if (k < c && next.compare_exchange_strong(k, k + 1, std::memory_order_relaxed)) copy_one(k);
+        else if (c < doc.launched) err = doc.wait(c);
+      }
+    }
+    if (err != hipSuccess) failed.store(true);
   });
   const hipError_t done = hipStreamSynchronize(e->stream);
-  for (unsigned t = 0; t < n_threads; ++t) HIPCHK(err[t]);
+  HIPCHK(err);
   HIPCHK(done);
   return KTJ_OK;
 }
@@ -1719,41 +1769,31 @@ int ktj_output_copy(ktj_engine* e, void* dst, uint64_t capacity, uint64_t* n_byt
   return KTJ_OK;
 }
 
-/* into the file: one writer (writers of one file wait for each other on its inode), the copies of the
- * next slots running meanwhile */
+/* into the file: one writer (writers of one file wait for each other on its inode), the next parts
+ * crossing meanwhile */
 static int stream_document_to_file(ktj_engine* e, int fd, float* copy_wait_ms) {
-  const uint64_t n = e->total_bytes;
   int rc = drain_stage(e);
-  if (rc == KTJ_OK) rc = ensure_stage(e, KTJ_STAGE_SLOT);
+  if (rc == KTJ_OK) rc = ensure_stage(e, KTJ_STAGE_SLOTS * KTJ_STAGE_SLOT);
   if (rc != KTJ_OK) return rc;
-  const uint64_t part = n < 4 * KTJ_STAGE_SLOT ? KTJ_STAGE_SLOT / 4 : KTJ_STAGE_SLOT;
-  const uint64_t n_chunks = (n + part - 1) / part;
-  auto chunk_len = [n, part](uint64_t c) { return std::min<uint64_t>(part, n - c * part); };
-  auto start_copy = [&](uint64_t c) -> hipError_t {
-    if (c >= n_chunks) return hipSuccess;
-    const size_t slot = c % KTJ_STAGE_SLOTS;
-    hipError_t err = hipMemcpyAsync(e->stage_big + slot * KTJ_STAGE_SLOT, static_cast<const char*>(e->out.p) + c * part, chunk_len(c),
-                                    hipMemcpyDeviceToHost, e->stream);
-    return err != hipSuccess ? err : hipEventRecord(e->ev_stage_big[slot], e->stream);
-  };
+  DocumentParts doc(e);
   double waited = 0;
-  for (uint64_t c = 0; c + 1 < KTJ_STAGE_SLOTS; ++c) HIPCHK(start_copy(c));
-  for (uint64_t c = 0; c < n_chunks; ++c) {
-    HIPCHK(start_copy(c + KTJ_STAGE_SLOTS - 1)); /* its slot is free: chunk c - 1 has been written */
+  for (uint64_t c = 0; c < doc.n_parts; ++c) {
+    while (doc.room(c)) HIPCHK(doc.launch());
     struct timespec t0, t1;
     clock_gettime(CLOCK_MONOTONIC, &t0);
-    HIPCHK(hipEventSynchronize(e->ev_stage_big[c % KTJ_STAGE_SLOTS]));
+    HIPCHK(doc.wait(c));
     clock_gettime(CLOCK_MONOTONIC, &t1);
     waited += (t1.tv_sec - t0.tv_sec) * 1e3 + (t1.tv_nsec - t0.tv_nsec) * 1e-6;
-    const char* src = e->stage_big + (c % KTJ_STAGE_SLOTS) * KTJ_STAGE_SLOT;
-    uint64_t left = chunk_len(c);
+    const char* src = doc.data(c);
+    size_t left = doc.len(c);
     while (left) {
       const ssize_t w = write(fd, src, left);
       if (w < 0 && errno == EINTR) continue;
       if (w <= 0) { (void)hipStreamSynchronize(e->stream); return KTJ_ERR_IO; }
-      src += w; left -= (uint64_t)w;
+      src += w; left -= (size_t)w;
     }
   }
+  HIPCHK(hipStreamSynchronize(e->stream));
   if (copy_wait_ms) *copy_wait_ms = (float)waited;
   return KTJ_OK;
 }

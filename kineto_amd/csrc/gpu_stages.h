@@ -116,6 +116,7 @@ struct Columns {
 #ifndef KTJ_COUNTER_SHARDS
 #define KTJ_COUNTER_SHARDS 64u
 #endif
+#define KTJ_PART_SLOTS 32u
 struct Scalars {
   unsigned long long ts_min_biased;   /* min over valid rows of ts ^ 2^63 */
   unsigned long long ts_max_biased;
@@ -137,6 +138,7 @@ struct Scalars {
   unsigned int n_queues;              /* distinct hardware queues entered into the queue -> stream table */
   unsigned int n_sync_rows;           /* distinct (device, row) pairs of Stream Sync activities */
   unsigned int ext_ids_repeat;        /* two external-correlation records share a correlation id */
+  unsigned int part_done[KTJ_PART_SLOTS]; /* copy_parts: workgroups that have finished the part in a slot */
   alignas(256) JoinPlan plan;         /* key ranges and modes of the join tables: read by every row of the join
                                          kernels, so kept off the cache lines that take the counters' atomics */
   /* The counters that most workgroups add to (KTJ_CNT_*) are kept in KTJ_COUNTER_SHARDS copies, one
@@ -188,6 +190,12 @@ struct PieceJobs {
   uint32_t count;
 };
 hipError_t put_pieces(const PieceJobs& jobs, hipStream_t st);
+/* Parts first .. last - 1 of n bytes of device memory into page-locked slots, part c (part_bytes long, the
+ * last one what is left) into slot c % n_slots at `slots + slot * part_bytes`; as soon as a part is there
+ * flag[slot] becomes seq + c.  src and slots 16-byte aligned, up to 15 bytes behind n are read; n_slots
+ * <= KTJ_PART_SLOTS; done: Scalars::part_done. */
+hipError_t copy_parts(const char* src, uint64_t n, uint64_t first, uint64_t last, uint64_t part_bytes, uint32_t n_slots, char* slots,
+                      uint64_t* flag, uint64_t seq, unsigned int* done, hipStream_t st);
 /* ---- utilities ---- */
 hipError_t fill_u64(uint64_t* p, uint64_t v, uint64_t n, hipStream_t st);
 hipError_t fill_u32(uint32_t* p, uint32_t v, uint64_t n, hipStream_t st);

@@ -204,6 +204,7 @@ __global__ void k_init_scalars(Scalars* s) {
     s->out_of_range = 0; s->out_of_order = 0; s->n_flow = 0; s->n_linked = 0; s->n_blank_names = 0; s->n_valid = 0;
     s->n_unresolved = 0; s->n_sync_typed = 0; s->n_device_orphans = 0; s->error = 0; s->have_stream_src = 0; s->n_dev_ranks = 0; s->n_res_ranks = 0; s->n_dense = 0; s->runtime_ids_repeat = 0;
     s->n_queues = 0; s->n_sync_rows = 0; s->ext_ids_repeat = 0;
+    for (uint32_t k = 0; k < KTJ_PART_SLOTS; ++k) s->part_done[k] = 0;
     for (int k = 0; k < 3; ++k) {
       s->plan.range[k].lo = ~0ULL; s->plan.range[k].hi = 0;
       s->plan.ctl[k].base = 0; s->plan.ctl[k].span = 0; s->plan.ctl[k].direct = 0; s->plan.ctl[k].pad = 0;
@@ -2768,6 +2769,42 @@ hipError_t put_pieces(const PieceJobs& jobs, hipStream_t st) {
     if (jobs.n[k] > most) most = jobs.n[k];
   }
   hipLaunchKernelGGL(k_put_pieces, dim3(grid_stride_for((most >> 4) + 1, KTJ_BLOCK), jobs.count), dim3(KTJ_BLOCK), 0, st, jobs);
+  return KTJ_LAUNCH_CHECK();
+}
+
+/* The document's way to the host: bound by the link (57 GB/s), which few workgroups fill; they take the
+ * parts one after the other so that the host can copy a part on while the next ones cross.  One launch
+ * for many parts: between copy engine transfers or launches of one part each, the event behind every
+ * part costs 15 us or 6 us (12.6 MB in 1 MiB parts: 463 and 385 us). */
+#define COPY_PARTS_GRID 64u
+__global__ void __launch_bounds__(KTJ_BLOCK)
+k_copy_parts(const uint4* src, uint64_t n16, uint64_t first, uint64_t last, uint64_t part16, uint32_t n_slots, uint4* slots,
+             uint64_t* flag, uint64_t seq, unsigned int* done) {
+  for (uint64_t c = first; c < last; ++c) {
+    const uint64_t from = c * part16, len = n16 - from < part16 ? n16 - from : part16;
+    const uint32_t slot = (uint32_t)(c % n_slots);
+    const uint4* s = src + from;
+    uint4* d = slots + (uint64_t)slot * part16;
+    for (uint64_t k = (uint64_t)blockIdx.x * KTJ_BLOCK + threadIdx.x; k < len; k += (uint64_t)gridDim.x * KTJ_BLOCK) d[k] = s[k];
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      __threadfence_system(); /* this workgroup's share is in host memory before it counts as done */
+      if (atomicAdd(&done[slot], 1u) == gridDim.x - 1u) {
+        done[slot] = 0;
+        __threadfence_system();
+        __hip_atomic_store(&flag[slot], seq + c, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+      }
+    }
+  }
+}
+hipError_t copy_parts(const char* src, uint64_t n, uint64_t first, uint64_t last, uint64_t part_bytes, uint32_t n_slots, char* slots,
+                      uint64_t* flag, uint64_t seq, unsigned int* done, hipStream_t st) {
+  if (first >= last) return hipSuccess;
+  if ((((uintptr_t)src | (uintptr_t)slots | part_bytes) & 15u) || n_slots == 0 || n_slots > KTJ_PART_SLOTS || last - first > n_slots ||
+      (last - 1) * part_bytes >= n)
+    return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_copy_parts, dim3(COPY_PARTS_GRID), dim3(KTJ_BLOCK), 0, st, reinterpret_cast<const uint4*>(src), (n + 15) / 16,
+                     first, last, part_bytes / 16, n_slots, reinterpret_cast<uint4*>(slots), flag, seq, done);
   return KTJ_LAUNCH_CHECK();
 }
 

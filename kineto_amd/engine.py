@@ -21,7 +21,7 @@ _new_bytes = C.pythonapi.PyBytes_FromStringAndSize
 _new_bytes.restype, _new_bytes.argtypes = C.py_object, [C.c_void_p, C.c_ssize_t]
 _madvise = C.CDLL(None).madvise
 _madvise.restype, _madvise.argtypes = C.c_int, [C.c_size_t, C.c_size_t, C.c_int]
-_MADV_HUGEPAGE, _PAGE, _FRESH_PAGES_BYTES = 14, 4096, 32 << 20
+_MADV_HUGEPAGE, _PAGE, _FRESH_PAGES_BYTES = 14, 4096, 4 << 20
 
 
 class EngineError(RuntimeError):
