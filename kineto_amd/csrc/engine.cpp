@@ -217,7 +217,7 @@ struct ktj_engine {
   RecordSet generic, runtime, devrows, extcorr, usercorr;
 
   /* working buffers */
-  DevBuf d_scalars, d_name_len, d_arg_len, d_sflags, d_name_off, d_arg_off, d_name_blob, d_arg_blob;
+  DevBuf d_scalars, d_entries, d_name_blob, d_arg_blob;
   DevBuf c_ts, c_dur, c_corr, c_dev, c_res, c_meta, c_ext;
   DevBuf t_full, t_narrow, t_cpu, f_has_runtime, f_first, f_stream_src, f_pay, n_ext_src, n_kern_src, n_copy_src, n_pay, slot_f, slot_n, dev_link, dev_brief, sync_keys, sync_pos, sync_first;
   DevBuf q_keys, q_stream, q_amb, dn_hash, dn_first, dn_dev, dn_key, dn_rank, range_parts;
@@ -1211,10 +1211,8 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
   for (int phase = e->noalloc ? 1 : 0; phase < 2; ++phase) { /* 0: add the sizes up and size the pool; 1: hand the buffers out */
   e->measuring = phase == 0;
   e->pool_need = 0;
-  NEED(e->d_name_len, (ns + 1) * 4ull); NEED(e->d_arg_len, (ns + 1) * 4ull);
-  NEED(e->d_sflags, (ns + 1) * 4ull);
-  NEED(e->d_name_off, (ns + 2) * 8ull); NEED(e->d_arg_off, (ns + 2) * 8ull);
-  NEED(e->d_name_blob, e->blob_bytes * 2 + 8ull * ns + 16); NEED(e->d_arg_blob, e->blob_bytes + 16);
+  NEED(e->d_entries, (ns + 1ull) * sizeof(DictEntry));
+  NEED(e->d_name_blob, e->blob_bytes * 2 + KTJ_DICT_ROOM * (ns + 1ull)); NEED(e->d_arg_blob, e->blob_bytes + KTJ_DICT_ROOM * (ns + 1ull));
   NEED(e->c_ts, Na * 8); NEED(e->c_dur, Na * 8); NEED(e->c_corr, Na * 8);
   NEED(e->c_dev, Na * 8); NEED(e->c_res, Na * 8); NEED(e->c_meta, Na * 4);
   NEED(e->c_ext, Na * 4);
@@ -1241,9 +1239,8 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
   NEED(e->hist, radix_tmp_elems(Na) * 4);
   {
     uint64_t m = scan_tmp_elems(radix_tmp_elems(Na));
-    const uint64_t m2 = scan_tmp_elems(Na), m3 = scan_tmp_elems(ns + 1ull);
+    const uint64_t m2 = scan_tmp_elems(Na);
     if (m2 > m) m = m2;
-    if (m3 > m) m = m3;
     NEED(e->scan_tmp, m * 8);
   }
   NEED(e->mat, Na * sizeof(MatRow)); NEED(e->len, Na * 4); NEED(e->len_sorted, Na * 4); NEED(e->kind_sorted, Na + 16);
@@ -1273,10 +1270,10 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
 
   /* ---- stage 0: dictionary ---- */
   EmitCtx ctx;
-  ctx.dict.name_blob = e->d_name_blob.as<char>(); ctx.dict.name_off = e->d_name_off.as<uint64_t>();
-  ctx.dict.arg_blob = e->d_arg_blob.as<char>(); ctx.dict.arg_off = e->d_arg_off.as<uint64_t>();
+  memset(&ctx.dict, 0, sizeof ctx.dict);
+  ctx.dict.name_blob = e->d_name_blob.as<char>(); ctx.dict.arg_blob = e->d_arg_blob.as<char>();
   ctx.dict.raw_blob = e->str_blob.buf.as<char>(); ctx.dict.raw_off = e->str_off.buf.as<uint64_t>();
-  ctx.dict.flags = e->d_sflags.as<uint32_t>(); ctx.dict.n = ns;
+  ctx.dict.entries = e->d_entries.as<DictEntry>(); ctx.dict.n = ns;
   ctx.fields = e->d_fields.as<ktj_field>(); ctx.schemas = e->d_schemas.as<ktj_schema_desc>();
   ctx.n_schemas = (uint32_t)e->schemas.size();
   ctx.args = e->args.buf.as<uint64_t>(); ctx.n_args = e->n_args;
@@ -1290,15 +1287,8 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
     HIPCHK(fill_u32(cpu_row, 0, cap_cpu + 1ull, st));
   }
   if (n_coll) NEED(e->d_coll_first, 2ull * n_coll * 4);
-  if (ns) {
-    HIPCHK(dict_measure(e->str_blob.buf.as<char>(), e->str_off.buf.as<uint64_t>(), ns, e->d_name_len.as<uint32_t>(),
-                        e->d_arg_len.as<uint32_t>(), e->d_sflags.as<uint32_t>(), st));
-    HIPCHK(scan_u32_to_u64(e->d_name_len.as<uint32_t>(), e->d_name_off.as<uint64_t>(), ns, e->scan_tmp.as<uint64_t>(), st));
-    HIPCHK(scan_u32_to_u64(e->d_arg_len.as<uint32_t>(), e->d_arg_off.as<uint64_t>(), ns, e->scan_tmp.as<uint64_t>(), st));
-    HIPCHK(dict_write(e->str_blob.buf.as<char>(), e->str_off.buf.as<uint64_t>(), ns, e->d_name_off.as<uint64_t>(),
-                      e->d_arg_off.as<uint64_t>(), e->d_sflags.as<uint32_t>(), e->d_name_blob.as<char>(),
-                      e->d_arg_blob.as<char>(), st));
-  }
+  HIPCHK(dict_views(e->str_blob.buf.as<char>(), e->str_off.buf.as<uint64_t>(), ns, e->d_entries.as<DictEntry>(), e->d_name_blob.as<char>(),
+                    e->d_arg_blob.as<char>(), st));
   if (stage_times) HIPCHK(hipEventRecord(e->ev[EV_DICT], st));
 
   /* ---- stage 1: decode ---- */
@@ -1882,10 +1872,22 @@ int ktj_debug_fetch(ktj_engine* e, int what, void* dst, uint64_t cap, uint64_t* 
     case KTJ_DBG_SORT_KEYS:
       if (!e->sorted_keys) { e->last_error = "the sorted keys exist only in an engine created with KTJ_CREATE_PAIR_SORT"; return KTJ_ERR_STATE; }
       src = e->sorted_keys; n = N * 8; break;
-    case KTJ_DBG_NAME_VIEW: src = e->d_name_blob.p; n = e->blob_bytes * 2 + 8ull * e->n_strings; break;
-    case KTJ_DBG_NAME_OFF: src = e->d_name_off.p; n = (e->n_strings + 1) * 8; break;
-    case KTJ_DBG_ARG_VIEW: src = e->d_arg_blob.p; n = e->blob_bytes; break;
-    case KTJ_DBG_ARG_OFF: src = e->d_arg_off.p; n = (e->n_strings + 1) * 8; break;
+    case KTJ_DBG_NAME_VIEW: case KTJ_DBG_NAME_OFF: case KTJ_DBG_ARG_VIEW: case KTJ_DBG_ARG_OFF: {
+      /* the views of all strings, one behind the other, and where each begins */
+      const bool names = what == KTJ_DBG_NAME_VIEW || what == KTJ_DBG_NAME_OFF;
+      std::vector<DictEntry> d(e->n_strings);
+      std::vector<char> blob((names ? 2 : 1) * e->blob_bytes + KTJ_DICT_ROOM * (e->n_strings + 1));
+      HIPCHK(hipSetDevice(e->device));
+      if (!d.empty()) HIPCHK(hipMemcpy(d.data(), e->d_entries.p, d.size() * sizeof(DictEntry), hipMemcpyDeviceToHost));
+      if (!d.empty()) HIPCHK(hipMemcpy(blob.data(), names ? e->d_name_blob.p : e->d_arg_blob.p, blob.size(), hipMemcpyDeviceToHost));
+      std::string view;
+      std::vector<uint64_t> off(1, 0);
+      for (const DictEntry& x : d) { view.append(blob.data() + (names ? x.name_off : x.arg_off), names ? x.name_len : x.arg_len); off.push_back(view.size()); }
+      const bool text = what == KTJ_DBG_NAME_VIEW || what == KTJ_DBG_ARG_VIEW;
+      *n_bytes = text ? view.size() : off.size() * 8;
+      if (dst) memcpy(dst, text ? static_cast<const void*>(view.data()) : off.data(), std::min<uint64_t>(*n_bytes, cap));
+      return KTJ_OK;
+    }
     default: return KTJ_ERR_ARG;
   }
   *n_bytes = n;

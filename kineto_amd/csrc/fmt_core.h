@@ -243,6 +243,7 @@ struct CountWriter {
   KTJ_HD KTJ_FI void dec(uint64_t v) { n += (uint32_t)ndigits_u64(v); }
   KTJ_HD KTJ_FI void dec3(uint32_t) { n += 3; }
   KTJ_HD KTJ_FI void str(const char*, uint64_t len) { n += len; }
+  KTJ_HD KTJ_FI void view(const char*, uint64_t len) { n += len; }
   KTJ_HD KTJ_FI void name(const char*, uint64_t len) { n += len; }
   /* a number that is printed more than once is prepared once */
   typedef uint32_t Prepared;
@@ -364,6 +365,7 @@ struct TileWriter {
     append((uint64_t)(ascii4(x) >> 8), 3);
   }
   KTJ_HD KTJ_FI void name(const char* src, uint64_t len) { str(src, len); }
+  KTJ_HD KTJ_FI void view(const char* src, uint64_t len) { str(src, len); }
   KTJ_HD KTJ_FI void str(const char* src, uint64_t len) {
     if (len == 0) return;
     end(); /* bytes gathered so far */
@@ -711,11 +713,33 @@ struct BlockWriter {
   KTJ_HD KTJ_FI void dec3(uint32_t x) { append((uint64_t)(ascii4(x) >> 8), 3); }
   /* a dictionary string copied by this lane: aligned 8-byte loads, funnel-shifted, sixteen bytes
    * per append while they last */
-  KTJ_HD KTJ_FI void str_own(const char* src, uint64_t len) { str_own_t<false>(src, len); }
+  KTJ_HD KTJ_FI void str_own(const char* src, uint64_t len) { str_own_t<false, false>(src, len); }
   /* RELIEF: with a relief() every 32 bytes, for the one string of an activity that is often longer
    * than the stage has room for (a kernel's name; everywhere else the call would only be code in the way) */
-  template <bool RELIEF> KTJ_HD KTJ_FI void str_own_t(const char* src, uint64_t len) {
+  /* ALIGNED: a dictionary view, which starts on a 16-byte boundary */
+  template <bool RELIEF, bool ALIGNED> KTJ_HD KTJ_FI void str_own_t(const char* src, uint64_t len) {
     if (len == 0) return;
+#if defined(__HIP_DEVICE_COMPILE__)
+    if (ALIGNED) {
+      typedef unsigned long long v2u64 __attribute__((ext_vector_type(2)));
+      typedef const __attribute__((address_space(1))) v2u64* blocks;
+      blocks sp = reinterpret_cast<blocks>((uintptr_t)src);
+      const uint32_t full = (uint32_t)(len >> 4);
+      v2u64 cur = sp[0];
+      KTJ_NOUNROLL
+      for (uint32_t k = 0; k < full; ++k) {
+        if (RELIEF && (k & 1u) != 0) relief();
+        const v2u64 next = sp[k + 1]; /* the view's room reaches one block past its end */
+        append16(cur.x, cur.y);
+        cur = next;
+      }
+      uint32_t rem = (uint32_t)len & 15u;
+      uint64_t v = cur.x;
+      if (rem >= 8u) { append(v, 8); v = cur.y; rem -= 8u; }
+      if (rem) append(v & ((1ULL << (8 * rem)) - 1ULL), rem);
+      return;
+    }
+#endif
     const uintptr_t sa = (uintptr_t)src;
     const uint32_t sh = (uint32_t)(sa & 7u) * 8u;
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -747,10 +771,11 @@ struct BlockWriter {
       append(v & ((1ULL << (8 * rem)) - 1ULL), rem);
     }
   }
-  KTJ_HD KTJ_FI void str(const char* src, uint64_t len) { str_t<false>(src, len); }
+  KTJ_HD KTJ_FI void str(const char* src, uint64_t len) { str_t<false, false>(src, len); }
+  KTJ_HD KTJ_FI void view(const char* src, uint64_t len) { str_t<false, true>(src, len); }
   /* an activity's name */
-  KTJ_HD KTJ_FI void name(const char* src, uint64_t len) { str_t<true>(src, len); }
-  template <bool RELIEF> KTJ_HD KTJ_FI void str_t(const char* src, uint64_t len) {
+  KTJ_HD KTJ_FI void name(const char* src, uint64_t len) { str_t<true, true>(src, len); }
+  template <bool RELIEF, bool ALIGNED> KTJ_HD KTJ_FI void str_t(const char* src, uint64_t len) {
 #if defined(__HIP_DEVICE_COMPILE__)
     const bool big = len >= KTJ_COOP_MIN_BYTES;
     if (__any(big)) { /* see cooperative_word_copy */
@@ -767,13 +792,13 @@ struct BlockWriter {
         dst = wptr;
         stage_close();
         wptr += n_words;
-      } else str_own_t<RELIEF>(src, len);
+      } else str_own_t<RELIEF, ALIGNED>(src, len);
       cooperative_word_copy(body, dst, n_words);
       if (big) str_own(body + (uint64_t)n_words * 8u, tail);
       return;
     }
 #endif
-    str_own_t<RELIEF>(src, len);
+    str_own_t<RELIEF, ALIGNED>(src, len);
   }
 };
 
@@ -934,10 +959,21 @@ KTJ_HD KTJ_FI inline int format_double(uint64_t bits, char* out) {
   return b.n;
 }
 
+KTJ_HD KTJ_FI inline uint32_t dict_flags(const DictViews& d, uint32_t id) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return d.entries[id].flags;
+#else
+  return d.flags[id];
+#endif
+}
 template <class W> KTJ_HD KTJ_FI inline void put_arg_string(W& w, const DictViews& d, uint32_t id, bool raw = false) {
   if (id >= d.n) return;
-  if (raw) w.str(d.raw_blob + d.raw_off[id], d.raw_off[id + 1] - d.raw_off[id]);
-  else w.str(d.arg_blob + d.arg_off[id], d.arg_off[id + 1] - d.arg_off[id]);
+  if (raw) { w.str(d.raw_blob + d.raw_off[id], d.raw_off[id + 1] - d.raw_off[id]); return; }
+#if defined(__HIP_DEVICE_COMPILE__)
+  w.view(d.arg_blob + d.entries[id].arg_off, d.entries[id].arg_len);
+#else
+  w.str(d.arg_blob + d.arg_off[id], d.arg_off[id + 1] - d.arg_off[id]);
+#endif
 }
 template <class W> KTJ_HD KTJ_FI inline void put_array3(W& w, uint64_t a, uint64_t b, uint64_t c) {
   w.ch('['); put_i64(w, (int64_t)a); KTJ_PUT(w, ", "); put_i64(w, (int64_t)b); KTJ_PUT(w, ", ");
@@ -1020,7 +1056,7 @@ KTJ_HD KTJ_FI inline bool has_fragment(const MatRow& r, const EmitCtx& c) {
       c.fields[sd.first_field + skip].type == KTJ_F_RAW) { /* a whole pre-rendered fragment */
     if (r.p[0] + skip >= c.n_args) return false;
     const uint32_t id = (uint32_t)c.args[r.p[0] + skip];
-    return id < c.dict.n && (c.dict.flags[id] & KTJ_SF_ARG_BLANK) == 0;
+    return id < c.dict.n && (dict_flags(c.dict, id) & KTJ_SF_ARG_BLANK) == 0;
   }
   return true;
 }
@@ -1249,15 +1285,20 @@ template <class W> KTJ_HD KTJ_FI inline void put_name(W& w, const MatRow& r, con
     else if (r.name_id == KTJ_NAME_UNKNOWN_OP) { KTJ_PUT(w, "<unknown operation:"); w.dec(r.aux); w.ch('>'); }
     return;
   }
-  if (r.name_id < c.dict.n)
+  if (r.name_id < c.dict.n) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    w.name(c.dict.name_blob + c.dict.entries[r.name_id].name_off, c.dict.entries[r.name_id].name_len);
+#else
     w.name(c.dict.name_blob + c.dict.name_off[r.name_id], c.dict.name_off[r.name_id + 1] - c.dict.name_off[r.name_id]);
+#endif
+  }
 }
 
 /* Generic rows only: marks a CUDA_SYNC activity named "Stream Sync" (output_json.cpp:915) and
  * whether it is the first of its (device, row) in emission order. */
 KTJ_HD KTJ_FI inline void mark_stream_sync(MatRow& m, const EmitCtx& c, bool first_of_row) {
   if ((m.meta & KTJ_M_TYPE_MASK) != KTJ_TYPE_CUDA_SYNC || (m.meta & KTJ_M_NAME_BUILTIN) || m.name_id >= c.dict.n) return;
-  if (!(c.dict.flags[m.name_id] & KTJ_SF_STREAM_SYNC)) return;
+  if (!(dict_flags(c.dict, m.name_id) & KTJ_SF_STREAM_SYNC)) return;
   m.meta |= KTJ_M_SYNC;
   if (first_of_row) m.meta |= KTJ_M_SYNC_FIRST;
 }

@@ -222,10 +222,9 @@ hipError_t scan_u32_to_u64(const uint32_t* in, uint64_t* out /* n+1 */, uint64_t
 hipError_t scan_u32_inplace(uint32_t* data, uint64_t n, uint64_t* tmp, hipStream_t st);
 
 /* ---- stage 0: dictionary ---- */
-hipError_t dict_measure(const char* blob, const uint64_t* off, uint32_t n, uint32_t* name_len, uint32_t* arg_len,
-                        uint32_t* flags, hipStream_t st);
-hipError_t dict_write(const char* blob, const uint64_t* off, uint32_t n, const uint64_t* name_off,
-                      const uint64_t* arg_off, const uint32_t* flags, char* name_blob, char* arg_blob, hipStream_t st);
+/* entries: n; name_blob: 2 * blob bytes + KTJ_DICT_ROOM * (n + 1), arg_blob: blob bytes + KTJ_DICT_ROOM * (n + 1) */
+hipError_t dict_views(const char* blob, const uint64_t* off, uint32_t n, DictEntry* entries, char* name_blob, char* arg_blob,
+                      hipStream_t st);
 
 /* ---- stage 1: decode ---- */
 /* id_range / narrow_range: one KeyRange per workgroup (decode_blocks(n) entries), smallest and

@@ -69,7 +69,21 @@ struct MatRow {
 #define KTJ_NAME_UNKNOWN_OP 6u     /* "<unknown operation:N>", N = aux */
 #define KTJ_NAME_EMPTY 7u
 
-/* string dictionary as the kernels see it */
+/* One string as the kernels read it: one 32-byte load tells where both of its views are.  A view starts
+ * on a 16-byte boundary (a copy then needs no shifting of its source) at a place that follows from the
+ * string's own offset alone, so that one kernel makes the views of all strings without a scan of their
+ * lengths in between. */
+struct DictEntry {
+  uint64_t name_off;
+  uint64_t arg_off;
+  uint32_t name_len;
+  uint32_t arg_len;
+  uint32_t flags;            /* KTJ_SF_*                                                       */
+  uint32_t pad;
+};
+#define KTJ_DICT_ROOM 32u    /* bytes per string beyond its own length (names: twice that) in a view blob */
+
+/* string dictionary as the kernels see it (the host build reads the offset arrays, the device the entries) */
 struct DictViews {
   const char* name_blob;     /* names after the logger's name pipeline                         */
   const uint64_t* name_off;  /* n + 1                                                          */
@@ -79,6 +93,7 @@ struct DictViews {
   const uint64_t* raw_off;   /* n + 1                                                          */
   const uint32_t* flags;     /* KTJ_SF_*                                                       */
   uint32_t n;
+  const DictEntry* entries;  /* device: n, in place of name_off, arg_off and flags              */
 };
 #define KTJ_SF_ARG_BLANK 1u  /* arg view is empty or whitespace only                           */
 #define KTJ_SF_NAME_UNKNOWN 2u /* name view was replaced by "unknown"                          */
