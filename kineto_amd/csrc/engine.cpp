@@ -159,6 +159,7 @@ struct HostCtl {
   uint64_t act_bytes;
   uint32_t n_out;
   uint32_t pad;
+  uint64_t end_clock;
   alignas(128) uint64_t part_flag[KTJ_PART_SLOTS]; /* copy_parts: what the slots hold */
 };
 #define KTJ_GUESS_BYTES_PER_ROW 480u /* the fixed text of an event with its flow event */
@@ -250,6 +251,12 @@ struct ktj_engine {
   size_t most_needed = 0;    /* the largest pass's working memory and document */
   uint32_t kit_lean = 0; /* engines in a row, this kit's, that needed little of what it holds */
   bool hip_failed = false; /* a HIP call failed at some point: nothing of this engine is handed on */
+
+  bool small_unfit = false;  /* these records need the launches of a large trace (Scalars::error of a small pass) */
+  bool small_last = false;   /* the last pass was a small one: it leaves no intermediate arrays for ktj_debug_fetch */
+  bool no_small = false;     /* ktj_debug_fetch makes them */
+  int64_t last_end_time = 0;
+  int wall_clock_khz = 0;
 
   /* results */
   uint64_t N = 0, prefix_len = 0, act_bytes = 0, total_bytes = 0;
@@ -952,6 +959,7 @@ int ktj_submit_records(ktj_engine* e, int rec_class, const void* packed, size_t 
   HIPCHK(hipSetDevice(e->device));
   { const int rc = append_from_host(e, set->owned, packed, n_records * rs); if (rc != KTJ_OK) return rc; }
   set->n += n_records;
+  e->small_unfit = false;
   if (rec_class == KTJ_REC_GENERIC || rec_class == KTJ_REC_RUNTIME || rec_class == KTJ_REC_DEVICE) e->activities_begun = true;
   e->processed = false;
   return KTJ_OK;
@@ -990,6 +998,7 @@ int ktj_submit_records_device(ktj_engine* e, int rec_class, const void* device_p
   if (set->owned.bytes != 0) return KTJ_ERR_STATE;
   set->external = n_records ? device_ptr : nullptr;
   set->n = n_records;
+  e->small_unfit = false;
   if (n_records && (rec_class == KTJ_REC_GENERIC || rec_class == KTJ_REC_RUNTIME || rec_class == KTJ_REC_DEVICE)) e->activities_begun = true;
   e->processed = false;
   return KTJ_OK;
@@ -1149,6 +1158,184 @@ int ktj_submit_stream(ktj_engine* e, const ktj_stream* s) {
   return rc;
 }
 
+/* page-locked room for the document's header, infos and footer */
+static int ensure_text(ktj_engine* e, size_t bytes) {
+  if (bytes <= e->pinned_small_cap) return KTJ_OK;
+  if (e->noalloc) {
+    e->last_error = "ktj_process_noalloc: header and footer text of " + std::to_string(bytes) + " bytes exceeds the pinned staging buffer";
+    return KTJ_ERR_LIMIT;
+  }
+  if (e->pinned_small) HIPCHK(hipHostFree(e->pinned_small));
+  e->pinned_small = nullptr;
+  e->pinned_small_cap = 0;
+  HIPCHK(hipHostMalloc(&e->pinned_small, bytes * 2 + 4096, hipHostMallocDefault));
+  e->pinned_small_cap = bytes * 2 + 4096;
+  void* d = nullptr;
+  HIPCHK(hipHostGetDevicePointer(&d, e->pinned_small, 0));
+  e->pinned_small_dev = static_cast<char*>(d);
+  return KTJ_OK;
+}
+static int short_output(ktj_engine* e) {
+  e->last_error = "ktj_process_noalloc: the document has " + std::to_string(e->total_bytes) + " bytes and needs an output buffer of " +
+                  std::to_string(e->total_bytes + 64);
+  return KTJ_ERR_LIMIT;
+}
+/* per row the fixed text of an event and one string of average length, at most 2 KB */
+static uint64_t guess_per_row(const ktj_engine* e) {
+  const uint64_t avg_string = e->n_strings ? e->blob_bytes / e->n_strings : 0;
+  return std::min<uint64_t>(KTJ_GUESS_BYTES_PER_ROW + avg_string, 2048);
+}
+static EmitCtx emit_context(const ktj_engine* e, uint32_t n_coll) {
+  EmitCtx ctx;
+  memset(&ctx, 0, sizeof ctx);
+  ctx.dict.name_blob = e->d_name_blob.as<char>(); ctx.dict.arg_blob = e->d_arg_blob.as<char>();
+  ctx.dict.raw_blob = e->str_blob.buf.as<char>(); ctx.dict.raw_off = e->str_off.buf.as<uint64_t>();
+  ctx.dict.entries = e->d_entries.as<DictEntry>(); ctx.dict.n = (uint32_t)e->n_strings;
+  ctx.fields = e->d_fields.as<ktj_field>(); ctx.schemas = e->d_schemas.as<ktj_schema_desc>();
+  ctx.n_schemas = (uint32_t)e->schemas.size();
+  ctx.args = e->args.buf.as<uint64_t>(); ctx.n_args = e->n_args;
+  ctx.base_time_ns = e->base_time_ns;
+  ctx.create_flags = e->flags;
+  ctx.coll_blob = e->d_coll_blob.as<char>(); ctx.coll_off = e->d_coll_off.as<uint64_t>(); ctx.n_coll = n_coll;
+  return ctx;
+}
+static ClockDev clock_of(const ktj_engine* e) {
+  ClockDev clk;
+  clk.t0_approx = e->clock.t0_approx; clk.t0 = e->clock.t0;
+  memcpy(&clk.scale_bits, &e->clock.scale, 8);
+  clk.async_offset = e->clock.async_offset; clk.runtime_mode = e->clock.runtime_mode; clk.device_mode = e->clock.device_mode;
+  return clk;
+}
+static Columns columns_of(const ktj_engine* e) {
+  Columns c;
+  c.ts = e->c_ts.as<int64_t>(); c.dur = e->c_dur.as<int64_t>(); c.corr = e->c_corr.as<uint64_t>();
+  c.dev = e->c_dev.as<int64_t>(); c.res = e->c_res.as<int64_t>(); c.meta = e->c_meta.as<uint32_t>();
+  c.ext = e->c_ext.as<int32_t>();
+  return c;
+}
+static void count_stats(ktj_engine* e, uint64_t N) {
+  const uint64_t ng = e->generic.n, nr = e->runtime.n, nd = e->devrows.n, nx = e->extcorr.n;
+  ktj_stats& s = e->stats;
+  memset(&s, 0, sizeof s);
+  s.n_generic = ng; s.n_runtime = nr; s.n_device = nd; s.n_extcorr = nx;
+  s.n_emitted = e->scalars.n_valid;
+  s.out_of_range_events = e->scalars.out_of_range;
+  s.gpu_and_cpu_op_out_of_order = e->scalars.out_of_order;
+  s.n_flow_events = e->scalars.n_flow;
+  s.n_linked = e->scalars.n_linked;
+  s.n_blank_names = e->scalars.n_blank_names;
+  s.output_bytes = e->total_bytes;
+  s.activity_bytes = e->act_bytes;
+  const uint64_t raw_in = ng * sizeof(ktj_generic_rec) + nr * sizeof(ktj_runtime_rec) + nd * sizeof(ktj_device_rec);
+  s.stage_bytes[KTJ_STAGE_DICT] = e->blob_bytes * 3;
+  /* clock conversion and window filter run inside the decode kernels on values that are in registers
+   * there: their bytes (two timestamps in, two out) are bytes of the decode stage already */
+  s.stage_bytes[KTJ_STAGE_DECODE] = raw_in + N * 48;
+  s.stage_bytes[KTJ_STAGE_CONVERT] = 0;
+  s.stage_bytes[KTJ_STAGE_JOIN] = nx * 12 + ng * 12 + nr * 12 + (nr + nd) * 12 * 2 +
+                                   nr * (sizeof(ktj_runtime_rec) + 48 + sizeof(MatRow) + 4); /* incl. the runtime rows' joined rows */
+  s.stage_bytes[KTJ_STAGE_SORT] = N * 56;
+  s.stage_bytes[KTJ_STAGE_SIZE] = (ng * sizeof(ktj_generic_rec) + nd * sizeof(ktj_device_rec)) + (ng + nd) * 48 +
+                                   (ng + nd) * (sizeof(MatRow) + 4) + N * 8;
+  s.stage_bytes[KTJ_STAGE_SCAN] = N * 12;
+  s.stage_bytes[KTJ_STAGE_EMIT] = e->scalars.n_valid * (sizeof(MatRow) + 12) + e->act_bytes;
+}
+
+/* The pass of a small trace: three launches and one wait (small.hip).  *done stays false where the trace
+ * turns out to need the launches of a large one. */
+static int process_small(ktj_engine* e, int64_t end_time_ns, void* out_device, uint64_t out_cap, bool* done) {
+  hipStream_t st = e->stream;
+  const uint64_t ng = e->generic.n, nr = e->runtime.n, nd = e->devrows.n, nx = e->extcorr.n, N = ng + nr + nd;
+  const uint32_t ns = (uint32_t)e->n_strings;
+  size_t pass_bytes = 0;
+  e->pool_used = 0;
+  for (int phase = e->noalloc ? 1 : 0; phase < 2; ++phase) {
+    e->measuring = phase == 0;
+    e->pool_need = 0;
+    NEED(e->d_entries, (ns + 1ull) * sizeof(DictEntry));
+    NEED(e->d_name_blob, e->blob_bytes * 2 + KTJ_DICT_ROOM * (ns + 1ull)); NEED(e->d_arg_blob, e->blob_bytes + KTJ_DICT_ROOM * (ns + 1ull));
+    NEED(e->c_ts, N * 8); NEED(e->c_dur, N * 8); NEED(e->c_corr, N * 8); NEED(e->c_dev, N * 8); NEED(e->c_res, N * 8);
+    NEED(e->c_meta, N * 4); NEED(e->c_ext, N * 4);
+    NEED(e->dev_link, nd * sizeof(DevLink) + 16); NEED(e->mat, N * sizeof(MatRow)); NEED(e->len, N * 4); NEED(e->vals_a, N * 4);
+    if (e->measuring) {
+      e->measuring = false;
+      pass_bytes = e->pool_need;
+      if (e->pool.cap < pass_bytes + 4096) HIPCHK(e->pool.ensure(pass_bytes + 4096));
+    }
+  }
+  const std::string prefix = e->txt_header + e->txt_before;
+  std::string suffix = e->txt_after;
+  append_trace_end(suffix, end_time_ns, e->base_time_ns, e->out_path, std::string());
+  const size_t at_suffix = (prefix.size() + 15) & ~(size_t)15;
+  { const int rc = ensure_text(e, at_suffix + suffix.size() + 64); if (rc != KTJ_OK) return rc; }
+  memcpy(e->pinned_small, prefix.data(), prefix.size());
+  memcpy(static_cast<char*>(e->pinned_small) + at_suffix, suffix.data(), suffix.size());
+  if (out_device) e->out.borrow(out_device, out_cap);
+  else HIPCHK(e->out.ensure(N * guess_per_row(e) + prefix.size() + suffix.size() + (64u << 10), false));
+
+  Scalars* sc = e->d_scalars.as<Scalars>();
+  SmallArgs a;
+  a.g = static_cast<const ktj_generic_rec*>(e->generic.ptr()); a.r = static_cast<const ktj_runtime_rec*>(e->runtime.ptr());
+  a.d = static_cast<const ktj_device_rec*>(e->devrows.ptr()); a.x = static_cast<const ktj_extcorr_rec*>(e->extcorr.ptr());
+  a.ng = (uint32_t)ng; a.nr = (uint32_t)nr; a.nd = (uint32_t)nd; a.nx = (uint32_t)nx;
+  a.slots = small_slots(ng, nr, nd, nx);
+  a.c = columns_of(e);
+  a.link = e->dev_link.as<DevLink>();
+  a.clk = clock_of(e); a.win_start = e->win_start; a.win_end = e->win_end;
+  a.ctx = emit_context(e, 0);
+  a.entries = e->d_entries.as<DictEntry>();
+  a.api = ApiTable{e->d_cid_names.as<uint32_t>(), (uint32_t)e->cid_names.size(), e->d_flow_bits.as<uint32_t>(), e->malloc_cid};
+  a.mat = e->mat.as<MatRow>(); a.len = e->len.as<uint32_t>(); a.perm = e->vals_a.as<uint32_t>();
+  a.sc = sc;
+  SmallText text;
+  text.prefix = e->pinned_small_dev; text.n_prefix = prefix.size();
+  text.suffix = e->pinned_small_dev + at_suffix; text.n_suffix = suffix.size();
+  text.out = e->out.as<char>(); text.out_cap = e->out.cap;
+  text.h_sc = &e->h_ctl_dev->scalars; text.h_total = &e->h_ctl_dev->act_bytes; text.h_end = &e->h_ctl_dev->end_clock;
+  HIPCHK(small_pass(a, ns, st));
+  HIPCHK(small_emit(a, text, st));
+  HIPCHK(hipStreamSynchronize(st));
+  e->stage_small_used = 0;
+  e->stage_big_used = 0;
+  e->scalars = e->h_ctl->scalars;
+  if (e->scalars.error & KTJ_DEVERR_SMALL_UNFIT) { e->small_unfit = true; return KTJ_OK; }
+  if (e->scalars.error) { e->last_error = limit_text(e->scalars.error); return KTJ_ERR_LIMIT; }
+  e->act_bytes = e->h_ctl->act_bytes;
+  e->prefix_len = prefix.size();
+  e->total_bytes = prefix.size() + e->act_bytes + suffix.size();
+  if (e->total_bytes + 64 > text.out_cap) { /* nothing has been written */
+    if (out_device) return short_output(e);
+    HIPCHK(e->out.ensure(e->total_bytes + 64));
+    text.out = e->out.as<char>(); text.out_cap = e->out.cap;
+    HIPCHK(small_emit(a, text, st));
+    HIPCHK(hipStreamSynchronize(st));
+  }
+  if (e->scalars.n_plain) {
+    HIPCHK(small_plain(a, text, st));
+    HIPCHK(hipStreamSynchronize(st));
+  }
+  if (!out_device) e->most_needed = std::max(e->most_needed, pass_bytes + (size_t)e->total_bytes);
+  count_stats(e, N);
+  if (e->wall_clock_khz <= 0) HIPCHK(hipDeviceGetAttribute(&e->wall_clock_khz, hipDeviceAttributeWallClockRate, e->device));
+  /* by the device's clock: decode includes the dictionary, which is made beside it; size is what making
+   * the joined rows takes beyond the sort that runs beside it */
+  const unsigned long long* ck = e->scalars.clock;
+  auto ms = [&](unsigned long long from, unsigned long long to) { return to > from ? (float)((double)(to - from) / e->wall_clock_khz) : 0.0f; };
+  ktj_stats& s = e->stats;
+  if (!(e->flags & KTJ_CREATE_NO_STAGE_TIMES)) {
+    s.stage_ms[KTJ_STAGE_DECODE] = ms(ck[0], ck[1]);
+    s.stage_ms[KTJ_STAGE_JOIN] = ms(ck[1], ck[2]);
+    s.stage_ms[KTJ_STAGE_SORT] = ms(ck[3], ck[4]);
+    s.stage_ms[KTJ_STAGE_SIZE] = ms(ck[4], ck[5]);
+    s.stage_ms[KTJ_STAGE_EMIT] = ms(ck[5], e->h_ctl->end_clock);
+  }
+  s.stage_ms[KTJ_STAGE_TOTAL_GPU] = ms(ck[0], e->h_ctl->end_clock);
+  e->small_last = true;
+  e->processed = true;
+  *done = true;
+  return KTJ_OK;
+}
+
 /* One pass of the whole path.  out_device == nullptr: the document goes into the engine's own
  * buffer and working memory is allocated as needed (ktj_process).  Otherwise (ktj_process_noalloc,
  * e->noalloc set by the caller): the document goes into the caller's buffer of out_cap bytes and
@@ -1199,6 +1386,15 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
     e->coll_dirty = false;
   }
   { const int rc = put_pending_pieces(e); if (rc != KTJ_OK) return rc; }
+  e->last_end_time = end_time_ns;
+  e->small_last = false;
+  if (!e->small_unfit && !e->no_small && nu == 0 && n_coll == 0 && small_fits(ng, nr, nd, nx) && !sort_packed_passes_forced() &&
+      !(e->flags & (KTJ_CREATE_TILE_EMIT | KTJ_CREATE_HASH_JOIN | KTJ_CREATE_PAIR_SORT))) {
+    bool done = false;
+    const int rc = process_small(e, end_time_ns, out_device, out_cap, &done);
+    if (rc != KTJ_OK || done) return rc;
+    e->arena_used = 0;
+  }
 
   /* working memory */
   const uint32_t ns = (uint32_t)e->n_strings;
@@ -1253,10 +1449,7 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
   }
 
   Scalars* sc = e->d_scalars.as<Scalars>();
-  Columns c;
-  c.ts = e->c_ts.as<int64_t>(); c.dur = e->c_dur.as<int64_t>(); c.corr = e->c_corr.as<uint64_t>();
-  c.dev = e->c_dev.as<int64_t>(); c.res = e->c_res.as<int64_t>(); c.meta = e->c_meta.as<uint32_t>();
-  c.ext = e->c_ext.as<int32_t>();
+  const Columns c = columns_of(e);
   const ktj_generic_rec* g_recs = static_cast<const ktj_generic_rec*>(e->generic.ptr());
   const ktj_runtime_rec* r_recs = static_cast<const ktj_runtime_rec*>(e->runtime.ptr());
   const ktj_device_rec* d_recs = static_cast<const ktj_device_rec*>(e->devrows.ptr());
@@ -1269,17 +1462,7 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
   HIPCHK(init_scalars(sc, st));
 
   /* ---- stage 0: dictionary ---- */
-  EmitCtx ctx;
-  memset(&ctx.dict, 0, sizeof ctx.dict);
-  ctx.dict.name_blob = e->d_name_blob.as<char>(); ctx.dict.arg_blob = e->d_arg_blob.as<char>();
-  ctx.dict.raw_blob = e->str_blob.buf.as<char>(); ctx.dict.raw_off = e->str_off.buf.as<uint64_t>();
-  ctx.dict.entries = e->d_entries.as<DictEntry>(); ctx.dict.n = ns;
-  ctx.fields = e->d_fields.as<ktj_field>(); ctx.schemas = e->d_schemas.as<ktj_schema_desc>();
-  ctx.n_schemas = (uint32_t)e->schemas.size();
-  ctx.args = e->args.buf.as<uint64_t>(); ctx.n_args = e->n_args;
-  ctx.base_time_ns = e->base_time_ns;
-  ctx.create_flags = e->flags;
-  ctx.coll_blob = e->d_coll_blob.as<char>(); ctx.coll_off = e->d_coll_off.as<uint64_t>(); ctx.n_coll = n_coll;
+  const EmitCtx ctx = emit_context(e, n_coll);
   uint32_t* cpu_row = nullptr; /* last CPU op per id: only where something is read from that op */
   if (n_coll || max_spans) {
     NEED(e->cpu_row, (cap_cpu + 1ull) * 4);
@@ -1294,10 +1477,7 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
   /* ---- stage 1: decode ---- */
   KeyRange* parts = e->range_parts.as<KeyRange>(); /* [generic | runtime | runtime narrowed | device] */
   /* stage 2a, clock conversion and window filter, happens inside the runtime and device decode */
-  ClockDev clk;
-  clk.t0_approx = e->clock.t0_approx; clk.t0 = e->clock.t0;
-  memcpy(&clk.scale_bits, &e->clock.scale, 8);
-  clk.async_offset = e->clock.async_offset; clk.runtime_mode = e->clock.runtime_mode; clk.device_mode = e->clock.device_mode;
+  const ClockDev clk = clock_of(e);
   HIPCHK(decode_generic(g_recs, ng, c, 0, sc, ctx, parts, st));
   HIPCHK(decode_runtime(r_recs, nr, c, ng, parts + decode_blocks(ng), parts + decode_blocks(ng) + decode_blocks(nr), clk,
                         e->win_start, e->win_end, sc, st));
@@ -1351,12 +1531,9 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
   HIPCHK(publish(sc, nullptr, nullptr, 0, &e->h_ctl_dev->scalars, nullptr, nullptr, st));
   if (!out_device && !e->noalloc && e->out.cap == 0) {
     /* An engine's first pass has no document buffer yet, and how long the document is comes out of
-     * the scan.  A first guess is allocated here, while the GPU is busy with the join: per row the
-     * fixed text of an event and one string of average length, at most 2 KB.  If that turns out too
+     * the scan.  A first guess is allocated here, while the GPU is busy with the join.  If that turns out too
      * small (or cannot be had) the buffer is allocated where its size is known, as in later passes. */
-    const uint64_t avg_string = e->n_strings ? e->blob_bytes / e->n_strings : 0;
-    const uint64_t per_row = KTJ_GUESS_BYTES_PER_ROW + avg_string < 2048 ? KTJ_GUESS_BYTES_PER_ROW + avg_string : 2048;
-    if (e->out.ensure(N * per_row + (1u << 20), false) != hipSuccess) (void)hipGetLastError();
+    if (e->out.ensure(N * guess_per_row(e) + (1u << 20), false) != hipSuccess) (void)hipGetLastError();
   }
   HIPCHK(hipStreamSynchronize(st));
   e->scalars = e->h_ctl->scalars;
@@ -1472,28 +1649,11 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
   e->act_bytes = act_bytes;
   e->total_bytes = prefix.size() + act_bytes + suffix.size();
   if (out_device) { /* the caller's buffer: whole 16-byte blocks are stored, so a little room past the end is needed */
-    if (e->total_bytes + 64 > out_cap) {
-      e->last_error = "ktj_process_noalloc: the document has " + std::to_string(e->total_bytes) + " bytes and needs an output buffer of " +
-                      std::to_string(e->total_bytes + 64);
-      return KTJ_ERR_LIMIT;
-    }
+    if (e->total_bytes + 64 > out_cap) return short_output(e);
     e->out.borrow(out_device, out_cap);
   } else NEED(e->out, e->total_bytes + 64);
   const size_t small = prefix.size() + suffix.size() + 64; /* each piece starts where its place in the document does, modulo 16 */
-  if (small > e->pinned_small_cap && e->noalloc) {
-    e->last_error = "ktj_process_noalloc: header and footer text of " + std::to_string(small) + " bytes exceeds the pinned staging buffer";
-    return KTJ_ERR_LIMIT;
-  }
-  if (small > e->pinned_small_cap) {
-    if (e->pinned_small) HIPCHK(hipHostFree(e->pinned_small));
-    e->pinned_small = nullptr;
-    e->pinned_small_cap = 0;
-    HIPCHK(hipHostMalloc(&e->pinned_small, small * 2 + 4096, hipHostMallocDefault));
-    e->pinned_small_cap = small * 2 + 4096;
-    void* d = nullptr;
-    HIPCHK(hipHostGetDevicePointer(&d, e->pinned_small, 0));
-    e->pinned_small_dev = static_cast<char*>(d);
-  }
+  { const int rc = ensure_text(e, small); if (rc != KTJ_OK) return rc; }
   {
     char* dst_a = e->out.as<char>();
     char* dst_b = dst_a + prefix.size() + act_bytes;
@@ -1522,17 +1682,8 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
   if (!out_device) e->most_needed = std::max(e->most_needed, pass_bytes + (size_t)e->total_bytes);
 
   /* ---- statistics ---- */
+  count_stats(e, N);
   ktj_stats& s = e->stats;
-  memset(&s, 0, sizeof s);
-  s.n_generic = ng; s.n_runtime = nr; s.n_device = nd; s.n_extcorr = nx;
-  s.n_emitted = e->scalars.n_valid;
-  s.out_of_range_events = e->scalars.out_of_range;
-  s.gpu_and_cpu_op_out_of_order = e->scalars.out_of_order;
-  s.n_flow_events = e->scalars.n_flow;
-  s.n_linked = e->scalars.n_linked;
-  s.n_blank_names = e->scalars.n_blank_names;
-  s.output_bytes = e->total_bytes;
-  s.activity_bytes = act_bytes;
   /* stage time = elapsed between the events that bracket it; the two host read-backs (after the
    * distinct-value ranking and after the scan) are excluded from the per-stage figures but are
    * part of KTJ_STAGE_TOTAL_GPU */
@@ -1553,19 +1704,6 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
     HIPCHK(hipEventElapsedTime(&ms, e->ev[EV_START], e->ev[EV_EMIT]));
     s.stage_ms[KTJ_STAGE_TOTAL_GPU] = ms;
   }
-  const uint64_t raw_in = ng * sizeof(ktj_generic_rec) + nr * sizeof(ktj_runtime_rec) + nd * sizeof(ktj_device_rec);
-  s.stage_bytes[KTJ_STAGE_DICT] = e->blob_bytes * 3;
-  /* clock conversion and window filter run inside the decode kernels on values that are in registers
-   * there: their bytes (two timestamps in, two out) are bytes of the decode stage already */
-  s.stage_bytes[KTJ_STAGE_DECODE] = raw_in + N * 48;
-  s.stage_bytes[KTJ_STAGE_CONVERT] = 0;
-  s.stage_bytes[KTJ_STAGE_JOIN] = nx * 12 + ng * 12 + nr * 12 + (nr + nd) * 12 * 2 +
-                                   nr * (sizeof(ktj_runtime_rec) + 48 + sizeof(MatRow) + 4); /* incl. the runtime rows' joined rows */
-  s.stage_bytes[KTJ_STAGE_SORT] = N * 56;
-  s.stage_bytes[KTJ_STAGE_SIZE] = (ng * sizeof(ktj_generic_rec) + nd * sizeof(ktj_device_rec)) + (ng + nd) * 48 +
-                                   (ng + nd) * (sizeof(MatRow) + 4) + N * 8;
-  s.stage_bytes[KTJ_STAGE_SCAN] = N * 12;
-  s.stage_bytes[KTJ_STAGE_EMIT] = e->scalars.n_valid * (sizeof(MatRow) + 12) + act_bytes;
   e->processed = true;
   return KTJ_OK;
 }
@@ -1855,6 +1993,12 @@ int ktj_debug_copy_reference(ktj_engine* e, uint64_t n_bytes, float* ms) {
 int ktj_debug_fetch(ktj_engine* e, int what, void* dst, uint64_t cap, uint64_t* n_bytes) {
   if (!e || !n_bytes) return KTJ_ERR_ARG;
   if (!e->processed) return KTJ_ERR_STATE;
+  if (e->small_last) { /* a small pass keeps none of these: the launches of a large trace make them (and the same document) */
+    e->no_small = true;
+    const int rc = ktj_process(e, e->last_end_time);
+    e->no_small = false;
+    if (rc != KTJ_OK) return rc;
+  }
   const void* src = nullptr;
   uint64_t n = 0;
   const uint64_t N = e->N;

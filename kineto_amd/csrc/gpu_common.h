@@ -1,0 +1,179 @@
+/*
+ * gpu_common.h — device helpers shared by the kernels of large traces (kernels.hip) and of small ones
+ * (small.hip): hashing, wavefront primitives, and the per-record steps that both take.
+ */
+#ifndef KTJ_GPU_COMMON_H_
+#define KTJ_GPU_COMMON_H_
+
+#include <hip/hip_runtime.h>
+
+#include "gpu_stages.h"
+
+namespace ktj {
+namespace gpu {
+
+#define KTJ_NOSLOT 0xFFFFFFFFu
+#define KTJ_BLOCK 256
+
+/* ------------------------------------------------------------------------------------------ */
+/* helpers                                                                                      */
+/* ------------------------------------------------------------------------------------------ */
+__device__ __forceinline__ uint64_t hash64(uint64_t x) {
+  x ^= x >> 33; x *= 0xff51afd7ed558ccdULL; x ^= x >> 33; x *= 0xc4ceb9fe1a85ec53ULL; x ^= x >> 33;
+  return x;
+}
+__device__ __forceinline__ uint32_t lane_id() { return threadIdx.x & 63u; }
+/* Values that a pass streams through once — a row's own columns and records, the rows it writes —
+ * are loaded and stored past the L2's usual replacement: what the cache is for in these passes are
+ * the table lines that rows reach at random. */
+template <typename T> __device__ __forceinline__ T load_once(const T* p) { return __builtin_nontemporal_load(p); }
+template <typename T> __device__ __forceinline__ void store_once(T* p, T v) { __builtin_nontemporal_store(v, p); }
+__device__ __forceinline__ uint64_t lanemask_lt() { return (1ULL << lane_id()) - 1ULL; }
+
+__device__ __forceinline__ uint32_t wave_sum_u32(uint32_t v) {
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+  return v;
+}
+__device__ __forceinline__ void flag_error(Scalars* sc, unsigned bit) { atomicOr(&sc->error, bit); }
+
+/* grid-stride kernels: enough workgroups to fill 256 CUs several times over */
+#define KTJ_MAX_GRID 4096u
+static inline unsigned grid_for(uint64_t n, unsigned per_block) { return (unsigned)((n + per_block - 1) / per_block); }
+static inline unsigned grid_stride_for(uint64_t n, unsigned per_block) {
+  const uint64_t g = (n + per_block - 1) / per_block;
+  return (unsigned)(g < KTJ_MAX_GRID ? g : KTJ_MAX_GRID);
+}
+#define KTJ_LAUNCH_CHECK() hipGetLastError()
+
+
+/* ---- stage 0, one string: both views, by one wavefront ---- */
+__device__ __forceinline__ void dict_string(const char* blob, const uint64_t* off, uint32_t id, DictEntry* entries, char* name_blob, char* arg_blob) {
+  const uint64_t start = off[id], len = off[id + 1] - start;
+  const char* p = blob + start;
+  uint32_t nl = 0, q = 0, bad = 0, nonblank = 0;
+  for (uint64_t k = lane_id(); k < len; k += 64) {
+    const unsigned char c = (unsigned char)p[k];
+    if (c == '\n') { ++nl; continue; }
+    if (c == '"') ++q;
+    if (c < 0x20 || c > 0x7e) ++bad;
+    if (!(c == ' ' || c == '\t' || c == '\v' || c == '\f' || c == '\r')) ++nonblank;
+  }
+  nl = wave_sum_u32(nl); q = wave_sum_u32(q); bad = wave_sum_u32(bad); nonblank = wave_sum_u32(nonblank);
+  const bool is_kernel = len == 6 && p[0] == 'k' && p[1] == 'e' && p[2] == 'r' && p[3] == 'n' && p[4] == 'e' && p[5] == 'l';
+  DictEntry d;
+  d.flags = is_kernel ? KTJ_SF_NAME_KERNEL : bad ? KTJ_SF_NAME_UNKNOWN : 0u;
+  d.name_len = is_kernel ? 6u : bad ? 7u : (uint32_t)len - nl + q;
+  d.arg_len = (uint32_t)len - nl;
+  /* behind the room of the strings before it, whatever their views' lengths are */
+  d.name_off = (2 * start + KTJ_DICT_ROOM * (uint64_t)id) & ~15ULL;
+  d.arg_off = (start + KTJ_DICT_ROOM * (uint64_t)id) & ~15ULL;
+  d.pad = 0;
+  if (nonblank == 0) d.flags |= KTJ_SF_ARG_BLANK;
+  if (len == 11) {
+    const char* want = "Stream Sync";
+    bool same = true;
+    for (int k = 0; k < 11; ++k) same = same && p[k] == want[k];
+    if (same) d.flags |= KTJ_SF_STREAM_SYNC;
+  }
+  if (lane_id() == 0) entries[id] = d;
+  char* an = arg_blob + d.arg_off;
+  char* nn = name_blob + d.name_off;
+  const bool literal_name = (d.flags & (KTJ_SF_NAME_KERNEL | KTJ_SF_NAME_UNKNOWN)) != 0;
+  if (literal_name) {
+    const char* lit = is_kernel ? "Kernel" : "unknown";
+    if (lane_id() < d.name_len) nn[lane_id()] = lit[lane_id()];
+  }
+  uint64_t aw = 0, nw = 0; /* bytes written so far (wave-uniform) */
+  const uint64_t lt = lanemask_lt();
+  for (uint64_t base = 0; base < len; base += 64) {
+    const uint64_t k = base + lane_id();
+    const bool in = k < len;
+    unsigned char c = in ? (unsigned char)p[k] : 0;
+    const bool keep = in && c != '\n';
+    if (c == '\\') c = '/';
+    const bool isq = keep && c == '"';
+    const uint64_t km = __ballot(keep ? 1 : 0);
+    const uint64_t qm = __ballot(isq ? 1 : 0);
+    const uint32_t kpos = (uint32_t)__popcll(km & lt);
+    if (keep) {
+      an[aw + kpos] = (char)c;
+      if (!literal_name) {
+        const uint64_t np = nw + kpos + (uint32_t)__popcll(qm & lt);
+        if (isq) { nn[np] = '\\'; nn[np + 1] = '"'; }
+        else nn[np] = (char)c;
+      }
+    }
+    aw += (uint32_t)__popcll(km);
+    nw += (uint32_t)__popcll(km) + (uint32_t)__popcll(qm);
+  }
+}
+
+/* ---- stage 1, one row: what the decode kernels put into the columns ---- */
+struct RowCols { int64_t ts, dur, dev, res; uint64_t corr; uint32_t meta; };
+__device__ __forceinline__ RowCols cols_generic(const ktj_generic_rec& g, const EmitCtx& ctx) {
+  RowCols r;
+  r.ts = g.start_ns;
+  r.dur = g.end_ns - g.start_ns;                  /* GenericTraceActivity.h:65-67 */
+  r.corr = (uint64_t)(int64_t)g.id;
+  r.dev = generic_device(g, ctx.args, ctx.n_args);
+  r.res = g.resource;
+  r.meta = (generic_record_prints(g, ctx) ? KTJ_M_VALID : 0u) | (KTJ_CLASS_GENERIC << KTJ_M_CLASS_SHIFT);
+  return r;
+}
+/* runtime and device rows: the clock is converted and the capture window applied (stage 2a:
+ * RocprofActivityApi.cpp:166-175, ApproximateClock.cpp:83-90, RocprofActivity.h:42-47 and 122-127,
+ * GenericActivityProfiler.cpp:329-340), so that timestamp and duration are written once */
+__device__ __forceinline__ RowCols cols_runtime(const ktj_runtime_rec& rec, const ClockDev& clk, int64_t win_start, int64_t win_end) {
+  RowCols r;
+  uint64_t b = rec.begin, e = rec.end;
+  convert_range(clk, clk.runtime_mode, &b, &e);
+  r.ts = (int64_t)b;
+  r.dur = (int64_t)(e - b);                       /* RocprofActivity.h:42-47 */
+  r.corr = rec.id;
+  r.dev = (int64_t)rec.pid;
+  r.res = (int64_t)rec.tid;
+  const uint32_t kind = rec.kind <= KTJ_RT_MALLOC ? rec.kind : KTJ_RT_DEFAULT;
+  const uint64_t stream = kind == KTJ_RT_KERNEL ? rec.u.kernel.stream : (kind == KTJ_RT_COPY ? rec.u.copy.stream : 0);
+  r.meta = (KTJ_CLASS_RUNTIME << KTJ_M_CLASS_SHIFT) | (kind << KTJ_M_KIND_SHIFT) | (stream != 0 ? KTJ_M_HAS_STREAM : 0u) |
+           (out_of_range(r.ts, r.dur, win_start, win_end) ? 0u : KTJ_M_VALID);
+  return r;
+}
+__device__ __forceinline__ RowCols cols_device(const ktj_device_rec& d, const ClockDev& clk, int64_t win_start, int64_t win_end) {
+  RowCols r;
+  const uint32_t dom = device_row_domain(d.domain);
+  uint64_t b = d.begin, e = d.end;
+  convert_range(clk, clk.device_mode, &b, &e);
+  device_times(dom, b, e, &r.ts, &r.dur);
+  r.corr = d.id;
+  r.dev = (int64_t)d.device;
+  r.res = device_row_stream(dom, d.stream);
+  r.meta = (KTJ_CLASS_DEVICE << KTJ_M_CLASS_SHIFT) | (dom << KTJ_M_KIND_SHIFT) |
+           (out_of_range(r.ts, r.dur, win_start, win_end) ? 0u : KTJ_M_VALID);
+  return r;
+}
+__device__ __forceinline__ void store_cols(const Columns& c, uint64_t a, const RowCols& r) {
+  c.ts[a] = r.ts; c.dur[a] = r.dur; c.corr[a] = r.corr; c.dev[a] = r.dev; c.res[a] = r.res; c.meta[a] = r.meta; c.ext[a] = 0;
+}
+
+__device__ __forceinline__ bool is_async_op(uint32_t domain) { return domain != KTJ_DOM_MEMSET; }
+
+__device__ __forceinline__ bool dense_key(const DevBrief& d, uint64_t stream, uint64_t* key) {
+  if (!is_async_op(d.domain)) return false;
+  if (stream != 0) *key = stream;
+  else if (d.queue != 0) *key = d.queue | (1ULL << 63);
+  else return false;
+  return true;
+}
+
+/* exact byte length in the low 30 bits, tail kind (see tail_kind) in the top two */
+__device__ __forceinline__ uint32_t row_length(const MatRow& m, const EmitCtx& ctx, Scalars* sc) {
+  if (!(m.meta & KTJ_M_VALID)) return 0;
+  CountWriter cw;
+  format_activity(cw, m, ctx);
+  if (cw.n >= (1ull << 30)) { flag_error(sc, KTJ_DEVERR_RECORD_TOO_LONG); return 0; }
+  return (uint32_t)cw.n | (tail_kind(m, has_args(m, ctx)) << 30);
+}
+
+}  // namespace gpu
+}  // namespace ktj
+#endif

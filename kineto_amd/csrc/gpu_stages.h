@@ -137,7 +137,10 @@ struct Scalars {
   unsigned int runtime_ids_repeat;    /* two runtime rows share a slot of the full table */
   unsigned int n_queues;              /* distinct hardware queues entered into the queue -> stream table */
   unsigned int n_sync_rows;           /* distinct (device, row) pairs of Stream Sync activities */
+  unsigned int n_plain;               /* small traces: activities that small_emit leaves to small_plain */
   unsigned int ext_ids_repeat;        /* two external-correlation records share a correlation id */
+  unsigned long long clock[6];        /* small traces: wall clock (wall_clock64) at the start of the pass, behind decode,
+                                         behind the joins, at the start and end of the sort, at the start of emit */
   unsigned int part_done[KTJ_PART_SLOTS]; /* copy_parts: workgroups that have finished the part in a slot */
   alignas(256) JoinPlan plan;         /* key ranges and modes of the join tables: read by every row of the join
                                          kernels, so kept off the cache lines that take the counters' atomics */
@@ -159,6 +162,8 @@ enum { KTJ_CNT_OUT_OF_RANGE = 0, KTJ_CNT_OUT_OF_ORDER, KTJ_CNT_FLOW, KTJ_CNT_LIN
 #define KTJ_DEVERR_STREAMS 32u            /* more than KTJ_MAX_STREAM_PAIRS (device, stream) pairs */
 #define KTJ_DEVERR_QUEUES 64u             /* more than KTJ_MAX_QUEUES hardware queues */
 #define KTJ_DEVERR_SYNC_ROWS 128u         /* more than KTJ_MAX_SYNC_ROWS (device, row) pairs of Stream Sync events */
+
+#define KTJ_DEVERR_SMALL_UNFIT 256u       /* a small trace that needs the launches of a large one; no error reaches the caller */
 
 #define KTJ_SET_CAP 16384u     /* slots of the distinct-value sets; KTJ_SET_MAX values get a rank */
 #define KTJ_SET_MAX 4096u
@@ -320,6 +325,7 @@ hipError_t clear_error_bits(Scalars* sc, unsigned int bits, hipStream_t st);
 /* The composite-key sort on single 64-bit words (key above the arrival index); perm receives the
  * arrival index per sorted position.  Usable when sort_packed_fits(n, key_bits). */
 bool sort_packed_fits(uint64_t n, uint32_t key_bits);
+bool sort_packed_passes_forced();
 void sort_packed_force_passes(bool on); /* tests: no one-launch sort of a single tile */
 hipError_t sort_packed(Columns c, uint64_t n, SortSets s, const Scalars* sc, uint32_t ts_bits, uint32_t res_bits,
                        uint32_t key_bits, uint64_t* buf_a, uint64_t* buf_b, uint32_t* perm, uint32_t* hist, uint64_t* scan_tmp,
@@ -371,6 +377,40 @@ hipError_t emit(const MatRow* mat, const uint32_t* perm, const uint64_t* offs /*
  * activity in emission order (gather_len); n_rows = number of activities that are written */
 hipError_t emit_direct(const MatRow* mat, const uint32_t* perm, const uint64_t* offs, const uint8_t* kind_sorted,
                        uint64_t n_rows, uint64_t act_bytes, EmitCtx ctx, char* out, uint64_t prefix_len, hipStream_t st);
+
+/* ---- small traces: the whole pass in three launches (small.hip) ---- */
+#define SMALL_ROWS 2048u       /* records of the three classes together: what LDS holds the join tables for */
+#define SMALL_EXT 2048u        /* external-correlation records */
+struct SmallArgs {
+  const ktj_generic_rec* g; const ktj_runtime_rec* r; const ktj_device_rec* d; const ktj_extcorr_rec* x;
+  uint32_t ng, nr, nd, nx;
+  uint32_t slots;              /* small_slots() */
+  Columns c;
+  DevLink* link;               /* nd */
+  ClockDev clk;
+  int64_t win_start, win_end;
+  EmitCtx ctx;
+  DictEntry* entries;
+  ApiTable api;
+  MatRow* mat; uint32_t* len;  /* per arrival index, as for a large trace */
+  uint32_t* perm;
+  Scalars* sc;
+};
+struct SmallText {
+  const char* prefix; uint64_t n_prefix;   /* page-locked, 16-byte aligned, readable up to the next multiple of 16 */
+  const char* suffix; uint64_t n_suffix;
+  char* out; uint64_t out_cap;             /* nothing is written if prefix, activities, suffix and 64 bytes do not fit */
+  Scalars* h_sc; uint64_t* h_total;        /* page-locked: the scalars in front of the shards, the activities' bytes */
+  uint64_t* h_end;                         /* and the wall clock when the last activities were written */
+};
+bool small_fits(uint64_t n_generic, uint64_t n_runtime, uint64_t n_device, uint64_t n_ext);
+uint32_t small_slots(uint64_t n_generic, uint64_t n_runtime, uint64_t n_device, uint64_t n_ext);
+/* decode to order and lengths; then the document.  Scalars::error holds KTJ_DEVERR_SMALL_UNFIT afterwards
+ * where the trace needs the launches of a large one: nothing is written then. */
+hipError_t small_pass(const SmallArgs& a, uint32_t n_strings, hipStream_t st);
+hipError_t small_emit(const SmallArgs& a, const SmallText& t, hipStream_t st);
+/* behind small_emit where Scalars::n_plain is not zero: the activities that it left out */
+hipError_t small_plain(const SmallArgs& a, const SmallText& t, hipStream_t st);
 
 }  // namespace gpu
 }  // namespace ktj

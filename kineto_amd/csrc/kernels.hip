@@ -18,28 +18,10 @@
 #include <cstdlib>
 #include <mutex>
 
-#include "gpu_stages.h"
+#include "gpu_common.h"
 
 namespace ktj {
 namespace gpu {
-
-#define KTJ_NOSLOT 0xFFFFFFFFu
-#define KTJ_BLOCK 256
-
-/* ------------------------------------------------------------------------------------------ */
-/* helpers                                                                                      */
-/* ------------------------------------------------------------------------------------------ */
-__device__ __forceinline__ uint64_t hash64(uint64_t x) {
-  x ^= x >> 33; x *= 0xff51afd7ed558ccdULL; x ^= x >> 33; x *= 0xc4ceb9fe1a85ec53ULL; x ^= x >> 33;
-  return x;
-}
-__device__ __forceinline__ uint32_t lane_id() { return threadIdx.x & 63u; }
-/* Values that a pass streams through once — a row's own columns and records, the rows it writes —
- * are loaded and stored past the L2's usual replacement: what the cache is for in these passes are
- * the table lines that rows reach at random. */
-template <typename T> __device__ __forceinline__ T load_once(const T* p) { return __builtin_nontemporal_load(p); }
-template <typename T> __device__ __forceinline__ void store_once(T* p, T v) { __builtin_nontemporal_store(v, p); }
-__device__ __forceinline__ uint64_t lanemask_lt() { return (1ULL << lane_id()) - 1ULL; }
 
 /* Returns the slot holding `key`, inserting it if absent; KTJ_NOSLOT when no free slot lies within
  * KTJ_TABLE_PROBES slots of the key's home slot (a table that is at most half full never gets
@@ -157,10 +139,6 @@ __device__ uint32_t slot_find(const Table& t, uint64_t key) {
   return KTJ_NOSLOT;
 }
 
-__device__ __forceinline__ uint32_t wave_sum_u32(uint32_t v) {
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-  return v;
-}
 /* Sums a per-thread count over the workgroup and adds it to a global counter with one atomic per
  * workgroup (a single hot address serialises atomics in L2, so they must be rare).  Must be
  * reached by every thread of the workgroup.  block_add_to: a counter of its own address, for counts
@@ -184,8 +162,6 @@ __device__ __forceinline__ void block_add(Scalars* sc, int which, uint32_t mine)
   const uint32_t t = block_sum(mine);
   if (threadIdx.x == 0 && t) atomicAdd(&sc->shard[blockIdx.x & (KTJ_COUNTER_SHARDS - 1u)][which], (unsigned long long)t);
 }
-/* grid-stride kernels: enough workgroups to fill 256 CUs several times over */
-#define KTJ_MAX_GRID 4096u
 
 __global__ void k_fill_u64(uint64_t* p, uint64_t v, uint64_t n) {
   uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -211,13 +187,6 @@ __global__ void k_init_scalars(Scalars* s) {
     }
   }
 }
-
-static inline unsigned grid_for(uint64_t n, unsigned per_block) { return (unsigned)((n + per_block - 1) / per_block); }
-static inline unsigned grid_stride_for(uint64_t n, unsigned per_block) {
-  const uint64_t g = (n + per_block - 1) / per_block;
-  return (unsigned)(g < KTJ_MAX_GRID ? g : KTJ_MAX_GRID);
-}
-#define KTJ_LAUNCH_CHECK() hipGetLastError()
 
 hipError_t fill_u64(uint64_t* p, uint64_t v, uint64_t n, hipStream_t st) {
   if (n == 0) return hipSuccess;
@@ -450,66 +419,6 @@ hipError_t scan_u32_inplace(uint32_t* data, uint64_t n, uint64_t* tmp, hipStream
 /*   name view = "kernel"→"Kernel", sanitize, non-printable → "unknown", quote escaping         */
 /*                                             (output_json.cpp:946-949, 86-112)                */
 /* ------------------------------------------------------------------------------------------ */
-__device__ __forceinline__ void dict_string(const char* blob, const uint64_t* off, uint32_t id, DictEntry* entries, char* name_blob, char* arg_blob) {
-  const uint64_t start = off[id], len = off[id + 1] - start;
-  const char* p = blob + start;
-  uint32_t nl = 0, q = 0, bad = 0, nonblank = 0;
-  for (uint64_t k = lane_id(); k < len; k += 64) {
-    const unsigned char c = (unsigned char)p[k];
-    if (c == '\n') { ++nl; continue; }
-    if (c == '"') ++q;
-    if (c < 0x20 || c > 0x7e) ++bad;
-    if (!(c == ' ' || c == '\t' || c == '\v' || c == '\f' || c == '\r')) ++nonblank;
-  }
-  nl = wave_sum_u32(nl); q = wave_sum_u32(q); bad = wave_sum_u32(bad); nonblank = wave_sum_u32(nonblank);
-  const bool is_kernel = len == 6 && p[0] == 'k' && p[1] == 'e' && p[2] == 'r' && p[3] == 'n' && p[4] == 'e' && p[5] == 'l';
-  DictEntry d;
-  d.flags = is_kernel ? KTJ_SF_NAME_KERNEL : bad ? KTJ_SF_NAME_UNKNOWN : 0u;
-  d.name_len = is_kernel ? 6u : bad ? 7u : (uint32_t)len - nl + q;
-  d.arg_len = (uint32_t)len - nl;
-  /* behind the room of the strings before it, whatever their views' lengths are */
-  d.name_off = (2 * start + KTJ_DICT_ROOM * (uint64_t)id) & ~15ULL;
-  d.arg_off = (start + KTJ_DICT_ROOM * (uint64_t)id) & ~15ULL;
-  d.pad = 0;
-  if (nonblank == 0) d.flags |= KTJ_SF_ARG_BLANK;
-  if (len == 11) {
-    const char* want = "Stream Sync";
-    bool same = true;
-    for (int k = 0; k < 11; ++k) same = same && p[k] == want[k];
-    if (same) d.flags |= KTJ_SF_STREAM_SYNC;
-  }
-  if (lane_id() == 0) entries[id] = d;
-  char* an = arg_blob + d.arg_off;
-  char* nn = name_blob + d.name_off;
-  const bool literal_name = (d.flags & (KTJ_SF_NAME_KERNEL | KTJ_SF_NAME_UNKNOWN)) != 0;
-  if (literal_name) {
-    const char* lit = is_kernel ? "Kernel" : "unknown";
-    if (lane_id() < d.name_len) nn[lane_id()] = lit[lane_id()];
-  }
-  uint64_t aw = 0, nw = 0; /* bytes written so far (wave-uniform) */
-  const uint64_t lt = lanemask_lt();
-  for (uint64_t base = 0; base < len; base += 64) {
-    const uint64_t k = base + lane_id();
-    const bool in = k < len;
-    unsigned char c = in ? (unsigned char)p[k] : 0;
-    const bool keep = in && c != '\n';
-    if (c == '\\') c = '/';
-    const bool isq = keep && c == '"';
-    const uint64_t km = __ballot(keep ? 1 : 0);
-    const uint64_t qm = __ballot(isq ? 1 : 0);
-    const uint32_t kpos = (uint32_t)__popcll(km & lt);
-    if (keep) {
-      an[aw + kpos] = (char)c;
-      if (!literal_name) {
-        const uint64_t np = nw + kpos + (uint32_t)__popcll(qm & lt);
-        if (isq) { nn[np] = '\\'; nn[np + 1] = '"'; }
-        else nn[np] = (char)c;
-      }
-    }
-    aw += (uint32_t)__popcll(km);
-    nw += (uint32_t)__popcll(km) + (uint32_t)__popcll(qm);
-  }
-}
 __global__ void k_dict(const char* blob, const uint64_t* off, uint32_t n, DictEntry* entries, char* name_blob, char* arg_blob) {
   const uint32_t id = blockIdx.x * (KTJ_BLOCK >> 6) + (threadIdx.x >> 6);
   if (id < n) dict_string(blob, off, id, entries, name_blob, arg_blob);
@@ -568,19 +477,8 @@ __global__ void k_decode_generic(const ktj_generic_rec* recs, uint64_t n, Column
   if (__syncthreads_or(sync_typed ? 1 : 0)) block_add(sc, KTJ_CNT_SYNC_TYPED, sync_typed ? 1u : 0u);
   if (id_range) block_key_range(threadIdx.x < cnt, threadIdx.x < cnt ? (uint64_t)(int64_t)l[threadIdx.x].id : 0, id_range);
   if (threadIdx.x >= cnt) return;
-  const ktj_generic_rec g = l[threadIdx.x];
-  const uint64_t a = first + (uint64_t)blockIdx.x * KTJ_BLOCK + threadIdx.x;
-  c.ts[a] = g.start_ns;
-  c.dur[a] = g.end_ns - g.start_ns;               /* GenericTraceActivity.h:65-67 */
-  c.corr[a] = (uint64_t)(int64_t)g.id;
-  c.dev[a] = generic_device(g, ctx.args, ctx.n_args);
-  c.res[a] = g.resource;
-  c.meta[a] = (generic_record_prints(g, ctx) ? KTJ_M_VALID : 0u) | (KTJ_CLASS_GENERIC << KTJ_M_CLASS_SHIFT);
-  c.ext[a] = 0;
+  store_cols(c, first + (uint64_t)blockIdx.x * KTJ_BLOCK + threadIdx.x, cols_generic(l[threadIdx.x], ctx));
 }
-/* The runtime and device kernels also convert the clock and apply the capture window (stage 2a:
- * RocprofActivityApi.cpp:166-175, ApproximateClock.cpp:83-90, RocprofActivity.h:42-47 and 122-127,
- * GenericActivityProfiler.cpp:329-340), so that timestamp and duration are written once. */
 __global__ void k_decode_runtime(const ktj_runtime_rec* recs, uint64_t n, Columns c, uint64_t first, KeyRange* id_range,
                                  KeyRange* narrow_range, ClockDev clk, int64_t win_start, int64_t win_end, Scalars* sc) {
   __shared__ uint4 stage[KTJ_BLOCK * sizeof(ktj_runtime_rec) / 16];
@@ -594,22 +492,9 @@ __global__ void k_decode_runtime(const ktj_runtime_rec* recs, uint64_t n, Column
   }
   uint32_t oor = 0;
   if (threadIdx.x < cnt) {
-  const ktj_runtime_rec* r = &l[threadIdx.x];
-  const uint64_t a = first + (uint64_t)blockIdx.x * KTJ_BLOCK + threadIdx.x;
-  uint64_t b = r->begin, e = r->end;
-  convert_range(clk, clk.runtime_mode, &b, &e);
-  const int64_t ts = (int64_t)b, dur = (int64_t)(e - b);   /* RocprofActivity.h:42-47 */
-  oor = out_of_range(ts, dur, win_start, win_end) ? 1u : 0u;
-  c.ts[a] = ts;
-  c.dur[a] = dur;
-  c.corr[a] = r->id;
-  c.dev[a] = (int64_t)r->pid;
-  c.res[a] = (int64_t)r->tid;
-  const uint32_t kind = r->kind <= KTJ_RT_MALLOC ? r->kind : KTJ_RT_DEFAULT;
-  const uint64_t stream = kind == KTJ_RT_KERNEL ? r->u.kernel.stream : (kind == KTJ_RT_COPY ? r->u.copy.stream : 0);
-  c.meta[a] = (KTJ_CLASS_RUNTIME << KTJ_M_CLASS_SHIFT) | (kind << KTJ_M_KIND_SHIFT) | (stream != 0 ? KTJ_M_HAS_STREAM : 0u) |
-              (oor ? 0u : KTJ_M_VALID);
-  c.ext[a] = 0;
+    const RowCols r = cols_runtime(l[threadIdx.x], clk, win_start, win_end);
+    oor = r.meta & KTJ_M_VALID ? 0u : 1u;
+    store_cols(c, first + (uint64_t)blockIdx.x * KTJ_BLOCK + threadIdx.x, r);
   }
   block_add(sc, KTJ_CNT_OUT_OF_RANGE, oor);
 }
@@ -621,24 +506,14 @@ __global__ void k_decode_device(const ktj_device_rec* recs, uint64_t n, Columns 
   block_key_range(threadIdx.x < cnt, threadIdx.x < cnt ? l[threadIdx.x].id : 0, id_range);
   uint32_t oor = 0;
   if (threadIdx.x < cnt) {
-  const ktj_device_rec* d = &l[threadIdx.x];
-  const uint64_t a = first + (uint64_t)blockIdx.x * KTJ_BLOCK + threadIdx.x;
-  const uint32_t dom = device_row_domain(d->domain);
-  uint64_t b = d->begin, e = d->end;
-  convert_range(clk, clk.device_mode, &b, &e);
-  int64_t ts, dur;
-  device_times(dom, b, e, &ts, &dur);
-  oor = out_of_range(ts, dur, win_start, win_end) ? 1u : 0u;
-  c.ts[a] = ts;
-  c.dur[a] = dur;
-  c.corr[a] = d->id;
-  c.dev[a] = (int64_t)d->device;
-  c.res[a] = device_row_stream(dom, d->stream);
-  c.meta[a] = (KTJ_CLASS_DEVICE << KTJ_M_CLASS_SHIFT) | (dom << KTJ_M_KIND_SHIFT) | (oor ? 0u : KTJ_M_VALID);
-  c.ext[a] = 0;
-  DevBrief br;
-  br.queue = d->queue; br.device = d->device; br.domain = dom;
-  brief[a - first] = br;
+    const ktj_device_rec* d = &l[threadIdx.x];
+    const uint64_t i = (uint64_t)blockIdx.x * KTJ_BLOCK + threadIdx.x;
+    const RowCols r = cols_device(*d, clk, win_start, win_end);
+    oor = r.meta & KTJ_M_VALID ? 0u : 1u;
+    store_cols(c, first + i, r);
+    DevBrief br;
+    br.queue = d->queue; br.device = d->device; br.domain = device_row_domain(d->domain);
+    brief[i] = br;
   }
   block_add(sc, KTJ_CNT_OUT_OF_RANGE, oor);
 }
@@ -671,8 +546,6 @@ hipError_t decode_device(const ktj_device_rec* r, uint64_t n, Columns c, uint64_
 /* What a device row takes over from "its" runtime row is then published into the table slot by  */
 /* the winning row, so that a device row needs one slot of each table and no other row.          */
 /* ------------------------------------------------------------------------------------------ */
-__device__ __forceinline__ void flag_error(Scalars* sc, unsigned bit) { atomicOr(&sc->error, bit); }
-
 /* min / max of p[i * stride] (optionally int-narrowed) into *out: one atomic pair per workgroup */
 __global__ void k_key_range(const uint64_t* p, uint32_t stride, uint64_t n, int narrow, KeyRange* out) {
   __shared__ unsigned long long s_lo[KTJ_BLOCK >> 6], s_hi[KTJ_BLOCK >> 6];
@@ -883,8 +756,6 @@ __global__ void k_resolve_external(const ktj_extcorr_rec* e, uint64_t n, Table t
     nc.pay[slot].info = info;
   }
 }
-__device__ __forceinline__ bool is_async_op(uint32_t domain) { return domain != KTJ_DOM_MEMSET; }
-
 /* One pass over the device rows with one slot of each table:
  *  - "External id" (output_json.cpp:871-874) from the narrow slot,
  *  - checkTimestampOrder (GenericActivityProfiler.cpp:363-395) against the first row of the id,
@@ -1138,13 +1009,6 @@ __global__ void k_queue_fill(const DevBrief* d, uint64_t n, Columns c, uint64_t 
   const uint32_t slot = table_find(t.q_keys, KTJ_QUEUE_CAP - 1u, d[i].queue);
   if (slot == KTJ_NOSLOT || t.q_amb[slot] != 0 || t.q_stream[slot] == 0) return;
   c.res[a] = (int64_t)t.q_stream[slot];
-}
-__device__ __forceinline__ bool dense_key(const DevBrief& d, uint64_t stream, uint64_t* key) {
-  if (!is_async_op(d.domain)) return false;
-  if (stream != 0) *key = stream;
-  else if (d.queue != 0) *key = d.queue | (1ULL << 63);
-  else return false;
-  return true;
 }
 __device__ __forceinline__ uint64_t dense_hash(int32_t device, uint64_t key) {
   uint64_t h = hash64(key ^ hash64((uint64_t)(int64_t)device + 0x9E3779B97F4A7C15ULL));
@@ -2024,6 +1888,7 @@ static hipError_t sort_packed_t(Columns c, uint64_t n, SortSets s, const Scalars
 /* tests: the one-launch sort of a single tile switched off, so that such a trace takes the passes of a large one */
 static bool g_sortp_no_single = false;
 void sort_packed_force_passes(bool on) { g_sortp_no_single = on; }
+bool sort_packed_passes_forced() { return g_sortp_no_single; }
 bool sort_packed_fits(uint64_t n, uint32_t key_bits) {
   const uint32_t total_bits = key_bits + 1u;
   const uint32_t idx_bits = (uint32_t)(64 - __builtin_clzll(n > 1 ? n - 1 : 1));
@@ -2090,14 +1955,6 @@ __device__ __forceinline__ void row_to_lds(const T& r, uint4* lds) {
   const uint4* s = reinterpret_cast<const uint4*>(&r);
 #pragma unroll
   for (int k = 0; k < (int)(sizeof(T) / 16); ++k) lds[threadIdx.x * (sizeof(T) / 16) + k] = s[k];
-}
-/* exact byte length in the low 30 bits, tail kind (see tail_kind) in the top two */
-__device__ __forceinline__ uint32_t row_length(const MatRow& m, const EmitCtx& ctx, Scalars* sc) {
-  if (!(m.meta & KTJ_M_VALID)) return 0;
-  CountWriter cw;
-  format_activity(cw, m, ctx);
-  if (cw.n >= (1ull << 30)) { flag_error(sc, KTJ_DEVERR_RECORD_TOO_LONG); return 0; }
-  return (uint32_t)cw.n | (tail_kind(m, has_args(m, ctx)) << 30);
 }
 struct RowStats { uint32_t n_flow = 0, n_blank = 0; };
 __device__ __forceinline__ void count_row_stats(const MatRow& m, const EmitCtx& ctx, RowStats* rs) {
