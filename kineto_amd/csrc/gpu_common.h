@@ -174,6 +174,36 @@ __device__ __forceinline__ uint32_t row_length(const MatRow& m, const EmitCtx& c
   return (uint32_t)cw.n | (tail_kind(m, has_args(m, ctx)) << 30);
 }
 
+/* ---- bytes to any address of the document ---- */
+typedef uint64_t u64_any __attribute__((aligned(1)));
+typedef uint32_t u32_any __attribute__((aligned(1)));
+typedef uint16_t u16_any __attribute__((aligned(1)));
+typedef __attribute__((address_space(1))) char* doc_ptr; /* global memory: no flat accesses */
+typedef const __attribute__((address_space(1))) char* text_ptr;
+__device__ __forceinline__ void put8(doc_ptr p, uint64_t v) { *reinterpret_cast<__attribute__((address_space(1))) u64_any*>(p) = v; }
+__device__ __forceinline__ uint64_t get8(text_ptr p) { return *reinterpret_cast<const __attribute__((address_space(1))) u64_any*>(p); }
+/* the n (0..7) low bytes of v */
+__device__ __forceinline__ void put_low(doc_ptr p, uint64_t v, uint32_t n) {
+  if (n & 4u) { *reinterpret_cast<__attribute__((address_space(1))) u32_any*>(p) = (uint32_t)v; p += 4; v >>= 32; }
+  if (n & 2u) { *reinterpret_cast<__attribute__((address_space(1))) u16_any*>(p) = (uint16_t)v; p += 2; v >>= 16; }
+  if (n & 1u) *p = (char)v;
+}
+
+/* n bytes of header or footer text, by the whole workgroup */
+__device__ __forceinline__ void put_text_block(const char* src, char* dst, uint64_t n) { /* src 16-byte aligned */
+  const doc_ptr d = reinterpret_cast<doc_ptr>((uintptr_t)dst);
+  const uint4* s = reinterpret_cast<const uint4*>(src);
+  for (uint64_t k = threadIdx.x; k < (n + 15u) / 16u; k += blockDim.x) {
+    const uint4 v = s[k];
+    const uint64_t lo = v.x | ((uint64_t)v.y << 32), hi = v.z | ((uint64_t)v.w << 32);
+    const uint64_t left = n - k * 16u;
+    if (left >= 16u) { put8(d + k * 16u, lo); put8(d + k * 16u + 8u, hi); }
+    else if (left >= 8u) { put8(d + k * 16u, lo); put_low(d + k * 16u + 8u, hi, (uint32_t)left - 8u); }
+    else put_low(d + k * 16u, lo, (uint32_t)left);
+  }
+}
+
+
 }  // namespace gpu
 }  // namespace ktj
 #endif
