@@ -122,9 +122,10 @@ k_emit(const MatRow* mat, const uint32_t* perm, const uint64_t* offs, uint64_t n
  * for the quads' sake.  The document's prefix and suffix are already in place when this kernel
  * runs; the first and the last activity merge with them. */
 __global__ void __launch_bounds__(KTJ_BLOCK) __attribute__((amdgpu_waves_per_eu(3)))
-k_emit_direct(const MatRow* mat, const uint32_t* perm, const uint64_t* offs, const uint8_t* kind_sorted, uint64_t n_rows,
-              EmitCtx ctx, char* out, uint64_t prefix_len) {
+k_emit_direct(const MatRow* mat, const uint32_t* perm, const uint64_t* offs, const uint8_t* kind_sorted,
+              EmitCtx ctx, char* out, uint64_t prefix_len, const Scalars* sc) {
   const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const uint64_t n_rows = sc->emit_rows;
   uint64_t o = 0;
   uint32_t row = 0;
   bool active = i < n_rows;
@@ -156,13 +157,12 @@ k_emit_direct(const MatRow* mat, const uint32_t* perm, const uint64_t* offs, con
   }
   w.flush(true);
 }
-hipError_t emit_direct(const MatRow* mat, const uint32_t* perm, const uint64_t* offs, const uint8_t* kind_sorted,
-                       uint64_t n_rows, uint64_t act_bytes, EmitCtx ctx, char* out, uint64_t prefix_len, hipStream_t st) {
-  if (n_rows == 0) return hipSuccess;
-  (void)act_bytes;
+hipError_t emit_direct(const MatRow* mat, const uint32_t* perm, const uint64_t* offs, const uint8_t* kind_sorted, uint64_t n_most, EmitCtx ctx,
+                       char* out, uint64_t prefix_len, const Scalars* sc, hipStream_t st) {
+  if (n_most == 0) return hipSuccess;
   const size_t stage_lds = (size_t)KTJ_BLOCK * KTJ_STAGE_BLOCKS * 16u;
-  hipLaunchKernelGGL(k_emit_direct, dim3(grid_for(n_rows, KTJ_BLOCK)), dim3(KTJ_BLOCK), stage_lds, st, mat, perm, offs,
-                     kind_sorted, n_rows, ctx, out, prefix_len);
+  hipLaunchKernelGGL(k_emit_direct, dim3(grid_for(n_most, KTJ_BLOCK)), dim3(KTJ_BLOCK), stage_lds, st, mat, perm, offs,
+                     kind_sorted, ctx, out, prefix_len, sc);
   return KTJ_LAUNCH_CHECK();
 }
 

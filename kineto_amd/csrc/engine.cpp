@@ -165,8 +165,7 @@ struct HostCtl {
 #define KTJ_GUESS_BYTES_PER_ROW 480u /* the fixed text of an event with its flow event */
 #define KTJ_PINNED_SMALL_BYTES (256u << 10) /* header/footer text and small tables of a pass that may not allocate */
 
-enum { EV_START = 0, EV_DICT, EV_DECODE, EV_CONVERT, EV_JOIN, EV_SORT_A, EV_SORT_B, EV_SORT, EV_SIZE, EV_SCAN,
-       EV_EMIT_START, EV_EMIT, EV_COUNT };
+enum { EV_START = 0, EV_EMIT, EV_COUNT };
 
 }  // namespace
 
@@ -221,8 +220,8 @@ struct ktj_engine {
   DevBuf d_scalars, d_entries, d_name_blob, d_arg_blob;
   DevBuf c_ts, c_dur, c_corr, c_dev, c_res, c_meta, c_ext;
   DevBuf t_full, t_narrow, t_cpu, f_has_runtime, f_first, f_stream_src, f_pay, n_ext_src, n_kern_src, n_copy_src, n_pay, slot_f, slot_n, dev_link, dev_brief, sync_keys, sync_pos, sync_first;
-  DevBuf q_keys, q_stream, q_amb, dn_hash, dn_first, dn_dev, dn_key, dn_rank, range_parts;
-  DevBuf s_dev_k, s_dev_r, s_res_k, s_res_r;
+  DevBuf q_keys, q_stream, q_amb, dn_hash, dn_first, dn_dev, dn_key, dn_rank, dn_list;
+  DevBuf s_dev_k, s_dev_r, s_dev_l, s_res_k, s_res_r, s_res_l;
   DevBuf keys_a, keys_b, vals_a, vals_b, hist, scan_tmp;
   DevBuf mat, len, len_sorted, kind_sorted, offs, out, tile_start;
   void* pinned_small = nullptr; size_t pinned_small_cap = 0;
@@ -253,6 +252,11 @@ struct ktj_engine {
   bool hip_failed = false; /* a HIP call failed at some point: nothing of this engine is handed on */
 
   bool small_unfit = false;  /* these records need the launches of a large trace (Scalars::error of a small pass) */
+  bool stepwise = false;     /* these records need a pass in which the host looks at the plan of the sort (KTJ_DEVERR_CAREFUL) */
+  /* six passes sort the records of one capture: 2^38 ns, four and a half minutes, beside 9 bits of devices and
+   * rows; a pass more than needed costs its three launches, a pass too few the launches behind the sort */
+  uint32_t sort_passes = 6;  /* to be launched: what these records took in the pass before, where there was one */
+  void other_records() { small_unfit = stepwise = false; sort_passes = std::max(sort_passes, 6u); }
   bool small_last = false;   /* the last pass was a small one: it leaves no intermediate arrays for ktj_debug_fetch */
   bool no_small = false;     /* ktj_debug_fetch makes them */
   int64_t last_end_time = 0;
@@ -627,7 +631,10 @@ int synthesise_user_spans(ktj_engine* e, Columns c, const EmitCtx& ctx, Table t_
   NEED(e->synth_recs, recs.size() * sizeof(ktj_generic_rec) + 16);
   HIPCHK(hipMemcpyAsync(e->synth_recs.p, recs.data(), recs.size() * sizeof(ktj_generic_rec), hipMemcpyHostToDevice, st));
   HIPCHK(hipStreamSynchronize(st));
-  HIPCHK(decode_generic(e->synth_recs.as<ktj_generic_rec>(), recs.size(), c, first_row, sc, ctx, nullptr, st));
+  DecodeJob job;
+  memset(&job, 0, sizeof job);
+  job.g = e->synth_recs.as<ktj_generic_rec>(); job.ng = recs.size(); job.first = first_row;
+  HIPCHK(decode(job, c, ctx, sc, st));
   e->n_spans = recs.size();
   return KTJ_OK;
 }
@@ -959,7 +966,7 @@ int ktj_submit_records(ktj_engine* e, int rec_class, const void* packed, size_t 
   HIPCHK(hipSetDevice(e->device));
   { const int rc = append_from_host(e, set->owned, packed, n_records * rs); if (rc != KTJ_OK) return rc; }
   set->n += n_records;
-  e->small_unfit = false;
+  e->other_records();
   if (rec_class == KTJ_REC_GENERIC || rec_class == KTJ_REC_RUNTIME || rec_class == KTJ_REC_DEVICE) e->activities_begun = true;
   e->processed = false;
   return KTJ_OK;
@@ -998,7 +1005,7 @@ int ktj_submit_records_device(ktj_engine* e, int rec_class, const void* device_p
   if (set->owned.bytes != 0) return KTJ_ERR_STATE;
   set->external = n_records ? device_ptr : nullptr;
   set->n = n_records;
-  e->small_unfit = false;
+  e->other_records();
   if (n_records && (rec_class == KTJ_REC_GENERIC || rec_class == KTJ_REC_RUNTIME || rec_class == KTJ_REC_DEVICE)) e->activities_begun = true;
   e->processed = false;
   return KTJ_OK;
@@ -1175,6 +1182,18 @@ static int ensure_text(ktj_engine* e, size_t bytes) {
   e->pinned_small_dev = static_cast<char*>(d);
   return KTJ_OK;
 }
+/* header and footer into page-locked memory, for the kernels that put them in front of and behind the activities */
+static int document_text(ktj_engine* e, const std::string& prefix, const std::string& suffix, DocText* text) {
+  const size_t at_suffix = (prefix.size() + 15) & ~(size_t)15;
+  const int rc = ensure_text(e, at_suffix + suffix.size() + 64);
+  if (rc != KTJ_OK) return rc;
+  memcpy(e->pinned_small, prefix.data(), prefix.size());
+  memcpy(static_cast<char*>(e->pinned_small) + at_suffix, suffix.data(), suffix.size());
+  text->prefix = e->pinned_small_dev; text->n_prefix = prefix.size();
+  text->suffix = e->pinned_small_dev + at_suffix; text->n_suffix = suffix.size();
+  text->h_sc = &e->h_ctl_dev->scalars; text->h_total = &e->h_ctl_dev->act_bytes; text->h_end = &e->h_ctl_dev->end_clock;
+  return KTJ_OK;
+}
 static int short_output(ktj_engine* e) {
   e->last_error = "ktj_process_noalloc: the document has " + std::to_string(e->total_bytes) + " bytes and needs an output buffer of " +
                   std::to_string(e->total_bytes + 64);
@@ -1212,6 +1231,12 @@ static Columns columns_of(const ktj_engine* e) {
   c.dev = e->c_dev.as<int64_t>(); c.res = e->c_res.as<int64_t>(); c.meta = e->c_meta.as<uint32_t>();
   c.ext = e->c_ext.as<int32_t>();
   return c;
+}
+static hipError_t know_wall_clock(ktj_engine* e) {
+  return e->wall_clock_khz > 0 ? hipSuccess : hipDeviceGetAttribute(&e->wall_clock_khz, hipDeviceAttributeWallClockRate, e->device);
+}
+static float clock_ms(const ktj_engine* e, unsigned long long from, unsigned long long to) {
+  return to > from ? (float)((double)(to - from) / e->wall_clock_khz) : 0.0f;
 }
 static void count_stats(ktj_engine* e, uint64_t N) {
   const uint64_t ng = e->generic.n, nr = e->runtime.n, nd = e->devrows.n, nx = e->extcorr.n;
@@ -1266,10 +1291,8 @@ static int process_small(ktj_engine* e, int64_t end_time_ns, void* out_device, u
   const std::string prefix = e->txt_header + e->txt_before;
   std::string suffix = e->txt_after;
   append_trace_end(suffix, end_time_ns, e->base_time_ns, e->out_path, std::string());
-  const size_t at_suffix = (prefix.size() + 15) & ~(size_t)15;
-  { const int rc = ensure_text(e, at_suffix + suffix.size() + 64); if (rc != KTJ_OK) return rc; }
-  memcpy(e->pinned_small, prefix.data(), prefix.size());
-  memcpy(static_cast<char*>(e->pinned_small) + at_suffix, suffix.data(), suffix.size());
+  DocText text;
+  { const int rc = document_text(e, prefix, suffix, &text); if (rc != KTJ_OK) return rc; }
   if (out_device) e->out.borrow(out_device, out_cap);
   else HIPCHK(e->out.ensure(N * guess_per_row(e) + prefix.size() + suffix.size() + (64u << 10), false));
 
@@ -1287,11 +1310,7 @@ static int process_small(ktj_engine* e, int64_t end_time_ns, void* out_device, u
   a.api = ApiTable{e->d_cid_names.as<uint32_t>(), (uint32_t)e->cid_names.size(), e->d_flow_bits.as<uint32_t>(), e->malloc_cid};
   a.mat = e->mat.as<MatRow>(); a.len = e->len.as<uint32_t>(); a.perm = e->vals_a.as<uint32_t>();
   a.sc = sc;
-  SmallText text;
-  text.prefix = e->pinned_small_dev; text.n_prefix = prefix.size();
-  text.suffix = e->pinned_small_dev + at_suffix; text.n_suffix = suffix.size();
   text.out = e->out.as<char>(); text.out_cap = e->out.cap;
-  text.h_sc = &e->h_ctl_dev->scalars; text.h_total = &e->h_ctl_dev->act_bytes; text.h_end = &e->h_ctl_dev->end_clock;
   HIPCHK(small_pass(a, ns, st));
   HIPCHK(small_emit(a, text, st));
   HIPCHK(hipStreamSynchronize(st));
@@ -1316,11 +1335,11 @@ static int process_small(ktj_engine* e, int64_t end_time_ns, void* out_device, u
   }
   if (!out_device) e->most_needed = std::max(e->most_needed, pass_bytes + (size_t)e->total_bytes);
   count_stats(e, N);
-  if (e->wall_clock_khz <= 0) HIPCHK(hipDeviceGetAttribute(&e->wall_clock_khz, hipDeviceAttributeWallClockRate, e->device));
+  HIPCHK(know_wall_clock(e));
   /* by the device's clock: decode includes the dictionary, which is made beside it; size is what making
    * the joined rows takes beyond the sort that runs beside it */
   const unsigned long long* ck = e->scalars.clock;
-  auto ms = [&](unsigned long long from, unsigned long long to) { return to > from ? (float)((double)(to - from) / e->wall_clock_khz) : 0.0f; };
+  auto ms = [&](unsigned long long from, unsigned long long to) { return clock_ms(e, from, to); };
   ktj_stats& s = e->stats;
   if (!(e->flags & KTJ_CREATE_NO_STAGE_TIMES)) {
     s.stage_ms[KTJ_STAGE_DECODE] = ms(ck[0], ck[1]);
@@ -1391,9 +1410,10 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
   if (!e->small_unfit && !e->no_small && nu == 0 && n_coll == 0 && small_fits(ng, nr, nd, nx) && !sort_packed_passes_forced() &&
       !(e->flags & (KTJ_CREATE_TILE_EMIT | KTJ_CREATE_HASH_JOIN | KTJ_CREATE_PAIR_SORT))) {
     bool done = false;
+    const size_t tables = e->arena_used; /* of the scratch array */
     const int rc = process_small(e, end_time_ns, out_device, out_cap, &done);
     if (rc != KTJ_OK || done) return rc;
-    e->arena_used = 0;
+    e->arena_used = tables;
   }
 
   /* working memory */
@@ -1426,16 +1446,15 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
   NEED(e->q_amb, (KTJ_QUEUE_CAP + 1ull) * 4);
   NEED(e->dn_hash, (KTJ_DENSE_CAP + 1ull) * 8); NEED(e->dn_first, (KTJ_DENSE_CAP + 1ull) * 4);
   NEED(e->dn_dev, (KTJ_DENSE_CAP + 1ull) * 4); NEED(e->dn_key, (KTJ_DENSE_CAP + 1ull) * 8);
-  NEED(e->dn_rank, (KTJ_DENSE_CAP + 1ull) * 4);
-  NEED(e->s_dev_k, (KTJ_SET_CAP + 1ull) * 8); NEED(e->s_dev_r, (KTJ_SET_CAP + 1ull) * 4);
-  NEED(e->s_res_k, (KTJ_SET_CAP + 1ull) * 8); NEED(e->s_res_r, (KTJ_SET_CAP + 1ull) * 4);
+  NEED(e->dn_rank, (KTJ_DENSE_CAP + 1ull) * 4); NEED(e->dn_list, KTJ_MAX_STREAM_PAIRS * 4ull);
+  NEED(e->s_dev_k, (KTJ_SET_CAP + 1ull) * 8); NEED(e->s_dev_r, (KTJ_SET_CAP + 1ull) * 4); NEED(e->s_dev_l, KTJ_SET_MAX * 4ull);
+  NEED(e->s_res_k, (KTJ_SET_CAP + 1ull) * 8); NEED(e->s_res_r, (KTJ_SET_CAP + 1ull) * 4); NEED(e->s_res_l, KTJ_SET_MAX * 4ull);
   NEED(e->keys_a, Na * 8); NEED(e->keys_b, Na * 8);
   NEED(e->vals_a, Na * 4); NEED(e->vals_b, Na * 4);
-  NEED(e->range_parts, (decode_blocks(ng) + 2 * decode_blocks(nr) + decode_blocks(nd) + 1) * sizeof(KeyRange));
   NEED(e->hist, radix_tmp_elems(Na) * 4);
   {
     uint64_t m = scan_tmp_elems(radix_tmp_elems(Na));
-    const uint64_t m2 = scan_tmp_elems(Na);
+    const uint64_t m2 = offsets_tmp_elems(Na);
     if (m2 > m) m = m2;
     NEED(e->scan_tmp, m * 8);
   }
@@ -1449,19 +1468,16 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
   }
 
   Scalars* sc = e->d_scalars.as<Scalars>();
+  const bool stage_times = !(e->flags & KTJ_CREATE_NO_STAGE_TIMES);
   const Columns c = columns_of(e);
   const ktj_generic_rec* g_recs = static_cast<const ktj_generic_rec*>(e->generic.ptr());
   const ktj_runtime_rec* r_recs = static_cast<const ktj_runtime_rec*>(e->runtime.ptr());
   const ktj_device_rec* d_recs = static_cast<const ktj_device_rec*>(e->devrows.ptr());
   const ktj_extcorr_rec* x_recs = static_cast<const ktj_extcorr_rec*>(e->extcorr.ptr());
 
-  /* an event on the stream costs the GPU a microsecond or two between two kernels: a trace of a few
-   * records can do without the ten that separate the stages (KTJ_CREATE_NO_STAGE_TIMES) */
-  const bool stage_times = !(e->flags & KTJ_CREATE_NO_STAGE_TIMES);
   HIPCHK(hipEventRecord(e->ev[EV_START], st));
-  HIPCHK(init_scalars(sc, st));
 
-  /* ---- stage 0: dictionary ---- */
+  /* ---- the start, stage 0: dictionary ---- */
   const EmitCtx ctx = emit_context(e, n_coll);
   uint32_t* cpu_row = nullptr; /* last CPU op per id: only where something is read from that op */
   if (n_coll || max_spans) {
@@ -1470,21 +1486,32 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
     HIPCHK(fill_u32(cpu_row, 0, cap_cpu + 1ull, st));
   }
   if (n_coll) NEED(e->d_coll_first, 2ull * n_coll * 4);
-  HIPCHK(dict_views(e->str_blob.buf.as<char>(), e->str_off.buf.as<uint64_t>(), ns, e->d_entries.as<DictEntry>(), e->d_name_blob.as<char>(),
-                    e->d_arg_blob.as<char>(), st));
-  if (stage_times) HIPCHK(hipEventRecord(e->ev[EV_DICT], st));
+  StreamTables stt{e->q_keys.as<uint64_t>(), e->q_stream.as<uint64_t>(), e->q_amb.as<uint32_t>(), e->dn_hash.as<uint64_t>(),
+                   e->dn_first.as<uint32_t>(), e->dn_dev.as<int32_t>(), e->dn_key.as<uint64_t>(), e->dn_rank.as<uint32_t>(),
+                   e->dn_list.as<uint32_t>()};
+  SortSets sets{e->s_dev_k.as<uint64_t>(), e->s_dev_r.as<uint32_t>(), e->s_res_k.as<uint64_t>(), e->s_res_r.as<uint32_t>(),
+                e->s_dev_l.as<uint32_t>(), e->s_res_l.as<uint32_t>()};
+  FillJobs fills;
+  fills.count = 0;
+  fills.add(stt.q_keys, KTJ_EMPTY_KEY, KTJ_QUEUE_CAP + 1ull, 8); fills.add(stt.q_stream, 0, KTJ_QUEUE_CAP + 1ull, 8);
+  fills.add(stt.q_amb, 0, KTJ_QUEUE_CAP + 1ull, 4);
+  fills.add(stt.d_hash, KTJ_EMPTY_KEY, KTJ_DENSE_CAP + 1ull, 8); fills.add(stt.d_first, 0xFFFFFFFFu, KTJ_DENSE_CAP + 1ull, 4);
+  fills.add(stt.d_rank, 0, KTJ_DENSE_CAP + 1ull, 4);
+  fills.add(sets.dev_keys, KTJ_EMPTY_KEY, KTJ_SET_CAP + 1ull, 8); fills.add(sets.res_keys, KTJ_EMPTY_KEY, KTJ_SET_CAP + 1ull, 8);
+  HIPCHK(begin_pass(sc, fills, e->str_blob.buf.as<char>(), e->str_off.buf.as<uint64_t>(), ns, e->d_entries.as<DictEntry>(),
+                    e->d_name_blob.as<char>(), e->d_arg_blob.as<char>(), st));
 
-  /* ---- stage 1: decode ---- */
-  KeyRange* parts = e->range_parts.as<KeyRange>(); /* [generic | runtime | runtime narrowed | device] */
-  /* stage 2a, clock conversion and window filter, happens inside the runtime and device decode */
-  const ClockDev clk = clock_of(e);
-  HIPCHK(decode_generic(g_recs, ng, c, 0, sc, ctx, parts, st));
-  HIPCHK(decode_runtime(r_recs, nr, c, ng, parts + decode_blocks(ng), parts + decode_blocks(ng) + decode_blocks(nr), clk,
-                        e->win_start, e->win_end, sc, st));
-  HIPCHK(decode_device(d_recs, nd, c, ng + nr, e->dev_brief.as<DevBrief>(), parts + decode_blocks(ng) + 2 * decode_blocks(nr), clk,
-                       e->win_start, e->win_end, sc, st));
-  if (stage_times) HIPCHK(hipEventRecord(e->ev[EV_DECODE], st));
-  if (stage_times) HIPCHK(hipEventRecord(e->ev[EV_CONVERT], st));
+  /* ---- stage 1: decode; stage 2a, clock conversion and window filter, happens inside ---- */
+  {
+    DecodeJob job;
+    memset(&job, 0, sizeof job);
+    job.g = g_recs; job.r = r_recs; job.d = d_recs; job.x = x_recs;
+    job.ng = ng; job.nr = nr; job.nd = nd; job.nx = nx;
+    job.whole_pass = true;
+    job.brief = e->dev_brief.as<DevBrief>();
+    job.clk = clock_of(e); job.win_start = e->win_start; job.win_end = e->win_end;
+    HIPCHK(decode(job, c, ctx, sc, st));
+  }
 
   /* ---- stage 2b: joins ---- */
   Table tf{e->t_full.as<uint64_t>(), cap_full - 1, 0u, &sc->plan.ctl[KTJ_TBL_FULL]};
@@ -1492,21 +1519,7 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
   Table t_cpu{e->t_cpu.as<uint64_t>(), cap_cpu - 1, 1u, &sc->plan.ctl[KTJ_TBL_CPU]};
   FullCols fc{e->f_has_runtime.as<uint32_t>(), e->f_first.as<uint32_t>(), e->f_stream_src.as<uint32_t>(), e->f_pay.as<FullPay>()};
   NarrowCols nc{e->n_ext_src.as<uint32_t>(), e->n_kern_src.as<uint32_t>(), e->n_copy_src.as<uint32_t>(), e->n_pay.as<NarrowPay>()};
-  HIPCHK(plan_tables(parts, ng, nr, nd, x_recs, nx, cap_full, cap_narrow, cap_cpu, (e->flags & KTJ_CREATE_HASH_JOIN) != 0, sc, st));
-  HIPCHK(clear_tables(tf, fc, tn, nc, t_cpu, st));
-  StreamTables stt{e->q_keys.as<uint64_t>(), e->q_stream.as<uint64_t>(), e->q_amb.as<uint32_t>(), e->dn_hash.as<uint64_t>(),
-                   e->dn_first.as<uint32_t>(), e->dn_dev.as<int32_t>(), e->dn_key.as<uint64_t>(), e->dn_rank.as<uint32_t>()};
-  SortSets sets{e->s_dev_k.as<uint64_t>(), e->s_dev_r.as<uint32_t>(), e->s_res_k.as<uint64_t>(), e->s_res_r.as<uint32_t>()};
-  {
-    FillJobs f;
-    f.count = 0;
-    f.add(stt.q_keys, KTJ_EMPTY_KEY, KTJ_QUEUE_CAP + 1ull, 8); f.add(stt.q_stream, 0, KTJ_QUEUE_CAP + 1ull, 8);
-    f.add(stt.q_amb, 0, KTJ_QUEUE_CAP + 1ull, 4);
-    f.add(stt.d_hash, KTJ_EMPTY_KEY, KTJ_DENSE_CAP + 1ull, 8); f.add(stt.d_first, 0xFFFFFFFFu, KTJ_DENSE_CAP + 1ull, 4);
-    f.add(stt.d_rank, 0, KTJ_DENSE_CAP + 1ull, 4);
-    f.add(sets.dev_keys, KTJ_EMPTY_KEY, KTJ_SET_CAP + 1ull, 8); f.add(sets.res_keys, KTJ_EMPTY_KEY, KTJ_SET_CAP + 1ull, 8);
-    HIPCHK(fill_many(f, st));
-  }
+  HIPCHK(plan_tables(tf, fc, tn, nc, t_cpu, (e->flags & KTJ_CREATE_HASH_JOIN) != 0, sc, st));
   ApiTable api{e->d_cid_names.as<uint32_t>(), (uint32_t)e->cid_names.size(), e->d_flow_bits.as<uint32_t>(), e->malloc_cid};
   MatRow* mat = e->mat.as<MatRow>();
   HIPCHK(build_cpu_ids(g_recs, ng, t_cpu, cpu_row, sc, st));
@@ -1515,26 +1528,70 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
                            e->len.as<uint32_t>(), sc, st));
   HIPCHK(republish_runtime_rows(r_recs, nr, c, ng, fc, nc, e->slot_f.as<uint32_t>(), e->slot_n.as<uint32_t>(), sc, st));
   HIPCHK(link_device_rows(nd, c, ng + nr, tf, fc, tn, nc, e->dev_link.as<DevLink>(), sc, st));
-  HIPCHK(backfill_streams(e->dev_brief.as<DevBrief>(), nd, c, ng + nr, stt, sc, st));
+  HIPCHK(backfill_streams(e->dev_brief.as<DevBrief>(), nd, c, ng + nr, tf, fc, e->dev_link.as<DevLink>(), stt, sc, st));
   if (max_spans) {
     const int rc = synthesise_user_spans(e, c, ctx, t_cpu, cpu_row, sc, N);
     if (rc != KTJ_OK) return rc;
     N += e->n_spans;
     e->N = N;
   }
-  if (stage_times) HIPCHK(hipEventRecord(e->ev[EV_JOIN], st));
 
   /* ---- stage 3: canonical order ---- */
-  HIPCHK(collect_distinct(c, N, sets, sc, st));
-  HIPCHK(rank_distinct(sets, sc, st));
-  if (stage_times) HIPCHK(hipEventRecord(e->ev[EV_SORT_A], st));
-  HIPCHK(publish(sc, nullptr, nullptr, 0, &e->h_ctl_dev->scalars, nullptr, nullptr, st));
+  /* The rest of the pass is put into the stream in one go where its launches can be told beforehand:
+   * the widths of the sort's keys stay on the device, the kernels behind it read what they need from
+   * there, and the host waits once, for the finished document.  (With a wait before the sort and one
+   * before emit the GPU stood still for 25 us each: 30 000 records took 346 us.)  It cannot be told with
+   * collective entries (the footer names those in use) and synthesised spans, and what else only the
+   * device sees, it flags: more sort passes than launched, keys too wide for the one-word sort, CUDA_SYNC
+   * activities, too many distinct values.  Such records take the stepwise rest of the pass from here on. */
+  bool straight = n_coll == 0 && max_spans == 0 && !e->stepwise && !(e->flags & KTJ_CREATE_TILE_EMIT) && e->sort_mode != 1;
+  HIPCHK(collect_distinct(c, N, sets, sc, straight, st));
   if (!out_device && !e->noalloc && e->out.cap == 0) {
     /* An engine's first pass has no document buffer yet, and how long the document is comes out of
      * the scan.  A first guess is allocated here, while the GPU is busy with the join.  If that turns out too
      * small (or cannot be had) the buffer is allocated where its size is known, as in later passes. */
-    if (e->out.ensure(N * guess_per_row(e) + (1u << 20), false) != hipSuccess) (void)hipGetLastError();
+    if (e->out.ensure(N * guess_per_row(e) + (1u << 20), false) != hipSuccess) { (void)hipGetLastError(); straight = false; }
   }
+  bool emitted = false;
+  if (straight) {
+    const std::string prefix = e->txt_header + e->txt_before;
+    std::string suffix = e->txt_after;
+    append_trace_end(suffix, end_time_ns, e->base_time_ns, e->out_path, std::string());
+    DocText text;
+    { const int rc = document_text(e, prefix, suffix, &text); if (rc != KTJ_OK) return rc; }
+    if (out_device) e->out.borrow(out_device, out_cap);
+    e->perm = e->vals_a.as<uint32_t>();
+    e->sorted_keys = nullptr;
+    HIPCHK(sort_packed(c, N, sets, sc, e->sort_passes, e->keys_a.as<uint64_t>(), e->keys_b.as<uint64_t>(), e->perm, e->hist.as<uint32_t>(), st));
+    HIPCHK(mat_rows(g_recs, ng, 0, nullptr, d_recs, nd, c, ng + nr, e->dev_link.as<DevLink>(), ctx, mat, e->len.as<uint32_t>(), sc, st));
+    for (;;) {
+      text.out = e->out.as<char>(); text.out_cap = e->out.cap;
+      HIPCHK(gather_offsets(e->perm, e->len.as<uint32_t>(), N, e->len_sorted.as<uint32_t>(), e->kind_sorted.as<uint8_t>(),
+                            e->scan_tmp.as<uint64_t>(), e->offs.as<uint64_t>(), sc, text, st));
+      HIPCHK(emit_direct(mat, e->perm, e->offs.as<uint64_t>(), e->kind_sorted.as<uint8_t>(), N, ctx, e->out.as<char>(), prefix.size(), sc, st));
+      HIPCHK(hipEventRecord(e->ev[EV_EMIT], st));
+      HIPCHK(hipStreamSynchronize(st));
+      e->scalars = e->h_ctl->scalars;
+      if (e->scalars.error) break;
+      e->act_bytes = e->h_ctl->act_bytes;
+      e->prefix_len = prefix.size();
+      e->total_bytes = prefix.size() + e->act_bytes + suffix.size();
+      emitted = e->total_bytes + 64 <= text.out_cap;
+      if (emitted) break;
+      if (out_device) return short_output(e); /* nothing has been written */
+      HIPCHK(e->out.ensure(e->total_bytes + 64));
+    }
+    if (emitted) e->sort_passes = sort_packed_passes(e->scalars.sort.key_bits);
+    else if (e->scalars.error & ~(KTJ_DEVERR_CAREFUL | KTJ_DEVERR_DISTINCT_DEVICES | KTJ_DEVERR_DISTINCT_RESOURCES)) {
+      e->last_error = limit_text(e->scalars.error);
+      return KTJ_ERR_LIMIT;
+    } else {
+      e->stepwise = true;
+      HIPCHK(clear_error_bits(sc, KTJ_DEVERR_CAREFUL, st));
+    }
+  }
+  if (!emitted) { /* the stepwise rest */
+  HIPCHK(publish(sc, nullptr, nullptr, 0, &e->h_ctl_dev->scalars, nullptr, nullptr, st));
   HIPCHK(hipStreamSynchronize(st));
   e->scalars = e->h_ctl->scalars;
   const unsigned distinct_overflow = e->scalars.error & (KTJ_DEVERR_DISTINCT_DEVICES | KTJ_DEVERR_DISTINCT_RESOURCES);
@@ -1550,7 +1607,6 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
     key_bits = ts_bits + res_bits + dev_bits;
     rank_bits = res_bits + dev_bits;
   }
-  if (stage_times) HIPCHK(hipEventRecord(e->ev[EV_SORT_B], st));
   {
     uint64_t* ka = e->keys_a.as<uint64_t>(); uint32_t* va = e->vals_a.as<uint32_t>();
     uint64_t* kb = e->keys_b.as<uint64_t>(); uint32_t* vb = e->vals_b.as<uint32_t>();
@@ -1574,7 +1630,7 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
       if (rc == KTJ_OK) rc = sort_again([&](const uint32_t* o, uint64_t* k, uint32_t* v) { return make_column_keys(c.dev, c.meta, o, N, 1, k, v, st); }, 1);
       if (rc != KTJ_OK) return rc;
     } else if (key_bits <= 62 && e->sort_mode != 1 && sort_packed_fits(N, key_bits)) {
-      HIPCHK(sort_packed(c, N, sets, sc, ts_bits, res_bits, key_bits, ka, kb, va, hist, scan_tmp, st));
+      HIPCHK(sort_packed(c, N, sets, sc, sort_packed_passes(key_bits), ka, kb, va, hist, st));
       e->perm = va;
       e->sorted_keys = nullptr;
     } else if (key_bits <= 62) {
@@ -1590,7 +1646,6 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
       if (rc != KTJ_OK) return rc;
     }
   }
-  if (stage_times) HIPCHK(hipEventRecord(e->ev[EV_SORT], st));
 
   /* ---- stage 4a: joined rows + lengths ---- */
   const uint32_t* sync_first = nullptr;
@@ -1601,17 +1656,14 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
                              e->sync_pos.as<uint32_t>(), e->sync_first.as<uint32_t>(), sc, st));
     sync_first = e->sync_first.as<uint32_t>();
   }
-  HIPCHK(mat_generic_rows(g_recs, ng, 0, ctx, sync_first, mat, e->len.as<uint32_t>(), sc, st));
-  HIPCHK(mat_generic_rows(e->synth_recs.as<ktj_generic_rec>(), e->n_spans, ng + nr + nd, ctx, nullptr, mat, e->len.as<uint32_t>(),
-                          sc, st));
-  HIPCHK(mat_device_rows(d_recs, nd, c, ng + nr, e->dev_link.as<DevLink>(), ctx, mat, e->len.as<uint32_t>(), sc, st));
-  HIPCHK(gather_len(e->perm, e->len.as<uint32_t>(), N, e->len_sorted.as<uint32_t>(), e->kind_sorted.as<uint8_t>(), st));
+  HIPCHK(mat_rows(g_recs, ng, 0, sync_first, d_recs, nd, c, ng + nr, e->dev_link.as<DevLink>(), ctx, mat, e->len.as<uint32_t>(), sc, st));
+  HIPCHK(mat_rows(e->synth_recs.as<ktj_generic_rec>(), e->n_spans, ng + nr + nd, nullptr, nullptr, 0, c, 0, nullptr, ctx, mat,
+                  e->len.as<uint32_t>(), sc, st));
   if (n_coll) HIPCHK(collective_first(mat, e->perm, e->scalars.n_valid, n_coll, e->d_coll_first.as<uint32_t>(), st));
-  if (stage_times) HIPCHK(hipEventRecord(e->ev[EV_SIZE], st));
 
   /* ---- scan ---- */
-  HIPCHK(scan_u32_to_u64(e->len_sorted.as<uint32_t>(), e->offs.as<uint64_t>(), N, e->scan_tmp.as<uint64_t>(), st));
-  if (stage_times) HIPCHK(hipEventRecord(e->ev[EV_SCAN], st));
+  HIPCHK(gather_offsets(e->perm, e->len.as<uint32_t>(), N, e->len_sorted.as<uint32_t>(), e->kind_sorted.as<uint8_t>(),
+                        e->scan_tmp.as<uint64_t>(), e->offs.as<uint64_t>(), sc, DocText{}, st));
   uint64_t act_bytes = 0;
   e->coll_first.assign(2ull * n_coll, 0xFFFFFFFFu);
   const bool list_fits = 2ull * n_coll * 4 <= e->pinned_small_cap; /* through the engine's pinned buffer when it fits */
@@ -1666,17 +1718,17 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
   }
   const uint32_t tile = emit_tile_bytes(act_bytes, e->scalars.n_valid);
   NEED(e->tile_start, (emit_tile_count(e->prefix_len, act_bytes, tile) + 2) * 4);
-  if (stage_times) HIPCHK(hipEventRecord(e->ev[EV_EMIT_START], st));
   {
     if (e->flags & KTJ_CREATE_TILE_EMIT)
       HIPCHK(emit(mat, e->perm, e->offs.as<uint64_t>(), N, ctx, e->out.as<char>(), e->prefix_len, act_bytes, tile,
                   e->tile_start.as<uint32_t>(), st));
     else
-      HIPCHK(emit_direct(mat, e->perm, e->offs.as<uint64_t>(), e->kind_sorted.as<uint8_t>(), e->scalars.n_valid, act_bytes, ctx,
-                         e->out.as<char>(), e->prefix_len, st));
+      HIPCHK(emit_direct(mat, e->perm, e->offs.as<uint64_t>(), e->kind_sorted.as<uint8_t>(), e->scalars.n_valid, ctx, e->out.as<char>(),
+                         e->prefix_len, sc, st));
   }
   HIPCHK(hipEventRecord(e->ev[EV_EMIT], st));
   HIPCHK(hipStreamSynchronize(st));
+  } /* the stepwise rest */
   e->stage_small_used = 0; /* the stream has passed every upload: ring and slots are free from their beginning */
   e->stage_big_used = 0;
   if (!out_device) e->most_needed = std::max(e->most_needed, pass_bytes + (size_t)e->total_bytes);
@@ -1684,25 +1736,24 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
   /* ---- statistics ---- */
   count_stats(e, N);
   ktj_stats& s = e->stats;
-  /* stage time = elapsed between the events that bracket it; the two host read-backs (after the
-   * distinct-value ranking and after the scan) are excluded from the per-stage figures but are
-   * part of KTJ_STAGE_TOTAL_GPU */
-  struct { int stage, from, to; } spans[] = {
-      {KTJ_STAGE_DICT, EV_START, EV_DICT},       {KTJ_STAGE_DECODE, EV_DICT, EV_DECODE},
-      {KTJ_STAGE_DECODE, EV_DECODE, EV_CONVERT}, {KTJ_STAGE_JOIN, EV_CONVERT, EV_JOIN},
-      {KTJ_STAGE_SORT, EV_JOIN, EV_SORT_A},      {KTJ_STAGE_SORT, EV_SORT_B, EV_SORT},
-      {KTJ_STAGE_SIZE, EV_SORT, EV_SIZE},        {KTJ_STAGE_SCAN, EV_SIZE, EV_SCAN},
-      {KTJ_STAGE_EMIT, EV_EMIT_START, EV_EMIT}};
-  for (const auto& sp : spans) {
-    if (!stage_times) break;
-    float ms = 0;
-    HIPCHK(hipEventElapsedTime(&ms, e->ev[sp.from], e->ev[sp.to]));
-    s.stage_ms[sp.stage] += ms;
-  }
+  /* A stage begins with its first kernel's first workgroup, by the device's clock (an event between two
+   * kernels leaves the GPU idle for 5 us, on a trace of some thousand records a tenth of the pass); a
+   * stage that launched nothing has no time.  Where the host looks at the plan of the sort its wait is part
+   * of the sort.  The whole pass is taken by events; emit, the last stage, is what the others leave of it. */
   {
     float ms = 0;
     HIPCHK(hipEventElapsedTime(&ms, e->ev[EV_START], e->ev[EV_EMIT]));
     s.stage_ms[KTJ_STAGE_TOTAL_GPU] = ms;
+  }
+  if (stage_times) {
+    HIPCHK(know_wall_clock(e));
+    const unsigned long long* ck = e->scalars.clock;
+    const int stages[] = {KTJ_STAGE_DICT, KTJ_STAGE_DECODE, KTJ_STAGE_JOIN, KTJ_STAGE_SORT, KTJ_STAGE_SIZE, KTJ_STAGE_SCAN};
+    static_assert(sizeof stages / sizeof stages[0] == KTJ_CLOCK_COUNT - 1, "a stage between every two of the clock's points");
+    unsigned long long end = ck[KTJ_CLOCK_EMIT];
+    for (int k = KTJ_CLOCK_COUNT - 2; k >= 0; --k)
+      if (ck[k]) { s.stage_ms[stages[k]] = clock_ms(e, ck[k], end); end = ck[k]; }
+    s.stage_ms[KTJ_STAGE_EMIT] = std::max(0.0f, s.stage_ms[KTJ_STAGE_TOTAL_GPU] - clock_ms(e, ck[KTJ_CLOCK_BEGIN], ck[KTJ_CLOCK_EMIT]));
   }
   e->processed = true;
   return KTJ_OK;

@@ -34,6 +34,7 @@ __device__ __forceinline__ uint32_t wave_sum_u32(uint32_t v) {
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
   return v;
 }
+__device__ __forceinline__ void stage_clock(Scalars* sc, int k) { sc->clock[k] = wall_clock64(); }
 __device__ __forceinline__ void flag_error(Scalars* sc, unsigned bit) { atomicOr(&sc->error, bit); }
 
 /* grid-stride kernels: enough workgroups to fill 256 CUs several times over */

@@ -117,6 +117,11 @@ struct Columns {
 #define KTJ_COUNTER_SHARDS 64u
 #endif
 #define KTJ_PART_SLOTS 32u
+struct SortPlan { unsigned int ts_bits, res_bits, key_bits; }; /* of the composite key, without the bit for dropped rows */
+/* wall clock (wall_clock64) at the points of a pass: its start and the start of each stage; the runs of
+ * small.hip name their own */
+enum { KTJ_CLOCK_BEGIN = 0, KTJ_CLOCK_DECODE, KTJ_CLOCK_JOIN, KTJ_CLOCK_SORT, KTJ_CLOCK_SIZE, KTJ_CLOCK_SCAN, KTJ_CLOCK_EMIT, KTJ_CLOCK_COUNT };
+enum { KTJ_DONE_DENSE = 0, KTJ_DONE_COLLECT, KTJ_DONE_COUNT };
 struct Scalars {
   unsigned long long ts_min_biased;   /* min over valid rows of ts ^ 2^63 */
   unsigned long long ts_max_biased;
@@ -139,8 +144,10 @@ struct Scalars {
   unsigned int n_sync_rows;           /* distinct (device, row) pairs of Stream Sync activities */
   unsigned int n_plain;               /* small traces: activities that small_emit leaves to small_plain */
   unsigned int ext_ids_repeat;        /* two external-correlation records share a correlation id */
-  unsigned long long clock[6];        /* small traces: wall clock (wall_clock64) at the start of the pass, behind decode,
-                                         behind the joins, at the start and end of the sort, at the start of emit */
+  unsigned long long emit_rows;       /* activities to format: n_valid, or none where the pass cannot end so */
+  unsigned long long clock[KTJ_CLOCK_COUNT];
+  SortPlan sort;
+  unsigned int done[KTJ_DONE_COUNT];  /* workgroups of a launch that have finished (last_workgroup) */
   unsigned int part_done[KTJ_PART_SLOTS]; /* copy_parts: workgroups that have finished the part in a slot */
   alignas(256) JoinPlan plan;         /* key ranges and modes of the join tables: read by every row of the join
                                          kernels, so kept off the cache lines that take the counters' atomics */
@@ -150,6 +157,8 @@ struct Scalars {
    * join more than its table lookups.  k_publish sums the copies into the fields above, which nothing
    * on the device reads; it hands the host everything in front of this array. */
   alignas(128) unsigned long long shard[KTJ_COUNTER_SHARDS][16];
+  alignas(128) unsigned long long range_shard[KTJ_COUNTER_SHARDS][16]; /* likewise the key ranges of the join tables: [2t] smallest,
+                                                                           [2t + 1] largest key of table t */
 };
 enum { KTJ_CNT_OUT_OF_RANGE = 0, KTJ_CNT_OUT_OF_ORDER, KTJ_CNT_FLOW, KTJ_CNT_LINKED, KTJ_CNT_BLANK_NAMES, KTJ_CNT_VALID,
        KTJ_CNT_SYNC_TYPED, KTJ_CNT_COUNT };
@@ -163,6 +172,7 @@ enum { KTJ_CNT_OUT_OF_RANGE = 0, KTJ_CNT_OUT_OF_ORDER, KTJ_CNT_FLOW, KTJ_CNT_LIN
 #define KTJ_DEVERR_QUEUES 64u             /* more than KTJ_MAX_QUEUES hardware queues */
 #define KTJ_DEVERR_SYNC_ROWS 128u         /* more than KTJ_MAX_SYNC_ROWS (device, row) pairs of Stream Sync events */
 
+#define KTJ_DEVERR_CAREFUL 512u           /* the pass went by assumptions that do not hold; no error reaches the caller */
 #define KTJ_DEVERR_SMALL_UNFIT 256u       /* a small trace that needs the launches of a large one; no error reaches the caller */
 
 #define KTJ_SET_CAP 16384u     /* slots of the distinct-value sets; KTJ_SET_MAX values get a rank */
@@ -212,8 +222,6 @@ struct FillJobs {          /* up to 12 fills in one launch */
   uint32_t count;
   void add(void* ptr, uint64_t v, uint64_t elems, uint32_t width) { p[count] = ptr; value[count] = v; n[count] = elems; bytes_each[count] = width; ++count; }
 };
-hipError_t fill_many(const FillJobs& jobs, hipStream_t st);
-hipError_t init_scalars(Scalars* s, hipStream_t st);
 hipError_t copy_reference(const void* src, void* dst, uint64_t bytes, hipStream_t st);
 
 /* Working memory for callers that cannot allocate: a static array in device memory, one copy per
@@ -221,36 +229,31 @@ hipError_t copy_reference(const void* src, void* dst, uint64_t bytes, hipStream_
  * the current device); the address is looked up once per device and kept. */
 hipError_t scratch_address(int device, void** ptr, size_t* bytes);
 
-/* exclusive scans; tmp must hold scan_tmp_elems(n) uint64 values */
+/* exclusive scan in place; tmp must hold scan_tmp_elems(n) uint64 values */
 uint64_t scan_tmp_elems(uint64_t n);
-hipError_t scan_u32_to_u64(const uint32_t* in, uint64_t* out /* n+1 */, uint64_t n, uint64_t* tmp, hipStream_t st);
 hipError_t scan_u32_inplace(uint32_t* data, uint64_t n, uint64_t* tmp, hipStream_t st);
 
-/* ---- stage 0: dictionary ---- */
-/* entries: n; name_blob: 2 * blob bytes + KTJ_DICT_ROOM * (n + 1), arg_blob: blob bytes + KTJ_DICT_ROOM * (n + 1) */
-hipError_t dict_views(const char* blob, const uint64_t* off, uint32_t n, DictEntry* entries, char* name_blob, char* arg_blob,
-                      hipStream_t st);
+/* ---- start of a pass: scalars, fills, and stage 0, the dictionary's views ----
+ * entries: n_strings; name_blob: 2 * blob bytes + KTJ_DICT_ROOM * (n + 1), arg_blob: blob bytes + KTJ_DICT_ROOM * (n + 1) */
+hipError_t begin_pass(Scalars* s, const FillJobs& jobs, const char* blob, const uint64_t* off, uint32_t n_strings, DictEntry* entries,
+                      char* name_blob, char* arg_blob, hipStream_t st);
 
-/* ---- stage 1: decode ---- */
-/* id_range / narrow_range: one KeyRange per workgroup (decode_blocks(n) entries), smallest and
- * largest id of the workgroup's records; id_range of decode_generic may be null */
-uint64_t decode_blocks(uint64_t n);
-hipError_t decode_generic(const ktj_generic_rec* r, uint64_t n, Columns c, uint64_t first, Scalars* sc, EmitCtx ctx,
-                          KeyRange* id_range, hipStream_t st);
-/* the runtime and device kernels also convert the clock and apply the capture window */
-hipError_t decode_runtime(const ktj_runtime_rec* r, uint64_t n, Columns c, uint64_t first, KeyRange* id_range,
-                          KeyRange* narrow_range, ClockDev clk, int64_t win_start, int64_t win_end, Scalars* sc, hipStream_t st);
-hipError_t decode_device(const ktj_device_rec* r, uint64_t n, Columns c, uint64_t first, DevBrief* brief, KeyRange* id_range,
-                         ClockDev clk, int64_t win_start, int64_t win_end, Scalars* sc, hipStream_t st);
+/* ---- stage 1: decode, with the clock conversion and the capture window (stage 2a) ---- */
+struct DecodeJob {
+  const ktj_generic_rec* g; const ktj_runtime_rec* r; const ktj_device_rec* d; const ktj_extcorr_rec* x;
+  uint64_t ng, nr, nd, nx;   /* x: only their correlation ids' range */
+  uint64_t first;            /* arrival index of the first generic record; runtime and device rows follow ng records */
+  bool whole_pass;           /* false: generic records made during the pass, which are in no table */
+  DevBrief* brief;
+  ClockDev clk;
+  int64_t win_start, win_end;
+  uint32_t gb, rb, db;       /* set by decode() */
+};
+hipError_t decode(DecodeJob job, Columns c, EmitCtx ctx, Scalars* sc, hipStream_t st);
 
 /* ---- stage 2b: joins ---- */
-/* key ranges of the three tables, then their modes (direct unless force_hash or the span is too wide).
- * parts: the decode kernels' per-workgroup ranges, laid out as [generic ids | runtime ids | runtime ids
- * narrowed | device ids] with decode_blocks() entries each */
-hipError_t plan_tables(const KeyRange* parts, uint64_t n_generic, uint64_t n_runtime, uint64_t n_device,
-                       const ktj_extcorr_rec* e, uint64_t n_ext, uint32_t cap_full, uint32_t cap_narrow, uint32_t cap_cpu,
-                       bool force_hash, Scalars* sc, hipStream_t st);
-hipError_t clear_tables(Table tf, FullCols fc, Table tn, NarrowCols nc, Table cpu, hipStream_t st);
+/* the tables' modes (direct unless force_hash or the span of their keys is too wide), and all of them cleared */
+hipError_t plan_tables(Table tf, FullCols fc, Table tn, NarrowCols nc, Table cpu, bool force_hash, Scalars* sc, hipStream_t st);
 hipError_t build_cpu_ids(const ktj_generic_rec* g, uint64_t n, Table cpu, uint32_t* cpu_row, Scalars* sc, hipStream_t st);
 /* after build_cpu_ids: enters the external-correlation records and resolves their external ids */
 hipError_t build_extcorr(const ktj_extcorr_rec* e, uint64_t n, Table tn, NarrowCols nc, Table cpu, const uint32_t* cpu_row,
@@ -271,9 +274,11 @@ struct StreamTables {
   int32_t* d_dev;
   uint64_t* d_key;
   uint32_t* d_rank;
+  uint32_t* d_list;   /* KTJ_MAX_STREAM_PAIRS: slots of the pairs */
 };
-hipError_t backfill_streams(const DevBrief* d, uint64_t n, Columns c, uint64_t first_device, StreamTables t,
-                            Scalars* sc, hipStream_t st);
+/* also checks the device rows whose id no runtime row has (tf, fc, link) */
+hipError_t backfill_streams(const DevBrief* d, uint64_t n, Columns c, uint64_t first_device, Table tf, FullCols fc, const DevLink* link,
+                            StreamTables t, Scalars* sc, hipStream_t st);
 
 /* ---- GPU user annotations (GenericActivityProfiler.cpp:277-327, 423-433): one span per
  * (device, resource, annotation id) over the device rows that the user-domain correlation
@@ -308,9 +313,12 @@ struct SortSets {
   uint32_t* dev_rank;
   uint64_t* res_keys;
   uint32_t* res_rank;
+  uint32_t* dev_list;  /* KTJ_SET_MAX: slots of the values */
+  uint32_t* res_list;
 };
-hipError_t collect_distinct(Columns c, uint64_t n, SortSets s, Scalars* sc, hipStream_t st);
-hipError_t rank_distinct(SortSets s, Scalars* sc, hipStream_t st);
+/* distinct values and their ranks, and Scalars::sort; straight: the host will not look at anything before
+ * the end of the pass, so what needs that is flagged (KTJ_DEVERR_CAREFUL) */
+hipError_t collect_distinct(Columns c, uint64_t n, SortSets s, Scalars* sc, bool straight, hipStream_t st);
 /* key = ((rank(dev) << res_bits | rank(res)) << ts_bits) | (ts - ts_min); dropped rows get 1 << key_bits */
 hipError_t make_keys(Columns c, uint64_t n, SortSets s, const Scalars* sc, uint32_t ts_bits, uint32_t res_bits,
                      uint32_t key_bits, uint64_t* keys, uint32_t* vals, hipStream_t st);
@@ -327,9 +335,11 @@ hipError_t clear_error_bits(Scalars* sc, unsigned int bits, hipStream_t st);
 bool sort_packed_fits(uint64_t n, uint32_t key_bits);
 bool sort_packed_passes_forced();
 void sort_packed_force_passes(bool on); /* tests: no one-launch sort of a single tile */
-hipError_t sort_packed(Columns c, uint64_t n, SortSets s, const Scalars* sc, uint32_t ts_bits, uint32_t res_bits,
-                       uint32_t key_bits, uint64_t* buf_a, uint64_t* buf_b, uint32_t* perm, uint32_t* hist, uint64_t* scan_tmp,
-                       hipStream_t st);
+uint32_t sort_packed_passes(uint32_t key_bits);
+/* key widths come from Scalars::sort; `passes` is how many are launched: those beyond the plan end at once, and
+ * a plan that needs more (or does not fit a word) sets KTJ_DEVERR_CAREFUL in Scalars::error */
+hipError_t sort_packed(Columns c, uint64_t n, SortSets s, Scalars* sc, uint32_t passes, uint64_t* buf_a, uint64_t* buf_b, uint32_t* perm,
+                       uint32_t* hist, hipStream_t st);
 hipError_t make_rank_keys(Columns c, const uint32_t* order, uint64_t n, SortSets s, uint32_t res_bits, uint32_t rank_bits,
                           uint64_t* keys, uint32_t* vals, hipStream_t st);
 /* stable LSD radix sort of (key, val) pairs on the low `bits` bits; result ends in keys_out/vals_out
@@ -345,10 +355,10 @@ hipError_t radix_sort(uint64_t* keys_a, uint32_t* vals_a, uint64_t* keys_b, uint
 hipError_t stream_sync_first(const uint32_t* perm, uint64_t n_sorted, const ktj_generic_rec* g, uint64_t n_generic,
                              const int64_t* dev, DictViews d, uint64_t* keys, uint32_t* first_pos, uint32_t* is_first, Scalars* sc,
                              hipStream_t st);
-/* sync_first: per generic row, from stream_sync_first, or null when there are no such rows */
-/* generic records whose rows start at arrival index `first` */
-hipError_t mat_generic_rows(const ktj_generic_rec* g, uint64_t n, uint64_t first, EmitCtx ctx, const uint32_t* sync_first,
-                            MatRow* mat, uint32_t* len, Scalars* sc, hipStream_t st);
+/* joined rows and lengths of generic records (arrival index first_generic on; sync_first: per record, from
+ * stream_sync_first, or null when there are no such rows) and of device records */
+hipError_t mat_rows(const ktj_generic_rec* g, uint64_t ng, uint64_t first_generic, const uint32_t* sync_first, const ktj_device_rec* d, uint64_t nd,
+                    Columns c, uint64_t first_device, const DevLink* link, EmitCtx ctx, MatRow* mat, uint32_t* len, Scalars* sc, hipStream_t st);
 /* the pass over the runtime rows: publishes what device rows take over (first timestamp, stream, grid,
  * size) into the tables, reads the "External id", makes the joined rows and their lengths; runs
  * after build_extcorr and before link_device_rows */
@@ -359,10 +369,19 @@ hipError_t join_runtime_rows(const ktj_runtime_rec* r, uint64_t n, Columns c, ui
  * runtime rows share a slot */
 hipError_t republish_runtime_rows(const ktj_runtime_rec* r, uint64_t n, Columns c, uint64_t first, FullCols fc, NarrowCols nc,
                                   const uint32_t* slot_f, const uint32_t* slot_n, Scalars* sc, hipStream_t st);
-hipError_t mat_device_rows(const ktj_device_rec* d, uint64_t n, Columns c, uint64_t first, const DevLink* link,
-                           EmitCtx ctx, MatRow* mat, uint32_t* len, Scalars* sc, hipStream_t st);
-hipError_t gather_len(const uint32_t* perm, const uint32_t* len, uint64_t n, uint32_t* len_sorted, uint8_t* kind_sorted,
-                      hipStream_t st);
+/* lengths and tail kinds in emission order, and the activities' offsets (n + 1).  With text.out set the
+ * document's header and footer text go to their places and scalars and total to the host: the emit kernels
+ * may follow without the host having seen anything. */
+struct DocText {
+  const char* prefix; uint64_t n_prefix;   /* page-locked, 16-byte aligned, readable up to the next multiple of 16 */
+  const char* suffix; uint64_t n_suffix;
+  char* out; uint64_t out_cap;             /* what does not fit with 64 bytes to spare is not written */
+  Scalars* h_sc; uint64_t* h_total;        /* page-locked: the scalars in front of the shards, the activities' bytes */
+  uint64_t* h_end;                         /* small traces: the wall clock when the last activities were written */
+};
+uint64_t offsets_tmp_elems(uint64_t n);
+hipError_t gather_offsets(const uint32_t* perm, const uint32_t* len, uint64_t n, uint32_t* len_sorted, uint8_t* kind_sorted, uint64_t* sums,
+                          uint64_t* offs, Scalars* sc, const DocText& text, hipStream_t st);
 
 /* ---- stage 4b: emit ---- */
 /* tile size (bytes of output per workgroup) for a document whose activity section has act_bytes
@@ -373,10 +392,10 @@ hipError_t emit(const MatRow* mat, const uint32_t* perm, const uint64_t* offs /*
                 EmitCtx ctx, char* out, uint64_t prefix_len, uint64_t act_bytes, uint32_t tile,
                 uint32_t* tile_start /* tiles + 1 */, hipStream_t st);
 
-/* direct variant: one lane per activity, no LDS staging; kind_sorted holds the tail kind of every
- * activity in emission order (gather_len); n_rows = number of activities that are written */
-hipError_t emit_direct(const MatRow* mat, const uint32_t* perm, const uint64_t* offs, const uint8_t* kind_sorted,
-                       uint64_t n_rows, uint64_t act_bytes, EmitCtx ctx, char* out, uint64_t prefix_len, hipStream_t st);
+/* direct variant: one lane per activity; kind_sorted holds the tail kind of every activity in emission order;
+ * Scalars::emit_rows of them, at most n_most */
+hipError_t emit_direct(const MatRow* mat, const uint32_t* perm, const uint64_t* offs, const uint8_t* kind_sorted, uint64_t n_most, EmitCtx ctx,
+                       char* out, uint64_t prefix_len, const Scalars* sc, hipStream_t st);
 
 /* ---- small traces: the whole pass in three launches (small.hip) ---- */
 #define SMALL_ROWS 2048u       /* records of the three classes together: what LDS holds the join tables for */
@@ -396,21 +415,14 @@ struct SmallArgs {
   uint32_t* perm;
   Scalars* sc;
 };
-struct SmallText {
-  const char* prefix; uint64_t n_prefix;   /* page-locked, 16-byte aligned, readable up to the next multiple of 16 */
-  const char* suffix; uint64_t n_suffix;
-  char* out; uint64_t out_cap;             /* nothing is written if prefix, activities, suffix and 64 bytes do not fit */
-  Scalars* h_sc; uint64_t* h_total;        /* page-locked: the scalars in front of the shards, the activities' bytes */
-  uint64_t* h_end;                         /* and the wall clock when the last activities were written */
-};
 bool small_fits(uint64_t n_generic, uint64_t n_runtime, uint64_t n_device, uint64_t n_ext);
 uint32_t small_slots(uint64_t n_generic, uint64_t n_runtime, uint64_t n_device, uint64_t n_ext);
 /* decode to order and lengths; then the document.  Scalars::error holds KTJ_DEVERR_SMALL_UNFIT afterwards
  * where the trace needs the launches of a large one: nothing is written then. */
 hipError_t small_pass(const SmallArgs& a, uint32_t n_strings, hipStream_t st);
-hipError_t small_emit(const SmallArgs& a, const SmallText& t, hipStream_t st);
+hipError_t small_emit(const SmallArgs& a, const DocText& t, hipStream_t st);
 /* behind small_emit where Scalars::n_plain is not zero: the activities that it left out */
-hipError_t small_plain(const SmallArgs& a, const SmallText& t, hipStream_t st);
+hipError_t small_plain(const SmallArgs& a, const DocText& t, hipStream_t st);
 
 }  // namespace gpu
 }  // namespace ktj

@@ -171,23 +171,6 @@ __global__ void k_fill_u32(uint32_t* p, uint32_t v, uint64_t n) {
   uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = v;
 }
-__global__ void k_init_scalars(Scalars* s) {
-  if (blockIdx.x == 0)
-    for (uint32_t c = threadIdx.x; c < KTJ_COUNTER_SHARDS; c += blockDim.x)
-      for (int k = 0; k < 16; ++k) s->shard[c][k] = 0;
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
-    s->ts_min_biased = ~0ULL; s->ts_max_biased = 0;
-    s->out_of_range = 0; s->out_of_order = 0; s->n_flow = 0; s->n_linked = 0; s->n_blank_names = 0; s->n_valid = 0;
-    s->n_unresolved = 0; s->n_sync_typed = 0; s->n_device_orphans = 0; s->error = 0; s->have_stream_src = 0; s->n_dev_ranks = 0; s->n_res_ranks = 0; s->n_dense = 0; s->runtime_ids_repeat = 0;
-    s->n_queues = 0; s->n_sync_rows = 0; s->ext_ids_repeat = 0;
-    for (uint32_t k = 0; k < KTJ_PART_SLOTS; ++k) s->part_done[k] = 0;
-    for (int k = 0; k < 3; ++k) {
-      s->plan.range[k].lo = ~0ULL; s->plan.range[k].hi = 0;
-      s->plan.ctl[k].base = 0; s->plan.ctl[k].span = 0; s->plan.ctl[k].direct = 0; s->plan.ctl[k].pad = 0;
-    }
-  }
-}
-
 hipError_t fill_u64(uint64_t* p, uint64_t v, uint64_t n, hipStream_t st) {
   if (n == 0) return hipSuccess;
   hipLaunchKernelGGL(k_fill_u64, dim3(grid_for(n, KTJ_BLOCK)), dim3(KTJ_BLOCK), 0, st, p, v, n);
@@ -198,28 +181,51 @@ hipError_t fill_u32(uint32_t* p, uint32_t v, uint64_t n, hipStream_t st) {
   hipLaunchKernelGGL(k_fill_u32, dim3(grid_for(n, KTJ_BLOCK)), dim3(KTJ_BLOCK), 0, st, p, v, n);
   return KTJ_LAUNCH_CHECK();
 }
-/* several fills in one launch (blockIdx.y picks the job): a small trace pays per launch, not per byte */
-__global__ void k_fill_many(FillJobs jobs) {
-  const uint32_t j = blockIdx.y;
-  const uint64_t n = jobs.n[j], v = jobs.value[j];
-  if (jobs.bytes_each[j] == 8) {
-    uint64_t* p = static_cast<uint64_t*>(jobs.p[j]);
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) p[i] = v;
+/* What a pass needs before its records are looked at, in one launch: the scalars (first workgroup), the
+ * dictionary views (a wavefront per string) and the fills of the small tables (the last workgroups). */
+#define BEGIN_FILL_BLOCKS 128u
+__global__ void __launch_bounds__(KTJ_BLOCK)
+k_begin(Scalars* s, FillJobs jobs, const char* blob, const uint64_t* off, uint32_t n_strings, uint32_t dict_blocks, DictEntry* entries,
+        char* name_blob, char* arg_blob) {
+  if (blockIdx.x == 0) {
+    for (uint32_t k = threadIdx.x; k < KTJ_COUNTER_SHARDS * 16u; k += KTJ_BLOCK) {
+      s->shard[k / 16u][k % 16u] = 0;
+      s->range_shard[k / 16u][k % 16u] = k % 2u ? 0 : ~0ULL; /* lo, hi of each range: empty */
+    }
+    if (threadIdx.x == 0) {
+      s->ts_min_biased = ~0ULL; s->ts_max_biased = 0;
+      s->out_of_range = 0; s->out_of_order = 0; s->n_flow = 0; s->n_linked = 0; s->n_blank_names = 0; s->n_valid = 0;
+      s->n_unresolved = 0; s->n_sync_typed = 0; s->n_device_orphans = 0; s->error = 0; s->have_stream_src = 0; s->n_dev_ranks = 0; s->n_res_ranks = 0; s->n_dense = 0; s->runtime_ids_repeat = 0;
+      s->n_queues = 0; s->n_sync_rows = 0; s->ext_ids_repeat = 0; s->n_plain = 0;
+      s->sort.ts_bits = s->sort.res_bits = s->sort.key_bits = 0;
+      for (int k = 0; k < KTJ_DONE_COUNT; ++k) s->done[k] = 0;
+      for (uint32_t k = 0; k < KTJ_PART_SLOTS; ++k) s->part_done[k] = 0;
+      for (int k = 0; k < KTJ_CLOCK_COUNT; ++k) s->clock[k] = 0;
+      stage_clock(s, KTJ_CLOCK_BEGIN);
+    }
+  } else if (blockIdx.x <= dict_blocks) {
+    const uint32_t id = (blockIdx.x - 1u) * (KTJ_BLOCK >> 6) + (threadIdx.x >> 6);
+    if (id < n_strings) dict_string(blob, off, id, entries, name_blob, arg_blob);
   } else {
-    uint32_t* p = static_cast<uint32_t*>(jobs.p[j]);
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) p[i] = (uint32_t)v;
+    const uint32_t b = blockIdx.x - 1u - dict_blocks;
+    for (uint32_t j = 0; j < jobs.count; ++j) {
+      const uint64_t n = jobs.n[j], v = jobs.value[j];
+      if (jobs.bytes_each[j] == 8) {
+        uint64_t* p = static_cast<uint64_t*>(jobs.p[j]);
+        for (uint64_t i = (uint64_t)b * KTJ_BLOCK + threadIdx.x; i < n; i += BEGIN_FILL_BLOCKS * KTJ_BLOCK) p[i] = v;
+      } else {
+        uint32_t* p = static_cast<uint32_t*>(jobs.p[j]);
+        for (uint64_t i = (uint64_t)b * KTJ_BLOCK + threadIdx.x; i < n; i += BEGIN_FILL_BLOCKS * KTJ_BLOCK) p[i] = (uint32_t)v;
+      }
+    }
   }
 }
-hipError_t fill_many(const FillJobs& jobs, hipStream_t st) {
-  if (jobs.count == 0) return hipSuccess;
-  uint64_t most = 1;
-  for (uint32_t j = 0; j < jobs.count; ++j) most = jobs.n[j] > most ? jobs.n[j] : most;
-  hipLaunchKernelGGL(k_fill_many, dim3(grid_stride_for(most, KTJ_BLOCK * 4), jobs.count), dim3(KTJ_BLOCK), 0, st, jobs);
-  return KTJ_LAUNCH_CHECK();
-}
-hipError_t init_scalars(Scalars* s, hipStream_t st) {
+hipError_t begin_pass(Scalars* s, const FillJobs& jobs, const char* blob, const uint64_t* off, uint32_t n_strings, DictEntry* entries,
+                      char* name_blob, char* arg_blob, hipStream_t st) {
   static_assert((KTJ_COUNTER_SHARDS & (KTJ_COUNTER_SHARDS - 1u)) == 0, "a workgroup's copy is its index modulo the number of copies");
-  hipLaunchKernelGGL(k_init_scalars, dim3(1), dim3(64), 0, st, s);
+  const uint32_t dict_blocks = grid_for(n_strings, KTJ_BLOCK >> 6);
+  hipLaunchKernelGGL(k_begin, dim3(1u + dict_blocks + BEGIN_FILL_BLOCKS), dim3(KTJ_BLOCK), 0, st, s, jobs, blob, off, n_strings, dict_blocks,
+                     entries, name_blob, arg_blob);
   return KTJ_LAUNCH_CHECK();
 }
 
@@ -314,8 +320,7 @@ __global__ void k_scan_of_sums(uint64_t* sums, uint64_t m) {
   if (threadIdx.x == 0) sums[m] = carry;
 }
 template <typename OutT>
-__global__ void k_scan_final(const uint32_t* in, uint64_t n, const uint64_t* sums, uint64_t m, OutT* out,
-                             bool write_total) {
+__global__ void k_scan_final(const uint32_t* in, uint64_t n, const uint64_t* sums, OutT* out) {
   __shared__ uint64_t lds_wave[SCAN_MAX_WAVES];
   const uint64_t base = (uint64_t)blockIdx.x * SCAN_TILE + (uint64_t)threadIdx.x * SCAN_ITEMS;
   uint32_t v[SCAN_ITEMS];
@@ -341,7 +346,6 @@ __global__ void k_scan_final(const uint32_t* in, uint64_t n, const uint64_t* sum
       ex += v[k];
     }
   }
-  if (write_total && blockIdx.x == 0 && threadIdx.x == 0) out[n] = (OutT)sums[m];
 }
 
 /* small inputs (one tile of SCAN_SMALL_THREADS lanes): the whole scan in one workgroup and one pass.
@@ -349,7 +353,7 @@ __global__ void k_scan_final(const uint32_t* in, uint64_t n, const uint64_t* sum
 #define SCAN_SMALL_THREADS 1024u
 #define SCAN_SMALL_MAX (SCAN_SMALL_THREADS * SCAN_ITEMS)
 template <typename OutT>
-__global__ void __launch_bounds__(SCAN_SMALL_THREADS) k_scan_small(const uint32_t* in, uint64_t n, OutT* out, bool write_total) {
+__global__ void __launch_bounds__(SCAN_SMALL_THREADS) k_scan_small(const uint32_t* in, uint64_t n, OutT* out) {
   __shared__ uint64_t wave_sum[SCAN_SMALL_THREADS >> 6];
   const uint64_t base = (uint64_t)threadIdx.x * SCAN_ITEMS;
   uint32_t v[SCAN_ITEMS];
@@ -376,68 +380,35 @@ __global__ void __launch_bounds__(SCAN_SMALL_THREADS) k_scan_small(const uint32_
     if (base + k < n) out[base + k] = (OutT)ex;
     ex += v[k];
   }
-  if (write_total && threadIdx.x == 0) out[n] = (OutT)tot;
 }
 
 uint64_t scan_tmp_elems(uint64_t n) { return (n + SCAN_TILE - 1) / SCAN_TILE + 2; }
 
-hipError_t scan_u32_to_u64(const uint32_t* in, uint64_t* out, uint64_t n, uint64_t* tmp, hipStream_t st) {
-  const uint64_t m = (n + SCAN_TILE - 1) / SCAN_TILE;
-  if (n <= SCAN_SMALL_MAX) {
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_scan_small<uint64_t>), dim3(1), dim3(SCAN_SMALL_THREADS), 0, st, in, n, out, true);
-    return KTJ_LAUNCH_CHECK();
-  }
-  if (m > 0) hipLaunchKernelGGL(k_scan_sums, dim3((unsigned)m), dim3(KTJ_BLOCK), 0, st, in, n, tmp);
-  hipLaunchKernelGGL(k_scan_of_sums, dim3(1), dim3(m > KTJ_BLOCK ? 1024 : KTJ_BLOCK), 0, st, tmp, m);
-  if (m > 0)
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_scan_final<uint64_t>), dim3((unsigned)m), dim3(KTJ_BLOCK), 0, st, in, n,
-                       (const uint64_t*)tmp, m, out, true);
-  else
-    hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, st, out, (uint64_t)0, (uint64_t)1);
-  return KTJ_LAUNCH_CHECK();
-}
 hipError_t scan_u32_inplace(uint32_t* data, uint64_t n, uint64_t* tmp, hipStream_t st) {
   const uint64_t m = (n + SCAN_TILE - 1) / SCAN_TILE;
   if (m == 0) return hipSuccess;
   if (n <= SCAN_SMALL_MAX) {
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_scan_small<uint32_t>), dim3(1), dim3(SCAN_SMALL_THREADS), 0, st, (const uint32_t*)data, n, data, false);
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_scan_small<uint32_t>), dim3(1), dim3(SCAN_SMALL_THREADS), 0, st, (const uint32_t*)data, n, data);
     return KTJ_LAUNCH_CHECK();
   }
   hipLaunchKernelGGL(k_scan_sums, dim3((unsigned)m), dim3(KTJ_BLOCK), 0, st, (const uint32_t*)data, n, tmp);
   hipLaunchKernelGGL(k_scan_of_sums, dim3(1), dim3(m > KTJ_BLOCK ? 1024 : KTJ_BLOCK), 0, st, tmp, m);
   /* every block reads its tile completely before writing it, and tiles do not overlap */
   hipLaunchKernelGGL(HIP_KERNEL_NAME(k_scan_final<uint32_t>), dim3((unsigned)m), dim3(KTJ_BLOCK), 0, st,
-                     (const uint32_t*)data, n, (const uint64_t*)tmp, m, data, false);
+                     (const uint32_t*)data, n, (const uint64_t*)tmp, data);
   return KTJ_LAUNCH_CHECK();
 }
 
 /* ------------------------------------------------------------------------------------------ */
-/* stage 0: dictionary.  One wavefront per string, both views in one launch: a string's place in */
-/* the view blobs follows from its own offset (DictEntry).  Four launches with two scans of the  */
-/* lengths before: 30 us of every pass, 266 us long for fifteen records.                         */
-/*   arg view  = sanitizeStrForJSON            (libkineto/src/output_json.cpp:72-78)            */
-/*   name view = "kernel"→"Kernel", sanitize, non-printable → "unknown", quote escaping         */
-/*                                             (output_json.cpp:946-949, 86-112)                */
-/* ------------------------------------------------------------------------------------------ */
-__global__ void k_dict(const char* blob, const uint64_t* off, uint32_t n, DictEntry* entries, char* name_blob, char* arg_blob) {
-  const uint32_t id = blockIdx.x * (KTJ_BLOCK >> 6) + (threadIdx.x >> 6);
-  if (id < n) dict_string(blob, off, id, entries, name_blob, arg_blob);
-}
-hipError_t dict_views(const char* blob, const uint64_t* off, uint32_t n, DictEntry* entries, char* name_blob, char* arg_blob,
-                      hipStream_t st) {
-  if (n == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_dict, dim3(grid_for(n, KTJ_BLOCK >> 6)), dim3(KTJ_BLOCK), 0, st, blob, off, n, entries, name_blob, arg_blob);
-  return KTJ_LAUNCH_CHECK();
-}
-
-/* ------------------------------------------------------------------------------------------ */
-/* stage 1: decode.  A workgroup pulls 256 packed records into LDS with lane-consecutive 16-byte */
-/* loads (fully coalesced), then each lane unpacks its own record into the columns.              */
+/* stage 1: decode, all record classes in one launch.  A workgroup pulls 256 packed records into   */
+/* LDS with lane-consecutive 16-byte loads (fully coalesced), then each lane unpacks its own       */
+/* record into the columns; the smallest and largest ids, from which the join tables are planned,  */
+/* go to one of 64 copies of the ranges (atomics on a single address are carried out one after     */
+/* the other, and an array of per-workgroup ranges takes another launch to reduce).                */
 /* ------------------------------------------------------------------------------------------ */
 template <typename Rec>
-__device__ __forceinline__ const Rec* stage_records(const Rec* recs, uint64_t n, uint4* stage, uint32_t* n_here) {
+__device__ __forceinline__ const Rec* stage_records(const Rec* recs, uint64_t base, uint64_t n, uint4* stage, uint32_t* n_here) {
   constexpr uint32_t U = sizeof(Rec) / 16;
-  const uint64_t base = (uint64_t)blockIdx.x * KTJ_BLOCK;
   const uint32_t cnt = (uint32_t)((n - base) < KTJ_BLOCK ? (n - base) : KTJ_BLOCK);
   const uint4* g = reinterpret_cast<const uint4*>(recs + base);
   for (uint32_t i = threadIdx.x; i < cnt * U; i += KTJ_BLOCK) stage[i] = g[i];
@@ -445,11 +416,9 @@ __device__ __forceinline__ const Rec* stage_records(const Rec* recs, uint64_t n,
   *n_here = cnt;
   return reinterpret_cast<const Rec*>(stage);
 }
-
-/* Smallest and largest key of the workgroup's rows into part[blockIdx.x] (empty: lo > hi).  The
- * join tables are planned from these ranges; collecting them here saves a pass over the ids.
- * Must be reached by every thread of the workgroup. */
-__device__ __forceinline__ void block_key_range(bool has, uint64_t key, KeyRange* part) {
+/* Smallest and largest key of the workgroup's rows into the ranges of table `which`.  Must be reached by
+ * every thread of the workgroup. */
+__device__ __forceinline__ void block_key_range(bool has, uint64_t key, Scalars* sc, int which) {
   __shared__ unsigned long long s_lo[KTJ_BLOCK >> 6], s_hi[KTJ_BLOCK >> 6];
   unsigned long long lo = has ? key : ~0ULL, hi = has ? key : 0ULL;
   for (int o = 32; o > 0; o >>= 1) {
@@ -462,81 +431,77 @@ __device__ __forceinline__ void block_key_range(bool has, uint64_t key, KeyRange
   __syncthreads();
   if (threadIdx.x == 0) {
     for (uint32_t k = 1; k < (blockDim.x >> 6); ++k) { lo = s_lo[k] < lo ? s_lo[k] : lo; hi = s_hi[k] > hi ? s_hi[k] : hi; }
-    KeyRange r;
-    r.lo = lo; r.hi = hi;
-    part[blockIdx.x] = r;
+    unsigned long long* r = &sc->range_shard[blockIdx.x & (KTJ_COUNTER_SHARDS - 1u)][2 * which];
+    if (lo <= hi) { atomicMin(&r[0], lo); atomicMax(&r[1], hi); }
   }
 }
-__global__ void k_decode_generic(const ktj_generic_rec* recs, uint64_t n, Columns c, uint64_t first, Scalars* sc,
-                                 EmitCtx ctx, KeyRange* id_range) {
-  __shared__ uint4 stage[KTJ_BLOCK * sizeof(ktj_generic_rec) / 16];
-  uint32_t cnt;
-  const ktj_generic_rec* l = stage_records(recs, n, stage, &cnt);
-  /* rows that may need a Stream Sync row of their own are rare: the extra passes run only if any */
-  const bool sync_typed = threadIdx.x < cnt && l[threadIdx.x].type == KTJ_TYPE_CUDA_SYNC;
-  if (__syncthreads_or(sync_typed ? 1 : 0)) block_add(sc, KTJ_CNT_SYNC_TYPED, sync_typed ? 1u : 0u);
-  if (id_range) block_key_range(threadIdx.x < cnt, threadIdx.x < cnt ? (uint64_t)(int64_t)l[threadIdx.x].id : 0, id_range);
-  if (threadIdx.x >= cnt) return;
-  store_cols(c, first + (uint64_t)blockIdx.x * KTJ_BLOCK + threadIdx.x, cols_generic(l[threadIdx.x], ctx));
-}
-__global__ void k_decode_runtime(const ktj_runtime_rec* recs, uint64_t n, Columns c, uint64_t first, KeyRange* id_range,
-                                 KeyRange* narrow_range, ClockDev clk, int64_t win_start, int64_t win_end, Scalars* sc) {
+#define EXT_PER_BLOCK (KTJ_BLOCK * 8u)
+__global__ void __launch_bounds__(KTJ_BLOCK) k_decode(DecodeJob J, Columns c, EmitCtx ctx, Scalars* sc) {
   __shared__ uint4 stage[KTJ_BLOCK * sizeof(ktj_runtime_rec) / 16];
+  static_assert(sizeof(ktj_runtime_rec) >= sizeof(ktj_generic_rec) && sizeof(ktj_runtime_rec) >= sizeof(ktj_device_rec), "the largest record");
+  if (blockIdx.x == 0 && threadIdx.x == 0 && J.whole_pass) stage_clock(sc, KTJ_CLOCK_DECODE);
+  uint64_t b = blockIdx.x;
   uint32_t cnt;
-  const ktj_runtime_rec* l = stage_records(recs, n, stage, &cnt);
-  {
+  if (b < J.gb) {
+    const ktj_generic_rec* l = stage_records(J.g, b * KTJ_BLOCK, J.ng, stage, &cnt);
+    /* rows that may need a Stream Sync row of their own are rare: the extra passes run only if any */
+    const bool has = threadIdx.x < cnt, sync_typed = has && l[threadIdx.x].type == KTJ_TYPE_CUDA_SYNC;
+    if (__syncthreads_or(sync_typed ? 1 : 0)) block_add(sc, KTJ_CNT_SYNC_TYPED, sync_typed ? 1u : 0u);
+    if (J.whole_pass) block_key_range(has, has ? (uint64_t)(int64_t)l[threadIdx.x].id : 0, sc, KTJ_TBL_CPU);
+    if (has) store_cols(c, J.first + b * KTJ_BLOCK + threadIdx.x, cols_generic(l[threadIdx.x], ctx));
+    return;
+  }
+  b -= J.gb;
+  if (b < J.rb) {
+    const ktj_runtime_rec* l = stage_records(J.r, b * KTJ_BLOCK, J.nr, stage, &cnt);
     const bool has = threadIdx.x < cnt;
     const uint64_t id = has ? l[threadIdx.x].id : 0;
-    block_key_range(has, id, id_range);
-    block_key_range(has, narrow_corr_key(id), narrow_range);
+    block_key_range(has, id, sc, KTJ_TBL_FULL);
+    block_key_range(has, narrow_corr_key(id), sc, KTJ_TBL_NARROW);
+    uint32_t oor = 0;
+    if (has) {
+      const RowCols r = cols_runtime(l[threadIdx.x], J.clk, J.win_start, J.win_end);
+      oor = r.meta & KTJ_M_VALID ? 0u : 1u;
+      store_cols(c, J.ng + b * KTJ_BLOCK + threadIdx.x, r);
+    }
+    block_add(sc, KTJ_CNT_OUT_OF_RANGE, oor);
+    return;
   }
-  uint32_t oor = 0;
-  if (threadIdx.x < cnt) {
-    const RowCols r = cols_runtime(l[threadIdx.x], clk, win_start, win_end);
-    oor = r.meta & KTJ_M_VALID ? 0u : 1u;
-    store_cols(c, first + (uint64_t)blockIdx.x * KTJ_BLOCK + threadIdx.x, r);
+  b -= J.rb;
+  if (b < J.db) {
+    const ktj_device_rec* l = stage_records(J.d, b * KTJ_BLOCK, J.nd, stage, &cnt);
+    const bool has = threadIdx.x < cnt;
+    block_key_range(has, has ? l[threadIdx.x].id : 0, sc, KTJ_TBL_FULL);
+    uint32_t oor = 0;
+    if (has) {
+      const ktj_device_rec* d = &l[threadIdx.x];
+      const uint64_t i = b * KTJ_BLOCK + threadIdx.x;
+      const RowCols r = cols_device(*d, J.clk, J.win_start, J.win_end);
+      oor = r.meta & KTJ_M_VALID ? 0u : 1u;
+      store_cols(c, J.ng + J.nr + i, r);
+      DevBrief br;
+      br.queue = d->queue; br.device = d->device; br.domain = device_row_domain(d->domain);
+      J.brief[i] = br;
+    }
+    block_add(sc, KTJ_CNT_OUT_OF_RANGE, oor);
+    return;
   }
-  block_add(sc, KTJ_CNT_OUT_OF_RANGE, oor);
-}
-__global__ void k_decode_device(const ktj_device_rec* recs, uint64_t n, Columns c, uint64_t first, DevBrief* brief,
-                                KeyRange* id_range, ClockDev clk, int64_t win_start, int64_t win_end, Scalars* sc) {
-  __shared__ uint4 stage[KTJ_BLOCK * sizeof(ktj_device_rec) / 16];
-  uint32_t cnt;
-  const ktj_device_rec* l = stage_records(recs, n, stage, &cnt);
-  block_key_range(threadIdx.x < cnt, threadIdx.x < cnt ? l[threadIdx.x].id : 0, id_range);
-  uint32_t oor = 0;
-  if (threadIdx.x < cnt) {
-    const ktj_device_rec* d = &l[threadIdx.x];
-    const uint64_t i = (uint64_t)blockIdx.x * KTJ_BLOCK + threadIdx.x;
-    const RowCols r = cols_device(*d, clk, win_start, win_end);
-    oor = r.meta & KTJ_M_VALID ? 0u : 1u;
-    store_cols(c, first + i, r);
-    DevBrief br;
-    br.queue = d->queue; br.device = d->device; br.domain = device_row_domain(d->domain);
-    brief[i] = br;
+  b -= J.db; /* correlation ids of the external-correlation records */
+  uint64_t lo = ~0ULL, hi = 0;
+#pragma unroll
+  for (uint32_t k = 0; k < 8; ++k) {
+    const uint64_t i = b * EXT_PER_BLOCK + k * KTJ_BLOCK + threadIdx.x;
+    const uint64_t v = i < J.nx ? J.x[i].correlation : 0;
+    if (i < J.nx) { lo = v < lo ? v : lo; hi = v > hi ? v : hi; }
   }
-  block_add(sc, KTJ_CNT_OUT_OF_RANGE, oor);
+  block_key_range(lo <= hi, lo, sc, KTJ_TBL_NARROW);
+  block_key_range(lo <= hi, hi, sc, KTJ_TBL_NARROW);
 }
-
-uint64_t decode_blocks(uint64_t n) { return grid_for(n, KTJ_BLOCK); }
-hipError_t decode_generic(const ktj_generic_rec* r, uint64_t n, Columns c, uint64_t first, Scalars* sc, EmitCtx ctx,
-                          KeyRange* id_range, hipStream_t st) {
-  if (n == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_decode_generic, dim3(grid_for(n, KTJ_BLOCK)), dim3(KTJ_BLOCK), 0, st, r, n, c, first, sc, ctx, id_range);
-  return KTJ_LAUNCH_CHECK();
-}
-hipError_t decode_runtime(const ktj_runtime_rec* r, uint64_t n, Columns c, uint64_t first, KeyRange* id_range,
-                          KeyRange* narrow_range, ClockDev clk, int64_t win_start, int64_t win_end, Scalars* sc, hipStream_t st) {
-  if (n == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_decode_runtime, dim3(grid_for(n, KTJ_BLOCK)), dim3(KTJ_BLOCK), 0, st, r, n, c, first, id_range,
-                     narrow_range, clk, win_start, win_end, sc);
-  return KTJ_LAUNCH_CHECK();
-}
-hipError_t decode_device(const ktj_device_rec* r, uint64_t n, Columns c, uint64_t first, DevBrief* brief, KeyRange* id_range,
-                         ClockDev clk, int64_t win_start, int64_t win_end, Scalars* sc, hipStream_t st) {
-  if (n == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_decode_device, dim3(grid_for(n, KTJ_BLOCK)), dim3(KTJ_BLOCK), 0, st, r, n, c, first, brief, id_range,
-                     clk, win_start, win_end, sc);
+hipError_t decode(DecodeJob job, Columns c, EmitCtx ctx, Scalars* sc, hipStream_t st) {
+  job.gb = grid_for(job.ng, KTJ_BLOCK); job.rb = grid_for(job.nr, KTJ_BLOCK); job.db = grid_for(job.nd, KTJ_BLOCK);
+  const uint64_t blocks = (uint64_t)job.gb + job.rb + job.db + grid_for(job.nx, EXT_PER_BLOCK);
+  if (blocks == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_decode, dim3((unsigned)blocks), dim3(KTJ_BLOCK), 0, st, job, c, ctx, sc);
   return KTJ_LAUNCH_CHECK();
 }
 
@@ -546,145 +511,66 @@ hipError_t decode_device(const ktj_device_rec* r, uint64_t n, Columns c, uint64_
 /* What a device row takes over from "its" runtime row is then published into the table slot by  */
 /* the winning row, so that a device row needs one slot of each table and no other row.          */
 /* ------------------------------------------------------------------------------------------ */
-/* min / max of p[i * stride] (optionally int-narrowed) into *out: one atomic pair per workgroup */
-__global__ void k_key_range(const uint64_t* p, uint32_t stride, uint64_t n, int narrow, KeyRange* out) {
-  __shared__ unsigned long long s_lo[KTJ_BLOCK >> 6], s_hi[KTJ_BLOCK >> 6];
-  unsigned long long lo = ~0ULL, hi = 0;
-  const uint64_t step = (uint64_t)gridDim.x * blockDim.x;
-  for (uint64_t i0 = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i0 < n; i0 += 4 * step) {
-    uint64_t k[4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) { const uint64_t i = i0 + u * step; k[u] = i < n ? p[i * stride] : p[i0 * stride]; }
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const uint64_t v = narrow ? narrow_corr_key(k[u]) : k[u];
-      lo = v < lo ? v : lo;
-      hi = v > hi ? v : hi;
+/* The join tables' modes from the ranges of their keys, and what can be reached of them cleared (the
+ * planned span in direct mode, the whole table otherwise).  Every workgroup reduces the 64 copies of the
+ * ranges for itself; the first one leaves the plan for the kernels that follow. */
+struct TableSpan { uint64_t n; bool direct; };
+__device__ __forceinline__ void clear_keys(const Table& t, const TableSpan& s, uint64_t at, uint64_t step) {
+  if (s.direct && !t.keyed_direct) return; /* keys are not used at all */
+  for (uint64_t i = at; i < s.n; i += step) t.keys[i] = KTJ_EMPTY_KEY;
+  if (at == 0) t.keys[t.mask + 1ull] = KTJ_EMPTY_KEY;
+}
+__global__ void __launch_bounds__(KTJ_BLOCK)
+k_plan_clear(Scalars* sc, Table tf, FullCols fc, Table tn, NarrowCols nc, Table cpu, int force_hash) {
+  __shared__ TableCtl ctl[3];
+  if (blockIdx.x == 0 && threadIdx.x == 0) stage_clock(sc, KTJ_CLOCK_JOIN);
+  if (threadIdx.x < 64) {
+    for (int k = 0; k < 3; ++k) {
+      unsigned long long lo = sc->range_shard[threadIdx.x][2 * k], hi = sc->range_shard[threadIdx.x][2 * k + 1];
+      for (int o = 32; o > 0; o >>= 1) {
+        const unsigned long long l2 = __shfl_xor(lo, o), h2 = __shfl_xor(hi, o);
+        lo = l2 < lo ? l2 : lo;
+        hi = h2 > hi ? h2 : hi;
+      }
+      const uint64_t cap = (uint64_t)(k == KTJ_TBL_FULL ? tf.mask : k == KTJ_TBL_NARROW ? tn.mask : cpu.mask) + 1u;
+      TableCtl x;
+      x.base = 0; x.span = 0; x.direct = 0; x.pad = 0;
+      /* the reserved key never takes part in direct addressing (it has its own slot) */
+      if (!force_hash && lo <= hi && hi - lo < cap) { x.base = lo; x.span = hi - lo; x.direct = 1; }
+      if (threadIdx.x == 0) {
+        ctl[k] = x;
+        if (blockIdx.x == 0) { sc->plan.range[k].lo = lo; sc->plan.range[k].hi = hi; sc->plan.ctl[k] = x; }
+      }
     }
   }
-  for (int o = 32; o > 0; o >>= 1) {
-    const unsigned long long l2 = __shfl_xor(lo, o), h2 = __shfl_xor(hi, o);
-    lo = l2 < lo ? l2 : lo;
-    hi = h2 > hi ? h2 : hi;
-  }
-  if (lane_id() == 0) { s_lo[threadIdx.x >> 6] = lo; s_hi[threadIdx.x >> 6] = hi; }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    for (uint32_t k = 1; k < (blockDim.x >> 6); ++k) { lo = s_lo[k] < lo ? s_lo[k] : lo; hi = s_hi[k] > hi ? s_hi[k] : hi; }
-    if (lo <= hi) { atomicMin(&out->lo, lo); atomicMax(&out->hi, hi); }
-  }
-}
-/* the per-workgroup ranges of the decode kernels into the plan's ranges: MERGE_SPLIT workgroups per job */
-#define MERGE_SPLIT 16u
-struct RangeJobs {
-  const KeyRange* src[4];
-  uint64_t n[4];
-  uint32_t dst[4]; /* KTJ_TBL_* */
-};
-__global__ void k_merge_ranges(RangeJobs jobs, Scalars* sc) {
-  __shared__ unsigned long long s_lo[1024 >> 6], s_hi[1024 >> 6];
-  const uint32_t job = blockIdx.x / MERGE_SPLIT, part = blockIdx.x % MERGE_SPLIT;
-  const KeyRange* src = jobs.src[job];
-  const uint64_t n = jobs.n[job];
-  unsigned long long lo = ~0ULL, hi = 0;
-  for (uint64_t i = (uint64_t)part * blockDim.x + threadIdx.x; i < n; i += (uint64_t)MERGE_SPLIT * blockDim.x) {
-    const KeyRange r = src[i];
-    if (r.lo <= r.hi) { lo = r.lo < lo ? r.lo : lo; hi = r.hi > hi ? r.hi : hi; }
-  }
-  for (int o = 32; o > 0; o >>= 1) {
-    const unsigned long long l2 = __shfl_xor(lo, o), h2 = __shfl_xor(hi, o);
-    lo = l2 < lo ? l2 : lo;
-    hi = h2 > hi ? h2 : hi;
-  }
-  if (lane_id() == 0) { s_lo[threadIdx.x >> 6] = lo; s_hi[threadIdx.x >> 6] = hi; }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    for (uint32_t k = 1; k < (blockDim.x >> 6); ++k) { lo = s_lo[k] < lo ? s_lo[k] : lo; hi = s_hi[k] > hi ? s_hi[k] : hi; }
-    KeyRange* out = &sc->plan.range[jobs.dst[job]];
-    if (lo <= hi) { atomicMin(&out->lo, lo); atomicMax(&out->hi, hi); }
-  }
-}
-__global__ void k_plan_tables(Scalars* sc, uint32_t cap_full, uint32_t cap_narrow, uint32_t cap_cpu, int force_hash) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  const uint32_t cap[3] = {cap_full, cap_narrow, cap_cpu};
-  for (int k = 0; k < 3; ++k) {
-    const KeyRange r = sc->plan.range[k];
-    TableCtl c;
-    c.base = 0; c.span = 0; c.direct = 0; c.pad = 0;
-    /* the reserved key never takes part in direct addressing (it has its own slot) */
-    if (!force_hash && r.lo <= r.hi && r.hi - r.lo < (unsigned long long)cap[k]) { c.base = r.lo; c.span = r.hi - r.lo; c.direct = 1; }
-    sc->plan.ctl[k] = c;
-  }
-}
-/* frees what can be reached: the planned span in direct mode, the whole table otherwise */
-__device__ __forceinline__ uint64_t table_extent(const Table& t) {
-  return t.ctl->direct ? t.ctl->span + 1ull : (uint64_t)t.mask + 1ull;
-}
-__device__ __forceinline__ void clear_keys(const Table& t) {
-  if (t.ctl->direct && !t.keyed_direct) return; /* keys are not used at all */
-  const uint64_t n = table_extent(t);
-  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) t.keys[i] = KTJ_EMPTY_KEY;
-  if (blockIdx.x == 0 && threadIdx.x == 0) t.keys[t.mask + 1ull] = KTJ_EMPTY_KEY;
-}
-__device__ __forceinline__ void clear_full(const Table& t, const FullCols& c) {
-  const uint64_t n = table_extent(t);
-  /* the payload is not cleared: every runtime row writes all of its slot's payload, and a slot
+  const uint64_t at = (uint64_t)blockIdx.x * KTJ_BLOCK + threadIdx.x, step = (uint64_t)gridDim.x * KTJ_BLOCK;
+  auto span = [&](int k, const Table& t) { TableSpan s; s.direct = ctl[k].direct != 0; s.n = s.direct ? ctl[k].span + 1ull : (uint64_t)t.mask + 1ull; return s; };
+  const TableSpan sf = span(KTJ_TBL_FULL, tf), sn = span(KTJ_TBL_NARROW, tn), scpu = span(KTJ_TBL_CPU, cpu);
+  clear_keys(tf, sf, at, step);
+  clear_keys(tn, sn, at, step);
+  clear_keys(cpu, scpu, at, step);
+  /* full table: the payload is not cleared: every runtime row writes all of its slot's payload, and a slot
    * without a runtime row (its bit in has_runtime is clear) is never read */
-  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i <= n; i += (uint64_t)gridDim.x * blockDim.x) {
-    const uint64_t k = i < n ? i : t.mask + 1ull; /* the last iteration clears the reserved slot */
-    c.first[k] = 0xFFFFFFFFu; c.stream_src[k] = 0;
+  for (uint64_t i = at; i <= sf.n; i += step) {
+    const uint64_t k = i < sf.n ? i : tf.mask + 1ull; /* the last one is the reserved slot */
+    fc.first[k] = 0xFFFFFFFFu; fc.stream_src[k] = 0;
   }
-  /* the bitmap: whole words up to the extent, and the word of the reserved slot */
-  const uint64_t words = (n + 31) / 32;
-  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i <= words; i += (uint64_t)gridDim.x * blockDim.x)
-    c.has_runtime[i < words ? i : (t.mask + 1ull) / 32] = 0;
-}
-__device__ __forceinline__ void clear_narrow(const Table& t, const NarrowCols& c) {
-  const uint64_t n = table_extent(t);
-  NarrowPay z; z.ext_val = 0; z.info = 0; z.pay[0] = z.pay[1] = z.pay[2] = 0;
-  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i <= n; i += (uint64_t)gridDim.x * blockDim.x) {
-    const uint64_t k = i < n ? i : t.mask + 1ull;
-    c.ext_src[k] = 0; c.kern_src[k] = 0; c.copy_src[k] = 0; c.pay[k] = z;
+  const uint64_t words = (sf.n + 31) / 32; /* the bitmap: whole words up to the extent, and the word of the reserved slot */
+  for (uint64_t i = at; i <= words; i += step) fc.has_runtime[i < words ? i : (tf.mask + 1ull) / 32] = 0;
+  NarrowPay z;
+  z.ext_val = 0; z.info = 0; z.pay[0] = z.pay[1] = z.pay[2] = 0;
+  for (uint64_t i = at; i <= sn.n; i += step) {
+    const uint64_t k = i < sn.n ? i : tn.mask + 1ull;
+    nc.ext_src[k] = 0; nc.kern_src[k] = 0; nc.copy_src[k] = 0; nc.pay[k] = z;
   }
 }
-
-/* all five in one launch: blockIdx.y picks the part */
-__global__ void k_clear_tables(Table tf, FullCols fc, Table tn, NarrowCols nc, Table cpu) {
-  switch (blockIdx.y) {
-    case 0: clear_keys(tf); break;
-    case 1: clear_keys(tn); break;
-    case 2: clear_keys(cpu); break;
-    case 3: clear_full(tf, fc); break;
-    default: clear_narrow(tn, nc); break;
-  }
-}
-
-hipError_t plan_tables(const KeyRange* parts, uint64_t n_generic, uint64_t n_runtime, uint64_t n_device,
-                       const ktj_extcorr_rec* e, uint64_t n_ext, uint32_t cap_full, uint32_t cap_narrow, uint32_t cap_cpu,
-                       bool force_hash, Scalars* sc, hipStream_t st) {
-  const dim3 b(KTJ_BLOCK);
-  /* parts: [generic ids | runtime ids | runtime ids narrowed | device ids], decode_blocks() entries each */
-  const uint64_t bg = decode_blocks(n_generic), br = decode_blocks(n_runtime), bd = decode_blocks(n_device);
-  RangeJobs jobs;
-  uint32_t n_jobs = 0;
-  auto job = [&](const KeyRange* src, uint64_t n, uint32_t dst) { if (n) { jobs.src[n_jobs] = src; jobs.n[n_jobs] = n; jobs.dst[n_jobs] = dst; ++n_jobs; } };
-  job(parts, bg, KTJ_TBL_CPU);
-  job(parts + bg, br, KTJ_TBL_FULL);
-  job(parts + bg + br, br, KTJ_TBL_NARROW);
-  job(parts + bg + 2 * br, bd, KTJ_TBL_FULL);
-  for (uint32_t k = n_jobs; k < 4; ++k) { jobs.src[k] = nullptr; jobs.n[k] = 0; jobs.dst[k] = 0; }
-  if (n_jobs) hipLaunchKernelGGL(k_merge_ranges, dim3(n_jobs * MERGE_SPLIT), dim3(256), 0, st, jobs, sc);
-  if (n_ext)
-    hipLaunchKernelGGL(k_key_range, dim3(n_ext < 512ull * KTJ_BLOCK * 4 ? grid_for(n_ext, KTJ_BLOCK * 4) : 512u), b, 0, st, reinterpret_cast<const uint64_t*>(e), 2u,
-                       n_ext, 0, &sc->plan.range[KTJ_TBL_NARROW]);
-  hipLaunchKernelGGL(k_plan_tables, dim3(1), dim3(64), 0, st, sc, cap_full, cap_narrow, cap_cpu, force_hash ? 1 : 0);
-  return KTJ_LAUNCH_CHECK();
-}
-hipError_t clear_tables(Table tf, FullCols fc, Table tn, NarrowCols nc, Table cpu, hipStream_t st) {
+hipError_t plan_tables(Table tf, FullCols fc, Table tn, NarrowCols nc, Table cpu, bool force_hash, Scalars* sc, hipStream_t st) {
   uint64_t most = (uint64_t)tf.mask + 1;
   if ((uint64_t)tn.mask + 1 > most) most = (uint64_t)tn.mask + 1;
   if ((uint64_t)cpu.mask + 1 > most) most = (uint64_t)cpu.mask + 1;
-  hipLaunchKernelGGL(k_clear_tables, dim3(grid_stride_for(most, KTJ_BLOCK * 4), 5), dim3(KTJ_BLOCK), 0, st, tf, fc, tn, nc, cpu);
+  const unsigned g = grid_stride_for(most, KTJ_BLOCK * 4);
+  hipLaunchKernelGGL(k_plan_clear, dim3(g < 2048u ? g : 2048u), dim3(KTJ_BLOCK), 0, st, sc, tf, fc, tn, nc, cpu, force_hash ? 1 : 0);
   return KTJ_LAUNCH_CHECK();
 }
 
@@ -833,23 +719,40 @@ __global__ void k_link_device(uint64_t n, Columns c, uint64_t first_device, Tabl
   block_add_to(&sc->n_unresolved, n_unresolved);
   block_add_to(&sc->n_device_orphans, n_orphans);
 }
-/* Only when some in-window device row has an id that no runtime row has: such a row is checked
- * against the first device row of its id (act1 = this row, act2 = the first one). */
-__global__ void k_device_orphans(uint64_t n, Columns c, uint64_t first_device, Table tf, FullCols fc, const DevLink* link,
-                                 Scalars* sc) {
-  if (sc->n_device_orphans == 0) return;
+/* What the device rows need once all of them are linked, both only where some row asks for it:
+ *  - an in-window row whose id no runtime row has is checked against the first device row of its id
+ *    (act1 = this row, act2 = the first one);
+ *  - a row without a stream may take its queue's (RocmStreamQueue.h:42-136; the first pass of that, the
+ *    stream of the correlation-matched runtime row, is part of k_link_device): which stream every queue
+ *    shows, ambiguous when one queue shows two different ones. */
+__global__ void k_after_link(uint64_t n, Columns c, uint64_t first_device, Table tf, FullCols fc, const DevLink* link, const DevBrief* d,
+                             StreamTables t, Scalars* sc) {
+  const bool orphans = sc->n_device_orphans != 0, queues = sc->have_stream_src != 0 && sc->n_unresolved != 0;
   uint32_t n_bad = 0;
-  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) {
-    if (!(link[i].flags & KTJ_DL_ORPHAN)) continue;
-    const uint64_t a = first_device + i;
-    const uint32_t sf = slot_find(tf, c.corr[a]);
-    if (sf == KTJ_NOSLOT) continue;
-    const uint64_t f = fc.first[sf];
-    if (f != a && f != 0xFFFFFFFFull) {
-      const int64_t t1 = c.ts[a], t2 = c.ts[f];
-      if (t2 != 0 && t1 > t2) ++n_bad;
+  if (orphans || queues)
+    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) {
+      const uint64_t a = first_device + i;
+      if (orphans && (link[i].flags & KTJ_DL_ORPHAN)) {
+        const uint32_t sf = slot_find(tf, c.corr[a]);
+        const uint64_t f = sf != KTJ_NOSLOT ? fc.first[sf] : a;
+        if (f != a && f != 0xFFFFFFFFull) {
+          const int64_t t1 = c.ts[a], t2 = c.ts[f];
+          if (t2 != 0 && t1 > t2) ++n_bad;
+        }
+      }
+      if (queues) {
+        const uint64_t stream = (uint64_t)c.res[a], queue = d[i].queue;
+        if (is_async_op(d[i].domain) && stream != 0 && queue != 0) {
+          const uint32_t slot = table_insert_counted(t.q_keys, KTJ_QUEUE_CAP - 1u, queue, &sc->n_queues, KTJ_MAX_QUEUES);
+          if (slot == KTJ_NOSLOT) flag_error(sc, KTJ_DEVERR_QUEUES);
+          else {
+            unsigned long long cur = t.q_stream[slot];
+            if (cur == 0) cur = atomicCAS((unsigned long long*)&t.q_stream[slot], 0ULL, (unsigned long long)stream);
+            if (cur != 0 && cur != stream) t.q_amb[slot] = 1u;
+          }
+        }
+      }
     }
-  }
   block_add(sc, KTJ_CNT_OUT_OF_ORDER, n_bad);
 }
 
@@ -872,8 +775,6 @@ hipError_t link_device_rows(uint64_t n, Columns c, uint64_t first_device, Table 
   if (n == 0) return hipSuccess;
   hipLaunchKernelGGL(k_link_device, dim3(grid_stride_for(n, KTJ_BLOCK)), dim3(KTJ_BLOCK), 0, st, n, c, first_device, tf, fc, tn,
                      nc, link, sc);
-  hipLaunchKernelGGL(k_device_orphans, dim3(grid_stride_for(n, KTJ_BLOCK)), dim3(KTJ_BLOCK), 0, st, n, c, first_device, tf, fc,
-                     (const DevLink*)link, sc);
   return KTJ_LAUNCH_CHECK();
 }
 
@@ -979,58 +880,84 @@ hipError_t span_members(const ktj_extcorr_rec* u, uint64_t n_device, Columns c, 
   return KTJ_LAUNCH_CHECK();
 }
 
-/* ---- stream back-fill: libkineto/src/RocmStreamQueue.h:42-136 (its first pass, the stream of
- * the correlation-matched runtime row, is part of k_link_device) ---- */
-/* pass 2a: queue → stream, ambiguous when one queue shows two different streams.  Passes 2a/2b
- * have no effect when the first pass left no row without a stream (the usual case: every device
- * row has a launching runtime row), and return at once then. */
-__global__ void k_queue_build(const DevBrief* d, uint64_t n, Columns c, uint64_t first_device, StreamTables t,
-                              Scalars* sc) {
-  if (sc->have_stream_src == 0 || sc->n_unresolved == 0) return;
-  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const uint64_t stream = (uint64_t)c.res[first_device + i];
-  const uint64_t queue = d[i].queue;
-  if (!is_async_op(d[i].domain) || stream == 0 || queue == 0) return;
-  const uint32_t slot = table_insert_counted(t.q_keys, KTJ_QUEUE_CAP - 1u, queue, &sc->n_queues, KTJ_MAX_QUEUES);
-  if (slot == KTJ_NOSLOT) { flag_error(sc, KTJ_DEVERR_QUEUES); return; }
-  unsigned long long cur = t.q_stream[slot];
-  if (cur == 0) cur = atomicCAS((unsigned long long*)&t.q_stream[slot], 0ULL, (unsigned long long)stream);
-  if (cur != 0 && cur != stream) t.q_amb[slot] = 1u;
+/* Every workgroup of a launch reports here when its results are in memory; true in all threads of the one
+ * that reports last.  What that one reads of the others must have been written with atomics or agent_store()
+ * and be read with agent_load(): these pass the caches of one XCD by.  (A fence for ordinary stores writes
+ * the XCD's L2 back each time: with one per wavefront k_collect_distinct took 75 instead of 30 us on 733 000
+ * rows.)  Must be reached by every thread of the workgroup. */
+template <typename T> __device__ __forceinline__ void agent_store(T* p, T v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+template <typename T> __device__ __forceinline__ T agent_load(const T* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ __forceinline__ bool last_workgroup(unsigned int* done) {
+  __shared__ int last;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); /* the wavefront's own are there */
+  __syncthreads();
+  if (threadIdx.x == 0) last = __hip_atomic_fetch_add(done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1u ? 1 : 0;
+  __syncthreads();
+  return last != 0;
 }
-/* pass 2b: rows still without a stream take their queue's stream */
-__global__ void k_queue_fill(const DevBrief* d, uint64_t n, Columns c, uint64_t first_device, StreamTables t,
-                             const Scalars* sc) {
-  if (sc->have_stream_src == 0 || sc->n_unresolved == 0) return;
-  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const uint64_t a = first_device + i;
-  if (!is_async_op(d[i].domain) || c.res[a] != 0) return;
-  const uint32_t slot = table_find(t.q_keys, KTJ_QUEUE_CAP - 1u, d[i].queue);
-  if (slot == KTJ_NOSLOT || t.q_amb[slot] != 0 || t.q_stream[slot] == 0) return;
-  c.res[a] = (int64_t)t.q_stream[slot];
+/* table_insert that also tells whether the key is new */
+__device__ uint32_t table_insert_fresh(uint64_t* keys, uint32_t mask, uint64_t key, bool* fresh) {
+  *fresh = false;
+  if (key == KTJ_EMPTY_KEY) {
+    *fresh = atomicExch((unsigned long long*)&keys[mask + 1u], 0ULL) != 0ULL;
+    return mask + 1u;
+  }
+  uint32_t slot = (uint32_t)hash64(key) & mask;
+  for (uint32_t probe = 0; probe <= mask && probe < KTJ_TABLE_PROBES; ++probe) {
+    uint64_t cur = keys[slot];
+    if (cur == key) return slot;
+    if (cur == KTJ_EMPTY_KEY) {
+      const unsigned long long prev = atomicCAS((unsigned long long*)&keys[slot], (unsigned long long)KTJ_EMPTY_KEY, (unsigned long long)key);
+      if (prev == KTJ_EMPTY_KEY) { *fresh = true; return slot; }
+      if (prev == key) return slot;
+    }
+    slot = (slot + 1u) & mask;
+  }
+  return KTJ_NOSLOT;
 }
+
+/* ---- stream back-fill: libkineto/src/RocmStreamQueue.h:42-136 ---- */
 __device__ __forceinline__ uint64_t dense_hash(int32_t device, uint64_t key) {
   uint64_t h = hash64(key ^ hash64((uint64_t)(int64_t)device + 0x9E3779B97F4A7C15ULL));
   return h == KTJ_EMPTY_KEY ? 0x5bd1e995ULL : h;
 }
-/* pass 3a: first arrival index per (device, stream key).  Millions of rows share a few hundred
- * pairs, so each workgroup first reduces its rows in an LDS table and touches the global table
- * once per pair. */
+/* Rows still without a stream take their queue's; then the first arrival index per (device, stream key).
+ * Millions of rows share a few hundred pairs, so each workgroup first reduces its rows in an LDS table
+ * and touches the global table once per pair.  The workgroup that ends last gives every pair its number:
+ * 1 + number of pairs of the same device seen earlier. */
 #define DENSE_LOCAL_SLOTS 1024u
-__global__ void k_dense_first(const DevBrief* d, uint64_t n, Columns c, uint64_t first_device, StreamTables t,
-                              Scalars* sc) {
+#define KTJ_DENSE_MAX KTJ_MAX_STREAM_PAIRS
+__device__ __forceinline__ void dense_enter(StreamTables& t, uint64_t h, uint32_t first, int32_t dev, uint64_t key, Scalars* sc) {
+  bool fresh;
+  const uint32_t g = table_insert_fresh(t.d_hash, KTJ_DENSE_CAP - 1u, h, &fresh);
+  if (g == KTJ_NOSLOT) { flag_error(sc, KTJ_DEVERR_STREAMS); return; }
+  if (t.d_first[g] > first) atomicMin(&t.d_first[g], first); /* (an old value that is still in a cache is larger) */
+  if (fresh) { /* two pairs with one hash are told apart when the rows read the table back */
+    agent_store(&t.d_dev[g], dev);
+    t.d_key[g] = key;
+    const uint32_t k = atomicAdd(&sc->n_dense, 1u);
+    if (k < KTJ_DENSE_MAX) agent_store(&t.d_list[k], g); else flag_error(sc, KTJ_DEVERR_STREAMS);
+  }
+}
+__global__ void __launch_bounds__(KTJ_BLOCK)
+k_dense_first(const DevBrief* d, uint64_t n, Columns c, uint64_t first_device, StreamTables t, Scalars* sc) {
   __shared__ unsigned long long l_key[DENSE_LOCAL_SLOTS];
   __shared__ unsigned long long l_pair_key[DENSE_LOCAL_SLOTS];
   __shared__ int32_t l_pair_dev[DENSE_LOCAL_SLOTS];
   __shared__ uint32_t l_min[DENSE_LOCAL_SLOTS];
   if (sc->have_stream_src == 0) return;
+  const bool fill = sc->n_unresolved != 0;
   for (uint32_t k = threadIdx.x; k < DENSE_LOCAL_SLOTS; k += blockDim.x) { l_key[k] = KTJ_EMPTY_KEY; l_min[k] = 0xFFFFFFFFu; }
   __syncthreads();
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) {
     uint64_t key;
     const DevBrief b = d[i];
-    if (!dense_key(b, (uint64_t)c.res[first_device + i], &key)) continue;
+    uint64_t stream = (uint64_t)c.res[first_device + i];
+    if (fill && stream == 0 && is_async_op(b.domain)) {
+      const uint32_t slot = table_find(t.q_keys, KTJ_QUEUE_CAP - 1u, b.queue);
+      if (slot != KTJ_NOSLOT && t.q_amb[slot] == 0 && t.q_stream[slot] != 0) { stream = t.q_stream[slot]; c.res[first_device + i] = (int64_t)stream; }
+    }
+    if (!dense_key(b, stream, &key)) continue;
     const uint64_t h = dense_hash(b.device, key);
     uint32_t slot = (uint32_t)(h >> 20) & (DENSE_LOCAL_SLOTS - 1u);
     bool placed = false;
@@ -1038,60 +965,36 @@ __global__ void k_dense_first(const DevBrief* d, uint64_t n, Columns c, uint64_t
       unsigned long long cur = l_key[slot];
       if (cur == KTJ_EMPTY_KEY) {
         cur = atomicCAS(&l_key[slot], (unsigned long long)KTJ_EMPTY_KEY, (unsigned long long)h);
-        /* the pair itself, for the table entry: every row of the pair would write the same two values
-         * (two pairs with one hash are told apart when the rows read the table back) */
+        /* the pair itself, for the table entry: every row of the pair would write the same two values */
         if (cur == KTJ_EMPTY_KEY) { l_pair_dev[slot] = b.device; l_pair_key[slot] = key; }
       }
       if (cur == KTJ_EMPTY_KEY || cur == h) { atomicMin(&l_min[slot], (uint32_t)i); placed = true; }
       else slot = (slot + 1u) & (DENSE_LOCAL_SLOTS - 1u);
     }
-    if (!placed) { /* local table crowded: straight to the global one */
-      const uint32_t g = table_insert(t.d_hash, KTJ_DENSE_CAP - 1u, h);
-      if (g == KTJ_NOSLOT) flag_error(sc, KTJ_DEVERR_STREAMS);
-      else {
-        if (t.d_first[g] > (uint32_t)i) atomicMin(&t.d_first[g], (uint32_t)i);
-        t.d_dev[g] = b.device; t.d_key[g] = key;
-      }
-    }
+    if (!placed) dense_enter(t, h, (uint32_t)i, b.device, key, sc); /* local table crowded: straight to the global one */
   }
   __syncthreads();
-  for (uint32_t k = threadIdx.x; k < DENSE_LOCAL_SLOTS; k += blockDim.x) {
-    const unsigned long long h = l_key[k];
-    if (h == KTJ_EMPTY_KEY) continue;
-    const uint32_t g = table_insert(t.d_hash, KTJ_DENSE_CAP - 1u, h);
-    if (g == KTJ_NOSLOT) { flag_error(sc, KTJ_DEVERR_STREAMS); continue; }
-    if (t.d_first[g] > l_min[k]) atomicMin(&t.d_first[g], l_min[k]);
-    t.d_dev[g] = l_pair_dev[k]; t.d_key[g] = l_pair_key[k];
-  }
-}
-/* pass 3b (one workgroup): index = 1 + number of pairs of the same device seen earlier */
-#define KTJ_DENSE_MAX KTJ_MAX_STREAM_PAIRS
-__global__ void k_dense_rank(StreamTables t, Scalars* sc) {
-  __shared__ uint32_t slots[KTJ_DENSE_MAX];
-  __shared__ uint32_t count;
-  if (sc->have_stream_src == 0) return;
-  if (threadIdx.x == 0) count = 0;
-  __syncthreads();
-  for (uint32_t s = threadIdx.x; s <= KTJ_DENSE_CAP; s += blockDim.x) {
-    if (t.d_hash[s] != KTJ_EMPTY_KEY && t.d_first[s] != 0xFFFFFFFFu) {
-      const uint32_t k = atomicAdd(&count, 1u);
-      if (k < KTJ_DENSE_MAX) slots[k] = s;
-    }
-  }
-  __syncthreads();
-  const uint32_t m = count;
-  if (m > KTJ_DENSE_MAX) { if (threadIdx.x == 0) flag_error(sc, KTJ_DEVERR_STREAMS); return; }
-  if (threadIdx.x == 0) sc->n_dense = m;
-  for (uint32_t k = threadIdx.x; k < m; k += blockDim.x) {
-    const uint32_t s = slots[k];
-    const int32_t dev = t.d_dev[s];
-    const uint32_t first = t.d_first[s];
+  for (uint32_t k = threadIdx.x; k < DENSE_LOCAL_SLOTS; k += blockDim.x)
+    if (l_key[k] != KTJ_EMPTY_KEY) dense_enter(t, l_key[k], l_min[k], l_pair_dev[k], l_pair_key[k], sc);
+  if (!last_workgroup(&sc->done[KTJ_DONE_DENSE])) return;
+  const uint32_t n_pairs = agent_load(&sc->n_dense), m = n_pairs < KTJ_DENSE_MAX ? n_pairs : KTJ_DENSE_MAX;
+  unsigned long long* l_pair = l_key; /* device and first row of a chunk of the pairs */
+  for (uint32_t p0 = 0; p0 < m; p0 += KTJ_BLOCK) { /* every thread one pair of this round, against all of them */
+    const uint32_t p = p0 + threadIdx.x;
+    const uint32_t s = p < m ? agent_load(&t.d_list[p]) : 0u;
+    const uint32_t dev = p < m ? (uint32_t)agent_load(&t.d_dev[s]) : 0u, first = p < m ? agent_load(&t.d_first[s]) : 0u;
     uint32_t rank = 1;
-    for (uint32_t j = 0; j < m; ++j) {
-      const uint32_t o = slots[j];
-      if (t.d_dev[o] == dev && t.d_first[o] < first) ++rank;
+    for (uint32_t q0 = 0; q0 < m; q0 += DENSE_LOCAL_SLOTS) {
+      const uint32_t here = m - q0 < DENSE_LOCAL_SLOTS ? m - q0 : DENSE_LOCAL_SLOTS;
+      __syncthreads();
+      for (uint32_t q = threadIdx.x; q < here; q += KTJ_BLOCK) {
+        const uint32_t o = agent_load(&t.d_list[q0 + q]);
+        l_pair[q] = ((unsigned long long)(uint32_t)agent_load(&t.d_dev[o]) << 32) | agent_load(&t.d_first[o]);
+      }
+      __syncthreads();
+      for (uint32_t q = 0; q < here; ++q) rank += (uint32_t)(l_pair[q] >> 32) == dev && (uint32_t)l_pair[q] < first ? 1u : 0u;
     }
-    t.d_rank[s] = rank;
+    if (p < m) t.d_rank[s] = rank;
   }
 }
 /* pass 3c: resourceId() = stream != 0 ? stream : queue (RocprofActivity.h:100-102) */
@@ -1115,14 +1018,16 @@ __global__ void k_dense_assign(const DevBrief* d, uint64_t n, Columns c, uint64_
   c.res[a] = (int64_t)(stream != 0 ? stream : b.queue);
 }
 
-hipError_t backfill_streams(const DevBrief* d, uint64_t n, Columns c, uint64_t first_device, StreamTables t,
-                            Scalars* sc, hipStream_t st) {
+hipError_t backfill_streams(const DevBrief* d, uint64_t n, Columns c, uint64_t first_device, Table tf, FullCols fc, const DevLink* link,
+                            StreamTables t, Scalars* sc, hipStream_t st) {
   if (n == 0) return hipSuccess;
   const dim3 g(grid_for(n, KTJ_BLOCK)), b(KTJ_BLOCK);
-  hipLaunchKernelGGL(k_queue_build, g, b, 0, st, d, n, c, first_device, t, sc);
-  hipLaunchKernelGGL(k_queue_fill, g, b, 0, st, d, n, c, first_device, t, (const Scalars*)sc);
-  hipLaunchKernelGGL(k_dense_first, dim3(grid_stride_for(n, KTJ_BLOCK * 8)), b, 0, st, d, n, c, first_device, t, sc);
-  hipLaunchKernelGGL(k_dense_rank, dim3(1), dim3(1024), 0, st, t, sc);
+  hipLaunchKernelGGL(k_after_link, dim3(grid_stride_for(n, KTJ_BLOCK)), b, 0, st, n, c, first_device, tf, fc, link, d, t, sc);
+  /* every workgroup pays for its local table and for each pair it has seen: 2048 rows each, fewer only while
+   * that leaves CUs without a workgroup, and at most four workgroups per CU */
+  const unsigned few = grid_stride_for(n, KTJ_BLOCK * 2), many = grid_stride_for(n, KTJ_BLOCK * 8);
+  const unsigned gd = many > 1024u ? 1024u : many > 256u ? many : few > 256u ? 256u : few;
+  hipLaunchKernelGGL(k_dense_first, dim3(gd), b, 0, st, d, n, c, first_device, t, sc);
   hipLaunchKernelGGL(k_dense_assign, g, b, 0, st, d, n, c, first_device, t, sc);
   return KTJ_LAUNCH_CHECK();
 }
@@ -1135,7 +1040,8 @@ hipError_t backfill_streams(const DevBrief* d, uint64_t n, Columns c, uint64_t f
  * millions of probes of the same few global slots serialise in L2.)  Returns true when the
  * caller is the first in its workgroup to see the key, or when the local set is full. */
 #define LOCAL_SET_SLOTS 1024u
-__device__ __forceinline__ bool local_set_first(unsigned long long* lds, uint64_t key) {
+__device__ __forceinline__ bool local_set_first(unsigned long long* lds /* LOCAL_SET_SLOTS + 1 */, uint64_t key) {
+  if (key == KTJ_EMPTY_KEY) return lds[LOCAL_SET_SLOTS] != 0 && atomicExch(&lds[LOCAL_SET_SLOTS], 0ULL) != 0;
   const uint32_t h = ((uint32_t)key ^ ((uint32_t)(key >> 32) * 0x9E3779B1u)) * 0x85EBCA6Bu;
   uint32_t slot = h >> 22; /* 10 bits */
   for (uint32_t probe = 0; probe < 16; ++probe) {
@@ -1150,21 +1056,45 @@ __device__ __forceinline__ bool local_set_first(unsigned long long* lds, uint64_
   }
   return true;
 }
-/* a wavefront's rows mostly share one value: only one lane of those that hold the value of the
- * first active lane goes on to probe, and lanes with another value probe for themselves */
-__device__ __forceinline__ bool wave_representative(uint64_t v) {
-  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-  const uint64_t first = ((uint64_t)hi << 32) | lo;
-  const uint64_t same = __ballot(v == first); /* never empty: the first active lane is in it */
-  return v != first || (uint32_t)__builtin_ctzll(same) == lane_id();
-}
 #define COLLECT_ROWS 4
-__global__ void k_collect_distinct(Columns c, uint64_t n, SortSets s, Scalars* sc) {
+__device__ __forceinline__ void set_enter(uint64_t* keys, uint32_t* list, unsigned int* count, uint64_t v, Scalars* sc, unsigned too_many) {
+  bool fresh;
+  const uint32_t g = table_insert_fresh(keys, KTJ_SET_CAP - 1u, v, &fresh);
+  if (g == KTJ_NOSLOT) { flag_error(sc, too_many); return; }
+  if (fresh) {
+    const uint32_t k = atomicAdd(count, 1u);
+    if (k < KTJ_SET_MAX) agent_store(&list[k], g); else flag_error(sc, too_many);
+  }
+}
+/* by one workgroup: rank of each distinct value = number of smaller values (signed) */
+__device__ void rank_values(const uint64_t* keys, const uint32_t* list, uint32_t* rank, uint32_t m, int64_t* lds /* LOCAL_SET_SLOTS */) {
+  auto value = [&](uint32_t slot) { return slot < KTJ_SET_CAP ? (int64_t)agent_load(&keys[slot]) : (int64_t)-1; };
+  for (uint32_t p0 = 0; p0 < m; p0 += KTJ_BLOCK) {
+    const uint32_t p = p0 + threadIdx.x;
+    const uint32_t s = p < m ? agent_load(&list[p]) : 0u;
+    const int64_t v = p < m ? value(s) : 0;
+    uint32_t r = 0;
+    for (uint32_t q0 = 0; q0 < m; q0 += LOCAL_SET_SLOTS) {
+      const uint32_t here = m - q0 < LOCAL_SET_SLOTS ? m - q0 : LOCAL_SET_SLOTS;
+      __syncthreads();
+      for (uint32_t q = threadIdx.x; q < here; q += KTJ_BLOCK) lds[q] = value(agent_load(&list[q0 + q]));
+      __syncthreads();
+      for (uint32_t q = 0; q < here; ++q) r += lds[q] < v ? 1u : 0u;
+    }
+    if (p < m) rank[s] = r;
+  }
+}
+/* Distinct deviceId and resourceId values, the range of the timestamps and the number of rows that are
+ * printed.  The workgroup that ends last ranks the values and plans the sort's keys. */
+__global__ void __launch_bounds__(KTJ_BLOCK) k_collect_distinct(Columns c, uint64_t n, SortSets s, Scalars* sc, int straight) {
   __shared__ uint64_t red_min[KTJ_BLOCK >> 6], red_max[KTJ_BLOCK >> 6];
-  __shared__ unsigned long long seen_dev[LOCAL_SET_SLOTS], seen_res[LOCAL_SET_SLOTS];
-  for (uint32_t k = threadIdx.x; k < LOCAL_SET_SLOTS; k += blockDim.x) { seen_dev[k] = KTJ_EMPTY_KEY; seen_res[k] = KTJ_EMPTY_KEY; }
+  __shared__ unsigned long long seen[2][LOCAL_SET_SLOTS + 1]; /* deviceId, resourceId values */
+  if (blockIdx.x == 0 && threadIdx.x == 0) stage_clock(sc, KTJ_CLOCK_SORT);
+  for (uint32_t k = threadIdx.x; k <= LOCAL_SET_SLOTS; k += blockDim.x) { seen[0][k] = KTJ_EMPTY_KEY; seen[1][k] = KTJ_EMPTY_KEY; }
   __syncthreads();
   uint64_t mn = ~0ULL, mx = 0ULL;
+  uint64_t last_dev = 0, last_res = 0; /* of the thread's rows so far: most rows repeat them */
+  bool any = false;
   uint32_t n_valid = 0;
   const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
   for (uint64_t a0 = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; a0 < n; a0 += stride * COLLECT_ROWS) {
@@ -1179,19 +1109,27 @@ __global__ void k_collect_distinct(Columns c, uint64_t n, SortSets s, Scalars* s
       res[r] = in ? (uint64_t)c.res[a] : 0;
       ts[r] = in ? (uint64_t)c.ts[a] : 0;
     }
+    uint32_t todo = 0;
 #pragma unroll
     for (int r = 0; r < COLLECT_ROWS; ++r) {
       if (!(meta[r] & KTJ_M_VALID)) continue;
-      if (wave_representative(dev[r]) && (dev[r] == KTJ_EMPTY_KEY || local_set_first(seen_dev, dev[r]))) {
-        if (table_insert(s.dev_keys, KTJ_SET_CAP - 1u, dev[r]) == KTJ_NOSLOT) flag_error(sc, KTJ_DEVERR_DISTINCT_DEVICES);
-      }
-      if (wave_representative(res[r]) && (res[r] == KTJ_EMPTY_KEY || local_set_first(seen_res, res[r]))) {
-        if (table_insert(s.res_keys, KTJ_SET_CAP - 1u, res[r]) == KTJ_NOSLOT) flag_error(sc, KTJ_DEVERR_DISTINCT_RESOURCES);
-      }
+      todo |= (!any || dev[r] != last_dev ? 1u : 0u) << r | (!any || res[r] != last_res ? 1u : 0u) << (COLLECT_ROWS + r);
+      last_dev = dev[r]; last_res = res[r];
+      any = true;
       const uint64_t tb = ts[r] ^ 0x8000000000000000ULL;
       mn = tb < mn ? tb : mn;
       mx = tb > mx ? tb : mx;
       ++n_valid;
+    }
+    while (todo) { /* one copy of the probing for all rows and both sets (unrolled it spilled 358 scalar registers) */
+      const uint32_t at = (uint32_t)__builtin_ctz(todo), is_res = at / COLLECT_ROWS;
+      todo &= todo - 1u;
+      uint64_t v = dev[0];
+#pragma unroll
+      for (uint32_t r = 1; r < 2 * COLLECT_ROWS; ++r) v = at == r ? (r < COLLECT_ROWS ? dev[r] : res[r - COLLECT_ROWS]) : v;
+      if (!local_set_first(seen[is_res], v)) continue;
+      set_enter(is_res ? s.res_keys : s.dev_keys, is_res ? s.res_list : s.dev_list, is_res ? &sc->n_res_ranks : &sc->n_dev_ranks, v, sc,
+                is_res ? KTJ_DEVERR_DISTINCT_RESOURCES : KTJ_DEVERR_DISTINCT_DEVICES);
     }
   }
   for (int o = 32; o > 0; o >>= 1) {
@@ -1212,35 +1150,22 @@ __global__ void k_collect_distinct(Columns c, uint64_t n, SortSets s, Scalars* s
     }
   }
   block_add(sc, KTJ_CNT_VALID, n_valid);
-}
-/* one workgroup per set: rank of each distinct value = number of smaller values (signed) */
-__global__ void k_rank_distinct(SortSets s, Scalars* sc) {
-  __shared__ int64_t vals[KTJ_SET_MAX];
-  __shared__ uint32_t slots[KTJ_SET_MAX];
-  __shared__ uint32_t count;
-  uint64_t* keys = blockIdx.x == 0 ? s.dev_keys : s.res_keys;
-  uint32_t* rank = blockIdx.x == 0 ? s.dev_rank : s.res_rank;
-  if (threadIdx.x == 0) count = 0;
-  __syncthreads();
-  for (uint32_t k = threadIdx.x; k <= KTJ_SET_CAP; k += blockDim.x) {
-    bool occupied = k < KTJ_SET_CAP ? keys[k] != KTJ_EMPTY_KEY : keys[k] == 0;
-    if (occupied) {
-      const uint32_t j = atomicAdd(&count, 1u);
-      if (j < KTJ_SET_MAX) { slots[j] = k; vals[j] = k < KTJ_SET_CAP ? (int64_t)keys[k] : (int64_t)-1; }
-    }
-  }
-  __syncthreads();
-  const uint32_t m = count;
-  if (m > KTJ_SET_MAX) {
-    if (threadIdx.x == 0) flag_error(sc, blockIdx.x == 0 ? KTJ_DEVERR_DISTINCT_DEVICES : KTJ_DEVERR_DISTINCT_RESOURCES);
-    return;
-  }
-  if (threadIdx.x == 0) { if (blockIdx.x == 0) sc->n_dev_ranks = m; else sc->n_res_ranks = m; }
-  for (uint32_t k = threadIdx.x; k < m; k += blockDim.x) {
-    const int64_t v = vals[k];
-    uint32_t r = 0;
-    for (uint32_t j = 0; j < m; ++j) r += vals[j] < v ? 1u : 0u;
-    rank[slots[k]] = r;
+  if (!last_workgroup(&sc->done[KTJ_DONE_COLLECT])) return;
+  const uint32_t nd = agent_load(&sc->n_dev_ranks), nr = agent_load(&sc->n_res_ranks);
+  const uint32_t md = nd < KTJ_SET_MAX ? nd : KTJ_SET_MAX, mr = nr < KTJ_SET_MAX ? nr : KTJ_SET_MAX;
+  rank_values(s.dev_keys, s.dev_list, s.dev_rank, md, reinterpret_cast<int64_t*>(seen[0]));
+  rank_values(s.res_keys, s.res_list, s.res_rank, mr, reinterpret_cast<int64_t*>(seen[0]));
+  if (threadIdx.x == 0) {
+    const uint64_t lo = agent_load(&sc->ts_min_biased), hi = agent_load(&sc->ts_max_biased), span = lo <= hi ? hi - lo : 0;
+    auto bits = [](uint64_t v) -> uint32_t { return v ? 64u - (uint32_t)__builtin_clzll(v) : 0u; }; /* to hold 0..v */
+    SortPlan p;
+    p.ts_bits = bits(span);
+    p.res_bits = bits(mr ? mr - 1u : 0u);
+    p.key_bits = p.ts_bits + p.res_bits + bits(md ? md - 1u : 0u);
+    sc->sort = p;
+    unsigned long long sync_typed = 0; /* the order decides which of them announces its row */
+    for (uint32_t k = 0; k < KTJ_COUNTER_SHARDS; ++k) sync_typed += sc->shard[k][KTJ_CNT_SYNC_TYPED];
+    if (straight && sync_typed) flag_error(sc, KTJ_DEVERR_CAREFUL);
   }
 }
 /* Rank of a value through its set.  The rows of a wavefront mostly share one value: then a single
@@ -1349,7 +1274,7 @@ hipError_t make_rank_keys(Columns c, const uint32_t* order, uint64_t n, SortSets
   return KTJ_LAUNCH_CHECK();
 }
 
-hipError_t collect_distinct(Columns c, uint64_t n, SortSets s, Scalars* sc, hipStream_t st) {
+hipError_t collect_distinct(Columns c, uint64_t n, SortSets s, Scalars* sc, bool straight, hipStream_t st) {
   if (n == 0) return hipSuccess;
   /* few, fat workgroups: each one pays for its own local set once (few rows: one group each) */
   /* at most four workgroups per CU: every workgroup pays for its local sets and its atomics at the
@@ -1357,11 +1282,7 @@ hipError_t collect_distinct(Columns c, uint64_t n, SortSets s, Scalars* sc, hipS
    * 1024: 0.17 ms) */
   unsigned g = grid_stride_for(n, n < (1u << 20) ? KTJ_BLOCK * COLLECT_ROWS : KTJ_BLOCK * 16);
   if (g > 1024u) g = 1024u;
-  hipLaunchKernelGGL(k_collect_distinct, dim3(g), dim3(KTJ_BLOCK), 0, st, c, n, s, sc);
-  return KTJ_LAUNCH_CHECK();
-}
-hipError_t rank_distinct(SortSets s, Scalars* sc, hipStream_t st) {
-  hipLaunchKernelGGL(k_rank_distinct, dim3(2), dim3(1024), 0, st, s, sc);
+  hipLaunchKernelGGL(k_collect_distinct, dim3(g), dim3(KTJ_BLOCK), 0, st, c, n, s, sc, straight ? 1 : 0);
   return KTJ_LAUNCH_CHECK();
 }
 hipError_t make_keys(Columns c, uint64_t n, SortSets s, const Scalars* sc, uint32_t ts_bits, uint32_t res_bits,
@@ -1511,7 +1432,16 @@ hipError_t radix_sort(uint64_t* keys_a, uint32_t* vals_a, uint64_t* keys_b, uint
  * the remaining key bits above the index: word = (key >> BITS) << idx_bits | index.  Later passes
  * take their digit from the word; the last one writes the bare indices.  The per-tile digit
  * counts of the first pass come from the kernel that builds the keys. */
-enum { SORTP_KEYS_TO_WORDS = 0, SORTP_WORDS_TO_WORDS = 1, SORTP_WORDS_TO_PERM = 2, SORTP_KEYS_TO_PERM = 3 };
+/* How many passes there are is the plan that k_collect_distinct leaves on the device: the host launches as
+ * many as it expects, those beyond the plan end at once, and a plan beyond them (or one that does not fit
+ * a word) is flagged for the host to take the pass again, looking at the plan (KTJ_DEVERR_CAREFUL). */
+#define SORTP_BITS 8
+__device__ __forceinline__ uint32_t sort_passes(const Scalars* sc) { return (sc->sort.key_bits + SORTP_BITS) / SORTP_BITS; } /* key and dropped bit */
+__device__ __forceinline__ bool sort_pass_idle(const Scalars* sc, uint32_t pass) { return sc->error != 0 || pass >= sort_passes(sc); }
+__device__ __forceinline__ bool sort_words_suffice(const Scalars* sc, uint32_t key_bits, uint32_t idx_bits, uint32_t passes_launched) {
+  return sc->error == 0 && key_bits <= 62u && (key_bits + 1u > SORTP_BITS ? key_bits + 1u - SORTP_BITS : 0u) + idx_bits <= 64u &&
+         (key_bits + SORTP_BITS) / SORTP_BITS <= passes_launched;
+}
 template <int BITS, int THREADS, int ITEMS_> struct SortP {
   static constexpr int NB = 1 << BITS;
   static constexpr int WAVES = THREADS / 64;
@@ -1523,9 +1453,14 @@ template <int BITS, int THREADS, int ITEMS_> struct SortP {
 
 template <int BITS, int THREADS, int ITEMS>
 __global__ void __launch_bounds__(THREADS)
-k_sortp_make_keys(Columns c, uint64_t n, SortSets s, const Scalars* sc, uint32_t ts_bits, uint32_t res_bits, uint32_t key_bits,
-                  uint64_t* keys, uint32_t* hist, uint32_t n_blocks) {
+k_sortp_make_keys(Columns c, uint64_t n, SortSets s, Scalars* sc, uint32_t idx_bits, uint32_t passes_launched, uint64_t* keys, uint32_t* hist,
+                  uint32_t n_blocks) {
   using P = SortP<BITS, THREADS, ITEMS>;
+  const uint32_t ts_bits = sc->sort.ts_bits, res_bits = sc->sort.res_bits, key_bits = sc->sort.key_bits;
+  if (!sort_words_suffice(sc, key_bits, idx_bits, passes_launched)) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) flag_error(sc, KTJ_DEVERR_CAREFUL);
+    return;
+  }
   __shared__ uint32_t h[P::NB];
   for (int d = threadIdx.x; d < P::NB; d += THREADS) h[d] = 0;
   __syncthreads();
@@ -1566,8 +1501,10 @@ k_sortp_make_keys(Columns c, uint64_t n, SortSets s, const Scalars* sc, uint32_t
 }
 template <int BITS, int THREADS, int ITEMS>
 __global__ void __launch_bounds__(THREADS)
-k_sortp_hist(const uint64_t* words, uint64_t n, uint32_t shift, uint32_t* hist, uint32_t n_blocks) {
+k_sortp_hist(const uint64_t* words, uint64_t n, uint32_t pass, uint32_t idx_bits, const Scalars* sc, uint32_t* hist, uint32_t n_blocks) {
   using P = SortP<BITS, THREADS, ITEMS>;
+  if (sort_pass_idle(sc, pass)) return;
+  const uint32_t shift = idx_bits + (pass - 1u) * BITS;
   __shared__ uint32_t h[P::NB];
   for (int d = threadIdx.x; d < P::NB; d += THREADS) h[d] = 0;
   __syncthreads();
@@ -1586,7 +1523,8 @@ k_sortp_hist(const uint64_t* words, uint64_t n, uint32_t shift, uint32_t* hist, 
  * over 256 totals) are left to every scatter workgroup. */
 template <int THREADS>
 __global__ void __launch_bounds__(THREADS)
-k_sortp_scan_digits(uint32_t* hist, uint32_t n_blocks, uint32_t* totals) {
+k_sortp_scan_digits(uint32_t* hist, uint32_t n_blocks, uint32_t* totals, uint32_t pass, const Scalars* sc) {
+  if (sort_pass_idle(sc, pass)) return;
   __shared__ uint32_t wave_tot[THREADS / 64];
   uint32_t* row = hist + (uint64_t)blockIdx.x * n_blocks;
   const uint32_t per = (n_blocks + THREADS - 1) / THREADS;
@@ -1606,13 +1544,14 @@ k_sortp_scan_digits(uint32_t* hist, uint32_t n_blocks, uint32_t* totals) {
   if (threadIdx.x == 0) totals[blockIdx.x] = all;
 }
 
-template <int BITS, int THREADS, int ITEMS, int MODE>
+template <int BITS, int THREADS, int ITEMS, bool FROM_KEYS>
 __global__ void __launch_bounds__(THREADS)
-k_sortp_scatter(const uint64_t* in, uint64_t* words_out, uint32_t* perm_out, uint64_t n, uint32_t shift, uint32_t idx_bits,
+k_sortp_scatter(const uint64_t* in, uint64_t* words_out, uint32_t* perm_out, uint64_t n, uint32_t pass, uint32_t idx_bits, const Scalars* sc,
                 const uint32_t* hist_scanned, const uint32_t* totals, uint32_t n_blocks) {
   using P = SortP<BITS, THREADS, ITEMS>;
-  constexpr bool FROM_KEYS = MODE == SORTP_KEYS_TO_WORDS || MODE == SORTP_KEYS_TO_PERM;
-  constexpr bool TO_PERM = MODE == SORTP_WORDS_TO_PERM || MODE == SORTP_KEYS_TO_PERM;
+  if (sort_pass_idle(sc, pass)) return;
+  const bool TO_PERM = pass + 1u == sort_passes(sc);
+  const uint32_t shift = FROM_KEYS ? 0u : idx_bits + (pass - 1u) * BITS;
   __shared__ uint64_t s_word[P::TILE];
   __shared__ uint16_t s_digit[FROM_KEYS ? P::TILE : 1]; /* the first pass's digit is no longer part of the word */
   __shared__ uint32_t wave_run[P::WAVES][P::NB]; /* count per (wavefront, digit), then its start inside the digit's run */
@@ -1672,7 +1611,7 @@ k_sortp_scatter(const uint64_t* in, uint64_t* words_out, uint32_t* perm_out, uin
     uint32_t digit;
     if (FROM_KEYS) {
       digit = (uint32_t)word[r] & (P::NB - 1u);
-      word[r] = (MODE == SORTP_KEYS_TO_PERM) ? i : ((((word[r] >> BITS)) << idx_bits) | i);
+      word[r] = (((word[r] >> BITS)) << idx_bits) | i;
     } else {
       digit = (uint32_t)(word[r] >> shift) & (P::NB - 1u);
     }
@@ -1747,9 +1686,13 @@ k_sortp_scatter(const uint64_t* in, uint64_t* words_out, uint32_t* perm_out, uin
  * where every thread takes the keys of its positions for the next pass. */
 template <int BITS, int THREADS, int ITEMS>
 __global__ void __launch_bounds__(THREADS)
-k_sortp_single(Columns c, uint32_t n, SortSets s, const Scalars* sc, uint32_t ts_bits, uint32_t res_bits, uint32_t key_bits,
-               uint32_t* perm_out) {
+k_sortp_single(Columns c, uint32_t n, SortSets s, Scalars* sc, uint32_t* perm_out) {
   using P = SortP<BITS, THREADS, ITEMS>;
+  const uint32_t ts_bits = sc->sort.ts_bits, res_bits = sc->sort.res_bits, key_bits = sc->sort.key_bits;
+  if (!sort_words_suffice(sc, key_bits, 0u, 64u)) { /* key and index are kept apart here */
+    if (threadIdx.x == 0) flag_error(sc, KTJ_DEVERR_CAREFUL);
+    return;
+  }
   __shared__ uint64_t s_key[P::TILE];
   __shared__ uint16_t s_idx[P::TILE];
   __shared__ uint32_t wave_run[P::WAVES][P::NB];
@@ -1842,13 +1785,10 @@ k_sortp_single(Columns c, uint32_t n, SortSets s, const Scalars* sc, uint32_t ts
 }
 
 template <int BITS, int THREADS, int ITEMS>
-static hipError_t sort_packed_t(Columns c, uint64_t n, SortSets s, const Scalars* sc, uint32_t ts_bits, uint32_t res_bits,
-                                uint32_t key_bits, uint32_t idx_bits, uint64_t* buf_a, uint64_t* buf_b, uint32_t* perm,
-                                uint32_t* hist, uint64_t* scan_tmp, hipStream_t st) {
+static hipError_t sort_packed_t(Columns c, uint64_t n, SortSets s, Scalars* sc, uint32_t passes, uint32_t idx_bits, uint64_t* buf_a, uint64_t* buf_b,
+                                uint32_t* perm, uint32_t* hist, hipStream_t st) {
   using P = SortP<BITS, THREADS, ITEMS>;
   const uint32_t n_blocks = (uint32_t)((n + P::TILE - 1) / P::TILE);
-  const uint32_t total_bits = key_bits + 1u;
-  const uint32_t passes = (total_bits + BITS - 1) / BITS;
   const dim3 g(n_blocks), b(THREADS);
   /* one tile: a pass needs no counts from other tiles, so no count and scan launches */
   const bool single = n_blocks == 1;
@@ -1856,62 +1796,47 @@ static hipError_t sort_packed_t(Columns c, uint64_t n, SortSets s, const Scalars
   /* the digits' totals live behind the counts (radix_tmp_elems leaves 256 spare entries) */
   uint32_t* totals = hist + (uint64_t)P::NB * n_blocks;
   static_assert(P::NB <= 256, "room for the totals behind the counts");
-  (void)scan_tmp;
-  hipLaunchKernelGGL((k_sortp_make_keys<BITS, THREADS, ITEMS>), g, b, 0, st, c, n, s, sc, ts_bits, res_bits, key_bits, buf_a, counts, n_blocks);
-  if (!single) hipLaunchKernelGGL((k_sortp_scan_digits<THREADS>), dim3(P::NB), b, 0, st, hist, n_blocks, totals);
-  if (passes == 1) {
-    hipLaunchKernelGGL((k_sortp_scatter<BITS, THREADS, ITEMS, SORTP_KEYS_TO_PERM>), g, b, 0, st, (const uint64_t*)buf_a, buf_b, perm, n,
-                       0u, idx_bits, (const uint32_t*)counts, (const uint32_t*)totals, n_blocks);
-    return KTJ_LAUNCH_CHECK();
-  }
-  hipLaunchKernelGGL((k_sortp_scatter<BITS, THREADS, ITEMS, SORTP_KEYS_TO_WORDS>), g, b, 0, st, (const uint64_t*)buf_a, buf_b, perm, n,
-                     0u, idx_bits, (const uint32_t*)counts, (const uint32_t*)totals, n_blocks);
+  hipLaunchKernelGGL((k_sortp_make_keys<BITS, THREADS, ITEMS>), g, b, 0, st, c, n, s, sc, idx_bits, passes, buf_a, counts, n_blocks);
+  if (!single) hipLaunchKernelGGL((k_sortp_scan_digits<THREADS>), dim3(P::NB), b, 0, st, hist, n_blocks, totals, 0u, (const Scalars*)sc);
+  hipLaunchKernelGGL((k_sortp_scatter<BITS, THREADS, ITEMS, true>), g, b, 0, st, (const uint64_t*)buf_a, buf_b, perm, n, 0u, idx_bits,
+                     (const Scalars*)sc, (const uint32_t*)counts, (const uint32_t*)totals, n_blocks);
   uint64_t* in = buf_b; uint64_t* out = buf_a;
   for (uint32_t p = 1; p < passes; ++p) {
-    const uint32_t shift = idx_bits + (p - 1u) * BITS;
     if (!single) {
-      hipLaunchKernelGGL((k_sortp_hist<BITS, THREADS, ITEMS>), g, b, 0, st, (const uint64_t*)in, n, shift, hist, n_blocks);
-      hipLaunchKernelGGL((k_sortp_scan_digits<THREADS>), dim3(P::NB), b, 0, st, hist, n_blocks, totals);
+      hipLaunchKernelGGL((k_sortp_hist<BITS, THREADS, ITEMS>), g, b, 0, st, (const uint64_t*)in, n, p, idx_bits, (const Scalars*)sc, hist, n_blocks);
+      hipLaunchKernelGGL((k_sortp_scan_digits<THREADS>), dim3(P::NB), b, 0, st, hist, n_blocks, totals, p, (const Scalars*)sc);
     }
-    if (p + 1 == passes)
-      hipLaunchKernelGGL((k_sortp_scatter<BITS, THREADS, ITEMS, SORTP_WORDS_TO_PERM>), g, b, 0, st, (const uint64_t*)in, out, perm, n,
-                         shift, idx_bits, (const uint32_t*)counts, (const uint32_t*)totals, n_blocks);
-    else
-      hipLaunchKernelGGL((k_sortp_scatter<BITS, THREADS, ITEMS, SORTP_WORDS_TO_WORDS>), g, b, 0, st, (const uint64_t*)in, out, perm, n,
-                         shift, idx_bits, (const uint32_t*)counts, (const uint32_t*)totals, n_blocks);
+    hipLaunchKernelGGL((k_sortp_scatter<BITS, THREADS, ITEMS, false>), g, b, 0, st, (const uint64_t*)in, out, perm, n, p, idx_bits,
+                       (const Scalars*)sc, (const uint32_t*)counts, (const uint32_t*)totals, n_blocks);
     uint64_t* t = in; in = out; out = t;
   }
   return KTJ_LAUNCH_CHECK();
 }
-#define SORTP_BITS 8
 #define SORTP_THREADS 256
 /* tests: the one-launch sort of a single tile switched off, so that such a trace takes the passes of a large one */
 static bool g_sortp_no_single = false;
 void sort_packed_force_passes(bool on) { g_sortp_no_single = on; }
 bool sort_packed_passes_forced() { return g_sortp_no_single; }
+static uint32_t sort_idx_bits(uint64_t n) { return (uint32_t)(64 - __builtin_clzll(n > 1 ? n - 1 : 1)); }
 bool sort_packed_fits(uint64_t n, uint32_t key_bits) {
   const uint32_t total_bits = key_bits + 1u;
-  const uint32_t idx_bits = (uint32_t)(64 - __builtin_clzll(n > 1 ? n - 1 : 1));
-  return (total_bits > SORTP_BITS ? total_bits - SORTP_BITS : 0u) + idx_bits <= 64u;
+  return (total_bits > SORTP_BITS ? total_bits - SORTP_BITS : 0u) + sort_idx_bits(n) <= 64u;
 }
-hipError_t sort_packed(Columns c, uint64_t n, SortSets s, const Scalars* sc, uint32_t ts_bits, uint32_t res_bits,
-                       uint32_t key_bits, uint64_t* buf_a, uint64_t* buf_b, uint32_t* perm, uint32_t* hist, uint64_t* scan_tmp,
-                       hipStream_t st) {
+uint32_t sort_packed_passes(uint32_t key_bits) { return (key_bits + SORTP_BITS) / SORTP_BITS; }
+hipError_t sort_packed(Columns c, uint64_t n, SortSets s, Scalars* sc, uint32_t passes, uint64_t* buf_a, uint64_t* buf_b, uint32_t* perm,
+                       uint32_t* hist, hipStream_t st) {
   if (n == 0) return hipSuccess;
-  const uint32_t idx_bits = (uint32_t)(64 - __builtin_clzll(n > 1 ? n - 1 : 1));
+  const uint32_t idx_bits = sort_idx_bits(n);
   if (n <= (uint64_t)SORTP_THREADS * 16u && !g_sortp_no_single) {
-    hipLaunchKernelGGL((k_sortp_single<SORTP_BITS, SORTP_THREADS, 16>), dim3(1), dim3(SORTP_THREADS), 0, st, c, (uint32_t)n, s, sc, ts_bits,
-                       res_bits, key_bits, perm);
+    hipLaunchKernelGGL((k_sortp_single<SORTP_BITS, SORTP_THREADS, 16>), dim3(1), dim3(SORTP_THREADS), 0, st, c, (uint32_t)n, s, sc, perm);
     return KTJ_LAUNCH_CHECK();
   }
   /* a few thousand keys are one tile; up to SORTP_SMALL_N keys, tiles of 512 spread over the GPU
    * finish a pass sooner than the few 4096-key tiles would (30 000 keys: 76 against 130 us for the
    * sort, 330 000 keys: 113 against 155 us; from a million keys on the large tiles win) */
   if (n > (uint64_t)SORTP_THREADS * 16u && n < SORTP_SMALL_N)
-    return sort_packed_t<SORTP_BITS, SORTP_THREADS, 2>(c, n, s, sc, ts_bits, res_bits, key_bits, idx_bits, buf_a, buf_b, perm, hist,
-                                                       scan_tmp, st);
-  return sort_packed_t<SORTP_BITS, SORTP_THREADS, 16>(c, n, s, sc, ts_bits, res_bits, key_bits, idx_bits, buf_a, buf_b, perm, hist,
-                                                      scan_tmp, st);
+    return sort_packed_t<SORTP_BITS, SORTP_THREADS, 2>(c, n, s, sc, passes, idx_bits, buf_a, buf_b, perm, hist, st);
+  return sort_packed_t<SORTP_BITS, SORTP_THREADS, 16>(c, n, s, sc, passes, idx_bits, buf_a, buf_b, perm, hist, st);
 }
 
 /* ------------------------------------------------------------------------------------------ */
@@ -2016,13 +1941,11 @@ hipError_t stream_sync_first(const uint32_t* perm, uint64_t n_sorted, const ktj_
   return KTJ_LAUNCH_CHECK();
 }
 
-__global__ void k_mat_generic(const ktj_generic_rec* g, uint64_t n, uint64_t first, EmitCtx ctx, const uint32_t* sync_first,
-                              MatRow* mat, uint32_t* len, Scalars* sc) {
-  static_assert(sizeof(MatRow) >= sizeof(ktj_generic_rec), "the staging area holds the records, then the joined rows");
-  __shared__ uint4 stage[KTJ_BLOCK * sizeof(MatRow) / 16];
+__device__ __forceinline__ void mat_generic_block(const ktj_generic_rec* g, uint64_t n, uint64_t first, const EmitCtx& ctx, const uint32_t* sync_first,
+                                                  MatRow* mat, uint32_t* len, Scalars* sc, uint64_t block, uint64_t blocks, uint4* stage) {
   RowStats rs;
-  for (uint64_t base = (uint64_t)blockIdx.x * blockDim.x; base < n; base += (uint64_t)gridDim.x * blockDim.x) {
-    const uint32_t cnt = (uint32_t)(n - base < blockDim.x ? n - base : blockDim.x);
+  for (uint64_t base = block * KTJ_BLOCK; base < n; base += blocks * KTJ_BLOCK) {
+    const uint32_t cnt = (uint32_t)(n - base < KTJ_BLOCK ? n - base : KTJ_BLOCK);
     __syncthreads(); /* the previous round's rows have left the staging area */
     rows_global_to_lds(g + base, cnt, stage);
     __syncthreads();
@@ -2255,12 +2178,12 @@ __global__ void k_republish_runtime(const ktj_runtime_rec* r, uint64_t n, Column
   }
   block_add(sc, KTJ_CNT_OUT_OF_ORDER, n_bad);
 }
-__global__ void k_mat_device(const ktj_device_rec* d, uint64_t n, Columns c, uint64_t first, const DevLink* link,
-                             EmitCtx ctx, MatRow* mat, uint32_t* len, Scalars* sc) {
-  __shared__ uint4 stage[KTJ_BLOCK * sizeof(MatRow) / 16]; /* the records, then the joined rows */
+__device__ __forceinline__ void mat_device_block(const ktj_device_rec* d, uint64_t n, const Columns& c, uint64_t first, const DevLink* link,
+                                                 const EmitCtx& ctx, MatRow* mat, uint32_t* len, Scalars* sc, uint64_t block, uint64_t blocks,
+                                                 uint4* stage) {
   RowStats rs;
-  for (uint64_t base = (uint64_t)blockIdx.x * blockDim.x; base < n; base += (uint64_t)gridDim.x * blockDim.x) {
-    const uint32_t cnt = (uint32_t)(n - base < blockDim.x ? n - base : blockDim.x);
+  for (uint64_t base = block * KTJ_BLOCK; base < n; base += blocks * KTJ_BLOCK) {
+    const uint32_t cnt = (uint32_t)(n - base < KTJ_BLOCK ? n - base : KTJ_BLOCK);
     __syncthreads(); /* the previous round's rows have left the staging area */
     rows_global_to_lds(d + base, cnt, stage);
     __syncthreads();
@@ -2290,6 +2213,22 @@ __global__ void k_mat_device(const ktj_device_rec* d, uint64_t n, Columns c, uin
   }
   flush_row_stats(rs, sc);
 }
+/* joined rows and lengths of the generic records (first workgroups) and of the device records (the others);
+ * the runtime rows' are made in k_join_runtime.  Few records: both classes in one launch.  Many: a launch for
+ * each, as the code for both at once needs more registers (22 million: 690 against 575 us). */
+template <bool GENERIC, bool DEVICE>
+__global__ void __launch_bounds__(KTJ_BLOCK) __attribute__((amdgpu_waves_per_eu(4)))
+k_mat_rows(const ktj_generic_rec* g, uint64_t ng, uint64_t first_generic, const uint32_t* sync_first, uint32_t generic_blocks, const ktj_device_rec* d,
+           uint64_t nd, Columns c, uint64_t first_device, const DevLink* link, EmitCtx ctx, MatRow* mat, uint32_t* len, Scalars* sc, int clock) {
+  static_assert(sizeof(MatRow) >= sizeof(ktj_generic_rec) && sizeof(MatRow) >= sizeof(ktj_device_rec), "the staging area holds the records, then the joined rows");
+  __shared__ uint4 stage[KTJ_BLOCK * sizeof(MatRow) / 16];
+  if (blockIdx.x == 0 && threadIdx.x == 0 && clock) stage_clock(sc, KTJ_CLOCK_SIZE);
+  if (sc->error != 0) return; /* the pass ends, or the host takes another way from the sort on */
+  if (GENERIC && (!DEVICE || blockIdx.x < generic_blocks))
+    mat_generic_block(g, ng, first_generic, ctx, sync_first, mat, len, sc, blockIdx.x, generic_blocks, stage);
+  else if (DEVICE)
+    mat_device_block(d, nd, c, first_device, link, ctx, mat, len, sc, blockIdx.x - generic_blocks, gridDim.x - generic_blocks, stage);
+}
 /* Collective metadata: the first activity, in emission order, that prints each entry, per
  * backend (first[2k] nccl, first[2k + 1] hccl).  The host replays appendCollectiveMetadata's
  * bookkeeping (output_json.cpp:799-835) over these.  Runs only for traces that carry any. */
@@ -2314,22 +2253,53 @@ hipError_t collective_first(const MatRow* mat, const uint32_t* perm, uint64_t n_
                      first);
   return KTJ_LAUNCH_CHECK();
 }
-/* lengths and tail kinds in emission order (the size pass leaves both in one word per arrival index) */
-__global__ void k_gather_len(const uint32_t* perm, const uint32_t* len, uint64_t n, uint32_t* len_sorted, uint8_t* kind_sorted) {
-  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const uint32_t v = len[load_once(&perm[i])];
-  store_once(&len_sorted[i], v & 0x3FFFFFFFu);
-  kind_sorted[i] = (uint8_t)(v >> 30);
+/* lengths and tail kinds in emission order (the size pass leaves both in one word per arrival index), and
+ * the lengths' sum per tile of 2048 for the scan that follows */
+__global__ void __launch_bounds__(KTJ_BLOCK)
+k_gather_len(const uint32_t* perm, const uint32_t* len, uint64_t n, uint32_t* len_sorted, uint8_t* kind_sorted, uint64_t* sums, Scalars* sc) {
+  __shared__ uint64_t wave_tot[KTJ_BLOCK >> 6];
+  if (blockIdx.x == 0 && threadIdx.x == 0) stage_clock(sc, KTJ_CLOCK_SCAN);
+  if (sc->error != 0) return; /* there may be no order */
+  const uint64_t base = (uint64_t)blockIdx.x * SCAN_TILE + threadIdx.x;
+  uint32_t v[SCAN_ITEMS];
+#pragma unroll
+  for (int k = 0; k < SCAN_ITEMS; ++k) { const uint64_t i = base + (uint64_t)k * KTJ_BLOCK; v[k] = i < n ? load_once(&perm[i]) : 0u; }
+#pragma unroll
+  for (int k = 0; k < SCAN_ITEMS; ++k) { const uint64_t i = base + (uint64_t)k * KTJ_BLOCK; v[k] = i < n ? len[v[k]] : 0u; }
+  unsigned long long sum = 0;
+#pragma unroll
+  for (int k = 0; k < SCAN_ITEMS; ++k) {
+    const uint64_t i = base + (uint64_t)k * KTJ_BLOCK;
+    if (i < n) { len_sorted[i] = v[k] & 0x3FFFFFFFu; kind_sorted[i] = (uint8_t)(v[k] >> 30); }
+    sum += v[k] & 0x3FFFFFFFu;
+  }
+  for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
+  if (lane_id() == 0) wave_tot[threadIdx.x >> 6] = sum;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    uint64_t s = 0;
+    for (uint32_t k = 0; k < (KTJ_BLOCK >> 6); ++k) s += wave_tot[k];
+    sums[blockIdx.x] = s;
+  }
 }
 
-hipError_t mat_generic_rows(const ktj_generic_rec* g, uint64_t n, uint64_t first, EmitCtx ctx, const uint32_t* sync_first,
-                            MatRow* mat, uint32_t* len, Scalars* sc, hipStream_t st) {
-  if (n == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_mat_generic, dim3(grid_stride_for(n, KTJ_BLOCK)), dim3(KTJ_BLOCK), 0, st, g, n, first, ctx, sync_first,
-                     mat, len, sc);
+#define MAT_ONE_LAUNCH_ROWS 262144u
+hipError_t mat_rows(const ktj_generic_rec* g, uint64_t ng, uint64_t first_generic, const uint32_t* sync_first, const ktj_device_rec* d, uint64_t nd,
+                    Columns c, uint64_t first_device, const DevLink* link, EmitCtx ctx, MatRow* mat, uint32_t* len, Scalars* sc, hipStream_t st) {
+  const unsigned gb = grid_stride_for(ng, KTJ_BLOCK), db = grid_stride_for(nd, KTJ_BLOCK);
+  auto launch = [&](auto kernel, unsigned g_blocks, unsigned d_blocks, bool clock) {
+    hipLaunchKernelGGL(kernel, dim3(g_blocks + d_blocks), dim3(KTJ_BLOCK), 0, st, g, ng, first_generic, sync_first, g_blocks, d, nd, c, first_device,
+                       link, ctx, mat, len, sc, clock ? 1 : 0);
+  };
+  const bool clock = first_generic == 0;
+  if (gb && db && ng + nd < MAT_ONE_LAUNCH_ROWS) launch(k_mat_rows<true, true>, gb, db, clock);
+  else {
+    if (gb) launch(k_mat_rows<true, false>, gb, 0, clock);
+    if (db) launch(k_mat_rows<false, true>, 0, db, clock && !gb);
+  }
   return KTJ_LAUNCH_CHECK();
 }
+
 hipError_t join_runtime_rows(const ktj_runtime_rec* r, uint64_t n, Columns c, uint64_t first, ApiTable api, Table tf, FullCols fc,
                              Table tn, NarrowCols nc, uint32_t* slot_f, uint32_t* slot_n, EmitCtx ctx, MatRow* mat,
                              uint32_t* len, Scalars* sc, hipStream_t st) {
@@ -2349,48 +2319,104 @@ hipError_t republish_runtime_rows(const ktj_runtime_rec* r, uint64_t n, Columns 
                      slot_f, slot_n, sc);
   return KTJ_LAUNCH_CHECK();
 }
-hipError_t mat_device_rows(const ktj_device_rec* d, uint64_t n, Columns c, uint64_t first, const DevLink* link,
-                           EmitCtx ctx, MatRow* mat, uint32_t* len, Scalars* sc, hipStream_t st) {
-  if (n == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_mat_device, dim3(grid_stride_for(n, KTJ_BLOCK)), dim3(KTJ_BLOCK), 0, st, d, n, c, first, link, ctx,
-                     mat, len, sc);
-  return KTJ_LAUNCH_CHECK();
+/* The activities' offsets from their lengths and the tiles' sums.  Few tiles: every workgroup adds up the
+ * sums before its own (OFFS_DIRECT_TILES of them are 16 KB from the L2), many: k_scan_of_sums has run.
+ * One more workgroup than tiles knows the total: with a document to prepare (out != null) it puts the footer
+ * text behind the activities and hands the scalars to the host, and more of them put the header, 4 KiB each
+ * (all of that takes some microseconds over the host link, which the offsets need not wait for; 40 KB of
+ * header by one workgroup took 20 us). */
+#define PREFIX_PIECE 4096u
+#define OFFS_DIRECT_TILES 2048u
+__device__ void publish_scalars(Scalars* sc, Scalars* h_sc, bool document_fits);
+__global__ void __launch_bounds__(KTJ_BLOCK)
+k_offsets(const uint32_t* len, uint64_t n, const uint64_t* sums, uint32_t n_tiles, uint64_t* offs, Scalars* sc, DocText T) {
+  __shared__ uint64_t lds_wave[SCAN_MAX_WAVES];
+  __shared__ uint64_t s_before;
+  if (blockIdx.x > n_tiles) {
+    const uint64_t at = (uint64_t)(blockIdx.x - n_tiles - 1u) * PREFIX_PIECE, left = T.n_prefix - at;
+    if (T.n_prefix + 64u <= T.out_cap) put_text_block(T.prefix + at, T.out + at, left < PREFIX_PIECE ? left : PREFIX_PIECE);
+    return;
+  }
+  const bool ok = sc->error == 0; /* otherwise there are no lengths: only the host is told */
+  uint64_t before = 0;
+  if (n_tiles <= OFFS_DIRECT_TILES) {
+    unsigned long long s = 0;
+    if (ok) for (uint32_t k = threadIdx.x; k < blockIdx.x; k += KTJ_BLOCK) s += sums[k];
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+    if (lane_id() == 0) lds_wave[threadIdx.x >> 6] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) { uint64_t b = 0; for (uint32_t k = 0; k < (KTJ_BLOCK >> 6); ++k) b += lds_wave[k]; s_before = b; }
+    __syncthreads();
+    before = s_before;
+  } else before = ok ? sums[blockIdx.x] : 0;
+  if (blockIdx.x == n_tiles) {
+    if (threadIdx.x == 0) offs[n] = before;
+    if (!T.out) return;
+    const bool fits = ok && T.n_prefix + before + T.n_suffix + 64u <= T.out_cap;
+    publish_scalars(sc, T.h_sc, fits);
+    if (threadIdx.x == 0) *T.h_total = before;
+    if (fits) put_text_block(T.suffix, T.out + T.n_prefix + before, T.n_suffix);
+    return;
+  }
+  if (!ok) return;
+  const uint64_t base = (uint64_t)blockIdx.x * SCAN_TILE + (uint64_t)threadIdx.x * SCAN_ITEMS;
+  uint32_t v[SCAN_ITEMS];
+  scan_load_items(len, n, base, v);
+  uint64_t s = 0;
+  for (int k = 0; k < SCAN_ITEMS; ++k) s += v[k];
+  uint64_t tot;
+  uint64_t ex = block_exclusive_scan_u64(s, lds_wave, &tot) + before;
+  if (base + SCAN_ITEMS <= n) { /* the lane's run as 16-byte stores (the offsets are a 16-byte aligned device buffer) */
+    typedef unsigned long long v2u64 __attribute__((ext_vector_type(2)));
+    v2u64* dst = reinterpret_cast<v2u64*>(offs + base);
+#pragma unroll
+    for (int q = 0; q < SCAN_ITEMS / 2; ++q) { v2u64 x; x.x = ex; ex += v[2 * q]; x.y = ex; ex += v[2 * q + 1]; dst[q] = x; }
+  } else {
+    for (int k = 0; k < SCAN_ITEMS; ++k) { if (base + k < n) offs[base + k] = ex; ex += v[k]; }
+  }
 }
-hipError_t gather_len(const uint32_t* perm, const uint32_t* len, uint64_t n, uint32_t* len_sorted, uint8_t* kind_sorted,
-                      hipStream_t st) {
-  if (n == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_gather_len, dim3(grid_for(n, KTJ_BLOCK)), dim3(KTJ_BLOCK), 0, st, perm, len, n, len_sorted, kind_sorted);
+uint64_t offsets_tmp_elems(uint64_t n) { return (n + SCAN_TILE - 1) / SCAN_TILE + 2; }
+hipError_t gather_offsets(const uint32_t* perm, const uint32_t* len, uint64_t n, uint32_t* len_sorted, uint8_t* kind_sorted, uint64_t* sums,
+                          uint64_t* offs, Scalars* sc, const DocText& text, hipStream_t st) {
+  const uint64_t tiles = n ? (n + SCAN_TILE - 1) / SCAN_TILE : 1;
+  hipLaunchKernelGGL(k_gather_len, dim3((unsigned)tiles), dim3(KTJ_BLOCK), 0, st, perm, len, n, len_sorted, kind_sorted, sums, sc);
+  if (tiles > OFFS_DIRECT_TILES) hipLaunchKernelGGL(k_scan_of_sums, dim3(1), dim3(1024), 0, st, sums, tiles);
+  const uint64_t prefix_blocks = text.out ? (text.n_prefix + PREFIX_PIECE - 1) / PREFIX_PIECE : 0;
+  hipLaunchKernelGGL(k_offsets, dim3((unsigned)(tiles + 1u + prefix_blocks)), dim3(KTJ_BLOCK), 0, st, (const uint32_t*)len_sorted, n, (const uint64_t*)sums,
+                     (uint32_t)tiles, offs, sc, text);
   return KTJ_LAUNCH_CHECK();
 }
 
 /* What the host needs during a pass goes straight into its pinned memory, and the text it made
  * (header, infos, footer) comes straight out of it: one small kernel each instead of one copy
  * engine transfer per value. */
+__device__ void publish_scalars(Scalars* sc, Scalars* h_sc, bool document_fits) { /* by one workgroup */
+  /* the sharded counters: their sums so far into the fields the host reads (written, not added: a pass
+   * may publish twice) */
+  static_assert(KTJ_COUNTER_SHARDS == 64, "a lane per copy");
+  if (threadIdx.x < 64) {
+    unsigned long long sum[KTJ_CNT_COUNT];
+    for (int k = 0; k < KTJ_CNT_COUNT; ++k) sum[k] = sc->shard[threadIdx.x][k];
+    for (int k = 0; k < KTJ_CNT_COUNT; ++k)
+      for (int o = 32; o > 0; o >>= 1) sum[k] += __shfl_xor(sum[k], o);
+    if (threadIdx.x == 0) {
+      sc->out_of_range = sum[KTJ_CNT_OUT_OF_RANGE]; sc->out_of_order = sum[KTJ_CNT_OUT_OF_ORDER];
+      sc->n_flow = sum[KTJ_CNT_FLOW]; sc->n_linked = sum[KTJ_CNT_LINKED]; sc->n_blank_names = sum[KTJ_CNT_BLANK_NAMES];
+      sc->n_valid = sum[KTJ_CNT_VALID]; sc->n_sync_typed = sum[KTJ_CNT_SYNC_TYPED];
+      sc->emit_rows = sc->error == 0 && document_fits ? sum[KTJ_CNT_VALID] : 0;
+    }
+  }
+  if (threadIdx.x == 0) stage_clock(sc, KTJ_CLOCK_EMIT);
+  __syncthreads();
+  constexpr uint32_t head_words = (uint32_t)(offsetof(Scalars, shard) / 4);
+  const uint32_t* src = reinterpret_cast<const uint32_t*>(sc);
+  uint32_t* dst = reinterpret_cast<uint32_t*>(h_sc);
+  for (uint32_t k = threadIdx.x; k < head_words; k += blockDim.x) dst[k] = src[k];
+}
 __global__ void k_publish(Scalars* sc, const uint64_t* total, const uint32_t* list, uint32_t n_list, Scalars* h_sc,
                           uint64_t* h_total, uint32_t* h_list) {
   const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x, stride = gridDim.x * blockDim.x;
-  if (blockIdx.x == 0) {
-    /* the sharded counters: their sums so far into the fields the host reads (written, not added:
-     * a pass publishes twice) */
-    if (threadIdx.x < KTJ_CNT_COUNT) {
-      unsigned long long sum = 0;
-      for (uint32_t k = 0; k < KTJ_COUNTER_SHARDS; ++k) sum += sc->shard[k][threadIdx.x];
-      switch (threadIdx.x) {
-        case KTJ_CNT_OUT_OF_RANGE: sc->out_of_range = sum; break;
-        case KTJ_CNT_OUT_OF_ORDER: sc->out_of_order = sum; break;
-        case KTJ_CNT_FLOW: sc->n_flow = sum; break;
-        case KTJ_CNT_LINKED: sc->n_linked = sum; break;
-        case KTJ_CNT_BLANK_NAMES: sc->n_blank_names = sum; break;
-        case KTJ_CNT_VALID: sc->n_valid = sum; break;
-        default: sc->n_sync_typed = sum; break;
-      }
-    }
-    __syncthreads();
-    constexpr uint32_t head_words = (uint32_t)(offsetof(Scalars, shard) / 4);
-    const uint32_t* src = reinterpret_cast<const uint32_t*>(sc);
-    uint32_t* dst = reinterpret_cast<uint32_t*>(h_sc);
-    for (uint32_t k = threadIdx.x; k < head_words; k += blockDim.x) dst[k] = src[k];
-  }
+  if (blockIdx.x == 0) publish_scalars(sc, h_sc, true);
   for (uint32_t k = t; k < n_list; k += stride) h_list[k] = list[k];
   if (t == 0 && total != nullptr) *h_total = *total;
   __threadfence_system();

@@ -26,8 +26,6 @@ namespace gpu {
 #define SMALL_PER ((SMALL_ROWS + SMALL_JOIN_THREADS - 1u) / SMALL_JOIN_THREADS) /* rows of a class per thread */
 #define SMALL_DICT_PER_BLOCK (SMALL_JOIN_THREADS / 64u)
 
-__device__ __forceinline__ void small_clock(Scalars* sc, int k) { sc->clock[k] = wall_clock64(); }
-
 /* ------------------------------------------------------------------------------------------ */
 /* first launch: decode and joins                                                               */
 /* ------------------------------------------------------------------------------------------ */
@@ -76,7 +74,7 @@ __global__ void __launch_bounds__(SMALL_JOIN_THREADS) k_small_join(SmallArgs A) 
   const uint32_t tid = threadIdx.x, ng = A.ng, nr = A.nr, nd = A.nd, nx = A.nx;
   const uint32_t mask = A.slots - 1u;
   const Columns c = A.c;
-  if (tid == 0) small_clock(A.sc, 0);
+  if (tid == 0) stage_clock(A.sc, 0);
   for (uint32_t k = tid; k < A.slots; k += SMALL_JOIN_THREADS) {
     t_cpu[k] = 0; t_full[k] = 0; f_first[k] = 0xFFFFFFFFu; f_stream[k] = 0;
     t_narrow[k] = 0; n_ext[k] = 0; n_kern[k] = 0; n_copy[k] = 0;
@@ -120,7 +118,7 @@ __global__ void __launch_bounds__(SMALL_JOIN_THREADS) k_small_join(SmallArgs A) 
     count(C_VALID, valid); count(C_OOR, oor); count(C_UNFIT, unfit);
   }
   __syncthreads();
-  if (tid == 0) small_clock(A.sc, 1);
+  if (tid == 0) stage_clock(A.sc, 1);
 
   auto cpu_key = [&](uint32_t e) { return c.corr[e - 1u]; };
   auto full_key = [&](uint32_t e) { return s_corr[e - 1u]; };
@@ -335,7 +333,7 @@ __global__ void __launch_bounds__(SMALL_JOIN_THREADS) k_small_join(SmallArgs A) 
     s->have_stream_src = have_stream ? 1u : 0u; s->n_dev_ranks = 0; s->n_res_ranks = 0; s->n_dense = s_cnt[C_DENSE];
     s->n_plain = 0; s->runtime_ids_repeat = 0; s->n_queues = 0; s->n_sync_rows = 0; s->ext_ids_repeat = 0;
     for (uint32_t k = 0; k < KTJ_PART_SLOTS; ++k) s->part_done[k] = 0;
-    small_clock(s, 2);
+    stage_clock(s, 2);
   }
 }
 
@@ -395,7 +393,7 @@ __device__ __forceinline__ void small_order(const SmallArgs& A) {
   __shared__ uint32_t n_pairs;
   const Columns c = A.c;
   const uint32_t n = A.ng + A.nr + A.nd, mask = A.slots - 1u, first = threadIdx.x * SORT_ITEMS;
-  if (threadIdx.x == 0) { s_min = ~0ULL; s_max = 0; n_pairs = 0; small_clock(A.sc, 3); }
+  if (threadIdx.x == 0) { s_min = ~0ULL; s_max = 0; n_pairs = 0; stage_clock(A.sc, 3); }
   for (uint32_t k = threadIdx.x; k < A.slots; k += ROWS_THREADS) t_pair[k] = 0;
   uint32_t slot[SORT_ITEMS];
   uint64_t ts[SORT_ITEMS];
@@ -454,7 +452,7 @@ __device__ __forceinline__ void small_order(const SmallArgs& A) {
 #pragma unroll
   for (uint32_t i = 0; i < SORT_ITEMS; ++i)
     if (first + i < n) A.perm[first + i] = (uint32_t)w[i] & (SMALL_ROWS - 1u);
-  if (threadIdx.x == 0) small_clock(A.sc, 4);
+  if (threadIdx.x == 0) stage_clock(A.sc, 4);
 }
 
 /* exact byte length, and whether some part of the activity has more pieces than a wavefront has lanes
@@ -691,13 +689,13 @@ __device__ __forceinline__ uint64_t small_offsets(const uint32_t* perm, const ui
   return total;
 }
 __global__ void __launch_bounds__(KTJ_BLOCK) k_small_emit(const MatRow* mat, const uint32_t* perm, const uint32_t* len, Scalars* sc, EmitCtx ctx,
-                                                          SmallText T) {
+                                                          DocText T) {
   __shared__ uint64_t offs[SMALL_ROWS];
   const uint32_t error = sc->error, n = (uint32_t)sc->n_valid;
   const uint64_t total = error == 0 ? small_offsets(perm, len, n, offs) : 0;
   if (blockIdx.x == 0) { /* what the host waits for; nothing here waits for the other workgroups */
     constexpr uint32_t head_words = (uint32_t)(offsetof(Scalars, shard) / 4);
-    if (threadIdx.x == 0) small_clock(sc, 5);
+    if (threadIdx.x == 0) stage_clock(sc, 5);
     __syncthreads();
     const uint32_t* src = reinterpret_cast<const uint32_t*>(sc);
     uint32_t* dst = reinterpret_cast<uint32_t*>(T.h_sc);
@@ -731,7 +729,7 @@ __global__ void __launch_bounds__(KTJ_BLOCK) k_small_emit(const MatRow* mat, con
 /* Only when the rows have shown activities with more pieces than lanes (InputShapes of many operands,
  * long arrays): one lane per workgroup writes each of them. */
 __global__ void __launch_bounds__(KTJ_BLOCK) k_small_plain(const MatRow* mat, const uint32_t* perm, const uint32_t* len, Scalars* sc, EmitCtx ctx,
-                                                           SmallText T) {
+                                                           DocText T) {
   __shared__ uint64_t offs[SMALL_ROWS];
   const uint32_t n = (uint32_t)sc->n_valid;
   small_offsets(perm, len, n, offs);
@@ -753,13 +751,13 @@ hipError_t small_pass(const SmallArgs& a, uint32_t n_strings, hipStream_t st) {
                      0, st, a);
   return KTJ_LAUNCH_CHECK();
 }
-hipError_t small_emit(const SmallArgs& a, const SmallText& t, hipStream_t st) {
+hipError_t small_emit(const SmallArgs& a, const DocText& t, hipStream_t st) {
   const uint64_t n = (uint64_t)a.ng + a.nr + a.nd; /* a wavefront per activity, two workgroups for the text */
   hipLaunchKernelGGL(k_small_emit, dim3(grid_for(n, KTJ_BLOCK >> 6) + 2u), dim3(KTJ_BLOCK), 0, st, (const MatRow*)a.mat, (const uint32_t*)a.perm,
                      (const uint32_t*)a.len, a.sc, a.ctx, t);
   return KTJ_LAUNCH_CHECK();
 }
-hipError_t small_plain(const SmallArgs& a, const SmallText& t, hipStream_t st) {
+hipError_t small_plain(const SmallArgs& a, const DocText& t, hipStream_t st) {
   const uint64_t n = (uint64_t)a.ng + a.nr + a.nd;
   hipLaunchKernelGGL(k_small_plain, dim3(grid_for(n, KTJ_BLOCK >> 6)), dim3(KTJ_BLOCK), 0, st, (const MatRow*)a.mat, (const uint32_t*)a.perm,
                      (const uint32_t*)a.len, a.sc, a.ctx, t);

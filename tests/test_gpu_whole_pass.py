@@ -1,0 +1,93 @@
+"""GPU: a pass that is put into the stream in one go, where it hands over to the stepwise one, and the sizes
+at which its launches change, against the oracle: same document, same counters."""
+import ctypes as C
+
+import pytest
+
+from kineto_amd import abi
+from kineto_amd.engine import TraceEngine
+
+pytestmark = pytest.mark.gpu
+
+
+def oracle(sp):
+    import oracle_glue as og
+    ora = og.OracleRun(sp)
+    want, cnt = ora.output(), ora.counters()
+    ora.close()
+    return want, (cnt["out_of_range"], cnt["out_of_order"], cnt["n_flow_events"], cnt["n_linked"])
+
+
+def check(eng, want, counters, passes=2):
+    for _ in range(passes):
+        eng.process()
+        st = eng.stats()
+        assert eng.output() == want
+        assert (st.out_of_range_events, st.gpu_and_cpu_op_out_of_order, st.n_flow_events, st.n_linked) == counters
+
+
+# one sort tile, one more; both classes of joined rows in one launch, in two; rows of one class only
+@pytest.mark.parametrize("config,rows", [(5, 4096), (5, 4097), (1, 1400), (3, 9000), (4, 5000), (5, 262143), (5, 262146), (5, 700001)])
+def test_sizes(config, rows):
+    sp, release = abi.synth_stream(config, rows, host_name="whole")
+    want, counters = oracle(sp)
+    with TraceEngine(sp.contents.trace_name.decode()) as eng:
+        eng.submit_stream(sp)
+        check(eng, want, counters)
+    release()
+
+
+def ops(spans, sync_at=None):
+    """CPU ops at base + offset for the offsets of each span, some of them on other rows."""
+    from stream_builder import B, StreamBuilder
+    b = StreamBuilder()
+    for k, off in enumerate(spans):
+        b.add_generic("op %d" % (k % 50), 0, B + off, B + off + 5, 1, k % 7, id=k + 1)
+    if sync_at is not None:
+        b.add_generic("Stream Sync", 15, B + sync_at, B + sync_at + 5, 0, 5, id=len(spans) + 1)
+    return b.build()
+
+
+@pytest.mark.parametrize("bits", [8, 44, 45, 52, 53, 60, 62])
+def test_timestamps_far_apart(bits):
+    """The sort's passes: fewer than launched, as many, more than launched, keys too wide for a word with the
+    index, for one key at all."""
+    sp = ops([(k * 2654435761) % (1 << bits) for k in range(4999)] + [0, (1 << bits) - 1])
+    want, counters = oracle(sp)
+    with TraceEngine(sp.contents.trace_name.decode(), base_time_ns=sp.contents.base_time_ns) as eng:
+        eng.submit_stream(sp)
+        check(eng, want, counters)
+
+
+@pytest.mark.parametrize("late,sync", [(1 << 20, None), (1 << 50, None), (2000, 1000)])
+def test_later_records_need_more(late, sync):
+    """The engine has seen records that sort in two passes; what is submitted afterwards needs more, or a row
+    for its Stream Sync activities."""
+    sp = ops([k % 3000 for k in range(5000)] + [late + k for k in range(100)], sync)
+    want, counters = oracle(sp)
+    s = sp.contents
+    whole = s.n_generic
+    with TraceEngine(s.trace_name.decode(), base_time_ns=s.base_time_ns) as eng:
+        s.n_generic = 5000
+        eng.submit_stream(sp)
+        eng.process()
+        eng.process()
+        rest = C.addressof(s.generic.contents) + 5000 * C.sizeof(s.generic.contents)
+        eng._chk(eng.lib.ktj_submit_records(eng.h, abi.REC_GENERIC, C.c_void_p(rest), whole - 5000), "ktj_submit_records")
+        s.n_generic = whole
+        check(eng, want, counters)
+
+
+def test_document_longer_than_the_first_buffer():
+    from stream_builder import B, StreamBuilder
+    b = StreamBuilder()
+    names = ["n%d" % k for k in range(4000)] + ["long" * 3000]
+    for n in names:
+        b.s(n)
+    for k in range(3000):
+        b.add_generic(names[-1], 5, B + k, B + k + 10, 0, 1, id=k + 1)
+    sp = b.build()
+    want, counters = oracle(sp)
+    with TraceEngine(sp.contents.trace_name.decode(), base_time_ns=sp.contents.base_time_ns) as eng:
+        eng.submit_stream(sp)
+        check(eng, want, counters)
