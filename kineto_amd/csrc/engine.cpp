@@ -1562,7 +1562,7 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
     if (out_device) e->out.borrow(out_device, out_cap);
     e->perm = e->vals_a.as<uint32_t>();
     e->sorted_keys = nullptr;
-    HIPCHK(sort_packed(c, N, sets, sc, e->sort_passes, e->keys_a.as<uint64_t>(), e->keys_b.as<uint64_t>(), e->perm, e->hist.as<uint32_t>(), st));
+    HIPCHK(sort_packed(c, N, sets, sc, e->sort_passes, e->keys_a.as<uint64_t>(), e->keys_b.as<uint64_t>(), e->perm, e->hist.as<uint32_t>(), e->offs.as<uint32_t>(), st));
     HIPCHK(mat_rows(g_recs, ng, 0, nullptr, d_recs, nd, c, ng + nr, e->dev_link.as<DevLink>(), ctx, mat, e->len.as<uint32_t>(), sc, st));
     for (;;) {
       text.out = e->out.as<char>(); text.out_cap = e->out.cap;
@@ -1630,7 +1630,7 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
       if (rc == KTJ_OK) rc = sort_again([&](const uint32_t* o, uint64_t* k, uint32_t* v) { return make_column_keys(c.dev, c.meta, o, N, 1, k, v, st); }, 1);
       if (rc != KTJ_OK) return rc;
     } else if (key_bits <= 62 && e->sort_mode != 1 && sort_packed_fits(N, key_bits)) {
-      HIPCHK(sort_packed(c, N, sets, sc, sort_packed_passes(key_bits), ka, kb, va, hist, st));
+      HIPCHK(sort_packed(c, N, sets, sc, sort_packed_passes(key_bits), ka, kb, va, hist, e->offs.as<uint32_t>(), st));
       e->perm = va;
       e->sorted_keys = nullptr;
     } else if (key_bits <= 62) {

@@ -339,7 +339,7 @@ uint32_t sort_packed_passes(uint32_t key_bits);
 /* key widths come from Scalars::sort; `passes` is how many are launched: those beyond the plan end at once, and
  * a plan that needs more (or does not fit a word) sets KTJ_DEVERR_CAREFUL in Scalars::error */
 hipError_t sort_packed(Columns c, uint64_t n, SortSets s, Scalars* sc, uint32_t passes, uint64_t* buf_a, uint64_t* buf_b, uint32_t* perm,
-                       uint32_t* hist, hipStream_t st);
+                       uint32_t* hist, uint32_t* chain_hist /* 8 bytes per row */, hipStream_t st);
 hipError_t make_rank_keys(Columns c, const uint32_t* order, uint64_t n, SortSets s, uint32_t res_bits, uint32_t rank_bits,
                           uint64_t* keys, uint32_t* vals, hipStream_t st);
 /* stable LSD radix sort of (key, val) pairs on the low `bits` bits; result ends in keys_out/vals_out

@@ -1451,7 +1451,9 @@ template <int BITS, int THREADS, int ITEMS_> struct SortP {
   static_assert(NB % THREADS == 0 || THREADS % NB == 0, "digits and threads must divide");
 };
 
-template <int BITS, int THREADS, int ITEMS>
+/* CHAIN: for k_sortp_chain, whose counts are tile by tile (hist[(pass * n_blocks + tile) * 256 + digit]) and, behind
+ * the first pass's, start from zero. */
+template <int BITS, int THREADS, int ITEMS, bool CHAIN>
 __global__ void __launch_bounds__(THREADS)
 k_sortp_make_keys(Columns c, uint64_t n, SortSets s, Scalars* sc, uint32_t idx_bits, uint32_t passes_launched, uint64_t* keys, uint32_t* hist,
                   uint32_t n_blocks) {
@@ -1496,7 +1498,11 @@ k_sortp_make_keys(Columns c, uint64_t n, SortSets s, Scalars* sc, uint32_t idx_b
     }
   }
   __syncthreads();
-  if (hist != nullptr)
+  if (CHAIN) {
+    const uint32_t passes = sort_passes(sc);
+    for (uint32_t k = threadIdx.x; k < passes * P::NB; k += THREADS)
+      hist[((uint64_t)(k / P::NB) * n_blocks + blockIdx.x) * P::NB + k % P::NB] = k < P::NB ? h[k] : 0u;
+  } else if (hist != nullptr)
     for (int d = threadIdx.x; d < P::NB; d += THREADS) hist[(uint64_t)d * n_blocks + blockIdx.x] = h[d]; /* digit-major */
 }
 template <int BITS, int THREADS, int ITEMS>
@@ -1796,7 +1802,7 @@ static hipError_t sort_packed_t(Columns c, uint64_t n, SortSets s, Scalars* sc, 
   /* the digits' totals live behind the counts (radix_tmp_elems leaves 256 spare entries) */
   uint32_t* totals = hist + (uint64_t)P::NB * n_blocks;
   static_assert(P::NB <= 256, "room for the totals behind the counts");
-  hipLaunchKernelGGL((k_sortp_make_keys<BITS, THREADS, ITEMS>), g, b, 0, st, c, n, s, sc, idx_bits, passes, buf_a, counts, n_blocks);
+  hipLaunchKernelGGL((k_sortp_make_keys<BITS, THREADS, ITEMS, false>), g, b, 0, st, c, n, s, sc, idx_bits, passes, buf_a, counts, n_blocks);
   if (!single) hipLaunchKernelGGL((k_sortp_scan_digits<THREADS>), dim3(P::NB), b, 0, st, hist, n_blocks, totals, 0u, (const Scalars*)sc);
   hipLaunchKernelGGL((k_sortp_scatter<BITS, THREADS, ITEMS, true>), g, b, 0, st, (const uint64_t*)buf_a, buf_b, perm, n, 0u, idx_bits,
                      (const Scalars*)sc, (const uint32_t*)counts, (const uint32_t*)totals, n_blocks);
@@ -1808,6 +1814,125 @@ static hipError_t sort_packed_t(Columns c, uint64_t n, SortSets s, Scalars* sc, 
     }
     hipLaunchKernelGGL((k_sortp_scatter<BITS, THREADS, ITEMS, false>), g, b, 0, st, (const uint64_t*)in, out, perm, n, p, idx_bits,
                        (const Scalars*)sc, (const uint32_t*)counts, (const uint32_t*)totals, n_blocks);
+    uint64_t* t = in; in = out; out = t;
+  }
+  return KTJ_LAUNCH_CHECK();
+}
+
+/* Up to CHAIN_MAX_N keys a pass is one launch instead of three (count, scan, scatter: with five passes that was
+ * half the launches of a trace of 30 000 records, each some 3 us for hardly a microsecond of work):
+ *   - a workgroup adds the digit counts of the tiles before its own, and of all, up by itself: a few dozen
+ *     loads per thread, all in flight together;
+ *   - while it puts its keys to their places it counts the next pass's digits per tile of the output, in LDS
+ *     (16 bits each: a tile holds 1024 keys), and adds what it has to the next pass's counts.
+ * Bound by the chain of its short phases, some 5 us whatever the tile holds: one key per thread is the
+ * shortest of them (a first form that put a tile in order before it was written out: 186 us for 30 000 records
+ * with tiles of 1024 keys, 203 with 2048, 212 with 4096).  Three launches a pass against this, whole pass:
+ * 30 000 records 218 -> 185 us, 60 000 223 -> 207, 90 000 258 -> 251, 118 000 243 both; counts to add up and
+ * cells to hand on grow with the tiles, and at 733 000 keys a pass took 30 us instead of 25. */
+#define CHAIN_THREADS 1024
+#define CHAIN_MAX_N 131072ull
+template <int BITS, bool FROM_KEYS>
+__global__ void __launch_bounds__(CHAIN_THREADS)
+k_sortp_chain(const uint64_t* in, uint64_t* words_out, uint32_t* perm_out, uint32_t n, uint32_t pass, uint32_t idx_bits, const Scalars* sc,
+              uint32_t* hist, uint32_t n_blocks) {
+  using P = SortP<BITS, CHAIN_THREADS, 1>;
+  constexpr uint32_t NB = P::NB, GROUPS = CHAIN_THREADS / NB;
+  if (sort_pass_idle(sc, pass)) return;
+  const bool TO_PERM = pass + 1u == sort_passes(sc);
+  const uint32_t shift = FROM_KEYS ? 0u : idx_bits + (pass - 1u) * BITS;
+  const uint32_t next_shift = FROM_KEYS ? idx_bits : shift + BITS;
+  __shared__ uint32_t next[CHAIN_MAX_N / P::TILE * (NB / 2u)]; /* two cells a word */
+  __shared__ uint32_t wave_run[P::WAVES][NB];
+  __shared__ uint32_t part[2][GROUPS][NB]; /* counts before this tile, of all tiles */
+  __shared__ uint32_t base_of[NB];
+  __shared__ uint32_t wave_tot[NB / 64];
+  const uint32_t w = threadIdx.x >> 6, lane = lane_id();
+  const uint32_t tile_base = blockIdx.x * P::TILE, i = tile_base + threadIdx.x;
+  const bool valid = i < n;
+  uint64_t word = in[valid ? i : n - 1u];
+  {
+    const uint32_t d = threadIdx.x & (NB - 1u), group = threadIdx.x / NB;
+    const uint32_t* row = hist + (uint64_t)pass * n_blocks * NB + d;
+    uint32_t before = 0, all = 0;
+#pragma unroll 8
+    for (uint32_t t = group; t < n_blocks; t += GROUPS) {
+      const uint32_t c = row[t * NB];
+      all += c;
+      before += t < blockIdx.x ? c : 0u;
+    }
+    part[0][group][d] = before;
+    part[1][group][d] = all;
+  }
+  for (uint32_t k = threadIdx.x; k < P::WAVES * NB; k += CHAIN_THREADS) (&wave_run[0][0])[k] = 0;
+  if (!TO_PERM)
+    for (uint32_t k = threadIdx.x; k < n_blocks * (NB / 2u); k += CHAIN_THREADS) next[k] = 0;
+  __syncthreads();
+  uint32_t digit;
+  if (FROM_KEYS) {
+    digit = (uint32_t)word & (NB - 1u);
+    word = ((word >> BITS) << idx_bits) | i;
+  } else digit = (uint32_t)(word >> shift) & (NB - 1u);
+  uint64_t peers = __ballot(valid ? 1 : 0);
+#pragma unroll
+  for (int b = 0; b < BITS; ++b) {
+    const uint64_t bal = __ballot((digit >> b) & 1u);
+    peers &= ((digit >> b) & 1u) ? bal : ~bal;
+  }
+  const uint32_t rank = (uint32_t)__popcll(peers & lanemask_lt());
+  if (valid && rank == 0) wave_run[w][digit] = (uint32_t)__popcll(peers);
+  __syncthreads();
+  /* thread d: where each wavefront's keys with digit d begin among the tile's, and where the tile's go */
+  uint32_t before = 0, in_all = 0, inc = 0;
+  const uint32_t d = threadIdx.x;
+  if (d < NB) {
+    uint32_t run = 0;
+#pragma unroll
+    for (int k = 0; k < P::WAVES; ++k) { const uint32_t cnt = wave_run[k][d]; wave_run[k][d] = run; run += cnt; }
+#pragma unroll
+    for (uint32_t g = 0; g < GROUPS; ++g) { before += part[0][g][d]; in_all += part[1][g][d]; }
+    inc = in_all;
+    for (int o = 1; o < 64; o <<= 1) { const uint32_t t = __shfl_up(inc, o); if (lane >= (uint32_t)o) inc += t; }
+    if (lane == 63) wave_tot[w] = inc;
+  }
+  __syncthreads();
+  if (d < NB) {
+    uint32_t base = inc - in_all + before;
+    for (uint32_t k = 0; k < w; ++k) base += wave_tot[k];
+    base_of[d] = base;
+  }
+  __syncthreads();
+  if (valid) { /* (a digit's keys of a tile lie together: hardly more lines than if the tile were put in order first) */
+    const uint32_t dst = base_of[digit] + wave_run[w][digit] + rank;
+    if (TO_PERM) perm_out[dst] = (uint32_t)(word & ((1ULL << idx_bits) - 1ULL));
+    else {
+      words_out[dst] = word;
+      const uint32_t cell = (dst / (uint32_t)P::TILE) * NB + ((uint32_t)(word >> next_shift) & (NB - 1u));
+      atomicAdd(&next[cell >> 1], cell & 1u ? 0x10000u : 1u);
+    }
+  }
+  if (TO_PERM) return;
+  __syncthreads();
+  uint32_t* next_hist = hist + (uint64_t)(pass + 1u) * n_blocks * NB;
+  for (uint32_t k = threadIdx.x; k < n_blocks * (NB / 2u); k += CHAIN_THREADS) {
+    const uint32_t c = next[k];
+    if (c & 0xFFFFu) atomicAdd(&next_hist[2u * k], c & 0xFFFFu);
+    if (c >> 16) atomicAdd(&next_hist[2u * k + 1u], c >> 16);
+  }
+}
+template <int BITS>
+static hipError_t sort_packed_chain(Columns c, uint64_t n, SortSets s, Scalars* sc, uint32_t passes, uint32_t idx_bits, uint64_t* buf_a,
+                                    uint64_t* buf_b, uint32_t* perm, uint32_t* hist, hipStream_t st) {
+  using P = SortP<BITS, CHAIN_THREADS, 1>;
+  const uint32_t n_blocks = (uint32_t)((n + P::TILE - 1) / P::TILE);
+  const dim3 g(n_blocks), b(CHAIN_THREADS);
+  hipLaunchKernelGGL((k_sortp_make_keys<BITS, CHAIN_THREADS, 1, true>), g, b, 0, st, c, n, s, sc, idx_bits, passes, buf_a, hist, n_blocks);
+  hipLaunchKernelGGL((k_sortp_chain<BITS, true>), g, b, 0, st, (const uint64_t*)buf_a, buf_b, perm, (uint32_t)n, 0u, idx_bits,
+                     (const Scalars*)sc, hist, n_blocks);
+  uint64_t* in = buf_b; uint64_t* out = buf_a;
+  for (uint32_t p = 1; p < passes; ++p) {
+    hipLaunchKernelGGL((k_sortp_chain<BITS, false>), g, b, 0, st, (const uint64_t*)in, out, perm, (uint32_t)n, p, idx_bits,
+                       (const Scalars*)sc, hist, n_blocks);
     uint64_t* t = in; in = out; out = t;
   }
   return KTJ_LAUNCH_CHECK();
@@ -1824,16 +1949,19 @@ bool sort_packed_fits(uint64_t n, uint32_t key_bits) {
 }
 uint32_t sort_packed_passes(uint32_t key_bits) { return (key_bits + SORTP_BITS) / SORTP_BITS; }
 hipError_t sort_packed(Columns c, uint64_t n, SortSets s, Scalars* sc, uint32_t passes, uint64_t* buf_a, uint64_t* buf_b, uint32_t* perm,
-                       uint32_t* hist, hipStream_t st) {
+                       uint32_t* hist, uint32_t* chain_hist, hipStream_t st) {
   if (n == 0) return hipSuccess;
   const uint32_t idx_bits = sort_idx_bits(n);
   if (n <= (uint64_t)SORTP_THREADS * 16u && !g_sortp_no_single) {
     hipLaunchKernelGGL((k_sortp_single<SORTP_BITS, SORTP_THREADS, 16>), dim3(1), dim3(SORTP_THREADS), 0, st, c, (uint32_t)n, s, sc, perm);
     return KTJ_LAUNCH_CHECK();
   }
-  /* a few thousand keys are one tile; up to SORTP_SMALL_N keys, tiles of 512 spread over the GPU
+  /* a few thousand keys are one tile; then one launch a pass, where the counts of all passes (1 KiB per pass and
+   * tile) fit the 8 bytes per row of chain_hist: eight passes of an odd few thousand keys do not; up to SORTP_SMALL_N keys, tiles of 512 spread over the GPU
    * finish a pass sooner than the few 4096-key tiles would (30 000 keys: 76 against 130 us for the
    * sort, 330 000 keys: 113 against 155 us; from a million keys on the large tiles win) */
+  if (n > (uint64_t)SORTP_THREADS * 16u && n <= CHAIN_MAX_N && 256ull * passes * ((n + CHAIN_THREADS - 1) / CHAIN_THREADS) <= 2 * (n + 1))
+    return sort_packed_chain<SORTP_BITS>(c, n, s, sc, passes, idx_bits, buf_a, buf_b, perm, chain_hist, st);
   if (n > (uint64_t)SORTP_THREADS * 16u && n < SORTP_SMALL_N)
     return sort_packed_t<SORTP_BITS, SORTP_THREADS, 2>(c, n, s, sc, passes, idx_bits, buf_a, buf_b, perm, hist, st);
   return sort_packed_t<SORTP_BITS, SORTP_THREADS, 16>(c, n, s, sc, passes, idx_bits, buf_a, buf_b, perm, hist, st);

@@ -78,6 +78,16 @@ def test_later_records_need_more(late, sync):
         check(eng, want, counters)
 
 
+# sorts with one launch a pass: a last tile of one key, the most keys and one more; a digit that all keys share
+@pytest.mark.parametrize("rows,bits", [(5121, 30), (5121, 55), (131072, 30), (131073, 30), (131072, 55), (20000, 1)])
+def test_sort_of_one_launch_a_pass(rows, bits):
+    sp = ops([(k * 0x9E3779B97F4A7C15) % (1 << 64) >> (64 - bits) for k in range(rows)])
+    want, counters = oracle(sp)
+    with TraceEngine(sp.contents.trace_name.decode(), base_time_ns=sp.contents.base_time_ns) as eng:
+        eng.submit_stream(sp)
+        check(eng, want, counters)
+
+
 def test_document_longer_than_the_first_buffer():
     from stream_builder import B, StreamBuilder
     b = StreamBuilder()
