@@ -1528,8 +1528,9 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
   HIPCHK(join_runtime_rows(r_recs, nr, c, ng, api, tf, fc, tn, nc, e->slot_f.as<uint32_t>(), e->slot_n.as<uint32_t>(), ctx, mat,
                            e->len.as<uint32_t>(), sc, st));
   HIPCHK(republish_runtime_rows(r_recs, nr, c, ng, fc, nc, e->slot_f.as<uint32_t>(), e->slot_n.as<uint32_t>(), sc, st));
-  HIPCHK(link_device_rows(nd, c, ng + nr, tf, fc, tn, nc, e->dev_link.as<DevLink>(), sc, st));
-  HIPCHK(backfill_streams(e->dev_brief.as<DevBrief>(), nd, c, ng + nr, tf, fc, e->dev_link.as<DevLink>(), stt, sc, st));
+  unsigned long long* orphans = e->keys_a.as<unsigned long long>(); /* a bit per device row: the sort's words come later */
+  HIPCHK(link_device_rows(nd, c, ng + nr, tf, fc, tn, nc, e->dev_link.as<DevLink>(), orphans, sc, st));
+  HIPCHK(backfill_streams(e->dev_brief.as<DevBrief>(), nd, c, ng + nr, tf, fc, orphans, stt, sc, st));
   if (max_spans) {
     const int rc = synthesise_user_spans(e, c, ctx, t_cpu, cpu_row, sc, N);
     if (rc != KTJ_OK) return rc;

@@ -99,7 +99,6 @@ struct DevBrief {
 };                         /* 16 bytes */
 #define KTJ_DL_HAS_SIZE 1u
 #define KTJ_DL_HAS_GRID 2u
-#define KTJ_DL_ORPHAN 4u   /* no runtime row has the id: the order check runs in a pass of its own */
 
 /* columns in arrival order: generic rows, then runtime rows, then device rows */
 struct Columns {
@@ -263,7 +262,7 @@ hipError_t collective_first(const MatRow* mat, const uint32_t* perm, uint64_t n_
 /* per device row: "External id", timestamp-order check, stream of the launching row, and the
  * size / grid hand-over (into link[]) */
 hipError_t link_device_rows(uint64_t n, Columns c, uint64_t first_device, Table tf, FullCols fc, Table tn, NarrowCols nc,
-                            DevLink* link, Scalars* sc, hipStream_t st);
+                            DevLink* link, unsigned long long* orphans /* a bit per row */, Scalars* sc, hipStream_t st);
 /* stream back-fill: queue table (keys/vals/ambiguous) and dense table are caller-provided, zeroed */
 struct StreamTables {
   uint64_t* q_keys;   /* KTJ_QUEUE_CAP + 1, filled with KTJ_EMPTY_KEY */
@@ -277,7 +276,7 @@ struct StreamTables {
   uint32_t* d_list;   /* KTJ_MAX_STREAM_PAIRS: slots of the pairs */
 };
 /* also checks the device rows whose id no runtime row has (tf, fc, link) */
-hipError_t backfill_streams(const DevBrief* d, uint64_t n, Columns c, uint64_t first_device, Table tf, FullCols fc, const DevLink* link,
+hipError_t backfill_streams(const DevBrief* d, uint64_t n, Columns c, uint64_t first_device, Table tf, FullCols fc, const unsigned long long* orphans,
                             StreamTables t, Scalars* sc, hipStream_t st);
 
 /* ---- GPU user annotations (GenericActivityProfiler.cpp:277-327, 423-433): one span per

@@ -653,7 +653,7 @@ __global__ void k_resolve_external(const ktj_extcorr_rec* e, uint64_t n, Table t
  * checked afterwards by k_device_orphans.  Rows outside the window still take a stream from the
  * slot (slots with a stream come from runtime rows and exist already). */
 __global__ void k_link_device(uint64_t n, Columns c, uint64_t first_device, Table tf, FullCols fc, Table tn, NarrowCols nc,
-                              DevLink* link, Scalars* sc) {
+                              DevLink* link, unsigned long long* orphans, Scalars* sc) {
   uint32_t n_linked = 0, n_bad = 0, n_unresolved = 0, n_orphans = 0;
   const bool have_stream_src = sc->have_stream_src != 0;
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) {
@@ -689,6 +689,7 @@ __global__ void k_link_device(uint64_t n, Columns c, uint64_t first_device, Tabl
       }
       l.coll = np.info >> KTJ_NP_COLL_SHIFT;
     }
+    bool orphan = false;
     store_once(&c.ext[a], np.ext_val);
     if (valid && sf == KTJ_NOSLOT) flag_error(sc, KTJ_DEVERR_TABLE_FULL);
     if (sf != KTJ_NOSLOT) {
@@ -698,7 +699,7 @@ __global__ void k_link_device(uint64_t n, Columns c, uint64_t first_device, Tabl
           if (t2 != 0 && t1 > t2) ++n_bad;
         } else {
           if (fc.first[sf] > (uint32_t)a) atomicMin(&fc.first[sf], (uint32_t)a);
-          l.flags |= KTJ_DL_ORPHAN;
+          orphan = true;
           ++n_orphans;
         }
       }
@@ -713,6 +714,10 @@ __global__ void k_link_device(uint64_t n, Columns c, uint64_t first_device, Tabl
       store_once(&dst[1], lv[1]);
     }
     if (is_async_op(domain) && res == 0) ++n_unresolved;
+    /* a bit per row, for k_after_link: with the flag in the 32-byte link it read 352 MB to find the few of 11 M
+     * rows (127 us, now 25); a wavefront's rows are 64 in a row */
+    const unsigned long long some = __ballot(orphan);
+    if (lane_id() == 0) orphans[i >> 6] = some;
   }
   block_add(sc, KTJ_CNT_LINKED, n_linked);
   block_add(sc, KTJ_CNT_OUT_OF_ORDER, n_bad);
@@ -725,14 +730,14 @@ __global__ void k_link_device(uint64_t n, Columns c, uint64_t first_device, Tabl
  *  - a row without a stream may take its queue's (RocmStreamQueue.h:42-136; the first pass of that, the
  *    stream of the correlation-matched runtime row, is part of k_link_device): which stream every queue
  *    shows, ambiguous when one queue shows two different ones. */
-__global__ void k_after_link(uint64_t n, Columns c, uint64_t first_device, Table tf, FullCols fc, const DevLink* link, const DevBrief* d,
-                             StreamTables t, Scalars* sc) {
+__global__ void k_after_link(uint64_t n, Columns c, uint64_t first_device, Table tf, FullCols fc, const unsigned long long* orphan_rows,
+                             const DevBrief* d, StreamTables t, Scalars* sc) {
   const bool orphans = sc->n_device_orphans != 0, queues = sc->have_stream_src != 0 && sc->n_unresolved != 0;
   uint32_t n_bad = 0;
   if (orphans || queues)
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) {
       const uint64_t a = first_device + i;
-      if (orphans && (link[i].flags & KTJ_DL_ORPHAN)) {
+      if (orphans && (orphan_rows[i >> 6] >> (i & 63u) & 1ULL)) {
         const uint32_t sf = slot_find(tf, c.corr[a]);
         const uint64_t f = sf != KTJ_NOSLOT ? fc.first[sf] : a;
         if (f != a && f != 0xFFFFFFFFull) {
@@ -771,10 +776,10 @@ hipError_t build_extcorr(const ktj_extcorr_rec* e, uint64_t n, Table tn, NarrowC
   return KTJ_LAUNCH_CHECK();
 }
 hipError_t link_device_rows(uint64_t n, Columns c, uint64_t first_device, Table tf, FullCols fc, Table tn, NarrowCols nc,
-                            DevLink* link, Scalars* sc, hipStream_t st) {
+                            DevLink* link, unsigned long long* orphans, Scalars* sc, hipStream_t st) {
   if (n == 0) return hipSuccess;
   hipLaunchKernelGGL(k_link_device, dim3(grid_stride_for(n, KTJ_BLOCK)), dim3(KTJ_BLOCK), 0, st, n, c, first_device, tf, fc, tn,
-                     nc, link, sc);
+                     nc, link, orphans, sc);
   return KTJ_LAUNCH_CHECK();
 }
 
@@ -1018,11 +1023,11 @@ __global__ void k_dense_assign(const DevBrief* d, uint64_t n, Columns c, uint64_
   c.res[a] = (int64_t)(stream != 0 ? stream : b.queue);
 }
 
-hipError_t backfill_streams(const DevBrief* d, uint64_t n, Columns c, uint64_t first_device, Table tf, FullCols fc, const DevLink* link,
+hipError_t backfill_streams(const DevBrief* d, uint64_t n, Columns c, uint64_t first_device, Table tf, FullCols fc, const unsigned long long* orphans,
                             StreamTables t, Scalars* sc, hipStream_t st) {
   if (n == 0) return hipSuccess;
   const dim3 g(grid_for(n, KTJ_BLOCK)), b(KTJ_BLOCK);
-  hipLaunchKernelGGL(k_after_link, dim3(grid_stride_for(n, KTJ_BLOCK)), b, 0, st, n, c, first_device, tf, fc, link, d, t, sc);
+  hipLaunchKernelGGL(k_after_link, dim3(grid_stride_for(n, KTJ_BLOCK)), b, 0, st, n, c, first_device, tf, fc, orphans, d, t, sc);
   /* every workgroup pays for its local table and for each pair it has seen: 2048 rows each, fewer only while
    * that leaves CUs without a workgroup, and at most four workgroups per CU */
   const unsigned few = grid_stride_for(n, KTJ_BLOCK * 2), many = grid_stride_for(n, KTJ_BLOCK * 8);
