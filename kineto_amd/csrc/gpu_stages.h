@@ -120,6 +120,7 @@ struct SortPlan { unsigned int ts_bits, res_bits, key_bits; }; /* of the composi
 /* wall clock (wall_clock64) at the points of a pass: its start and the start of each stage; the runs of
  * small.hip name their own */
 enum { KTJ_CLOCK_BEGIN = 0, KTJ_CLOCK_DECODE, KTJ_CLOCK_JOIN, KTJ_CLOCK_SORT, KTJ_CLOCK_SIZE, KTJ_CLOCK_SCAN, KTJ_CLOCK_EMIT, KTJ_CLOCK_COUNT };
+#define KTJ_RANGE_TS 4 /* place of the timestamps' range (biased) behind those of the join tables in Scalars::range_shard */
 enum { KTJ_DONE_DENSE = 0, KTJ_DONE_COLLECT, KTJ_DONE_COUNT };
 struct Scalars {
   unsigned long long ts_min_biased;   /* min over valid rows of ts ^ 2^63 */
