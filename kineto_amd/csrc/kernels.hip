@@ -650,7 +650,7 @@ __global__ void k_resolve_external(const ktj_extcorr_rec* e, uint64_t n, Table t
  * The first row of an id is its first runtime row wherever one exists (runtime rows arrive before
  * device rows), which a bitmap tells, and the slot's payload holds that row's timestamp, so the
  * array of first rows is only touched for ids that no runtime row has: in-window device rows take part in "first seen" there and are
- * checked afterwards by k_device_orphans.  Rows outside the window still take a stream from the
+ * checked afterwards by k_after_link.  Rows outside the window still take a stream from the
  * slot (slots with a stream come from runtime rows and exist already). */
 __global__ void k_link_device(uint64_t n, Columns c, uint64_t first_device, Table tf, FullCols fc, Table tn, NarrowCols nc,
                               DevLink* link, unsigned long long* orphans, Scalars* sc) {
@@ -1980,9 +1980,9 @@ hipError_t sort_packed(Columns c, uint64_t n, SortSets s, Scalars* sc, uint32_t 
     return KTJ_LAUNCH_CHECK();
   }
   /* a few thousand keys are one tile; then one launch a pass, where the counts of all passes (1 KiB per pass and
-   * tile) fit the 8 bytes per row of chain_hist: eight passes of an odd few thousand keys do not; up to SORTP_SMALL_N keys, tiles of 512 spread over the GPU
-   * finish a pass sooner than the few 4096-key tiles would (30 000 keys: 76 against 130 us for the
-   * sort, 330 000 keys: 113 against 155 us; from a million keys on the large tiles win) */
+   * tile) fit the 8 bytes per row of chain_hist: eight passes of an odd few thousand keys do not.  Up to
+   * SORTP_SMALL_N keys, tiles of 512 spread over the GPU finish a pass sooner than the few 4096-key tiles
+   * would (330 000 keys: 113 against 155 us; from a million keys on the large tiles win) */
   if (n > (uint64_t)SORTP_THREADS * 16u && n <= CHAIN_MAX_N && 256ull * passes * ((n + CHAIN_THREADS - 1) / CHAIN_THREADS) <= 2 * (n + 1))
     return sort_packed_chain<SORTP_BITS>(c, n, s, sc, passes, idx_bits, buf_a, buf_b, perm, chain_hist, st);
   if (n > (uint64_t)SORTP_THREADS * 16u && n < SORTP_SMALL_N)

@@ -55,7 +55,7 @@ __device__ __forceinline__ uint32_t lds_find(const uint32_t* table, uint32_t mas
 }
 
 /* The steps and their rules are those of the kernels of a large trace (k_build_cpu_ids, k_build_extcorr,
- * k_join_runtime with its winners, k_link_device, k_device_orphans, k_queue_*, k_dense_*); here the
+ * k_join_runtime with its winners, k_link_device, k_after_link, k_dense_*); here the
  * winner of every slot is always known before it is read, so there is one form of each step. */
 __global__ void __launch_bounds__(SMALL_JOIN_THREADS) k_small_join(SmallArgs A) {
   if (blockIdx.x != 0) {
