@@ -1373,6 +1373,9 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
   e->N = N;
   e->n_spans = 0;
   e->host_copy_valid = false;
+  /* The document of the pass before may lie in a buffer of ktj_process_noalloc's caller, which that caller has had
+   * back since: a pass of ktj_process begins with the engine's own buffer (or none). */
+  if (!out_device) e->out.unborrow();
   const uint64_t Na = N + max_spans ? N + max_spans : 1;
 
   /* small tables */
@@ -1705,7 +1708,7 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
   if (out_device) { /* the caller's buffer: whole 16-byte blocks are stored, so a little room past the end is needed */
     if (e->total_bytes + 64 > out_cap) return short_output(e);
     e->out.borrow(out_device, out_cap);
-  } else NEED(e->out, e->total_bytes + 64);
+  } else HIPCHK(e->out.ensure(e->total_bytes + 64)); /* never a piece of the pool, which the next pass deals out anew */
   const size_t small = prefix.size() + suffix.size() + 64; /* each piece starts where its place in the document does, modulo 16 */
   { const int rc = ensure_text(e, small); if (rc != KTJ_OK) return rc; }
   {
