@@ -885,6 +885,10 @@ hipError_t span_members(const ktj_extcorr_rec* u, uint64_t n_device, Columns c, 
   return KTJ_LAUNCH_CHECK();
 }
 
+/* This wavefront's stores and atomics have been carried out.  A barrier of the workgroup does not say that, and a
+ * fence waits for those of the wavefront it is in only: where one thread speaks for the workgroup afterwards, every
+ * wavefront has to come by here before the barrier. */
+__device__ __forceinline__ void wave_stores_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 /* Every workgroup of a launch reports here when its results are in memory; true in all threads of the one
  * that reports last.  What that one reads of the others must have been written with atomics or agent_store()
  * and be read with agent_load(): these pass the caches of one XCD by.  (A fence for ordinary stores writes
@@ -894,7 +898,7 @@ template <typename T> __device__ __forceinline__ void agent_store(T* p, T v) { _
 template <typename T> __device__ __forceinline__ T agent_load(const T* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ __forceinline__ bool last_workgroup(unsigned int* done) {
   __shared__ int last;
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); /* the wavefront's own are there */
+  wave_stores_done();
   __syncthreads();
   if (threadIdx.x == 0) last = __hip_atomic_fetch_add(done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1u ? 1 : 0;
   __syncthreads();
@@ -2644,9 +2648,10 @@ k_copy_parts(const uint4* src, uint64_t n16, uint64_t first, uint64_t last, uint
     const uint4* s = src + from;
     uint4* d = slots + (uint64_t)slot * part16;
     for (uint64_t k = (uint64_t)blockIdx.x * KTJ_BLOCK + threadIdx.x; k < len; k += (uint64_t)gridDim.x * KTJ_BLOCK) d[k] = s[k];
+    wave_stores_done();
     __syncthreads();
     if (threadIdx.x == 0) {
-      __threadfence_system(); /* this workgroup's share is in host memory before it counts as done */
+      __threadfence_system(); /* this workgroup's share, all of it stored by now, is in host memory before it counts as done */
       if (atomicAdd(&done[slot], 1u) == gridDim.x - 1u) {
         done[slot] = 0;
         __threadfence_system();

@@ -33,3 +33,41 @@ def test_document_reaches_the_host_whole(tmp_path, config, rows):
         with open(path, "rb") as f:
             assert f.read() == first
     release()
+
+
+def test_two_engines_copy_at_once(tmp_path):
+    """Two threads, an engine each, their documents (more parts than slots, fewer) crossing at the same time, again and
+    again into a buffer that held something else, and into a file."""
+    import threading
+    failures = []
+    start = threading.Barrier(2)
+
+    def work(name, config, rows):
+        try:
+            sp, release = abi.synth_stream(config, rows, host_name=name)
+            path = str(tmp_path / (name + ".json"))
+            with TraceEngine(path, device=0, no_file=False) as eng, TraceEngine(path, device=0) as other:
+                other.submit_stream(sp)
+                other.process()
+                want = other.output_view()
+                eng.submit_stream(sp)
+                eng.process()
+                dst, n = np.empty(len(want), dtype=np.uint8), abi.C.c_uint64()
+                start.wait(60)
+                for k in range(8):
+                    dst.fill(k)
+                    eng._chk(eng.lib.ktj_output_copy(eng.h, dst.ctypes.data, len(dst), abi.C.byref(n)), "ktj_output_copy")
+                    assert n.value == len(want) and np.array_equal(dst, want), "copy %d of %s" % (k, name)
+                assert eng.finalize() == len(want)
+                assert np.array_equal(np.fromfile(path, dtype=np.uint8), want), "the file of " + name
+            release()
+        except BaseException as x:
+            failures.append(x)
+            start.abort()
+
+    threads = [threading.Thread(target=work, args=a) for a in (("long", 2, 20000), ("short", 1, 6700))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failures, failures
