@@ -1549,14 +1549,18 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
    * collective entries (the footer names those in use) and synthesised spans, and what else only the
    * device sees, it flags: more sort passes than launched, keys too wide for the one-word sort, CUDA_SYNC
    * activities, too many distinct values.  Such records take the stepwise rest of the pass from here on. */
-  bool straight = n_coll == 0 && max_spans == 0 && !e->stepwise && !(e->flags & KTJ_CREATE_TILE_EMIT) && e->sort_mode != 1;
-  HIPCHK(collect_distinct(c, N, sets, sc, straight, st));
-  if (!out_device && !e->noalloc && e->out.cap == 0) {
+  bool has_room = true;
+  if (!out_device && e->out.cap == 0) {
     /* An engine's first pass has no document buffer yet, and how long the document is comes out of
      * the scan.  A first guess is allocated here, while the GPU is busy with the join.  If that turns out too
-     * small (or cannot be had) the buffer is allocated where its size is known, as in later passes. */
-    if (e->out.ensure(N * guess_per_row(e) + (1u << 20), false) != hipSuccess) { (void)hipGetLastError(); straight = false; }
+     * small the buffer is allocated where its size is known, as in later passes; if it cannot be had, the
+     * stepwise rest does that from the start. */
+    has_room = e->out.ensure(N * guess_per_row(e) + (1u << 20), false) == hipSuccess;
+    if (!has_room) (void)hipGetLastError();
   }
+  /* (settled here: collect_distinct flags what only a host that does not look would get wrong) */
+  const bool straight = has_room && n_coll == 0 && max_spans == 0 && !e->stepwise && !(e->flags & KTJ_CREATE_TILE_EMIT) && e->sort_mode != 1;
+  HIPCHK(collect_distinct(c, N, sets, sc, straight, st));
   bool emitted = false;
   if (straight) {
     const std::string prefix = e->txt_header + e->txt_before;
