@@ -2476,10 +2476,10 @@ hipError_t republish_runtime_rows(const ktj_runtime_rec* r, uint64_t n, Columns 
 }
 /* The activities' offsets from their lengths and the tiles' sums.  Few tiles: every workgroup adds up the
  * sums before its own (OFFS_DIRECT_TILES of them are 16 KB from the L2), many: k_scan_of_sums has run.
- * One more workgroup than tiles knows the total: with a document to prepare (out != null) it puts the footer
- * text behind the activities and hands the scalars to the host, and more of them put the header, 4 KiB each
- * (all of that takes some microseconds over the host link, which the offsets need not wait for; 40 KB of
- * header by one workgroup took 20 us). */
+ * The workgroups behind the tiles' know the total: with a document to prepare (out != null) the first of them
+ * puts the footer text behind the activities and hands the scalars to the host, and the others put the header,
+ * 4 KiB each (all of that takes some microseconds over the host link, which the offsets need not wait for; 40 KB
+ * of header by one workgroup took 20 us). */
 #define PREFIX_PIECE 4096u
 #define OFFS_DIRECT_TILES 2048u
 __device__ void publish_scalars(Scalars* sc, Scalars* h_sc, bool document_fits);
@@ -2487,27 +2487,29 @@ __global__ void __launch_bounds__(KTJ_BLOCK)
 k_offsets(const uint32_t* len, uint64_t n, const uint64_t* sums, uint32_t n_tiles, uint64_t* offs, Scalars* sc, DocText T) {
   __shared__ uint64_t lds_wave[SCAN_MAX_WAVES];
   __shared__ uint64_t s_before;
-  if (blockIdx.x > n_tiles) {
-    const uint64_t at = (uint64_t)(blockIdx.x - n_tiles - 1u) * PREFIX_PIECE, left = T.n_prefix - at;
-    if (T.n_prefix + 64u <= T.out_cap) put_text_block(T.prefix + at, T.out + at, left < PREFIX_PIECE ? left : PREFIX_PIECE);
-    return;
-  }
   const bool ok = sc->error == 0; /* otherwise there are no lengths: only the host is told */
+  const uint32_t tile = blockIdx.x < n_tiles ? blockIdx.x : n_tiles; /* behind the tiles: all of them */
   uint64_t before = 0;
   if (n_tiles <= OFFS_DIRECT_TILES) {
     unsigned long long s = 0;
-    if (ok) for (uint32_t k = threadIdx.x; k < blockIdx.x; k += KTJ_BLOCK) s += sums[k];
+    if (ok) for (uint32_t k = threadIdx.x; k < tile; k += KTJ_BLOCK) s += sums[k];
     for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
     if (lane_id() == 0) lds_wave[threadIdx.x >> 6] = s;
     __syncthreads();
     if (threadIdx.x == 0) { uint64_t b = 0; for (uint32_t k = 0; k < (KTJ_BLOCK >> 6); ++k) b += lds_wave[k]; s_before = b; }
     __syncthreads();
     before = s_before;
-  } else before = ok ? sums[blockIdx.x] : 0;
-  if (blockIdx.x == n_tiles) {
+  } else before = ok ? sums[tile] : 0;
+  if (blockIdx.x >= n_tiles) {
+    /* no text where the document does not fit or there is none: the buffer stays as it was */
+    const bool fits = ok && T.n_prefix + before + T.n_suffix + 64u <= T.out_cap;
+    if (blockIdx.x > n_tiles) {
+      const uint64_t at = (uint64_t)(blockIdx.x - n_tiles - 1u) * PREFIX_PIECE, left = T.n_prefix - at;
+      if (fits) put_text_block(T.prefix + at, T.out + at, left < PREFIX_PIECE ? left : PREFIX_PIECE);
+      return;
+    }
     if (threadIdx.x == 0) offs[n] = before;
     if (!T.out) return;
-    const bool fits = ok && T.n_prefix + before + T.n_suffix + 64u <= T.out_cap;
     publish_scalars(sc, T.h_sc, fits);
     if (threadIdx.x == 0) *T.h_total = before;
     if (fits) put_text_block(T.suffix, T.out + T.n_prefix + before, T.n_suffix);

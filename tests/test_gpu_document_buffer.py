@@ -70,6 +70,32 @@ def test_process_leaves_the_buffer_of_an_earlier_call_alone(way):
     release()
 
 
+# three launches; in one go; in one go as far as that goes, then step by step
+@pytest.mark.parametrize("way", ["small", "one_go", "stepwise"])
+def test_a_buffer_that_is_too_short_stays_as_it_was(way):
+    import torch
+    release = lambda: None
+    if way == "stepwise":
+        sp = with_stream_sync(5000)
+    else:
+        sp, release = abi.synth_stream(1, 3000 if way == "one_go" else 200, host_name="owner")
+    want = oracle_document(sp)
+    with TraceEngine(sp.contents.trace_name.decode(), base_time_ns=sp.contents.base_time_ns) as eng:
+        eng.submit_stream(sp)
+        out = torch.full((len(want) + 4096,), 0xA5, dtype=torch.uint8, device="cuda:0")
+        n = C.c_uint64()
+        for cap in (len(want) // 2, len(want) + 63, 16):
+            for _ in range(2):
+                rc = eng.lib.ktj_process_noalloc(eng.h, eng.end_time_ns, out.data_ptr(), cap, C.byref(n))
+                assert rc == abi.KTJ_ERR_LIMIT and n.value == len(want) and b"output buffer" in eng.lib.ktj_last_error(eng.h)
+            assert bool((out == 0xA5).all()), "a part of the document in a buffer of %d bytes" % cap
+        rc = eng.lib.ktj_process_noalloc(eng.h, eng.end_time_ns, out.data_ptr(), len(want) + 64, C.byref(n))
+        assert rc == 0 and n.value == len(want)
+        same(bytes(out[:n.value].cpu().numpy()), want)
+        assert bool((out[n.value + 64:] == 0xA5).all())
+    release()
+
+
 def test_document_of_a_stepwise_pass_is_not_working_memory_of_the_next():
     """A few records with long names go step by step behind a pass that left much working memory; then many
     records with short names, whose document fits where the first one was."""
