@@ -1311,6 +1311,7 @@ static int process_small(ktj_engine* e, int64_t end_time_ns, void* out_device, u
   a.mat = e->mat.as<MatRow>(); a.len = e->len.as<uint32_t>(); a.perm = e->vals_a.as<uint32_t>();
   a.sc = sc;
   text.out = e->out.as<char>(); text.out_cap = e->out.cap;
+  e->h_ctl->end_clock = 0;
   HIPCHK(small_pass(a, ns, st));
   HIPCHK(small_emit(a, text, st));
   HIPCHK(hipStreamSynchronize(st));

@@ -706,25 +706,28 @@ __global__ void __launch_bounds__(KTJ_BLOCK) k_small_emit(const MatRow* mat, con
   if (blockIdx.x + 2u >= gridDim.x) {
     if (blockIdx.x + 2u == gridDim.x) put_text_block(T.prefix, T.out, T.n_prefix);
     else put_text_block(T.suffix, T.out + T.n_prefix + total, T.n_suffix);
+    if (threadIdx.x == 0) *T.h_end = wall_clock64();
     return;
   }
   const uint32_t p = __builtin_amdgcn_readfirstlane(blockIdx.x * (KTJ_BLOCK >> 6) + (threadIdx.x >> 6));
   if (p >= n) return;
   const uint32_t row = __builtin_amdgcn_readfirstlane(perm[p]);
-  if (__builtin_amdgcn_readfirstlane(len[row]) & SMALL_LEN_PLAIN) return; /* k_small_plain's */
-  const MatRow m = mat[row];
-  doc_ptr at = reinterpret_cast<doc_ptr>((uintptr_t)(T.out + T.n_prefix + offs[p]));
-  SegWriter w;
-  w.lane = lane_id();
-  w.start();
-  ActivityParts<SegWriter> parts;
-  format_head(w, m, ctx, parts);
-  at += w.flush(at);
-  format_args(w, m, ctx, parts);
-  at += w.flush(at);
-  format_flow(w, m, ctx, parts);
-  w.flush(at);
-  if (threadIdx.x == 0) *T.h_end = wall_clock64(); /* the last workgroup's stays */
+  if (!(__builtin_amdgcn_readfirstlane(len[row]) & SMALL_LEN_PLAIN)) { /* those are k_small_plain's */
+    const MatRow m = mat[row];
+    doc_ptr at = reinterpret_cast<doc_ptr>((uintptr_t)(T.out + T.n_prefix + offs[p]));
+    SegWriter w;
+    w.lane = lane_id();
+    w.start();
+    ActivityParts<SegWriter> parts;
+    format_head(w, m, ctx, parts);
+    at += w.flush(at);
+    format_args(w, m, ctx, parts);
+    at += w.flush(at);
+    format_flow(w, m, ctx, parts);
+    w.flush(at);
+  }
+  /* what arrives last stays: the pass's end, to within what the other wavefronts of that workgroup still have to do */
+  if (threadIdx.x == 0) *T.h_end = wall_clock64();
 }
 /* Only when the rows have shown activities with more pieces than lanes (InputShapes of many operands,
  * long arrays): one lane per workgroup writes each of them. */
@@ -741,6 +744,7 @@ __global__ void __launch_bounds__(KTJ_BLOCK) k_small_plain(const MatRow* mat, co
     w.p = reinterpret_cast<doc_ptr>((uintptr_t)(T.out + T.n_prefix + offs[p]));
     format_activity(w, m, ctx);
   }
+  if (threadIdx.x == 0) *T.h_end = wall_clock64();
 }
 
 hipError_t small_pass(const SmallArgs& a, uint32_t n_strings, hipStream_t st) {

@@ -70,3 +70,24 @@ def test_document_longer_than_the_first_buffer():
     for k in range(60):
         b.add_generic(names[-1], 5, B + k, B + k + 10, 0, 1, id=k + 1)
     check(b.build())
+
+
+@pytest.mark.parametrize("elements,dropped", [(1, False), (400, False), (400, True)])
+def test_pass_has_a_time(elements, dropped):
+    """Also where one wavefront after the other writes all of its activities, and where none is printed."""
+    from stream_builder import B, StreamBuilder
+    b = StreamBuilder(window=(B + 10**6, None) if dropped else (None, None))
+    schema = b.schema([("values", abi.F_I64_ARRAY, elements)])
+    for k in range(9):
+        if dropped:
+            b.add_device(k + 1, B + 10 * k, B + 10 * k + 5, name="kernel")
+        else:
+            b.add_generic("op %d" % k, 0, B + 1000 * k, B + 1000 * k + 500, 1, 2, id=k + 1, schema=schema, values=list(range(elements)))
+    sp = b.build()
+    with TraceEngine("t.json") as eng:
+        eng.submit_stream(sp)
+        for _ in range(2):
+            eng.process()
+            ms = eng.stats().stage_ms
+            assert 0 < ms[abi.STAGE_NAMES.index("emit")] <= ms[abi.STAGE_NAMES.index("total_gpu")] < 60000
+        assert eng.stats().n_emitted == (0 if dropped else 9)
