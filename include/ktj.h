@@ -472,15 +472,15 @@ typedef struct ktj_engine ktj_engine;
  * reports the time of the whole pass only (stage_ms[KTJ_STAGE_TOTAL_GPU]), and a trace of a few
  * records is finished a tenth sooner.
  *
- * ktj_destroy leaves what every engine needs before its first record (its stream and events, the
- * small page-locked buffers, 1 to 64 MiB of device memory for inputs), the 16 or 64 MiB of
- * page-locked staging for larger submissions and documents if the engine made one, and, up to
- * 512 MiB together, the working memory and the document buffer of its last pass behind
- * for the next ktj_create on the same device, which starts from them instead of allocating: one
- * such set per device, held until the process ends (working memory and document buffer only until
- * sixteen engines in a row have needed less than an eighth of them, or an allocation fails).  A trace of a few records otherwise spends
- * more time creating and destroying these than on the GPU.  Nothing is kept of an engine that saw
- * a HIP error.
+ * ktj_destroy leaves what every engine needs before its first record behind for the next ktj_create on
+ * the same device, which starts from it instead of allocating (a trace of a few records otherwise spends
+ * more time creating and destroying these than on the GPU): one such set per device.  Until the process
+ * ends it holds a stream, its events and at most 2.5 MiB of page-locked buffers.  Besides, the device
+ * memory of the engine that left it: up to 64 MiB for inputs and, up to 512 MiB together, the working memory
+ * and the document buffer of its last pass.  These are given back when sixteen engines in a row have
+ * needed less than an eighth of them (above 64 MiB), when an allocation of this library fails, and by
+ * ktj_trim; so are, by ktj_trim only, the 16 or 64 MiB of page-locked staging for larger submissions
+ * and documents if the engine made one.  Nothing is kept of an engine that saw a HIP error.
  * ---------------------------------------------------------------------------------------- */
 #define KTJ_CREATE_NO_FILE 0x1u
 #define KTJ_CREATE_TILE_EMIT 0x2u
@@ -492,6 +492,11 @@ typedef struct ktj_engine ktj_engine;
 int ktj_create(ktj_engine** out, const char* out_path, int64_t base_time_ns, int hip_device,
                uint32_t flags);
 void ktj_destroy(ktj_engine* e);
+
+/* Gives back the memory that waits for the next engine on this device (see above), for a program that
+ * needs it elsewhere now: between captures, or when another allocator of the process has run out.  Engines
+ * that exist keep theirs; the next one allocates anew.  May be called from any thread. */
+int ktj_trim(int hip_device);
 const char* ktj_last_error(const ktj_engine* e);
 
 /* ChromeTraceLogger::handleTraceStart (output_json.cpp:445-479).  meta_kv holds n_kv key/value

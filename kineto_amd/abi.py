@@ -198,7 +198,7 @@ def load_synth():
 
 
 ENGINE_SYMBOLS = [
-    "ktj_create", "ktj_destroy", "ktj_last_error", "ktj_trace_start", "ktj_intern_strings",
+    "ktj_create", "ktj_destroy", "ktj_trim", "ktj_last_error", "ktj_trace_start", "ktj_intern_strings",
     "ktj_register_schema", "ktj_add_collective", "ktj_submit_args", "ktj_set_api_table", "ktj_set_clock_model",
     "ktj_set_window", "ktj_submit_records", "ktj_submit_records_device", "ktj_host_alloc", "ktj_host_free", "ktj_submit_info", "ktj_submit_stream", "ktj_begin_activities",
     "ktj_process", "ktj_process_noalloc", "ktj_output_device", "ktj_output_host", "ktj_output_copy", "ktj_finalize", "ktj_get_stats",
@@ -221,6 +221,8 @@ def load_engine():
         lib.ktj_create.argtypes = [C.POINTER(vp), C.c_char_p, C.c_int64, C.c_int, C.c_uint32]
         lib.ktj_destroy.restype = None
         lib.ktj_destroy.argtypes = [vp]
+        lib.ktj_trim.restype = C.c_int
+        lib.ktj_trim.argtypes = [C.c_int]
         lib.ktj_last_error.restype = C.c_char_p
         lib.ktj_last_error.argtypes = [vp]
         lib.ktj_trace_start.restype = C.c_int

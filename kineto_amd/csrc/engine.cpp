@@ -37,7 +37,7 @@ using namespace ktj::gpu;
 namespace {
 
 #define KTJ_INPUT_ARENA_BYTES (1ull << 20)     /* device memory for the inputs of an engine, to begin with */
-#define KTJ_INPUT_ARENA_MAX (64ull << 20)      /* what it may grow to for the engines that follow */
+#define KTJ_INPUT_ARENA_MAX (64ull << 20)      /* what it may grow to for the engines that follow, room to spare included */
 #define KTJ_STAGE_SMALL_BYTES (256u << 10) /* pinned ring that small submissions pass through */
 #define KTJ_STAGE_SMALL_MAX (64u << 10)    /* largest submission that does */
 /* large submissions: pinned chunks, two per copying thread.  Measured for 1.9 GB of records from
@@ -53,10 +53,11 @@ static_assert(KTJ_STAGE_SLOTS >= 2 * KTJ_STAGE_THREADS_MAX, "two per copying thr
  * through sixteen pinned slots of this size (the first part of the memory that large submissions use
  * whole): the copy engine works on some while the host fills or empties the others. */
 #define KTJ_STAGE_SLOT (1ull << 20)
-/* Working and document memory that waits for the next engine, per device: a thousandth of the card's
+/* Working and document memory that waits for the next engine, per device: a five-hundredth of the card's
  * memory, enough for traces of a few hundred thousand records, which otherwise spend more time in
- * hipMalloc and hipFree than on the GPU.  What KTJ_KIT_LEAN engines in a row could have done with an
- * eighth of is given back (above KTJ_KIT_SMALL_BYTES), and all of it when an allocation fails. */
+ * hipMalloc and hipFree than on the GPU.  It and the input arena are given back when KTJ_KIT_LEAN engines in
+ * a row could have done with an eighth of them (above KTJ_KIT_SMALL_BYTES), when an allocation of this library
+ * fails, and when the program asks for it (ktj_trim). */
 #define KTJ_KIT_DEVICE_BYTES_MAX (512ull << 20)
 #define KTJ_KIT_SMALL_BYTES (64ull << 20)
 #define KTJ_KIT_LEAN 16u
@@ -102,7 +103,8 @@ struct DevBuf {
 /* Device memory for an engine's inputs: one allocation that its arrays are carved out of (a trace of
  * a few records otherwise spends more time in hipMalloc than on the GPU, a session of a few
  * megabytes as much as on its copies).  Pieces are never given back; a new engine that inherits the
- * arena starts at its beginning, and finds it large enough for what its predecessor asked for. */
+ * arena starts at its beginning, and finds it large enough for what its predecessor asked for (as far as
+ * KTJ_INPUT_ARENA_MAX goes; an engine whose kit had given the arena back does without). */
 struct InputArena {
   DevBuf mem;
   size_t used = 0, missed = 0; /* missed: what it had no room for */
@@ -115,7 +117,11 @@ struct InputArena {
     used = off + bytes;
     return static_cast<char*>(mem.p) + off;
   }
-  size_t wanted() const { const size_t w = used + missed; return missed && w <= KTJ_INPUT_ARENA_MAX && w > mem.cap ? w : 0; }
+  size_t asked() const { return used + missed; }
+  size_t wanted() const { /* by an engine like this one, with some room to spare; 0: no more than there is */
+    const size_t w = std::max<size_t>(std::min<size_t>(asked() + asked() / 4, KTJ_INPUT_ARENA_MAX), KTJ_INPUT_ARENA_BYTES);
+    return asked() <= KTJ_INPUT_ARENA_MAX && (missed || !mem.p) && w > mem.cap ? w : 0;
+  }
 };
 
 /* append-only device array fed from host memory */
@@ -645,9 +651,10 @@ int synthesise_user_spans(ktj_engine* e, Columns c, const EmitCtx& ctx, Table t_
  * the document, while they are small) costs several times what a trace of a few records takes on
  * the GPU.  ktj_destroy leaves one such set per device behind for the next ktj_create, which takes
  * it whole; a second engine alive at the same time makes its own.  Nothing of an engine that saw a
- * HIP error is kept.  Device and pinned memory that is kept: at most KTJ_KIT_DEVICE_BYTES_MAX of
- * working and document memory, the input arena, the small pinned buffers; it is held until the
- * process ends. */
+ * HIP error is kept.  What is kept until the process ends: the stream, the events, Scalars and the small
+ * pinned buffers, at most 2.5 MiB.  What may be given back before (see KTJ_KIT_LEAN): at most
+ * KTJ_KIT_DEVICE_BYTES_MAX of working and document memory, the input arena, KTJ_INPUT_ARENA_MAX at most, and,
+ * by ktj_trim only, the pinned slots, 16 or 64 MiB. */
 struct Kit {
   bool full = false;
   hipStream_t stream = nullptr;
@@ -665,17 +672,20 @@ struct Kit {
 std::mutex g_kit_mutex;
 std::map<int, Kit*>& kits() { static auto* m = new std::map<int, Kit*>(); return *m; } /* never destroyed: the runtime may be gone by then */
 
+/* the kit's device is current, its mutex held */
+bool drop_device_memory(Kit& k) {
+  const bool any = k.pool.own_cap + k.out.own_cap + k.arena_mem.own_cap != 0;
+  k.pool.release();
+  k.out.release();
+  k.arena_mem.release();
+  return any;
+}
 bool drop_waiting_memory() {
   int device = 0;
   if (hipGetDevice(&device) != hipSuccess) return false;
   std::lock_guard<std::mutex> lock(g_kit_mutex);
   auto it = kits().find(device);
-  if (it == kits().end() || !it->second->full) return false;
-  Kit& k = *it->second;
-  const bool any = k.pool.own_cap + k.out.own_cap != 0;
-  k.pool.release();
-  k.out.release();
-  return any;
+  return it != kits().end() && it->second->full && drop_device_memory(*it->second);
 }
 
 /* the engine's device is current */
@@ -708,13 +718,13 @@ void give_kit(ktj_engine* e) {
   /* back from whatever they were lent (the pool never is; the document may sit in a caller's buffer) */
   e->pool.unborrow();
   e->out.unborrow();
-  const size_t held = e->pool.own_cap + e->out.own_cap;
-  if (held > KTJ_KIT_SMALL_BYTES && (e->most_needed < held / 8)) {
-    if (++e->kit_lean >= KTJ_KIT_LEAN) { e->pool.release(); e->out.release(); e->kit_lean = 0; }
+  const size_t held = e->pool.own_cap + e->out.own_cap + e->input_arena.mem.own_cap;
+  if (held > KTJ_KIT_SMALL_BYTES && e->most_needed + e->input_arena.asked() < held / 8) {
+    if (++e->kit_lean >= KTJ_KIT_LEAN) { e->pool.release(); e->out.release(); e->input_arena.mem.release(); e->kit_lean = 0; }
   } else e->kit_lean = 0;
   if (const size_t want = e->input_arena.wanted()) { /* room for the inputs of another engine like this one */
     e->input_arena.mem.release();
-    if (e->input_arena.mem.ensure(want + want / 4, false) != hipSuccess) (void)hipGetLastError();
+    if (e->input_arena.mem.ensure(want - 256, false) != hipSuccess) (void)hipGetLastError(); /* ensure adds 256 */
   }
   std::lock_guard<std::mutex> lock(g_kit_mutex);
   Kit* slot = nullptr;
@@ -789,8 +799,8 @@ int ktj_create(ktj_engine** out, const char* out_path, int64_t base_time_ns, int
     e->stage_small = static_cast<char*>(p);
     HIPCHK(hipHostGetDevicePointer(&d, e->stage_small, 0));
     e->stage_small_dev = static_cast<char*>(d);
-    HIPCHK(e->input_arena.mem.ensure(KTJ_INPUT_ARENA_BYTES, false));
   }
+  if (!e->input_arena.mem.p) HIPCHK(e->input_arena.mem.ensure(KTJ_INPUT_ARENA_BYTES, false));
   memset(e->h_ctl, 0, sizeof(HostCtl));
   { /* this device's copy of the static scratch array (ktj_process_noalloc) */
     void* p = nullptr;
@@ -819,6 +829,22 @@ void ktj_destroy(ktj_engine* e) {
   if (e->stream) (void)hipStreamDestroy(e->stream);
   if (e->sink) { fclose(e->sink); remove(e->tmp_path.c_str()); }
   delete e;
+}
+
+int ktj_trim(int hip_device) {
+  int current = 0;
+  if (hipGetDevice(&current) != hipSuccess) return KTJ_ERR_HIP;
+  std::lock_guard<std::mutex> lock(g_kit_mutex);
+  auto it = kits().find(hip_device);
+  if (it == kits().end() || !it->second->full) return KTJ_OK;
+  if (hipSetDevice(hip_device) != hipSuccess) return KTJ_ERR_HIP;
+  Kit& k = *it->second;
+  (void)drop_device_memory(k);
+  hipError_t err = k.stage_big ? hipHostFree(k.stage_big) : hipSuccess;
+  k.stage_big = k.stage_big_dev = nullptr;
+  k.stage_big_bytes = 0;
+  if (err == hipSuccess) err = hipSetDevice(current);
+  return err == hipSuccess ? KTJ_OK : KTJ_ERR_HIP;
 }
 
 const char* ktj_last_error(const ktj_engine* e) { return e ? e->last_error.c_str() : "null engine"; }
