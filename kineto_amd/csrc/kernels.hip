@@ -2378,7 +2378,9 @@ k_mat_rows(const ktj_generic_rec* g, uint64_t ng, uint64_t first_generic, const 
   static_assert(sizeof(MatRow) >= sizeof(ktj_generic_rec) && sizeof(MatRow) >= sizeof(ktj_device_rec), "the staging area holds the records, then the joined rows");
   __shared__ uint4 stage[KTJ_BLOCK * sizeof(MatRow) / 16];
   if (blockIdx.x == 0 && threadIdx.x == 0 && clock) stage_clock(sc, KTJ_CLOCK_SIZE);
-  if (sc->error != 0) return; /* the pass ends, or the host takes another way from the sort on */
+  /* The pass ends, or the host takes another way from the sort on.  All wavefronts of a workgroup must see the same
+   * here, as they move records for each other: the one bit that this launch sets does not count. */
+  if (sc->error & ~KTJ_DEVERR_RECORD_TOO_LONG) return;
   if (GENERIC && (!DEVICE || blockIdx.x < generic_blocks))
     mat_generic_block(g, ng, first_generic, ctx, sync_first, mat, len, sc, blockIdx.x, generic_blocks, stage);
   else if (DEVICE)
