@@ -574,7 +574,7 @@ int ktj_submit_info(ktj_engine* e, int info_kind, const void* info);
 /* A whole input in one call: everything of the bundle of include/ktj_stream.h, in the order of the calls
  * that it stands for (trace start, strings, schemas, collectives, args, API table, clock, window, device,
  * resource and overhead infos, records, spans).  The bundle may be released when the call returns.
- * Status of the first of those calls that failed, KTJ_OK otherwise. */
+ * Status of the first of those calls that failed, which ktj_last_error then names; KTJ_OK otherwise. */
 struct ktj_stream;
 int ktj_submit_stream(ktj_engine* e, const struct ktj_stream* stream);
 

@@ -1167,27 +1167,43 @@ int ktj_submit_info(ktj_engine* e, int info_kind, const void* info) {
  * replay (libkineto/src/output_membuf.h:91-107): device and resource infos, the activities, the spans. */
 int ktj_submit_stream(ktj_engine* e, const ktj_stream* s) {
   if (!e || !s) return KTJ_ERR_ARG;
-  int rc = ktj_trace_start(e, s->meta_kv, s->n_meta, s->device_properties);
+  int rc = KTJ_OK;
   uint32_t id;
   uint64_t slot;
-  if (rc == KTJ_OK) rc = ktj_intern_strings(e, s->str_blob, s->str_off, s->n_strings, &id);
+  /* the calls that follow one that failed are not made; ktj_last_error says which one it was (the calls leave a
+   * text of their own only for a failed HIP call) */
+  auto call = [&](const char* name, auto make) {
+    if (rc != KTJ_OK) return;
+    rc = make();
+    if (rc != KTJ_OK) e->last_error = std::string("ktj_submit_stream: ") + name + (rc == KTJ_ERR_HIP ? ": " + e->last_error : " returned " + std::to_string(rc));
+  };
+  auto records = [&](const char* name, int rec_class, const void* packed, uint64_t n) {
+    call(name, [&] { return ktj_submit_records(e, rec_class, packed, n); });
+  };
+  auto infos = [&](const char* name, int kind, auto* first, uint64_t n) {
+    for (uint64_t i = 0; i < n && rc == KTJ_OK; ++i) call(name, [&] { return ktj_submit_info(e, kind, first + i); });
+  };
+  call("ktj_trace_start", [&] { return ktj_trace_start(e, s->meta_kv, s->n_meta, s->device_properties); });
+  call("ktj_intern_strings", [&] { return ktj_intern_strings(e, s->str_blob, s->str_off, s->n_strings, &id); });
   for (uint64_t i = 0; i < s->n_schemas && rc == KTJ_OK; ++i)
-    rc = ktj_register_schema(e, s->fields + s->schemas[i].first_field, s->schemas[i].n_fields, &id);
-  for (uint64_t i = 0; i < s->n_collectives && rc == KTJ_OK; ++i) rc = ktj_add_collective(e, &s->collectives[i], nullptr);
-  if (rc == KTJ_OK) rc = ktj_submit_args(e, s->args, s->n_args, &slot);
-  if (rc == KTJ_OK) rc = ktj_set_api_table(e, s->cid_name_ids, s->n_cids, s->flow_start_cids, s->n_flow_start, s->malloc_cid);
-  if (rc == KTJ_OK) rc = ktj_set_clock_model(e, &s->clock);
-  if (rc == KTJ_OK) rc = ktj_set_window(e, s->window_start_ns, s->window_end_ns);
-  for (uint64_t i = 0; i < s->n_device_infos && rc == KTJ_OK; ++i) rc = ktj_submit_info(e, KTJ_INFO_DEVICE, &s->device_infos[i]);
-  for (uint64_t i = 0; i < s->n_resource_infos && rc == KTJ_OK; ++i) rc = ktj_submit_info(e, KTJ_INFO_RESOURCE, &s->resource_infos[i]);
-  for (uint64_t i = 0; i < s->n_overhead_infos && rc == KTJ_OK; ++i) rc = ktj_submit_info(e, KTJ_INFO_OVERHEAD, &s->overhead_infos[i]);
-  if (rc == KTJ_OK) rc = ktj_begin_activities(e);
-  if (rc == KTJ_OK) rc = ktj_submit_records(e, KTJ_REC_GENERIC, s->generic, s->n_generic);
-  if (rc == KTJ_OK) rc = ktj_submit_records(e, KTJ_REC_RUNTIME, s->runtime, s->n_runtime);
-  if (rc == KTJ_OK) rc = ktj_submit_records(e, KTJ_REC_DEVICE, s->device, s->n_device);
-  if (rc == KTJ_OK) rc = ktj_submit_records(e, KTJ_REC_EXTCORR, s->extcorr, s->n_extcorr);
-  if (rc == KTJ_OK) rc = ktj_submit_records(e, KTJ_REC_USERCORR, s->usercorr, s->n_usercorr);
-  for (uint64_t i = 0; i < s->n_spans && rc == KTJ_OK; ++i) rc = ktj_submit_info(e, KTJ_INFO_SPAN, &s->spans[i]);
+    call("ktj_register_schema", [&] { return ktj_register_schema(e, s->fields + s->schemas[i].first_field, s->schemas[i].n_fields, &id); });
+  for (uint64_t i = 0; i < s->n_collectives && rc == KTJ_OK; ++i)
+    call("ktj_add_collective", [&] { return ktj_add_collective(e, &s->collectives[i], nullptr); });
+  call("ktj_submit_args", [&] { return ktj_submit_args(e, s->args, s->n_args, &slot); });
+  call("ktj_set_api_table",
+       [&] { return ktj_set_api_table(e, s->cid_name_ids, s->n_cids, s->flow_start_cids, s->n_flow_start, s->malloc_cid); });
+  call("ktj_set_clock_model", [&] { return ktj_set_clock_model(e, &s->clock); });
+  call("ktj_set_window", [&] { return ktj_set_window(e, s->window_start_ns, s->window_end_ns); });
+  infos("ktj_submit_info (device)", KTJ_INFO_DEVICE, s->device_infos, s->n_device_infos);
+  infos("ktj_submit_info (resource)", KTJ_INFO_RESOURCE, s->resource_infos, s->n_resource_infos);
+  infos("ktj_submit_info (overhead)", KTJ_INFO_OVERHEAD, s->overhead_infos, s->n_overhead_infos);
+  call("ktj_begin_activities", [&] { return ktj_begin_activities(e); });
+  records("ktj_submit_records (generic)", KTJ_REC_GENERIC, s->generic, s->n_generic);
+  records("ktj_submit_records (runtime)", KTJ_REC_RUNTIME, s->runtime, s->n_runtime);
+  records("ktj_submit_records (device)", KTJ_REC_DEVICE, s->device, s->n_device);
+  records("ktj_submit_records (external correlation)", KTJ_REC_EXTCORR, s->extcorr, s->n_extcorr);
+  records("ktj_submit_records (user correlation)", KTJ_REC_USERCORR, s->usercorr, s->n_usercorr);
+  infos("ktj_submit_info (span)", KTJ_INFO_SPAN, s->spans, s->n_spans);
   return rc;
 }
 
