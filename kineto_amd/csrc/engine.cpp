@@ -29,6 +29,7 @@
 #include "../../include/ktj_rocprofiler.h"
 #include "gpu_stages.h"
 #include "host_events.h"
+#include "part_queue.h"
 #include "sdk_api_rows.h"
 
 using namespace ktj;
@@ -1915,8 +1916,9 @@ struct DocumentParts {
   }
   /* part c is waited for: a launch that failed must not be waited for forever */
   hipError_t wait(uint64_t c) const {
-    for (unsigned spins = 1; !here(c); ++spins)
-      if (spins % 65536 == 0) {
+    Patience patience;
+    for (unsigned naps = 0; !here(c);)
+      if (patience.pause() && ++naps % 8 == 0) {
         const hipError_t q = hipStreamQuery(e->stream);
         if (q != hipErrorNotReady && !here(c)) return q == hipSuccess ? hipErrorUnknown : q;
       }
@@ -1945,8 +1947,7 @@ static int copy_document_out(ktj_engine* e, char* dst) {
   while (doc.room(0) && err == hipSuccess) err = doc.launch();
   HIPCHK(err);
   const unsigned n_threads = copy_threads(doc.n, KTJ_COPY_OUT_PER_THREAD, KTJ_COPY_OUT_THREADS);
-  std::atomic<uint64_t> arrived{0}, next{0};
-  std::atomic<bool> failed{false};
+  PartQueue queue(doc.n_parts);
   std::atomic<uint64_t> left[KTJ_PART_SLOTS]; /* 1 + the last part that was copied out of the slot */
   for (auto& x : left) x.store(0, std::memory_order_relaxed);
   auto copy_one = [&](uint64_t c) {
@@ -1954,28 +1955,22 @@ static int copy_document_out(ktj_engine* e, char* dst) {
     left[c % doc.slots].store(c + 1, std::memory_order_release);
   };
   run_workers(n_threads, [&](unsigned t) {
+    uint64_t k;
     if (t != 0) {
-      for (uint64_t c; (c = next.fetch_add(1, std::memory_order_relaxed)) < doc.n_parts;) {
-        for (unsigned spins = 1; arrived.load(std::memory_order_acquire) <= c; ++spins) {
-          if (failed.load(std::memory_order_relaxed)) return;
-          if (spins % 4096 == 0) std::this_thread::yield();
-        }
-        copy_one(c);
-      }
+      while (queue.take(&k)) copy_one(k);
       return;
     }
     uint64_t taken = 0; /* parts 0 .. taken - 1 have left their slots */
+    Patience patience;
     for (uint64_t c = 0; taken < doc.n_parts && err == hipSuccess;) {
-      while (taken < c && left[taken % doc.slots].load(std::memory_order_acquire) > taken) ++taken;
+      while (taken < c && left[taken % doc.slots].load(std::memory_order_acquire) > taken) { ++taken; patience = Patience(); }
       if (doc.room(taken)) err = doc.launch();
-      else if (c < doc.launched && doc.here(c)) arrived.store(++c, std::memory_order_release);
-      else {
-        uint64_t k = next.load(std::memory_order_relaxed); /* nothing new: help with what is here */
-        if (k < c && next.compare_exchange_strong(k, k + 1, std::memory_order_relaxed)) copy_one(k);
-        else if (c < doc.launched) err = doc.wait(c);
-      }
+      else if (c < doc.launched && doc.here(c)) { ++c; queue.arrive(); }
+      else if (queue.try_help(&k)) copy_one(k); /* nothing new: help with what is here */
+      else if (c < doc.launched) err = doc.wait(c);
+      else patience.pause(); /* the others are at the last parts, or at those that hold the slots */
     }
-    if (err != hipSuccess) failed.store(true);
+    if (err != hipSuccess) queue.give_up();
   });
   const hipError_t done = hipStreamSynchronize(e->stream);
   HIPCHK(err);
