@@ -101,3 +101,19 @@ def test_document_longer_than_the_first_buffer():
     with TraceEngine(sp.contents.trace_name.decode(), base_time_ns=sp.contents.base_time_ns) as eng:
         eng.submit_stream(sp)
         check(eng, want, counters)
+
+
+@pytest.mark.parametrize("rows", [300, 2047, 5000, 140000])
+def test_sessions_that_fall_back(rows):
+    """One engine per trace, as a profiler's session has it: the first pass over the records is the only one.  Stream
+    Sync activities and timestamps too far apart send it from three launches to one go and on to step by step; what
+    that leaves for the next engine must not show."""
+    near = [k * 3 % 5000 for k in range(rows)]
+    apart = [(k * 0x9E3779B97F4A7C15) % (1 << 61) for k in range(rows)]
+    cases = [(sp,) + oracle(sp) for sp in (ops(near), ops(near, 100), ops(apart), ops(apart, 1 << 60))]
+    for k in (0, 1, 0, 2, 1, 3, 0, 3):
+        sp, want, counters = cases[k]
+        with TraceEngine(sp.contents.trace_name.decode(), base_time_ns=sp.contents.base_time_ns, no_stage_times=k % 2 == 1) as eng:
+            eng.submit_stream(sp)
+            check(eng, want, counters, passes=1)
+            assert eng.stats().stage_ms[abi.STAGE_NAMES.index("total_gpu")] > 0
