@@ -1853,12 +1853,12 @@ static hipError_t sort_packed_t(Columns c, uint64_t n, SortSets s, Scalars* sc, 
  *   - while it puts its keys to their places it counts the next pass's digits per tile of the output, in LDS
  *     (16 bits each: a tile holds 1024 keys), and adds what it has to the next pass's counts.
  * Bound by the chain of its short phases, some 5 us whatever the tile holds: one key per thread is the
- * shortest of them (a first form that put a tile in order before it was written out: 186 us for 30 000 records
- * with tiles of 1024 keys, 203 with 2048, 212 with 4096).  Three launches a pass against this, whole pass:
- * 30 000 records 218 -> 185 us, 60 000 223 -> 207, 90 000 258 -> 251, 118 000 243 both; counts to add up and
- * cells to hand on grow with the tiles, and at 733 000 keys a pass took 30 us instead of 25. */
+ * shortest of them (a first form that put a tile in order before it was written out took 17 us more for 30 000
+ * records with tiles of 2048 keys, and 26 us more with 4096).  Three launches a pass against this, whole pass:
+ * 4500 records 203 -> 177 us, 30 000 219 -> 202, 60 000 224 -> 216, 90 000 228 both, 120 000 229 -> 234; counts to
+ * add up and cells to hand on grow with the tiles (at 733 000 keys a pass took 30 us instead of 25). */
 #define CHAIN_THREADS 1024
-#define CHAIN_MAX_N 131072ull
+#define CHAIN_MAX_N 98304ull
 template <int BITS, bool FROM_KEYS>
 __global__ void __launch_bounds__(CHAIN_THREADS)
 k_sortp_chain(const uint64_t* in, uint64_t* words_out, uint32_t* perm_out, uint32_t n, uint32_t pass, uint32_t idx_bits, const Scalars* sc,

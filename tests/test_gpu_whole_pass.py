@@ -79,7 +79,7 @@ def test_later_records_need_more(late, sync):
 
 
 # sorts with one launch a pass: a last tile of one key, the most keys and one more; a digit that all keys share
-@pytest.mark.parametrize("rows,bits", [(5121, 30), (5121, 55), (131072, 30), (131073, 30), (131072, 55), (20000, 1)])
+@pytest.mark.parametrize("rows,bits", [(5121, 30), (5121, 55), (98304, 30), (98305, 30), (98304, 55), (131072, 30), (131073, 30), (131072, 55), (20000, 1)])
 def test_sort_of_one_launch_a_pass(rows, bits):
     sp = ops([(k * 0x9E3779B97F4A7C15) % (1 << 64) >> (64 - bits) for k in range(rows)])
     want, counters = oracle(sp)
