@@ -230,8 +230,8 @@ def host_to_file_legs(sp, n_records):
 
 def small_trace_legs():
     """What a trace of a few records and configuration 1 at its full size (30 000 records) cost: the
-    fixed cost of the pass (some forty short kernels and two read-backs), not throughput.  Median over
-    repeated passes on a warm engine, with and without the events between the stages
+    fixed cost of the pass (three launches, or two dozen short ones, and a wait), not throughput.
+    Median over repeated passes on a warm engine, with and without the times of its stages
     (KTJ_CREATE_NO_STAGE_TIMES, which the ActivityLogger shim sets), and from ktj_create to
     ktj_destroy on engines that start from what the previous one left behind."""
     import statistics

@@ -468,9 +468,9 @@ typedef struct ktj_engine ktj_engine;
  * KTJ_CREATE_CUDA12_ARGS prints the "graph id", "graph node id", "channel" and "channel_type" keys
  * of memset rows (ktj_memset_rec), which the reference compiles in for CUDA >= 12 only
  * (CuptiActivity.h:424-458).
- * KTJ_CREATE_NO_STAGE_TIMES leaves the events between the stages of a pass out: ktj_stats then
- * reports the time of the whole pass only (stage_ms[KTJ_STAGE_TOTAL_GPU]), and a trace of a few
- * records is finished a tenth sooner.
+ * KTJ_CREATE_NO_STAGE_TIMES: ktj_stats reports the time of the whole pass only
+ * (stage_ms[KTJ_STAGE_TOTAL_GPU]).  The stages' times are readings of the device's clock that the
+ * kernels leave on their way; a pass takes the same time with and without them.
  *
  * ktj_destroy leaves what every engine needs before its first record behind for the next ktj_create on
  * the same device, which starts from it instead of allocating (a trace of a few records otherwise spends

@@ -1,6 +1,6 @@
 /*
  * emit.hip — stage 4b: the activities formatted into the document, for traces of any size beyond the small
- * ones (small.hip).  A file of its own because it takes as long to compile as everything else together.
+ * ones (small.hip).  A file of its own because it takes twice as long to compile as everything else together.
  */
 #include "gpu_common.h"
 

@@ -154,8 +154,8 @@ struct Scalars {
   /* The counters that most workgroups add to (KTJ_CNT_*) are kept in KTJ_COUNTER_SHARDS copies, one
    * 128-byte line each; a workgroup adds to the copy of its index.  Atomics on one address are carried
    * out one after the other, and tens of thousands of workgroups adding to the same few words cost the
-   * join more than its table lookups.  k_publish sums the copies into the fields above, which nothing
-   * on the device reads; it hands the host everything in front of this array. */
+   * join more than its table lookups.  publish_scalars sums the copies into the fields above, of which the
+   * device reads emit_rows only, and hands the host everything in front of this array. */
   alignas(128) unsigned long long shard[KTJ_COUNTER_SHARDS][16];
   alignas(128) unsigned long long range_shard[KTJ_COUNTER_SHARDS][16]; /* likewise the key ranges of the join tables: [2t] smallest,
                                                                            [2t + 1] largest key of table t */

@@ -2582,7 +2582,7 @@ __global__ void k_publish(Scalars* sc, const uint64_t* total, const uint32_t* li
 }
 hipError_t publish(Scalars* sc, const uint64_t* total, const uint32_t* list, uint32_t n_list, Scalars* h_sc,
                    uint64_t* h_total, uint32_t* h_list, hipStream_t st) {
-  static_assert(KTJ_CNT_COUNT == 7, "k_publish names every sharded counter");
+  static_assert(KTJ_CNT_COUNT == 7, "publish_scalars names every sharded counter");
   hipLaunchKernelGGL(k_publish, dim3(n_list > 4096 ? 16 : 1), dim3(KTJ_BLOCK), 0, st, sc, total, list, n_list, h_sc, h_total, h_list);
   return KTJ_LAUNCH_CHECK();
 }
