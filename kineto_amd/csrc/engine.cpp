@@ -1962,13 +1962,14 @@ static int copy_document_out(ktj_engine* e, char* dst) {
     }
     uint64_t taken = 0; /* parts 0 .. taken - 1 have left their slots */
     Patience patience;
-    for (uint64_t c = 0; taken < doc.n_parts && err == hipSuccess;) {
+    for (uint64_t c = 0; err == hipSuccess;) {
       while (taken < c && left[taken % doc.slots].load(std::memory_order_acquire) > taken) { ++taken; patience = Patience(); }
       if (doc.room(taken)) err = doc.launch();
       else if (c < doc.launched && doc.here(c)) { ++c; queue.arrive(); }
       else if (queue.try_help(&k)) copy_one(k); /* nothing new: help with what is here */
       else if (c < doc.launched) err = doc.wait(c);
-      else patience.pause(); /* the others are at the last parts, or at those that hold the slots */
+      else if (c == doc.n_parts) break; /* all have been there: the others are at the last of them, and are waited for below */
+      else patience.pause(); /* the others are at the parts that hold the slots */
     }
     if (err != hipSuccess) queue.give_up();
   });

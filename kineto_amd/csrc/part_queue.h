@@ -14,8 +14,9 @@
 
 namespace ktj {
 
-/* A wait for something that is mostly there within microseconds: looked for without a break for about as long as
- * a few parts take to cross, then between naps, so that a wait that takes longer does not keep a core. */
+/* A wait for something that is mostly there within microseconds: looked for without a break for much longer than a
+ * part takes to cross (9 us) and the first one to arrive, then between naps, so that a wait that takes longer does
+ * not keep a core.  (A nap of 20 us takes 70 or more.) */
 class Patience {
  public:
   /* true: the wait has come to its naps */
@@ -36,15 +37,16 @@ class Patience {
   }
 
  private:
-  static constexpr unsigned kLooks = 2000; /* some 30 us; a part of 512 KiB crosses in 9 us */
+  static constexpr unsigned kLooks = 12000; /* some 200 us */
   unsigned looks_ = 0;
 };
 
 /* A thread takes a part only once that is there: what has nothing to do sleeps, and as many threads are awake as
  * the parts keep busy.  With every part dealt out beforehand and each thread awake for its own, 1.03 GB into memory
  * that was there before (21.1 ms) took 125 ms of processor time, 59 MB (1.25 ms) 7.0 ms; now 86 ms and 4.5 ms in the
- * same time.  Sleeping after 400, 1000 or 2000 looks makes no difference to the sessions (30 000 records 641, 647 and
- * 646 us, 634 with all awake), and 400 the most to the processor time. */
+ * same time.  Sleeping after 400, 1500 or 6000 looks makes no difference to the sessions (medians of eight runs in
+ * turn: 30 000 records 656, 663 and 662 us, 650 with all awake; 118 000 kernels 2783, 2772 and 2834, 2826 with all
+ * awake), and 400 the most to the processor time. */
 class PartQueue {
  public:
   explicit PartQueue(uint64_t n_parts) : n_(n_parts) {}
