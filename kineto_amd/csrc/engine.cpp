@@ -1812,13 +1812,25 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
   return KTJ_OK;
 }
 
+/* A pass that ends early leaves nothing behind on the device: neither launches that still read the caller's records
+ * or use the scratch array, which are theirs and another engine's again when the call returns, nor small tables on
+ * their way into that array. */
+static int run_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, uint64_t out_cap) {
+  const int rc = process_pass(e, end_time_ns, out_device, out_cap);
+  if (rc != KTJ_OK) {
+    (void)put_pending_pieces(e);
+    (void)hipStreamSynchronize(e->stream);
+  }
+  return rc;
+}
+
 int ktj_process(ktj_engine* e, int64_t end_time_ns) {
   if (!e) return KTJ_ERR_ARG;
   if (e->bad_sink) return KTJ_OK;
   const int flushed = flush_sdk_api_rows(e);
   if (flushed != KTJ_OK) return flushed;
   e->noalloc = false;
-  return process_pass(e, end_time_ns, nullptr, 0);
+  return run_pass(e, end_time_ns, nullptr, 0);
 }
 
 /* The pass with no allocation in it: working memory is this GPU's copy of the static scratch
@@ -1838,7 +1850,7 @@ int ktj_process_noalloc(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
     return KTJ_ERR_LIMIT;
   }
   e->noalloc = true;
-  const int rc = process_pass(e, end_time_ns, out_device, out_capacity);
+  const int rc = run_pass(e, end_time_ns, out_device, out_capacity);
   e->noalloc = false;
   /* The small tables of this pass sit in the scratch array, which every engine on this GPU shares:
    * whatever the pass returned, the next allocating pass must upload them into its own buffers again. */
