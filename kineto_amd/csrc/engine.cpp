@@ -230,7 +230,8 @@ struct ktj_engine {
   DevBuf q_keys, q_stream, q_amb, dn_hash, dn_first, dn_dev, dn_key, dn_rank, dn_list;
   DevBuf s_dev_k, s_dev_r, s_dev_l, s_res_k, s_res_r, s_res_l;
   DevBuf keys_a, keys_b, vals_a, vals_b, hist, scan_tmp;
-  DevBuf mat, len, len_sorted, kind_sorted, offs, out, tile_start;
+  bool rows_are_text = false;              /* of the last pass: TextRows in mat */
+  DevBuf mat, schema_book, len, len_sorted, kind_sorted, offs, out, tile_start;
   void* pinned_small = nullptr; size_t pinned_small_cap = 0;
   HostCtl* h_ctl = nullptr;                  /* pinned: what the device hands back during a pass */
   HostCtl* h_ctl_dev = nullptr;              /* the same memory as the kernels address it */
@@ -266,6 +267,8 @@ struct ktj_engine {
   void other_records() { small_unfit = stepwise = false; sort_passes = std::max(sort_passes, 6u); }
   bool small_last = false;   /* the last pass was a small one: it leaves no intermediate arrays for ktj_debug_fetch */
   bool no_small = false;     /* ktj_debug_fetch makes them */
+  bool no_weave = false;     /* joined rows as they are: ktj_debug_fetch, and where text rows do not fit */
+  hipError_t hip_error = hipSuccess; /* of the last call that failed */
   int64_t last_end_time = 0;
   int wall_clock_khz = 0;
 
@@ -281,6 +284,7 @@ namespace {
 
 int fail_hip(ktj_engine* e, hipError_t err, const char* what) {
   e->hip_failed = true;
+  e->hip_error = err;
   e->last_error = std::string(what) + ": " + hipGetErrorString(err);
   return KTJ_ERR_HIP;
 }
@@ -1454,6 +1458,7 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
   { const int rc = put_pending_pieces(e); if (rc != KTJ_OK) return rc; }
   e->last_end_time = end_time_ns;
   e->small_last = false;
+  e->rows_are_text = false;
   if (!e->small_unfit && !e->no_small && nu == 0 && n_coll == 0 && small_fits(ng, nr, nd, nx) && !sort_packed_passes_forced() &&
       !(e->flags & (KTJ_CREATE_TILE_EMIT | KTJ_CREATE_HASH_JOIN | KTJ_CREATE_PAIR_SORT))) {
     bool done = false;
@@ -1469,6 +1474,10 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
   /* capacities for the hash mode (load <= 2/3); the direct mode uses a prefix of the same buffers */
   const uint32_t cap_full = pow2_at_least((nr + nd) + (nr + nd) / 2);
   const uint32_t cap_narrow = pow2_at_least((nx + nr) + (nx + nr) / 2), cap_cpu = pow2_at_least(2 * ng);
+  /* Joined rows as text for the weaver, but where something reads them as they are, and where their 32 bytes more
+   * would not fit the scratch array with as many records. */
+  const bool woven = n_coll == 0 && !e->noalloc && !e->no_weave && !(e->flags & KTJ_CREATE_TILE_EMIT);
+  e->rows_are_text = woven;
   e->pool_used = 0;
   size_t pass_bytes = 0;
   for (int phase = e->noalloc ? 1 : 0; phase < 2; ++phase) { /* 0: add the sizes up and size the pool; 1: hand the buffers out */
@@ -1505,7 +1514,9 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
     if (m2 > m) m = m2;
     NEED(e->scan_tmp, m * 8);
   }
-  NEED(e->mat, Na * sizeof(MatRow)); NEED(e->len, Na * 4); NEED(e->len_sorted, Na * 4); NEED(e->kind_sorted, Na + 16);
+  NEED(e->mat, Na * (woven ? sizeof(weave::TextRow) : sizeof(MatRow)));
+  if (woven) NEED(e->schema_book, sizeof(weave::SchemaBook));
+  NEED(e->len, Na * 4); NEED(e->len_sorted, Na * 4); NEED(e->kind_sorted, Na + 16);
   NEED(e->offs, (Na + 1) * 8);
   if (e->measuring) {
     e->measuring = false;
@@ -1568,11 +1579,15 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
   NarrowCols nc{e->n_ext_src.as<uint32_t>(), e->n_kern_src.as<uint32_t>(), e->n_copy_src.as<uint32_t>(), e->n_pay.as<NarrowPay>()};
   HIPCHK(plan_tables(tf, fc, tn, nc, t_cpu, (e->flags & KTJ_CREATE_HASH_JOIN) != 0, sc, st));
   ApiTable api{e->d_cid_names.as<uint32_t>(), (uint32_t)e->cid_names.size(), e->d_flow_bits.as<uint32_t>(), e->malloc_cid};
-  MatRow* mat = e->mat.as<MatRow>();
+  weave::SchemaBook* book = woven ? e->schema_book.as<weave::SchemaBook>() : nullptr;
+  const Rows rows{e->mat.p, book};
+  const MatRow* mat = e->mat.as<MatRow>();
+  /* places of the rows that are not text: in the sort's buffer that does not hold its result */
+  auto left = [&]() -> uint32_t* { return !woven ? nullptr : e->sorted_keys == e->keys_b.p ? e->keys_a.as<uint32_t>() : e->keys_b.as<uint32_t>(); };
   /* only external-correlation records and user spans ask for the CPU ops' ids (5 M records without any: 58 us) */
   if (nx || max_spans) HIPCHK(build_cpu_ids(g_recs, ng, t_cpu, cpu_row, sc, st));
   HIPCHK(build_extcorr(x_recs, nx, tn, nc, t_cpu, cpu_row, g_recs, ctx, sc, st));
-  HIPCHK(join_runtime_rows(r_recs, nr, c, ng, api, tf, fc, tn, nc, e->slot_f.as<uint32_t>(), e->slot_n.as<uint32_t>(), ctx, mat,
+  HIPCHK(join_runtime_rows(r_recs, nr, c, ng, api, tf, fc, tn, nc, e->slot_f.as<uint32_t>(), e->slot_n.as<uint32_t>(), ctx, rows,
                            e->len.as<uint32_t>(), sc, st));
   HIPCHK(republish_runtime_rows(r_recs, nr, c, ng, fc, nc, e->slot_f.as<uint32_t>(), e->slot_n.as<uint32_t>(), sc, st));
   unsigned long long* orphans = e->keys_a.as<unsigned long long>(); /* a bit per device row: the sort's words come later */
@@ -1604,7 +1619,13 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
   }
   /* (settled here: collect_distinct flags what only a host that does not look would get wrong) */
   const bool straight = has_room && n_coll == 0 && max_spans == 0 && !e->stepwise && !(e->flags & KTJ_CREATE_TILE_EMIT) && e->sort_mode != 1;
-  HIPCHK(collect_distinct(c, N, sets, sc, straight, st));
+  HIPCHK(collect_distinct(c, N, sets, sc, straight, ctx, book, st));
+  auto put_activities = [&](uint64_t n_most, uint64_t at) -> int { /* the documents' activities, but for the tile variant */
+    if (woven)
+      HIPCHK(weave_activities(e->mat.as<weave::TextRow>(), e->perm, e->offs.as<uint64_t>(), e->kind_sorted.as<uint8_t>(), n_most, ctx, e->out.as<char>(), at, sc, book, st));
+    HIPCHK(emit_direct(rows.p, e->perm, e->offs.as<uint64_t>(), e->kind_sorted.as<uint8_t>(), n_most, ctx, e->out.as<char>(), at, sc, left(), st));
+    return KTJ_OK;
+  };
   bool emitted = false;
   if (straight) {
     const std::string prefix = e->txt_header + e->txt_before;
@@ -1616,12 +1637,12 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
     e->perm = e->vals_a.as<uint32_t>();
     e->sorted_keys = nullptr;
     HIPCHK(sort_packed(c, N, sets, sc, e->sort_passes, e->keys_a.as<uint64_t>(), e->keys_b.as<uint64_t>(), e->perm, e->hist.as<uint32_t>(), e->offs.as<uint32_t>(), st));
-    HIPCHK(mat_rows(g_recs, ng, 0, nullptr, d_recs, nd, c, ng + nr, e->dev_link.as<DevLink>(), ctx, mat, e->len.as<uint32_t>(), sc, st));
+    HIPCHK(mat_rows(g_recs, ng, 0, nullptr, d_recs, nd, c, ng + nr, e->dev_link.as<DevLink>(), ctx, rows, e->len.as<uint32_t>(), sc, st));
     for (;;) {
       text.out = e->out.as<char>(); text.out_cap = e->out.cap;
       HIPCHK(gather_offsets(e->perm, e->len.as<uint32_t>(), N, e->len_sorted.as<uint32_t>(), e->kind_sorted.as<uint8_t>(),
-                            e->scan_tmp.as<uint64_t>(), e->offs.as<uint64_t>(), sc, text, st));
-      HIPCHK(emit_direct(mat, e->perm, e->offs.as<uint64_t>(), e->kind_sorted.as<uint8_t>(), N, ctx, e->out.as<char>(), prefix.size(), sc, st));
+                            e->scan_tmp.as<uint64_t>(), e->offs.as<uint64_t>(), left(), sc, text, st));
+      { const int rc = put_activities(N, prefix.size()); if (rc != KTJ_OK) return rc; }
       HIPCHK(hipEventRecord(e->ev[EV_EMIT], st));
       HIPCHK(hipStreamSynchronize(st));
       e->scalars = e->h_ctl->scalars;
@@ -1633,6 +1654,7 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
       if (emitted) break;
       if (out_device) return short_output(e); /* nothing has been written */
       HIPCHK(e->out.ensure(e->total_bytes + 64));
+      HIPCHK(fill_u32(&sc->n_left, 0, 1, st)); /* the list is made anew */
     }
     if (emitted) e->sort_passes = sort_packed_passes(e->scalars.sort.key_bits);
     else if (e->scalars.error & ~(KTJ_DEVERR_CAREFUL | KTJ_DEVERR_DISTINCT_DEVICES | KTJ_DEVERR_DISTINCT_RESOURCES)) {
@@ -1709,14 +1731,15 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
                              e->sync_pos.as<uint32_t>(), e->sync_first.as<uint32_t>(), sc, st));
     sync_first = e->sync_first.as<uint32_t>();
   }
-  HIPCHK(mat_rows(g_recs, ng, 0, sync_first, d_recs, nd, c, ng + nr, e->dev_link.as<DevLink>(), ctx, mat, e->len.as<uint32_t>(), sc, st));
-  HIPCHK(mat_rows(e->synth_recs.as<ktj_generic_rec>(), e->n_spans, ng + nr + nd, nullptr, nullptr, 0, c, 0, nullptr, ctx, mat,
+  HIPCHK(mat_rows(g_recs, ng, 0, sync_first, d_recs, nd, c, ng + nr, e->dev_link.as<DevLink>(), ctx, rows, e->len.as<uint32_t>(), sc, st));
+  HIPCHK(mat_rows(e->synth_recs.as<ktj_generic_rec>(), e->n_spans, ng + nr + nd, nullptr, nullptr, 0, c, 0, nullptr, ctx, rows,
                   e->len.as<uint32_t>(), sc, st));
   if (n_coll) HIPCHK(collective_first(mat, e->perm, e->scalars.n_valid, n_coll, e->d_coll_first.as<uint32_t>(), st));
 
   /* ---- scan ---- */
+  if (straight) HIPCHK(fill_u32(&sc->n_left, 0, 1, st));
   HIPCHK(gather_offsets(e->perm, e->len.as<uint32_t>(), N, e->len_sorted.as<uint32_t>(), e->kind_sorted.as<uint8_t>(),
-                        e->scan_tmp.as<uint64_t>(), e->offs.as<uint64_t>(), sc, DocText{}, st));
+                        e->scan_tmp.as<uint64_t>(), e->offs.as<uint64_t>(), left(), sc, DocText{}, st));
   uint64_t act_bytes = 0;
   e->coll_first.assign(2ull * n_coll, 0xFFFFFFFFu);
   const bool list_fits = 2ull * n_coll * 4 <= e->pinned_small_cap; /* through the engine's pinned buffer when it fits */
@@ -1776,8 +1799,7 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
       HIPCHK(emit(mat, e->perm, e->offs.as<uint64_t>(), N, ctx, e->out.as<char>(), e->prefix_len, act_bytes, tile,
                   e->tile_start.as<uint32_t>(), st));
     else
-      HIPCHK(emit_direct(mat, e->perm, e->offs.as<uint64_t>(), e->kind_sorted.as<uint8_t>(), e->scalars.n_valid, ctx, e->out.as<char>(),
-                         e->prefix_len, sc, st));
+    { const int rc = put_activities(e->scalars.n_valid, e->prefix_len); if (rc != KTJ_OK) return rc; }
   }
   HIPCHK(hipEventRecord(e->ev[EV_EMIT], st));
   HIPCHK(hipStreamSynchronize(st));
@@ -1816,10 +1838,25 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
  * or use the scratch array, which are theirs and another engine's again when the call returns, nor small tables on
  * their way into that array. */
 static int run_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, uint64_t out_cap) {
-  const int rc = process_pass(e, end_time_ns, out_device, out_cap);
-  if (rc != KTJ_OK) {
-    (void)put_pending_pieces(e);
-    (void)hipStreamSynchronize(e->stream);
+  const bool failed_before = e->hip_failed;
+  auto pass = [&]() {
+    e->hip_error = hipSuccess;
+    const int rc = process_pass(e, end_time_ns, out_device, out_cap);
+    if (rc != KTJ_OK) {
+      (void)put_pending_pieces(e);
+      (void)hipStreamSynchronize(e->stream);
+    }
+    return rc;
+  };
+  int rc = pass();
+  if (rc != KTJ_OK && e->hip_error == hipErrorOutOfMemory && e->rows_are_text) { /* as many records as without text rows */
+    const bool before = e->no_weave;
+    (void)hipGetLastError();
+    e->pool.release();
+    e->hip_failed = failed_before;
+    e->no_weave = true;
+    rc = pass();
+    e->no_weave = before;
   }
   return rc;
 }
@@ -2104,10 +2141,12 @@ int ktj_debug_copy_reference(ktj_engine* e, uint64_t n_bytes, float* ms) {
 int ktj_debug_fetch(ktj_engine* e, int what, void* dst, uint64_t cap, uint64_t* n_bytes) {
   if (!e || !n_bytes) return KTJ_ERR_ARG;
   if (!e->processed) return KTJ_ERR_STATE;
-  if (e->small_last) { /* a small pass keeps none of these: the launches of a large trace make them (and the same document) */
+  const bool as_text = what == KTJ_DBG_MAT && e->rows_are_text;
+  if (e->small_last || as_text) { /* a small pass keeps none of these: the launches of a large trace make them (and the same document) */
     e->no_small = true;
+    e->no_weave = what == KTJ_DBG_MAT;
     const int rc = ktj_process(e, e->last_end_time);
-    e->no_small = false;
+    e->no_small = e->no_weave = false;
     if (rc != KTJ_OK) return rc;
   }
   const void* src = nullptr;

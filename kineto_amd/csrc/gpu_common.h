@@ -111,6 +111,10 @@ __device__ __forceinline__ void dict_string(const char* blob, const uint64_t* of
   if (lane_id() == 0) entries[id] = d;
   char* an = arg_blob + d.arg_off;
   char* nn = name_blob + d.name_off;
+  /* zeros up to the next 16-byte boundary: a view is read in whole blocks */
+  auto pad = [&](char* view, uint32_t n) { if (lane_id() < 16u && lane_id() >= (n & 15u) && (n & 15u)) view[(n & ~15u) + lane_id()] = 0; };
+  pad(an, d.arg_len);
+  pad(nn, d.name_len);
   const bool literal_name = (d.flags & (KTJ_SF_NAME_KERNEL | KTJ_SF_NAME_UNKNOWN)) != 0;
   if (literal_name) {
     const char* lit = is_kernel ? "Kernel" : "unknown";
@@ -217,6 +221,14 @@ __device__ __forceinline__ uint32_t row_length(const MatRow& m, const EmitCtx& c
   format_activity(cw, m, ctx);
   if (cw.n >= (1ull << 30)) { flag_error(sc, KTJ_DEVERR_RECORD_TOO_LONG); return 0; }
   return (uint32_t)cw.n | (tail_kind(m, has_args(m, ctx)) << 30);
+}
+
+/* the tail kind of the activity at a place of the emission order */
+__device__ __forceinline__ uint32_t tail_kind_at(const uint8_t* kind_sorted, const weave::TextRow* rows, const uint32_t* perm, uint64_t i, const EmitCtx& ctx) {
+  const uint32_t k = kind_sorted[i];
+  if (k != KTJ_KIND_LEFT) return k;
+  const MatRow m = *reinterpret_cast<const MatRow*>(&rows[perm[i]]);
+  return tail_kind(m, has_args(m, ctx));
 }
 
 /* ---- bytes to any address of the document ---- */

@@ -9,6 +9,7 @@
 #include <hip/hip_runtime_api.h>
 
 #include "mat_core.h"
+#include "weave_core.h"
 
 namespace ktj {
 namespace gpu {
@@ -143,6 +144,7 @@ struct Scalars {
   unsigned int n_queues;              /* distinct hardware queues entered into the queue -> stream table */
   unsigned int n_sync_rows;           /* distinct (device, row) pairs of Stream Sync activities */
   unsigned int n_plain;               /* small traces: activities that small_emit leaves to small_plain */
+  unsigned int n_left;                /* activities that weave leaves to emit_direct */
   unsigned int ext_ids_repeat;        /* two external-correlation records share a correlation id */
   unsigned long long emit_rows;       /* activities to format: n_valid, or none where the pass cannot end so */
   unsigned long long clock[KTJ_CLOCK_COUNT];
@@ -317,8 +319,9 @@ struct SortSets {
   uint32_t* res_list;
 };
 /* distinct values and their ranks, and Scalars::sort; straight: the host will not look at anything before
- * the end of the pass, so what needs that is flagged (KTJ_DEVERR_CAREFUL) */
-hipError_t collect_distinct(Columns c, uint64_t n, SortSets s, Scalars* sc, bool straight, hipStream_t st);
+ * the end of the pass, so what needs that is flagged (KTJ_DEVERR_CAREFUL).  book, if not null: what text_row and
+ * weave_activities need to know of the schemas, from the dictionary views */
+hipError_t collect_distinct(Columns c, uint64_t n, SortSets s, Scalars* sc, bool straight, const EmitCtx& ctx, weave::SchemaBook* book, hipStream_t st);
 /* key = ((rank(dev) << res_bits | rank(res)) << ts_bits) | (ts - ts_min); dropped rows get 1 << key_bits */
 hipError_t make_keys(Columns c, uint64_t n, SortSets s, const Scalars* sc, uint32_t ts_bits, uint32_t res_bits,
                      uint32_t key_bits, uint64_t* keys, uint32_t* vals, hipStream_t st);
@@ -350,6 +353,13 @@ hipError_t radix_sort(uint64_t* keys_a, uint32_t* vals_a, uint64_t* keys_b, uint
                       uint64_t** res_keys, uint32_t** res_vals, hipStream_t st);
 
 /* ---- stage 4a: joined rows + exact byte length (arrival order) ---- */
+/* With schemas set the rows are TextRows (those that the weaver does not print MatRows in the same places, marked:
+ * KTJ_ROW_LEFT, and tail kind KTJ_KIND_LEFT beside their lengths); otherwise all are MatRows. */
+struct Rows {
+  void* p;
+  const weave::SchemaBook* schemas;
+};
+#define KTJ_KIND_LEFT 3u
 /* keys: KTJ_SYNC_CAP + 1, first_pos: KTJ_SYNC_CAP + 1, is_first: n_generic (all caller-provided);
  * dev: the deviceId column */
 hipError_t stream_sync_first(const uint32_t* perm, uint64_t n_sorted, const ktj_generic_rec* g, uint64_t n_generic,
@@ -358,12 +368,12 @@ hipError_t stream_sync_first(const uint32_t* perm, uint64_t n_sorted, const ktj_
 /* joined rows and lengths of generic records (arrival index first_generic on; sync_first: per record, from
  * stream_sync_first, or null when there are no such rows) and of device records */
 hipError_t mat_rows(const ktj_generic_rec* g, uint64_t ng, uint64_t first_generic, const uint32_t* sync_first, const ktj_device_rec* d, uint64_t nd,
-                    Columns c, uint64_t first_device, const DevLink* link, EmitCtx ctx, MatRow* mat, uint32_t* len, Scalars* sc, hipStream_t st);
+                    Columns c, uint64_t first_device, const DevLink* link, EmitCtx ctx, Rows rows, uint32_t* len, Scalars* sc, hipStream_t st);
 /* the pass over the runtime rows: publishes what device rows take over (first timestamp, stream, grid,
  * size) into the tables, reads the "External id", makes the joined rows and their lengths; runs
  * after build_extcorr and before link_device_rows */
 hipError_t join_runtime_rows(const ktj_runtime_rec* r, uint64_t n, Columns c, uint64_t first, ApiTable api, Table tf, FullCols fc,
-                             Table tn, NarrowCols nc, uint32_t* slot_f, uint32_t* slot_n, EmitCtx ctx, MatRow* mat,
+                             Table tn, NarrowCols nc, uint32_t* slot_f, uint32_t* slot_n, EmitCtx ctx, Rows rows,
                              uint32_t* len, Scalars* sc, hipStream_t st);
 /* winners write the payload again and repeated ids are checked; returns at once where no two
  * runtime rows share a slot */
@@ -380,8 +390,9 @@ struct DocText {
   uint64_t* h_end;                         /* small traces: the wall clock when the last activities were written */
 };
 uint64_t offsets_tmp_elems(uint64_t n);
+/* left: where the places of the rows that are left to emit_direct go (Scalars::n_left of them, at most n) */
 hipError_t gather_offsets(const uint32_t* perm, const uint32_t* len, uint64_t n, uint32_t* len_sorted, uint8_t* kind_sorted, uint64_t* sums,
-                          uint64_t* offs, Scalars* sc, const DocText& text, hipStream_t st);
+                          uint64_t* offs, uint32_t* left, Scalars* sc, const DocText& text, hipStream_t st);
 
 /* ---- stage 4b: emit ---- */
 /* tile size (bytes of output per workgroup) for a document whose activity section has act_bytes
@@ -393,9 +404,14 @@ hipError_t emit(const MatRow* mat, const uint32_t* perm, const uint64_t* offs /*
                 uint32_t* tile_start /* tiles + 1 */, hipStream_t st);
 
 /* direct variant: one lane per activity; kind_sorted holds the tail kind of every activity in emission order;
- * Scalars::emit_rows of them, at most n_most */
-hipError_t emit_direct(const MatRow* mat, const uint32_t* perm, const uint64_t* offs, const uint8_t* kind_sorted, uint64_t n_most, EmitCtx ctx,
-                       char* out, uint64_t prefix_len, const Scalars* sc, hipStream_t st);
+ * Scalars::emit_rows of them, at most n_most.  left: only the Scalars::n_left activities on this list, rows are sizeof(TextRow) apart */
+hipError_t emit_direct(const void* rows, const uint32_t* perm, const uint64_t* offs, const uint8_t* kind_sorted, uint64_t n_most, EmitCtx ctx,
+                       char* out, uint64_t prefix_len, const Scalars* sc, const uint32_t* left, hipStream_t st);
+
+/* The activities of rows that are text (TextRow), one lane per segment (weave.hip).  The others, if any, are on the list
+ * that gather_offsets made: emit_direct's. */
+hipError_t weave_activities(const weave::TextRow* rows, const uint32_t* perm, const uint64_t* offs, const uint8_t* kind_sorted, uint64_t n_most, EmitCtx ctx, char* out,
+                 uint64_t prefix_len, const Scalars* sc, const weave::SchemaBook* schemas, hipStream_t st);
 
 /* ---- small traces: the whole pass in three launches (small.hip) ---- */
 #define SMALL_ROWS 2048u       /* records of the three classes together: what LDS holds the join tables for */

@@ -196,7 +196,7 @@ k_begin(Scalars* s, FillJobs jobs, const char* blob, const uint64_t* off, uint32
       s->ts_min_biased = ~0ULL; s->ts_max_biased = 0;
       s->out_of_range = 0; s->out_of_order = 0; s->n_flow = 0; s->n_linked = 0; s->n_blank_names = 0; s->n_valid = 0;
       s->n_unresolved = 0; s->n_sync_typed = 0; s->n_device_orphans = 0; s->error = 0; s->have_stream_src = 0; s->n_dev_ranks = 0; s->n_res_ranks = 0; s->n_dense = 0; s->runtime_ids_repeat = 0;
-      s->n_queues = 0; s->n_sync_rows = 0; s->ext_ids_repeat = 0; s->n_plain = 0;
+      s->n_queues = 0; s->n_sync_rows = 0; s->ext_ids_repeat = 0; s->n_plain = 0; s->n_left = 0;
       s->sort.ts_bits = s->sort.res_bits = s->sort.key_bits = 0;
       for (int k = 0; k < KTJ_DONE_COUNT; ++k) s->done[k] = 0;
       for (uint32_t k = 0; k < KTJ_PART_SLOTS; ++k) s->part_done[k] = 0;
@@ -1093,20 +1093,88 @@ __device__ void rank_values(const uint64_t* keys, const uint32_t* list, uint32_t
     if (p < m) rank[s] = r;
   }
 }
+/* The schemas' texts for the weaver, by one workgroup: a lane measures each schema, a lane lays it out, a lane writes the
+ * characters of each field.  (One lane for all of it, in a launch of its own: 13 us for four schemas, 20 for five.) */
+struct SchemaLds {
+  uint4 key[KTJ_WEAVE_FIELDS * (KTJ_WEAVE_KEY / 16u)];
+  uint32_t text[weave::SCHEMA_TEXT * 4], desc[weave::SCHEMA_DESC];
+  ktj_field field[KTJ_WEAVE_FIELDS];
+  uint32_t key_len[KTJ_WEAVE_FIELDS], place[KTJ_WEAVE_FIELDS];
+  uint32_t n_fields[weave::MAX_SCHEMAS], first[weave::MAX_SCHEMAS];
+  weave::SchemaPlan plan[weave::MAX_SCHEMAS];
+};
+__device__ void lay_out_schemas(const EmitCtx& c, weave::SchemaBook* out, SchemaLds* l) {
+  const uint32_t n = c.n_schemas < weave::MAX_SCHEMAS ? c.n_schemas : weave::MAX_SCHEMAS, k = threadIdx.x;
+  static_assert(KTJ_BLOCK >= KTJ_WEAVE_FIELDS && weave::MAX_SCHEMAS <= 64u, "a lane per field, a lane of one wavefront per schema");
+  for (uint32_t j = k; j < weave::SCHEMA_TEXT * 4u; j += KTJ_BLOCK) l->text[j] = 0;
+  if (k < weave::SCHEMA_DESC) l->desc[k] = 0;
+  if (k < KTJ_WEAVE_FIELDS) l->place[k] = ~0u;
+  ktj_schema_desc schema{};
+  if (k < n) schema = c.schemas[k];
+  if (k < 64u) {
+    uint32_t upto = schema.n_fields < KTJ_WEAVE_FIELDS ? schema.n_fields : KTJ_WEAVE_FIELDS;
+    const uint32_t mine = upto;
+    for (int o = 1; o < (int)weave::MAX_SCHEMAS; o <<= 1) { const uint32_t x = __shfl_up(upto, o); if ((int)k >= o) upto += x; }
+    if (k < weave::MAX_SCHEMAS) { l->first[k] = upto - mine; l->n_fields[k] = schema.n_fields; }
+  }
+  __syncthreads();
+  if (k < KTJ_WEAVE_FIELDS && n != 0) {
+    uint32_t of = 0;
+    while (of + 1u < n && l->first[of + 1u] <= k) ++of;
+    if (k - l->first[of] < l->n_fields[of]) {
+      const ktj_field fd = c.fields[c.schemas[of].first_field + (k - l->first[of])];
+      uint32_t len = 0;
+      if (fd.key_id != KTJ_NONE && fd.key_id < c.dict.n) {
+        const DictEntry e = c.dict.entries[fd.key_id];
+        const uint4* src = reinterpret_cast<const uint4*>(c.dict.arg_blob + e.arg_off);
+        len = e.arg_len;
+        if (len <= KTJ_WEAVE_KEY) for (uint32_t j = 0; j * 16u < len; ++j) l->key[k * (KTJ_WEAVE_KEY / 16u) + j] = src[j];
+      }
+      l->field[k] = fd;
+      l->key_len[k] = len;
+    }
+  }
+  __syncthreads();
+  if (k < 64u) {
+    const uint32_t first = k < n ? l->first[k] : 0u;
+    weave::SchemaPlan* const plan = &l->plan[k < weave::MAX_SCHEMAS ? k : 0u];
+    weave::SchemaSize size{0, 0};
+    bool taken = k < n && first + l->n_fields[k] <= KTJ_WEAVE_FIELDS;
+    if (taken) { size = weave::lay_out_schema(l->field + first, l->key_len + first, l->n_fields[k], 0, 0, plan, nullptr, nullptr); taken = plan->what != 0; }
+    uint32_t upto = size.desc | (size.units << 16);
+    for (int o = 1; o < (int)weave::MAX_SCHEMAS; o <<= 1) { const uint32_t x = __shfl_up(upto, o); if ((int)k >= o) upto += x; }
+    if ((upto & 0xFFFFu) > weave::SCHEMA_DESC || (upto >> 16) > weave::SCHEMA_TEXT) taken = false; /* its rows are format_activity's */
+    if (taken) weave::lay_out_schema(l->field + first, l->key_len + first, l->n_fields[k], (upto & 0xFFFFu) - size.desc, (upto >> 16) - size.units, plan, l->desc, l->place + first);
+    else if (k < weave::MAX_SCHEMAS) plan->what = 0;
+    if (k < weave::MAX_SCHEMAS) out->plan[k] = *plan;
+  }
+  __syncthreads();
+  if (k < KTJ_WEAVE_FIELDS && l->place[k] != ~0u)
+    weave::put_field_text(l->field[k], reinterpret_cast<const char*>(l->key + k * (KTJ_WEAVE_KEY / 16u)), l->key_len[k], l->place[k], reinterpret_cast<char*>(l->text));
+  __syncthreads();
+  for (uint32_t j = k; j < weave::SCHEMA_TEXT * 4u; j += KTJ_BLOCK) out->text[j] = l->text[j];
+  if (k < weave::SCHEMA_DESC) out->desc[k] = l->desc[k];
+}
 /* Distinct deviceId and resourceId values, the range of the timestamps and the number of rows that are
- * printed.  The workgroup that ends last ranks the values and plans the sort's keys. */
-__global__ void __launch_bounds__(KTJ_BLOCK) k_collect_distinct(Columns c, uint64_t n, SortSets s, Scalars* sc, int straight) {
+ * printed.  The workgroup that ends last ranks the values and plans the sort's keys.  With a book the first
+ * workgroup lays out the schemas instead of taking rows: this is the longest launch before the size pass that
+ * small passes have, too. */
+__global__ void __launch_bounds__(KTJ_BLOCK) k_collect_distinct(Columns c, uint64_t n, SortSets s, Scalars* sc, int straight, EmitCtx ctx, weave::SchemaBook* book) {
   __shared__ uint64_t red_min[KTJ_BLOCK >> 6], red_max[KTJ_BLOCK >> 6];
   __shared__ unsigned long long seen[2][LOCAL_SET_SLOTS + 1]; /* deviceId, resourceId values */
+  static_assert(sizeof(SchemaLds) <= sizeof(seen), "laid out where the values would be");
+  const uint32_t books = book ? 1u : 0u;
+  const bool lays_out = blockIdx.x < books;
   if (blockIdx.x == 0 && threadIdx.x == 0) stage_clock(sc, KTJ_CLOCK_SORT);
-  for (uint32_t k = threadIdx.x; k <= LOCAL_SET_SLOTS; k += blockDim.x) { seen[0][k] = KTJ_EMPTY_KEY; seen[1][k] = KTJ_EMPTY_KEY; }
+  if (lays_out) lay_out_schemas(ctx, book, reinterpret_cast<SchemaLds*>(seen));
+  else for (uint32_t k = threadIdx.x; k <= LOCAL_SET_SLOTS; k += blockDim.x) { seen[0][k] = KTJ_EMPTY_KEY; seen[1][k] = KTJ_EMPTY_KEY; }
   __syncthreads();
   uint64_t mn = ~0ULL, mx = 0ULL;
   uint64_t last_dev = 0, last_res = 0; /* of the thread's rows so far: most rows repeat them */
   bool any = false;
   uint32_t n_valid = 0;
-  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-  for (uint64_t a0 = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; a0 < n; a0 += stride * COLLECT_ROWS) {
+  const uint64_t stride = (uint64_t)(gridDim.x - books) * blockDim.x;
+  for (uint64_t a0 = lays_out ? n : (uint64_t)(blockIdx.x - books) * blockDim.x + threadIdx.x; a0 < n; a0 += stride * COLLECT_ROWS) {
     uint32_t meta[COLLECT_ROWS];
     uint64_t dev[COLLECT_ROWS], res[COLLECT_ROWS], ts[COLLECT_ROWS];
 #pragma unroll
@@ -1296,7 +1364,7 @@ hipError_t make_rank_keys(Columns c, const uint32_t* order, uint64_t n, SortSets
   return KTJ_LAUNCH_CHECK();
 }
 
-hipError_t collect_distinct(Columns c, uint64_t n, SortSets s, Scalars* sc, bool straight, hipStream_t st) {
+hipError_t collect_distinct(Columns c, uint64_t n, SortSets s, Scalars* sc, bool straight, const EmitCtx& ctx, weave::SchemaBook* book, hipStream_t st) {
   if (n == 0) return hipSuccess;
   /* few, fat workgroups: each one pays for its own local set once (few rows: one group each) */
   /* at most four workgroups per CU: every workgroup pays for its local sets and its atomics at the
@@ -1304,7 +1372,7 @@ hipError_t collect_distinct(Columns c, uint64_t n, SortSets s, Scalars* sc, bool
    * 1024: 0.17 ms) */
   unsigned g = grid_stride_for(n, n < (1u << 20) ? KTJ_BLOCK * COLLECT_ROWS : KTJ_BLOCK * 16);
   if (g > 1024u) g = 1024u;
-  hipLaunchKernelGGL(k_collect_distinct, dim3(g), dim3(KTJ_BLOCK), 0, st, c, n, s, sc, straight ? 1 : 0);
+  hipLaunchKernelGGL(k_collect_distinct, dim3(g + (book ? 1u : 0u)), dim3(KTJ_BLOCK), 0, st, c, n, s, sc, straight ? 1 : 0, ctx, book);
   return KTJ_LAUNCH_CHECK();
 }
 hipError_t make_keys(Columns c, uint64_t n, SortSets s, const Scalars* sc, uint32_t ts_bits, uint32_t res_bits,
@@ -2022,6 +2090,14 @@ __device__ __forceinline__ void rows_lds_to_global(T* rows, uint32_t cnt, const 
   const v4u* l = reinterpret_cast<const v4u*>(lds);
   for (uint32_t k = threadIdx.x; k < cnt * (uint32_t)(sizeof(T) / 16); k += blockDim.x) store_once(&g[k], l[k]);
 }
+/* rows that are a line of eight blocks, block b of row r at b ^ (r & 7): neighbouring lanes write theirs to other banks */
+template <>
+__device__ __forceinline__ void rows_lds_to_global(weave::TextRow* rows, uint32_t cnt, const uint4* lds) {
+  typedef unsigned int v4u __attribute__((ext_vector_type(4)));
+  v4u* g = reinterpret_cast<v4u*>(rows);
+  const v4u* l = reinterpret_cast<const v4u*>(lds);
+  for (uint32_t k = threadIdx.x; k < cnt * 8u; k += blockDim.x) store_once(&g[k], l[k ^ ((k >> 3) & 7u)]);
+}
 template <typename T>
 __device__ __forceinline__ T row_from_lds(const uint4* lds) {
   T r;
@@ -2096,8 +2172,28 @@ hipError_t stream_sync_first(const uint32_t* perm, uint64_t n_sorted, const ktj_
   return KTJ_LAUNCH_CHECK();
 }
 
+/* A joined row and its length are done: the row goes to the staging area as the emit kernels want it, and this is what is
+ * stored of its length. */
+template <bool TEXT> struct RowOf { typedef MatRow T; };
+template <> struct RowOf<true> { typedef weave::TextRow T; };
+template <bool TEXT>
+__device__ __forceinline__ uint32_t stage_row(const MatRow& m, const EmitCtx& ctx, const weave::SchemaBook* schemas, Scalars* sc, uint4* stage) {
+  if (!TEXT) { row_to_lds(m, stage); return row_length(m, ctx, sc); }
+  weave::TextRow* const t = reinterpret_cast<weave::TextRow*>(stage) + threadIdx.x;
+  uint32_t n, tail;
+  if (!(m.meta & KTJ_M_VALID)) n = 0;
+  else if (weave::text_row(m, ctx, schemas->plan, t, threadIdx.x & 7u, &n, &tail)) return n | (tail << 30);
+  else n = row_length(m, ctx, sc) | (KTJ_KIND_LEFT << 30);
+  static_assert(sizeof(MatRow) == 96, "six blocks");
+  auto block = [&](uint32_t k) { __builtin_memcpy(t->w[k ^ (threadIdx.x & 7u)], reinterpret_cast<const char*>(&m) + 16u * k, 16); };
+  block(0); block(1); block(2); block(3); block(4); block(5); /* (a loop would keep m in memory) */
+  t->w[7u ^ (threadIdx.x & 7u)][3] = KTJ_ROW_LEFT << 24;
+  return n;
+}
+
+template <bool TEXT>
 __device__ __forceinline__ void mat_generic_block(const ktj_generic_rec* g, uint64_t n, uint64_t first, const EmitCtx& ctx, const uint32_t* sync_first,
-                                                  MatRow* mat, uint32_t* len, Scalars* sc, uint64_t block, uint64_t blocks, uint4* stage) {
+                                                  Rows rows, uint32_t* len, Scalars* sc, uint64_t block, uint64_t blocks, uint4* stage) {
   RowStats rs;
   for (uint64_t base = block * KTJ_BLOCK; base < n; base += blocks * KTJ_BLOCK) {
     const uint32_t cnt = (uint32_t)(n - base < KTJ_BLOCK ? n - base : KTJ_BLOCK);
@@ -2113,13 +2209,12 @@ __device__ __forceinline__ void mat_generic_block(const ktj_generic_rec* g, uint
       if (!generic_record_prints(rec, ctx)) m.meta &= ~KTJ_M_VALID;
       attach_own_collective(m, rec, ctx);
       mark_stream_sync(m, ctx, sync_first != nullptr && sync_first[i] != 0);
-      len[first + i] = row_length(m, ctx, sc);
       count_row_stats(m, ctx, &rs);
     }
     __syncthreads(); /* every lane has taken its record */
-    if (active) row_to_lds(m, stage);
+    if (active) len[first + i] = stage_row<TEXT>(m, ctx, rows.schemas, sc, stage);
     __syncthreads();
-    rows_lds_to_global(mat + first + base, cnt, stage);
+    rows_lds_to_global(static_cast<typename RowOf<TEXT>::T*>(rows.p) + first + base, cnt, stage);
   }
   flush_row_stats(rs, sc);
 }
@@ -2180,8 +2275,9 @@ __device__ __forceinline__ bool bitmap_test_and_set(uint32_t* bitmap, uint32_t s
 #ifndef KX_JOIN_ATTR
 #define KX_JOIN_ATTR
 #endif
+template <bool TEXT>
 __global__ void KX_JOIN_ATTR k_join_runtime(const ktj_runtime_rec* r, uint64_t n, Columns c, uint64_t first_runtime, ApiTable api, Table tf,
-                               FullCols fc, Table tn, NarrowCols nc, uint32_t* slot_f, uint32_t* slot_n, EmitCtx ctx, MatRow* mat,
+                               FullCols fc, Table tn, NarrowCols nc, uint32_t* slot_f, uint32_t* slot_n, EmitCtx ctx, Rows rows,
                                uint32_t* len, Scalars* sc, int rounds) {
   RowStats rs;
   uint32_t n_linked = 0;
@@ -2189,7 +2285,7 @@ __global__ void KX_JOIN_ATTR k_join_runtime(const ktj_runtime_rec* r, uint64_t n
   /* a workgroup takes `rounds` consecutive groups of blockDim.x rows: the per-workgroup counters
    * at the end (one atomic each on a hot address) are paid once for all of them */
   static_assert(sizeof(MatRow) == sizeof(ktj_runtime_rec), "the staging area holds the records, then the joined rows");
-  __shared__ uint4 stage[KTJ_BLOCK * sizeof(ktj_runtime_rec) / 16];
+  __shared__ uint4 stage[KTJ_BLOCK * sizeof(typename RowOf<TEXT>::T) / 16];
   for (int round = 0; round < rounds; ++round) {
     const uint64_t base = ((uint64_t)blockIdx.x * rounds + round) * blockDim.x;
     if (base >= n) break;
@@ -2200,6 +2296,7 @@ __global__ void KX_JOIN_ATTR k_join_runtime(const ktj_runtime_rec* r, uint64_t n
     const uint64_t i = base + threadIdx.x;
     bool carries_stream = false;
     uint32_t sf = KTJ_NOSLOT;
+    MatRow m;
     /* everything the row reads from its own record and columns is requested up front, so that the
      * table accesses below (each a round trip of its own) overlap with it */
     const uint64_t a = first_runtime + (i < n ? i : 0);
@@ -2256,13 +2353,23 @@ __global__ void KX_JOIN_ATTR k_join_runtime(const ktj_runtime_rec* r, uint64_t n
       const bool known = rec.cid < api.n_cids;
       const uint32_t name = known ? api.cid_name_ids[rec.cid] : KTJ_NONE;
       const bool fstart = known && ((api.flow_start_bits[rec.cid >> 5] >> (rec.cid & 31u)) & 1u);
-      MatRow* m = reinterpret_cast<MatRow*>(my_slot);
-      *m = mat_runtime(rec, ts, dur, valid, ext, name, fstart, rec.cid == api.malloc_cid);
-      store_once(&len[a], row_length(*m, ctx, sc));
-      count_row_stats(*m, ctx, &rs);
+      if (TEXT) m = mat_runtime(rec, ts, dur, valid, ext, name, fstart, rec.cid == api.malloc_cid);
+      else {
+        MatRow* in_place = reinterpret_cast<MatRow*>(my_slot);
+        *in_place = mat_runtime(rec, ts, dur, valid, ext, name, fstart, rec.cid == api.malloc_cid);
+        store_once(&len[a], row_length(*in_place, ctx, sc));
+        count_row_stats(*in_place, ctx, &rs);
+      }
+    }
+    if (TEXT) { /* (its rows are longer than the records: every lane has taken its own before any is put down) */
+      __syncthreads();
+      if (i < n) {
+        count_row_stats(m, ctx, &rs);
+        store_once(&len[a], stage_row<true>(m, ctx, rows.schemas, sc, stage));
+      }
     }
     __syncthreads(); /* the joined rows go out the way the records came in */
-    rows_lds_to_global(mat + first_runtime + base, cnt, stage);
+    rows_lds_to_global(static_cast<typename RowOf<TEXT>::T*>(rows.p) + first_runtime + base, cnt, stage);
     any_carries_stream |= carries_stream;
     any_repeats |= repeats;
   }
@@ -2333,8 +2440,9 @@ __global__ void k_republish_runtime(const ktj_runtime_rec* r, uint64_t n, Column
   }
   block_add(sc, KTJ_CNT_OUT_OF_ORDER, n_bad);
 }
+template <bool TEXT>
 __device__ __forceinline__ void mat_device_block(const ktj_device_rec* d, uint64_t n, const Columns& c, uint64_t first, const DevLink* link,
-                                                 const EmitCtx& ctx, MatRow* mat, uint32_t* len, Scalars* sc, uint64_t block, uint64_t blocks,
+                                                 const EmitCtx& ctx, Rows rows, uint32_t* len, Scalars* sc, uint64_t block, uint64_t blocks,
                                                  uint4* stage) {
   RowStats rs;
   for (uint64_t base = block * KTJ_BLOCK; base < n; base += blocks * KTJ_BLOCK) {
@@ -2358,33 +2466,32 @@ __device__ __forceinline__ void mat_device_block(const ktj_device_rec* d, uint64
       m = mat_device_v(rec, load_once(&c.ts[a]), load_once(&c.dur[a]), load_once(&c.res[a]),
                        (load_once(&c.meta[a]) & KTJ_M_VALID) != 0, load_once(&c.ext[a]),
                        (l.flags & KTJ_DL_HAS_GRID) != 0, l.p[0], l.p[1], l.p[2], (l.flags & KTJ_DL_HAS_SIZE) != 0, l.p[0], l.coll);
-      store_once(&len[a], row_length(m, ctx, sc));
       count_row_stats(m, ctx, &rs);
     }
     __syncthreads(); /* every lane has taken its record */
-    if (active) row_to_lds(m, stage);
+    if (active) store_once(&len[a], stage_row<TEXT>(m, ctx, rows.schemas, sc, stage));
     __syncthreads();
-    rows_lds_to_global(mat + first + base, cnt, stage);
+    rows_lds_to_global(static_cast<typename RowOf<TEXT>::T*>(rows.p) + first + base, cnt, stage);
   }
   flush_row_stats(rs, sc);
 }
 /* joined rows and lengths of the generic records (first workgroups) and of the device records (the others);
  * the runtime rows' are made in k_join_runtime.  Few records: both classes in one launch.  Many: a launch for
  * each, as the code for both at once needs more registers (22 million: 690 against 575 us). */
-template <bool GENERIC, bool DEVICE>
+template <bool GENERIC, bool DEVICE, bool TEXT>
 __global__ void __launch_bounds__(KTJ_BLOCK) __attribute__((amdgpu_waves_per_eu(4)))
 k_mat_rows(const ktj_generic_rec* g, uint64_t ng, uint64_t first_generic, const uint32_t* sync_first, uint32_t generic_blocks, const ktj_device_rec* d,
-           uint64_t nd, Columns c, uint64_t first_device, const DevLink* link, EmitCtx ctx, MatRow* mat, uint32_t* len, Scalars* sc, int clock) {
+           uint64_t nd, Columns c, uint64_t first_device, const DevLink* link, EmitCtx ctx, Rows rows, uint32_t* len, Scalars* sc, int clock) {
   static_assert(sizeof(MatRow) >= sizeof(ktj_generic_rec) && sizeof(MatRow) >= sizeof(ktj_device_rec), "the staging area holds the records, then the joined rows");
-  __shared__ uint4 stage[KTJ_BLOCK * sizeof(MatRow) / 16];
+  __shared__ uint4 stage[KTJ_BLOCK * sizeof(typename RowOf<TEXT>::T) / 16];
   if (blockIdx.x == 0 && threadIdx.x == 0 && clock) stage_clock(sc, KTJ_CLOCK_SIZE);
   /* The pass ends, or the host takes another way from the sort on.  All wavefronts of a workgroup must see the same
    * here, as they move records for each other: the one bit that this launch sets does not count. */
   if (sc->error & ~KTJ_DEVERR_RECORD_TOO_LONG) return;
   if (GENERIC && (!DEVICE || blockIdx.x < generic_blocks))
-    mat_generic_block(g, ng, first_generic, ctx, sync_first, mat, len, sc, blockIdx.x, generic_blocks, stage);
+    mat_generic_block<TEXT>(g, ng, first_generic, ctx, sync_first, rows, len, sc, blockIdx.x, generic_blocks, stage);
   else if (DEVICE)
-    mat_device_block(d, nd, c, first_device, link, ctx, mat, len, sc, blockIdx.x - generic_blocks, gridDim.x - generic_blocks, stage);
+    mat_device_block<TEXT>(d, nd, c, first_device, link, ctx, rows, len, sc, blockIdx.x - generic_blocks, gridDim.x - generic_blocks, stage);
 }
 /* Collective metadata: the first activity, in emission order, that prints each entry, per
  * backend (first[2k] nccl, first[2k + 1] hccl).  The host replays appendCollectiveMetadata's
@@ -2413,8 +2520,9 @@ hipError_t collective_first(const MatRow* mat, const uint32_t* perm, uint64_t n_
 /* lengths and tail kinds in emission order (the size pass leaves both in one word per arrival index), and
  * the lengths' sum per tile of 2048 for the scan that follows */
 __global__ void __launch_bounds__(KTJ_BLOCK)
-k_gather_len(const uint32_t* perm, const uint32_t* len, uint64_t n, uint32_t* len_sorted, uint8_t* kind_sorted, uint64_t* sums, Scalars* sc) {
+k_gather_len(const uint32_t* perm, const uint32_t* len, uint64_t n, uint32_t* len_sorted, uint8_t* kind_sorted, uint64_t* sums, uint32_t* left, Scalars* sc) {
   __shared__ uint64_t wave_tot[KTJ_BLOCK >> 6];
+  __shared__ uint32_t n_left, left_at;
   if (blockIdx.x == 0 && threadIdx.x == 0) stage_clock(sc, KTJ_CLOCK_SCAN);
   if (sc->error != 0) return; /* there may be no order */
   const uint64_t base = (uint64_t)blockIdx.x * SCAN_TILE + threadIdx.x;
@@ -2423,10 +2531,12 @@ k_gather_len(const uint32_t* perm, const uint32_t* len, uint64_t n, uint32_t* le
   for (int k = 0; k < SCAN_ITEMS; ++k) { const uint64_t i = base + (uint64_t)k * KTJ_BLOCK; v[k] = i < n ? load_once(&perm[i]) : 0u; }
 #pragma unroll
   for (int k = 0; k < SCAN_ITEMS; ++k) { const uint64_t i = base + (uint64_t)k * KTJ_BLOCK; v[k] = i < n ? len[v[k]] : 0u; }
+  uint32_t n_mine = 0;
   unsigned long long sum = 0;
 #pragma unroll
   for (int k = 0; k < SCAN_ITEMS; ++k) {
     const uint64_t i = base + (uint64_t)k * KTJ_BLOCK;
+    n_mine += (v[k] >> 30) == KTJ_KIND_LEFT ? 1u : 0u;
     if (i < n) { len_sorted[i] = v[k] & 0x3FFFFFFFu; kind_sorted[i] = (uint8_t)(v[k] >> 30); }
     sum += v[k] & 0x3FFFFFFFu;
   }
@@ -2438,33 +2548,49 @@ k_gather_len(const uint32_t* perm, const uint32_t* len, uint64_t n, uint32_t* le
     for (uint32_t k = 0; k < (KTJ_BLOCK >> 6); ++k) s += wave_tot[k];
     sums[blockIdx.x] = s;
   }
+  /* the places of the rows that are left to emit_direct, in no particular order: one atomic per tile that has any */
+  if (!__syncthreads_or(n_mine != 0 ? 1 : 0)) return;
+  if (threadIdx.x == 0) n_left = 0;
+  __syncthreads();
+  uint32_t at = n_mine ? atomicAdd(&n_left, n_mine) : 0u;
+  __syncthreads();
+  if (threadIdx.x == 0) left_at = atomicAdd(&sc->n_left, n_left);
+  __syncthreads();
+  at += left_at;
+#pragma unroll
+  for (int k = 0; k < SCAN_ITEMS; ++k)
+    if ((v[k] >> 30) == KTJ_KIND_LEFT) left[at++] = (uint32_t)(base + (uint64_t)k * KTJ_BLOCK);
 }
 
 #define MAT_ONE_LAUNCH_ROWS 262144u
 hipError_t mat_rows(const ktj_generic_rec* g, uint64_t ng, uint64_t first_generic, const uint32_t* sync_first, const ktj_device_rec* d, uint64_t nd,
-                    Columns c, uint64_t first_device, const DevLink* link, EmitCtx ctx, MatRow* mat, uint32_t* len, Scalars* sc, hipStream_t st) {
+                    Columns c, uint64_t first_device, const DevLink* link, EmitCtx ctx, Rows rows, uint32_t* len, Scalars* sc, hipStream_t st) {
   const unsigned gb = grid_stride_for(ng, KTJ_BLOCK), db = grid_stride_for(nd, KTJ_BLOCK);
   auto launch = [&](auto kernel, unsigned g_blocks, unsigned d_blocks, bool clock) {
     hipLaunchKernelGGL(kernel, dim3(g_blocks + d_blocks), dim3(KTJ_BLOCK), 0, st, g, ng, first_generic, sync_first, g_blocks, d, nd, c, first_device,
-                       link, ctx, mat, len, sc, clock ? 1 : 0);
+                       link, ctx, rows, len, sc, clock ? 1 : 0);
   };
   const bool clock = first_generic == 0;
-  if (gb && db && ng + nd < MAT_ONE_LAUNCH_ROWS) launch(k_mat_rows<true, true>, gb, db, clock);
-  else {
-    if (gb) launch(k_mat_rows<true, false>, gb, 0, clock);
-    if (db) launch(k_mat_rows<false, true>, 0, db, clock && !gb);
+  if (gb && db && ng + nd < MAT_ONE_LAUNCH_ROWS) {
+    if (rows.schemas) launch(k_mat_rows<true, true, true>, gb, db, clock); else launch(k_mat_rows<true, true, false>, gb, db, clock);
+  } else {
+    if (gb) { if (rows.schemas) launch(k_mat_rows<true, false, true>, gb, 0, clock); else launch(k_mat_rows<true, false, false>, gb, 0, clock); }
+    if (db) { if (rows.schemas) launch(k_mat_rows<false, true, true>, 0, db, clock && !gb); else launch(k_mat_rows<false, true, false>, 0, db, clock && !gb); }
   }
   return KTJ_LAUNCH_CHECK();
 }
 
 hipError_t join_runtime_rows(const ktj_runtime_rec* r, uint64_t n, Columns c, uint64_t first, ApiTable api, Table tf, FullCols fc,
-                             Table tn, NarrowCols nc, uint32_t* slot_f, uint32_t* slot_n, EmitCtx ctx, MatRow* mat,
+                             Table tn, NarrowCols nc, uint32_t* slot_f, uint32_t* slot_n, EmitCtx ctx, Rows rows,
                              uint32_t* len, Scalars* sc, hipStream_t st) {
   if (n == 0) return hipSuccess;
   /* few rows: one group per workgroup, so that the launch is as wide and as short as it can be */
   const int rounds = n < JOIN_SMALL_ROWS ? 1 : JOIN_ROWS;
-  hipLaunchKernelGGL(k_join_runtime, dim3(grid_for(n, KTJ_BLOCK * rounds)), dim3(KTJ_BLOCK), 0, st, r, n, c, first, api, tf, fc, tn, nc,
-                     slot_f, slot_n, ctx, mat, len, sc, rounds);
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(grid_for(n, KTJ_BLOCK * rounds)), dim3(KTJ_BLOCK), 0, st, r, n, c, first, api, tf, fc, tn, nc,
+                       slot_f, slot_n, ctx, rows, len, sc, rounds);
+  };
+  if (rows.schemas) launch(k_join_runtime<true>); else launch(k_join_runtime<false>);
   return KTJ_LAUNCH_CHECK();
 }
 hipError_t republish_runtime_rows(const ktj_runtime_rec* r, uint64_t n, Columns c, uint64_t first, FullCols fc, NarrowCols nc,
@@ -2536,9 +2662,9 @@ k_offsets(const uint32_t* len, uint64_t n, const uint64_t* sums, uint32_t n_tile
 }
 uint64_t offsets_tmp_elems(uint64_t n) { return (n + SCAN_TILE - 1) / SCAN_TILE + 2; }
 hipError_t gather_offsets(const uint32_t* perm, const uint32_t* len, uint64_t n, uint32_t* len_sorted, uint8_t* kind_sorted, uint64_t* sums,
-                          uint64_t* offs, Scalars* sc, const DocText& text, hipStream_t st) {
+                          uint64_t* offs, uint32_t* left, Scalars* sc, const DocText& text, hipStream_t st) {
   const uint64_t tiles = n ? (n + SCAN_TILE - 1) / SCAN_TILE : 1;
-  hipLaunchKernelGGL(k_gather_len, dim3((unsigned)tiles), dim3(KTJ_BLOCK), 0, st, perm, len, n, len_sorted, kind_sorted, sums, sc);
+  hipLaunchKernelGGL(k_gather_len, dim3((unsigned)tiles), dim3(KTJ_BLOCK), 0, st, perm, len, n, len_sorted, kind_sorted, sums, left, sc);
   if (tiles > OFFS_DIRECT_TILES) hipLaunchKernelGGL(k_scan_of_sums, dim3(1), dim3(1024), 0, st, sums, tiles);
   const uint64_t prefix_blocks = text.out ? (text.n_prefix + PREFIX_PIECE - 1) / PREFIX_PIECE : 0;
   hipLaunchKernelGGL(k_offsets, dim3((unsigned)(tiles + 1u + prefix_blocks)), dim3(KTJ_BLOCK), 0, st, (const uint32_t*)len_sorted, n, (const uint64_t*)sums,

@@ -21,11 +21,11 @@ struct MatRow {
   int64_t dur;       /* duration(), unclamped                                                   */
   int64_t dev;       /* deviceId()                                                              */
   int64_t res;       /* resourceId()                                                            */
-  int64_t flow_id;   /* flowId()                                                                */
   uint32_t name_id;  /* dictionary id, or a KTJ_NAME_* code when KTJ_M_NAME_BUILTIN              */
   uint32_t meta;     /* KTJ_M_* bit fields                                                      */
   int32_t ext;       /* "External id" value, 0 = none                                           */
   uint32_t aux;      /* generic: schema id; runtime: cid; device: op                            */
+  int64_t flow_id;   /* flowId()                                                                */
   uint64_t p[5];     /* payload, see below                                                      */
 };
 /* payload by class:

@@ -1,0 +1,482 @@
+/*
+ * weave.hip — stage 4b: the activities' text into the document, one lane per segment (weave_core.h).
+ *
+ * A lane per activity (k_emit_direct) walks its text piece by piece: 4420 vector instructions for 64 activities with
+ * the lanes of a wavefront at different pieces, 168 registers for three wavefronts per SIMD, and no pass shorter than 38 us
+ * as every wavefront runs through all of the formatter's code.  Here the text of 16 activities is laid out by the four
+ * lanes that load each row, as a list of parts; then 64 segments at a time are fetched (a descriptor, up to 64 bytes of
+ * text from LDS, a number of the row's), a prefix sum of their lengths gives their places, and they are OR-ed into a
+ * zero-filled piece of the document in LDS, whose whole lines leave with lane-consecutive stores.  Numbers were made
+ * into text in the size pass, which needs their lengths anyway; the texts with process and thread are made once per
+ * track.  3220 vector and 770 LDS instructions for 64 kernel events, 119 registers, four wavefronts per SIMD.
+ *
+ * What bounds it: the LDS pipe (1.02 of 1.9 ms for 11 million kernels, a third of that bank conflicts) and the
+ * vector units (0.9 ms) together with the waits between them; the bytes alone (1.4 GB of rows, 5.4 GB of document)
+ * take 1.3 ms.  Measured against k_emit_direct: 10 000 x 3 records 38.7 -> 17.5 us, 4000 operators with long strings
+ * 71 -> 35 us, 733 000 records 176 -> 153 us, 3 million 795 -> 490 us, 11 million kernels 2.06 -> 1.91 ms, 22 million
+ * records 4.59 -> 3.80 ms, 5 million operators with long strings (1.4 KB each: strings beyond 128 bytes are fetched from
+ * memory piece by piece) 3.20 -> 3.24 ms; the size pass has become 4 to 13 % longer for the numbers' text.
+ * Of the places: 16 activities a turn (32 need more LDS than two workgroups of eight wavefronts have); 2688 bytes of
+ * document, room for nearly all groups of 64 segments.
+ */
+#include "gpu_common.h"
+#include "weave_core.h"
+
+namespace ktj {
+namespace gpu {
+
+using namespace weave;
+
+#define WV_ROWS 16u                                   /* activities at a time, four lanes to each */
+#define WV_WAVES 8u                                   /* wavefronts per workgroup, at most */
+#define WV_PARTS (WV_ROWS * 7u)
+#define WV_VAL_BYTES (S_COUNT * 16u)                  /* an odd number of sixteens: the same slot of neighbours lies in other banks */
+#define WV_NAMES 1280u                                /* bytes of strings that wait in LDS */
+#define WV_NAME_MOST 128u
+#define WV_TILE 2688u                                 /* bytes of document that wait in LDS */
+#define WV_TILE_ROOM (WV_TILE + 128u)                 /* a line behind it, and what texts write beyond their end */
+/* of a wavefront: */
+#define WV_NAMES_AT (WV_ROWS * WV_VAL_BYTES)
+#define WV_DESC_AT (WV_NAMES_AT + WV_NAMES)
+#define WV_TRACK_AT (WV_DESC_AT + (MAX_DESC + SCHEMA_DESC) * 4u)
+#define WV_PARTS_AT (WV_TRACK_AT + T_COUNT * KTJ_WEAVE_LIT)
+#define WV_TILE_AT (WV_PARTS_AT + WV_PARTS * 4u + 32u)
+#define WV_WAVE_BYTES (WV_TILE_AT + WV_TILE_ROOM)
+/* of the workgroup, in front of them: the book up to its descriptors */
+#define WV_BOOK_REF (MAX_TEXT * 16u)
+#define WV_BOOK_PATCH (WV_BOOK_REF + R_COUNT * 4u)
+#define WV_BOOK_SCHEMA (SCHEMA_UNIT * 16u)            /* texts and plans of the schemas */
+#define WV_BOOK_PLANS (WV_BOOK_SCHEMA + SCHEMA_TEXT * 16u)
+#define WV_BOOK_BYTES (WV_BOOK_PLANS + MAX_SCHEMAS * (uint32_t)sizeof(SchemaPlan))
+
+/* a part: first segment | kind << 15 (text, or the string of S_RUN0 or S_RUN1) | first descriptor << 17 | activity << 26 */
+#define WV_PART_START(x) ((x) & 0x7FFFu)
+#define WV_PART_KIND(x) (((x) >> 15) & 3u)
+#define WV_PART_DESC(x) (((x) >> 17) & 0x1FFu)
+#define WV_PART_ACT(x) ((x) >> 26)
+
+static __device__ constexpr Book g_book = BOOK;
+
+__device__ __forceinline__ uint32_t dpp_add(uint32_t v) { /* inclusive sum over the wavefront */
+#define WV_DPP(ctrl, rows) v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, rows, 0xF, false)
+  WV_DPP(0x111, 0xF); WV_DPP(0x112, 0xF); WV_DPP(0x114, 0xF); WV_DPP(0x118, 0xF);
+  WV_DPP(0x142, 0xA); WV_DPP(0x143, 0xC);
+#undef WV_DPP
+  return v;
+}
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+__device__ __forceinline__ void or_word(char* p, uint32_t v) {
+  __hip_atomic_fetch_or(reinterpret_cast<uint32_t*>(p), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+}
+typedef unsigned long long v2u64 __attribute__((ext_vector_type(2)));
+typedef uint32_t v4u32 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ void or_text(char* q, uint32_t sh, const v4u32& x, uint32_t before) { /* four words of a text: those at q on */
+  or_word(q, __builtin_amdgcn_alignbyte(x.x, before, sh)); or_word(q + 4, __builtin_amdgcn_alignbyte(x.y, x.x, sh));
+  or_word(q + 8, __builtin_amdgcn_alignbyte(x.z, x.y, sh)); or_word(q + 12, __builtin_amdgcn_alignbyte(x.w, x.z, sh));
+}
+/* a segment (zeros behind its text and its number) to byte p of a zero-filled buffer */
+__device__ __forceinline__ void or_segment(char* buf, uint32_t p, uint32_t len, const v4u32& a, const v4u32& b, const v4u32& c, const v4u32& d,
+                                           uint32_t n_num, const v4u32& num) {
+  const uint32_t sh = 0u - p;                                   /* bits 0 and 1 count */
+  char* q = buf + (int32_t)(((int32_t)p - 1) & ~3);             /* the word of the byte before */
+  or_text(q, sh, a, 0u);
+  or_word(q + 16, __builtin_amdgcn_alignbyte(b.x, a.w, sh));
+  if (n_num) {
+    const uint32_t p2 = p + len, sh2 = 0u - p2;
+    char* q2 = buf + (int32_t)(((int32_t)p2 - 1) & ~3);
+    or_word(q2, __builtin_amdgcn_alignbyte(num.x, 0u, sh2)); or_word(q2 + 4, __builtin_amdgcn_alignbyte(num.y, num.x, sh2));
+    or_word(q2 + 8, __builtin_amdgcn_alignbyte(num.z, num.y, sh2));
+    if (n_num > 8u) { or_word(q2 + 12, __builtin_amdgcn_alignbyte(num.w, num.z, sh2)); or_word(q2 + 16, __builtin_amdgcn_alignbyte(0u, num.w, sh2)); }
+  }
+  if (len > 16u) {
+    or_word(q + 20, __builtin_amdgcn_alignbyte(b.y, b.x, sh)); or_word(q + 24, __builtin_amdgcn_alignbyte(b.z, b.y, sh));
+    or_word(q + 28, __builtin_amdgcn_alignbyte(b.w, b.z, sh)); or_word(q + 32, __builtin_amdgcn_alignbyte(c.x, b.w, sh));
+    if (len > 32u) {
+      or_word(q + 36, __builtin_amdgcn_alignbyte(c.y, c.x, sh)); or_word(q + 40, __builtin_amdgcn_alignbyte(c.z, c.y, sh));
+      or_word(q + 44, __builtin_amdgcn_alignbyte(c.w, c.z, sh)); or_word(q + 48, __builtin_amdgcn_alignbyte(d.x, c.w, sh));
+      if (len > 48u) {
+        or_word(q + 52, __builtin_amdgcn_alignbyte(d.y, d.x, sh)); or_word(q + 56, __builtin_amdgcn_alignbyte(d.z, d.y, sh));
+        or_word(q + 60, __builtin_amdgcn_alignbyte(d.w, d.z, sh)); or_word(q + 64, __builtin_amdgcn_alignbyte(0u, d.w, sh));
+      }
+    }
+  }
+}
+extern __shared__ __attribute__((aligned(16))) char wv_lds[];
+/* a double's text to the 32 bytes at `at`; its length.  Not inlined: it takes more registers than what surrounds it. */
+static __device__ __attribute__((noinline)) uint32_t double_text(uint64_t bits, uint32_t at) {
+  LongText t;
+  t.w[0] = t.w[1] = t.w[2] = t.w[3] = 0; t.n = 0;
+  put_f64(t, bits);
+  v2u64* v = reinterpret_cast<v2u64*>(wv_lds + at);
+  v[0] = (v2u64){t.w[0], t.w[1]};
+  v[1] = (v2u64){t.w[2], 0};
+  return t.n;
+}
+/* the track's texts and the descriptors that use them */
+__device__ __forceinline__ void make_track(char* lds, uint32_t mine, uint64_t dev, uint64_t thread) {
+  const uint32_t lane = lane_id();
+  char* const track = lds + mine + WV_TRACK_AT;
+  if (lane < T_COUNT * 4u) *reinterpret_cast<uint4*>(track + lane * 16u) = make_uint4(0, 0, 0, 0);
+  const Text pid = text_of(dev), tid = text_of(thread);
+  const uint32_t desc = lane < N_PIECES ? *reinterpret_cast<const uint32_t*>(lds + mine + WV_DESC_AT + (KTJ_WREF_BASE(g_book.ref[R_PIECES]) + lane) * 4u) : 0u;
+  const uint32_t len = KTJ_WD_LEN(desc), slot = KTJ_WD_SLOT(desc), n_num = slot == S_PID ? pid.n : slot == S_TID ? tid.n : 0u;
+  const v4u32 zero = {0, 0, 0, 0};
+  v4u32 a = zero, b = zero, num = zero;
+  const v4u32* t = reinterpret_cast<const v4u32*>(lds) + KTJ_WD_UNIT(desc);
+  if (len) a = t[0];
+  if (len > 16u) b = t[1];
+  if (slot == S_PID) { num.x = (uint32_t)pid.lo; num.y = (uint32_t)(pid.lo >> 32); num.z = (uint32_t)pid.hi; num.w = (uint32_t)(pid.hi >> 32); }
+  if (slot == S_TID) { num.x = (uint32_t)tid.lo; num.y = (uint32_t)(tid.lo >> 32); num.z = (uint32_t)tid.hi; num.w = (uint32_t)(tid.hi >> 32); }
+  const uint32_t end = dpp_add(len + n_num);
+  /* pieces 0-2, 3-5, 6-8, 9-10, 11-12 are a text each */
+  const uint32_t which = lane < 9u ? lane / 3u : lane < 11u ? 3u : 4u;
+  const uint32_t e2 = __builtin_amdgcn_readlane(end, 2), e5 = __builtin_amdgcn_readlane(end, 5), e8 = __builtin_amdgcn_readlane(end, 8),
+                 e10 = __builtin_amdgcn_readlane(end, 10), e12 = __builtin_amdgcn_readlane(end, 12);
+  const uint32_t start = which == 0 ? 0u : which == 1 ? e2 : which == 2 ? e5 : which == 3 ? e8 : e10;
+  wave_lds_order();
+  if (lane < N_PIECES) or_segment(track, which * KTJ_WEAVE_LIT + (end - len - n_num - start), len, a, b, zero, zero, n_num, num);
+  if (lane < g_book.n_patch) {
+    const uint32_t p = *reinterpret_cast<const uint32_t*>(lds + WV_BOOK_PATCH + lane * 4u), text = p >> 16;
+    const uint32_t n = text == 0 ? e2 : text == 1 ? e5 - e2 : text == 2 ? e8 - e5 : text == 3 ? e10 - e8 : e12 - e10;
+    uint32_t* d = reinterpret_cast<uint32_t*>(lds + mine + WV_DESC_AT + (p & 0xFFFFu) * 4u);
+    *d = KTJ_WD(n, KTJ_WD_SLOT(*d), text * (KTJ_WEAVE_LIT / 16u)) | KTJ_WD_TRACK;
+  }
+}
+
+__global__ void __launch_bounds__(WV_WAVES * 64u) __attribute__((amdgpu_waves_per_eu(4)))
+k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const uint8_t* kind_sorted, EmitCtx ctx, char* out, uint64_t prefix_len,
+        const Scalars* sc, uint32_t rounds, const SchemaBook* schemas) {
+  const uint32_t lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  for (uint32_t k = threadIdx.x; k < (WV_BOOK_BYTES - WV_BOOK_SCHEMA) / 16u; k += blockDim.x)
+    reinterpret_cast<uint4*>(wv_lds + WV_BOOK_SCHEMA)[k] = reinterpret_cast<const uint4*>(schemas)[k];
+  for (uint32_t k = threadIdx.x; k < WV_BOOK_SCHEMA / 4u; k += blockDim.x) /* texts, parts and patches lie one behind the other */
+    reinterpret_cast<uint32_t*>(wv_lds)[k] = reinterpret_cast<const uint32_t*>(&g_book)[k];
+  const uint32_t mine = WV_BOOK_BYTES + wave * WV_WAVE_BYTES; /* this wavefront's LDS */
+  const uint32_t* const refs = reinterpret_cast<const uint32_t*>(wv_lds + WV_BOOK_REF);
+  uint32_t* const parts = reinterpret_cast<uint32_t*>(wv_lds + mine + WV_PARTS_AT);
+  char* const tile = wv_lds + mine + WV_TILE_AT;
+  for (uint32_t k = lane; k < WV_TILE_ROOM / 16u; k += 64u) reinterpret_cast<uint4*>(tile)[k] = make_uint4(0, 0, 0, 0);
+  for (uint32_t k = lane; k < MAX_DESC + SCHEMA_DESC; k += 64u)
+    *reinterpret_cast<uint32_t*>(wv_lds + mine + WV_DESC_AT + k * 4u) = k < MAX_DESC ? g_book.desc[k] : schemas->desc[k - MAX_DESC];
+  if (lane < WV_ROWS) *reinterpret_cast<uint4*>(wv_lds + mine + lane * WV_VAL_BYTES) = make_uint4(0, 0, 0, 0); /* S_NONE */
+  __syncthreads();
+  const uint64_t n_rows = sc->emit_rows;
+  typedef __attribute__((address_space(1))) v2u64* gptr;
+  typedef const __attribute__((address_space(1))) v4u32* gsrc;
+
+  const uint32_t h = lane & 3u, act = lane >> 2;
+  v2u64* const vals = reinterpret_cast<v2u64*>(wv_lds + mine + act * WV_VAL_BYTES);
+  uint64_t track_made = ~0ull; /* what the track's texts are made of */
+  uint32_t track_made_high = ~0u;
+  const uint64_t i_begin = ((uint64_t)blockIdx.x * (blockDim.x >> 6) + wave) * rounds * WV_ROWS;
+  if (i_begin >= n_rows) return;
+  const uint64_t i_end = i_begin + rounds * WV_ROWS < n_rows ? i_begin + rounds * WV_ROWS : n_rows;
+  /* A row's four lanes load it together, two blocks each.  The rows of the next turn are on their way while this one's are
+   * put together. */
+  v4u32 q0, q1;
+  auto load_row = [&](uint32_t row) {
+    const gsrc r = reinterpret_cast<gsrc>((uint64_t)(uintptr_t)rows + (uint64_t)row * sizeof(TextRow));
+    q0 = r[h];                           /* S_Z, S_EXT, S_FLOW, S_DUR and plan, name, lens, more */
+    q1 = r[4u + h];                      /* S_A and the track, S_TS, S_X, S_Y */
+  };
+  uint32_t row = i_begin + act < i_end ? perm[i_begin + act] : 0u;
+  load_row(row);
+  row = i_begin + WV_ROWS + act < i_end ? perm[i_begin + WV_ROWS + act] : 0u;
+
+  uint32_t part = 0, pend = 0, own = 0;
+  char* doc = nullptr;
+  bool open = false;
+  /* the document's bytes end here for this wavefront: the block shared with what follows */
+  auto close_document = [&](uint64_t i_next) {
+    open = false;
+    const uint32_t fill = pend & 15u, at = pend & ~15u;
+    if (lane == 0 && fill) {
+      uint64_t* t = reinterpret_cast<uint64_t*>(tile + at);
+      uint64_t* w = reinterpret_cast<uint64_t*>(doc + at);
+      if (i_next == n_rows) {
+        if (fill < 8) { const uint64_t k = (1ull << (8 * fill)) - 1ull; t[0] |= w[0] & ~k; t[1] = w[1]; }
+        else if (fill > 8) { const uint64_t k = (1ull << (8 * (fill - 8))) - 1ull; t[1] |= w[1] & ~k; }
+        else t[1] = w[1];
+      } else if (fill >= 8) { /* the successor's first bytes complete it */
+        const uint32_t n = 16u - fill;
+        const uint64_t hb = BlockWriter::head_bytes() & (n == 8 ? ~0ull : (1ull << (8 * n)) - 1ull);
+        t[1] |= hb << (8 * (fill - 8));
+      }
+    }
+    wave_lds_order();
+    const uint32_t blocks = (pend >> 4) + (fill >= 8 || (fill && i_next == n_rows) ? 1u : 0u);
+    if (lane <= 8u) {
+      v2u64* tb = reinterpret_cast<v2u64*>(tile);
+      const v2u64 x = tb[lane];
+      tb[lane] = (v2u64){0, 0};
+      if (lane >= own && lane < blocks) reinterpret_cast<gptr>((uintptr_t)doc)[lane] = x;
+    }
+    wave_lds_order();
+  };
+
+  for (uint64_t i0 = i_begin; i0 < i_end; i0 += WV_ROWS) {
+    const bool active = i0 + act < i_end;
+    /* rows that format_activity prints are another kernel's */
+    const uint64_t left_of = __ballot(!active || (h == 3u && (q1.w >> 24) == KTJ_ROW_LEFT));
+    const uint64_t ok_mask = ~(left_of | (left_of >> 3)) & 0x1111111111111111ull; /* a bit at the first lane of each of the others */
+    const bool mine_ok = (ok_mask >> (lane & ~3u)) & 1u;
+#define WV_QUAD(x, k) ((uint32_t)__builtin_amdgcn_mov_dpp((int)(x), (k) * 0x55, 0xF, 0xF, true)) /* the k-th lane's, for all four */
+    /* (the first lane's:) */
+    const uint32_t plan = q0.w, name_off = WV_QUAD(q0.w, KTJ_TR_NAME), lens = WV_QUAD(q0.w, KTJ_TR_LENS), more = WV_QUAD(q0.w, KTJ_TR_MORE);
+    const uint64_t track = (uint64_t)q1.z | ((uint64_t)q1.w << 32);
+    /* activities whose track is not that of the one before: a bit at the first lane of each */
+    uint64_t new_track;
+    {
+      uint64_t before = __shfl_up((unsigned long long)track, 4);
+      uint32_t before_high = __shfl_up(KTJ_TR_TID_HIGH(plan), 4);
+      if (lane == 0u) { before = track_made; before_high = track_made_high; }
+      new_track = __ballot(h == 0u && (track != before || KTJ_TR_TID_HIGH(plan) != before_high));
+    }
+    const v4u32 z = {q0.x, q0.y, q0.z & 0xFFFFFFu, q0.z & 0xFF000000u};
+    vals[S_Z + h] = __builtin_bit_cast(v2u64, z);
+    {
+      const v4u32 a = {q1.x, q1.y & 0xFFFFFFu, 0u, q1.y & 0xFF000000u}, x = h == 0u ? a : q1;
+      vals[S_A + h] = __builtin_bit_cast(v2u64, x);
+    }
+    /* how many segments and parts, and the room for the name (the first lane) */
+    uint32_t counts = 0, units = 0, args_ref = 0, args2_ref = 0;
+    uint32_t len0 = lens & 0xFFFFu, len1 = lens >> 16;
+    if (h == 0u && mine_ok) {
+      if (KTJ_TR_ARGS(plan) == A_COPY) { /* a copy's kind, up to four characters */
+        const uint32_t n = (32u - (uint32_t)__clz((int)more) + 7u) >> 3;
+        vals[S_K] = (v2u64){more, (uint64_t)n << 56};
+      }
+      if (KTJ_TR_BETWEEN(plan) == 3u) len1 = double_text(ctx.args[more], mine + act * WV_VAL_BYTES + S_K * 16u);
+      const uint32_t a = KTJ_TR_ARGS(plan);
+      if (a >= KTJ_TR_SCHEMA) {
+        if (a != KTJ_TR_NO_ARGS) {
+          const SchemaPlan* p = reinterpret_cast<const SchemaPlan*>(wv_lds + WV_BOOK_PLANS) + (a - KTJ_TR_SCHEMA);
+          args_ref = p->args; args2_ref = p->args2;
+        }
+      } else { args_ref = refs[R_ARGS + a]; args2_ref = refs[R_ARGS2 + a]; }
+      const uint32_t name = KTJ_TR_NAMED(plan) != KTJ_TR_NAME_RUN ? KTJ_WREF_COUNT(refs[KTJ_TR_NAMED(plan)]) : (len0 + KTJ_WEAVE_LIT - 1u) / KTJ_WEAVE_LIT;
+      const uint32_t runs = (len1 + KTJ_WEAVE_LIT - 1u) / KTJ_WEAVE_LIT;
+      const uint32_t head = KTJ_WREF_COUNT(refs[R_HEAD + KTJ_TR_TYPE(plan)]), body = KTJ_WREF_COUNT(refs[R_BODY_NONE + KTJ_TR_BODY(plan)]);
+      const uint32_t tail = KTJ_WREF_COUNT(refs[R_TAIL + KTJ_TR_TAIL(plan)]);
+      const uint32_t args = KTJ_WREF_COUNT(args_ref), args2 = KTJ_WREF_COUNT(args2_ref);
+      counts = ((2u + (name ? 1u : 0u) + (args ? 1u : 0u) + (runs ? 1u : 0u) + (args2 ? 1u : 0u) + (tail ? 1u : 0u)) << 16) |
+               (head + name + body + args + runs + args2 + tail);
+      units = len0 <= WV_NAME_MOST ? (len0 + 15u) / 16u : 0u;
+    }
+    const uint32_t upto = dpp_add(counts), before = upto - counts; /* of the first lane of each */
+    const uint32_t units_upto = dpp_add(units);
+    const bool near = units != 0 && units_upto <= WV_NAMES / 16u;
+    const uint32_t name_at = WV_NAMES_AT + (units_upto - units) * 16u;
+    v4u32 nx, ny;
+    const uint32_t q_units = WV_QUAD(near ? units : 0u, 0), q_at = mine + WV_QUAD(name_at, 0);
+    {
+      const gsrc src = reinterpret_cast<gsrc>((uint64_t)(uintptr_t)ctx.dict.name_blob + (uint64_t)name_off * 16u);
+      if (h < q_units) { nx = src[h]; if (h + 4u < q_units) ny = src[h + 4u]; }
+    }
+#undef WV_QUAD
+    if (counts) {
+      uint32_t* w = parts + (before >> 16);
+      uint32_t seg = (before & 0x7FFFu) | (act << 26); /* (segments stay below their 15 bits) */
+      auto put_part = [&](uint32_t ref) { const uint32_t n = KTJ_WREF_COUNT(ref); if (n) { *w++ = seg | (KTJ_WREF_BASE(ref) << 17); seg += n; } };
+      put_part(refs[R_HEAD + KTJ_TR_TYPE(plan)]);
+      if (KTJ_TR_NAMED(plan) != KTJ_TR_NAME_RUN) put_part(refs[KTJ_TR_NAMED(plan)]);
+      else if (len0) { *w++ = seg | (1u << 15); seg += (len0 + KTJ_WEAVE_LIT - 1u) / KTJ_WEAVE_LIT; }
+      put_part(refs[R_BODY_NONE + KTJ_TR_BODY(plan)]);
+      put_part(args_ref);
+      if (len1) { *w++ = seg | (2u << 15); seg += (len1 + KTJ_WEAVE_LIT - 1u) / KTJ_WEAVE_LIT; }
+      put_part(args2_ref);
+      put_part(refs[R_TAIL + KTJ_TR_TAIL(plan)]);
+      v2u64 z;
+      z.x = (uint64_t)(uintptr_t)ctx.dict.name_blob + (uint64_t)name_off * 16u;
+      z.y = len0 | ((uint64_t)(near ? name_at : 0u) << 32);
+      vals[S_RUN0] = z;
+      if (len1) {
+        const uint32_t what = KTJ_TR_BETWEEN(plan);
+        z.x = (uint64_t)(uintptr_t)ctx.dict.arg_blob + (uint64_t)more * 16u;
+        z.y = len1 | ((uint64_t)(what == 1u ? 0u : act * WV_VAL_BYTES + (what == 2u ? S_Y : S_K) * 16u) << 32);
+        vals[S_RUN1] = z;
+      }
+    }
+    const uint32_t totals = __builtin_amdgcn_readlane(upto, 63);
+    if (lane == 0) parts[totals >> 16] = totals & 0x7FFFu;
+    if (h < q_units) {
+      *reinterpret_cast<v4u32*>(wv_lds + q_at + h * 16u) = nx;
+      if (h + 4u < q_units) *reinterpret_cast<v4u32*>(wv_lds + q_at + (h + 4u) * 16u) = ny;
+    }
+    /* the next turn's rows */
+    if (i0 + WV_ROWS < i_end) {
+      load_row(row);
+      row = i0 + 2u * WV_ROWS + act < i_end ? perm[i0 + 2u * WV_ROWS + act] : 0u;
+    }
+
+    /* ---- neighbouring activities of a track ---- */
+    if (open && !(ok_mask & 1u)) close_document(i0);
+    uint64_t todo = ok_mask, track_seen = 0; /* ..: activities whose change of track the texts have followed */
+    while (todo) {
+      const uint32_t first = (uint32_t)__ffsll((unsigned long long)todo) - 1u; /* lanes: four to an activity */
+      const uint64_t later = first >= 60u ? 0ull : ~0ull << (first + 4u);
+      const uint64_t gap = ((~todo & 0x1111111111111111ull) | new_track) & later;
+      const uint32_t next_lane = gap ? (uint32_t)__ffsll((unsigned long long)gap) - 1u : 64u, last = next_lane - 4u;
+      todo &= next_lane == 64u ? 0ull : ~0ull << next_lane;
+      uint32_t g = __builtin_amdgcn_readlane(before, first) & 0x7FFFu;
+      const uint32_t g_end = __builtin_amdgcn_readlane(upto, last) & 0x7FFFu;
+      part = __builtin_amdgcn_readlane(before, first) >> 16;
+      const uint64_t upto_first = first >= 60u ? ~0ull : (1ull << (first + 4u)) - 1ull;
+      if (new_track & upto_first & ~track_seen) {
+        const uint32_t low = __builtin_amdgcn_readlane((uint32_t)track, first), high = __builtin_amdgcn_readlane((uint32_t)(track >> 32), first);
+        track_made_high = KTJ_TR_TID_HIGH(__builtin_amdgcn_readlane(plan, first));
+        track_made = (uint64_t)low | ((uint64_t)high << 32);
+        make_track(wv_lds, mine, low & ((1u << KTJ_TR_DEV_BITS) - 1u), (track_made >> KTJ_TR_DEV_BITS) | ((uint64_t)track_made_high << 42));
+        track_seen = upto_first;
+      }
+      if (!open) {
+        open = true;
+        const uint64_t i_first = i0 + (first >> 2), pos = prefix_len + offs[i_first];
+        doc = out + (pos & ~127ull);
+        pend = (uint32_t)(pos & 127u);   /* bytes of the tile in use */
+        own = pend >> 4;                 /* first block of the tile that this wavefront stores */
+        const uint32_t fill = pend & 15u;
+        if (fill) {
+          if (i_first == 0) { /* what precedes the first activity is in the document already */
+            if (lane == 0) {
+              uint64_t* w = reinterpret_cast<uint64_t*>(doc + (pend & ~15u));
+              uint64_t lo = w[0], hi = w[1];
+              if (fill < 8) { lo &= (1ull << (8 * fill)) - 1ull; hi = 0; } else if (fill > 8) hi &= (1ull << (8 * (fill - 8))) - 1ull; else hi = 0;
+              uint64_t* t = reinterpret_cast<uint64_t*>(tile + (pend & ~15u));
+              t[0] = lo; t[1] = hi;
+            }
+          } else if (fill < 8) {
+            if (lane == 0) *reinterpret_cast<uint64_t*>(tile + (pend & ~15u)) = tail_bytes(tail_kind_at(kind_sorted, rows, perm, i_first - 1, ctx), fill);
+          } else ++own; /* the predecessor writes this block */
+        }
+      }
+      wave_lds_order();
+      /* 64 segments at a time: what the next ones are made of is read before these are put together */
+      struct Piece { v4u32 a, num; uint32_t desc, at, pr, s; bool valid; };
+      auto fetch = [&](uint32_t g, uint32_t& part) {
+        Piece x;
+        /* which part each segment belongs to: a part's first segment is marked, the marks counted */
+        const uint32_t rel = WV_PART_START(parts[part + lane]) - g; /* (behind the last part: what lies there, which does not count) */
+        const bool inside = part + lane <= (totals >> 16) && rel - 1u < 64u;
+        const uint64_t marks = __ballot(__builtin_amdgcn_ds_permute((int)(inside && rel < 64u ? rel * 4u : 0u), 1) != 0);
+        const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(marks >> 33), __builtin_amdgcn_mbcnt_lo((uint32_t)(marks >> 1), 0u));
+        x.pr = parts[part + rank];
+        part += (uint32_t)__popcll(__ballot(inside && rel <= g_end - g)); /* (the next activities' are theirs) */
+        x.valid = g + lane < g_end;
+        x.s = g + lane - WV_PART_START(x.pr);
+        if (!x.valid) x.pr = 0;
+        const uint32_t kind = WV_PART_KIND(x.pr), vrow = mine + WV_PART_ACT(x.pr) * WV_VAL_BYTES;
+        const uint32_t idx = kind == 0 && x.valid ? WV_PART_DESC(x.pr) + x.s : 0u;
+        x.desc = *reinterpret_cast<const uint32_t*>(wv_lds + mine + WV_DESC_AT + idx * 4u);
+        x.at = KTJ_WD_UNIT(x.desc) * 16u + (x.desc & KTJ_WD_TRACK ? mine + WV_TRACK_AT : 0u);
+        if (kind != 0) {
+          const uint64_t r = *reinterpret_cast<const uint64_t*>(wv_lds + vrow + S_RUN0 * 16u + (kind - 1u) * 16u + 8u);
+          const uint32_t rest = (uint32_t)r - x.s * KTJ_WEAVE_LIT, near = (uint32_t)(r >> 32);
+          x.at = near ? mine + near + x.s * KTJ_WEAVE_LIT : ~0u;
+          x.desc = KTJ_WD(rest < KTJ_WEAVE_LIT ? rest : KTJ_WEAVE_LIT, S_NONE, 0u);
+        }
+        x.a = *reinterpret_cast<const v4u32*>(wv_lds + (x.at != ~0u ? x.at : 0u));
+        x.num = *reinterpret_cast<const v4u32*>(wv_lds + vrow + KTJ_WD_SLOT(x.desc) * 16u);
+        return x;
+      };
+      auto put = [&](Piece& x) {
+        const uint32_t len = KTJ_WD_LEN(x.desc);
+        const bool far = x.at == ~0u;
+        v4u32 b = {0, 0, 0, 0}, c = b, d = b;
+        if (len > 16u && !far) {
+          b = *reinterpret_cast<const v4u32*>(wv_lds + x.at + 16u);
+          if (len > 32u) {
+            c = *reinterpret_cast<const v4u32*>(wv_lds + x.at + 32u);
+            if (len > 48u) d = *reinterpret_cast<const v4u32*>(wv_lds + x.at + 48u);
+          }
+        }
+        if (__any(far)) {
+          if (far) {
+            const uint64_t p = *reinterpret_cast<const uint64_t*>(wv_lds + mine + WV_PART_ACT(x.pr) * WV_VAL_BYTES + (S_RUN0 - 1u + WV_PART_KIND(x.pr)) * 16u);
+            const gsrc src = reinterpret_cast<gsrc>(p + (uint64_t)x.s * KTJ_WEAVE_LIT);
+            x.a = src[0];
+            if (len > 16u) { b = src[1]; if (len > 32u) { c = src[2]; if (len > 48u) d = src[3]; } }
+          }
+          /* waited for here, so that no wait of the loop is for the document's stores */
+          asm volatile("" : "+v"(x.a), "+v"(b), "+v"(c), "+v"(d));
+        }
+        const uint32_t n_num = x.valid ? x.num.w >> 24 : 0u;
+        x.num.w &= 0xFFFFFFu;
+        const uint32_t mine_len = x.valid ? len + n_num : 0u;
+        const uint32_t end = dpp_add(mine_len), all = __builtin_amdgcn_readlane(end, 63);
+        uint32_t gone = 0; /* bytes of these segments that are in the tile */
+        do {
+          uint32_t upto_byte = all;
+          bool now = x.valid && end - mine_len >= gone; /* (the others are there already) */
+          if (pend + (all - gone) > WV_TILE) { /* not all of them at once */
+            now = now && end + pend - gone <= WV_TILE;
+            const uint64_t these = __ballot(now);
+            if (these == 0) break; /* (a segment is shorter than the tile: never) */
+            upto_byte = __builtin_amdgcn_readlane(end, 63 - __builtin_clzll(these));
+          }
+          if (now) or_segment(tile, pend + (end - mine_len - gone), len, x.a, b, c, d, n_num, x.num);
+          pend += upto_byte - gone;
+          gone = upto_byte;
+          wave_lds_order();
+          /* whole lines leave */
+          const uint32_t nb = (pend >> 7) * 8u;
+          if (nb) {
+            const gptr dst = reinterpret_cast<gptr>((uintptr_t)doc);
+            v2u64* tb = reinterpret_cast<v2u64*>(tile);
+            const v2u64 zero = {0, 0};
+            /* (three turns reach the end of the tile; read first, all of them, then cleared) */
+            v2u64 y0, y1, y2, rest;
+            if (lane < nb) y0 = tb[lane];
+            if (lane + 64u < nb) y1 = tb[lane + 64u];
+            if (lane + 128u < nb) y2 = tb[lane + 128u];
+            if (lane < 8u) rest = tb[nb + lane];
+            if (lane < nb) tb[lane] = zero;
+            if (lane + 64u < nb) tb[lane + 64u] = zero;
+            if (lane + 128u < nb) tb[lane + 128u] = zero;
+            if (lane < 8u) { tb[nb + lane] = zero; tb[lane] = rest; }
+            if (lane < nb && lane >= own) dst[lane] = y0;
+            if (lane + 64u < nb) dst[lane + 64u] = y1;
+            if (lane + 128u < nb) dst[lane + 128u] = y2;
+            wave_lds_order();
+            doc += (uint64_t)nb * 16u;
+            pend &= 127u;
+            own = 0;
+          }
+        } while (gone < all);
+      };
+      Piece x = fetch(g, part), y;
+      for (;;) {
+        const bool two = g + 64u < g_end, three = g + 128u < g_end;
+        if (two) y = fetch(g + 64u, part);
+        put(x);
+        if (!two) break;
+        if (three) x = fetch(g + 128u, part);
+        put(y);
+        if (!three) break;
+        g += 128u;
+      }
+      if (next_lane != 64u && !(todo & (1ull << next_lane))) close_document(i0 + (next_lane >> 2));
+    }
+  }
+  if (open) close_document(i_end);
+}
+
+hipError_t weave_activities(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const uint8_t* kind_sorted, uint64_t n_most, EmitCtx ctx, char* out,
+                 uint64_t prefix_len, const Scalars* sc, const SchemaBook* schemas, hipStream_t st) {
+  if (n_most == 0) return hipSuccess;
+  static_assert(WV_TILE_ROOM / 16u <= 3u * 64u, "the tile leaves in three turns at most");
+  const uint64_t turns = (n_most + WV_ROWS - 1) / WV_ROWS;
+  const uint32_t waves = turns >= 256u * WV_WAVES ? WV_WAVES : turns <= 256u ? 1u : (uint32_t)((turns + 255u) / 256u);
+  const uint32_t rounds = turns >= 256u * 16u * 32u ? 16u : turns >= 256u * 16u * 4u ? 4u : turns > 256u * 16u ? 2u : 1u;
+  hipLaunchKernelGGL(k_weave, dim3(grid_for(turns, waves * rounds)), dim3(waves * 64u), WV_BOOK_BYTES + waves * WV_WAVE_BYTES, st, rows, perm, offs,
+                     kind_sorted, ctx, out, prefix_len, sc, rounds, schemas);
+  return KTJ_LAUNCH_CHECK();
+}
+
+}  // namespace gpu
+}  // namespace ktj

@@ -10,6 +10,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <map>
+#include <memory>
 #include <set>
 #include <string>
 #include <unordered_map>
@@ -18,6 +19,7 @@
 
 #include "../../kineto_amd/csrc/host_events.h"
 #include "../../kineto_amd/csrc/mat_core.h"
+#include "../../kineto_amd/csrc/weave_core.h"
 
 using namespace ktj;
 
@@ -59,9 +61,106 @@ void build_views(const ktj_stream* s, Views& v) {
   }
 }
 
+// The schemas' texts as the kernels lay them out (lay_out_schema and put_field_text do the work there too).
+void lay_out_schemas(const EmitCtx& c, weave::SchemaBook* book) {
+  memset(book, 0, sizeof *book);
+  const uint32_t n = std::min<uint32_t>(c.n_schemas, weave::MAX_SCHEMAS);
+  uint32_t fields = 0, desc = 0, units = 0;
+  for (uint32_t k = 0; k < n; ++k) {
+    const ktj_schema_desc sd = c.schemas[k];
+    const uint32_t first = fields;
+    fields = std::min(fields + std::min(sd.n_fields, KTJ_WEAVE_FIELDS), KTJ_WEAVE_FIELDS);
+    if (first + sd.n_fields > KTJ_WEAVE_FIELDS) continue;
+    const ktj_field* f = c.fields + sd.first_field;
+    std::vector<uint32_t> key_len(sd.n_fields + 1), place(sd.n_fields + 1, ~0u);
+    std::vector<std::string> key(sd.n_fields + 1);
+    for (uint32_t j = 0; j < sd.n_fields; ++j)
+      if (f[j].key_id != KTJ_NONE && f[j].key_id < c.dict.n) {
+        key[j].assign(c.dict.arg_blob + c.dict.arg_off[f[j].key_id], c.dict.arg_blob + c.dict.arg_off[f[j].key_id + 1]);
+        key_len[j] = (uint32_t)key[j].size();
+      }
+    const weave::SchemaSize size = weave::lay_out_schema(f, key_len.data(), sd.n_fields, 0, 0, &book->plan[k], nullptr, nullptr);
+    desc += size.desc; units += size.units;
+    if (desc > weave::SCHEMA_DESC || units > weave::SCHEMA_TEXT) { book->plan[k].what = 0; continue; }
+    if (!book->plan[k].what) continue;
+    weave::lay_out_schema(f, key_len.data(), sd.n_fields, desc - size.desc, units - size.units, &book->plan[k], book->desc, place.data());
+    for (uint32_t j = 0; j < sd.n_fields; ++j) weave::put_field_text(f[j], key[j].data(), key_len[j], place[j], reinterpret_cast<char*>(book->text));
+  }
+}
+// What the weaver prints for a row that is text, one segment after the other.
+std::string woven_text(const weave::TextRow& row, const EmitCtx& c, const weave::SchemaBook& book) {
+  using namespace weave;
+  const Book& b = BOOK;
+  std::string out;
+  auto number = [&](uint32_t slot) -> std::string {
+    const uint32_t* w = row.w[KTJ_TR_BLOCK(slot)];
+    if (slot == S_A) return std::string(reinterpret_cast<const char*>(w), w[1] >> 24);
+    return std::string(reinterpret_cast<const char*>(w), w[slot >= S_Z ? 2 : 3] >> 24);
+  };
+  const uint32_t plan = row.w[KTJ_TR_PLAN][3], lens = row.w[KTJ_TR_LENS][3], more = row.w[KTJ_TR_MORE][3], name = row.w[KTJ_TR_NAME][3];
+  uint64_t track;
+  memcpy(&track, &row.w[KTJ_TR_BLOCK(S_A)][2], 8);
+  const std::string pid = std::to_string(track & ((1u << KTJ_TR_DEV_BITS) - 1u));
+  const std::string tid = std::to_string((track >> KTJ_TR_DEV_BITS) | ((uint64_t)KTJ_TR_TID_HIGH(plan) << 42));
+  auto text = [&](uint32_t d) {
+    const uint32_t unit = KTJ_WD_UNIT(d);
+    const uint32_t* t = unit >= SCHEMA_UNIT ? book.text + (unit - SCHEMA_UNIT) * 4 : b.text + unit * 4;
+    return std::string(reinterpret_cast<const char*>(t), KTJ_WD_LEN(d));
+  };
+  std::string track_text[T_COUNT];
+  for (uint32_t k = 0; k < N_PIECES; ++k) {
+    const uint32_t d = b.desc[KTJ_WREF_BASE(b.ref[R_PIECES]) + k];
+    std::string& t = track_text[k < 9 ? k / 3 : k < 11 ? 3 : 4];
+    t += text(d);
+    if (KTJ_WD_SLOT(d) == S_PID) t += pid;
+    if (KTJ_WD_SLOT(d) == S_TID) t += tid;
+  }
+  for (const std::string& t : track_text) if (t.size() > KTJ_WEAVE_LIT) return "a track's text is longer than a segment";
+  auto part = [&](uint32_t ref) {
+    for (uint32_t k = 0; k < KTJ_WREF_COUNT(ref); ++k) {
+      const uint32_t i = KTJ_WREF_BASE(ref) + k;
+      const uint32_t d = i >= MAX_DESC ? book.desc[i - MAX_DESC] : b.desc[i];
+      bool patched = false;
+      for (uint32_t j = 0; j < b.n_patch; ++j) if ((b.patch[j] & 0xFFFFu) == i) { out += track_text[b.patch[j] >> 16]; patched = true; }
+      if (!patched) out += text(d);
+      const uint32_t slot = KTJ_WD_SLOT(d);
+      if (slot == S_K) for (uint32_t x = more; x; x >>= 8) out += (char)x;
+      else if (slot != S_NONE) out += number(slot);
+    }
+  };
+  part(b.ref[R_HEAD + KTJ_TR_TYPE(plan)]);
+  if (KTJ_TR_NAMED(plan) != KTJ_TR_NAME_RUN) part(b.ref[KTJ_TR_NAMED(plan)]);
+  else if (lens & 0xFFFFu) out.append(c.dict.name_blob + c.dict.name_off[name], lens & 0xFFFFu);
+  part(b.ref[R_BODY_NONE + KTJ_TR_BODY(plan)]);
+  const uint32_t a = KTJ_TR_ARGS(plan);
+  const SchemaPlan none{};
+  const SchemaPlan& s = a >= KTJ_TR_SCHEMA && a != KTJ_TR_NO_ARGS ? book.plan[a - KTJ_TR_SCHEMA] : none;
+  part(a >= KTJ_TR_SCHEMA ? s.args : b.ref[R_ARGS + a]);
+  switch (KTJ_TR_BETWEEN(plan)) {
+    case 1: out.append(c.dict.arg_blob + (more < c.dict.n ? c.dict.arg_off[more] : 0), lens >> 16); break;
+    case 2: out += std::string(reinterpret_cast<const char*>(row.w[KTJ_TR_BLOCK(S_Y)]), 16).append(reinterpret_cast<const char*>(row.w[KTJ_TR_BLOCK(S_Z)]), 8).substr(0, lens >> 16); break;
+    case 3: {
+      LongText t;
+      t.w[0] = t.w[1] = t.w[2] = t.w[3] = 0; t.n = 0;
+      put_f64(t, c.args[more]);
+      out.append(reinterpret_cast<const char*>(t.w), t.n);
+      break;
+    }
+    default: break;
+  }
+  part(a >= KTJ_TR_SCHEMA ? s.args2 : b.ref[R_ARGS2 + a]);
+  part(b.ref[R_TAIL + KTJ_TR_TAIL(plan)]);
+  return out;
+}
+uint64_t n_woven = 0, n_not_woven = 0;
+
 }  // namespace
 
 extern "C" {
+
+// activities of the last document rendered with KTJSIM_WOVEN that were text rows, and that were not
+void ktjsim_woven(uint64_t* woven, uint64_t* left) { *woven = n_woven; *left = n_not_woven; }
+#define KTJSIM_WOVEN 1u
 
 // Returns a malloc'ed buffer with the complete document.
 int ktjsim_render(const ktj_stream* s, uint32_t tile_bytes, char** out, uint64_t* out_n) {
@@ -328,6 +427,37 @@ int ktjsim_render(const ktj_stream* s, uint32_t tile_bytes, char** out, uint64_t
       format_activity(w, mat[perm[i]], ctx);
       if (w.position(buf) != P + offs[i + 1]) { free(buf); return -2; }
       w.end(i + 1 == perm.size());
+    }
+    *out = buf;
+    *out_n = total;
+    return 0;
+  }
+  if (tile_bytes == KTJSIM_WOVEN) {
+    // rows as text and what the weaver makes of them; those that are not text from format_activity
+    std::unique_ptr<weave::SchemaBook> book(new weave::SchemaBook);
+    lay_out_schemas(ctx, book.get());
+    n_woven = n_not_woven = 0;
+    for (size_t i = 0; i < perm.size(); ++i) {
+      const MatRow& m = mat[perm[i]];
+      weave::TextRow row;
+      memset(&row, 0xA5, sizeof row);
+      uint32_t len = 0, tail = 0;
+      char* at = buf + prefix.size() + offs[i];
+      if (weave::text_row(m, ctx, book->plan, &row, 0, &len, &tail)) {
+        if (len != offs[i + 1] - offs[i] || tail != tail_kind(m, has_args(m, ctx)) || row.w[7][3] >> 24 == KTJ_ROW_LEFT) { free(buf); return -4; }
+        const std::string t = woven_text(row, ctx, *book);
+        if (t.size() != len) { free(buf); return -5; }
+        memcpy(at, t.data(), len);
+        ++n_woven;
+      } else {
+        BlockWriter w;
+        std::vector<uint64_t> one(len / 8 + 8 + (offs[i + 1] - offs[i]) / 8);
+        w.begin(reinterpret_cast<char*>(one.data()), 0, 0, true);
+        format_activity(w, m, ctx);
+        w.end(true);
+        memcpy(at, one.data(), offs[i + 1] - offs[i]);
+        ++n_not_woven;
+      }
     }
     *out = buf;
     *out_n = total;

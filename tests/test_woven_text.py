@@ -1,0 +1,162 @@
+"""Activities put together from segments (weave_core.h, weave.hip): the rows' texts, lengths and tail kinds and the schemas'
+texts against the oracle's documents, on the CPU for every kind of row and at the edges of what a row has room for, and on the
+GPU at the edges of a turn, of the strings that wait in LDS and of the activities that are left to the other kernel."""
+import ctypes as C
+import os
+
+import pytest
+
+import oracle_glue as og
+from kineto_amd import abi
+from stream_builder import B, StreamBuilder
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+NAME_LENGTHS = (0, 1, 15, 16, 17, 63, 64, 65, 127, 128, 129, 257, 2600, 12800, 12801)
+PIDS = (0, 1, 4194303, 4194304, (1 << 31) - 1, -3)                       # 22 bits, and beyond
+TIDS = (0, 5, (1 << 42) - 1, 1 << 42, (1 << 47) - 1, 1 << 47, -5, (1 << 63) - 1)
+NUMBERS = (0, 9, 10, 99999999, 100000000, 10**10, 10**11 - 1, 10**11, 10**15 - 1, 10**15, (1 << 63) - 1, -1, -(10**9), -(10**10), -(1 << 63))
+
+
+def _text(n, salt=0):
+    return "".join(chr(97 + (k * 7 + salt) % 26) for k in range(n))
+
+
+def edge_stream(n):
+    """n activities: ordinary kernels and launches, and among them one after the other what a text row has just room for and what
+    it has not."""
+    b = StreamBuilder(window=(B, B + 10**13), host_name="edge")
+    b.api(["hipLaunchKernel", "hipMemcpyAsync", "hipMalloc", None, "hipFree"], flow_start=[0, 1], malloc_cid=2)
+    names = [b.s(_text(k, k)) for k in NAME_LENGTHS] + [b.s('"quoted"\\'), b.s("kernel"), b.s("Stream Sync")]
+    fields = [
+        [("Sequence number", abi.F_I64, 1)],
+        [("Trace name", abi.F_STR, 1)],
+        [("Value", abi.F_F64, 1)],
+        [(None, abi.F_RAW, 1)],
+        [("A", abi.F_I64, 1), ("B", abi.F_U64, 1), ("C", abi.F_BOOL, 1), ("D", abi.F_I64, 1)],
+        [("A", abi.F_I64, 1), ("B", abi.F_U64, 1), ("C", abi.F_BOOL, 1), ("D", abi.F_I64, 1), ("E", abi.F_I64, 1)],
+        [("grid", abi.F_I64_ARRAY, 3), ("block", abi.F_I64_ARRAY, 2), ("n", abi.F_U64, 1), ("m", abi.F_I64, 1)],
+        [("none", abi.F_I64_ARRAY, 0), ("one", abi.F_I64_ARRAY, 1)],
+        [("four", abi.F_I64_ARRAY, 4)],
+        [("d", abi.F_DICT_BEGIN, 0), ("x", abi.F_I64, 1), (None, abi.F_DICT_END, 0), ("s", abi.F_STR, 1), ("y", abi.F_I64, 1)],
+        [(_text(48), abi.F_I64, 1), (_text(40, 3), abi.F_STR, 1)],
+        [(_text(49), abi.F_I64, 1)],
+        [("s", abi.F_STR, 1), ("t", abi.F_STR, 1)],
+        [],
+    ]
+    schemas = [b.schema(f) for f in fields + [[("late %d" % k, abi.F_I64, 1)] for k in range(5)]]   # the last lie behind the sixteenth
+    fields += [[(None, abi.F_I64, 1)]] * 5
+
+    def number(k):
+        return NUMBERS[k % len(NUMBERS)]
+
+    def op_id(j):
+        return (j, -j, 2**31 - 1 - j, j - 2**31)[j % 4]
+
+    def rare(k, ts):
+        kind, j = k % 4, k // 4
+        if kind == 0:                                # generic
+            values = []
+            f = fields[j % len(fields)]
+            for i, (_key, typ, count) in enumerate(f):
+                if typ == abi.F_F64:
+                    values.append((0.5, 1e22, 123456.789, -2.2250738585072014e-308, float("inf"), float("nan"))[(j // 3 + i) % 6])
+                elif typ in (abi.F_STR, abi.F_RAW):
+                    values.append((names + [abi.KTJ_NONE - 1])[(j + i) % (len(names) + 1)])
+                elif typ == abi.F_BOOL:
+                    values.append(j & 1)
+                else:
+                    values += [number(j + i + c) if j & 1 else (j + c) % 1200000 for c in range(count)]
+            r = b.add_generic(None, (0, 1, 2, 10, 17, 9, 0, 0)[j % 8], ts, ts + (0, 999, 1000, 10**10 - 1, 10**10, -4)[j % 6], PIDS[j % 6], TIDS[j % 8] if j % 3 else 5,
+                              id=op_id(j), schema=schemas[j % len(fields)], values=values, flow_id=number(j) if j % 2 else 0, flow_type=1 + j % 2, flow_start=j % 4 < 2)
+            r.name_id = names[j % len(names)]
+        elif kind == 1:                              # launches
+            dim = ((1, 1, 1), (99999, 999, 999), (999999, 999, 999), (4294967295, 1, 1), (1, 999999, 1), (1, 1000000, 1))[j % 6]
+            r = b.add_runtime(number(j) & 0xFFFFFFFFFFFFFFFF if j % 2 else 1 << 20 | j, ts, ts + 1500, 0, 1, TIDS[j % 5], kind=1, grid=dim, workgroup=dim if j % 2 else (256, 1, 1),
+                              lds=(0, 4294967295)[j % 2], stream=j % 3)
+            r.u.kernel.kernel_name_id = (names + [abi.KTJ_NONE])[j % (len(names) + 1)]
+        elif kind == 2:                              # copies and allocations
+            size = (0, 10**11 - 1, 10**11, 1 << 40, 4096)[j % 5]
+            if j % 2:
+                b.add_runtime(1 << 21 | j, ts, ts + 999, 1, 1, 5, kind=2, src=(1 << 60) - 1 if j % 3 else 1 << 60, dst=j, size=size, copy_kind=(0, 4, -1, 9999, -1000)[j % 5])
+            else:
+                b.add_runtime(1 << 21 | j, ts, ts + 999, (2, 3, 4)[j % 3], 1, 5, kind=(3, 0)[j // 2 % 2], ptr=(0, 0x7F0000000000, (1 << 64) - 1)[j % 3], size=size)
+        else:                                        # device rows
+            domain, op = ((0, 0), (1, 2), (1, 4), (2, 0), (3, 0))[j % 5]
+            if domain == abi.KTJ_DOM_MEMSET:
+                b.add_memset(1 << 22 | j, ts, ts + (1, 0, 77)[j % 3], device=j % 2, context=(1, 9999999, 10000000)[j % 3], stream=j % 4, nbytes=number(j) & 0xFFFFFFFFFF,
+                             memory_kind=j % 10)
+            else:
+                b.add_device(number(j) & 0xFFFFFFFFFFFFFFFF if j % 2 else 1 << 20 | (j - 1), ts, ts + (0, 1, 12345678, 10**10)[j % 4], domain=domain, op=op, device=j % 3, name=None,
+                             queue=(1, 9999999, 10000000)[j % 3], nbytes=number(j) & 0xFFFFFFFFFFFF).name_id = names[j % len(names)]
+
+    for k in range(n):
+        ts = B + 1000 + 2001 * k
+        if k % 5 < 2:
+            if k % 2:
+                b.add_extcorr(k + 1, op_id(k // 40))
+            b.add_device(k + 1, ts, ts + 1234, device=0, name="gemm_%d" % (k % 7), queue=1 + k // 97 % 2)
+        elif k % 5 == 2:
+            b.add_runtime(k, ts, ts + 1234, 0, 1, 5, kind=1, grid=(k, 1, 1), workgroup=(256, 1, 1))
+        else:
+            rare(k // 5 * 2 + k % 5 - 3, ts)
+    return b.build()
+
+
+@pytest.fixture(scope="module")
+def sim():
+    lib = C.CDLL(os.path.join(ROOT, "tests", "host_sim", "libktjsim.so"))
+    lib.ktjsim_render.argtypes = [C.POINTER(abi.Stream), C.c_uint32, C.POINTER(C.c_void_p), C.POINTER(C.c_uint64)]
+    lib.ktjsim_free.argtypes = [C.c_void_p]
+    return lib
+
+
+def _woven_vs_oracle(sim, sp):
+    o = og.OracleRun(sp)
+    want = o.output()
+    o.close()
+    p, nb, woven, left = C.c_void_p(), C.c_uint64(), C.c_uint64(), C.c_uint64()
+    assert sim.ktjsim_render(sp, 1, C.byref(p), C.byref(nb)) == 0   # 1: from segments; it fails where a length or tail kind differs
+    sim.ktjsim_woven(C.byref(woven), C.byref(left))
+    got = C.string_at(p, nb.value)
+    sim.ktjsim_free(p)
+    if got != want:
+        i = next((k for k in range(min(len(got), len(want))) if got[k] != want[k]), min(len(got), len(want)))
+        raise AssertionError(f"byte {i}: got {got[max(0, i - 80):i + 60]!r} want {want[max(0, i - 80):i + 60]!r}")
+    return woven.value, left.value
+
+
+def test_segments_of_every_kind_of_row(sim):
+    import kat_cases
+    import random_streams
+    for cfg in range(1, 6):
+        sp, release = abi.synth_stream(cfg, 2000, host_name="box")
+        assert _woven_vs_oracle(sim, sp)[1] == 0, cfg        # ordinary records are text rows, all of them
+        release()
+    for case in kat_cases.SUBSTRING_CASES + [kat_cases.case_rocm_sync_trace]:
+        _woven_vs_oracle(sim, case()[0].build())
+    for seed in range(60):
+        _woven_vs_oracle(sim, random_streams.random_stream(seed, wide_ids=seed % 2 == 1).build())
+    woven, left = _woven_vs_oracle(sim, edge_stream(3000))
+    assert woven > 1800 and left > 300, (woven, left)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", (1, 3, 15, 16, 17, 40, 255, 257, 2053, 9001))
+def test_woven_documents_at_the_edges(n):
+    """Through the large passes whatever the size; the document twice from one engine, so that the second pass meets used buffers."""
+    from kineto_amd.engine import TraceEngine
+    lib = abi.load_engine()
+    sp = edge_stream(n)
+    o = og.OracleRun(sp)
+    want = o.output()
+    o.close()
+    lib.ktj_debug_force_sort_passes(1)
+    try:
+        e = TraceEngine(sp.contents.trace_name.decode())
+        e.submit_stream(sp)
+        for _ in range(2):
+            e.process()
+            assert e.output() == want
+        e.close()
+    finally:
+        lib.ktj_debug_force_sort_passes(0)
