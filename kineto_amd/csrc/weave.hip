@@ -12,12 +12,13 @@
  *
  * What bounds it: the LDS pipe (1.02 of 1.9 ms for 11 million kernels, a third of that bank conflicts) and the
  * vector units (0.9 ms) together with the waits between them; the bytes alone (1.4 GB of rows, 5.4 GB of document)
- * take 1.3 ms.  Measured against k_emit_direct: 10 000 x 3 records 38.7 -> 17.5 us, 4000 operators with long strings
- * 71 -> 35 us, 733 000 records 176 -> 153 us, 3 million 795 -> 490 us, 11 million kernels 2.06 -> 1.91 ms, 22 million
- * records 4.59 -> 3.80 ms, 5 million operators with long strings (1.4 KB each: strings beyond 128 bytes are fetched from
- * memory piece by piece) 3.20 -> 3.24 ms; the size pass has become 4 to 13 % longer for the numbers' text.
- * Of the places: 16 activities a turn (32 need more LDS than two workgroups of eight wavefronts have); 2688 bytes of
- * document, room for nearly all groups of 64 segments.
+ * take 1.3 ms.  Measured against k_emit_direct: 10 000 x 3 records 38.7 -> 16 us, 4000 operators with long strings
+ * 71 -> 34 us, 733 000 records 176 -> 142 us, 3 million 795 -> 465 us, 11 million kernels 2.06 -> 1.71 ms, 22 million
+ * records 4.59 -> 3.48 ms, 5 million operators with long strings (1.4 KB each: strings beyond 128 bytes are fetched from
+ * memory piece by piece) 3.20 -> 3.02 ms; the size pass has become 4 to 13 % longer for the numbers' text.
+ * Fewer wavefronts cost: three per SIMD 2.48 ms for the kernels, two 2.83.  Five (96 registers, 2048 bytes of tile, 512
+ * of names) gave 2.22, 2048 bytes being short of most groups of 64 segments; with the tile as it is 96 registers alone
+ * 1.97.  Workgroups of four wavefronts: eight, with the book in LDS twice per CU instead of four times, 1.74.
  */
 #include "gpu_common.h"
 #include "weave_core.h"
@@ -28,28 +29,27 @@ namespace gpu {
 using namespace weave;
 
 #define WV_ROWS 16u                                   /* activities at a time, four lanes to each */
-#define WV_WAVES 8u                                   /* wavefronts per workgroup, at most */
+#define WV_WAVES 4u                                   /* wavefronts per workgroup, at most */
 #define WV_PARTS (WV_ROWS * 7u)
-#define WV_VAL_BYTES (S_COUNT * 16u)                  /* an odd number of sixteens: the same slot of neighbours lies in other banks */
+#define WV_VAL_BYTES (S_RUN * 16u)                    /* S_A and the following; an odd number of sixteens: the same slot of neighbours lies in other banks */
+#define WV_VAL(slot) (((slot) - 1u) * 16u)
 #define WV_NAMES 1280u                                /* bytes of strings that wait in LDS */
 #define WV_NAME_MOST 128u
-#define WV_TILE 2688u                                 /* bytes of document that wait in LDS */
+#define WV_TILE 2944u                                 /* bytes of document that wait in LDS */
 #define WV_TILE_ROOM (WV_TILE + 128u)                 /* a line behind it, and what texts write beyond their end */
 /* of a wavefront: */
 #define WV_NAMES_AT (WV_ROWS * WV_VAL_BYTES)
-#define WV_DESC_AT (WV_NAMES_AT + WV_NAMES)
-#define WV_TRACK_AT (WV_DESC_AT + (MAX_DESC + SCHEMA_DESC) * 4u)
+#define WV_TRACK_AT (WV_NAMES_AT + WV_NAMES)
 #define WV_PARTS_AT (WV_TRACK_AT + T_COUNT * KTJ_WEAVE_LIT)
 #define WV_TILE_AT (WV_PARTS_AT + WV_PARTS * 4u + 32u)
 #define WV_WAVE_BYTES (WV_TILE_AT + WV_TILE_ROOM)
-/* of the workgroup, in front of them: the book up to its descriptors */
-#define WV_BOOK_REF (MAX_TEXT * 16u)
-#define WV_BOOK_PATCH (WV_BOOK_REF + R_COUNT * 4u)
-#define WV_BOOK_SCHEMA (SCHEMA_UNIT * 16u)            /* texts and plans of the schemas */
-#define WV_BOOK_PLANS (WV_BOOK_SCHEMA + SCHEMA_TEXT * 16u)
-#define WV_BOOK_BYTES (WV_BOOK_PLANS + MAX_SCHEMAS * (uint32_t)sizeof(SchemaPlan))
+/* of the workgroup, in front of them: the texts, the book's and the schemas'; the schemas' plans; where the parts are; descriptors */
+#define WV_BOOK_PLANS ((MAX_TEXT + SCHEMA_TEXT) * 16u)
+#define WV_BOOK_REF (WV_BOOK_PLANS + MAX_SCHEMAS * (uint32_t)sizeof(SchemaPlan))
+#define WV_BOOK_DESC (WV_BOOK_REF + R_COUNT * 4u)
+#define WV_BOOK_BYTES ((WV_BOOK_DESC + (MAX_DESC + SCHEMA_DESC) * 4u + 15u) / 16u * 16u)
 
-/* a part: first segment | kind << 15 (text, or the string of S_RUN0 or S_RUN1) | first descriptor << 17 | activity << 26 */
+/* a part: first segment | kind << 15 (text, or one of the strings of S_RUN) | first descriptor << 17 | activity << 26 */
 #define WV_PART_START(x) ((x) & 0x7FFFu)
 #define WV_PART_KIND(x) (((x) >> 15) & 3u)
 #define WV_PART_DESC(x) (((x) >> 17) & 0x1FFu)
@@ -107,23 +107,13 @@ __device__ __forceinline__ void or_segment(char* buf, uint32_t p, uint32_t len, 
   }
 }
 extern __shared__ __attribute__((aligned(16))) char wv_lds[];
-/* a double's text to the 32 bytes at `at`; its length.  Not inlined: it takes more registers than what surrounds it. */
-static __device__ __attribute__((noinline)) uint32_t double_text(uint64_t bits, uint32_t at) {
-  LongText t;
-  t.w[0] = t.w[1] = t.w[2] = t.w[3] = 0; t.n = 0;
-  put_f64(t, bits);
-  v2u64* v = reinterpret_cast<v2u64*>(wv_lds + at);
-  v[0] = (v2u64){t.w[0], t.w[1]};
-  v[1] = (v2u64){t.w[2], 0};
-  return t.n;
-}
-/* the track's texts and the descriptors that use them */
-__device__ __forceinline__ void make_track(char* lds, uint32_t mine, uint64_t dev, uint64_t thread) {
+/* the track's texts; their lengths, a byte each */
+__device__ __forceinline__ uint64_t make_track(char* lds, uint32_t mine, uint64_t dev, uint64_t thread) {
   const uint32_t lane = lane_id();
   char* const track = lds + mine + WV_TRACK_AT;
   if (lane < T_COUNT * 4u) *reinterpret_cast<uint4*>(track + lane * 16u) = make_uint4(0, 0, 0, 0);
   const Text pid = text_of(dev), tid = text_of(thread);
-  const uint32_t desc = lane < N_PIECES ? *reinterpret_cast<const uint32_t*>(lds + mine + WV_DESC_AT + (KTJ_WREF_BASE(g_book.ref[R_PIECES]) + lane) * 4u) : 0u;
+  const uint32_t desc = lane < N_PIECES ? *reinterpret_cast<const uint32_t*>(lds + WV_BOOK_DESC + (KTJ_WREF_BASE(g_book.ref[R_PIECES]) + lane) * 4u) : 0u;
   const uint32_t len = KTJ_WD_LEN(desc), slot = KTJ_WD_SLOT(desc), n_num = slot == S_PID ? pid.n : slot == S_TID ? tid.n : 0u;
   const v4u32 zero = {0, 0, 0, 0};
   v4u32 a = zero, b = zero, num = zero;
@@ -140,30 +130,24 @@ __device__ __forceinline__ void make_track(char* lds, uint32_t mine, uint64_t de
   const uint32_t start = which == 0 ? 0u : which == 1 ? e2 : which == 2 ? e5 : which == 3 ? e8 : e10;
   wave_lds_order();
   if (lane < N_PIECES) or_segment(track, which * KTJ_WEAVE_LIT + (end - len - n_num - start), len, a, b, zero, zero, n_num, num);
-  if (lane < g_book.n_patch) {
-    const uint32_t p = *reinterpret_cast<const uint32_t*>(lds + WV_BOOK_PATCH + lane * 4u), text = p >> 16;
-    const uint32_t n = text == 0 ? e2 : text == 1 ? e5 - e2 : text == 2 ? e8 - e5 : text == 3 ? e10 - e8 : e12 - e10;
-    uint32_t* d = reinterpret_cast<uint32_t*>(lds + mine + WV_DESC_AT + (p & 0xFFFFu) * 4u);
-    *d = KTJ_WD(n, KTJ_WD_SLOT(*d), text * (KTJ_WEAVE_LIT / 16u)) | KTJ_WD_TRACK;
-  }
+  return (uint64_t)(e2 | ((e5 - e2) << 8) | ((e8 - e5) << 16) | ((e10 - e8) << 24)) | ((uint64_t)(e12 - e10) << 32);
 }
 
 __global__ void __launch_bounds__(WV_WAVES * 64u) __attribute__((amdgpu_waves_per_eu(4)))
 k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const uint8_t* kind_sorted, EmitCtx ctx, char* out, uint64_t prefix_len,
         const Scalars* sc, uint32_t rounds, const SchemaBook* schemas) {
   const uint32_t lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  for (uint32_t k = threadIdx.x; k < (WV_BOOK_BYTES - WV_BOOK_SCHEMA) / 16u; k += blockDim.x)
-    reinterpret_cast<uint4*>(wv_lds + WV_BOOK_SCHEMA)[k] = reinterpret_cast<const uint4*>(schemas)[k];
-  for (uint32_t k = threadIdx.x; k < WV_BOOK_SCHEMA / 4u; k += blockDim.x) /* texts, parts and patches lie one behind the other */
-    reinterpret_cast<uint32_t*>(wv_lds)[k] = reinterpret_cast<const uint32_t*>(&g_book)[k];
+  static_assert(WV_BOOK_PLANS % 16u == 0 && sizeof(SchemaPlan) % 16u == 0, "in sixteens");
+  for (uint32_t k = threadIdx.x; k < MAX_TEXT; k += blockDim.x) reinterpret_cast<uint4*>(wv_lds)[k] = reinterpret_cast<const uint4*>(g_book.text)[k];
+  for (uint32_t k = threadIdx.x; k < (WV_BOOK_REF - MAX_TEXT * 16u) / 16u; k += blockDim.x) /* the schemas' texts and plans */
+    reinterpret_cast<uint4*>(wv_lds)[MAX_TEXT + k] = reinterpret_cast<const uint4*>(schemas)[k];
+  for (uint32_t k = threadIdx.x; k < R_COUNT + MAX_DESC + SCHEMA_DESC; k += blockDim.x)
+    reinterpret_cast<uint32_t*>(wv_lds + WV_BOOK_REF)[k] = k < R_COUNT ? g_book.ref[k] : k < R_COUNT + MAX_DESC ? g_book.desc[k - R_COUNT] : schemas->desc[k - R_COUNT - MAX_DESC];
   const uint32_t mine = WV_BOOK_BYTES + wave * WV_WAVE_BYTES; /* this wavefront's LDS */
   const uint32_t* const refs = reinterpret_cast<const uint32_t*>(wv_lds + WV_BOOK_REF);
   uint32_t* const parts = reinterpret_cast<uint32_t*>(wv_lds + mine + WV_PARTS_AT);
   char* const tile = wv_lds + mine + WV_TILE_AT;
   for (uint32_t k = lane; k < WV_TILE_ROOM / 16u; k += 64u) reinterpret_cast<uint4*>(tile)[k] = make_uint4(0, 0, 0, 0);
-  for (uint32_t k = lane; k < MAX_DESC + SCHEMA_DESC; k += 64u)
-    *reinterpret_cast<uint32_t*>(wv_lds + mine + WV_DESC_AT + k * 4u) = k < MAX_DESC ? g_book.desc[k] : schemas->desc[k - MAX_DESC];
-  if (lane < WV_ROWS) *reinterpret_cast<uint4*>(wv_lds + mine + lane * WV_VAL_BYTES) = make_uint4(0, 0, 0, 0); /* S_NONE */
   __syncthreads();
   const uint64_t n_rows = sc->emit_rows;
   typedef __attribute__((address_space(1))) v2u64* gptr;
@@ -173,6 +157,7 @@ k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const u
   v2u64* const vals = reinterpret_cast<v2u64*>(wv_lds + mine + act * WV_VAL_BYTES);
   uint64_t track_made = ~0ull; /* what the track's texts are made of */
   uint32_t track_made_high = ~0u;
+  uint64_t track_lens = 0;
   const uint64_t i_begin = ((uint64_t)blockIdx.x * (blockDim.x >> 6) + wave) * rounds * WV_ROWS;
   if (i_begin >= n_rows) return;
   const uint64_t i_end = i_begin + rounds * WV_ROWS < n_rows ? i_begin + rounds * WV_ROWS : n_rows;
@@ -238,20 +223,15 @@ k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const u
       new_track = __ballot(h == 0u && (track != before || KTJ_TR_TID_HIGH(plan) != before_high));
     }
     const v4u32 z = {q0.x, q0.y, q0.z & 0xFFFFFFu, q0.z & 0xFF000000u};
-    vals[S_Z + h] = __builtin_bit_cast(v2u64, z);
+    vals[S_Z - 1u + h] = __builtin_bit_cast(v2u64, z);
     {
       const v4u32 a = {q1.x, q1.y & 0xFFFFFFu, 0u, q1.y & 0xFF000000u}, x = h == 0u ? a : q1;
-      vals[S_A + h] = __builtin_bit_cast(v2u64, x);
+      vals[S_A - 1u + h] = __builtin_bit_cast(v2u64, x);
     }
     /* how many segments and parts, and the room for the name (the first lane) */
     uint32_t counts = 0, units = 0, args_ref = 0, args2_ref = 0;
-    uint32_t len0 = lens & 0xFFFFu, len1 = lens >> 16;
+    const uint32_t len0 = lens & 0xFFFFu, len1 = lens >> 16;
     if (h == 0u && mine_ok) {
-      if (KTJ_TR_ARGS(plan) == A_COPY) { /* a copy's kind, up to four characters */
-        const uint32_t n = (32u - (uint32_t)__clz((int)more) + 7u) >> 3;
-        vals[S_K] = (v2u64){more, (uint64_t)n << 56};
-      }
-      if (KTJ_TR_BETWEEN(plan) == 3u) len1 = double_text(ctx.args[more], mine + act * WV_VAL_BYTES + S_K * 16u);
       const uint32_t a = KTJ_TR_ARGS(plan);
       if (a >= KTJ_TR_SCHEMA) {
         if (a != KTJ_TR_NO_ARGS) {
@@ -266,12 +246,16 @@ k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const u
       const uint32_t args = KTJ_WREF_COUNT(args_ref), args2 = KTJ_WREF_COUNT(args2_ref);
       counts = ((2u + (name ? 1u : 0u) + (args ? 1u : 0u) + (runs ? 1u : 0u) + (args2 ? 1u : 0u) + (tail ? 1u : 0u)) << 16) |
                (head + name + body + args + runs + args2 + tail);
-      units = len0 <= WV_NAME_MOST ? (len0 + 15u) / 16u : 0u;
+      units = (len0 <= WV_NAME_MOST ? (len0 + 15u) / 16u : 0u) | (KTJ_TR_BETWEEN(plan) == 3u ? 2u << 16 : 0u);
     }
     const uint32_t upto = dpp_add(counts), before = upto - counts; /* of the first lane of each */
-    const uint32_t units_upto = dpp_add(units);
-    const bool near = units != 0 && units_upto <= WV_NAMES / 16u;
-    const uint32_t name_at = WV_NAMES_AT + (units_upto - units) * 16u;
+    /* the strings in LDS: doubles that are printed here, two units each, and names as far as there is room */
+    static_assert(WV_ROWS * 32u <= WV_NAMES, "the doubles have room");
+    const uint32_t units_upto = dpp_add(units), double_at = WV_NAMES_AT + ((units_upto - units) >> 16) * 16u;
+    const uint32_t name_upto = (units_upto & 0xFFFFu) + (__builtin_amdgcn_readlane(units_upto, 63) >> 16);
+    units &= 0xFFFFu;
+    const bool near = units != 0 && name_upto <= WV_NAMES / 16u;
+    const uint32_t name_at = WV_NAMES_AT + (name_upto - units) * 16u;
     v4u32 nx, ny;
     const uint32_t q_units = WV_QUAD(near ? units : 0u, 0), q_at = mine + WV_QUAD(name_at, 0);
     {
@@ -291,16 +275,21 @@ k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const u
       if (len1) { *w++ = seg | (2u << 15); seg += (len1 + KTJ_WEAVE_LIT - 1u) / KTJ_WEAVE_LIT; }
       put_part(args2_ref);
       put_part(refs[R_TAIL + KTJ_TR_TAIL(plan)]);
-      v2u64 z;
-      z.x = (uint64_t)(uintptr_t)ctx.dict.name_blob + (uint64_t)name_off * 16u;
-      z.y = len0 | ((uint64_t)(near ? name_at : 0u) << 32);
-      vals[S_RUN0] = z;
-      if (len1) {
-        const uint32_t what = KTJ_TR_BETWEEN(plan);
-        z.x = (uint64_t)(uintptr_t)ctx.dict.arg_blob + (uint64_t)more * 16u;
-        z.y = len1 | ((uint64_t)(what == 1u ? 0u : act * WV_VAL_BYTES + (what == 2u ? S_Y : S_K) * 16u) << 32);
-        vals[S_RUN1] = z;
+      const uint32_t between = KTJ_TR_BETWEEN(plan);
+      const uint32_t at = between < 2u ? 0u : between == 2u ? act * WV_VAL_BYTES + WV_VAL(S_Y) : double_at;
+      if (between == 3u) {
+        LongText t;
+        t.w[0] = t.w[1] = t.w[2] = t.w[3] = 0; t.n = 0;
+        put_f64(t, ctx.args[more]);
+        v2u64* const v = reinterpret_cast<v2u64*>(wv_lds + mine + double_at);
+        v[0] = (v2u64){t.w[0], t.w[1]};
+        v[1] = (v2u64){t.w[2], 0};
       }
+      v4u32 runs;
+      runs.x = more; runs.y = len1 | (at << 16);
+      if (KTJ_TR_ARGS(plan) == A_COPY) runs.y = ((32u - (uint32_t)__clz((int)more) + 7u) >> 3) << 24; /* of the kind's characters, up to four */
+      runs.z = name_off; runs.w = len0 | ((near ? name_at : 0u) << 16);
+      vals[S_RUN - 1u] = __builtin_bit_cast(v2u64, runs);
     }
     const uint32_t totals = __builtin_amdgcn_readlane(upto, 63);
     if (lane == 0) parts[totals >> 16] = totals & 0x7FFFu;
@@ -331,7 +320,7 @@ k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const u
         const uint32_t low = __builtin_amdgcn_readlane((uint32_t)track, first), high = __builtin_amdgcn_readlane((uint32_t)(track >> 32), first);
         track_made_high = KTJ_TR_TID_HIGH(__builtin_amdgcn_readlane(plan, first));
         track_made = (uint64_t)low | ((uint64_t)high << 32);
-        make_track(wv_lds, mine, low & ((1u << KTJ_TR_DEV_BITS) - 1u), (track_made >> KTJ_TR_DEV_BITS) | ((uint64_t)track_made_high << 42));
+        track_lens = make_track(wv_lds, mine, low & ((1u << KTJ_TR_DEV_BITS) - 1u), (track_made >> KTJ_TR_DEV_BITS) | ((uint64_t)track_made_high << 42));
         track_seen = upto_first;
       }
       if (!open) {
@@ -357,36 +346,83 @@ k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const u
       }
       wave_lds_order();
       /* 64 segments at a time: what the next ones are made of is read before these are put together */
-      struct Piece { v4u32 a, num; uint32_t desc, at, pr, s; bool valid; };
-      auto fetch = [&](uint32_t g, uint32_t& part) {
+      struct Piece { v4u32 a, num; uint32_t desc, at, part; }; /* at: in LDS; WV_FAR: place in the string's blob, in units of sixteen bytes */
+#define WV_FAR (1u << 30)
+#define WV_FAR_ARG (1u << 31)
+      uint32_t part_after = 0;
+      auto fetch = [&]() {
         Piece x;
         /* which part each segment belongs to: a part's first segment is marked, the marks counted */
         const uint32_t rel = WV_PART_START(parts[part + lane]) - g; /* (behind the last part: what lies there, which does not count) */
         const bool inside = part + lane <= (totals >> 16) && rel - 1u < 64u;
         const uint64_t marks = __ballot(__builtin_amdgcn_ds_permute((int)(inside && rel < 64u ? rel * 4u : 0u), 1) != 0);
         const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(marks >> 33), __builtin_amdgcn_mbcnt_lo((uint32_t)(marks >> 1), 0u));
-        x.pr = parts[part + rank];
-        part += (uint32_t)__popcll(__ballot(inside && rel <= g_end - g)); /* (the next activities' are theirs) */
-        x.valid = g + lane < g_end;
-        x.s = g + lane - WV_PART_START(x.pr);
-        if (!x.valid) x.pr = 0;
-        const uint32_t kind = WV_PART_KIND(x.pr), vrow = mine + WV_PART_ACT(x.pr) * WV_VAL_BYTES;
-        const uint32_t idx = kind == 0 && x.valid ? WV_PART_DESC(x.pr) + x.s : 0u;
-        x.desc = *reinterpret_cast<const uint32_t*>(wv_lds + mine + WV_DESC_AT + idx * 4u);
-        x.at = KTJ_WD_UNIT(x.desc) * 16u + (x.desc & KTJ_WD_TRACK ? mine + WV_TRACK_AT : 0u);
-        if (kind != 0) {
-          const uint64_t r = *reinterpret_cast<const uint64_t*>(wv_lds + vrow + S_RUN0 * 16u + (kind - 1u) * 16u + 8u);
-          const uint32_t rest = (uint32_t)r - x.s * KTJ_WEAVE_LIT, near = (uint32_t)(r >> 32);
-          x.at = near ? mine + near + x.s * KTJ_WEAVE_LIT : ~0u;
-          x.desc = KTJ_WD(rest < KTJ_WEAVE_LIT ? rest : KTJ_WEAVE_LIT, S_NONE, 0u);
+        x.part = part + rank;
+        uint32_t pr = parts[x.part];
+        part_after = part + (uint32_t)__popcll(__ballot(inside && rel <= g_end - g)); /* (the next activities' are theirs) */
+        const bool valid = g + lane < g_end;
+        const uint32_t seg = g + lane - WV_PART_START(pr);
+        if (!valid) pr = 0;
+        const uint32_t kind = WV_PART_KIND(pr), vrow = mine + WV_PART_ACT(pr) * WV_VAL_BYTES;
+        const uint32_t idx = kind == 0 && valid ? WV_PART_DESC(pr) + seg : 0u;
+        x.desc = *reinterpret_cast<const uint32_t*>(wv_lds + WV_BOOK_DESC + idx * 4u);
+        x.at = KTJ_WD_UNIT(x.desc) * 16u;
+        if (x.desc & KTJ_WD_TRACK) {
+          x.desc |= (uint32_t)(track_lens >> (KTJ_WD_UNIT(x.desc) * 2u)) & 0x7Fu; /* (four units to a text) */
+          x.at += mine + WV_TRACK_AT;
         }
-        x.a = *reinterpret_cast<const v4u32*>(wv_lds + (x.at != ~0u ? x.at : 0u));
-        x.num = *reinterpret_cast<const v4u32*>(wv_lds + vrow + KTJ_WD_SLOT(x.desc) * 16u);
+        if (kind != 0) {
+          const uint64_t r = *reinterpret_cast<const uint64_t*>(wv_lds + vrow + WV_VAL(S_RUN) + (2u - kind) * 8u);
+          const uint32_t rest = ((uint32_t)(r >> 32) & 0xFFFFu) - seg * KTJ_WEAVE_LIT, near = (uint32_t)(r >> 48);
+          x.at = near ? mine + near + seg * KTJ_WEAVE_LIT : (uint32_t)r + seg * (KTJ_WEAVE_LIT / 16u);
+          x.desc = KTJ_WD(rest < KTJ_WEAVE_LIT ? rest : KTJ_WEAVE_LIT, S_NONE, 0u) | (near ? 0u : kind == 1u ? WV_FAR : WV_FAR | WV_FAR_ARG);
+        }
+        x.a = *reinterpret_cast<const v4u32*>(wv_lds + (x.desc & WV_FAR ? 0u : x.at));
+        const uint32_t slot = KTJ_WD_SLOT(x.desc);
+        x.num = *reinterpret_cast<const v4u32*>(wv_lds + vrow + (slot == S_K ? WV_VAL(S_RUN) : WV_VAL(slot))); /* (S_NONE: what lies there, which does not count) */
+        if (slot == S_K) { x.num.w = x.num.y; x.num.y = 0; x.num.z = 0; }
+        if (slot == S_NONE) x.num.w = 0;
         return x;
       };
+      uint32_t nb = 0;
+      v2u64 y0, y1, y2, rest;
+      /* The tile's whole lines are taken out of it and leave.  Between the two the next segments are fetched, so that neither
+       * waits for the other's LDS accesses (the segments after next fetched instead, twelve registers more: the same). */
+      auto take_lines = [&]() {
+        nb = (pend >> 7) * 8u;
+        if (nb) {
+          v2u64* tb = reinterpret_cast<v2u64*>(tile);
+          const v2u64 zero = {0, 0};
+          /* (three turns reach the end of the tile; read first, all of them, then cleared) */
+          if (lane < nb) y0 = tb[lane];
+          if (lane + 64u < nb) y1 = tb[lane + 64u];
+          if (lane + 128u < nb) y2 = tb[lane + 128u];
+          if (lane < 8u) rest = tb[nb + lane];
+          if (lane < nb) tb[lane] = zero;
+          if (lane + 64u < nb) tb[lane + 64u] = zero;
+          if (lane + 128u < nb) tb[lane + 128u] = zero;
+          if (lane < 8u) tb[nb + lane] = zero;
+        }
+      };
+      auto store_lines = [&]() {
+        if (nb) {
+          const gptr dst = reinterpret_cast<gptr>((uintptr_t)doc);
+          if (lane < 8u) reinterpret_cast<v2u64*>(tile)[lane] = rest;
+          if (lane < nb && lane >= own) dst[lane] = y0;
+          if (lane + 64u < nb) dst[lane + 64u] = y1;
+          if (lane + 128u < nb) dst[lane + 128u] = y2;
+          wave_lds_order();
+          doc += (uint64_t)nb * 16u;
+          pend &= 127u;
+          own = 0;
+          nb = 0;
+        }
+      };
+      /* As many of them as the tile has room for; the others are fetched again.  (All of them, in two turns over the tile:
+       * 5 % more for 11 million kernels.) */
       auto put = [&](Piece& x) {
         const uint32_t len = KTJ_WD_LEN(x.desc);
-        const bool far = x.at == ~0u;
+        const bool far = (x.desc & WV_FAR) != 0;
         v4u32 b = {0, 0, 0, 0}, c = b, d = b;
         if (len > 16u && !far) {
           b = *reinterpret_cast<const v4u32*>(wv_lds + x.at + 16u);
@@ -397,69 +433,33 @@ k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const u
         }
         if (__any(far)) {
           if (far) {
-            const uint64_t p = *reinterpret_cast<const uint64_t*>(wv_lds + mine + WV_PART_ACT(x.pr) * WV_VAL_BYTES + (S_RUN0 - 1u + WV_PART_KIND(x.pr)) * 16u);
-            const gsrc src = reinterpret_cast<gsrc>(p + (uint64_t)x.s * KTJ_WEAVE_LIT);
+            const gsrc src = reinterpret_cast<gsrc>((uint64_t)(uintptr_t)(x.desc & WV_FAR_ARG ? ctx.dict.arg_blob : ctx.dict.name_blob)) + x.at;
             x.a = src[0];
             if (len > 16u) { b = src[1]; if (len > 32u) { c = src[2]; if (len > 48u) d = src[3]; } }
           }
           /* waited for here, so that no wait of the loop is for the document's stores */
           asm volatile("" : "+v"(x.a), "+v"(b), "+v"(c), "+v"(d));
         }
-        const uint32_t n_num = x.valid ? x.num.w >> 24 : 0u;
+        const uint32_t n_num = x.num.w >> 24;
         x.num.w &= 0xFFFFFFu;
-        const uint32_t mine_len = x.valid ? len + n_num : 0u;
-        const uint32_t end = dpp_add(mine_len), all = __builtin_amdgcn_readlane(end, 63);
-        uint32_t gone = 0; /* bytes of these segments that are in the tile */
-        do {
-          uint32_t upto_byte = all;
-          bool now = x.valid && end - mine_len >= gone; /* (the others are there already) */
-          if (pend + (all - gone) > WV_TILE) { /* not all of them at once */
-            now = now && end + pend - gone <= WV_TILE;
-            const uint64_t these = __ballot(now);
-            if (these == 0) break; /* (a segment is shorter than the tile: never) */
-            upto_byte = __builtin_amdgcn_readlane(end, 63 - __builtin_clzll(these));
-          }
-          if (now) or_segment(tile, pend + (end - mine_len - gone), len, x.a, b, c, d, n_num, x.num);
-          pend += upto_byte - gone;
-          gone = upto_byte;
-          wave_lds_order();
-          /* whole lines leave */
-          const uint32_t nb = (pend >> 7) * 8u;
-          if (nb) {
-            const gptr dst = reinterpret_cast<gptr>((uintptr_t)doc);
-            v2u64* tb = reinterpret_cast<v2u64*>(tile);
-            const v2u64 zero = {0, 0};
-            /* (three turns reach the end of the tile; read first, all of them, then cleared) */
-            v2u64 y0, y1, y2, rest;
-            if (lane < nb) y0 = tb[lane];
-            if (lane + 64u < nb) y1 = tb[lane + 64u];
-            if (lane + 128u < nb) y2 = tb[lane + 128u];
-            if (lane < 8u) rest = tb[nb + lane];
-            if (lane < nb) tb[lane] = zero;
-            if (lane + 64u < nb) tb[lane + 64u] = zero;
-            if (lane + 128u < nb) tb[lane + 128u] = zero;
-            if (lane < 8u) { tb[nb + lane] = zero; tb[lane] = rest; }
-            if (lane < nb && lane >= own) dst[lane] = y0;
-            if (lane + 64u < nb) dst[lane + 64u] = y1;
-            if (lane + 128u < nb) dst[lane + 128u] = y2;
-            wave_lds_order();
-            doc += (uint64_t)nb * 16u;
-            pend &= 127u;
-            own = 0;
-          }
-        } while (gone < all);
+        const bool valid = g + lane < g_end;
+        const uint32_t mine_len = valid ? len + n_num : 0u;
+        const uint32_t end = dpp_add(mine_len);
+        const bool now = valid && end + pend <= WV_TILE;
+        const uint32_t n = (uint32_t)__popcll(__ballot(now)); /* (never 0: a segment is shorter than the tile) */
+        if (now) or_segment(tile, pend + (end - mine_len), len, x.a, b, c, d, n_num, x.num);
+        pend += __builtin_amdgcn_readlane(end, n - 1u);
+        wave_lds_order();
+        take_lines();
+        part = n == 64u ? part_after : __builtin_amdgcn_readlane(x.part, n);
+        g += n;
       };
-      Piece x = fetch(g, part), y;
-      for (;;) {
-        const bool two = g + 64u < g_end, three = g + 128u < g_end;
-        if (two) y = fetch(g + 64u, part);
+      while (g < g_end) {
+        Piece x = fetch();
+        store_lines();
         put(x);
-        if (!two) break;
-        if (three) x = fetch(g + 128u, part);
-        put(y);
-        if (!three) break;
-        g += 128u;
       }
+      store_lines();
       if (next_lane != 64u && !(todo & (1ull << next_lane))) close_document(i0 + (next_lane >> 2));
     }
   }

@@ -25,14 +25,13 @@ enum : uint32_t {
   S_NONE = 0,
   S_A,                             /* cid, or queue, or context */
   S_TS,
-  S_X, S_Y,                        /* grid and block ("a, b, c"), addresses, or bytes; a device row's double: S_Y and S_Z */
+  S_X, S_Y,                        /* grid and block ("a, b, c"), addresses, or bytes; a double of up to 24 characters: S_Y and S_Z */
   S_Z,                             /* shared memory or bytes */
   S_EXT,                           /* with the comma behind it where something follows */
   S_FLOW, S_DUR,
-  S_K,                             /* copy kind; or a generic record's double of up to 24 characters, which takes */
-  S_K2,                            /* this one too */
-  S_RUN0, S_RUN1,                  /* strings: address, length, place in LDS (0: they stay where they are) */
-  S_COUNT,
+  S_RUN,                           /* the strings between the args and of the name, eight bytes each: place in the blob in units of sixteen bytes,
+                                      length, place in LDS (0: it stays in the blob) */
+  S_K,                             /* copy kind, in place of the first of them */
   S_PID = S_TS, S_TID = S_DUR      /* in the pieces of the track's texts */
 };
 
@@ -46,7 +45,7 @@ struct alignas(16) TextRow { uint32_t w[8][4]; };
 #define KTJ_TR_PLAN 0u             /* KTJ_TR_*, the thread's bits from 42 on */
 #define KTJ_TR_NAME 1u             /* place of the name in its blob, in units of sixteen bytes */
 #define KTJ_TR_LENS 2u             /* its length; << 16: that of the string or double between the args' parts */
-#define KTJ_TR_MORE 3u             /* the string's place in its blob; a generic record's double: its argument slot; a copy's kind as text */
+#define KTJ_TR_MORE 3u             /* the string's place in its blob; the double's place among the arguments; a copy's kind as text */
 static_assert(sizeof(TextRow) == 128 && sizeof(TextRow) >= sizeof(MatRow), "a row that is left to format_activity is a MatRow in the same place");
 /* a row of the other kind: the last byte, S_Y's count of characters otherwise */
 #define KTJ_ROW_LEFT 0xFFu
@@ -58,7 +57,7 @@ static_assert(sizeof(TextRow) == 128 && sizeof(TextRow) >= sizeof(MatRow), "a ro
 #define KTJ_TR_SCHEMA 64u
 #define KTJ_TR_NO_ARGS 127u
 #define KTJ_TR_TAIL(x) (((x) >> 21) & 15u)     /* R_TAIL and the following */
-#define KTJ_TR_BETWEEN(x) (((x) >> 25) & 3u)   /* 1 string, 2 double in S_Y, 3 double of a generic record */
+#define KTJ_TR_BETWEEN(x) (((x) >> 25) & 3u)   /* 1 string, 2 double in S_Y and S_Z, 3 double that the weaver prints */
 #define KTJ_TR_TID_HIGH(x) ((x) >> 27)
 #define KTJ_TR_DEV_BITS 22u                    /* a track's process or device, and 42 of the thread's or stream's 47 bits */
 
@@ -73,7 +72,7 @@ enum : uint32_t { T_BODY = 0, T_FLOW, T_DEVICE, T_MEMSET, T_STREAM, T_COUNT };
 #define KTJ_WD_LEN(x) ((x) & 0x7Fu)
 #define KTJ_WD_SLOT(x) (((x) >> 8) & 0xFu)
 #define KTJ_WD_UNIT(x) (((x) >> 12) & 0xFFFu)
-#define KTJ_WD_TRACK (1u << 24)
+#define KTJ_WD_TRACK (1u << 24)    /* (the length is the wavefront's) */
 
 /* An activity is: head by its category, name, body up to the args, the args (one part, or two around a string or a
  * double), and the end with its flow event. */
@@ -103,13 +102,13 @@ enum : uint32_t {
 /* The args of generic records follow their schema: descriptors and texts for the first schemas of a trace are made on the
  * device (render_schemas), behind the fixed ones.  A schema takes up to four numbers (two of them may be arrays of up to
  * three), and one string or one double. */
-constexpr uint32_t MAX_DESC = 208, MAX_TEXT = 232, MAX_PATCH = 40, N_PIECES = 13;
+constexpr uint32_t MAX_DESC = 208, MAX_TEXT = 232, N_PIECES = 13;
 constexpr uint32_t MAX_SCHEMAS = 16, SCHEMA_DESC = 56, SCHEMA_TEXT = 60;
 enum : uint32_t { I_NONE = 0, I_I64, I_U64, I_BOOL, I_ARRAY }; /* I_ARRAY + number of elements */
 struct SchemaPlan {
   uint32_t args, args2;            /* parts (0: the schema is none of these) */
   uint32_t what;                   /* 1: taken, 2: prints something, 4: one string and nothing else, which may be blank; << 8: argument
-                                      slots; << 16: between the parts, 1 a string, 2 a double; << 24: its slot */
+                                      slots; << 16: KTJ_TR_BETWEEN; << 24: its slot */
   uint32_t item[4];                /* of item_slot(0..3): I_* | slot << 8 */
   uint32_t chars;                  /* of the parts' texts */
 };
@@ -122,13 +121,12 @@ struct SchemaBook {
 struct Book {
   uint32_t text[MAX_TEXT * 4];
   uint32_t ref[R_COUNT];
-  uint32_t patch[MAX_PATCH];       /* descriptors whose text is the track's: index | text << 16 */
   uint32_t desc[MAX_DESC];
-  uint32_t n_desc, n_text, n_patch;
+  uint32_t n_desc, n_text;
 };
 
-/* In the weaver's LDS the schemas' texts lie behind the book's texts, parts and patches: unit of the first of them. */
-constexpr uint32_t SCHEMA_UNIT = MAX_TEXT + (R_COUNT * 4 + MAX_PATCH * 4 + 15) / 16;
+/* In the weaver's LDS the schemas' texts lie behind the book's texts: unit of the first of them. */
+constexpr uint32_t SCHEMA_UNIT = MAX_TEXT;
 
 /* In the texts byte 1 and a letter is a number, which ends a segment; byte 2 and a letter is a text of the track's. */
 #define WN(c) "\x01" c
@@ -140,8 +138,7 @@ struct Builder {
   constexpr void begin() { at = b.n_desc; n = 0; track = T_COUNT; }
   constexpr void segment(uint32_t slot) {
     if (track != T_COUNT) { /* its text is put in by the wavefront */
-      b.patch[b.n_patch++] = b.n_desc | (track << 16);
-      b.desc[b.n_desc++] = KTJ_WD(0u, slot, 0u);
+      b.desc[b.n_desc++] = KTJ_WD(0u, slot, track * (KTJ_WEAVE_LIT / 16u)) | KTJ_WD_TRACK;
       track = T_COUNT;
       return;
     }
@@ -164,7 +161,7 @@ struct Builder {
   constexpr void flush() { if (n) segment(S_NONE); }
   constexpr void number(char c) {
     const char* const codes = "auxyzefrk"; /* S_A and the following */
-    for (uint32_t k = 0; codes[k]; ++k) if (codes[k] == c) segment(S_A + k);
+    for (uint32_t k = 0; codes[k]; ++k) if (codes[k] == c) segment(c == 'k' ? S_K : S_A + k);
   }
   constexpr void add(const char* s) {
     for (; *s; ++s) {
@@ -261,7 +258,7 @@ constexpr Chars count_chars(const Book& b) {
     for (uint32_t k = 0; k < KTJ_WREF_COUNT(b.ref[r]); ++k) {
       const uint32_t i = KTJ_WREF_BASE(b.ref[r]) + k;
       c.of[r] += KTJ_WD_LEN(b.desc[i]);
-      for (uint32_t j = 0; j < b.n_patch; ++j) if ((b.patch[j] & 0xFFFFu) == i) c.of[r] += track[b.patch[j] >> 16];
+      if (b.desc[i] & KTJ_WD_TRACK) c.of[r] += track[KTJ_WD_UNIT(b.desc[i]) / (KTJ_WEAVE_LIT / 16u)];
     }
   return c;
 }
@@ -308,8 +305,16 @@ KTJ_HD inline SchemaSize lay_out_schema(const ktj_field* field, const uint32_t* 
     p.item[j] = what | (slot << 8);
     end(item_slot(j));
   };
-  for (uint32_t f = 0; f < n_fields; ++f) arrays += field[f].type == KTJ_F_I64_ARRAY && field[f].count != 0 ? 1u : 0u;
+  uint32_t numbers = 0;
+  bool real = false;
+  for (uint32_t f = 0; f < n_fields; ++f) {
+    const uint32_t type = field[f].type;
+    arrays += type == KTJ_F_I64_ARRAY && field[f].count != 0 ? 1u : 0u;
+    numbers += type == KTJ_F_I64 || type == KTJ_F_U64 || type == KTJ_F_BOOL ? 1u : 0u;
+    real = real || type == KTJ_F_F64;
+  }
   if (arrays > 2u) taken = false;
+  real = real && arrays + numbers <= 2u && arrays <= 1u; /* a double takes S_Y and S_Z where the others leave them */
   for (uint32_t f = 0; taken && f < n_fields; ++f) {
     const ktj_field fd = field[f];
     const bool key = fd.key_id != KTJ_NONE, commas = key && comma;
@@ -321,8 +326,8 @@ KTJ_HD inline SchemaSize lay_out_schema(const ktj_field* field, const uint32_t* 
     }
     /* a place for a number: S_Z, what the arrays leave of S_X and S_Y, S_A */
     auto simple = [&](uint32_t what) {
-      const uint32_t left = 2u - arrays, i = n_simple++;
-      number(i == 0 ? 2u : i <= left ? arrays + i - 1u : i == left + 1u ? 3u : 4u, what);
+      const uint32_t left = (real ? 1u : 2u) - arrays, i = n_simple++, k = real ? i + 1u : i;
+      number(k == 0 ? 2u : k <= left ? arrays + k - 1u : k == left + 1u ? 3u : 4u, what);
     };
     switch (fd.type) {
       case KTJ_F_DICT_BEGIN: chars(1); comma = false; break;
@@ -342,7 +347,7 @@ KTJ_HD inline SchemaSize lay_out_schema(const ktj_field* field, const uint32_t* 
         if (fd.type == KTJ_F_STR) chars(1);
         if (fd.type == KTJ_F_RAW && !key && n_fields == 1u) p.what |= 4u;
         if (len) end(S_NONE);
-        between = fd.type == KTJ_F_F64 ? 2u : 1u; between_slot = slot;
+        between = fd.type != KTJ_F_F64 ? 1u : real ? 2u : 3u; between_slot = slot;
         p.args = KTJ_WREF(MAX_DESC + d_at + d_args, n_desc - d_args);
         d_args = n_desc;
         at |= here() << 16;
@@ -510,6 +515,14 @@ KTJ_HD KTJ_FI inline bool text_row(const MatRow& m, const EmitCtx& c, const Sche
     return id;
 #endif
   };
+  auto real = [&](uint64_t bits) KTJ_FI { /* a double */
+    LongText t;
+    t.w[0] = t.w[1] = t.w[2] = t.w[3] = 0; t.n = 0;
+    put_f64(t, bits);
+    two(block(S_Y), t.w[0]); two(block(S_Y) + 2, t.w[1]);
+    two(block(S_Z), t.w[2]); block(S_Z)[2] = 0;
+    return t.n;
+  };
   block(S_Y)[3] = 0; /* (its last byte is not KTJ_ROW_LEFT) */
   uint32_t n = 0; /* the length, but for the strings */
   /* the name */
@@ -555,14 +568,12 @@ KTJ_HD KTJ_FI inline bool text_row(const MatRow& m, const EmitCtx& c, const Sche
         }
         between = (s.what >> 16) & 3u;
         if (between == 1u) at_more = string((uint32_t)c.args[m.p[0] + (s.what >> 24)], false, &len1);
-        else if (between == 2u) {
+        else if (between) {
           const uint64_t at = m.p[0] + (s.what >> 24);
           if (at >> 32) return false;
           at_more = (uint32_t)at;
-          between = 3u;
-          CountWriter w;
-          put_f64(w, c.args[at]);
-          n += (uint32_t)w.n;
+          if (between == 2u) len1 = real(c.args[at]);
+          else { CountWriter w; put_f64(w, c.args[at]); len1 = (uint32_t)w.n; }
         }
       }
     }
@@ -611,12 +622,7 @@ KTJ_HD KTJ_FI inline bool text_row(const MatRow& m, const EmitCtx& c, const Sche
       if (bandwidth) {
         const double d = (double)m.p[0] / (memset_row ? (double)m.dur : (double)((uint64_t)m.dur + 1u));
         uint64_t bits; __builtin_memcpy(&bits, &d, 8);
-        LongText t;
-        t.w[0] = t.w[1] = t.w[2] = t.w[3] = 0; t.n = 0;
-        put_f64(t, bits);
-        between = 2u; len1 = t.n;
-        two(block(S_Y), t.w[0]); two(block(S_Y) + 2, t.w[1]);
-        two(block(S_Z), t.w[2]); block(S_Z)[2] = 0;
+        between = 2u; len1 = real(bits);
       }
     }
     n += chars_table.of[R_ARGS + args] + chars_table.of[R_ARGS2 + args];

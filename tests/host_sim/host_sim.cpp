@@ -120,9 +120,7 @@ std::string woven_text(const weave::TextRow& row, const EmitCtx& c, const weave:
     for (uint32_t k = 0; k < KTJ_WREF_COUNT(ref); ++k) {
       const uint32_t i = KTJ_WREF_BASE(ref) + k;
       const uint32_t d = i >= MAX_DESC ? book.desc[i - MAX_DESC] : b.desc[i];
-      bool patched = false;
-      for (uint32_t j = 0; j < b.n_patch; ++j) if ((b.patch[j] & 0xFFFFu) == i) { out += track_text[b.patch[j] >> 16]; patched = true; }
-      if (!patched) out += text(d);
+      out += d & KTJ_WD_TRACK ? track_text[KTJ_WD_UNIT(d) / (KTJ_WEAVE_LIT / 16u)] : text(d);
       const uint32_t slot = KTJ_WD_SLOT(d);
       if (slot == S_K) for (uint32_t x = more; x; x >>= 8) out += (char)x;
       else if (slot != S_NONE) out += number(slot);
