@@ -126,51 +126,44 @@ __global__ void __launch_bounds__(KTJ_BLOCK) __attribute__((amdgpu_waves_per_eu(
 k_emit_direct(const char* rows, const uint32_t* perm, const uint64_t* offs, const uint8_t* kind_sorted,
               EmitCtx ctx, char* out, uint64_t prefix_len, const Scalars* sc, const uint32_t* left) {
   const uint64_t n_rows = sc->emit_rows, n_mine = !LIST ? n_rows : n_rows ? sc->n_left : 0u;
-  if (!LIST && (uint64_t)blockIdx.x * blockDim.x >= n_mine) return;
-  uint64_t first = (uint64_t)blockIdx.x * blockDim.x;
-  do {
-    if (LIST && first >= n_mine) break;
-    uint64_t i = first + threadIdx.x, o = 0;
-    uint32_t row = 0;
-    bool active = i < n_mine;
-    if (LIST && active) i = left[i];
-    /* A wavefront that has just started comes first on its SIMD until the loads of its joined row are
-     * on their way (two dependent loads with a few instructions between them, which would otherwise
-     * queue behind the formatting of the two older wavefronts): config 3 4.70 -> 4.61 ms, config 4
-     * 2.12 -> 2.07 ms.  Priority 1, 2 or 3: the same.  Kept up until the name is copied, lowered in
-     * steps, lowered behind the branch below or before the row's loads: slower or no gain; a
-     * scheduling barrier in place of the priority: no gain. */
-    __builtin_amdgcn_s_setprio(3);
-    if (active) { row = perm[i]; o = offs[i]; active = offs[i + 1] != o; } /* one wait for both */
-    MatRow m;
-    BlockWriter w;
-    w.stage_init((uint32_t)threadIdx.x * (KTJ_STAGE_BLOCKS * 16u));
-    ActivityParts<BlockWriter> parts;
-    if (active) {
-      m = *reinterpret_cast<const MatRow*>(rows + (uint64_t)row * (LIST ? sizeof(weave::TextRow) : sizeof(MatRow)));
-      __builtin_amdgcn_s_setprio(0); /* (a wavefront without any activity keeps it: it ends at once) */
-      w.begin(out, prefix_len + o, !i ? 0u : LIST ? tail_kind_at(kind_sorted, reinterpret_cast<const weave::TextRow*>(rows), perm, i - 1, ctx) : kind_sorted[i - 1], i == 0);
-      w.stage_follow();
-      format_head(w, m, ctx, parts);
-    }
-    w.flush(false);
-    if (active) format_args(w, m, ctx, parts);
-    w.flush_if_full();
-    if (active) {
-      format_flow(w, m, ctx, parts);
-      w.end(i + 1 == n_rows);
-    }
-    w.flush(true);
-    first += (uint64_t)gridDim.x * blockDim.x;
-  } while (LIST);
+  if ((uint64_t)blockIdx.x * blockDim.x >= n_mine) return; /* (an empty list: 4 us for 30 000 rows, 20 for 22 million) */
+  uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x, o = 0;
+  uint32_t row = 0;
+  bool active = i < n_mine;
+  if (LIST && active) i = left[i];
+  /* A wavefront that has just started comes first on its SIMD until the loads of its joined row are
+   * on their way (two dependent loads with a few instructions between them, which would otherwise
+   * queue behind the formatting of the two older wavefronts): config 3 4.70 -> 4.61 ms, config 4
+   * 2.12 -> 2.07 ms.  Priority 1, 2 or 3: the same.  Kept up until the name is copied, lowered in
+   * steps, lowered behind the branch below or before the row's loads: slower or no gain; a
+   * scheduling barrier in place of the priority: no gain. */
+  __builtin_amdgcn_s_setprio(3);
+  if (active) { row = perm[i]; o = offs[i]; active = offs[i + 1] != o; } /* one wait for both */
+  MatRow m;
+  BlockWriter w;
+  w.stage_init((uint32_t)threadIdx.x * (KTJ_STAGE_BLOCKS * 16u));
+  ActivityParts<BlockWriter> parts;
+  if (active) {
+    m = *reinterpret_cast<const MatRow*>(rows + (uint64_t)row * (LIST ? sizeof(weave::TextRow) : sizeof(MatRow)));
+    __builtin_amdgcn_s_setprio(0); /* (a wavefront without any activity keeps it: it ends at once) */
+    w.begin(out, prefix_len + o, !i ? 0u : LIST ? tail_kind_at(kind_sorted, reinterpret_cast<const weave::TextRow*>(rows), perm, i - 1, ctx) : kind_sorted[i - 1], i == 0);
+    w.stage_follow();
+    format_head(w, m, ctx, parts);
+  }
+  w.flush(false);
+  if (active) format_args(w, m, ctx, parts);
+  w.flush_if_full();
+  if (active) {
+    format_flow(w, m, ctx, parts);
+    w.end(i + 1 == n_rows);
+  }
+  w.flush(true);
 }
 hipError_t emit_direct(const void* rows, const uint32_t* perm, const uint64_t* offs, const uint8_t* kind_sorted, uint64_t n_most, EmitCtx ctx,
                        char* out, uint64_t prefix_len, const Scalars* sc, const uint32_t* left, hipStream_t st) {
   if (n_most == 0) return hipSuccess;
   const size_t stage_lds = (size_t)KTJ_BLOCK * KTJ_STAGE_BLOCKS * 16u;
-  uint32_t grid = grid_for(n_most, KTJ_BLOCK);
-  if (left && grid > 256u * 3u) grid = 256u * 3u; /* as many as run at a time: mostly the list is empty (22 M rows: 20 us for a grid over them all) */
-  hipLaunchKernelGGL(left ? k_emit_direct<true> : k_emit_direct<false>, dim3(grid), dim3(KTJ_BLOCK), stage_lds, st, static_cast<const char*>(rows), perm, offs,
+  hipLaunchKernelGGL(left ? k_emit_direct<true> : k_emit_direct<false>, dim3(grid_for(n_most, KTJ_BLOCK)), dim3(KTJ_BLOCK), stage_lds, st, static_cast<const char*>(rows), perm, offs,
                      kind_sorted, ctx, out, prefix_len, sc, left);
   return KTJ_LAUNCH_CHECK();
 }

@@ -540,16 +540,16 @@ KTJ_HD KTJ_FI inline bool text_row(const MatRow& m, const EmitCtx& c, const Sche
     frag = false;
     if (m.aux < c.n_schemas) {
       if (m.aux >= MAX_SCHEMAS) return false;
-      const SchemaPlan s = schemas[m.aux];
-      if (!(s.what & 1u) || m.p[0] + ((s.what >> 8) & 0xFFu) > c.n_args) return false;
-      frag = (s.what & 2u) != 0;
-      if (s.what & 4u) {
+      const uint32_t what_plan = schemas[m.aux].what;
+      if (!(what_plan & 1u) || m.p[0] + ((what_plan >> 8) & 0xFFu) > c.n_args) return false;
+      frag = (what_plan & 2u) != 0;
+      if (what_plan & 4u) {
         const uint32_t id = (uint32_t)c.args[m.p[0]];
         frag = id < c.dict.n && (dict_flags(c.dict, id) & KTJ_SF_ARG_BLANK) == 0;
       }
       if (frag) {
         args = KTJ_TR_SCHEMA + m.aux;
-        n += s.chars;
+        n += schemas[m.aux].chars;
         KTJ_NOUNROLL
         for (uint32_t j = 0; j < 4; ++j) {
           const uint32_t item = schemas[m.aux].item[j], what = item & 0xFFu;
@@ -566,10 +566,10 @@ KTJ_HD KTJ_FI inline bool text_row(const MatRow& m, const EmitCtx& c, const Sche
           if (what > I_ARRAY + 2u) append_next(t, a[2]);
           n += put(item_slot(j), t);
         }
-        between = (s.what >> 16) & 3u;
-        if (between == 1u) at_more = string((uint32_t)c.args[m.p[0] + (s.what >> 24)], false, &len1);
+        between = (what_plan >> 16) & 3u;
+        if (between == 1u) at_more = string((uint32_t)c.args[m.p[0] + (what_plan >> 24)], false, &len1);
         else if (between) {
-          const uint64_t at = m.p[0] + (s.what >> 24);
+          const uint64_t at = m.p[0] + (what_plan >> 24);
           if (at >> 32) return false;
           at_more = (uint32_t)at;
           if (between == 2u) len1 = real(c.args[at]);
