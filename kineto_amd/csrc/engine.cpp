@@ -231,7 +231,7 @@ struct ktj_engine {
   DevBuf s_dev_k, s_dev_r, s_dev_l, s_res_k, s_res_r, s_res_l;
   DevBuf keys_a, keys_b, vals_a, vals_b, hist, scan_tmp;
   bool rows_are_text = false;              /* of the last pass: TextRows in mat */
-  DevBuf mat, schema_book, len, len_sorted, kind_sorted, offs, out, tile_start;
+  DevBuf mat, schema_book, wide_text, len, len_sorted, kind_sorted, offs, out, tile_start;
   void* pinned_small = nullptr; size_t pinned_small_cap = 0;
   HostCtl* h_ctl = nullptr;                  /* pinned: what the device hands back during a pass */
   HostCtl* h_ctl_dev = nullptr;              /* the same memory as the kernels address it */
@@ -1478,6 +1478,7 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
    * would not fit the scratch array with as many records. */
   const bool woven = n_coll == 0 && !e->noalloc && !e->no_weave && !(e->flags & KTJ_CREATE_TILE_EMIT);
   e->rows_are_text = woven;
+  const bool wide = woven && std::any_of(e->fields.begin(), e->fields.end(), [](const ktj_field& f) { return f.type == KTJ_F_F64; });
   e->pool_used = 0;
   size_t pass_bytes = 0;
   for (int phase = e->noalloc ? 1 : 0; phase < 2; ++phase) { /* 0: add the sizes up and size the pool; 1: hand the buffers out */
@@ -1516,6 +1517,7 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
   }
   NEED(e->mat, Na * (woven ? sizeof(weave::TextRow) : sizeof(MatRow)));
   if (woven) NEED(e->schema_book, sizeof(weave::SchemaBook));
+  if (wide) NEED(e->wide_text, ng * sizeof(weave::WideText));
   NEED(e->len, Na * 4); NEED(e->len_sorted, Na * 4); NEED(e->kind_sorted, Na + 16);
   NEED(e->offs, (Na + 1) * 8);
   if (e->measuring) {
@@ -1580,7 +1582,7 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
   HIPCHK(plan_tables(tf, fc, tn, nc, t_cpu, (e->flags & KTJ_CREATE_HASH_JOIN) != 0, sc, st));
   ApiTable api{e->d_cid_names.as<uint32_t>(), (uint32_t)e->cid_names.size(), e->d_flow_bits.as<uint32_t>(), e->malloc_cid};
   weave::SchemaBook* book = woven ? e->schema_book.as<weave::SchemaBook>() : nullptr;
-  const Rows rows{e->mat.p, book};
+  const Rows rows{e->mat.p, book, wide ? e->wide_text.as<weave::WideText>() : nullptr};
   const MatRow* mat = e->mat.as<MatRow>();
   /* places of the rows that are not text: in the sort's buffer that does not hold its result */
   auto left = [&]() -> uint32_t* { return !woven ? nullptr : e->sorted_keys == e->keys_b.p ? e->keys_a.as<uint32_t>() : e->keys_b.as<uint32_t>(); };
@@ -1622,7 +1624,7 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
   HIPCHK(collect_distinct(c, N, sets, sc, straight, ctx, book, st));
   auto put_activities = [&](uint64_t n_most, uint64_t at) -> int { /* the documents' activities, but for the tile variant */
     if (woven)
-      HIPCHK(weave_activities(e->mat.as<weave::TextRow>(), e->perm, e->offs.as<uint64_t>(), e->kind_sorted.as<uint8_t>(), n_most, ctx, e->out.as<char>(), at, sc, book, st));
+      HIPCHK(weave_activities(e->mat.as<weave::TextRow>(), e->perm, e->offs.as<uint64_t>(), e->kind_sorted.as<uint8_t>(), n_most, ctx, e->out.as<char>(), at, sc, book, rows.wide, st));
     HIPCHK(emit_direct(rows.p, e->perm, e->offs.as<uint64_t>(), e->kind_sorted.as<uint8_t>(), n_most, ctx, e->out.as<char>(), at, sc, left(), st));
     return KTJ_OK;
   };

@@ -358,6 +358,7 @@ hipError_t radix_sort(uint64_t* keys_a, uint32_t* vals_a, uint64_t* keys_b, uint
 struct Rows {
   void* p;
   const weave::SchemaBook* schemas;
+  weave::WideText* wide; /* of the generic records */
 };
 #define KTJ_KIND_LEFT 3u
 /* keys: KTJ_SYNC_CAP + 1, first_pos: KTJ_SYNC_CAP + 1, is_first: n_generic (all caller-provided);
@@ -411,7 +412,7 @@ hipError_t emit_direct(const void* rows, const uint32_t* perm, const uint64_t* o
 /* The activities of rows that are text (TextRow), one lane per segment (weave.hip).  The others, if any, are on the list
  * that gather_offsets made: emit_direct's. */
 hipError_t weave_activities(const weave::TextRow* rows, const uint32_t* perm, const uint64_t* offs, const uint8_t* kind_sorted, uint64_t n_most, EmitCtx ctx, char* out,
-                 uint64_t prefix_len, const Scalars* sc, const weave::SchemaBook* schemas, hipStream_t st);
+                 uint64_t prefix_len, const Scalars* sc, const weave::SchemaBook* schemas, const weave::WideText* wide, hipStream_t st);
 
 /* ---- small traces: the whole pass in three launches (small.hip) ---- */
 #define SMALL_ROWS 2048u       /* records of the three classes together: what LDS holds the join tables for */

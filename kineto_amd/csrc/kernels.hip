@@ -2177,12 +2177,12 @@ hipError_t stream_sync_first(const uint32_t* perm, uint64_t n_sorted, const ktj_
 template <bool TEXT> struct RowOf { typedef MatRow T; };
 template <> struct RowOf<true> { typedef weave::TextRow T; };
 template <bool TEXT>
-__device__ __forceinline__ uint32_t stage_row(const MatRow& m, const EmitCtx& ctx, const weave::SchemaBook* schemas, Scalars* sc, uint4* stage) {
+__device__ __forceinline__ uint32_t stage_row(const MatRow& m, const EmitCtx& ctx, const Rows& rows, uint32_t wide_at, Scalars* sc, uint4* stage) {
   if (!TEXT) { row_to_lds(m, stage); return row_length(m, ctx, sc); }
   weave::TextRow* const t = reinterpret_cast<weave::TextRow*>(stage) + threadIdx.x;
   uint32_t n, tail;
   if (!(m.meta & KTJ_M_VALID)) n = 0;
-  else if (weave::text_row(m, ctx, schemas->plan, t, threadIdx.x & 7u, &n, &tail)) return n | (tail << 30);
+  else if (weave::text_row(m, ctx, rows.schemas->plan, t, threadIdx.x & 7u, rows.wide, wide_at, &n, &tail)) return n | (tail << 30);
   else n = row_length(m, ctx, sc) | (KTJ_KIND_LEFT << 30);
   static_assert(sizeof(MatRow) == 96, "six blocks");
   auto block = [&](uint32_t k) { __builtin_memcpy(t->w[k ^ (threadIdx.x & 7u)], reinterpret_cast<const char*>(&m) + 16u * k, 16); };
@@ -2212,7 +2212,7 @@ __device__ __forceinline__ void mat_generic_block(const ktj_generic_rec* g, uint
       count_row_stats(m, ctx, &rs);
     }
     __syncthreads(); /* every lane has taken its record */
-    if (active) len[first + i] = stage_row<TEXT>(m, ctx, rows.schemas, sc, stage);
+    if (active) len[first + i] = stage_row<TEXT>(m, ctx, rows, (uint32_t)i, sc, stage);
     __syncthreads();
     rows_lds_to_global(static_cast<typename RowOf<TEXT>::T*>(rows.p) + first + base, cnt, stage);
   }
@@ -2365,7 +2365,7 @@ __global__ void KX_JOIN_ATTR k_join_runtime(const ktj_runtime_rec* r, uint64_t n
       __syncthreads();
       if (i < n) {
         count_row_stats(m, ctx, &rs);
-        store_once(&len[a], stage_row<true>(m, ctx, rows.schemas, sc, stage));
+        store_once(&len[a], stage_row<true>(m, ctx, rows, 0, sc, stage));
       }
     }
     __syncthreads(); /* the joined rows go out the way the records came in */
@@ -2469,7 +2469,7 @@ __device__ __forceinline__ void mat_device_block(const ktj_device_rec* d, uint64
       count_row_stats(m, ctx, &rs);
     }
     __syncthreads(); /* every lane has taken its record */
-    if (active) store_once(&len[a], stage_row<TEXT>(m, ctx, rows.schemas, sc, stage));
+    if (active) store_once(&len[a], stage_row<TEXT>(m, ctx, rows, 0, sc, stage));
     __syncthreads();
     rows_lds_to_global(static_cast<typename RowOf<TEXT>::T*>(rows.p) + first + base, cnt, stage);
   }

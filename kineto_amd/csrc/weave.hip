@@ -8,14 +8,16 @@
  * text from LDS, a number of the row's), a prefix sum of their lengths gives their places, and they are OR-ed into a
  * zero-filled piece of the document in LDS, whose whole lines leave with lane-consecutive stores.  Numbers were made
  * into text in the size pass, which needs their lengths anyway; the texts with process and thread are made once per
- * track.  3220 vector and 770 LDS instructions for 64 kernel events, 119 registers, four wavefronts per SIMD.
+ * track.  3220 vector and 770 LDS instructions for 64 kernel events, 99 registers, four wavefronts per SIMD.
  *
  * What bounds it: the LDS pipe (1.02 of 1.9 ms for 11 million kernels, a third of that bank conflicts) and the
  * vector units (0.9 ms) together with the waits between them; the bytes alone (1.4 GB of rows, 5.4 GB of document)
  * take 1.3 ms.  Measured against k_emit_direct: 10 000 x 3 records 38.7 -> 16 us, 4000 operators with long strings
- * 71 -> 34 us, 733 000 records 176 -> 142 us, 3 million 795 -> 465 us, 11 million kernels 2.06 -> 1.71 ms, 22 million
- * records 4.59 -> 3.48 ms, 5 million operators with long strings (1.4 KB each: strings beyond 128 bytes are fetched from
- * memory piece by piece) 3.20 -> 3.02 ms; the size pass has become 4 to 13 % longer for the numbers' text.
+ * 71 -> 24 us, 733 000 records 176 -> 142 us, 3 million 795 -> 465 us, 11 million kernels 2.06 -> 1.71 ms, 22 million
+ * records 4.59 -> 3.47 ms, 5 million operators with long strings (1.4 KB each: strings beyond 128 bytes are fetched from
+ * memory piece by piece) 3.20 -> 2.67 ms; the size pass has become 4 to 13 % longer for the numbers' text.
+ * (Long strings' whole lines from the dictionary to the document past the tile, the loads of four strings at a time in
+ * front of any store: 2.70 ms, and 26 instead of 24 us for 4000 of them.)
  * Fewer wavefronts cost: three per SIMD 2.48 ms for the kernels, two 2.83.  Five (96 registers, 2048 bytes of tile, 512
  * of names) gave 2.22, 2048 bytes being short of most groups of 64 segments; with the tile as it is 96 registers alone
  * 1.97.  Workgroups of four wavefronts: eight, with the book in LDS twice per CU instead of four times, 1.74.
@@ -135,7 +137,7 @@ __device__ __forceinline__ uint64_t make_track(char* lds, uint32_t mine, uint64_
 
 __global__ void __launch_bounds__(WV_WAVES * 64u) __attribute__((amdgpu_waves_per_eu(4)))
 k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const uint8_t* kind_sorted, EmitCtx ctx, char* out, uint64_t prefix_len,
-        const Scalars* sc, uint32_t rounds, const SchemaBook* schemas) {
+        const Scalars* sc, uint32_t rounds, const SchemaBook* schemas, const WideText* wide) {
   const uint32_t lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   static_assert(WV_BOOK_PLANS % 16u == 0 && sizeof(SchemaPlan) % 16u == 0, "in sixteens");
   for (uint32_t k = threadIdx.x; k < MAX_TEXT; k += blockDim.x) reinterpret_cast<uint4*>(wv_lds)[k] = reinterpret_cast<const uint4*>(g_book.text)[k];
@@ -249,14 +251,19 @@ k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const u
       units = (len0 <= WV_NAME_MOST ? (len0 + 15u) / 16u : 0u) | (KTJ_TR_BETWEEN(plan) == 3u ? 2u << 16 : 0u);
     }
     const uint32_t upto = dpp_add(counts), before = upto - counts; /* of the first lane of each */
-    /* the strings in LDS: doubles that are printed here, two units each, and names as far as there is room */
-    static_assert(WV_ROWS * 32u <= WV_NAMES, "the doubles have room");
+    /* the strings in LDS: wide texts, two units each, and names as far as there is room */
+    static_assert(WV_ROWS * sizeof(WideText) <= WV_NAMES && sizeof(WideText) == 32, "the wide texts have room");
     const uint32_t units_upto = dpp_add(units), double_at = WV_NAMES_AT + ((units_upto - units) >> 16) * 16u;
     const uint32_t name_upto = (units_upto & 0xFFFFu) + (__builtin_amdgcn_readlane(units_upto, 63) >> 16);
     units &= 0xFFFFu;
     const bool near = units != 0 && name_upto <= WV_NAMES / 16u;
     const uint32_t name_at = WV_NAMES_AT + (name_upto - units) * 16u;
-    v4u32 nx, ny;
+    v4u32 nx, ny, wx, wy;
+    const bool wide_text = counts != 0 && KTJ_TR_BETWEEN(plan) == 3u;
+    if (wide_text) {
+      const gsrc src = reinterpret_cast<gsrc>((uint64_t)(uintptr_t)wide + (uint64_t)more * sizeof(WideText));
+      wx = src[0]; wy = src[1];
+    }
     const uint32_t q_units = WV_QUAD(near ? units : 0u, 0), q_at = mine + WV_QUAD(name_at, 0);
     {
       const gsrc src = reinterpret_cast<gsrc>((uint64_t)(uintptr_t)ctx.dict.name_blob + (uint64_t)name_off * 16u);
@@ -277,14 +284,6 @@ k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const u
       put_part(refs[R_TAIL + KTJ_TR_TAIL(plan)]);
       const uint32_t between = KTJ_TR_BETWEEN(plan);
       const uint32_t at = between < 2u ? 0u : between == 2u ? act * WV_VAL_BYTES + WV_VAL(S_Y) : double_at;
-      if (between == 3u) {
-        LongText t;
-        t.w[0] = t.w[1] = t.w[2] = t.w[3] = 0; t.n = 0;
-        put_f64(t, ctx.args[more]);
-        v2u64* const v = reinterpret_cast<v2u64*>(wv_lds + mine + double_at);
-        v[0] = (v2u64){t.w[0], t.w[1]};
-        v[1] = (v2u64){t.w[2], 0};
-      }
       v4u32 runs;
       runs.x = more; runs.y = len1 | (at << 16);
       if (KTJ_TR_ARGS(plan) == A_COPY) runs.y = ((32u - (uint32_t)__clz((int)more) + 7u) >> 3) << 24; /* of the kind's characters, up to four */
@@ -293,6 +292,10 @@ k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const u
     }
     const uint32_t totals = __builtin_amdgcn_readlane(upto, 63);
     if (lane == 0) parts[totals >> 16] = totals & 0x7FFFu;
+    if (wide_text) {
+      *reinterpret_cast<v4u32*>(wv_lds + mine + double_at) = wx;
+      *reinterpret_cast<v4u32*>(wv_lds + mine + double_at + 16u) = wy;
+    }
     if (h < q_units) {
       *reinterpret_cast<v4u32*>(wv_lds + q_at + h * 16u) = nx;
       if (h + 4u < q_units) *reinterpret_cast<v4u32*>(wv_lds + q_at + (h + 4u) * 16u) = ny;
@@ -467,14 +470,14 @@ k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const u
 }
 
 hipError_t weave_activities(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const uint8_t* kind_sorted, uint64_t n_most, EmitCtx ctx, char* out,
-                 uint64_t prefix_len, const Scalars* sc, const SchemaBook* schemas, hipStream_t st) {
+                 uint64_t prefix_len, const Scalars* sc, const SchemaBook* schemas, const WideText* wide, hipStream_t st) {
   if (n_most == 0) return hipSuccess;
   static_assert(WV_TILE_ROOM / 16u <= 3u * 64u, "the tile leaves in three turns at most");
   const uint64_t turns = (n_most + WV_ROWS - 1) / WV_ROWS;
   const uint32_t waves = turns >= 256u * WV_WAVES ? WV_WAVES : turns <= 256u ? 1u : (uint32_t)((turns + 255u) / 256u);
   const uint32_t rounds = turns >= 256u * 16u * 32u ? 16u : turns >= 256u * 16u * 4u ? 4u : turns > 256u * 16u ? 2u : 1u;
   hipLaunchKernelGGL(k_weave, dim3(grid_for(turns, waves * rounds)), dim3(waves * 64u), WV_BOOK_BYTES + waves * WV_WAVE_BYTES, st, rows, perm, offs,
-                     kind_sorted, ctx, out, prefix_len, sc, rounds, schemas);
+                     kind_sorted, ctx, out, prefix_len, sc, rounds, schemas, wide);
   return KTJ_LAUNCH_CHECK();
 }
 

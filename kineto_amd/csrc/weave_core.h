@@ -41,11 +41,14 @@ enum : uint32_t {
  * for each number, 160 for a row: the size pass, whose rows wait in LDS, ran three instead of four wavefronts per SIMD,
  * 22 million records 1.32 + 0.70 + 0.15 ms instead of 1.15 + 0.57 + 0.13.) */
 struct alignas(16) TextRow { uint32_t w[8][4]; };
+/* The text of a double that has no room in its row, for generic records whose schemas have one among too many numbers.  (Printed
+ * by the weaver, with a quarter of the lanes, it took two thirds of its time for 5 million such records.) */
+struct alignas(16) WideText { uint64_t w[4]; };
 #define KTJ_TR_BLOCK(slot) (((slot) + 3u) & 7u)
 #define KTJ_TR_PLAN 0u             /* KTJ_TR_*, the thread's bits from 42 on */
 #define KTJ_TR_NAME 1u             /* place of the name in its blob, in units of sixteen bytes */
 #define KTJ_TR_LENS 2u             /* its length; << 16: that of the string or double between the args' parts */
-#define KTJ_TR_MORE 3u             /* the string's place in its blob; the double's place among the arguments; a copy's kind as text */
+#define KTJ_TR_MORE 3u             /* the string's place in its blob; the WideText's number; a copy's kind as text */
 static_assert(sizeof(TextRow) == 128 && sizeof(TextRow) >= sizeof(MatRow), "a row that is left to format_activity is a MatRow in the same place");
 /* a row of the other kind: the last byte, S_Y's count of characters otherwise */
 #define KTJ_ROW_LEFT 0xFFu
@@ -57,7 +60,7 @@ static_assert(sizeof(TextRow) == 128 && sizeof(TextRow) >= sizeof(MatRow), "a ro
 #define KTJ_TR_SCHEMA 64u
 #define KTJ_TR_NO_ARGS 127u
 #define KTJ_TR_TAIL(x) (((x) >> 21) & 15u)     /* R_TAIL and the following */
-#define KTJ_TR_BETWEEN(x) (((x) >> 25) & 3u)   /* 1 string, 2 double in S_Y and S_Z, 3 double that the weaver prints */
+#define KTJ_TR_BETWEEN(x) (((x) >> 25) & 3u)   /* 1 string, 2 double in S_Y and S_Z, 3 double beside the row (WideText) */
 #define KTJ_TR_TID_HIGH(x) ((x) >> 27)
 #define KTJ_TR_DEV_BITS 22u                    /* a track's process or device, and 42 of the thread's or stream's 47 bits */
 
@@ -463,21 +466,110 @@ KTJ_HD KTJ_FI inline Text time_text_of(int64_t ns) { /* put_ts */
   append(t, (ascii4((uint32_t)ns - (uint32_t)us * 1000u) & 0xFFFFFF00u) | (uint32_t)'.', 4);
   return t;
 }
-/* a double as put_f64 prints it, 24 characters at most */
+/* up to 24 characters, zeros behind them */
 struct LongText {
-  uint64_t w[4]; uint32_t n;
-  KTJ_HD KTJ_FI void ch(char c) {
-    const uint64_t x = (uint64_t)(unsigned char)c << ((n & 7u) * 8u);
-    w[0] |= n < 8u ? x : 0; w[1] |= n >= 8u && n < 16u ? x : 0; w[2] |= n >= 16u ? x : 0;
-    ++n;
+  uint64_t w[3]; uint32_t n;
+  KTJ_HD KTJ_FI void up(uint32_t k) { /* k characters further on */
+    const uint32_t s = (k & 7u) * 8u;
+    if (k >= 16u) { w[2] = w[0]; w[1] = w[0] = 0; }
+    else if (k >= 8u) { w[2] = w[1]; w[1] = w[0]; w[0] = 0; }
+    w[2] = (w[2] << s) | ((w[1] >> 1) >> (63u - s));
+    w[1] = (w[1] << s) | ((w[0] >> 1) >> (63u - s));
+    w[0] <<= s;
   }
-  template <unsigned N> KTJ_HD KTJ_FI void lit(const PackedLit<N>& l) { for (unsigned i = 0; i < N; ++i) ch((char)(l.w[i / 8] >> (8 * (i % 8)))); }
+  KTJ_HD KTJ_FI void down(uint32_t k) {
+    const uint32_t s = (k & 7u) * 8u;
+    if (k >= 16u) { w[0] = w[2]; w[1] = w[2] = 0; }
+    else if (k >= 8u) { w[0] = w[1]; w[1] = w[2]; w[2] = 0; }
+    w[0] = (w[0] >> s) | ((w[1] << 1) << (63u - s));
+    w[1] = (w[1] >> s) | ((w[2] << 1) << (63u - s));
+    w[2] >>= s;
+  }
+  KTJ_HD KTJ_FI void add(const LongText& o) { w[0] |= o.w[0]; w[1] |= o.w[1]; w[2] |= o.w[2]; }
+  /* the first k characters only */
+  KTJ_HD KTJ_FI void keep(uint32_t k) {
+    const uint64_t part = (1ull << ((k & 7u) * 8u)) - 1u;
+    w[0] &= k >= 8u ? ~0ull : part;
+    w[1] &= k >= 16u ? ~0ull : k >= 8u ? part : 0u;
+    w[2] &= k >= 24u ? ~0ull : k >= 16u ? part : 0u;
+  }
+  KTJ_HD KTJ_FI void put(uint64_t x, uint32_t k) { /* up to eight more, behind the last */
+    LongText t;
+    t.w[0] = x; t.w[1] = t.w[2] = 0;
+    t.up(n);
+    add(t);
+    n += k;
+  }
 };
+/* A double as put_f64 prints it, with shifts of the whole text where that takes a turn per character (a size pass over
+ * 5 million of them 0.54 -> 0.47 ms). */
+KTJ_HD KTJ_FI inline LongText real_text(uint64_t bits) {
+  LongText t;
+  t.w[0] = t.w[1] = t.w[2] = 0; t.n = 0;
+  const bool neg = (bits >> 63) != 0;
+  const uint64_t mag = bits & 0x7FFFFFFFFFFFFFFFull;
+  if (mag >= 0x7FF0000000000000ull || mag == 0) {
+    if (mag == 0) { t.w[0] = neg ? 0x302Dull : 0x30ull; t.n = neg ? 2u : 1u; return t; }
+    const uint64_t word = mag > 0x7FF0000000000000ull ? 0x226E616Eull : 0x22666E69ull; /* nan", inf" */
+    t.w[0] = neg ? (word << 16) | 0x2D22ull : (word << 8) | 0x22ull;
+    t.n = neg ? 6u : 5u;
+    return t;
+  }
+  uint64_t sig;
+  int32_t k;
+  shortest_decimal(mag, &sig, &k);
+  const uint32_t nd = (uint32_t)ndigits_u64(sig);
+  const int E = k + (int)nd - 1;
+  {
+    const uint64_t top = sig / 10000000000000000ull, rest = sig - top * 10000000000000000ull, mid = rest / 100000000ull;
+    t.w[0] = ascii8((uint32_t)top); t.w[1] = ascii8((uint32_t)mid); t.w[2] = ascii8((uint32_t)(rest - mid * 100000000ull));
+  }
+  t.down(24u - nd);
+  t.n = nd;
+  if (E < 0 && E >= -4) { /* 0.000ddd */
+    const uint32_t z = (uint32_t)(1 - E); /* "0." and zeros */
+    t.up(z);
+    t.w[0] |= 0x3030302E30ull & ((1ull << (8u * z)) - 1u);
+    t.n += z;
+  } else {
+    const bool plain = E >= 0 && E < 16;
+    const uint32_t whole = plain ? (uint32_t)E + 1u : 1u; /* digits in front of the point */
+    if (nd > whole) {
+      LongText behind = t;
+      t.keep(whole);
+      behind.down(whole);
+      behind.up(whole + 1u);
+      t.add(behind);
+      LongText point;
+      point.w[0] = '.'; point.w[1] = point.w[2] = 0;
+      point.up(whole);
+      t.add(point);
+      t.n = nd + 1u;
+    } else if (plain) { /* zeros in front of it */
+      LongText zeros;
+      zeros.w[0] = zeros.w[1] = zeros.w[2] = 0x3030303030303030ull;
+      zeros.keep(whole);
+      LongText digits = zeros;
+      digits.keep(nd);
+      zeros.w[0] ^= digits.w[0]; zeros.w[1] ^= digits.w[1]; zeros.w[2] ^= digits.w[2];
+      t.add(zeros);
+      t.n = whole;
+    }
+    if (!plain) {
+      const uint32_t a = (uint32_t)(E < 0 ? -E : E), hundreds = a / 100u, tens = (a - hundreds * 100u) / 10u, ones = a - hundreds * 100u - tens * 10u;
+      const uint64_t two = (uint64_t)('0' + tens) | ((uint64_t)('0' + ones) << 8);
+      t.put((uint64_t)'e' | ((uint64_t)(E < 0 ? '-' : '+') << 8) | ((hundreds ? (two << 8) | ('0' + hundreds) : two) << 16), hundreds ? 5u : 4u);
+    }
+  }
+  if (neg) { t.up(1); t.w[0] |= '-'; ++t.n; }
+  return t;
+}
 
 /* ---- a joined row as text, its length and its tail kind (see tail_kind): false, and nothing that counts in *r, for the rows
  * that only format_activity prints.  *r is where the row waits to be stored, in LDS on the device, block b at b ^ turn (rows of
- * neighbouring lanes are a line apart): nothing of it is held in registers. ---- */
-KTJ_HD KTJ_FI inline bool text_row(const MatRow& m, const EmitCtx& c, const SchemaPlan* schemas, TextRow* r, uint32_t turn, uint32_t* len, uint32_t* tail) {
+ * neighbouring lanes are a line apart): nothing of it is held in registers.  wide[wide_at]: this row's, if there are any. ---- */
+KTJ_HD KTJ_FI inline bool text_row(const MatRow& m, const EmitCtx& c, const SchemaPlan* schemas, TextRow* r, uint32_t turn, WideText* wide, uint32_t wide_at, uint32_t* len,
+                                     uint32_t* tail) {
   const uint32_t meta = m.meta, type = meta & KTJ_M_TYPE_MASK;
   const uint32_t cls = (meta & KTJ_M_CLASS_MASK) >> KTJ_M_CLASS_SHIFT, kind = (meta & KTJ_M_KIND_MASK) >> KTJ_M_KIND_SHIFT;
   const bool device = cls == KTJ_CLASS_DEVICE, generic = cls == KTJ_CLASS_GENERIC, flow = (meta & KTJ_M_FLOW) != 0;
@@ -515,12 +607,14 @@ KTJ_HD KTJ_FI inline bool text_row(const MatRow& m, const EmitCtx& c, const Sche
     return id;
 #endif
   };
-  auto real = [&](uint64_t bits) KTJ_FI { /* a double */
-    LongText t;
-    t.w[0] = t.w[1] = t.w[2] = t.w[3] = 0; t.n = 0;
-    put_f64(t, bits);
-    two(block(S_Y), t.w[0]); two(block(S_Y) + 2, t.w[1]);
-    two(block(S_Z), t.w[2]); block(S_Z)[2] = 0;
+  auto real = [&](uint64_t bits, bool here) KTJ_FI { /* a double */
+    const LongText t = real_text(bits);
+    if (here) {
+      two(block(S_Y), t.w[0]); two(block(S_Y) + 2, t.w[1]);
+      two(block(S_Z), t.w[2]); block(S_Z)[2] = 0;
+    } else {
+      wide[wide_at].w[0] = t.w[0]; wide[wide_at].w[1] = t.w[1]; wide[wide_at].w[2] = t.w[2]; wide[wide_at].w[3] = 0;
+    }
     return t.n;
   };
   block(S_Y)[3] = 0; /* (its last byte is not KTJ_ROW_LEFT) */
@@ -569,11 +663,8 @@ KTJ_HD KTJ_FI inline bool text_row(const MatRow& m, const EmitCtx& c, const Sche
         between = (what_plan >> 16) & 3u;
         if (between == 1u) at_more = string((uint32_t)c.args[m.p[0] + (what_plan >> 24)], false, &len1);
         else if (between) {
-          const uint64_t at = m.p[0] + (what_plan >> 24);
-          if (at >> 32) return false;
-          at_more = (uint32_t)at;
-          if (between == 2u) len1 = real(c.args[at]);
-          else { CountWriter w; put_f64(w, c.args[at]); len1 = (uint32_t)w.n; }
+          at_more = wide_at;
+          len1 = real(c.args[m.p[0] + (what_plan >> 24)], between == 2u);
         }
       }
     }
@@ -622,7 +713,7 @@ KTJ_HD KTJ_FI inline bool text_row(const MatRow& m, const EmitCtx& c, const Sche
       if (bandwidth) {
         const double d = (double)m.p[0] / (memset_row ? (double)m.dur : (double)((uint64_t)m.dur + 1u));
         uint64_t bits; __builtin_memcpy(&bits, &d, 8);
-        between = 2u; len1 = real(bits);
+        between = 2u; len1 = real(bits, true);
       }
     }
     n += chars_table.of[R_ARGS + args] + chars_table.of[R_ARGS2 + args];

@@ -88,7 +88,7 @@ void lay_out_schemas(const EmitCtx& c, weave::SchemaBook* book) {
   }
 }
 // What the weaver prints for a row that is text, one segment after the other.
-std::string woven_text(const weave::TextRow& row, const EmitCtx& c, const weave::SchemaBook& book) {
+std::string woven_text(const weave::TextRow& row, const weave::WideText* wide, const EmitCtx& c, const weave::SchemaBook& book) {
   using namespace weave;
   const Book& b = BOOK;
   std::string out;
@@ -137,13 +137,7 @@ std::string woven_text(const weave::TextRow& row, const EmitCtx& c, const weave:
   switch (KTJ_TR_BETWEEN(plan)) {
     case 1: out.append(c.dict.arg_blob + (more < c.dict.n ? c.dict.arg_off[more] : 0), lens >> 16); break;
     case 2: out += std::string(reinterpret_cast<const char*>(row.w[KTJ_TR_BLOCK(S_Y)]), 16).append(reinterpret_cast<const char*>(row.w[KTJ_TR_BLOCK(S_Z)]), 8).substr(0, lens >> 16); break;
-    case 3: {
-      LongText t;
-      t.w[0] = t.w[1] = t.w[2] = t.w[3] = 0; t.n = 0;
-      put_f64(t, c.args[more]);
-      out.append(reinterpret_cast<const char*>(t.w), t.n);
-      break;
-    }
+    case 3: out.append(reinterpret_cast<const char*>(wide[more].w), lens >> 16); break;
     default: break;
   }
   part(a >= KTJ_TR_SCHEMA ? s.args2 : b.ref[R_ARGS2 + a]);
@@ -159,6 +153,13 @@ extern "C" {
 // activities of the last document rendered with KTJSIM_WOVEN that were text rows, and that were not
 void ktjsim_woven(uint64_t* woven, uint64_t* left) { *woven = n_woven; *left = n_not_woven; }
 #define KTJSIM_WOVEN 1u
+int ktjsim_real_text(double v, char* out) {
+  uint64_t b;
+  memcpy(&b, &v, 8);
+  const weave::LongText t = weave::real_text(b);
+  memcpy(out, t.w, 24);
+  return (int)t.n;
+}
 
 // Returns a malloc'ed buffer with the complete document.
 int ktjsim_render(const ktj_stream* s, uint32_t tile_bytes, char** out, uint64_t* out_n) {
@@ -438,12 +439,13 @@ int ktjsim_render(const ktj_stream* s, uint32_t tile_bytes, char** out, uint64_t
     for (size_t i = 0; i < perm.size(); ++i) {
       const MatRow& m = mat[perm[i]];
       weave::TextRow row;
+      weave::WideText wide[2];
       memset(&row, 0xA5, sizeof row);
       uint32_t len = 0, tail = 0;
       char* at = buf + prefix.size() + offs[i];
-      if (weave::text_row(m, ctx, book->plan, &row, 0, &len, &tail)) {
+      if (weave::text_row(m, ctx, book->plan, &row, 0, wide, 1, &len, &tail)) {
         if (len != offs[i + 1] - offs[i] || tail != tail_kind(m, has_args(m, ctx)) || row.w[7][3] >> 24 == KTJ_ROW_LEFT) { free(buf); return -4; }
-        const std::string t = woven_text(row, ctx, *book);
+        const std::string t = woven_text(row, wide, ctx, *book);
         if (t.size() != len) { free(buf); return -5; }
         memcpy(at, t.data(), len);
         ++n_woven;

@@ -11,7 +11,7 @@ from kineto_amd import abi
 from stream_builder import B, StreamBuilder
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
-NAME_LENGTHS = (0, 1, 15, 16, 17, 63, 64, 65, 127, 128, 129, 257, 2600, 12800, 12801)
+NAME_LENGTHS = (0, 1, 15, 16, 17, 63, 64, 65, 127, 128, 129, 255, 256, 257, 259, 300, 383, 384, 385, 500, 511, 512, 513, 1200, 2600, 12800, 12801)
 PIDS = (0, 1, 4194303, 4194304, (1 << 31) - 1, -3)                       # 22 bits, and beyond
 TIDS = (0, 5, (1 << 42) - 1, 1 << 42, (1 << 47) - 1, 1 << 47, -5, (1 << 63) - 1)
 NUMBERS = (0, 9, 10, 99999999, 100000000, 10**10, 10**11 - 1, 10**11, 10**15 - 1, 10**15, (1 << 63) - 1, -1, -(10**9), -(10**10), -(1 << 63))
@@ -138,6 +138,28 @@ def test_segments_of_every_kind_of_row(sim):
         _woven_vs_oracle(sim, random_streams.random_stream(seed, wide_ids=seed % 2 == 1).build())
     woven, left = _woven_vs_oracle(sim, edge_stream(3000))
     assert woven > 1800 and left > 300, (woven, left)
+
+
+def test_doubles_as_text(sim):
+    """Shifted together, against the formatter's characters one by one: zeros behind the text, too."""
+    import random
+    import struct
+    rng = random.Random(11)
+    values = [0.0, -0.0, float("inf"), float("-inf"), float("nan"), 5e-324, 1.7976931348623157e308, -2.2250738585072014e-308, 0.1, 1e-4, 9.999e-5, 1e-5, 1e15, 1e16,
+              123456789012345680.0, 9999999999999998.0, 1.0, 10.0, 12.5, -0.001234]
+    values += [m * 10.0**e for e in range(-8, 20) for m in (1, 1.5, 12.25, 0.6666666666666666)]
+    values += [struct.unpack("<d", struct.pack("<Q", rng.getrandbits(64)))[0] for _ in range(20000)]
+    values += [rng.choice((-1, 1)) * rng.uniform(0, 1) * 10.0**rng.randrange(-7, 20) for _ in range(20000)]
+    sim.ktjsim_fmt_double.argtypes = sim.ktjsim_real_text.argtypes = [C.c_double, C.c_char_p]
+    got, want = C.create_string_buffer(64), C.create_string_buffer(64)
+    for v in values:
+        n, m = sim.ktjsim_real_text(v, got), sim.ktjsim_fmt_double(v, want)
+        if v != v or v in (float("inf"), float("-inf")):   # (quoted where the formatter prints an argument)
+            assert got.raw[:n].strip(b'"') == want.raw[:m].strip(b'"'), v
+            assert got.raw[:n].startswith(b'"') and got.raw[:n].endswith(b'"')
+        else:
+            assert got.raw[:n] == want.raw[:m], v
+        assert got.raw[n:24] == bytes(24 - n), v
 
 
 @pytest.mark.gpu
