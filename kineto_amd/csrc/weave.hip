@@ -475,7 +475,11 @@ hipError_t weave_activities(const TextRow* rows, const uint32_t* perm, const uin
   static_assert(WV_TILE_ROOM / 16u <= 3u * 64u, "the tile leaves in three turns at most");
   const uint64_t turns = (n_most + WV_ROWS - 1) / WV_ROWS;
   const uint32_t waves = turns >= 256u * WV_WAVES ? WV_WAVES : turns <= 256u ? 1u : (uint32_t)((turns + 255u) / 256u);
-  const uint32_t rounds = turns >= 256u * 16u * 32u ? 16u : turns >= 256u * 16u * 4u ? 4u : turns > 256u * 16u ? 2u : 1u;
+  /* Turns of a wavefront: all that run at a time end together, up to about 24 (fewer: the book is copied more often, 22 million
+   * records 3.62 ms with 6, 3.47 with 16, 3.42 with 24; more: the last are late, 3 million 460 us with 24, 529 with 32).  733 000
+   * records, whose turns make 12 for each: 136 us, with 4 141, with 8, one and a half times as many wavefronts as run, 150. */
+  const uint64_t at_once = 256u * 16u, times = (turns + at_once * 24u - 1u) / (at_once * 24u);
+  const uint32_t rounds = (uint32_t)((turns + at_once * times - 1u) / (at_once * times));
   hipLaunchKernelGGL(k_weave, dim3(grid_for(turns, waves * rounds)), dim3(waves * 64u), WV_BOOK_BYTES + waves * WV_WAVE_BYTES, st, rows, perm, offs,
                      kind_sorted, ctx, out, prefix_len, sc, rounds, schemas, wide);
   return KTJ_LAUNCH_CHECK();
