@@ -126,7 +126,7 @@ __global__ void __launch_bounds__(KTJ_BLOCK) __attribute__((amdgpu_waves_per_eu(
 k_emit_direct(const char* rows, const uint32_t* perm, const uint64_t* offs, const uint8_t* kind_sorted,
               EmitCtx ctx, char* out, uint64_t prefix_len, const Scalars* sc, const uint32_t* left) {
   const uint64_t n_rows = sc->emit_rows, n_mine = !LIST ? n_rows : n_rows ? sc->n_left : 0u;
-  if ((uint64_t)blockIdx.x * blockDim.x >= n_mine) return; /* (an empty list: 4 us for 30 000 rows, 20 for 22 million) */
+  if ((uint64_t)blockIdx.x * blockDim.x >= n_mine) return;
   uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x, o = 0;
   uint32_t row = 0;
   bool active = i < n_mine;
