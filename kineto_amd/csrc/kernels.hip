@@ -1093,67 +1093,76 @@ __device__ void rank_values(const uint64_t* keys, const uint32_t* list, uint32_t
     if (p < m) rank[s] = r;
   }
 }
-/* The schemas' texts for the weaver, by one workgroup: a lane measures each schema, a lane lays it out, a lane writes the
- * characters of each field.  (One lane for all of it, in a launch of its own: 13 us for four schemas, 20 for five.) */
+/* The schemas' texts for the weaver, by one workgroup: a lane lays out each schema, sixteen move its descriptors behind the others',
+ * a lane writes the characters of each field.  (One lane for all of it, in a launch of its own: 13 us for four schemas, 20 for
+ * five.) */
 struct SchemaLds {
   uint4 key[KTJ_WEAVE_FIELDS * (KTJ_WEAVE_KEY / 16u)];
-  uint32_t text[weave::SCHEMA_TEXT * 4], desc[weave::SCHEMA_DESC];
+  uint32_t text[weave::SCHEMA_TEXT * 4], desc[weave::MAX_SCHEMAS][weave::SCHEMA_DESC];
   ktj_field field[KTJ_WEAVE_FIELDS];
   uint32_t key_len[KTJ_WEAVE_FIELDS], place[KTJ_WEAVE_FIELDS];
-  uint32_t n_fields[weave::MAX_SCHEMAS], first[weave::MAX_SCHEMAS];
   weave::SchemaPlan plan[weave::MAX_SCHEMAS];
+  uint32_t size[weave::MAX_SCHEMAS], upto[weave::MAX_SCHEMAS]; /* descriptors | units of text << 16; the sum up to here, or none where it is not taken */
 };
 __device__ void lay_out_schemas(const EmitCtx& c, weave::SchemaBook* out, SchemaLds* l) {
   const uint32_t n = c.n_schemas < weave::MAX_SCHEMAS ? c.n_schemas : weave::MAX_SCHEMAS, k = threadIdx.x;
-  static_assert(KTJ_BLOCK >= KTJ_WEAVE_FIELDS && weave::MAX_SCHEMAS <= 64u, "a lane per field, a lane of one wavefront per schema");
+  static_assert(KTJ_BLOCK >= KTJ_WEAVE_FIELDS && KTJ_BLOCK == weave::MAX_SCHEMAS * 16u, "a lane per field, sixteen per schema");
   for (uint32_t j = k; j < weave::SCHEMA_TEXT * 4u; j += KTJ_BLOCK) l->text[j] = 0;
-  if (k < weave::SCHEMA_DESC) l->desc[k] = 0;
   if (k < KTJ_WEAVE_FIELDS) l->place[k] = ~0u;
-  ktj_schema_desc schema{};
-  if (k < n) schema = c.schemas[k];
-  if (k < 64u) {
-    uint32_t upto = schema.n_fields < KTJ_WEAVE_FIELDS ? schema.n_fields : KTJ_WEAVE_FIELDS;
-    const uint32_t mine = upto;
-    for (int o = 1; o < (int)weave::MAX_SCHEMAS; o <<= 1) { const uint32_t x = __shfl_up(upto, o); if ((int)k >= o) upto += x; }
-    if (k < weave::MAX_SCHEMAS) { l->first[k] = upto - mine; l->n_fields[k] = schema.n_fields; }
+  /* which schema the lane's field is of, and which fields the lane's schema has */
+  uint32_t of = ~0u, of_field = 0, first = 0, n_fields = 0;
+  for (uint32_t j = 0, at = 0; j < n; ++j) {
+    const ktj_schema_desc d = c.schemas[j];
+    if (k >= at && k - at < d.n_fields && k < KTJ_WEAVE_FIELDS) { of = j; of_field = d.first_field + (k - at); }
+    if (j == k) { first = at; n_fields = d.n_fields; }
+    at = d.n_fields < KTJ_WEAVE_FIELDS - at ? at + d.n_fields : KTJ_WEAVE_FIELDS;
+  }
+  if (of != ~0u) {
+    const ktj_field fd = c.fields[of_field];
+    uint32_t len = 0;
+    if (fd.key_id != KTJ_NONE && fd.key_id < c.dict.n) {
+      const DictEntry e = c.dict.entries[fd.key_id];
+      const uint4* src = reinterpret_cast<const uint4*>(c.dict.arg_blob + e.arg_off);
+      len = e.arg_len;
+      if (len <= KTJ_WEAVE_KEY) for (uint32_t j = 0; j * 16u < len; ++j) l->key[k * (KTJ_WEAVE_KEY / 16u) + j] = src[j];
+    }
+    l->field[k] = fd;
+    l->key_len[k] = len;
   }
   __syncthreads();
-  if (k < KTJ_WEAVE_FIELDS && n != 0) {
-    uint32_t of = 0;
-    while (of + 1u < n && l->first[of + 1u] <= k) ++of;
-    if (k - l->first[of] < l->n_fields[of]) {
-      const ktj_field fd = c.fields[c.schemas[of].first_field + (k - l->first[of])];
-      uint32_t len = 0;
-      if (fd.key_id != KTJ_NONE && fd.key_id < c.dict.n) {
-        const DictEntry e = c.dict.entries[fd.key_id];
-        const uint4* src = reinterpret_cast<const uint4*>(c.dict.arg_blob + e.arg_off);
-        len = e.arg_len;
-        if (len <= KTJ_WEAVE_KEY) for (uint32_t j = 0; j * 16u < len; ++j) l->key[k * (KTJ_WEAVE_KEY / 16u) + j] = src[j];
-      }
-      l->field[k] = fd;
-      l->key_len[k] = len;
+  if (k < 64u) {
+    weave::SchemaPlan* const plan = &l->plan[k < weave::MAX_SCHEMAS ? k : 0u];
+    weave::SchemaSize size{0, 0};
+    if (k < weave::MAX_SCHEMAS) plan->what = 0;
+    if (k < n && first + n_fields <= KTJ_WEAVE_FIELDS) size = weave::lay_out_schema(l->field + first, l->key_len + first, n_fields, plan, l->desc[k], l->place + first);
+    const uint32_t mine = size.desc | (size.units << 16);
+    uint32_t upto = mine;
+    for (int o = 1; o < (int)weave::MAX_SCHEMAS; o <<= 1) { const uint32_t x = __shfl_up(upto, o); if ((int)k >= o) upto += x; }
+    if (k < weave::MAX_SCHEMAS) {
+      const uint32_t before = upto - mine;
+      const bool taken = plan->what != 0 && (upto & 0xFFFFu) <= weave::SCHEMA_DESC && (upto >> 16) <= weave::SCHEMA_TEXT; /* (otherwise its rows are format_activity's) */
+      l->size[k] = mine;
+      l->upto[k] = taken ? upto : 0u;
+      weave::SchemaPlan p = *plan;
+      if (!taken) p.what = 0;
+      p.args = KTJ_WREF_MOVED(p.args, before & 0xFFFFu);
+      p.args2 = KTJ_WREF_MOVED(p.args2, KTJ_WREF_COUNT(p.args2) ? before & 0xFFFFu : 0u);
+      out->plan[k] = p;
     }
   }
   __syncthreads();
-  if (k < 64u) {
-    const uint32_t first = k < n ? l->first[k] : 0u;
-    weave::SchemaPlan* const plan = &l->plan[k < weave::MAX_SCHEMAS ? k : 0u];
-    weave::SchemaSize size{0, 0};
-    bool taken = k < n && first + l->n_fields[k] <= KTJ_WEAVE_FIELDS;
-    if (taken) { size = weave::lay_out_schema(l->field + first, l->key_len + first, l->n_fields[k], 0, 0, plan, nullptr, nullptr); taken = plan->what != 0; }
-    uint32_t upto = size.desc | (size.units << 16);
-    for (int o = 1; o < (int)weave::MAX_SCHEMAS; o <<= 1) { const uint32_t x = __shfl_up(upto, o); if ((int)k >= o) upto += x; }
-    if ((upto & 0xFFFFu) > weave::SCHEMA_DESC || (upto >> 16) > weave::SCHEMA_TEXT) taken = false; /* its rows are format_activity's */
-    if (taken) weave::lay_out_schema(l->field + first, l->key_len + first, l->n_fields[k], (upto & 0xFFFFu) - size.desc, (upto >> 16) - size.units, plan, l->desc, l->place + first);
-    else if (k < weave::MAX_SCHEMAS) plan->what = 0;
-    if (k < weave::MAX_SCHEMAS) out->plan[k] = *plan;
+  {
+    const uint32_t schema = k >> 4, size = l->size[schema], upto = l->upto[schema];
+    if (upto) {
+      const uint32_t before = upto - size;
+      for (uint32_t j = k & 15u; j < (size & 0xFFFFu); j += 16u) out->desc[(before & 0xFFFFu) + j] = KTJ_WD_MOVED(l->desc[schema][j], before >> 16);
+    }
   }
-  __syncthreads();
-  if (k < KTJ_WEAVE_FIELDS && l->place[k] != ~0u)
-    weave::put_field_text(l->field[k], reinterpret_cast<const char*>(l->key + k * (KTJ_WEAVE_KEY / 16u)), l->key_len[k], l->place[k], reinterpret_cast<char*>(l->text));
+  if (of != ~0u && l->upto[of] != 0 && l->place[k] != ~0u)
+    weave::put_field_text(l->field[k], reinterpret_cast<const char*>(l->key + k * (KTJ_WEAVE_KEY / 16u)), l->key_len[k],
+                          KTJ_PLACE_MOVED(l->place[k], (l->upto[of] - l->size[of]) >> 16), reinterpret_cast<char*>(l->text));
   __syncthreads();
   for (uint32_t j = k; j < weave::SCHEMA_TEXT * 4u; j += KTJ_BLOCK) out->text[j] = l->text[j];
-  if (k < weave::SCHEMA_DESC) out->desc[k] = l->desc[k];
 }
 /* Distinct deviceId and resourceId values, the range of the timestamps and the number of rows that are
  * printed.  The workgroup that ends last ranks the values and plans the sort's keys.  With a book the first

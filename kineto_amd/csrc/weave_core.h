@@ -279,11 +279,13 @@ KTJ_HD KTJ_FI inline uint32_t item_slot(uint32_t j) { return j == 0 ? S_X : j ==
 #define KTJ_WEAVE_FIELDS 128u      /* fields of all schemas together (and of those behind, none is taken) */
 #define KTJ_WEAVE_KEY 48u          /* longest key */
 struct SchemaSize { uint32_t desc, units; };
-/* One schema: its plan, and with desc its descriptors from there on, its texts from unit u_at on.  Where the characters of its
- * fields go: place[], in bytes, those behind the field's value << 16, KTJ_WEAVE_COMMA. */
+/* One schema by itself, as if it were the first: its plan, its descriptors, and where the characters of its fields go: place[],
+ * in bytes, those behind the field's value << 16, KTJ_WEAVE_COMMA.  Behind others it is moved by what they have. */
+#define KTJ_WD_MOVED(desc, units) ((desc) + ((units) << 12))
+#define KTJ_WREF_MOVED(ref, descs) ((ref) + (descs))
+#define KTJ_PLACE_MOVED(place, units) ((place) + (units) * 16u * (((place) >> 16) ? 0x10001u : 1u))
 #define KTJ_WEAVE_COMMA (1u << 15)
-KTJ_HD inline SchemaSize lay_out_schema(const ktj_field* field, const uint32_t* key_len, uint32_t n_fields, uint32_t d_at, uint32_t u_at, SchemaPlan* plan,
-                                        uint32_t* desc, uint32_t* place) {
+KTJ_HD inline SchemaSize lay_out_schema(const ktj_field* field, const uint32_t* key_len, uint32_t n_fields, SchemaPlan* plan, uint32_t* desc, uint32_t* place) {
   SchemaPlan& p = *plan; /* (in LDS on the device: its items have no fixed places) */
   p.args = p.args2 = p.what = p.chars = 0;
   for (uint32_t j = 0; j < 4; ++j) p.item[j] = I_NONE;
@@ -291,8 +293,7 @@ KTJ_HD inline SchemaSize lay_out_schema(const ktj_field* field, const uint32_t* 
   bool taken = true, comma = false;
   auto end = [&](uint32_t number) {
     if (n_desc >= SCHEMA_DESC || n_unit >= SCHEMA_TEXT) { taken = false; len = 0; return; }
-    if (desc) desc[d_at + n_desc] = KTJ_WD(len, number, SCHEMA_UNIT + u_at + n_unit);
-    ++n_desc;
+    desc[n_desc++] = KTJ_WD(len, number, SCHEMA_UNIT + n_unit);
     p.chars += len;
     n_unit += (len + 15u) / 16u;
     len = 0;
@@ -302,7 +303,7 @@ KTJ_HD inline SchemaSize lay_out_schema(const ktj_field* field, const uint32_t* 
     while (len + n > KTJ_WEAVE_LIT) { n -= KTJ_WEAVE_LIT - len; len = KTJ_WEAVE_LIT; end(S_NONE); }
     len += n;
   };
-  auto here = [&]() { return (u_at + n_unit) * 16u + len; };
+  auto here = [&]() { return n_unit * 16u + len; };
   auto number = [&](uint32_t j, uint32_t what) {
     if (j >= 4u) { taken = false; return; }
     p.item[j] = what | (slot << 8);
@@ -351,19 +352,19 @@ KTJ_HD inline SchemaSize lay_out_schema(const ktj_field* field, const uint32_t* 
         if (fd.type == KTJ_F_RAW && !key && n_fields == 1u) p.what |= 4u;
         if (len) end(S_NONE);
         between = fd.type != KTJ_F_F64 ? 1u : real ? 2u : 3u; between_slot = slot;
-        p.args = KTJ_WREF(MAX_DESC + d_at + d_args, n_desc - d_args);
+        p.args = KTJ_WREF(MAX_DESC + d_args, n_desc - d_args);
         d_args = n_desc;
         at |= here() << 16;
         if (fd.type == KTJ_F_STR) chars(1);
         break;
       default: taken = false; break;
     }
-    if (desc) place[f] = at | (commas ? KTJ_WEAVE_COMMA : 0u);
+    place[f] = at | (commas ? KTJ_WEAVE_COMMA : 0u);
     slot += fd.count;
   }
   if (len) end(S_NONE);
   if (slot > 255u || n_unit > SCHEMA_TEXT) taken = false;
-  const uint32_t ref = KTJ_WREF(MAX_DESC + d_at + d_args, n_desc - d_args);
+  const uint32_t ref = KTJ_WREF(MAX_DESC + d_args, n_desc - d_args);
   if (between) p.args2 = ref; else p.args = ref;
   p.what |= 1u | (n_fields ? 2u : 0u) | (slot << 8) | (between << 16) | (between_slot << 24);
   SchemaSize size;

@@ -79,12 +79,18 @@ void lay_out_schemas(const EmitCtx& c, weave::SchemaBook* book) {
         key[j].assign(c.dict.arg_blob + c.dict.arg_off[f[j].key_id], c.dict.arg_blob + c.dict.arg_off[f[j].key_id + 1]);
         key_len[j] = (uint32_t)key[j].size();
       }
-    const weave::SchemaSize size = weave::lay_out_schema(f, key_len.data(), sd.n_fields, 0, 0, &book->plan[k], nullptr, nullptr);
+    std::vector<uint32_t> own(weave::SCHEMA_DESC);
+    const weave::SchemaSize size = weave::lay_out_schema(f, key_len.data(), sd.n_fields, &book->plan[k], own.data(), place.data());
     desc += size.desc; units += size.units;
     if (desc > weave::SCHEMA_DESC || units > weave::SCHEMA_TEXT) { book->plan[k].what = 0; continue; }
     if (!book->plan[k].what) continue;
-    weave::lay_out_schema(f, key_len.data(), sd.n_fields, desc - size.desc, units - size.units, &book->plan[k], book->desc, place.data());
-    for (uint32_t j = 0; j < sd.n_fields; ++j) weave::put_field_text(f[j], key[j].data(), key_len[j], place[j], reinterpret_cast<char*>(book->text));
+    const uint32_t d_at = desc - size.desc, u_at = units - size.units;
+    weave::SchemaPlan& p = book->plan[k];
+    p.args = KTJ_WREF_MOVED(p.args, d_at);
+    if (KTJ_WREF_COUNT(p.args2)) p.args2 = KTJ_WREF_MOVED(p.args2, d_at);
+    for (uint32_t j = 0; j < size.desc; ++j) book->desc[d_at + j] = KTJ_WD_MOVED(own[j], u_at);
+    for (uint32_t j = 0; j < sd.n_fields; ++j)
+      weave::put_field_text(f[j], key[j].data(), key_len[j], KTJ_PLACE_MOVED(place[j], u_at), reinterpret_cast<char*>(book->text));
   }
 }
 // What the weaver prints for a row that is text, one segment after the other.
