@@ -24,7 +24,7 @@ sys.path.insert(0, ROOT)
 sys.path.insert(0, os.path.join(ROOT, "tests"))
 
 HBM_PEAK_GBS = 8000.0
-DOMINANT_KERNEL = "k_emit_direct"
+DOMINANT_KERNEL = "k_weave"
 FULL_SIZE = {1: 10000, 2: 1000000, 3: 10000000, 4: 11000000, 5: 5000000}
 WORKLOAD = {
     1: "config1: 10k CPU ops + 10k launches + 10k kernels, 4 streams",

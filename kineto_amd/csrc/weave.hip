@@ -10,11 +10,11 @@
  * into text in the size pass, which needs their lengths anyway; the texts with process and thread are made once per
  * track.  3220 vector and 770 LDS instructions for 64 kernel events, 99 registers, four wavefronts per SIMD.
  *
- * What bounds it: the LDS pipe (1.02 of 1.9 ms for 11 million kernels, a third of that bank conflicts) and the
- * vector units (0.9 ms) together with the waits between them; the bytes alone (1.4 GB of rows, 5.4 GB of document)
- * take 1.3 ms.  Measured against k_emit_direct: 10 000 x 3 records 38.7 -> 16 us, 4000 operators with long strings
- * 71 -> 24 us, 733 000 records 176 -> 142 us, 3 million 795 -> 465 us, 11 million kernels 2.06 -> 1.71 ms, 22 million
- * records 4.59 -> 3.47 ms, 5 million operators with long strings (1.4 KB each: strings beyond 128 bytes are fetched from
+ * What bounds it: memory (22 million records 13.6 GB in 3.44 ms, 0.89 of what a plain copy reaches; 11 million kernels 0.95),
+ * with the vector units busy for 2.1 and the LDS pipes for 1.9 of the 3.44 ms, a third of that bank conflicts.
+ * Measured against k_emit_direct: 10 000 x 3 records 38.7 -> 15.5 us, 4000 operators with long strings
+ * 71 -> 24 us, 733 000 records 176 -> 136 us, 3 million 795 -> 451 us, 11 million kernels 2.06 -> 1.70 ms, 22 million
+ * records 4.59 -> 3.44 ms, 5 million operators with long strings (1.4 KB each: strings beyond 128 bytes are fetched from
  * memory piece by piece) 3.20 -> 2.67 ms; the size pass has become 4 to 13 % longer for the numbers' text.
  * (Long strings' whole lines from the dictionary to the document past the tile, the loads of four strings at a time in
  * front of any store: 2.70 ms, and 26 instead of 24 us for 4000 of them.)

@@ -67,7 +67,6 @@ static_assert(sizeof(TextRow) == 128 && sizeof(TextRow) >= sizeof(MatRow), "a ro
 /* Neighbouring activities share their track, so process and thread (device and stream) are printed once for many: these
  * texts are made where the track changes, and are the text of one segment each. */
 enum : uint32_t { T_BODY = 0, T_FLOW, T_DEVICE, T_MEMSET, T_STREAM, T_COUNT };
-#define KTJ_WEAVE_TRACK_CHARS 25u  /* digits of both together that the longest of them has room for */
 
 /* descriptor of a segment: length of its text, number behind it, place of the text in units of sixteen bytes (in the
  * book, or among the track's texts) */
@@ -266,6 +265,17 @@ constexpr Chars count_chars(const Book& b) {
   return c;
 }
 constexpr Chars CHARS = count_chars(BOOK);
+constexpr bool tracks_fit(const Book& b) { /* with process or device of 22 bits and thread or stream of 47 */
+  uint32_t track[T_COUNT] = {};
+  for (uint32_t k = 0; k < N_PIECES; ++k) {
+    const uint32_t d = b.desc[KTJ_WREF_BASE(b.ref[R_PIECES]) + k], slot = KTJ_WD_SLOT(d);
+    track[k < 9 ? k / 3 : k < 11 ? 3 : 4] += KTJ_WD_LEN(d) + (slot == S_PID ? 7u : slot == S_TID ? 15u : 0u);
+  }
+  for (uint32_t k = 0; k < T_COUNT; ++k) if (track[k] > KTJ_WEAVE_LIT) return false;
+  return true;
+}
+static_assert(tracks_fit(BOOK), "a track's text is the text of one segment");
+static_assert(BOOK.n_text <= MAX_TEXT && BOOK.n_desc <= MAX_DESC, "the book's tables");
 #if defined(__HIP_DEVICE_COMPILE__)
 static __device__ constexpr Chars chars_table = CHARS;
 #else
