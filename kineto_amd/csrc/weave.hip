@@ -321,7 +321,7 @@ k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const u
       const uint64_t upto_first = first >= 60u ? ~0ull : (1ull << (first + 4u)) - 1ull;
       if (new_track & upto_first & ~track_seen) {
         const uint32_t low = __builtin_amdgcn_readlane((uint32_t)track, first), high = __builtin_amdgcn_readlane((uint32_t)(track >> 32), first);
-        track_made_high = KTJ_TR_TID_HIGH(__builtin_amdgcn_readlane(plan, first));
+        track_made_high = KTJ_TR_TID_HIGH((uint32_t)__builtin_amdgcn_readlane(plan, first)); /* (it gives an int) */
         track_made = (uint64_t)low | ((uint64_t)high << 32);
         track_lens = make_track(wv_lds, mine, low & ((1u << KTJ_TR_DEV_BITS) - 1u), (track_made >> KTJ_TR_DEV_BITS) | ((uint64_t)track_made_high << 42));
         track_seen = upto_first;
