@@ -231,6 +231,7 @@ struct ktj_engine {
   DevBuf s_dev_k, s_dev_r, s_dev_l, s_res_k, s_res_r, s_res_l;
   DevBuf keys_a, keys_b, vals_a, vals_b, hist, scan_tmp;
   bool rows_are_text = false;              /* of the last pass: TextRows in mat */
+  uint64_t not_woven = 0;                  /* number of records with which the last woven pass left too many activities (too_many_left) */
   bool some_left = false;                  /* the last pass had activities that the weaver leaves to emit_direct */
   DevBuf mat, schema_book, wide_text, len, len_sorted, kind_sorted, offs, out, tile_start;
   void* pinned_small = nullptr; size_t pinned_small_cap = 0;
@@ -1477,7 +1478,7 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
   const uint32_t cap_narrow = pow2_at_least((nx + nr) + (nx + nr) / 2), cap_cpu = pow2_at_least(2 * ng);
   /* Joined rows as text for the weaver, but where something reads them as they are, and where their 32 bytes more
    * would not fit the scratch array with as many records. */
-  const bool woven = n_coll == 0 && !e->noalloc && !e->no_weave && !(e->flags & KTJ_CREATE_TILE_EMIT);
+  const bool woven = n_coll == 0 && !e->noalloc && !e->no_weave && !(e->flags & KTJ_CREATE_TILE_EMIT) && (e->not_woven == 0 || e->not_woven != ng + nr + nd);
   e->rows_are_text = woven;
   const bool wide = woven && std::any_of(e->fields.begin(), e->fields.end(), [](const ktj_field& f) { return f.type == KTJ_F_F64; });
   e->pool_used = 0;
@@ -1580,7 +1581,7 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
   Table t_cpu{e->t_cpu.as<uint64_t>(), cap_cpu - 1, 1u, &sc->plan.ctl[KTJ_TBL_CPU]};
   FullCols fc{e->f_has_runtime.as<uint32_t>(), e->f_first.as<uint32_t>(), e->f_stream_src.as<uint32_t>(), e->f_pay.as<FullPay>()};
   NarrowCols nc{e->n_ext_src.as<uint32_t>(), e->n_kern_src.as<uint32_t>(), e->n_copy_src.as<uint32_t>(), e->n_pay.as<NarrowPay>()};
-  HIPCHK(plan_tables(tf, fc, tn, nc, t_cpu, (e->flags & KTJ_CREATE_HASH_JOIN) != 0, sc, st));
+  HIPCHK(plan_tables(tf, fc, tn, nc, t_cpu, (e->flags & KTJ_CREATE_HASH_JOIN) != 0, woven ? ng + nr + nd : 0u, sc, st));
   ApiTable api{e->d_cid_names.as<uint32_t>(), (uint32_t)e->cid_names.size(), e->d_flow_bits.as<uint32_t>(), e->malloc_cid};
   weave::SchemaBook* book = woven ? e->schema_book.as<weave::SchemaBook>() : nullptr;
   const Rows rows{e->mat.p, book, wide ? e->wide_text.as<weave::WideText>() : nullptr};
@@ -1660,6 +1661,7 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
       emitted = e->total_bytes + 64 <= text.out_cap;
       if (emitted) {
         e->some_left = e->scalars.n_left != 0;
+        if (woven) e->not_woven = too_many_left(e->scalars.n_left, e->scalars.n_valid) ? ng + nr + nd : 0u;
         if (woven && e->some_left && !others) {
           { const int rc = put_activities(0, e->scalars.n_left, prefix.size()); if (rc != KTJ_OK) return rc; }
           HIPCHK(hipEventRecord(e->ev[EV_EMIT], st));
@@ -1814,7 +1816,11 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
       HIPCHK(emit(mat, e->perm, e->offs.as<uint64_t>(), N, ctx, e->out.as<char>(), e->prefix_len, act_bytes, tile,
                   e->tile_start.as<uint32_t>(), st));
     else
-    { const int rc = put_activities(e->scalars.n_valid, e->scalars.n_left, e->prefix_len); if (rc != KTJ_OK) return rc; }
+    {
+      const int rc = put_activities(e->scalars.n_valid, e->scalars.n_left, e->prefix_len);
+      if (rc != KTJ_OK) return rc;
+      if (woven) e->not_woven = too_many_left(e->scalars.n_left, e->scalars.n_valid) ? ng + nr + nd : 0u;
+    }
   }
   HIPCHK(hipEventRecord(e->ev[EV_EMIT], st));
   HIPCHK(hipStreamSynchronize(st));

@@ -145,6 +145,7 @@ struct Scalars {
   unsigned int n_sync_rows;           /* distinct (device, row) pairs of Stream Sync activities */
   unsigned int n_plain;               /* small traces: activities that small_emit leaves to small_plain */
   unsigned int n_left;                /* activities that weave leaves to emit_direct */
+  unsigned int no_text;               /* leave them all (too_many_left) */
   unsigned int ext_ids_repeat;        /* two external-correlation records share a correlation id */
   unsigned long long emit_rows;       /* activities to format: n_valid, or none where the pass cannot end so */
   unsigned long long clock[KTJ_CLOCK_COUNT];
@@ -163,7 +164,8 @@ struct Scalars {
                                                                            [2t + 1] largest key of table t */
 };
 enum { KTJ_CNT_OUT_OF_RANGE = 0, KTJ_CNT_OUT_OF_ORDER, KTJ_CNT_FLOW, KTJ_CNT_LINKED, KTJ_CNT_BLANK_NAMES, KTJ_CNT_VALID,
-       KTJ_CNT_SYNC_TYPED, KTJ_CNT_COUNT };
+       KTJ_CNT_SYNC_TYPED, KTJ_CNT_COUNT,
+       KTJ_CNT_NOT_TEXT = KTJ_CNT_COUNT }; /* (not the host's) generic rows that can be no text rows, by their type or schema */
 #define KTJ_DEVERR_TABLE_FULL 1u         /* a join table sized from the record counts filled up (a defect) */
 #define KTJ_DEVERR_DISTINCT_DEVICES 2u   /* more distinct deviceId values than the rank set holds: the sort
                                             takes its slower path without ranks, no error reaches the caller */
@@ -255,7 +257,13 @@ hipError_t decode(DecodeJob job, Columns c, EmitCtx ctx, Scalars* sc, hipStream_
 
 /* ---- stage 2b: joins ---- */
 /* the tables' modes (direct unless force_hash or the span of their keys is too wide), and all of them cleared */
-hipError_t plan_tables(Table tf, FullCols fc, Table tn, NarrowCols nc, Table cpu, bool force_hash, Scalars* sc, hipStream_t st);
+/* n_rows: of all classes, in a pass that makes text rows (0: it makes none) */
+hipError_t plan_tables(Table tf, FullCols fc, Table tn, NarrowCols nc, Table cpu, bool force_hash, uint64_t n_rows, Scalars* sc, hipStream_t st);
+/* Whether the weaver prints nothing where it would leave n_left of n activities.  Each that it leaves ends what it
+ * has begun (a fifth of 120 000 CPU ops instant events: k_weave 43 us instead of 25), and the second launch takes 11 us and more;
+ * from 300 000 activities on it gains more than that as long as it leaves few. */
+#define KTJ_FEW_ACTIVITIES 262144u
+static inline __host__ __device__ bool too_many_left(uint64_t n_left, uint64_t n) { return n_left != 0 && (n <= KTJ_FEW_ACTIVITIES || n_left * 32u > n); }
 hipError_t build_cpu_ids(const ktj_generic_rec* g, uint64_t n, Table cpu, uint32_t* cpu_row, Scalars* sc, hipStream_t st);
 /* after build_cpu_ids: enters the external-correlation records and resolves their external ids */
 hipError_t build_extcorr(const ktj_extcorr_rec* e, uint64_t n, Table tn, NarrowCols nc, Table cpu, const uint32_t* cpu_row,

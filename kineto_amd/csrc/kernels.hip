@@ -196,7 +196,7 @@ k_begin(Scalars* s, FillJobs jobs, const char* blob, const uint64_t* off, uint32
       s->ts_min_biased = ~0ULL; s->ts_max_biased = 0;
       s->out_of_range = 0; s->out_of_order = 0; s->n_flow = 0; s->n_linked = 0; s->n_blank_names = 0; s->n_valid = 0;
       s->n_unresolved = 0; s->n_sync_typed = 0; s->n_device_orphans = 0; s->error = 0; s->have_stream_src = 0; s->n_dev_ranks = 0; s->n_res_ranks = 0; s->n_dense = 0; s->runtime_ids_repeat = 0;
-      s->n_queues = 0; s->n_sync_rows = 0; s->ext_ids_repeat = 0; s->n_plain = 0; s->n_left = 0;
+      s->n_queues = 0; s->n_sync_rows = 0; s->ext_ids_repeat = 0; s->n_plain = 0; s->n_left = 0; s->no_text = 0;
       s->sort.ts_bits = s->sort.res_bits = s->sort.key_bits = 0;
       for (int k = 0; k < KTJ_DONE_COUNT; ++k) s->done[k] = 0;
       for (uint32_t k = 0; k < KTJ_PART_SLOTS; ++k) s->part_done[k] = 0;
@@ -447,7 +447,12 @@ __global__ void __launch_bounds__(KTJ_BLOCK) k_decode(DecodeJob J, Columns c, Em
     /* rows that may need a Stream Sync row of their own are rare: the extra passes run only if any */
     const bool has = threadIdx.x < cnt, sync_typed = has && l[threadIdx.x].type == KTJ_TYPE_CUDA_SYNC;
     if (__syncthreads_or(sync_typed ? 1 : 0)) block_add(sc, KTJ_CNT_SYNC_TYPED, sync_typed ? 1u : 0u);
-    if (J.whole_pass) block_key_range(has, has ? (uint64_t)(int64_t)l[threadIdx.x].id : 0, sc, KTJ_TBL_CPU);
+    if (J.whole_pass) {
+      block_key_range(has, has ? (uint64_t)(int64_t)l[threadIdx.x].id : 0, sc, KTJ_TBL_CPU);
+      const bool no_text = has && (l[threadIdx.x].type == KTJ_TYPE_CPU_INSTANT_EVENT || is_counter_type(l[threadIdx.x].type) ||
+                                   (l[threadIdx.x].schema_id >= weave::MAX_SCHEMAS && l[threadIdx.x].schema_id < ctx.n_schemas));
+      if (__syncthreads_or(no_text ? 1 : 0)) block_add(sc, KTJ_CNT_NOT_TEXT, no_text ? 1u : 0u);
+    }
     if (has) store_cols(c, J.first + b * KTJ_BLOCK + threadIdx.x, cols_generic(l[threadIdx.x], ctx));
     return;
   }
@@ -521,7 +526,7 @@ __device__ __forceinline__ void clear_keys(const Table& t, const TableSpan& s, u
   if (at == 0) t.keys[t.mask + 1ull] = KTJ_EMPTY_KEY;
 }
 __global__ void __launch_bounds__(KTJ_BLOCK)
-k_plan_clear(Scalars* sc, Table tf, FullCols fc, Table tn, NarrowCols nc, Table cpu, int force_hash) {
+k_plan_clear(Scalars* sc, Table tf, FullCols fc, Table tn, NarrowCols nc, Table cpu, int force_hash, uint64_t n_rows) {
   __shared__ TableCtl ctl[3];
   if (blockIdx.x == 0 && threadIdx.x == 0) stage_clock(sc, KTJ_CLOCK_JOIN);
   if (threadIdx.x < 64) {
@@ -541,6 +546,11 @@ k_plan_clear(Scalars* sc, Table tf, FullCols fc, Table tn, NarrowCols nc, Table 
         ctl[k] = x;
         if (blockIdx.x == 0) { sc->plan.range[k].lo = lo; sc->plan.range[k].hi = hi; sc->plan.ctl[k] = x; }
       }
+    }
+    if (blockIdx.x == 0 && n_rows != 0) {
+      uint32_t n = (uint32_t)sc->shard[threadIdx.x][KTJ_CNT_NOT_TEXT];
+      for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o);
+      if (threadIdx.x == 0) sc->no_text = too_many_left(n, n_rows) ? 1u : 0u;
     }
   }
   __syncthreads();
@@ -565,12 +575,12 @@ k_plan_clear(Scalars* sc, Table tf, FullCols fc, Table tn, NarrowCols nc, Table 
     nc.ext_src[k] = 0; nc.kern_src[k] = 0; nc.copy_src[k] = 0; nc.pay[k] = z;
   }
 }
-hipError_t plan_tables(Table tf, FullCols fc, Table tn, NarrowCols nc, Table cpu, bool force_hash, Scalars* sc, hipStream_t st) {
+hipError_t plan_tables(Table tf, FullCols fc, Table tn, NarrowCols nc, Table cpu, bool force_hash, uint64_t n_rows, Scalars* sc, hipStream_t st) {
   uint64_t most = (uint64_t)tf.mask + 1;
   if ((uint64_t)tn.mask + 1 > most) most = (uint64_t)tn.mask + 1;
   if ((uint64_t)cpu.mask + 1 > most) most = (uint64_t)cpu.mask + 1;
   const unsigned g = grid_stride_for(most, KTJ_BLOCK * 4);
-  hipLaunchKernelGGL(k_plan_clear, dim3(g < 2048u ? g : 2048u), dim3(KTJ_BLOCK), 0, st, sc, tf, fc, tn, nc, cpu, force_hash ? 1 : 0);
+  hipLaunchKernelGGL(k_plan_clear, dim3(g < 2048u ? g : 2048u), dim3(KTJ_BLOCK), 0, st, sc, tf, fc, tn, nc, cpu, force_hash ? 1 : 0, n_rows);
   return KTJ_LAUNCH_CHECK();
 }
 
@@ -2191,7 +2201,7 @@ __device__ __forceinline__ uint32_t stage_row(const MatRow& m, const EmitCtx& ct
   weave::TextRow* const t = reinterpret_cast<weave::TextRow*>(stage) + threadIdx.x;
   uint32_t n, tail;
   if (!(m.meta & KTJ_M_VALID)) n = 0;
-  else if (weave::text_row(m, ctx, rows.schemas->plan, t, threadIdx.x & 7u, rows.wide, wide_at, &n, &tail)) return n | (tail << 30);
+  else if (sc->no_text == 0 && weave::text_row(m, ctx, rows.schemas->plan, t, threadIdx.x & 7u, rows.wide, wide_at, &n, &tail)) return n | (tail << 30);
   else n = row_length(m, ctx, sc) | (KTJ_KIND_LEFT << 30);
   static_assert(sizeof(MatRow) == 96, "six blocks");
   auto block = [&](uint32_t k) { __builtin_memcpy(t->w[k ^ (threadIdx.x & 7u)], reinterpret_cast<const char*>(&m) + 16u * k, 16); };

@@ -138,6 +138,7 @@ __device__ __forceinline__ uint64_t make_track(char* lds, uint32_t mine, uint64_
 __global__ void __launch_bounds__(WV_WAVES * 64u) __attribute__((amdgpu_waves_per_eu(4)))
 k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const uint8_t* kind_sorted, EmitCtx ctx, char* out, uint64_t prefix_len,
         const Scalars* sc, uint32_t rounds, const SchemaBook* schemas, const WideText* wide) {
+  if (sc->no_text) return;
   const uint32_t lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   static_assert(WV_BOOK_PLANS % 16u == 0 && sizeof(SchemaPlan) % 16u == 0, "in sixteens");
   for (uint32_t k = threadIdx.x; k < MAX_TEXT; k += blockDim.x) reinterpret_cast<uint4*>(wv_lds)[k] = reinterpret_cast<const uint4*>(g_book.text)[k];

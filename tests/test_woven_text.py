@@ -170,7 +170,8 @@ def test_doubles_as_text(sim):
 @pytest.mark.parametrize("n", (1, 3, 15, 16, 17, 40, 255, 257, 2053, 9001))
 def test_woven_documents_at_the_edges(n, other_types):
     """Through the large passes whatever the size; the document three times from one engine, so that later passes meet used buffers.
-    (Without other types there are threads of 47 bits among the text rows at most sizes.)"""
+    With other types the first pass leaves all activities to the other kernel, without them it leaves those with no room; the
+    second makes no text rows where too many had none."""
     from kineto_amd.engine import TraceEngine
     lib = abi.load_engine()
     sp = edge_stream(n, other_types)
