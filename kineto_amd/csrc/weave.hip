@@ -109,14 +109,16 @@ __device__ __forceinline__ void or_segment(char* buf, uint32_t p, uint32_t len, 
   }
 }
 extern __shared__ __attribute__((aligned(16))) char wv_lds[];
-/* the track's texts; their lengths, a byte each */
-__device__ __forceinline__ uint64_t make_track(char* lds, uint32_t mine, uint64_t dev, uint64_t thread) {
+/* the track's texts, with the lead of its times; their lengths, a byte each */
+__device__ __forceinline__ uint64_t make_track(char* lds, uint32_t mine, uint64_t dev, uint64_t thread, uint32_t lead) {
   const uint32_t lane = lane_id();
   char* const track = lds + mine + WV_TRACK_AT;
   if (lane < T_COUNT * 4u) *reinterpret_cast<uint4*>(track + lane * 16u) = make_uint4(0, 0, 0, 0);
   const Text pid = text_of(dev), tid = text_of(thread);
+  Text time = text_of(lead);
+  if (lead == 0) { time.lo = 0; time.n = 0; }
   const uint32_t desc = lane < N_PIECES ? *reinterpret_cast<const uint32_t*>(lds + WV_BOOK_DESC + (KTJ_WREF_BASE(g_book.ref[R_PIECES]) + lane) * 4u) : 0u;
-  const uint32_t len = KTJ_WD_LEN(desc), slot = KTJ_WD_SLOT(desc), n_num = slot == S_PID ? pid.n : slot == S_TID ? tid.n : 0u;
+  const uint32_t len = KTJ_WD_LEN(desc), slot = KTJ_WD_SLOT(desc), n_num = slot == S_PID ? pid.n : slot == S_TID ? tid.n : slot == S_LEAD ? time.n : 0u;
   const v4u32 zero = {0, 0, 0, 0};
   v4u32 a = zero, b = zero, num = zero;
   const v4u32* t = reinterpret_cast<const v4u32*>(lds) + KTJ_WD_UNIT(desc);
@@ -124,6 +126,7 @@ __device__ __forceinline__ uint64_t make_track(char* lds, uint32_t mine, uint64_
   if (len > 16u) b = t[1];
   if (slot == S_PID) { num.x = (uint32_t)pid.lo; num.y = (uint32_t)(pid.lo >> 32); num.z = (uint32_t)pid.hi; num.w = (uint32_t)(pid.hi >> 32); }
   if (slot == S_TID) { num.x = (uint32_t)tid.lo; num.y = (uint32_t)(tid.lo >> 32); num.z = (uint32_t)tid.hi; num.w = (uint32_t)(tid.hi >> 32); }
+  if (slot == S_LEAD) num.x = (uint32_t)time.lo, num.y = (uint32_t)(time.lo >> 32);
   const uint32_t end = dpp_add(len + n_num);
   /* pieces 0-2, 3-5, 6-8, 9-10, 11-12 are a text each */
   const uint32_t which = lane < 9u ? lane / 3u : lane < 11u ? 3u : 4u;
@@ -217,15 +220,20 @@ k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const u
     /* (the first lane's:) */
     const uint32_t plan = q0.w, name_off = WV_QUAD(q0.w, KTJ_TR_NAME), lens = WV_QUAD(q0.w, KTJ_TR_LENS), more = WV_QUAD(q0.w, KTJ_TR_MORE);
     const uint64_t track = (uint64_t)q1.z | ((uint64_t)q1.w << 32);
-    /* activities whose track is not that of the one before: a bit at the first lane of each */
+    /* the times' lead and the thread's upper bits */
+    uint32_t lead = KTJ_TR_LEAD_NIBBLE(q0.z) << (4u * h);
+    lead |= (uint32_t)__builtin_amdgcn_mov_dpp((int)lead, 0xB1, 0xF, 0xF, true); /* the quad's: its lanes 1 0 3 2, then 2 3 0 1 */
+    lead |= (uint32_t)__builtin_amdgcn_mov_dpp((int)lead, 0x4E, 0xF, 0xF, true);
+    const uint32_t track_high = KTJ_TR_TID_HIGH(plan) | (lead << 5);
+    /* activities whose track or lead is not that of the one before: a bit at the first lane of each */
     uint64_t new_track;
     {
       uint64_t before = __shfl_up((unsigned long long)track, 4);
-      uint32_t before_high = __shfl_up(KTJ_TR_TID_HIGH(plan), 4);
+      uint32_t before_high = __shfl_up(track_high, 4);
       if (lane == 0u) { before = track_made; before_high = track_made_high; }
-      new_track = __ballot(h == 0u && (track != before || KTJ_TR_TID_HIGH(plan) != before_high));
+      new_track = __ballot(h == 0u && (track != before || track_high != before_high));
     }
-    const v4u32 z = {q0.x, q0.y, q0.z & 0xFFFFFFu, q0.z & 0xFF000000u};
+    const v4u32 z = {q0.x, q0.y, q0.z & 0xFFFFFFu, KTJ_TR_COUNT(q0.z) << 24};
     vals[S_Z - 1u + h] = __builtin_bit_cast(v2u64, z);
     {
       const v4u32 a = {q1.x, q1.y & 0xFFFFFFu, 0u, q1.y & 0xFF000000u}, x = h == 0u ? a : q1;
@@ -322,9 +330,9 @@ k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const u
       const uint64_t upto_first = first >= 60u ? ~0ull : (1ull << (first + 4u)) - 1ull;
       if (new_track & upto_first & ~track_seen) {
         const uint32_t low = __builtin_amdgcn_readlane((uint32_t)track, first), high = __builtin_amdgcn_readlane((uint32_t)(track >> 32), first);
-        track_made_high = KTJ_TR_TID_HIGH((uint32_t)__builtin_amdgcn_readlane(plan, first)); /* (it gives an int) */
+        track_made_high = (uint32_t)__builtin_amdgcn_readlane(track_high, first);
         track_made = (uint64_t)low | ((uint64_t)high << 32);
-        track_lens = make_track(wv_lds, mine, low & ((1u << KTJ_TR_DEV_BITS) - 1u), (track_made >> KTJ_TR_DEV_BITS) | ((uint64_t)track_made_high << 42));
+        track_lens = make_track(wv_lds, mine, low & ((1u << KTJ_TR_DEV_BITS) - 1u), (track_made >> KTJ_TR_DEV_BITS) | ((uint64_t)(track_made_high & 31u) << 42), track_made_high >> 5);
         track_seen = upto_first;
       }
       if (!open) {

@@ -32,12 +32,17 @@ enum : uint32_t {
   S_RUN,                           /* the strings between the args and of the name, eight bytes each: place in the blob in units of sixteen bytes,
                                       length, place in LDS (0: it stays in the blob) */
   S_K,                             /* copy kind, in place of the first of them */
-  S_PID = S_TS, S_TID = S_DUR      /* in the pieces of the track's texts */
+  S_PID = S_TS, S_TID = S_DUR, S_LEAD = S_X /* in the pieces of the track's texts */
 };
 
 /* A joined row as the size pass leaves it for the weaver: a line of eight blocks of sixteen bytes.  Most numbers are
  * short: S_Z, S_EXT, S_FLOW and S_DUR have twelve bytes (eleven characters) of the first four blocks, whose last words are
- * plan, name, lens and more; S_A has eight of the fifth, in front of the track; the others a block each.  (Sixteen bytes
+ * plan, name, lens and more; S_A has eight of the fifth, in front of the track; the others a block each.
+ *
+ * A time has eighteen characters and more where the base lies months behind (libkineto floors it to 91 days) or at 0, more than
+ * S_TS has.  What is above 10^11 us (28 hours) is the same for nearly all rows: that number, the time's lead, is printed once
+ * for many, with the track's texts, and S_TS then has the eleven digits behind it with their zeros.  The lead's sixteen bits
+ * stand in the count bytes of the first four blocks, whose counts take four bits each.  (Sixteen bytes
  * for each number, 160 for a row: the size pass, whose rows wait in LDS, ran three instead of four wavefronts per SIMD,
  * 22 million records 1.32 + 0.70 + 0.15 ms instead of 1.15 + 0.57 + 0.13.) */
 struct alignas(16) TextRow { uint32_t w[8][4]; };
@@ -62,10 +67,13 @@ static_assert(sizeof(TextRow) == 128 && sizeof(TextRow) >= sizeof(MatRow), "a ro
 #define KTJ_TR_TAIL(x) (((x) >> 21) & 15u)     /* R_TAIL and the following */
 #define KTJ_TR_BETWEEN(x) (((x) >> 25) & 3u)   /* 1 string, 2 double in S_Y and S_Z, 3 double beside the row (WideText) */
 #define KTJ_TR_TID_HIGH(x) ((x) >> 27)
+#define KTJ_LEAD_UNIT 100000000000ull          /* us */
+#define KTJ_TR_LEAD_NIBBLE(w) ((w) >> 28)      /* of the third word of a block: the first block has the lead's lowest */
+#define KTJ_TR_COUNT(w) (((w) >> 24) & 15u)    /* of the same word */
 #define KTJ_TR_DEV_BITS 22u                    /* a track's process or device, and 42 of the thread's or stream's 47 bits */
 
-/* Neighbouring activities share their track, so process and thread (device and stream) are printed once for many: these
- * texts are made where the track changes, and are the text of one segment each. */
+/* Neighbouring activities share their track, so process and thread (device and stream), and the lead of the time behind
+ * them, are printed once for many: these texts are made where the track or the lead changes, and are the text of one segment each. */
 enum : uint32_t { T_BODY = 0, T_FLOW, T_DEVICE, T_MEMSET, T_STREAM, T_COUNT };
 
 /* descriptor of a segment: length of its text, number behind it, place of the text in units of sixteen bytes (in the
@@ -237,9 +245,10 @@ constexpr Book make_book() {
       ",\n    \"cat\": \"fwdbwd\",\n    \"name\": \"fwdbwd\"\n    , \"bp\": \"e\"\n  },"};
   for (uint32_t c = 0; c < 3; ++c)
     for (uint32_t f = 0; f < 5; ++f) b.part(R_TAIL + 5 * c + f, close[c], flow[f], last[f]);
-  /* the pieces of the track's texts, in their order: WN("u") stands for the process (device), WN("r") for the thread (stream) */
-  b.part(R_PIECES, "\",\n    \"pid\": " WN("u") ",\n    \"tid\": " WN("r") ",\n    \"ts\": ");
-  b.add(",\n    \"pid\": " WN("u") ",\n    \"tid\": " WN("r") ",\n    \"ts\": "); b.flush();
+  /* the pieces of the track's texts, in their order: WN("u") stands for the process (device), WN("r") for the thread (stream),
+   * WN("x") for the time's lead */
+  b.part(R_PIECES, "\",\n    \"pid\": " WN("u") ",\n    \"tid\": " WN("r") ",\n    \"ts\": " WN("x"));
+  b.add(",\n    \"pid\": " WN("u") ",\n    \"tid\": " WN("r") ",\n    \"ts\": " WN("x"));
   b.add("\"device\": " WN("u") ", \"stream\": " WN("r") ", \"hsa_queue\": "); b.flush();
   b.add("\"device\": " WN("u") ", \"context\": "); b.flush();
   b.add(", \"stream\": " WN("r") ", \"correlation\": "); b.flush();
@@ -249,13 +258,14 @@ constexpr Book make_book() {
 static_assert(KTJ_COPY_H2H == 1 && KTJ_COPY_D2D == 4, "the directions' names are in this order");
 
 constexpr Book BOOK = make_book();
-/* characters of the parts' texts, the track's without their two numbers */
-struct Chars { uint32_t of[R_COUNT]; };
+/* characters of the parts' texts, the track's without their numbers; and of these by themselves */
+struct Chars { uint32_t of[R_COUNT], track[T_COUNT]; };
 constexpr Chars count_chars(const Book& b) {
   Chars c{};
   uint32_t track[T_COUNT] = {}; /* pieces 0-2, 3-5, 6-8, 9-10, 11-12 are a text each */
   for (uint32_t k = 0; k < N_PIECES; ++k)
     track[k < 9 ? k / 3 : k < 11 ? 3 : 4] += KTJ_WD_LEN(b.desc[KTJ_WREF_BASE(b.ref[R_PIECES]) + k]);
+  for (uint32_t k = 0; k < T_COUNT; ++k) c.track[k] = track[k];
   for (uint32_t r = 0; r < R_COUNT; ++r)
     for (uint32_t k = 0; k < KTJ_WREF_COUNT(b.ref[r]); ++k) {
       const uint32_t i = KTJ_WREF_BASE(b.ref[r]) + k;
@@ -265,7 +275,7 @@ constexpr Chars count_chars(const Book& b) {
   return c;
 }
 constexpr Chars CHARS = count_chars(BOOK);
-constexpr bool tracks_fit(const Book& b) { /* with process or device of 22 bits and thread or stream of 47 */
+constexpr bool tracks_fit(const Book& b) { /* with process or device of 22 bits and thread or stream of 47, and no lead */
   uint32_t track[T_COUNT] = {};
   for (uint32_t k = 0; k < N_PIECES; ++k) {
     const uint32_t d = b.desc[KTJ_WREF_BASE(b.ref[R_PIECES]) + k], slot = KTJ_WD_SLOT(d);
@@ -275,6 +285,8 @@ constexpr bool tracks_fit(const Book& b) { /* with process or device of 22 bits 
   return true;
 }
 static_assert(tracks_fit(BOOK), "a track's text is the text of one segment");
+/* characters that process, thread and lead may have together */
+constexpr uint32_t TRACK_ROOM = KTJ_WEAVE_LIT - (CHARS.track[T_BODY] > CHARS.track[T_FLOW] ? CHARS.track[T_BODY] : CHARS.track[T_FLOW]);
 static_assert(BOOK.n_text <= MAX_TEXT && BOOK.n_desc <= MAX_DESC, "the book's tables");
 #if defined(__HIP_DEVICE_COMPILE__)
 static __device__ constexpr Chars chars_table = CHARS;
@@ -470,11 +482,21 @@ KTJ_HD KTJ_FI inline Text three_text_of(uint64_t a, uint64_t b, uint64_t c) {
   append_next(t, c);
   return t;
 }
+KTJ_HD KTJ_FI inline uint64_t whole_us(int64_t ns) { return ((uint64_t)ns >> 35) == 0 ? (uint32_t)((uint64_t)ns >> 3) / 125u : (uint64_t)ns / 1000u; }
 KTJ_HD KTJ_FI inline Text time_text_of(int64_t ns) { /* put_ts */
-  uint64_t us;
-  if (((uint64_t)ns >> 35) == 0) us = (uint32_t)((uint64_t)ns >> 3) / 125u; else us = (uint64_t)ns / 1000u;
+  const uint64_t us = whole_us(ns);
   Text t = text_of(us);
   append(t, (ascii4((uint32_t)ns - (uint32_t)us * 1000u) & 0xFFFFFF00u) | (uint32_t)'.', 4);
+  return t;
+}
+/* the same behind a lead: always fifteen characters */
+KTJ_HD KTJ_FI inline Text time_text_behind(int64_t ns, uint32_t lead) {
+  const uint64_t us = whole_us(ns), low = us - lead * KTJ_LEAD_UNIT;
+  const uint32_t high8 = (uint32_t)(low / 1000u);
+  Text t;
+  t.lo = ascii8(high8);
+  t.hi = (uint64_t)((ascii4((uint32_t)low - high8 * 1000u) >> 8) | ((uint32_t)'.' << 24)) | ((uint64_t)(ascii4((uint32_t)ns - (uint32_t)us * 1000u) >> 8) << 32);
+  t.n = 15u;
   return t;
 }
 /* up to 24 characters, zeros behind them */
@@ -591,10 +613,20 @@ KTJ_HD KTJ_FI inline bool text_row(const MatRow& m, const EmitCtx& c, const Sche
   if ((tid >> 47) != 0 || (device && m.res < 0)) return false;
   if (type >= 29u || (generic && (type == KTJ_TYPE_CPU_INSTANT_EVENT || is_counter_type(type)))) return false;
   if ((meta & KTJ_M_SYNC) || (type == KTJ_TYPE_GPU_USER_ANNOTATION && flow) || collective_of(m) != 0) return false;
+  /* the time and its lead */
+  const bool wider = type == KTJ_TYPE_GPU_USER_ANNOTATION;
+  int64_t rel = m.ts - (wider ? 1 : 0) - c.base_time_ns;
+  if (rel < 0) rel = 0;
+  uint32_t lead = 0;
+  if ((uint64_t)rel >= KTJ_LEAD_UNIT * 1000u) {
+    lead = (uint32_t)(((uint64_t)rel / 1000u) / KTJ_LEAD_UNIT);
+    if (lead > 0xFFFFu) return false;
+  }
   bool fits = true;
   auto block = [&](uint32_t slot) KTJ_FI { return r->w[KTJ_TR_BLOCK(slot) ^ turn]; };
   typedef uint64_t __attribute__((may_alias)) word_pair;
   auto two = [](uint32_t* w, uint64_t x) KTJ_FI { *reinterpret_cast<word_pair*>(w) = x; }; /* (eight-byte aligned) */
+  auto nibble = [&](uint32_t slot) KTJ_FI { return (lead >> (4u * (slot - S_Z))) << 28; };
   auto put = [&](uint32_t slot, const Text& t) KTJ_FI {
     uint32_t* const w = block(slot);
     const uint32_t most = slot == S_A ? 7u : slot >= S_Z ? 11u : 15u;
@@ -602,7 +634,7 @@ KTJ_HD KTJ_FI inline bool text_row(const MatRow& m, const EmitCtx& c, const Sche
     if (slot == S_A) two(w, t.lo | ((uint64_t)t.n << 56));
     else {
       two(w, t.lo);
-      if (slot >= S_Z) w[2] = (uint32_t)t.hi | (t.n << 24);
+      if (slot >= S_Z) w[2] = (uint32_t)t.hi | (t.n << 24) | nibble(slot);
       else two(w + 2, t.hi | ((uint64_t)t.n << 56));
     }
     return t.n;
@@ -622,14 +654,21 @@ KTJ_HD KTJ_FI inline bool text_row(const MatRow& m, const EmitCtx& c, const Sche
     const LongText t = real_text(bits);
     if (here) {
       two(block(S_Y), t.w[0]); two(block(S_Y) + 2, t.w[1]);
-      two(block(S_Z), t.w[2]); block(S_Z)[2] = 0;
+      two(block(S_Z), t.w[2]);
     } else {
       wide[wide_at].w[0] = t.w[0]; wide[wide_at].w[1] = t.w[1]; wide[wide_at].w[2] = t.w[2]; wide[wide_at].w[3] = 0;
     }
     return t.n;
   };
   block(S_Y)[3] = 0; /* (its last byte is not KTJ_ROW_LEFT) */
-  uint32_t n = 0; /* the length, but for the strings */
+  block(S_Z)[2] = nibble(S_Z); block(S_EXT)[2] = nibble(S_EXT); block(S_FLOW)[2] = nibble(S_FLOW); /* (also where the number is none) */
+  uint32_t n; /* the length, but for the strings; to begin with that of the times and the track (first, so that only the lead stays in a register) */
+  {
+    const uint32_t track = (uint32_t)(ndigits_u64((uint64_t)m.dev) + ndigits_u64(tid)), lead_chars = lead ? (uint32_t)ndigits_u64(lead) : 0u;
+    if (track + lead_chars > TRACK_ROOM) return false;
+    const uint32_t k = put(S_TS, lead ? time_text_behind(rel, lead) : time_text_of(rel)) + lead_chars;
+    n = track * (1u + (device ? 1u : 0u) + (flow ? 1u : 0u)) + (flow ? 2u * k : k);
+  }
   /* the name */
   uint32_t name = KTJ_TR_NAME_RUN, name_len = 0, at_name = 0, len1 = 0, at_more = 0, between = 0, args = KTJ_TR_NO_ARGS, close = 5u;
   if (meta & KTJ_M_NAME_BUILTIN) {
@@ -734,14 +773,7 @@ KTJ_HD KTJ_FI inline bool text_row(const MatRow& m, const EmitCtx& c, const Sche
     }
   }
   if (name_len > KTJ_WEAVE_MAX_RUN || len1 > KTJ_WEAVE_MAX_RUN) return false;
-  /* the times, the External id, the track */
-  const bool wider = type == KTJ_TYPE_GPU_USER_ANNOTATION;
-  int64_t rel = m.ts - (wider ? 1 : 0) - c.base_time_ns;
-  if (rel < 0) rel = 0;
-  {
-    const uint32_t k = put(S_TS, time_text_of(rel));
-    n += flow ? 2u * k : k;
-  }
+  /* the duration, the External id */
   n += put(S_DUR, time_text_of((m.dur < 0 ? 0 : m.dur) + (wider ? 2 : 0)));
   uint32_t body = 0;
   if (m.ext != 0) {
@@ -753,8 +785,6 @@ KTJ_HD KTJ_FI inline bool text_row(const MatRow& m, const EmitCtx& c, const Sche
     n += frag ? chars_of<R_BODY_ARGS>() : chars_of<R_BODY_NONE>();
     body = frag ? 1u : 0u;
   }
-  const uint32_t track = (uint32_t)(ndigits_u64((uint64_t)m.dev) + ndigits_u64(tid));
-  n += track * (1u + (device ? 1u : 0u) + (flow ? 1u : 0u));
   const uint32_t last = close + (flow ? (meta & KTJ_M_FLOW_START ? 1u : 2u) + (meta & KTJ_M_FLOW_FWDBWD ? 2u : 0u) : 0u);
   n += chars_table.of[R_TAIL + last];
   block(S_Z)[3] = type | (name << 5) | (body << 12) | (args << 14) | (last << 21) | (between << 25) | ((uint32_t)(tid >> 42) << 27);

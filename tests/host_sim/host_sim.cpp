@@ -101,13 +101,15 @@ std::string woven_text(const weave::TextRow& row, const weave::WideText* wide, c
   auto number = [&](uint32_t slot) -> std::string {
     const uint32_t* w = row.w[KTJ_TR_BLOCK(slot)];
     if (slot == S_A) return std::string(reinterpret_cast<const char*>(w), w[1] >> 24);
-    return std::string(reinterpret_cast<const char*>(w), w[slot >= S_Z ? 2 : 3] >> 24);
+    return std::string(reinterpret_cast<const char*>(w), slot >= S_Z ? KTJ_TR_COUNT(w[2]) : w[3] >> 24);
   };
   const uint32_t plan = row.w[KTJ_TR_PLAN][3], lens = row.w[KTJ_TR_LENS][3], more = row.w[KTJ_TR_MORE][3], name = row.w[KTJ_TR_NAME][3];
   uint64_t track;
   memcpy(&track, &row.w[KTJ_TR_BLOCK(S_A)][2], 8);
   const std::string pid = std::to_string(track & ((1u << KTJ_TR_DEV_BITS) - 1u));
   const std::string tid = std::to_string((track >> KTJ_TR_DEV_BITS) | ((uint64_t)KTJ_TR_TID_HIGH(plan) << 42));
+  uint32_t lead = 0;
+  for (uint32_t k = 0; k < 4; ++k) lead |= KTJ_TR_LEAD_NIBBLE(row.w[k][2]) << (4 * k);
   auto text = [&](uint32_t d) {
     const uint32_t unit = KTJ_WD_UNIT(d);
     const uint32_t* t = unit >= SCHEMA_UNIT ? book.text + (unit - SCHEMA_UNIT) * 4 : b.text + unit * 4;
@@ -120,6 +122,7 @@ std::string woven_text(const weave::TextRow& row, const weave::WideText* wide, c
     t += text(d);
     if (KTJ_WD_SLOT(d) == S_PID) t += pid;
     if (KTJ_WD_SLOT(d) == S_TID) t += tid;
+    if (KTJ_WD_SLOT(d) == S_LEAD && lead) t += std::to_string(lead);
   }
   for (const std::string& t : track_text) if (t.size() > KTJ_WEAVE_LIT) return "a track's text is longer than a segment";
   auto part = [&](uint32_t ref) {

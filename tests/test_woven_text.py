@@ -143,6 +143,44 @@ def test_segments_of_every_kind_of_row(sim):
     assert woven > 1800 and left > 300, (woven, left)
 
 
+HOUR, DAY, LEAD = 3600 * 10**9, 86400 * 10**9, 10**14   # ns; a time's lead counts the last
+
+
+def _base_back(sp, ns):
+    """The same records ns further behind the base of the times."""
+    sp.contents.base_time_ns -= ns
+    return sp
+
+
+@pytest.mark.parametrize("back", (27 * HOUR, 28 * HOUR, LEAD - 10**9, LEAD - 1, LEAD, 62 * DAY, 91 * DAY, 10 * LEAD - 10**9, B))
+def test_times_long_behind_the_base(sim, back):
+    """libkineto's base is the clock floored to 91 days; B: a base of 0.  Times of twelve digits and more are text rows as any, the
+    carry into another lead inside the trace too."""
+    for cfg in range(1, 6):
+        sp, release = abi.synth_stream(cfg, 2000, host_name="box")
+        assert _woven_vs_oracle(sim, _base_back(sp, back))[1] == 0, cfg
+        release()
+    at_base = _woven_vs_oracle(sim, edge_stream(3000, False))
+    left = _woven_vs_oracle(sim, _base_back(edge_stream(3000, False), back))[1]
+    assert left <= at_base[1] + 60, (left, at_base)   # a track of 22 digits has no room for five more
+
+
+def test_leads_with_no_room_are_left(sim):
+    """Process, thread and lead share the room that the segment of their text has; a lead has sixteen bits."""
+    def stream(base, pid, tid):
+        b = StreamBuilder(base=base, window=(B, B + 10**13), host_name="edge")
+        for k in range(3):
+            b.add_generic("op", 0, B + 1000 + 2000 * k, B + 2000 + 2000 * k, pid, tid, id=k + 1)
+        return b.build()
+    pid, tid = 4194303, (1 << 47) - 1
+    assert _woven_vs_oracle(sim, stream(B, pid, tid)) == (3, 0)
+    assert _woven_vs_oracle(sim, stream(B - 999 * LEAD, pid, tid)) == (3, 0)
+    assert _woven_vs_oracle(sim, stream(B - 1000 * LEAD, pid, tid)) == (0, 3)
+    assert _woven_vs_oracle(sim, stream(B - 1000 * LEAD, pid // 10, tid)) == (3, 0)
+    assert _woven_vs_oracle(sim, stream(B - 65535 * LEAD, pid, tid // 100)) == (3, 0)
+    assert _woven_vs_oracle(sim, stream(B - 65536 * LEAD, 1, 1)) == (0, 3)
+
+
 def test_doubles_as_text(sim):
     """Shifted together, against the formatter's characters one by one: zeros behind the text, too."""
     import random
@@ -165,6 +203,35 @@ def test_doubles_as_text(sim):
         assert got.raw[n:24] == bytes(24 - n), v
 
 
+def _gpu_vs_oracle(sp, passes=3):
+    """Through the large passes whatever the size, several times from one engine."""
+    from kineto_amd.engine import TraceEngine
+    lib = abi.load_engine()
+    o = og.OracleRun(sp)
+    want = o.output()
+    o.close()
+    lib.ktj_debug_force_sort_passes(1)
+    try:
+        with TraceEngine(sp.contents.trace_name.decode(), base_time_ns=sp.contents.base_time_ns) as e:
+            e.submit_stream(sp)
+            for _ in range(passes):
+                e.process()
+                assert e.output() == want
+    finally:
+        lib.ktj_debug_force_sort_passes(0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("back", (28 * HOUR, LEAD - 10**9, LEAD - 2001 * 1000, 62 * DAY, B))
+def test_woven_documents_long_behind_the_base(back):
+    """Times with a lead, and (the second and third) its carry between activities of one track and one turn."""
+    _gpu_vs_oracle(_base_back(edge_stream(2053, False), back))
+    for cfg in (2, 3):
+        sp, release = abi.synth_stream(cfg, 3001, host_name="box")
+        _gpu_vs_oracle(_base_back(sp, back), passes=2)
+        release()
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("other_types", (False, True))
 @pytest.mark.parametrize("n", (1, 3, 15, 16, 17, 40, 255, 257, 2053, 9001))
@@ -172,19 +239,4 @@ def test_woven_documents_at_the_edges(n, other_types):
     """Through the large passes whatever the size; the document three times from one engine, so that later passes meet used buffers.
     With other types the first pass leaves all activities to the other kernel, without them it leaves those with no room; the
     second makes no text rows where too many had none."""
-    from kineto_amd.engine import TraceEngine
-    lib = abi.load_engine()
-    sp = edge_stream(n, other_types)
-    o = og.OracleRun(sp)
-    want = o.output()
-    o.close()
-    lib.ktj_debug_force_sort_passes(1)
-    try:
-        e = TraceEngine(sp.contents.trace_name.decode())
-        e.submit_stream(sp)
-        for _ in range(3):
-            e.process()
-            assert e.output() == want
-        e.close()
-    finally:
-        lib.ktj_debug_force_sort_passes(0)
+    _gpu_vs_oracle(edge_stream(n, other_types))
