@@ -221,10 +221,13 @@ k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const u
     const uint32_t plan = q0.w, name_off = WV_QUAD(q0.w, KTJ_TR_NAME), lens = WV_QUAD(q0.w, KTJ_TR_LENS), more = WV_QUAD(q0.w, KTJ_TR_MORE);
     const uint64_t track = (uint64_t)q1.z | ((uint64_t)q1.w << 32);
     /* the times' lead and the thread's upper bits */
-    uint32_t lead = KTJ_TR_LEAD_NIBBLE(q0.z) << (4u * h);
-    lead |= (uint32_t)__builtin_amdgcn_mov_dpp((int)lead, 0xB1, 0xF, 0xF, true); /* the quad's: its lanes 1 0 3 2, then 2 3 0 1 */
-    lead |= (uint32_t)__builtin_amdgcn_mov_dpp((int)lead, 0x4E, 0xF, 0xF, true);
-    const uint32_t track_high = KTJ_TR_TID_HIGH(plan) | (lead << 5);
+    uint32_t track_high = KTJ_TR_TID_HIGH(plan);
+    if (__any((lens & KTJ_TR_HAS_LEAD) != 0)) {
+      uint32_t lead = KTJ_TR_LEAD_NIBBLE(q0.z) << (4u * h);
+      lead |= (uint32_t)__builtin_amdgcn_mov_dpp((int)lead, 0xB1, 0xF, 0xF, true); /* the quad's: its lanes 1 0 3 2, then 2 3 0 1 */
+      lead |= (uint32_t)__builtin_amdgcn_mov_dpp((int)lead, 0x4E, 0xF, 0xF, true);
+      if (lens & KTJ_TR_HAS_LEAD) track_high |= lead << 5;
+    }
     /* activities whose track or lead is not that of the one before: a bit at the first lane of each */
     uint64_t new_track;
     {
@@ -241,7 +244,7 @@ k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const u
     }
     /* how many segments and parts, and the room for the name (the first lane) */
     uint32_t counts = 0, units = 0, args_ref = 0, args2_ref = 0;
-    const uint32_t len0 = lens & 0xFFFFu, len1 = lens >> 16;
+    const uint32_t len0 = lens & 0xFFFFu, len1 = KTJ_TR_LEN1(lens);
     if (h == 0u && mine_ok) {
       const uint32_t a = KTJ_TR_ARGS(plan);
       if (a >= KTJ_TR_SCHEMA) {

@@ -41,8 +41,11 @@ enum : uint32_t {
  *
  * A time has eighteen characters and more where the base lies months behind (libkineto floors it to 91 days) or at 0, more than
  * S_TS has.  What is above 10^11 us (28 hours) is the same for nearly all rows: that number, the time's lead, is printed once
- * for many, with the track's texts, and S_TS then has the eleven digits behind it with their zeros.  The lead's sixteen bits
- * stand in the count bytes of the first four blocks, whose counts take four bits each.  (Sixteen bytes
+ * for many, with the track's texts, and S_TS then has the eleven digits behind it with their zeros.  Where a row has a lead, its
+ * sixteen bits stand in the count bytes of the first four blocks, whose counts take four bits each.  (In every row, without
+ * the bit that says so: size pass of 22 million records 27 us longer.)
+ *
+ * (Sixteen bytes
  * for each number, 160 for a row: the size pass, whose rows wait in LDS, ran three instead of four wavefronts per SIMD,
  * 22 million records 1.32 + 0.70 + 0.15 ms instead of 1.15 + 0.57 + 0.13.) */
 struct alignas(16) TextRow { uint32_t w[8][4]; };
@@ -52,8 +55,9 @@ struct alignas(16) WideText { uint64_t w[4]; };
 #define KTJ_TR_BLOCK(slot) (((slot) + 3u) & 7u)
 #define KTJ_TR_PLAN 0u             /* KTJ_TR_*, the thread's bits from 42 on */
 #define KTJ_TR_NAME 1u             /* place of the name in its blob, in units of sixteen bytes */
-#define KTJ_TR_LENS 2u             /* its length; << 16: that of the string or double between the args' parts */
+#define KTJ_TR_LENS 2u             /* its length; << 16: that of the string or double between the args' parts; KTJ_TR_HAS_LEAD */
 #define KTJ_TR_MORE 3u             /* the string's place in its blob; the WideText's number; a copy's kind as text */
+static_assert(KTJ_WEAVE_MAX_RUN < 0x8000u, "a length and a bit");
 static_assert(sizeof(TextRow) == 128 && sizeof(TextRow) >= sizeof(MatRow), "a row that is left to format_activity is a MatRow in the same place");
 /* a row of the other kind: the last byte, S_Y's count of characters otherwise */
 #define KTJ_ROW_LEFT 0xFFu
@@ -68,6 +72,8 @@ static_assert(sizeof(TextRow) == 128 && sizeof(TextRow) >= sizeof(MatRow), "a ro
 #define KTJ_TR_BETWEEN(x) (((x) >> 25) & 3u)   /* 1 string, 2 double in S_Y and S_Z, 3 double beside the row (WideText) */
 #define KTJ_TR_TID_HIGH(x) ((x) >> 27)
 #define KTJ_LEAD_UNIT 100000000000ull          /* us */
+#define KTJ_TR_HAS_LEAD (1u << 31)
+#define KTJ_TR_LEN1(lens) (((lens) >> 16) & 0x7FFFu)
 #define KTJ_TR_LEAD_NIBBLE(w) ((w) >> 28)      /* of the third word of a block: the first block has the lead's lowest */
 #define KTJ_TR_COUNT(w) (((w) >> 24) & 15u)    /* of the same word */
 #define KTJ_TR_DEV_BITS 22u                    /* a track's process or device, and 42 of the thread's or stream's 47 bits */
@@ -482,20 +488,19 @@ KTJ_HD KTJ_FI inline Text three_text_of(uint64_t a, uint64_t b, uint64_t c) {
   append_next(t, c);
   return t;
 }
-KTJ_HD KTJ_FI inline uint64_t whole_us(int64_t ns) { return ((uint64_t)ns >> 35) == 0 ? (uint32_t)((uint64_t)ns >> 3) / 125u : (uint64_t)ns / 1000u; }
 KTJ_HD KTJ_FI inline Text time_text_of(int64_t ns) { /* put_ts */
-  const uint64_t us = whole_us(ns);
+  uint64_t us;
+  if (((uint64_t)ns >> 35) == 0) us = (uint32_t)((uint64_t)ns >> 3) / 125u; else us = (uint64_t)ns / 1000u;
   Text t = text_of(us);
   append(t, (ascii4((uint32_t)ns - (uint32_t)us * 1000u) & 0xFFFFFF00u) | (uint32_t)'.', 4);
   return t;
 }
-/* the same behind a lead: always fifteen characters */
-KTJ_HD KTJ_FI inline Text time_text_behind(int64_t ns, uint32_t lead) {
-  const uint64_t us = whole_us(ns), low = us - lead * KTJ_LEAD_UNIT;
-  const uint32_t high8 = (uint32_t)(low / 1000u);
+/* what stands behind a lead: always fifteen characters */
+KTJ_HD KTJ_FI inline Text time_text_behind(uint64_t us, uint32_t ns) {
+  const uint32_t high8 = (uint32_t)(us / 1000u);
   Text t;
   t.lo = ascii8(high8);
-  t.hi = (uint64_t)((ascii4((uint32_t)low - high8 * 1000u) >> 8) | ((uint32_t)'.' << 24)) | ((uint64_t)(ascii4((uint32_t)ns - (uint32_t)us * 1000u) >> 8) << 32);
+  t.hi = (uint64_t)((ascii4((uint32_t)us - high8 * 1000u) >> 8) | ((uint32_t)'.' << 24)) | ((uint64_t)(ascii4(ns) >> 8) << 32);
   t.n = 15u;
   return t;
 }
@@ -613,20 +618,10 @@ KTJ_HD KTJ_FI inline bool text_row(const MatRow& m, const EmitCtx& c, const Sche
   if ((tid >> 47) != 0 || (device && m.res < 0)) return false;
   if (type >= 29u || (generic && (type == KTJ_TYPE_CPU_INSTANT_EVENT || is_counter_type(type)))) return false;
   if ((meta & KTJ_M_SYNC) || (type == KTJ_TYPE_GPU_USER_ANNOTATION && flow) || collective_of(m) != 0) return false;
-  /* the time and its lead */
-  const bool wider = type == KTJ_TYPE_GPU_USER_ANNOTATION;
-  int64_t rel = m.ts - (wider ? 1 : 0) - c.base_time_ns;
-  if (rel < 0) rel = 0;
-  uint32_t lead = 0;
-  if ((uint64_t)rel >= KTJ_LEAD_UNIT * 1000u) {
-    lead = (uint32_t)(((uint64_t)rel / 1000u) / KTJ_LEAD_UNIT);
-    if (lead > 0xFFFFu) return false;
-  }
   bool fits = true;
   auto block = [&](uint32_t slot) KTJ_FI { return r->w[KTJ_TR_BLOCK(slot) ^ turn]; };
   typedef uint64_t __attribute__((may_alias)) word_pair;
   auto two = [](uint32_t* w, uint64_t x) KTJ_FI { *reinterpret_cast<word_pair*>(w) = x; }; /* (eight-byte aligned) */
-  auto nibble = [&](uint32_t slot) KTJ_FI { return (lead >> (4u * (slot - S_Z))) << 28; };
   auto put = [&](uint32_t slot, const Text& t) KTJ_FI {
     uint32_t* const w = block(slot);
     const uint32_t most = slot == S_A ? 7u : slot >= S_Z ? 11u : 15u;
@@ -634,7 +629,7 @@ KTJ_HD KTJ_FI inline bool text_row(const MatRow& m, const EmitCtx& c, const Sche
     if (slot == S_A) two(w, t.lo | ((uint64_t)t.n << 56));
     else {
       two(w, t.lo);
-      if (slot >= S_Z) w[2] = (uint32_t)t.hi | (t.n << 24) | nibble(slot);
+      if (slot >= S_Z) w[2] = (uint32_t)t.hi | (t.n << 24);
       else two(w + 2, t.hi | ((uint64_t)t.n << 56));
     }
     return t.n;
@@ -654,21 +649,14 @@ KTJ_HD KTJ_FI inline bool text_row(const MatRow& m, const EmitCtx& c, const Sche
     const LongText t = real_text(bits);
     if (here) {
       two(block(S_Y), t.w[0]); two(block(S_Y) + 2, t.w[1]);
-      two(block(S_Z), t.w[2]);
+      two(block(S_Z), t.w[2]); block(S_Z)[2] = 0;
     } else {
       wide[wide_at].w[0] = t.w[0]; wide[wide_at].w[1] = t.w[1]; wide[wide_at].w[2] = t.w[2]; wide[wide_at].w[3] = 0;
     }
     return t.n;
   };
   block(S_Y)[3] = 0; /* (its last byte is not KTJ_ROW_LEFT) */
-  block(S_Z)[2] = nibble(S_Z); block(S_EXT)[2] = nibble(S_EXT); block(S_FLOW)[2] = nibble(S_FLOW); /* (also where the number is none) */
-  uint32_t n; /* the length, but for the strings; to begin with that of the times and the track (first, so that only the lead stays in a register) */
-  {
-    const uint32_t track = (uint32_t)(ndigits_u64((uint64_t)m.dev) + ndigits_u64(tid)), lead_chars = lead ? (uint32_t)ndigits_u64(lead) : 0u;
-    if (track + lead_chars > TRACK_ROOM) return false;
-    const uint32_t k = put(S_TS, lead ? time_text_behind(rel, lead) : time_text_of(rel)) + lead_chars;
-    n = track * (1u + (device ? 1u : 0u) + (flow ? 1u : 0u)) + (flow ? 2u * k : k);
-  }
+  uint32_t n = 0; /* the length, but for the strings */
   /* the name */
   uint32_t name = KTJ_TR_NAME_RUN, name_len = 0, at_name = 0, len1 = 0, at_more = 0, between = 0, args = KTJ_TR_NO_ARGS, close = 5u;
   if (meta & KTJ_M_NAME_BUILTIN) {
@@ -773,7 +761,24 @@ KTJ_HD KTJ_FI inline bool text_row(const MatRow& m, const EmitCtx& c, const Sche
     }
   }
   if (name_len > KTJ_WEAVE_MAX_RUN || len1 > KTJ_WEAVE_MAX_RUN) return false;
-  /* the duration, the External id */
+  /* the times, the External id, the track */
+  const bool wider = type == KTJ_TYPE_GPU_USER_ANNOTATION;
+  int64_t rel = m.ts - (wider ? 1 : 0) - c.base_time_ns;
+  if (rel < 0) rel = 0;
+  const uint32_t track = (uint32_t)(ndigits_u64((uint64_t)m.dev) + ndigits_u64(tid));
+  uint32_t lead = 0;
+  {
+    uint32_t k;
+    if ((uint64_t)rel < KTJ_LEAD_UNIT * 1000u) k = put(S_TS, time_text_of(rel));
+    else {
+      const uint64_t us = (uint64_t)rel / 1000u, all = us / KTJ_LEAD_UNIT;
+      lead = (uint32_t)all;
+      const uint32_t chars = (uint32_t)ndigits_u64(lead);
+      if (all > 0xFFFFu || track + chars > TRACK_ROOM) return false;
+      k = put(S_TS, time_text_behind(us - all * KTJ_LEAD_UNIT, (uint32_t)rel - (uint32_t)us * 1000u)) + chars;
+    }
+    n += flow ? 2u * k : k;
+  }
   n += put(S_DUR, time_text_of((m.dur < 0 ? 0 : m.dur) + (wider ? 2 : 0)));
   uint32_t body = 0;
   if (m.ext != 0) {
@@ -785,11 +790,16 @@ KTJ_HD KTJ_FI inline bool text_row(const MatRow& m, const EmitCtx& c, const Sche
     n += frag ? chars_of<R_BODY_ARGS>() : chars_of<R_BODY_NONE>();
     body = frag ? 1u : 0u;
   }
+  n += track * (1u + (device ? 1u : 0u) + (flow ? 1u : 0u));
   const uint32_t last = close + (flow ? (meta & KTJ_M_FLOW_START ? 1u : 2u) + (meta & KTJ_M_FLOW_FWDBWD ? 2u : 0u) : 0u);
   n += chars_table.of[R_TAIL + last];
   block(S_Z)[3] = type | (name << 5) | (body << 12) | (args << 14) | (last << 21) | (between << 25) | ((uint32_t)(tid >> 42) << 27);
   block(S_EXT)[3] = at_name;
   block(S_FLOW)[3] = name_len | (len1 << 16);
+  if (lead) {
+    block(S_FLOW)[3] = name_len | (len1 << 16) | KTJ_TR_HAS_LEAD;
+    for (uint32_t k = 0; k < 4u; ++k) { uint32_t* const w = &block(S_Z + k)[2]; *w = (*w & 0x0FFFFFFFu) | ((lead >> (4u * k)) << 28); }
+  }
   block(S_DUR)[3] = at_more;
   two(block(S_A) + 2, (uint64_t)m.dev | (tid << KTJ_TR_DEV_BITS));
   *len = n + name_len + len1;

@@ -109,7 +109,7 @@ std::string woven_text(const weave::TextRow& row, const weave::WideText* wide, c
   const std::string pid = std::to_string(track & ((1u << KTJ_TR_DEV_BITS) - 1u));
   const std::string tid = std::to_string((track >> KTJ_TR_DEV_BITS) | ((uint64_t)KTJ_TR_TID_HIGH(plan) << 42));
   uint32_t lead = 0;
-  for (uint32_t k = 0; k < 4; ++k) lead |= KTJ_TR_LEAD_NIBBLE(row.w[k][2]) << (4 * k);
+  if (lens & KTJ_TR_HAS_LEAD) for (uint32_t k = 0; k < 4; ++k) lead |= KTJ_TR_LEAD_NIBBLE(row.w[k][2]) << (4 * k);
   auto text = [&](uint32_t d) {
     const uint32_t unit = KTJ_WD_UNIT(d);
     const uint32_t* t = unit >= SCHEMA_UNIT ? book.text + (unit - SCHEMA_UNIT) * 4 : b.text + unit * 4;
@@ -144,9 +144,9 @@ std::string woven_text(const weave::TextRow& row, const weave::WideText* wide, c
   const SchemaPlan& s = a >= KTJ_TR_SCHEMA && a != KTJ_TR_NO_ARGS ? book.plan[a - KTJ_TR_SCHEMA] : none;
   part(a >= KTJ_TR_SCHEMA ? s.args : b.ref[R_ARGS + a]);
   switch (KTJ_TR_BETWEEN(plan)) {
-    case 1: out.append(c.dict.arg_blob + (more < c.dict.n ? c.dict.arg_off[more] : 0), lens >> 16); break;
-    case 2: out += std::string(reinterpret_cast<const char*>(row.w[KTJ_TR_BLOCK(S_Y)]), 16).append(reinterpret_cast<const char*>(row.w[KTJ_TR_BLOCK(S_Z)]), 8).substr(0, lens >> 16); break;
-    case 3: out.append(reinterpret_cast<const char*>(wide[more].w), lens >> 16); break;
+    case 1: out.append(c.dict.arg_blob + (more < c.dict.n ? c.dict.arg_off[more] : 0), KTJ_TR_LEN1(lens)); break;
+    case 2: out += std::string(reinterpret_cast<const char*>(row.w[KTJ_TR_BLOCK(S_Y)]), 16).append(reinterpret_cast<const char*>(row.w[KTJ_TR_BLOCK(S_Z)]), 8).substr(0, KTJ_TR_LEN1(lens)); break;
+    case 3: out.append(reinterpret_cast<const char*>(wide[more].w), KTJ_TR_LEN1(lens)); break;
     default: break;
   }
   part(a >= KTJ_TR_SCHEMA ? s.args2 : b.ref[R_ARGS2 + a]);
