@@ -198,6 +198,7 @@ struct ktj_engine {
   std::vector<ktj_schema_desc> schemas;
   DevBuf d_fields, d_schemas;
   bool schemas_dirty = true;
+  uint32_t schemas_not_taken = 0;          /* by the weaver, a bit each of the first */
   DevVec args;
   uint64_t n_args = 0;
   std::vector<CollectiveInfo> collectives; /* ktj_add_collective entries */
@@ -1434,6 +1435,7 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
     if (rc) return rc;
     rc = upload_small(e, e->d_schemas, e->schemas.data(), e->schemas.size() * sizeof(ktj_schema_desc));
     if (rc) return rc;
+    e->schemas_not_taken = weave::schemas_not_taken(e->fields.data(), e->schemas.data(), (uint32_t)e->schemas.size());
     e->schemas_dirty = false;
   }
   if (e->api_dirty) {
@@ -1570,6 +1572,8 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
     job.g = g_recs; job.r = r_recs; job.d = d_recs; job.x = x_recs;
     job.ng = ng; job.nr = nr; job.nd = nd; job.nx = nx;
     job.whole_pass = true;
+    job.text = woven;
+    job.schemas_not_taken = e->schemas_not_taken;
     job.brief = e->dev_brief.as<DevBrief>();
     job.clk = clock_of(e); job.win_start = e->win_start; job.win_end = e->win_end;
     HIPCHK(decode(job, c, ctx, sc, st));

@@ -165,7 +165,7 @@ struct Scalars {
 };
 enum { KTJ_CNT_OUT_OF_RANGE = 0, KTJ_CNT_OUT_OF_ORDER, KTJ_CNT_FLOW, KTJ_CNT_LINKED, KTJ_CNT_BLANK_NAMES, KTJ_CNT_VALID,
        KTJ_CNT_SYNC_TYPED, KTJ_CNT_COUNT,
-       KTJ_CNT_NOT_TEXT = KTJ_CNT_COUNT }; /* (not the host's) generic rows that can be no text rows, by their type or schema */
+       KTJ_CNT_NOT_TEXT = KTJ_CNT_COUNT }; /* (not the host's) printed rows that can be no text rows (left_generic and the following) */
 #define KTJ_DEVERR_TABLE_FULL 1u         /* a join table sized from the record counts filled up (a defect) */
 #define KTJ_DEVERR_DISTINCT_DEVICES 2u   /* more distinct deviceId values than the rank set holds: the sort
                                             takes its slower path without ranks, no error reaches the caller */
@@ -248,6 +248,8 @@ struct DecodeJob {
   uint64_t ng, nr, nd, nx;   /* x: only their correlation ids' range */
   uint64_t first;            /* arrival index of the first generic record; runtime and device rows follow ng records */
   bool whole_pass;           /* false: generic records made during the pass, which are in no table */
+  bool text;                 /* a pass that makes text rows: those that will be none are counted, as far as their records say so */
+  uint32_t schemas_not_taken;
   DevBrief* brief;
   ClockDev clk;
   int64_t win_start, win_end;

@@ -163,6 +163,16 @@ __device__ __forceinline__ void block_add(Scalars* sc, int which, uint32_t mine)
   if (threadIdx.x == 0 && t) atomicAdd(&sc->shard[blockIdx.x & (KTJ_COUNTER_SHARDS - 1u)][which], (unsigned long long)t);
 }
 
+/* two of them that are one or none per thread */
+__device__ __forceinline__ void block_add_two(Scalars* sc, int which, bool mine, int which2, bool mine2) {
+  const uint32_t t = block_sum((mine ? 1u : 0u) | (mine2 ? 0x10000u : 0u));
+  if (threadIdx.x == 0 && t) {
+    unsigned long long* const counter = sc->shard[blockIdx.x & (KTJ_COUNTER_SHARDS - 1u)];
+    if (t & 0xFFFFu) atomicAdd(&counter[which], (unsigned long long)(t & 0xFFFFu));
+    if (t >> 16) atomicAdd(&counter[which2], (unsigned long long)(t >> 16));
+  }
+}
+
 __global__ void k_fill_u64(uint64_t* p, uint64_t v, uint64_t n) {
   uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = v;
@@ -444,16 +454,16 @@ __global__ void __launch_bounds__(KTJ_BLOCK) k_decode(DecodeJob J, Columns c, Em
   uint32_t cnt;
   if (b < J.gb) {
     const ktj_generic_rec* l = stage_records(J.g, b * KTJ_BLOCK, J.ng, stage, &cnt);
-    /* rows that may need a Stream Sync row of their own are rare: the extra passes run only if any */
-    const bool has = threadIdx.x < cnt, sync_typed = has && l[threadIdx.x].type == KTJ_TYPE_CUDA_SYNC;
-    if (__syncthreads_or(sync_typed ? 1 : 0)) block_add(sc, KTJ_CNT_SYNC_TYPED, sync_typed ? 1u : 0u);
-    if (J.whole_pass) {
-      block_key_range(has, has ? (uint64_t)(int64_t)l[threadIdx.x].id : 0, sc, KTJ_TBL_CPU);
-      const bool no_text = has && (l[threadIdx.x].type == KTJ_TYPE_CPU_INSTANT_EVENT || is_counter_type(l[threadIdx.x].type) ||
-                                   (l[threadIdx.x].schema_id >= weave::MAX_SCHEMAS && l[threadIdx.x].schema_id < ctx.n_schemas));
-      if (__syncthreads_or(no_text ? 1 : 0)) block_add(sc, KTJ_CNT_NOT_TEXT, no_text ? 1u : 0u);
+    const bool has = threadIdx.x < cnt;
+    if (J.whole_pass) block_key_range(has, has ? (uint64_t)(int64_t)l[threadIdx.x].id : 0, sc, KTJ_TBL_CPU);
+    bool left = false;
+    if (has) {
+      const RowCols r = cols_generic(l[threadIdx.x], ctx);
+      left = J.text && (r.meta & KTJ_M_VALID) && weave::left_generic(l[threadIdx.x], r.dev, ctx, J.schemas_not_taken);
+      store_cols(c, J.first + b * KTJ_BLOCK + threadIdx.x, r);
     }
-    if (has) store_cols(c, J.first + b * KTJ_BLOCK + threadIdx.x, cols_generic(l[threadIdx.x], ctx));
+    /* rows that may need a Stream Sync row of their own are rare: the extra passes run only if any */
+    block_add_two(sc, KTJ_CNT_SYNC_TYPED, has && l[threadIdx.x].type == KTJ_TYPE_CUDA_SYNC, KTJ_CNT_NOT_TEXT, left);
     return;
   }
   b -= J.gb;
@@ -463,13 +473,14 @@ __global__ void __launch_bounds__(KTJ_BLOCK) k_decode(DecodeJob J, Columns c, Em
     const uint64_t id = has ? l[threadIdx.x].id : 0;
     block_key_range(has, id, sc, KTJ_TBL_FULL);
     block_key_range(has, narrow_corr_key(id), sc, KTJ_TBL_NARROW);
-    uint32_t oor = 0;
+    bool oor = false, left = false;
     if (has) {
       const RowCols r = cols_runtime(l[threadIdx.x], J.clk, J.win_start, J.win_end);
-      oor = r.meta & KTJ_M_VALID ? 0u : 1u;
+      oor = !(r.meta & KTJ_M_VALID);
+      left = J.text && !oor && weave::left_runtime(l[threadIdx.x], r.ts, r.dur, ctx);
       store_cols(c, J.ng + b * KTJ_BLOCK + threadIdx.x, r);
     }
-    block_add(sc, KTJ_CNT_OUT_OF_RANGE, oor);
+    block_add_two(sc, KTJ_CNT_OUT_OF_RANGE, oor, KTJ_CNT_NOT_TEXT, left);
     return;
   }
   b -= J.rb;
@@ -477,18 +488,19 @@ __global__ void __launch_bounds__(KTJ_BLOCK) k_decode(DecodeJob J, Columns c, Em
     const ktj_device_rec* l = stage_records(J.d, b * KTJ_BLOCK, J.nd, stage, &cnt);
     const bool has = threadIdx.x < cnt;
     block_key_range(has, has ? l[threadIdx.x].id : 0, sc, KTJ_TBL_FULL);
-    uint32_t oor = 0;
+    bool oor = false, left = false;
     if (has) {
       const ktj_device_rec* d = &l[threadIdx.x];
       const uint64_t i = b * KTJ_BLOCK + threadIdx.x;
       const RowCols r = cols_device(*d, J.clk, J.win_start, J.win_end);
-      oor = r.meta & KTJ_M_VALID ? 0u : 1u;
+      oor = !(r.meta & KTJ_M_VALID);
+      left = J.text && !oor && weave::left_device(*d, r.ts, r.dur, r.res, ctx);
       store_cols(c, J.ng + J.nr + i, r);
       DevBrief br;
       br.queue = d->queue; br.device = d->device; br.domain = device_row_domain(d->domain);
       J.brief[i] = br;
     }
-    block_add(sc, KTJ_CNT_OUT_OF_RANGE, oor);
+    block_add_two(sc, KTJ_CNT_OUT_OF_RANGE, oor, KTJ_CNT_NOT_TEXT, left);
     return;
   }
   b -= J.db; /* correlation ids of the external-correlation records */

@@ -12,6 +12,7 @@
 #define KTJ_WEAVE_CORE_H_
 
 #include "fmt_core.h"
+#include "mat_core.h"
 
 namespace ktj {
 namespace weave {
@@ -413,6 +414,68 @@ KTJ_HD inline void put_field_text(const ktj_field& fd, const char* key, uint32_t
   else if (fd.type == KTJ_F_DICT_END) *t = '}';
   else if (fd.type == KTJ_F_I64_ARRAY) { *t = '['; text[place >> 16] = ']'; }
   else if (fd.type == KTJ_F_STR) { *t = '"'; text[place >> 16] = '"'; }
+}
+
+/* A bit for each of the first schemas that is not taken whatever its keys are (they lie on the device: a schema whose
+ * keys are too long is not among these). */
+inline uint32_t schemas_not_taken(const ktj_field* fields, const ktj_schema_desc* schemas, uint32_t n_schemas) {
+  const uint32_t key_len[KTJ_WEAVE_FIELDS] = {};
+  uint32_t desc[SCHEMA_DESC], place[KTJ_WEAVE_FIELDS], bits = 0, at = 0, n_desc = 0, n_unit = 0;
+  for (uint32_t k = 0; k < n_schemas && k < MAX_SCHEMAS; ++k) {
+    SchemaPlan plan;
+    plan.what = 0;
+    if (schemas[k].n_fields <= KTJ_WEAVE_FIELDS - at) {
+      const SchemaSize size = lay_out_schema(fields + schemas[k].first_field, key_len, schemas[k].n_fields, &plan, desc, place);
+      n_desc += size.desc; n_unit += size.units;
+      at += schemas[k].n_fields;
+    } else at = KTJ_WEAVE_FIELDS;
+    if (!plan.what || n_desc > SCHEMA_DESC || n_unit > SCHEMA_TEXT) bits |= 1u << k;
+  }
+  return bits;
+}
+
+/* ---- records that text_row will refuse, as far as their own numbers say so; for rows inside the capture window.  What it does
+ * not say: names beyond KTJ_WEAVE_MAX_RUN, the values of typed arguments, keys, what a device row takes over from a runtime row
+ * (counted there), leads beside tracks of many digits ---- */
+#define KTJ_SEVEN_DIGITS 10000000ull
+#define KTJ_ELEVEN_DIGITS 100000000000ull
+KTJ_HD KTJ_FI inline bool left_by_track(int64_t dev, int64_t res, int64_t rel_ns, int64_t dur) {
+  return ((uint64_t)dev >> KTJ_TR_DEV_BITS) != 0 || ((uint64_t)res >> 47) != 0 || rel_ns >= (int64_t)(65536u * KTJ_LEAD_UNIT * 1000u) || dur >= 10000000000ll;
+}
+KTJ_HD KTJ_FI inline bool left_by_three(uint32_t a, uint32_t b, uint32_t c) { /* three_text_of: eleven digits together */
+  if (a < 100000u && b < 1000u && c < 1000u) return false;
+  return b >= 1000000u || c >= 1000000u || ndigits_u64(a) + ndigits_u64(b) + ndigits_u64(c) > 11;
+}
+KTJ_HD KTJ_FI inline bool left_generic(const ktj_generic_rec& g, int64_t dev, const EmitCtx& c, uint32_t not_taken) {
+  const uint32_t type = g.type & KTJ_M_TYPE_MASK;
+  if (type >= 29u || type == KTJ_TYPE_CPU_INSTANT_EVENT || is_counter_type(type)) return true;
+  if (g.schema_id < c.n_schemas && (g.schema_id >= MAX_SCHEMAS || ((not_taken >> g.schema_id) & 1u))) return true;
+  if (type == KTJ_TYPE_CUDA_SYNC && g.name_id < c.dict.n && (dict_flags(c.dict, g.name_id) & KTJ_SF_STREAM_SYNC)) return true;
+  const MatRow m = mat_generic(g, dev);
+  const bool wider = type == KTJ_TYPE_GPU_USER_ANNOTATION, flow = (m.meta & KTJ_M_FLOW) != 0;
+  bool args = false; /* that are printed whatever they are */
+  if (m.ext <= -1000000000 && g.schema_id < c.n_schemas) {
+    const ktj_schema_desc sd = c.schemas[g.schema_id];
+    args = sd.n_fields != 0 && (sd.n_fields != 1 || c.fields[sd.first_field].type != KTJ_F_RAW);
+  }
+  return (flow && (wider || (uint64_t)m.flow_id >= KTJ_ELEVEN_DIGITS)) || args ||
+         left_by_track(dev, (int64_t)sanitize_tid(m.res), m.ts - c.base_time_ns, m.dur + (wider ? 2 : 0));
+}
+KTJ_HD KTJ_FI inline bool left_runtime(const ktj_runtime_rec& r, int64_t ts, int64_t dur, const EmitCtx& c) {
+  bool left = r.cid >= KTJ_SEVEN_DIGITS || r.id >= KTJ_ELEVEN_DIGITS || left_by_track((int64_t)r.pid, (int64_t)sanitize_tid((int64_t)r.tid), ts - c.base_time_ns, dur);
+  if (r.kind == KTJ_RT_KERNEL)
+    left = left || left_by_three(r.u.kernel.grid[0], r.u.kernel.grid[1], r.u.kernel.grid[2]) ||
+           left_by_three(r.u.kernel.workgroup[0], r.u.kernel.workgroup[1], r.u.kernel.workgroup[2]);
+  else if (r.kind == KTJ_RT_COPY) {
+    const int32_t kind = (int32_t)r.u.copy.copy_kind;
+    left = left || ((r.u.copy.src | r.u.copy.dst) >> 60) != 0 || r.u.copy.size >= KTJ_ELEVEN_DIGITS || kind < -999 || kind > 9999;
+  } else if (r.kind == KTJ_RT_MALLOC) left = left || (r.u.malloc_.ptr >> 60) != 0;
+  return left;
+}
+KTJ_HD KTJ_FI inline bool left_device(const ktj_device_rec& d, int64_t ts, int64_t dur, int64_t res, const EmitCtx& c) {
+  const bool memset_row = device_row_domain(d.domain) == KTJ_DOM_MEMSET;
+  return (memset_row && (c.create_flags & KTJ_CREATE_CUDA12_ARGS)) || (memset_row ? d.queue & 0xFFFFFFFFull : d.queue) >= KTJ_SEVEN_DIGITS || d.id >= KTJ_ELEVEN_DIGITS ||
+         left_by_track((int64_t)d.device, res, ts - c.base_time_ns, dur);
 }
 
 /* ---- numbers as text ---- */

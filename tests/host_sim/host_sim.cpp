@@ -153,7 +153,7 @@ std::string woven_text(const weave::TextRow& row, const weave::WideText* wide, c
   part(b.ref[R_TAIL + KTJ_TR_TAIL(plan)]);
   return out;
 }
-uint64_t n_woven = 0, n_not_woven = 0;
+uint64_t n_woven = 0, n_not_woven = 0, n_left_known = 0;
 
 }  // namespace
 
@@ -161,6 +161,8 @@ extern "C" {
 
 // activities of the last document rendered with KTJSIM_WOVEN that were text rows, and that were not
 void ktjsim_woven(uint64_t* woven, uint64_t* left) { *woven = n_woven; *left = n_not_woven; }
+// of the latter, those that are known from their records
+uint64_t ktjsim_left_known() { return n_left_known; }
 #define KTJSIM_WOVEN 1u
 int ktjsim_real_text(double v, char* out) {
   uint64_t b;
@@ -444,15 +446,24 @@ int ktjsim_render(const ktj_stream* s, uint32_t tile_bytes, char** out, uint64_t
     // rows as text and what the weaver makes of them; those that are not text from format_activity
     std::unique_ptr<weave::SchemaBook> book(new weave::SchemaBook);
     lay_out_schemas(ctx, book.get());
-    n_woven = n_not_woven = 0;
+    n_woven = n_not_woven = n_left_known = 0;
+    const uint32_t not_taken = weave::schemas_not_taken(ctx.fields, ctx.schemas, ctx.n_schemas);
+    for (uint32_t k = 0; k < std::min<uint32_t>(ctx.n_schemas, weave::MAX_SCHEMAS); ++k)
+      if (((not_taken >> k) & 1u) && book->plan[k].what) { free(buf); return -6; }
     for (size_t i = 0; i < perm.size(); ++i) {
       const MatRow& m = mat[perm[i]];
+      const uint64_t a = perm[i];
+      const bool known = a < ng ? weave::left_generic(s->generic[a], m.dev, ctx, not_taken)
+                       : a < ng + nr ? weave::left_runtime(s->runtime[a - ng], m.ts, m.dur, ctx)
+                       : a < ng + nr + nd && weave::left_device(s->device[a - ng - nr], m.ts, m.dur, m.res, ctx);
+      n_left_known += known;
       weave::TextRow row;
       weave::WideText wide[2];
       memset(&row, 0xA5, sizeof row);
       uint32_t len = 0, tail = 0;
       char* at = buf + prefix.size() + offs[i];
       if (weave::text_row(m, ctx, book->plan, &row, 0, wide, 1, &len, &tail)) {
+        if (known) { free(buf); return -7; }
         if (len != offs[i + 1] - offs[i] || tail != tail_kind(m, has_args(m, ctx)) || row.w[7][3] >> 24 == KTJ_ROW_LEFT) { free(buf); return -4; }
         const std::string t = woven_text(row, wide, ctx, *book);
         if (t.size() != len) { free(buf); return -5; }

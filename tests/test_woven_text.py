@@ -181,6 +181,66 @@ def test_leads_with_no_room_are_left(sim):
     assert _woven_vs_oracle(sim, stream(B - 65536 * LEAD, 1, 1)) == (0, 3)
 
 
+def _odd_streams():
+    """Streams of three ordinary CPU ops, a launch, a copy, an allocation and a kernel, each with one row that is no text row, as its record says."""
+    def base():
+        b = StreamBuilder(window=(B, B + 10**13), host_name="odd")
+        b.api(["hipLaunchKernel", "hipMemcpyAsync", "hipMalloc"], flow_start=[0], malloc_cid=2)
+        for k in range(3):
+            b.add_generic("op", 0, B + 1000 + k, B + 2000 + k, 1, 5, id=k + 1)
+        b.add_runtime(1, B + 3000, B + 4000, 0, 1, 5, kind=1, grid=(99999, 999, 999), workgroup=(256, 1, 1))
+        b.add_runtime(2, B + 5000, B + 6000, 1, 1, 5, kind=2, src=1, dst=2, size=10**11 - 1, copy_kind=-999)
+        b.add_runtime(3, B + 7000, B + 8000, 2, 1, 5, kind=3, ptr=(1 << 60) - 1, size=5)
+        b.add_device(1, B + 9000, B + 9500, name="k", queue=9999999)
+        return b
+    t = B + 20000
+    def generic(b, typ=0, end=t + 5, dev=1, res=5, **kw):
+        b.add_generic(kw.pop("name", "op"), typ, t, end, dev, res, **kw)
+    def runtime(b, **kw):
+        b.add_runtime(kw.pop("id", 9), t, kw.pop("end", t + 5), kw.pop("cid", 0), kw.pop("pid", 1), kw.pop("tid", 5), **kw)
+    def device(b, **kw):
+        b.add_device(kw.pop("id", 9), t, kw.pop("end", t + 5), **kw)
+    def two_strings(b):
+        generic(b, schema=b.schema([("Input type", abi.F_STR, 1), ("Input Dims", abi.F_STR, 1)]), values=[b.s("x"), b.s("y")])
+    def five_numbers(b):
+        generic(b, schema=b.schema([("n%d" % k, abi.F_I64, 1) for k in range(5)]), values=[1] * 5)
+    def late_schema(b):
+        ids = [b.schema([("k%d" % k, abi.F_I64, 1)]) for k in range(17)]
+        generic(b, schema=ids[16], values=[1])
+    def many_schemas(b):   # more descriptors than there is room for
+        ids = [b.schema([("k%d_%d" % (k, j), abi.F_I64, 1) for j in range(4)]) for k in range(16)]
+        generic(b, schema=ids[15], values=[1] * 4)
+    edits = dict(
+        instant=lambda b: generic(b, 17), counter=lambda b: generic(b, 9, schema=b.schema([("v", abi.F_F64, 1)]), values=[0.5]), two_strings=two_strings, five_numbers=five_numbers,
+        late_schema=late_schema, many_schemas=many_schemas, stream_sync=lambda b: generic(b, 15, name="Stream Sync"),
+        annotation_flow=lambda b: generic(b, 2, flow_id=3, flow_type=1), flow=lambda b: generic(b, flow_id=10**11, flow_type=1), external=lambda b: generic(b, id=-10**9, schema=b.schema([("n", abi.F_I64, 1)]), values=[1]),
+        process=lambda b: generic(b, dev=1 << 22), negative_process=lambda b: generic(b, dev=-1), thread=lambda b: generic(b, res=1 << 47),
+        duration=lambda b: generic(b, end=t + 10**10), annotation_duration=lambda b: generic(b, 2, end=t + 10**10 - 2),
+        runtime_duration=lambda b: runtime(b, end=t + 10**10), correlation=lambda b: runtime(b, id=10**11),
+        grid=lambda b: runtime(b, kind=1, grid=(999999, 999, 999)), block=lambda b: runtime(b, kind=1, grid=(1, 1, 1), workgroup=(1, 1000000, 1)),
+        address=lambda b: runtime(b, cid=1, kind=2, src=1 << 60), size=lambda b: runtime(b, cid=1, kind=2, size=10**11), copy_kind=lambda b: runtime(b, cid=1, kind=2, copy_kind=-1000),
+        pointer=lambda b: runtime(b, cid=2, kind=3, ptr=1 << 60), device_duration=lambda b: device(b, end=t + 1 + 10**10, name="k"), queue=lambda b: device(b, queue=10**7, name="k"),
+        device_correlation=lambda b: device(b, id=10**11, name="k"), context=lambda b: b.add_memset(9, t, t + 5, context=10**7))
+    for name, edit in edits.items():
+        b = base()
+        edit(b)
+        yield name, b.build()
+    b = base()
+    b.create_flags = abi.KTJ_CREATE_CUDA12_ARGS
+    b.add_memset(9, t, t + 5)
+    yield "cuda12", b.build()
+
+
+def test_rows_left_are_known_when_decoded(sim):
+    """Whether too many rows are left is decided before any is made: what a record says by itself is counted (and nothing that is
+    a text row after all: ktjsim_render fails there)."""
+    sim.ktjsim_left_known.restype = C.c_uint64
+    for name, sp in _odd_streams():
+        assert (_woven_vs_oracle(sim, sp)[1], sim.ktjsim_left_known()) == (1, 1), name
+    _woven, left = _woven_vs_oracle(sim, edge_stream(3000))
+    assert left * 0.6 < sim.ktjsim_left_known() < left
+
+
 def test_doubles_as_text(sim):
     """Shifted together, against the formatter's characters one by one: zeros behind the text, too."""
     import random
@@ -212,7 +272,7 @@ def _gpu_vs_oracle(sp, passes=3):
     o.close()
     lib.ktj_debug_force_sort_passes(1)
     try:
-        with TraceEngine(sp.contents.trace_name.decode(), base_time_ns=sp.contents.base_time_ns) as e:
+        with TraceEngine(sp.contents.trace_name.decode(), base_time_ns=sp.contents.base_time_ns, cuda12_args=sp.contents.create_flags != 0) as e:
             e.submit_stream(sp)
             for _ in range(passes):
                 e.process()
@@ -240,3 +300,10 @@ def test_woven_documents_at_the_edges(n, other_types):
     With other types the first pass leaves all activities to the other kernel, without them it leaves those with no room; the
     second makes no text rows where too many had none."""
     _gpu_vs_oracle(edge_stream(n, other_types))
+
+
+@pytest.mark.gpu
+def test_documents_with_one_row_left():
+    for name, sp in _odd_streams():
+        print(name, flush=True)
+        _gpu_vs_oracle(sp)
