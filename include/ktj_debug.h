@@ -27,13 +27,16 @@ enum {
   KTJ_DBG_NAME_VIEW = 11, /* bytes: all names after the name pipeline           */
   KTJ_DBG_NAME_OFF = 12,  /* uint64[n_strings+1]                                */
   KTJ_DBG_ARG_VIEW = 13,
-  KTJ_DBG_ARG_OFF = 14
+  KTJ_DBG_ARG_OFF = 14,
+  KTJ_DBG_PASS = 15       /* uint64[4]  of the last pass that was no small one: it made text rows; none of them, as it left
+                             too many; activities that the weaver left; these had a wait of their own */
 };
 
 /* Copies the array to dst (at most cap bytes) and reports its full size.  Valid after
- * ktj_process.  A trace of up to 2048 records keeps none of the arrays: it is processed once more,
- * with the launches of a large trace and as ktj_process does it (the document is then in the engine's
- * own buffer, also if ktj_process_noalloc had put it into one of the caller's). */
+ * ktj_process.  A trace of up to 2048 records keeps none of the arrays, and KTJ_DBG_MAT is not what
+ * a larger one keeps mostly (rows as text): it is processed once more, with the launches of a large
+ * trace and as ktj_process does it (the document is then in the engine's own buffer, also if
+ * ktj_process_noalloc had put it into one of the caller's). */
 int ktj_debug_fetch(ktj_engine* e, int what, void* dst, uint64_t cap, uint64_t* n_bytes);
 
 /* Runs a plain device-to-device copy kernel of n_bytes (16 bytes per lane) twice and reports the

@@ -121,16 +121,17 @@ k_emit(const MatRow* mat, const uint32_t* perm, const uint64_t* offs, uint64_t n
  * a lane whose stage is nearly full stores its line itself (BlockWriter::relief).  Lanes without an activity stay until the end
  * for the quads' sake.  The document's prefix and suffix are already in place when this kernel
  * runs; the first and the last activity merge with them. */
-template <bool LIST> /* only the activities on the list */
+template <bool LIST> /* only the activities on the list, or all where the weaver prints none */
 __global__ void __launch_bounds__(KTJ_BLOCK) __attribute__((amdgpu_waves_per_eu(3)))
 k_emit_direct(const char* rows, const uint32_t* perm, const uint64_t* offs, const uint8_t* kind_sorted,
               EmitCtx ctx, char* out, uint64_t prefix_len, const Scalars* sc, const uint32_t* left) {
-  const uint64_t n_rows = sc->emit_rows, n_mine = !LIST ? n_rows : n_rows ? sc->n_left : 0u;
+  const bool all = !LIST || sc->no_text;
+  const uint64_t n_rows = sc->emit_rows, n_mine = all ? n_rows : n_rows ? sc->n_left : 0u;
   if ((uint64_t)blockIdx.x * blockDim.x >= n_mine) return;
   uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x, o = 0;
   uint32_t row = 0;
   bool active = i < n_mine;
-  if (LIST && active) i = left[i];
+  if (!all && active) i = left[i];
   /* A wavefront that has just started comes first on its SIMD until the loads of its joined row are
    * on their way (two dependent loads with a few instructions between them, which would otherwise
    * queue behind the formatting of the two older wavefronts): config 3 4.70 -> 4.61 ms, config 4

@@ -233,7 +233,8 @@ struct ktj_engine {
   DevBuf keys_a, keys_b, vals_a, vals_b, hist, scan_tmp;
   bool rows_are_text = false;              /* of the last pass: TextRows in mat */
   uint64_t not_woven = 0;                  /* number of records with which the last woven pass left too many activities (too_many_left) */
-  bool some_left = false;                  /* the last pass had activities that the weaver leaves to emit_direct */
+  bool some_left = true;                   /* the last pass had activities that the weaver leaves to emit_direct; not known before the first */
+  uint64_t pass_info[4] = {};              /* of the last pass (KTJ_DBG_PASS) */
   DevBuf mat, schema_book, wide_text, len, len_sorted, kind_sorted, offs, out, tile_start;
   void* pinned_small = nullptr; size_t pinned_small_cap = 0;
   HostCtl* h_ctl = nullptr;                  /* pinned: what the device hands back during a pass */
@@ -1482,6 +1483,7 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
    * would not fit the scratch array with as many records. */
   const bool woven = n_coll == 0 && !e->noalloc && !e->no_weave && !(e->flags & KTJ_CREATE_TILE_EMIT) && (e->not_woven == 0 || e->not_woven != ng + nr + nd);
   e->rows_are_text = woven;
+  e->pass_info[0] = woven; e->pass_info[1] = e->pass_info[2] = e->pass_info[3] = 0;
   const bool wide = woven && std::any_of(e->fields.begin(), e->fields.end(), [](const ktj_field& f) { return f.type == KTJ_F_F64; });
   e->pool_used = 0;
   size_t pass_bytes = 0;
@@ -1635,6 +1637,14 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
     HIPCHK(emit_direct(rows.p, e->perm, e->offs.as<uint64_t>(), e->kind_sorted.as<uint8_t>(), woven ? n_left : n_most, ctx, e->out.as<char>(), at, sc, left(), st));
     return KTJ_OK;
   };
+  /* when the scalars are the host's: how many others there are */
+  auto was_woven = [&]() -> uint64_t {
+    if (!woven) return 0;
+    const uint64_t n = e->scalars.no_text ? e->scalars.n_valid : e->scalars.n_left;
+    e->not_woven = too_many_left(n, e->scalars.n_valid) ? ng + nr + nd : 0u;
+    e->pass_info[1] = e->scalars.no_text; e->pass_info[2] = n;
+    return n;
+  };
   bool emitted = false;
   if (straight) {
     const std::string prefix = e->txt_header + e->txt_before;
@@ -1651,8 +1661,10 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
       text.out = e->out.as<char>(); text.out_cap = e->out.cap;
       HIPCHK(gather_offsets(e->perm, e->len.as<uint32_t>(), N, e->len_sorted.as<uint32_t>(), e->kind_sorted.as<uint8_t>(),
                             e->scan_tmp.as<uint64_t>(), e->offs.as<uint64_t>(), left(), sc, text, st));
-      /* Mostly there are no others, and a launch that finds its list empty takes 4 us, 20 with 22 million rows: it is left out until
-       * a pass has had some.  The first pass that has waits twice. */
+      /* Mostly there are no others, and a launch that finds its list empty takes 4 us, 20 with 22 million rows: it is left out where
+       * the last pass had none.  The first pass of an engine, a session's only one mostly, makes it: without it 30 000 records with one
+       * number too long for its row took 218 us instead of 203, with a row known to be left 217 instead of 203, without any 176
+       * instead of 180. */
       const bool others = e->some_left;
       { const int rc = put_activities(N, others ? N : 0u, prefix.size()); if (rc != KTJ_OK) return rc; }
       HIPCHK(hipEventRecord(e->ev[EV_EMIT], st));
@@ -1664,10 +1676,11 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
       e->total_bytes = prefix.size() + e->act_bytes + suffix.size();
       emitted = e->total_bytes + 64 <= text.out_cap;
       if (emitted) {
-        e->some_left = e->scalars.n_left != 0;
-        if (woven) e->not_woven = too_many_left(e->scalars.n_left, e->scalars.n_valid) ? ng + nr + nd : 0u;
-        if (woven && e->some_left && !others) {
-          { const int rc = put_activities(0, e->scalars.n_left, prefix.size()); if (rc != KTJ_OK) return rc; }
+        const uint64_t n_left = was_woven();
+        if (woven) e->some_left = n_left != 0;
+        if (n_left != 0 && !others) {
+          e->pass_info[3] = 1;
+          { const int rc = put_activities(0, n_left, prefix.size()); if (rc != KTJ_OK) return rc; }
           HIPCHK(hipEventRecord(e->ev[EV_EMIT], st));
           HIPCHK(hipStreamSynchronize(st));
         }
@@ -1821,9 +1834,8 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
                   e->tile_start.as<uint32_t>(), st));
     else
     {
-      const int rc = put_activities(e->scalars.n_valid, e->scalars.n_left, e->prefix_len);
+      const int rc = put_activities(e->scalars.n_valid, was_woven(), e->prefix_len);
       if (rc != KTJ_OK) return rc;
-      if (woven) e->not_woven = too_many_left(e->scalars.n_left, e->scalars.n_valid) ? ng + nr + nd : 0u;
     }
   }
   HIPCHK(hipEventRecord(e->ev[EV_EMIT], st));
@@ -2166,6 +2178,11 @@ int ktj_debug_copy_reference(ktj_engine* e, uint64_t n_bytes, float* ms) {
 int ktj_debug_fetch(ktj_engine* e, int what, void* dst, uint64_t cap, uint64_t* n_bytes) {
   if (!e || !n_bytes) return KTJ_ERR_ARG;
   if (!e->processed) return KTJ_ERR_STATE;
+  if (what == KTJ_DBG_PASS) { /* (says what the last pass did: makes none) */
+    *n_bytes = sizeof e->pass_info;
+    if (dst) memcpy(dst, e->pass_info, std::min<uint64_t>(*n_bytes, cap));
+    return KTJ_OK;
+  }
   const bool as_text = what == KTJ_DBG_MAT && e->rows_are_text;
   if (e->small_last || as_text) { /* a small pass keeps none of these: the launches of a large trace make them (and the same document) */
     e->no_small = true;

@@ -145,7 +145,7 @@ struct Scalars {
   unsigned int n_sync_rows;           /* distinct (device, row) pairs of Stream Sync activities */
   unsigned int n_plain;               /* small traces: activities that small_emit leaves to small_plain */
   unsigned int n_left;                /* activities that weave leaves to emit_direct */
-  unsigned int no_text;               /* leave them all (too_many_left) */
+  unsigned int no_text;               /* it leaves them all (too_many_left); n_left is 0 then */
   unsigned int ext_ids_repeat;        /* two external-correlation records share a correlation id */
   unsigned long long emit_rows;       /* activities to format: n_valid, or none where the pass cannot end so */
   unsigned long long clock[KTJ_CLOCK_COUNT];
@@ -364,7 +364,7 @@ hipError_t radix_sort(uint64_t* keys_a, uint32_t* vals_a, uint64_t* keys_b, uint
 
 /* ---- stage 4a: joined rows + exact byte length (arrival order) ---- */
 /* With schemas set the rows are TextRows (those that the weaver does not print MatRows in the same places, marked:
- * KTJ_ROW_LEFT, and tail kind KTJ_KIND_LEFT beside their lengths); otherwise all are MatRows. */
+ * KTJ_ROW_LEFT, and tail kind KTJ_KIND_LEFT beside their lengths but where Scalars::no_text leaves all); otherwise all are MatRows. */
 struct Rows {
   void* p;
   const weave::SchemaBook* schemas;
@@ -415,7 +415,8 @@ hipError_t emit(const MatRow* mat, const uint32_t* perm, const uint64_t* offs /*
                 uint32_t* tile_start /* tiles + 1 */, hipStream_t st);
 
 /* direct variant: one lane per activity; kind_sorted holds the tail kind of every activity in emission order;
- * Scalars::emit_rows of them, at most n_most.  left: only the Scalars::n_left activities on this list, rows are sizeof(TextRow) apart */
+ * Scalars::emit_rows of them, at most n_most.  left: only the Scalars::n_left activities on this list, rows are sizeof(TextRow) apart;
+ * all of them, in order, where Scalars::no_text says so */
 hipError_t emit_direct(const void* rows, const uint32_t* perm, const uint64_t* offs, const uint8_t* kind_sorted, uint64_t n_most, EmitCtx ctx,
                        char* out, uint64_t prefix_len, const Scalars* sc, const uint32_t* left, hipStream_t st);
 

@@ -1197,8 +1197,9 @@ __global__ void __launch_bounds__(KTJ_BLOCK) k_collect_distinct(Columns c, uint6
   const uint32_t books = book ? 1u : 0u;
   const bool lays_out = blockIdx.x < books;
   if (blockIdx.x == 0 && threadIdx.x == 0) stage_clock(sc, KTJ_CLOCK_SORT);
-  if (lays_out) lay_out_schemas(ctx, book, reinterpret_cast<SchemaLds*>(seen));
-  else for (uint32_t k = threadIdx.x; k <= LOCAL_SET_SLOTS; k += blockDim.x) { seen[0][k] = KTJ_EMPTY_KEY; seen[1][k] = KTJ_EMPTY_KEY; }
+  if (lays_out) {
+    if (sc->no_text == 0) lay_out_schemas(ctx, book, reinterpret_cast<SchemaLds*>(seen));
+  } else for (uint32_t k = threadIdx.x; k <= LOCAL_SET_SLOTS; k += blockDim.x) { seen[0][k] = KTJ_EMPTY_KEY; seen[1][k] = KTJ_EMPTY_KEY; }
   __syncthreads();
   uint64_t mn = ~0ULL, mx = 0ULL;
   uint64_t last_dev = 0, last_res = 0; /* of the thread's rows so far: most rows repeat them */
@@ -2211,10 +2212,12 @@ template <bool TEXT>
 __device__ __forceinline__ uint32_t stage_row(const MatRow& m, const EmitCtx& ctx, const Rows& rows, uint32_t wide_at, Scalars* sc, uint4* stage) {
   if (!TEXT) { row_to_lds(m, stage); return row_length(m, ctx, sc); }
   weave::TextRow* const t = reinterpret_cast<weave::TextRow*>(stage) + threadIdx.x;
-  uint32_t n, tail;
-  if (!(m.meta & KTJ_M_VALID)) n = 0;
-  else if (sc->no_text == 0 && weave::text_row(m, ctx, rows.schemas->plan, t, threadIdx.x & 7u, rows.wide, wide_at, &n, &tail)) return n | (tail << 30);
-  else n = row_length(m, ctx, sc) | (KTJ_KIND_LEFT << 30);
+  uint32_t n = 0, tail;
+  if (m.meta & KTJ_M_VALID) {
+    const bool text = sc->no_text == 0;
+    if (text && weave::text_row(m, ctx, rows.schemas->plan, t, threadIdx.x & 7u, rows.wide, wide_at, &n, &tail)) return n | (tail << 30);
+    n = row_length(m, ctx, sc) | (text ? KTJ_KIND_LEFT << 30 : 0u); /* (all are left: no list is made, they are printed in order) */
+  }
   static_assert(sizeof(MatRow) == 96, "six blocks");
   auto block = [&](uint32_t k) { __builtin_memcpy(t->w[k ^ (threadIdx.x & 7u)], reinterpret_cast<const char*>(&m) + 16u * k, 16); };
   block(0); block(1); block(2); block(3); block(4); block(5); /* (a loop would keep m in memory) */

@@ -264,7 +264,7 @@ def test_doubles_as_text(sim):
 
 
 def _gpu_vs_oracle(sp, passes=3):
-    """Through the large passes whatever the size, several times from one engine."""
+    """Through the large passes whatever the size, several times from one engine; what each says of itself (KTJ_DBG_PASS)."""
     from kineto_amd.engine import TraceEngine
     lib = abi.load_engine()
     o = og.OracleRun(sp)
@@ -274,9 +274,12 @@ def _gpu_vs_oracle(sp, passes=3):
     try:
         with TraceEngine(sp.contents.trace_name.decode(), base_time_ns=sp.contents.base_time_ns, cuda12_args=sp.contents.create_flags != 0) as e:
             e.submit_stream(sp)
+            info = []
             for _ in range(passes):
                 e.process()
                 assert e.output() == want
+                info.append([int(x) for x in e.debug("pass_info")])
+            return info
     finally:
         lib.ktj_debug_force_sort_passes(0)
 
@@ -304,6 +307,16 @@ def test_woven_documents_at_the_edges(n, other_types):
 
 @pytest.mark.gpu
 def test_documents_with_one_row_left():
+    """Known when decoded: the first pass makes no text row, the next none of them, and nothing waits for a second launch."""
     for name, sp in _odd_streams():
         print(name, flush=True)
-        _gpu_vs_oracle(sp)
+        n = sp.contents.n_generic + sp.contents.n_runtime + sp.contents.n_device
+        assert _gpu_vs_oracle(sp) == [[1, 1, n, 0]] + 2 * [[0, 0, 0, 0]], name
+
+
+@pytest.mark.gpu
+def test_first_pass_with_rows_left_does_not_wait_twice():
+    """Not known when decoded: the first pass of an engine prints them behind the others without a wait between."""
+    sp = edge_stream(40, False)
+    first, *later = _gpu_vs_oracle(sp)
+    assert first[0] == 1 and first[2] > 0 and first[3] == 0 and all(i[0] == 0 for i in later), (first, later)
