@@ -232,7 +232,7 @@ struct ktj_engine {
   DevBuf s_dev_k, s_dev_r, s_dev_l, s_res_k, s_res_r, s_res_l;
   DevBuf keys_a, keys_b, vals_a, vals_b, hist, scan_tmp;
   bool rows_are_text = false;              /* of the last pass: TextRows in mat */
-  uint64_t not_woven = 0;                  /* number of records with which the last woven pass left too many activities (too_many_left) */
+  uint64_t not_woven = 0;                  /* number of these records with which a woven pass left too many activities (too_many_left) */
   bool some_left = true;                   /* the last pass had activities that the weaver leaves to emit_direct; not known before the first */
   uint64_t pass_info[4] = {};              /* of the last pass (KTJ_DBG_PASS) */
   DevBuf mat, schema_book, wide_text, len, len_sorted, kind_sorted, offs, out, tile_start;
@@ -268,7 +268,7 @@ struct ktj_engine {
   /* six passes sort the records of one capture: 2^38 ns, four and a half minutes, beside 9 bits of devices and
    * rows; a pass more than needed costs its three launches, a pass too few the launches behind the sort */
   uint32_t sort_passes = 6;  /* to be launched: what these records took in the pass before, where there was one */
-  void other_records() { small_unfit = stepwise = false; sort_passes = std::max(sort_passes, 6u); }
+  void other_records() { small_unfit = stepwise = false; not_woven = 0; sort_passes = std::max(sort_passes, 6u); }
   bool small_last = false;   /* the last pass was a small one: it leaves no intermediate arrays for ktj_debug_fetch */
   bool no_small = false;     /* ktj_debug_fetch makes them */
   bool no_weave = false;     /* joined rows as they are: ktj_debug_fetch, and where text rows do not fit */

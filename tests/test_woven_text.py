@@ -315,6 +315,34 @@ def test_documents_with_one_row_left():
 
 
 @pytest.mark.gpu
+def test_other_records_are_woven_again():
+    """That a pass left too many is known of its records and not of others that are as many."""
+    import torch
+    from kineto_amd.engine import TraceEngine
+    lib = abi.load_engine()
+    lib.ktj_debug_force_sort_passes(1)
+    try:
+        b = StreamBuilder(window=(B, B + 10**13), host_name="odd")
+        b.s("op")
+        sp = b.build()
+        with TraceEngine(sp.contents.trace_name.decode()) as e:
+            e.submit_stream(sp)
+            for typ, want in ((17, ([1, 1, 99, 0], [0, 0, 0, 0], [0, 0, 0, 0])), (0, ([1, 0, 0, 0], [1, 0, 0, 0])), (17, ([1, 1, 99, 1], [0, 0, 0, 0]))):
+                rec = (abi.GenericRec * 99)()
+                for k, r in enumerate(rec):
+                    r.start_ns, r.end_ns, r.resource, r.device, r.id, r.name_id, r.type, r.schema_id = B + k, B + k + 5, 5, 1, k + 1, 0, typ, abi.KTJ_NONE
+                on_gpu = torch.frombuffer(bytearray(rec), dtype=torch.uint8).cuda()
+                torch.cuda.synchronize()
+                e._chk(lib.ktj_submit_records_device(e.h, abi.REC_GENERIC, on_gpu.data_ptr(), 99), "ktj_submit_records_device")
+                for info in want:
+                    e.process()
+                    assert [int(x) for x in e.debug("pass_info")] == info, typ
+                    assert e.output().count(b'"cat": "cpu_op"') == (99 if typ == 0 else 0)
+    finally:
+        lib.ktj_debug_force_sort_passes(0)
+
+
+@pytest.mark.gpu
 def test_first_pass_with_rows_left_does_not_wait_twice():
     """Not known when decoded: the first pass of an engine prints them behind the others without a wait between."""
     sp = edge_stream(40, False)
