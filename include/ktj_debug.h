@@ -48,6 +48,10 @@ int ktj_debug_copy_reference(ktj_engine* e, uint64_t n_bytes, float* ms);
  * that run small cases through both.  Process-wide. */
 void ktj_debug_force_sort_passes(int on);
 
+/* The next n allocations of device memory fail as if there were no more; returns how many of those asked for
+ * before have not come to it.  For the tests of what is done then.  Process-wide. */
+int ktj_debug_fail_allocations(int n);
+
 #ifdef __cplusplus
 }
 #endif

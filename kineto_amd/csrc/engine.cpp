@@ -66,6 +66,12 @@ static_assert(KTJ_STAGE_SLOTS >= 2 * KTJ_STAGE_THREADS_MAX, "two per copying thr
 
 bool drop_waiting_memory(); /* gives back what the current device's kit holds; true if that was anything */
 
+std::atomic<int> g_failing_allocations{0}; /* ktj_debug_fail_allocations */
+hipError_t allocate(void** p, size_t bytes) {
+  if (g_failing_allocations.load(std::memory_order_relaxed) > 0 && g_failing_allocations.fetch_sub(1) > 0) return hipErrorOutOfMemory;
+  return hipMalloc(p, bytes);
+}
+
 /* One working buffer in device memory.  `p` is what the kernels use: either the buffer's own
  * allocation (freed with the engine; the engine's device is current then) or, for the entry point
  * that allocates nothing, a borrowed range that somebody else owns (a piece of the library's static
@@ -88,8 +94,8 @@ struct DevBuf {
     if (bytes <= cap) return hipSuccess;
     if (own) { hipError_t e = hipFree(own); p = own = nullptr; cap = own_cap = 0; if (e != hipSuccess) return e; }
     size_t want = bytes + (with_slack ? bytes / 8 : 0) + 256;
-    hipError_t e = hipMalloc(&own, want);
-    if (e == hipErrorOutOfMemory && drop_waiting_memory()) { (void)hipGetLastError(); e = hipMalloc(&own, want); }
+    hipError_t e = allocate(&own, want);
+    if (e == hipErrorOutOfMemory && drop_waiting_memory()) { (void)hipGetLastError(); e = allocate(&own, want); }
     if (e != hipSuccess) { p = own = nullptr; return e; }
     p = own;
     cap = own_cap = want;
@@ -268,10 +274,11 @@ struct ktj_engine {
   /* six passes sort the records of one capture: 2^38 ns, four and a half minutes, beside 9 bits of devices and
    * rows; a pass more than needed costs its three launches, a pass too few the launches behind the sort */
   uint32_t sort_passes = 6;  /* to be launched: what these records took in the pass before, where there was one */
-  void other_records() { small_unfit = stepwise = false; not_woven = 0; sort_passes = std::max(sort_passes, 6u); }
+  void other_records() { small_unfit = stepwise = no_room_for_text = false; not_woven = 0; sort_passes = std::max(sort_passes, 6u); }
   bool small_last = false;   /* the last pass was a small one: it leaves no intermediate arrays for ktj_debug_fetch */
   bool no_small = false;     /* ktj_debug_fetch makes them */
-  bool no_weave = false;     /* joined rows as they are: ktj_debug_fetch, and where text rows do not fit */
+  bool no_weave = false;     /* joined rows as they are: ktj_debug_fetch */
+  bool no_room_for_text = false; /* and where these records' text rows do not fit into memory */
   hipError_t hip_error = hipSuccess; /* of the last call that failed */
   int64_t last_end_time = 0;
   int wall_clock_khz = 0;
@@ -1481,7 +1488,7 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
   const uint32_t cap_narrow = pow2_at_least((nx + nr) + (nx + nr) / 2), cap_cpu = pow2_at_least(2 * ng);
   /* Joined rows as text for the weaver, but where something reads them as they are, and where their 32 bytes more
    * would not fit the scratch array with as many records. */
-  const bool woven = n_coll == 0 && !e->noalloc && !e->no_weave && !(e->flags & KTJ_CREATE_TILE_EMIT) && (e->not_woven == 0 || e->not_woven != ng + nr + nd);
+  const bool woven = n_coll == 0 && !e->noalloc && !e->no_weave && !e->no_room_for_text && !(e->flags & KTJ_CREATE_TILE_EMIT) && (e->not_woven == 0 || e->not_woven != ng + nr + nd);
   e->rows_are_text = woven;
   e->pass_info[0] = woven; e->pass_info[1] = e->pass_info[2] = e->pass_info[3] = 0;
   const bool wide = woven && std::any_of(e->fields.begin(), e->fields.end(), [](const ktj_field& f) { return f.type == KTJ_F_F64; });
@@ -1887,13 +1894,12 @@ static int run_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, uint64
   };
   int rc = pass();
   if (rc != KTJ_OK && e->hip_error == hipErrorOutOfMemory && e->rows_are_text) { /* as many records as without text rows */
-    const bool before = e->no_weave;
     (void)hipGetLastError();
     e->pool.release();
     e->hip_failed = failed_before;
-    e->no_weave = true;
+    e->no_room_for_text = true; /* until other records are submitted: the next pass begins with what has fitted */
     rc = pass();
-    e->no_weave = before;
+    if (rc != KTJ_OK) e->no_room_for_text = false;
   }
   return rc;
 }
@@ -2156,6 +2162,8 @@ int ktj_get_stats(ktj_engine* e, ktj_stats* out) {
 }
 
 void ktj_debug_force_sort_passes(int on) { sort_packed_force_passes(on != 0); }
+
+int ktj_debug_fail_allocations(int n) { return std::max(g_failing_allocations.exchange(n), 0); }
 
 int ktj_debug_copy_reference(ktj_engine* e, uint64_t n_bytes, float* ms) {
   if (!e || !ms) return KTJ_ERR_ARG;

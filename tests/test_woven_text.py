@@ -343,6 +343,45 @@ def test_other_records_are_woven_again():
 
 
 @pytest.mark.gpu
+def test_pass_without_room_for_text_rows():
+    """It is made again with the shorter rows, and the next passes over these records do not try."""
+    from kineto_amd.engine import EngineError, TraceEngine
+    lib = abi.load_engine()
+    sp = edge_stream(4001, False)
+    o = og.OracleRun(sp)
+    want = o.output()
+    o.close()
+
+    def process(e, failing):
+        """How many of that many failing allocations the pass met."""
+        lib.ktj_debug_fail_allocations(failing)
+        try:
+            e.process()
+        finally:
+            left = lib.ktj_debug_fail_allocations(0)
+        return failing - left, int(e.debug("pass_info")[0])
+
+    lib.ktj_trim(0)   # (a new engine would take the memory of the one before)
+    with TraceEngine(sp.contents.trace_name.decode()) as e:
+        e.submit_stream(sp)
+        assert process(e, 1) == (1, 0)
+        assert e.output() == want
+        for _ in range(2):
+            assert process(e, 1) == (0, 0)
+            assert e.output() == want
+        one = (abi.GenericRec * 1).from_buffer_copy(C.string_at(sp.contents.generic, C.sizeof(abi.GenericRec)))
+        e._chk(lib.ktj_submit_records(e.h, abi.REC_GENERIC, one, 1), "ktj_submit_records")
+        assert process(e, 0) == (0, 1)   # other records are tried again
+    lib.ktj_trim(0)
+    with TraceEngine(sp.contents.trace_name.decode()) as e:   # no room either way
+        e.submit_stream(sp)
+        with pytest.raises(EngineError):
+            process(e, 2)
+        e.process()
+        assert e.output() == want and int(e.debug("pass_info")[0]) == 1
+
+
+@pytest.mark.gpu
 def test_first_pass_with_rows_left_does_not_wait_twice():
     """Not known when decoded: the first pass of an engine prints them behind the others without a wait between."""
     sp = edge_stream(40, False)
