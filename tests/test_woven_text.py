@@ -3,6 +3,7 @@ texts against the oracle's documents, on the CPU for every kind of row and at th
 GPU at the edges of a turn, of the strings that wait in LDS and of the activities that are left to the other kernel."""
 import ctypes as C
 import os
+import struct
 
 import pytest
 
@@ -263,6 +264,54 @@ def test_doubles_as_text(sim):
         assert got.raw[n:24] == bytes(24 - n), v
 
 
+def large_stream(n, left_known, long_names=False):
+    """n CPU ops on five threads, so many that a wavefront takes several turns of sixteen: every 800 activities some at the edges of
+    turns that are left (left_known: their records say so; the others have a typed number with no room), flow events, names that
+    wait in LDS and names that do not, doubles beside their rows.  long_names: and most of them far longer than the dictionary's
+    average, so that the first guess of the document's size is too small."""
+    import numpy as np
+    rng = np.random.default_rng(n)
+    b = StreamBuilder(window=(B, B + 10**15), host_name="large")
+    names = [b.s(_text(k, k)) for k in (1, 16, 17, 40, 127, 128, 129, 300, 700)]
+    plain = b.schema([("Sequence number", abi.F_I64, 1)])
+    wide = b.schema([("A", abi.F_I64, 1), ("B", abi.F_U64, 1), ("C", abi.F_BOOL, 1), ("x", abi.F_F64, 1)])
+    text = b.schema([("s", abi.F_STR, 1), ("y", abi.F_I64, 1)])
+    if long_names:
+        for k in range(200):
+            b.s("s%d" % k)
+    values = [7, 12, 34567, 1, struct.unpack("<Q", struct.pack("<d", -1.2345678901234567e-300))[0], names[7], 3, 1 << 62]
+    b.arg_slots(values)
+    sp = b.build()
+    rec = np.zeros(n, dtype=np.dtype(abi.GenericRec))
+    k = np.arange(n)
+    rec["start_ns"] = B + 1000 + 777 * k
+    rec["end_ns"] = rec["start_ns"] + rng.integers(0, 100000, n)
+    rec["resource"] = 5 + k // 37 % 5
+    rec["device"] = 4242
+    rec["id"] = k + 1
+    rec["name_id"] = np.array(names)[rng.integers(0, len(names), n)]
+    if long_names:
+        rec["name_id"] = np.where(k % 8 != 0, names[8], rec["name_id"])
+    kind = rng.integers(0, 4, n)
+    rec["schema_id"] = np.array([abi.KTJ_NONE, plain, wide, text], dtype=np.uint32)[kind]
+    rec["args_off"] = np.array([0, 0, 1, 5])[kind]
+    flow = rng.integers(0, 3, n)
+    rec["flow_id"], rec["flow_type"], rec["flags"] = np.where(flow, k + 1, 0), 1, flow == 1
+    place = np.empty(n, dtype=np.int64)
+    place[np.lexsort((rec["start_ns"], rec["resource"]))] = k   # of each in the document
+    left = np.isin(place % 800, (0, 15, 16, 17, 399)) | (place == n - 1) | (rng.integers(0, 200, n) == 0)
+    if left_known:
+        rec["end_ns"] = np.where(left, rec["start_ns"] + 10**10, rec["end_ns"])
+    else:
+        rec["schema_id"] = np.where(left, plain, rec["schema_id"])
+        rec["args_off"] = np.where(left, 7, rec["args_off"])
+    assert 0 < left.sum() * 32 < n
+    held = (abi.GenericRec * n).from_buffer_copy(rec.tobytes())
+    sp.contents.generic, sp.contents.n_generic = C.cast(held, type(sp.contents.generic)), n
+    sp.held = held
+    return sp, int(left.sum())
+
+
 def _gpu_vs_oracle(sp, passes=3):
     """Through the large passes whatever the size, several times from one engine; what each says of itself (KTJ_DBG_PASS)."""
     from kineto_amd.engine import TraceEngine
@@ -312,6 +361,47 @@ def test_documents_with_one_row_left():
         print(name, flush=True)
         n = sp.contents.n_generic + sp.contents.n_runtime + sp.contents.n_device
         assert _gpu_vs_oracle(sp) == [[1, 1, n, 0]] + 2 * [[0, 0, 0, 0]], name
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", (65537, 70000, 262144))
+def test_several_turns_with_rows_left(n):
+    """Few enough activities that any left make the next pass one without text rows; woven in the first."""
+    sp, left = large_stream(n, False)
+    assert _gpu_vs_oracle(sp, passes=2) == [[1, 0, left, 0], [0, 0, 0, 0]]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n, left_known, long_names", ((262145, True, False), (300007, False, False), (300007, True, True)))
+def test_many_turns_with_few_rows_left(n, left_known, long_names):
+    """Woven in every pass, the others behind; with long names the list of these is made twice in the first pass."""
+    sp, left = large_stream(n, left_known, long_names)
+    assert _gpu_vs_oracle(sp) == 3 * [[1, 0, left, 0]]
+
+
+@pytest.mark.gpu
+def test_rows_left_that_no_pass_before_had():
+    """Behind a wait of their own: the engine's last pass had none."""
+    from kineto_amd.engine import TraceEngine
+    sp, left = large_stream(300007, False)
+    n, few = sp.contents.n_generic, 3000
+    o = og.OracleRun(sp)
+    want = o.output()
+    o.close()
+    size = C.sizeof(abi.GenericRec)
+    records = C.string_at(sp.contents.generic, n * size)
+    first = [k for k in range(few) if abi.GenericRec.from_buffer_copy(records, k * size).args_off != 7]
+    then = sorted(set(range(n)) - set(first))
+    halves = [(abi.GenericRec * len(x)).from_buffer_copy(b"".join(records[k * size:(k + 1) * size] for k in x)) for x in (first, then)]
+    sp.contents.generic, sp.contents.n_generic = C.cast(halves[0], type(sp.contents.generic)), len(first)
+    with TraceEngine(sp.contents.trace_name.decode()) as e:
+        e.submit_stream(sp)
+        e.process()
+        assert [int(x) for x in e.debug("pass_info")] == [1, 0, 0, 0]
+        e._chk(abi.load_engine().ktj_submit_records(e.h, abi.REC_GENERIC, halves[1], len(then)), "ktj_submit_records")
+        e.process()
+        assert [int(x) for x in e.debug("pass_info")] == [1, 0, left, 1]
+        assert e.output() == want
 
 
 @pytest.mark.gpu
