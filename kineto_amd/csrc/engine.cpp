@@ -171,7 +171,7 @@ struct HostCtl {
   Scalars scalars;
   uint64_t act_bytes;
   uint32_t n_out;
-  uint32_t pad;
+  uint32_t weave;                                  /* plan_tables: KTJ_WEAVE_* of this pass */
   uint64_t end_clock;
   alignas(128) uint64_t part_flag[KTJ_PART_SLOTS]; /* copy_parts: what the slots hold */
 };
@@ -239,7 +239,7 @@ struct ktj_engine {
   DevBuf keys_a, keys_b, vals_a, vals_b, hist, scan_tmp;
   bool rows_are_text = false;              /* of the last pass: TextRows in mat */
   uint64_t not_woven = 0;                  /* number of these records with which a woven pass left too many activities (too_many_left) */
-  bool some_left = true;                   /* the last pass had activities that the weaver leaves to emit_direct; not known before the first */
+  int some_left = -1;                      /* the last woven pass had activities that the weaver leaves to emit_direct (1, 0; -1: there was none) */
   uint64_t pass_info[4] = {};              /* of the last pass (KTJ_DBG_PASS) */
   DevBuf mat, schema_book, wide_text, len, len_sorted, kind_sorted, offs, out, tile_start;
   void* pinned_small = nullptr; size_t pinned_small_cap = 0;
@@ -1594,7 +1594,8 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
   Table t_cpu{e->t_cpu.as<uint64_t>(), cap_cpu - 1, 1u, &sc->plan.ctl[KTJ_TBL_CPU]};
   FullCols fc{e->f_has_runtime.as<uint32_t>(), e->f_first.as<uint32_t>(), e->f_stream_src.as<uint32_t>(), e->f_pay.as<FullPay>()};
   NarrowCols nc{e->n_ext_src.as<uint32_t>(), e->n_kern_src.as<uint32_t>(), e->n_copy_src.as<uint32_t>(), e->n_pay.as<NarrowPay>()};
-  HIPCHK(plan_tables(tf, fc, tn, nc, t_cpu, (e->flags & KTJ_CREATE_HASH_JOIN) != 0, woven ? ng + nr + nd : 0u, sc, st));
+  e->h_ctl->weave = KTJ_WEAVE_UNKNOWN;
+  HIPCHK(plan_tables(tf, fc, tn, nc, t_cpu, (e->flags & KTJ_CREATE_HASH_JOIN) != 0, woven ? ng + nr + nd : 0u, &e->h_ctl_dev->weave, sc, st));
   ApiTable api{e->d_cid_names.as<uint32_t>(), (uint32_t)e->cid_names.size(), e->d_flow_bits.as<uint32_t>(), e->malloc_cid};
   weave::SchemaBook* book = woven ? e->schema_book.as<weave::SchemaBook>() : nullptr;
   const Rows rows{e->mat.p, book, wide ? e->wide_text.as<weave::WideText>() : nullptr};
@@ -1638,8 +1639,8 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
   const bool straight = has_room && n_coll == 0 && max_spans == 0 && !e->stepwise && !(e->flags & KTJ_CREATE_TILE_EMIT) && e->sort_mode != 1;
   HIPCHK(collect_distinct(c, N, sets, sc, straight, ctx, book, st));
   /* The document's activities, but for the tile variant: what the weaver prints, and at most n_left others. */
-  auto put_activities = [&](uint64_t n_most, uint64_t n_left, uint64_t at) -> int {
-    if (woven && n_most)
+  auto put_activities = [&](uint64_t n_most, uint64_t n_left, uint64_t at, bool weave = true) -> int {
+    if (woven && n_most && weave)
       HIPCHK(weave_activities(e->mat.as<weave::TextRow>(), e->perm, e->offs.as<uint64_t>(), e->kind_sorted.as<uint8_t>(), n_most, ctx, e->out.as<char>(), at, sc, book, rows.wide, st));
     HIPCHK(emit_direct(rows.p, e->perm, e->offs.as<uint64_t>(), e->kind_sorted.as<uint8_t>(), woven ? n_left : n_most, ctx, e->out.as<char>(), at, sc, left(), st));
     return KTJ_OK;
@@ -1668,12 +1669,13 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
       text.out = e->out.as<char>(); text.out_cap = e->out.cap;
       HIPCHK(gather_offsets(e->perm, e->len.as<uint32_t>(), N, e->len_sorted.as<uint32_t>(), e->kind_sorted.as<uint8_t>(),
                             e->scan_tmp.as<uint64_t>(), e->offs.as<uint64_t>(), left(), sc, text, st));
-      /* Mostly there are no others, and a launch that finds its list empty takes 4 us, 20 with 22 million rows: it is left out where
-       * the last pass had none.  The first pass of an engine, a session's only one mostly, makes it: without it 30 000 records with one
-       * number too long for its row took 218 us instead of 203, with a row known to be left 217 instead of 203, without any 176
-       * instead of 180. */
-      const bool others = e->some_left;
-      { const int rc = put_activities(N, others ? N : 0u, prefix.size()); if (rc != KTJ_OK) return rc; }
+      /* Mostly there are no others, and a launch that finds its list empty takes 4 us, 20 with 22 million rows.  What k_decode
+       * has counted is here by now, unless the trace is so large that such a launch does not matter; others that it cannot
+       * know of are printed behind a wait of their own the first time.  (No look at the count: 30 000 records of which some are left
+       * 217 instead of 200 us; the launch in every first pass: 180 instead of 176 us with none left.) */
+      const uint32_t counted = woven ? __atomic_load_n(&e->h_ctl->weave, __ATOMIC_ACQUIRE) : (uint32_t)KTJ_WEAVE_UNKNOWN;
+      const bool others = counted >= KTJ_WEAVE_MOST || (counted == KTJ_WEAVE_ALL ? e->some_left > 0 : e->some_left != 0);
+      { const int rc = put_activities(N, others ? N : 0u, prefix.size(), counted != KTJ_WEAVE_NONE); if (rc != KTJ_OK) return rc; }
       HIPCHK(hipEventRecord(e->ev[EV_EMIT], st));
       HIPCHK(hipStreamSynchronize(st));
       e->scalars = e->h_ctl->scalars;
@@ -1684,7 +1686,7 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
       emitted = e->total_bytes + 64 <= text.out_cap;
       if (emitted) {
         const uint64_t n_left = was_woven();
-        if (woven) e->some_left = n_left != 0;
+        if (woven) e->some_left = n_left != 0 ? 1 : 0;
         if (n_left != 0 && !others) {
           e->pass_info[3] = 1;
           { const int rc = put_activities(0, n_left, prefix.size()); if (rc != KTJ_OK) return rc; }

@@ -259,8 +259,10 @@ hipError_t decode(DecodeJob job, Columns c, EmitCtx ctx, Scalars* sc, hipStream_
 
 /* ---- stage 2b: joins ---- */
 /* the tables' modes (direct unless force_hash or the span of their keys is too wide), and all of them cleared */
-/* n_rows: of all classes, in a pass that makes text rows (0: it makes none) */
-hipError_t plan_tables(Table tf, FullCols fc, Table tn, NarrowCols nc, Table cpu, bool force_hash, uint64_t n_rows, Scalars* sc, hipStream_t st);
+/* n_rows: of all classes, in a pass that makes text rows (0: it makes none); h_weave: page-locked, what k_decode has counted for the
+ * weaver (KTJ_WEAVE_*) */
+enum { KTJ_WEAVE_UNKNOWN = 0, KTJ_WEAVE_ALL, KTJ_WEAVE_MOST, KTJ_WEAVE_NONE };
+hipError_t plan_tables(Table tf, FullCols fc, Table tn, NarrowCols nc, Table cpu, bool force_hash, uint64_t n_rows, uint32_t* h_weave, Scalars* sc, hipStream_t st);
 /* Whether the weaver prints nothing where it would leave n_left of n activities.  Each that it leaves ends what it
  * has begun (a fifth of 120 000 CPU ops instant events: k_weave 43 us instead of 25), and the second launch takes 11 us and more;
  * from 300 000 activities on it gains more than that as long as it leaves few. */

@@ -538,7 +538,7 @@ __device__ __forceinline__ void clear_keys(const Table& t, const TableSpan& s, u
   if (at == 0) t.keys[t.mask + 1ull] = KTJ_EMPTY_KEY;
 }
 __global__ void __launch_bounds__(KTJ_BLOCK)
-k_plan_clear(Scalars* sc, Table tf, FullCols fc, Table tn, NarrowCols nc, Table cpu, int force_hash, uint64_t n_rows) {
+k_plan_clear(Scalars* sc, Table tf, FullCols fc, Table tn, NarrowCols nc, Table cpu, int force_hash, uint64_t n_rows, uint32_t* h_weave) {
   __shared__ TableCtl ctl[3];
   if (blockIdx.x == 0 && threadIdx.x == 0) stage_clock(sc, KTJ_CLOCK_JOIN);
   if (threadIdx.x < 64) {
@@ -562,7 +562,11 @@ k_plan_clear(Scalars* sc, Table tf, FullCols fc, Table tn, NarrowCols nc, Table 
     if (blockIdx.x == 0 && n_rows != 0) {
       uint32_t n = (uint32_t)sc->shard[threadIdx.x][KTJ_CNT_NOT_TEXT];
       for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o);
-      if (threadIdx.x == 0) sc->no_text = too_many_left(n, n_rows) ? 1u : 0u;
+      if (threadIdx.x == 0) {
+        const bool none = too_many_left(n, n_rows);
+        sc->no_text = none ? 1u : 0u;
+        __hip_atomic_store(h_weave, (uint32_t)(none ? KTJ_WEAVE_NONE : n ? KTJ_WEAVE_MOST : KTJ_WEAVE_ALL), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      }
     }
   }
   __syncthreads();
@@ -587,12 +591,12 @@ k_plan_clear(Scalars* sc, Table tf, FullCols fc, Table tn, NarrowCols nc, Table 
     nc.ext_src[k] = 0; nc.kern_src[k] = 0; nc.copy_src[k] = 0; nc.pay[k] = z;
   }
 }
-hipError_t plan_tables(Table tf, FullCols fc, Table tn, NarrowCols nc, Table cpu, bool force_hash, uint64_t n_rows, Scalars* sc, hipStream_t st) {
+hipError_t plan_tables(Table tf, FullCols fc, Table tn, NarrowCols nc, Table cpu, bool force_hash, uint64_t n_rows, uint32_t* h_weave, Scalars* sc, hipStream_t st) {
   uint64_t most = (uint64_t)tf.mask + 1;
   if ((uint64_t)tn.mask + 1 > most) most = (uint64_t)tn.mask + 1;
   if ((uint64_t)cpu.mask + 1 > most) most = (uint64_t)cpu.mask + 1;
   const unsigned g = grid_stride_for(most, KTJ_BLOCK * 4);
-  hipLaunchKernelGGL(k_plan_clear, dim3(g < 2048u ? g : 2048u), dim3(KTJ_BLOCK), 0, st, sc, tf, fc, tn, nc, cpu, force_hash ? 1 : 0, n_rows);
+  hipLaunchKernelGGL(k_plan_clear, dim3(g < 2048u ? g : 2048u), dim3(KTJ_BLOCK), 0, st, sc, tf, fc, tn, nc, cpu, force_hash ? 1 : 0, n_rows, h_weave);
   return KTJ_LAUNCH_CHECK();
 }
 
