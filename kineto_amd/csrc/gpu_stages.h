@@ -264,8 +264,9 @@ hipError_t decode(DecodeJob job, Columns c, EmitCtx ctx, Scalars* sc, hipStream_
 enum { KTJ_WEAVE_UNKNOWN = 0, KTJ_WEAVE_ALL, KTJ_WEAVE_MOST, KTJ_WEAVE_NONE };
 hipError_t plan_tables(Table tf, FullCols fc, Table tn, NarrowCols nc, Table cpu, bool force_hash, uint64_t n_rows, uint32_t* h_weave, Scalars* sc, hipStream_t st);
 /* Whether the weaver prints nothing where it would leave n_left of n activities.  Each that it leaves ends what it
- * has begun (a fifth of 120 000 CPU ops instant events: k_weave 43 us instead of 25), and the second launch takes 11 us and more;
- * from 300 000 activities on it gains more than that as long as it leaves few. */
+ * has begun (a fifth of 120 000 CPU ops instant events: k_weave 43 us instead of 25), and the launch for these is never shorter
+ * than 30 us, however few.  Passes of 100 000 / 260 000 / 733 000 / 3 million records with one of them left: woven 266 / 315 / 587 /
+ * 1280 us, not woven 254 / 302 / 590 / 1565. */
 #define KTJ_FEW_ACTIVITIES 262144u
 static inline __host__ __device__ bool too_many_left(uint64_t n_left, uint64_t n) { return n_left != 0 && (n <= KTJ_FEW_ACTIVITIES || n_left * 32u > n); }
 hipError_t build_cpu_ids(const ktj_generic_rec* g, uint64_t n, Table cpu, uint32_t* cpu_row, Scalars* sc, hipStream_t st);

@@ -459,7 +459,7 @@ __global__ void __launch_bounds__(KTJ_BLOCK) k_decode(DecodeJob J, Columns c, Em
     bool left = false;
     if (has) {
       const RowCols r = cols_generic(l[threadIdx.x], ctx);
-      left = J.text && (r.meta & KTJ_M_VALID) && weave::left_generic(l[threadIdx.x], r.dev, ctx, J.schemas_not_taken);
+      left = J.text && (r.meta & KTJ_M_VALID) && (weave::left_generic(l[threadIdx.x], r.dev, ctx, J.schemas_not_taken) || weave::far_apart(l[threadIdx.x].start_ns, l[0].start_ns));
       store_cols(c, J.first + b * KTJ_BLOCK + threadIdx.x, r);
     }
     /* rows that may need a Stream Sync row of their own are rare: the extra passes run only if any */
@@ -477,7 +477,7 @@ __global__ void __launch_bounds__(KTJ_BLOCK) k_decode(DecodeJob J, Columns c, Em
     if (has) {
       const RowCols r = cols_runtime(l[threadIdx.x], J.clk, J.win_start, J.win_end);
       oor = !(r.meta & KTJ_M_VALID);
-      left = J.text && !oor && weave::left_runtime(l[threadIdx.x], r.ts, r.dur, ctx);
+      left = J.text && !oor && (weave::left_runtime(l[threadIdx.x], r.ts, r.dur, ctx) || weave::far_apart(l[threadIdx.x].begin, l[0].begin));
       store_cols(c, J.ng + b * KTJ_BLOCK + threadIdx.x, r);
     }
     block_add_two(sc, KTJ_CNT_OUT_OF_RANGE, oor, KTJ_CNT_NOT_TEXT, left);
@@ -494,7 +494,7 @@ __global__ void __launch_bounds__(KTJ_BLOCK) k_decode(DecodeJob J, Columns c, Em
       const uint64_t i = b * KTJ_BLOCK + threadIdx.x;
       const RowCols r = cols_device(*d, J.clk, J.win_start, J.win_end);
       oor = !(r.meta & KTJ_M_VALID);
-      left = J.text && !oor && weave::left_device(*d, r.ts, r.dur, r.res, ctx);
+      left = J.text && !oor && (weave::left_device(*d, r.ts, r.dur, r.res, ctx) || weave::far_apart(d->begin, l[0].begin));
       store_cols(c, J.ng + J.nr + i, r);
       DevBrief br;
       br.queue = d->queue; br.device = d->device; br.domain = device_row_domain(d->domain);

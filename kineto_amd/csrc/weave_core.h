@@ -442,6 +442,9 @@ inline uint32_t schemas_not_taken(const ktj_field* fields, const ktj_schema_desc
 KTJ_HD KTJ_FI inline bool left_by_track(int64_t dev, int64_t res, int64_t rel_ns, int64_t dur) {
   return ((uint64_t)dev >> KTJ_TR_DEV_BITS) != 0 || ((uint64_t)res >> 47) != 0 || rel_ns >= (int64_t)(65536u * KTJ_LEAD_UNIT * 1000u) || dur >= 10000000000ll;
 }
+/* Times so far apart that their leads differ.  Where that is so for the rows of a workgroup, nearly every row ends the run of
+ * the one before it, and k_emit_direct is the better one (10 000 CPU ops over 2^61 ns: 271 us a pass instead of 301). */
+KTJ_HD KTJ_FI inline bool far_apart(uint64_t a, uint64_t b) { const uint64_t d = a - b; return (d < 0ull - d ? d : 0ull - d) >= KTJ_LEAD_UNIT * 1000u; }
 KTJ_HD KTJ_FI inline bool left_by_three(uint32_t a, uint32_t b, uint32_t c) { /* three_text_of: eleven digits together */
   if (a < 100000u && b < 1000u && c < 1000u) return false;
   return b >= 1000000u || c >= 1000000u || ndigits_u64(a) + ndigits_u64(b) + ndigits_u64(c) > 11;

@@ -409,6 +409,20 @@ def test_rows_left_that_no_pass_before_had():
 
 
 @pytest.mark.gpu
+def test_times_with_a_lead_each_are_not_woven():
+    """Nearly every activity would end the run of its neighbours; a few that do (a row at time 0) do not matter to many."""
+    b = StreamBuilder(base=0, window=(0, 1 << 62), host_name="apart")
+    for k in range(700):
+        b.add_generic("op", 0, (k << 61) // 700, ((k << 61) // 700) + 5, 1, 5, id=k + 1)
+    assert _gpu_vs_oracle(b.build(), passes=2) == [[1, 1, 700, 0], [0, 0, 0, 0]]
+    sp, left = large_stream(300007, False)
+    rec = (abi.GenericRec * sp.contents.n_generic).from_address(C.addressof(sp.contents.generic.contents))
+    for k in (1, 2, 999, 200001):
+        rec[k].start_ns, rec[k].end_ns = 0, 17
+    assert [x[:3] for x in _gpu_vs_oracle(_base_back(sp, B), passes=2)] == 2 * [[1, 0, left, ]]
+
+
+@pytest.mark.gpu
 def test_other_records_are_woven_again():
     """That a pass left too many is known of its records and not of others that are as many."""
     import torch
