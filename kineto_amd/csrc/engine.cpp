@@ -1582,7 +1582,7 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
     job.ng = ng; job.nr = nr; job.nd = nd; job.nx = nx;
     job.whole_pass = true;
     job.text = woven;
-    job.schemas_not_taken = e->schemas_not_taken;
+    job.schemas_not_taken = e->schemas_not_taken; job.n_cids = (uint32_t)e->cid_names.size();
     job.brief = e->dev_brief.as<DevBrief>();
     job.clk = clock_of(e); job.win_start = e->win_start; job.win_end = e->win_end;
     HIPCHK(decode(job, c, ctx, sc, st));

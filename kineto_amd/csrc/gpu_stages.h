@@ -249,7 +249,7 @@ struct DecodeJob {
   uint64_t first;            /* arrival index of the first generic record; runtime and device rows follow ng records */
   bool whole_pass;           /* false: generic records made during the pass, which are in no table */
   bool text;                 /* a pass that makes text rows: those that will be none are counted, as far as their records say so */
-  uint32_t schemas_not_taken;
+  uint32_t schemas_not_taken, n_cids;
   DevBrief* brief;
   ClockDev clk;
   int64_t win_start, win_end;

@@ -477,7 +477,7 @@ __global__ void __launch_bounds__(KTJ_BLOCK) k_decode(DecodeJob J, Columns c, Em
     if (has) {
       const RowCols r = cols_runtime(l[threadIdx.x], J.clk, J.win_start, J.win_end);
       oor = !(r.meta & KTJ_M_VALID);
-      left = J.text && !oor && (weave::left_runtime(l[threadIdx.x], r.ts, r.dur, ctx) || weave::far_apart(l[threadIdx.x].begin, l[0].begin));
+      left = J.text && !oor && (weave::left_runtime(l[threadIdx.x], r.ts, r.dur, ctx, J.n_cids) || weave::far_apart(l[threadIdx.x].begin, l[0].begin));
       store_cols(c, J.ng + b * KTJ_BLOCK + threadIdx.x, r);
     }
     block_add_two(sc, KTJ_CNT_OUT_OF_RANGE, oor, KTJ_CNT_NOT_TEXT, left);

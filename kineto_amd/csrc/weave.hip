@@ -239,7 +239,8 @@ k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const u
     const v4u32 z = {q0.x, q0.y, q0.z & 0xFFFFFFu, KTJ_TR_COUNT(q0.z) << 24};
     vals[S_Z - 1u + h] = __builtin_bit_cast(v2u64, z);
     {
-      const v4u32 a = {q1.x, q1.y & 0xFFFFFFu, 0u, q1.y & 0xFF000000u}, x = h == 0u ? a : q1;
+      const uint32_t on = (q1.y >> 24) > KTJ_TR_A_NEAR ? more : 0u; /* (of the first lane) */
+      const v4u32 a = {q1.x, (q1.y & 0xFFFFFFu) | (on << 24), on >> 8, q1.y & 0xFF000000u}, x = h == 0u ? a : q1;
       vals[S_A - 1u + h] = __builtin_bit_cast(v2u64, x);
     }
     /* how many segments and parts, and the room for the name (the first lane) */

@@ -24,7 +24,7 @@ namespace weave {
  * in the last byte.  Activities with longer ones are left to format_activity. */
 enum : uint32_t {
   S_NONE = 0,
-  S_A,                             /* cid, or queue, or context */
+  S_A,                             /* cid, or queue, or context, or the fourth of a schema's numbers */
   S_TS,
   S_X, S_Y,                        /* grid and block ("a, b, c"), addresses, or bytes; a double of up to 24 characters: S_Y and S_Z */
   S_Z,                             /* shared memory or bytes */
@@ -38,7 +38,9 @@ enum : uint32_t {
 
 /* A joined row as the size pass leaves it for the weaver: a line of eight blocks of sixteen bytes.  Most numbers are
  * short: S_Z, S_EXT, S_FLOW and S_DUR have twelve bytes (eleven characters) of the first four blocks, whose last words are
- * plan, name, lens and more; S_A has eight of the fifth, in front of the track; the others a block each.
+ * plan, name, lens and more; S_A has eight of the fifth (seven characters), in front of the track, and where there is nothing else
+ * for it four more in the word for more (the sequence number of an operator is the fourth number of its schema, and a long job
+ * has more than 10 million of them); the others a block each.
  *
  * A time has eighteen characters and more where the base lies months behind (libkineto floors it to 91 days) or at 0, more than
  * S_TS has.  What is above 10^11 us (28 hours) is the same for nearly all rows: that number, the time's lead, is printed once
@@ -57,7 +59,8 @@ struct alignas(16) WideText { uint64_t w[4]; };
 #define KTJ_TR_PLAN 0u             /* KTJ_TR_*, the thread's bits from 42 on */
 #define KTJ_TR_NAME 1u             /* place of the name in its blob, in units of sixteen bytes */
 #define KTJ_TR_LENS 2u             /* its length; << 16: that of the string or double between the args' parts; KTJ_TR_HAS_LEAD */
-#define KTJ_TR_MORE 3u             /* the string's place in its blob; the WideText's number; a copy's kind as text */
+#define KTJ_TR_MORE 3u             /* the string's place in its blob; the WideText's number; a copy's kind as text; S_A's eighth character and the following */
+#define KTJ_TR_A_NEAR 7u           /* characters of S_A in its block */
 static_assert(KTJ_WEAVE_MAX_RUN < 0x8000u, "a length and a bit");
 static_assert(sizeof(TextRow) == 128 && sizeof(TextRow) >= sizeof(MatRow), "a row that is left to format_activity is a MatRow in the same place");
 /* a row of the other kind: the last byte, S_Y's count of characters otherwise */
@@ -436,8 +439,7 @@ inline uint32_t schemas_not_taken(const ktj_field* fields, const ktj_schema_desc
 
 /* ---- records that text_row will refuse, as far as their own numbers say so; for rows inside the capture window.  What it does
  * not say: names beyond KTJ_WEAVE_MAX_RUN, the values of typed arguments, keys, what a device row takes over from a runtime row
- * (counted there), leads beside tracks of many digits ---- */
-#define KTJ_SEVEN_DIGITS 10000000ull
+ * (counted there), API numbers with no name in the table, leads beside tracks of many digits ---- */
 #define KTJ_ELEVEN_DIGITS 100000000000ull
 KTJ_HD KTJ_FI inline bool left_by_track(int64_t dev, int64_t res, int64_t rel_ns, int64_t dur) {
   return ((uint64_t)dev >> KTJ_TR_DEV_BITS) != 0 || ((uint64_t)res >> 47) != 0 || rel_ns >= (int64_t)(65536u * KTJ_LEAD_UNIT * 1000u) || dur >= 10000000000ll;
@@ -464,8 +466,8 @@ KTJ_HD KTJ_FI inline bool left_generic(const ktj_generic_rec& g, int64_t dev, co
   return (flow && (wider || (uint64_t)m.flow_id >= KTJ_ELEVEN_DIGITS)) || args ||
          left_by_track(dev, (int64_t)sanitize_tid(m.res), m.ts - c.base_time_ns, m.dur + (wider ? 2 : 0));
 }
-KTJ_HD KTJ_FI inline bool left_runtime(const ktj_runtime_rec& r, int64_t ts, int64_t dur, const EmitCtx& c) {
-  bool left = r.cid >= KTJ_SEVEN_DIGITS || r.id >= KTJ_ELEVEN_DIGITS || left_by_track((int64_t)r.pid, (int64_t)sanitize_tid((int64_t)r.tid), ts - c.base_time_ns, dur);
+KTJ_HD KTJ_FI inline bool left_runtime(const ktj_runtime_rec& r, int64_t ts, int64_t dur, const EmitCtx& c, uint32_t n_cids) { /* (beyond them an API has no name) */
+  bool left = r.cid >= n_cids || r.id >= KTJ_ELEVEN_DIGITS || left_by_track((int64_t)r.pid, (int64_t)sanitize_tid((int64_t)r.tid), ts - c.base_time_ns, dur);
   if (r.kind == KTJ_RT_KERNEL)
     left = left || left_by_three(r.u.kernel.grid[0], r.u.kernel.grid[1], r.u.kernel.grid[2]) ||
            left_by_three(r.u.kernel.workgroup[0], r.u.kernel.workgroup[1], r.u.kernel.workgroup[2]);
@@ -476,8 +478,10 @@ KTJ_HD KTJ_FI inline bool left_runtime(const ktj_runtime_rec& r, int64_t ts, int
   return left;
 }
 KTJ_HD KTJ_FI inline bool left_device(const ktj_device_rec& d, int64_t ts, int64_t dur, int64_t res, const EmitCtx& c) {
-  const bool memset_row = device_row_domain(d.domain) == KTJ_DOM_MEMSET;
-  return (memset_row && (c.create_flags & KTJ_CREATE_CUDA12_ARGS)) || (memset_row ? d.queue & 0xFFFFFFFFull : d.queue) >= KTJ_SEVEN_DIGITS || d.id >= KTJ_ELEVEN_DIGITS ||
+  const uint32_t domain = device_row_domain(d.domain);
+  const bool memset_row = domain == KTJ_DOM_MEMSET;
+  return (memset_row && (c.create_flags & KTJ_CREATE_CUDA12_ARGS)) || (!memset_row && d.queue >= KTJ_ELEVEN_DIGITS) ||
+         (domain == KTJ_DOM_KERNEL_DISPATCH && d.name_id == KTJ_NONE) || d.id >= KTJ_ELEVEN_DIGITS ||
          left_by_track((int64_t)d.device, res, ts - c.base_time_ns, dur);
 }
 
@@ -684,16 +688,19 @@ KTJ_HD KTJ_FI inline bool text_row(const MatRow& m, const EmitCtx& c, const Sche
   if ((tid >> 47) != 0 || (device && m.res < 0)) return false;
   if (type >= 29u || (generic && (type == KTJ_TYPE_CPU_INSTANT_EVENT || is_counter_type(type)))) return false;
   if ((meta & KTJ_M_SYNC) || (type == KTJ_TYPE_GPU_USER_ANNOTATION && flow) || collective_of(m) != 0) return false;
-  bool fits = true;
+  bool fits = true, a_long = false;
   auto block = [&](uint32_t slot) KTJ_FI { return r->w[KTJ_TR_BLOCK(slot) ^ turn]; };
   typedef uint64_t __attribute__((may_alias)) word_pair;
   auto two = [](uint32_t* w, uint64_t x) KTJ_FI { *reinterpret_cast<word_pair*>(w) = x; }; /* (eight-byte aligned) */
   auto put = [&](uint32_t slot, const Text& t) KTJ_FI {
     uint32_t* const w = block(slot);
-    const uint32_t most = slot == S_A ? 7u : slot >= S_Z ? 11u : 15u;
+    const uint32_t most = slot == S_A || slot >= S_Z ? 11u : 15u;
     fits = fits && t.n <= most;
-    if (slot == S_A) two(w, t.lo | ((uint64_t)t.n << 56));
-    else {
+    if (slot == S_A) {
+      two(w, (t.lo & 0xFFFFFFFFFFFFFFull) | ((uint64_t)t.n << 56));
+      a_long = t.n > KTJ_TR_A_NEAR;
+      if (a_long) block(S_DUR)[3] = (uint32_t)(t.lo >> 56) | ((uint32_t)t.hi << 8);
+    } else {
       two(w, t.lo);
       if (slot >= S_Z) w[2] = (uint32_t)t.hi | (t.n << 24);
       else two(w + 2, t.hi | ((uint64_t)t.n << 56));
@@ -866,7 +873,8 @@ KTJ_HD KTJ_FI inline bool text_row(const MatRow& m, const EmitCtx& c, const Sche
     block(S_FLOW)[3] = name_len | (len1 << 16) | KTJ_TR_HAS_LEAD;
     for (uint32_t k = 0; k < 4u; ++k) { uint32_t* const w = &block(S_Z + k)[2]; *w = (*w & 0x0FFFFFFFu) | ((lead >> (4u * k)) << 28); }
   }
-  block(S_DUR)[3] = at_more;
+  if (!a_long) block(S_DUR)[3] = at_more;
+  else fits = fits && (between & 1u) == 0 && args != A_COPY; /* (nothing else is there) */
   two(block(S_A) + 2, (uint64_t)m.dev | (tid << KTJ_TR_DEV_BITS));
   *len = n + name_len + len1;
   *tail = flow ? (meta & KTJ_M_FLOW_START ? 0u : 2u) : close ? 1u : 0u;

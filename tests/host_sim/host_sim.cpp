@@ -100,7 +100,11 @@ std::string woven_text(const weave::TextRow& row, const weave::WideText* wide, c
   std::string out;
   auto number = [&](uint32_t slot) -> std::string {
     const uint32_t* w = row.w[KTJ_TR_BLOCK(slot)];
-    if (slot == S_A) return std::string(reinterpret_cast<const char*>(w), w[1] >> 24);
+    if (slot == S_A) {
+      const uint32_t n = w[1] >> 24, more = row.w[KTJ_TR_MORE][3];
+      const std::string near(reinterpret_cast<const char*>(w), std::min(n, KTJ_TR_A_NEAR));
+      return n > KTJ_TR_A_NEAR ? near + std::string(reinterpret_cast<const char*>(&more), n - KTJ_TR_A_NEAR) : near;
+    }
     return std::string(reinterpret_cast<const char*>(w), slot >= S_Z ? KTJ_TR_COUNT(w[2]) : w[3] >> 24);
   };
   const uint32_t plan = row.w[KTJ_TR_PLAN][3], lens = row.w[KTJ_TR_LENS][3], more = row.w[KTJ_TR_MORE][3], name = row.w[KTJ_TR_NAME][3];
@@ -454,7 +458,7 @@ int ktjsim_render(const ktj_stream* s, uint32_t tile_bytes, char** out, uint64_t
       const MatRow& m = mat[perm[i]];
       const uint64_t a = perm[i];
       const bool known = a < ng ? weave::left_generic(s->generic[a], m.dev, ctx, not_taken)
-                       : a < ng + nr ? weave::left_runtime(s->runtime[a - ng], m.ts, m.dur, ctx)
+                       : a < ng + nr ? weave::left_runtime(s->runtime[a - ng], m.ts, m.dur, ctx, (uint32_t)s->n_cids)
                        : a < ng + nr + nd && weave::left_device(s->device[a - ng - nr], m.ts, m.dur, m.res, ctx);
       n_left_known += known;
       weave::TextRow row;

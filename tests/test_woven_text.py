@@ -220,8 +220,8 @@ def _odd_streams():
         runtime_duration=lambda b: runtime(b, end=t + 10**10), correlation=lambda b: runtime(b, id=10**11),
         grid=lambda b: runtime(b, kind=1, grid=(999999, 999, 999)), block=lambda b: runtime(b, kind=1, grid=(1, 1, 1), workgroup=(1, 1000000, 1)),
         address=lambda b: runtime(b, cid=1, kind=2, src=1 << 60), size=lambda b: runtime(b, cid=1, kind=2, size=10**11), copy_kind=lambda b: runtime(b, cid=1, kind=2, copy_kind=-1000),
-        pointer=lambda b: runtime(b, cid=2, kind=3, ptr=1 << 60), device_duration=lambda b: device(b, end=t + 1 + 10**10, name="k"), queue=lambda b: device(b, queue=10**7, name="k"),
-        device_correlation=lambda b: device(b, id=10**11, name="k"), context=lambda b: b.add_memset(9, t, t + 5, context=10**7))
+        pointer=lambda b: runtime(b, cid=2, kind=3, ptr=1 << 60), device_duration=lambda b: device(b, end=t + 1 + 10**10, name="k"), queue=lambda b: device(b, queue=10**11, name="k"),
+        device_correlation=lambda b: device(b, id=10**11, name="k"), api=lambda b: runtime(b, cid=3), kernel_without_name=device)
     for name, edit in edits.items():
         b = base()
         edit(b)
@@ -240,6 +240,26 @@ def test_rows_left_are_known_when_decoded(sim):
         assert (_woven_vs_oracle(sim, sp)[1], sim.ktjsim_left_known()) == (1, 1), name
     _woven, left = _woven_vs_oracle(sim, edge_stream(3000))
     assert left * 0.6 < sim.ktjsim_left_known() < left
+
+
+def test_long_jobs(sim):
+    """What grows with a job is text however long it has run: the fourth number of its operators' schema (the sequence number), and
+    the queues."""
+    def stream(n):
+        b = StreamBuilder(window=(B, B + 10**13), host_name="long")
+        op = b.schema([("Ev Idx", abi.F_I64, 1), ("Record function id", abi.F_U64, 1), ("Fwd thread id", abi.F_U64, 1), ("Sequence number", abi.F_I64, 1)])
+        string = b.schema([("a", abi.F_I64, 1), ("b", abi.F_I64, 1), ("c", abi.F_I64, 1), ("d", abi.F_I64, 1), ("s", abi.F_STR, 1)])
+        t = B + 1000
+        b.add_generic("op", 0, t, t + 5, 1, 5, id=1, schema=op, values=[1, 2, 3, n])
+        b.add_generic("op", 0, t + 10, t + 15, 1, 5, id=2, schema=op, values=[1, 2, 3, -(n // 10)])
+        b.add_generic("op", 0, t + 20, t + 25, 1, 5, id=3, schema=string, values=[1, 2, 3, n, b.s("text")])
+        b.add_device(4, t + 70, t + 75, name="k", queue=n)
+        b.add_device(6, t + 80, t + 85, domain=1, op=2, queue=n)
+        b.add_memset(8, t + 90, t + 95, context=n & 0xFFFFFFFF, nbytes=5)
+        return b.build()
+    for digits in range(1, 12):   # (beside a string there is room for seven)
+        assert _woven_vs_oracle(sim, stream(10**digits - 1)) == ((6, 0) if digits < 8 else (5, 1)), digits
+    assert _woven_vs_oracle(sim, stream(10**11)) == (1, 5)   # (a minus is a character)
 
 
 def test_doubles_as_text(sim):
