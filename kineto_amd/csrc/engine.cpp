@@ -11,6 +11,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cerrno>
+#include <chrono>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -1670,10 +1671,13 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
       HIPCHK(gather_offsets(e->perm, e->len.as<uint32_t>(), N, e->len_sorted.as<uint32_t>(), e->kind_sorted.as<uint8_t>(),
                             e->scan_tmp.as<uint64_t>(), e->offs.as<uint64_t>(), left(), sc, text, st));
       /* Mostly there are no others, and a launch that finds its list empty takes 4 us, 20 with 22 million rows.  What k_decode
-       * has counted is here by now, unless the trace is so large that such a launch does not matter; others that it cannot
-       * know of are printed behind a wait of their own the first time.  (No look at the count: 30 000 records of which some are left
+       * has counted is here by now or soon: in the first pass of an engine that is waited for, with ten launches and more behind
+       * it in the stream.  Others that it cannot know of are printed behind a wait of their own the first time.  (No look at the count: 30 000 records of which some are left
        * 217 instead of 200 us; the launch in every first pass: 180 instead of 176 us with none left.) */
-      const uint32_t counted = woven ? __atomic_load_n(&e->h_ctl->weave, __ATOMIC_ACQUIRE) : (uint32_t)KTJ_WEAVE_UNKNOWN;
+      auto look = [&]() -> uint32_t { return woven ? __atomic_load_n(&e->h_ctl->weave, __ATOMIC_ACQUIRE) : (uint32_t)KTJ_WEAVE_UNKNOWN; };
+      uint32_t counted = look();
+      if (woven && e->some_left < 0)
+        for (const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(1); counted == KTJ_WEAVE_UNKNOWN && std::chrono::steady_clock::now() < until;) counted = look();
       const bool others = counted >= KTJ_WEAVE_MOST || (counted == KTJ_WEAVE_ALL ? e->some_left > 0 : e->some_left != 0);
       { const int rc = put_activities(N, others ? N : 0u, prefix.size(), counted != KTJ_WEAVE_NONE); if (rc != KTJ_OK) return rc; }
       HIPCHK(hipEventRecord(e->ev[EV_EMIT], st));
