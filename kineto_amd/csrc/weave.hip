@@ -8,14 +8,15 @@
  * text from LDS, a number of the row's), a prefix sum of their lengths gives their places, and they are OR-ed into a
  * zero-filled piece of the document in LDS, whose whole lines leave with lane-consecutive stores.  Numbers were made
  * into text in the size pass, which needs their lengths anyway; the texts with process and thread are made once per
- * track.  3220 vector and 770 LDS instructions for 64 kernel events, 99 registers, four wavefronts per SIMD.
+ * track.  3730 vector and 740 LDS instructions for 64 activities (22 million records: kernels, runtime calls and operators),
+ * four wavefronts per SIMD.
  *
  * What bounds it: memory (22 million records 13.6 GB in 3.44 ms, 0.89 of what a plain copy reaches; 11 million kernels 0.95),
  * with the vector units busy for 2.1 and the LDS pipes for 1.9 of the 3.44 ms, a third of that bank conflicts.
  * Measured against k_emit_direct: 10 000 x 3 records 38.7 -> 15.5 us, 4000 operators with long strings
  * 71 -> 24 us, 733 000 records 176 -> 136 us, 3 million 795 -> 451 us, 11 million kernels 2.06 -> 1.70 ms, 22 million
  * records 4.59 -> 3.44 ms, 5 million operators with long strings (1.4 KB each: strings beyond 128 bytes are fetched from
- * memory piece by piece) 3.20 -> 2.67 ms; the size pass has become 4 to 13 % longer for the numbers' text.
+ * memory piece by piece) 3.20 -> 2.67 ms; the size pass has become up to 18 % longer for the numbers' text.
  * (Long strings' whole lines from the dictionary to the document past the tile, the loads of four strings at a time in
  * front of any store: 2.70 ms, and 26 instead of 24 us for 4000 of them.)
  * Fewer wavefronts cost: three per SIMD 2.48 ms for the kernels, two 2.83.  Five (96 registers, 2048 bytes of tile, 512
@@ -453,7 +454,8 @@ k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const u
             x.a = src[0];
             if (len > 16u) { b = src[1]; if (len > 32u) { c = src[2]; if (len > 48u) d = src[3]; } }
           }
-          /* waited for here, so that no wait of the loop is for the document's stores */
+          /* waited for here, once for the four of them and only where there are any: this wait is also for the lines that
+           * store_lines has just stored, as loads and stores are counted together and in order */
           asm volatile("" : "+v"(x.a), "+v"(b), "+v"(c), "+v"(d));
         }
         const uint32_t n_num = x.num.w >> 24;
