@@ -102,8 +102,8 @@ enum : uint32_t {
   R_MEMSET_NAME = 37,                            /* + memory kind, 8 = any other */
   R_BODY_NONE = 46, R_BODY_ARGS, R_BODY_EXT,
   R_ARGS,                                        /* + A_* */
-  R_ARGS2 = R_ARGS + 28,                         /* the same, behind the string */
-  R_TAIL = R_ARGS2 + 28,                         /* + 5 where an args object closes, + 10 where an array does before it;
+  R_ARGS2 = R_ARGS + 32,                         /* the same, behind the string */
+  R_TAIL = R_ARGS2 + 32,                         /* + 5 where an args object closes, + 10 where an array does before it;
                                                     + flow: none, start, end, the same of fwdbwd */
   R_PIECES = R_TAIL + 15,
   R_COUNT
@@ -112,8 +112,12 @@ enum : uint32_t {
   A_DEFAULT = 0, A_LAUNCH, A_LAUNCH_NAMED, A_COPY, A_MALLOC, A_MALLOC_BYTES,
   A_KERNEL, A_KERNEL_SIZE, A_KERNEL_GRID, A_MEMSET, A_MEMSET_BANDWIDTH,
   A_COPIED,                                      /* + 3 * direction, + 1 with bytes, + 2 with a grid */
-  A_COUNT = A_COPIED + 15
+  /* Bytes without a bandwidth, as copies of no duration have: + 0 a kernel's, + 1 + direction a copy's.  (Left to k_emit_direct, 50 of
+   * them among 3 million records cost a launch of 33 us: a pass of 1251 us, 1217 now.) */
+  A_BYTES_ONLY = A_COPIED + 15,
+  A_COUNT = A_BYTES_ONLY + 6
 };
+static_assert(A_COUNT <= R_ARGS2 - R_ARGS && A_COUNT <= KTJ_TR_SCHEMA, "the args' parts");
 /* a part: first descriptor, their number */
 #define KTJ_WREF(base, count) ((base) | ((count) << 16))
 #define KTJ_WREF_BASE(r) ((r) & 0xFFFFu)
@@ -244,6 +248,10 @@ constexpr Book make_book() {
     b.part(R_ARGS + A_COPIED + 3 * d, KTJ_WEAVE_DEVICE, direction[d], "\"");
     b.part(R_ARGS + A_COPIED + 3 * d + 1, KTJ_WEAVE_DEVICE, direction[d], "\"" KTJ_WEAVE_SIZE);
     b.part(R_ARGS + A_COPIED + 3 * d + 2, KTJ_WEAVE_DEVICE, direction[d], "\"" KTJ_WEAVE_GRID);
+  }
+  for (uint32_t k = 0; k < 6; ++k) { /* as with a bandwidth, but for the text in front of it, which is the last segment */
+    const uint32_t with = b.b.ref[R_ARGS + (k ? A_COPIED + 3 * (k - 1) + 1 : (uint32_t)A_KERNEL_SIZE)];
+    b.b.ref[R_ARGS + A_BYTES_ONLY + k] = KTJ_WREF(KTJ_WREF_BASE(with), KTJ_WREF_COUNT(with) - 1);
   }
   const char* const close[3] = {"", "\n    }\n  },", "]\n    }\n  },"};
   const char* const flow[5] = {
@@ -816,8 +824,11 @@ KTJ_HD KTJ_FI inline bool text_row(const MatRow& m, const EmitCtx& c, const Sche
         bandwidth = m.dur != 0;
         args = bandwidth ? A_MEMSET_BANDWIDTH : A_MEMSET;
       } else {
-        if (size && m.dur == -1) return false; /* bytes without a bandwidth */
-        args = (kind == KTJ_DOM_MEMORY_COPY ? A_COPIED + 3u * (m.aux <= KTJ_COPY_D2D ? m.aux : 0u) : (uint32_t)A_KERNEL) + (size ? 1u : triple ? 2u : 0u);
+        const bool copied = kind == KTJ_DOM_MEMORY_COPY;
+        const uint32_t direction = m.aux <= KTJ_COPY_D2D ? m.aux : 0u;
+        bandwidth = size && m.dur != -1;
+        if (size && !bandwidth) args = A_BYTES_ONLY + (copied ? 1u + direction : 0u);
+        else args = (copied ? A_COPIED + 3u * direction : (uint32_t)A_KERNEL) + (size ? 1u : triple ? 2u : 0u);
         if (triple) close = 10u;
       }
       if (size) n += put(S_X, text_of(m.p[0]));

@@ -262,6 +262,23 @@ def test_long_jobs(sim):
     assert _woven_vs_oracle(sim, stream(10**11)) == (1, 5)   # (a minus is a character)
 
 
+def test_bytes_without_a_bandwidth(sim):
+    """A copy of no duration has bytes and no bandwidth, and so has a kernel with a copy's id: text rows as any."""
+    b = StreamBuilder(window=(B, B + 10**13), host_name="copies")
+    b.api(["hipLaunchKernel", "hipMemcpyAsync"], flow_start=[0, 1])
+    for k in range(14):   # directions 0 to 6, the last two unknown ones
+        t = B + 10000 * (k + 1)
+        b.add_runtime(k + 1, t, t + 10, 1, 1, 5, kind=2, src=1, dst=2, size=(0, 7, 10**10)[k % 3], copy_kind=1, stream=k % 2)
+        b.add_device(k + 1, t + 50, t + 50 + k // 7, domain=1, op=k % 7, queue=k)
+    for k in range(20, 23):
+        b.add_runtime(k, B + k, B + k + 5, 1, 1, 5, kind=2, size=4096, copy_kind=1)
+        b.add_device(k, B + k + 50, B + k + 50 + k % 2, name="kernel with bytes", queue=1)
+    assert _woven_vs_oracle(sim, b.build()) == (34, 0)
+    sp, release = abi.synth_stream(2, 60000, host_name="box")
+    assert _woven_vs_oracle(sim, sp)[1] == 0
+    release()
+
+
 def test_doubles_as_text(sim):
     """Shifted together, against the formatter's characters one by one: zeros behind the text, too."""
     import random
