@@ -2309,7 +2309,6 @@ __device__ __forceinline__ bool bitmap_test_and_set(uint32_t* bitmap, uint32_t s
   return active && (twice || (old & bit) != 0);
 }
 #define JOIN_ROWS 4
-#define JOIN_SMALL_ROWS (1u << 18)
 #ifndef KX_JOIN_ATTR
 #define KX_JOIN_ATTR
 #endif
@@ -2622,8 +2621,11 @@ hipError_t join_runtime_rows(const ktj_runtime_rec* r, uint64_t n, Columns c, ui
                              Table tn, NarrowCols nc, uint32_t* slot_f, uint32_t* slot_n, EmitCtx ctx, Rows rows,
                              uint32_t* len, Scalars* sc, hipStream_t st) {
   if (n == 0) return hipSuccess;
-  /* few rows: one group per workgroup, so that the launch is as wide and as short as it can be */
-  const int rounds = n < JOIN_SMALL_ROWS ? 1 : JOIN_ROWS;
+  /* As many groups per workgroup as let all workgroups run at a time (four per CU, by their registers and LDS), up to JOIN_ROWS:
+   * with fewer the last ones run alone, with more CUs stand idle (333 000 rows, 1 / 2 / 4 groups: 56 / 50 / 66 us; a million
+   * 97 / 99 / 102; 10 million 1173 / 1160 / 1181). */
+  const uint64_t groups = grid_for(n, KTJ_BLOCK), at_once = 1024u;
+  const int rounds = groups <= at_once ? 1 : groups >= at_once * JOIN_ROWS ? JOIN_ROWS : (int)((groups + at_once - 1u) / at_once);
   auto launch = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3(grid_for(n, KTJ_BLOCK * rounds)), dim3(KTJ_BLOCK), 0, st, r, n, c, first, api, tf, fc, tn, nc,
                        slot_f, slot_n, ctx, rows, len, sc, rounds);
