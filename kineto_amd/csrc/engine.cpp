@@ -272,10 +272,17 @@ struct ktj_engine {
 
   bool small_unfit = false;  /* these records need the launches of a large trace (Scalars::error of a small pass) */
   bool stepwise = false;     /* these records need a pass in which the host looks at the plan of the sort (KTJ_DEVERR_CAREFUL) */
-  /* six passes sort the records of one capture: 2^38 ns, four and a half minutes, beside 9 bits of devices and
-   * rows; a pass more than needed costs its three launches, a pass too few the launches behind the sort */
-  uint32_t sort_passes = 6;  /* to be launched: what these records took in the pass before, where there was one */
-  void other_records() { small_unfit = stepwise = no_room_for_text = false; not_woven = 0; sort_passes = std::max(sort_passes, 6u); }
+  bool sort_all_bits = false; /* by passes: their order of arrival is not that of their times where many are close together */
+  uint32_t sort_passes = 0;  /* what these records took in the pass before, where there was one */
+  uint32_t sort_passes_most = 0; /* of others before them */
+  void other_records() {
+    small_unfit = stepwise = no_room_for_text = sort_all_bits = false; not_woven = 0;
+    sort_passes_most = std::max(sort_passes_most, sort_passes); sort_passes = 0;
+  }
+  /* Six passes sort the records of one capture: 2^38 ns, four and a half minutes, beside 9 bits of devices and rows; four
+   * do where the lowest sixteen of these 48 bits need none, as the word has room for them beside the index and the rows lie far enough apart.  A
+   * pass more than needed costs its three launches, a pass too few the launches behind the sort. */
+  uint32_t passes_to_launch(uint64_t n) const { return sort_passes ? sort_passes : std::max(sort_passes_most, n <= 65536u ? 4u : 6u); }
   bool small_last = false;   /* the last pass was a small one: it leaves no intermediate arrays for ktj_debug_fetch */
   bool no_small = false;     /* ktj_debug_fetch makes them */
   bool no_weave = false;     /* joined rows as they are: ktj_debug_fetch */
@@ -1638,7 +1645,7 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
   }
   /* (settled here: collect_distinct flags what only a host that does not look would get wrong) */
   const bool straight = has_room && n_coll == 0 && max_spans == 0 && !e->stepwise && !(e->flags & KTJ_CREATE_TILE_EMIT) && e->sort_mode != 1;
-  HIPCHK(collect_distinct(c, N, sets, sc, straight, ctx, book, st));
+  HIPCHK(collect_distinct(c, N, nd, sets, sc, straight, ctx, book, st));
   /* The document's activities, but for the tile variant: what the weaver prints, and at most n_left others. */
   auto put_activities = [&](uint64_t n_most, uint64_t n_left, uint64_t at, bool weave = true) -> int {
     if (woven && n_most && weave)
@@ -1664,7 +1671,7 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
     if (out_device) e->out.borrow(out_device, out_cap);
     e->perm = e->vals_a.as<uint32_t>();
     e->sorted_keys = nullptr;
-    HIPCHK(sort_packed(c, N, sets, sc, e->sort_passes, e->keys_a.as<uint64_t>(), e->keys_b.as<uint64_t>(), e->perm, e->hist.as<uint32_t>(), e->offs.as<uint32_t>(), st));
+    HIPCHK(sort_packed(c, N, sets, sc, e->passes_to_launch(N), !e->sort_all_bits, e->keys_a.as<uint64_t>(), e->keys_b.as<uint64_t>(), e->perm, e->hist.as<uint32_t>(), e->offs.as<uint32_t>(), st));
     HIPCHK(mat_rows(g_recs, ng, 0, nullptr, d_recs, nd, c, ng + nr, e->dev_link.as<DevLink>(), ctx, rows, e->len.as<uint32_t>(), sc, st));
     for (;;) {
       text.out = e->out.as<char>(); text.out_cap = e->out.cap;
@@ -1703,13 +1710,14 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
       HIPCHK(e->out.ensure(e->total_bytes + 64));
       HIPCHK(fill_u32(&sc->n_left, 0, 1, st)); /* the list is made anew */
     }
-    if (emitted) e->sort_passes = sort_packed_passes(e->scalars.sort.key_bits);
-    else if (e->scalars.error & ~(KTJ_DEVERR_CAREFUL | KTJ_DEVERR_DISTINCT_DEVICES | KTJ_DEVERR_DISTINCT_RESOURCES)) {
+    if (emitted) e->sort_passes = sort_packed_passes(e->scalars.sort, !e->sort_all_bits);
+    else if (e->scalars.error & ~(KTJ_DEVERR_CAREFUL | KTJ_DEVERR_UNSORTED | KTJ_DEVERR_DISTINCT_DEVICES | KTJ_DEVERR_DISTINCT_RESOURCES)) {
       e->last_error = limit_text(e->scalars.error);
       return KTJ_ERR_LIMIT;
     } else {
-      e->stepwise = true;
-      HIPCHK(clear_error_bits(sc, KTJ_DEVERR_CAREFUL, st));
+      if (e->scalars.error == KTJ_DEVERR_UNSORTED) { e->sort_all_bits = true; e->sort_passes = sort_packed_passes(e->scalars.sort, false); }
+      else e->stepwise = true;
+      HIPCHK(clear_error_bits(sc, KTJ_DEVERR_CAREFUL | KTJ_DEVERR_UNSORTED, st));
     }
   }
   if (!emitted) { /* the stepwise rest */
@@ -1751,8 +1759,8 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
       if (rc == KTJ_OK) rc = sort_again([&](const uint32_t* o, uint64_t* k, uint32_t* v) { return make_column_keys(c.dev, c.meta, o, N, 0, k, v, st); }, 64);
       if (rc == KTJ_OK) rc = sort_again([&](const uint32_t* o, uint64_t* k, uint32_t* v) { return make_column_keys(c.dev, c.meta, o, N, 1, k, v, st); }, 1);
       if (rc != KTJ_OK) return rc;
-    } else if (key_bits <= 62 && e->sort_mode != 1 && sort_packed_fits(N, key_bits)) {
-      HIPCHK(sort_packed(c, N, sets, sc, sort_packed_passes(key_bits), ka, kb, va, hist, e->offs.as<uint32_t>(), st));
+    } else if (e->sort_mode != 1 && sort_packed_fits(N, e->scalars.sort)) {
+      HIPCHK(sort_packed(c, N, sets, sc, sort_packed_passes(e->scalars.sort, false), false, ka, kb, va, hist, e->offs.as<uint32_t>(), st));
       e->perm = va;
       e->sorted_keys = nullptr;
     } else if (key_bits <= 62) {

@@ -117,7 +117,10 @@ struct Columns {
 #define KTJ_COUNTER_SHARDS 64u
 #endif
 #define KTJ_PART_SLOTS 32u
-struct SortPlan { unsigned int ts_bits, res_bits, key_bits; }; /* of the composite key, without the bit for dropped rows */
+struct SortPlan { /* of the composite key */
+  unsigned int ts_bits, res_bits, key_bits, low_bits; /* .., of all of it, of what the passes may leave to sort_finish */
+  unsigned int n_dev;                                 /* dropped rows have this device's rank */
+};
 /* wall clock (wall_clock64) at the points of a pass: its start and the start of each stage; the runs of
  * small.hip name their own */
 enum { KTJ_CLOCK_BEGIN = 0, KTJ_CLOCK_DECODE, KTJ_CLOCK_JOIN, KTJ_CLOCK_SORT, KTJ_CLOCK_SIZE, KTJ_CLOCK_SCAN, KTJ_CLOCK_EMIT, KTJ_CLOCK_COUNT };
@@ -176,6 +179,7 @@ enum { KTJ_CNT_OUT_OF_RANGE = 0, KTJ_CNT_OUT_OF_ORDER, KTJ_CNT_FLOW, KTJ_CNT_LIN
 #define KTJ_DEVERR_QUEUES 64u             /* more than KTJ_MAX_QUEUES hardware queues */
 #define KTJ_DEVERR_SYNC_ROWS 128u         /* more than KTJ_MAX_SYNC_ROWS (device, row) pairs of Stream Sync events */
 
+#define KTJ_DEVERR_UNSORTED 1024u         /* the sort's passes have to take all bits; no error reaches the caller */
 #define KTJ_DEVERR_CAREFUL 512u           /* the pass went by assumptions that do not hold; no error reaches the caller */
 #define KTJ_DEVERR_SMALL_UNFIT 256u       /* a small trace that needs the launches of a large one; no error reaches the caller */
 
@@ -334,7 +338,7 @@ struct SortSets {
 /* distinct values and their ranks, and Scalars::sort; straight: the host will not look at anything before
  * the end of the pass, so what needs that is flagged (KTJ_DEVERR_CAREFUL).  book, if not null: what text_row and
  * weave_activities need to know of the schemas, from the dictionary views */
-hipError_t collect_distinct(Columns c, uint64_t n, SortSets s, Scalars* sc, bool straight, const EmitCtx& ctx, weave::SchemaBook* book, hipStream_t st);
+hipError_t collect_distinct(Columns c, uint64_t n, uint64_t n_device, SortSets s, Scalars* sc, bool straight, const EmitCtx& ctx, weave::SchemaBook* book, hipStream_t st);
 /* key = ((rank(dev) << res_bits | rank(res)) << ts_bits) | (ts - ts_min); dropped rows get 1 << key_bits */
 hipError_t make_keys(Columns c, uint64_t n, SortSets s, const Scalars* sc, uint32_t ts_bits, uint32_t res_bits,
                      uint32_t key_bits, uint64_t* keys, uint32_t* vals, hipStream_t st);
@@ -347,14 +351,14 @@ hipError_t make_column_keys(const int64_t* column, const uint32_t* meta, const u
                             uint64_t* keys, uint32_t* vals, hipStream_t st);
 hipError_t clear_error_bits(Scalars* sc, unsigned int bits, hipStream_t st);
 /* The composite-key sort on single 64-bit words (key above the arrival index); perm receives the
- * arrival index per sorted position.  Usable when sort_packed_fits(n, key_bits). */
-bool sort_packed_fits(uint64_t n, uint32_t key_bits);
+ * arrival index per sorted position.  Usable when sort_packed_fits(n, plan). */
+bool sort_packed_fits(uint64_t n, const SortPlan& plan);
 bool sort_packed_passes_forced();
 void sort_packed_force_passes(bool on); /* tests: no one-launch sort of a single tile */
-uint32_t sort_packed_passes(uint32_t key_bits);
+uint32_t sort_packed_passes(const SortPlan& plan, bool finish); /* finish: the lowest bits are left to a launch behind the passes */
 /* key widths come from Scalars::sort; `passes` is how many are launched: those beyond the plan end at once, and
  * a plan that needs more (or does not fit a word) sets KTJ_DEVERR_CAREFUL in Scalars::error */
-hipError_t sort_packed(Columns c, uint64_t n, SortSets s, Scalars* sc, uint32_t passes, uint64_t* buf_a, uint64_t* buf_b, uint32_t* perm,
+hipError_t sort_packed(Columns c, uint64_t n, SortSets s, Scalars* sc, uint32_t passes, bool finish, uint64_t* buf_a, uint64_t* buf_b, uint32_t* perm,
                        uint32_t* hist, uint32_t* chain_hist /* 8 bytes per row */, hipStream_t st);
 hipError_t make_rank_keys(Columns c, const uint32_t* order, uint64_t n, SortSets s, uint32_t res_bits, uint32_t rank_bits,
                           uint64_t* keys, uint32_t* vals, hipStream_t st);

@@ -207,7 +207,7 @@ k_begin(Scalars* s, FillJobs jobs, const char* blob, const uint64_t* off, uint32
       s->out_of_range = 0; s->out_of_order = 0; s->n_flow = 0; s->n_linked = 0; s->n_blank_names = 0; s->n_valid = 0;
       s->n_unresolved = 0; s->n_sync_typed = 0; s->n_device_orphans = 0; s->error = 0; s->have_stream_src = 0; s->n_dev_ranks = 0; s->n_res_ranks = 0; s->n_dense = 0; s->runtime_ids_repeat = 0;
       s->n_queues = 0; s->n_sync_rows = 0; s->ext_ids_repeat = 0; s->n_plain = 0; s->n_left = 0; s->no_text = 0;
-      s->sort.ts_bits = s->sort.res_bits = s->sort.key_bits = 0;
+      s->sort.ts_bits = s->sort.res_bits = s->sort.key_bits = s->sort.low_bits = s->sort.n_dev = 0;
       for (int k = 0; k < KTJ_DONE_COUNT; ++k) s->done[k] = 0;
       for (uint32_t k = 0; k < KTJ_PART_SLOTS; ++k) s->part_done[k] = 0;
       for (int k = 0; k < KTJ_CLOCK_COUNT; ++k) s->clock[k] = 0;
@@ -1092,6 +1092,7 @@ __device__ __forceinline__ bool local_set_first(unsigned long long* lds /* LOCAL
   return true;
 }
 #define COLLECT_ROWS 4
+#define SORTP_BITS 8 /* of a digit of the one-word sort */
 __device__ __forceinline__ void set_enter(uint64_t* keys, uint32_t* list, unsigned int* count, uint64_t v, Scalars* sc, unsigned too_many) {
   bool fresh;
   const uint32_t g = table_insert_fresh(keys, KTJ_SET_CAP - 1u, v, &fresh);
@@ -1194,7 +1195,7 @@ __device__ void lay_out_schemas(const EmitCtx& c, weave::SchemaBook* out, Schema
  * printed.  The workgroup that ends last ranks the values and plans the sort's keys.  With a book the first
  * workgroup lays out the schemas instead of taking rows: this is the longest launch before the size pass that
  * small passes have, too. */
-__global__ void __launch_bounds__(KTJ_BLOCK) k_collect_distinct(Columns c, uint64_t n, SortSets s, Scalars* sc, int straight, EmitCtx ctx, weave::SchemaBook* book) {
+__global__ void __launch_bounds__(KTJ_BLOCK) k_collect_distinct(Columns c, uint64_t n, uint64_t n_device, SortSets s, Scalars* sc, int straight, EmitCtx ctx, weave::SchemaBook* book) {
   __shared__ uint64_t red_min[KTJ_BLOCK >> 6], red_max[KTJ_BLOCK >> 6];
   __shared__ unsigned long long seen[2][LOCAL_SET_SLOTS + 1]; /* deviceId, resourceId values */
   static_assert(sizeof(SchemaLds) <= sizeof(seen), "laid out where the values would be");
@@ -1281,6 +1282,8 @@ __global__ void __launch_bounds__(KTJ_BLOCK) k_collect_distinct(Columns c, uint6
     hi = ox > hi ? ox : hi;
   }
   const uint64_t sync_typed = __ballot(sc->shard[threadIdx.x][KTJ_CNT_SYNC_TYPED] != 0); /* the order decides which of them announces its row */
+  unsigned long long valid = agent_load(&sc->shard[threadIdx.x][KTJ_CNT_VALID]);
+  for (int o = 32; o > 0; o >>= 1) valid += __shfl_xor(valid, o);
   if (threadIdx.x == 0) {
     sc->ts_min_biased = lo;
     sc->ts_max_biased = hi;
@@ -1289,7 +1292,19 @@ __global__ void __launch_bounds__(KTJ_BLOCK) k_collect_distinct(Columns c, uint6
     SortPlan p;
     p.ts_bits = bits(span);
     p.res_bits = bits(mr ? mr - 1u : 0u);
-    p.key_bits = p.ts_bits + p.res_bits + bits(md ? md - 1u : 0u);
+    p.n_dev = md;
+    p.key_bits = p.ts_bits + p.res_bits + bits(valid < n ? md : md ? md - 1u : 0u); /* rows that are dropped: a device behind the others */
+    /* The lowest bits that need no pass (k_sortp_finish): in 2^low ns, 65 us at most, a track has sixteen rows or fewer, were they
+     * spread evenly over the trace and over the streams and threads; and no more bits than the passes that remain leave over.  (15
+     * bits instead of 7 for 22 million, groups of 67 rows: a pass less, 135 us, but 220 us more behind the passes.) */
+    const uint32_t pairs = sc->n_dense, threads = mr > pairs ? mr - pairs : 1u;
+    const float of_thread = (float)(n - n_device) / (float)threads;
+    const float of_stream = (float)n_device / (pairs ? (float)pairs : 0.5f * (float)threads); /* (no pairs: the streams are among the others) */
+    const float rows = of_stream > of_thread ? of_stream : of_thread, times = p.ts_bits < 60u ? 16.0f * (float)(1ull << p.ts_bits) : 1e30f;
+    uint32_t low = 0;
+    while (low < 16u && rows * (float)(2u << low) <= times) ++low;
+    const uint32_t passes = (p.key_bits > low ? p.key_bits - low + SORTP_BITS - 1u : SORTP_BITS) / SORTP_BITS;
+    p.low_bits = p.key_bits > passes * SORTP_BITS && p.key_bits + bits(n - 1u) <= 64u ? p.key_bits - passes * SORTP_BITS : 0u;
     sc->sort = p;
     if (straight && sync_typed) flag_error(sc, KTJ_DEVERR_CAREFUL);
   }
@@ -1400,7 +1415,7 @@ hipError_t make_rank_keys(Columns c, const uint32_t* order, uint64_t n, SortSets
   return KTJ_LAUNCH_CHECK();
 }
 
-hipError_t collect_distinct(Columns c, uint64_t n, SortSets s, Scalars* sc, bool straight, const EmitCtx& ctx, weave::SchemaBook* book, hipStream_t st) {
+hipError_t collect_distinct(Columns c, uint64_t n, uint64_t n_device, SortSets s, Scalars* sc, bool straight, const EmitCtx& ctx, weave::SchemaBook* book, hipStream_t st) {
   if (n == 0) return hipSuccess;
   /* few, fat workgroups: each one pays for its own local set once (few rows: one group each) */
   /* at most four workgroups per CU: every workgroup pays for its local sets and its atomics at the
@@ -1408,7 +1423,7 @@ hipError_t collect_distinct(Columns c, uint64_t n, SortSets s, Scalars* sc, bool
    * 1024: 0.17 ms) */
   unsigned g = grid_stride_for(n, n < (1u << 20) ? KTJ_BLOCK * COLLECT_ROWS : KTJ_BLOCK * 16);
   if (g > 1024u) g = 1024u;
-  hipLaunchKernelGGL(k_collect_distinct, dim3(g + (book ? 1u : 0u)), dim3(KTJ_BLOCK), 0, st, c, n, s, sc, straight ? 1 : 0, ctx, book);
+  hipLaunchKernelGGL(k_collect_distinct, dim3(g + (book ? 1u : 0u)), dim3(KTJ_BLOCK), 0, st, c, n, n_device, s, sc, straight ? 1 : 0, ctx, book);
   return KTJ_LAUNCH_CHECK();
 }
 hipError_t make_keys(Columns c, uint64_t n, SortSets s, const Scalars* sc, uint32_t ts_bits, uint32_t res_bits,
@@ -1561,13 +1576,26 @@ hipError_t radix_sort(uint64_t* keys_a, uint32_t* vals_a, uint64_t* keys_b, uint
 /* How many passes there are is the plan that k_collect_distinct leaves on the device: the host launches as
  * many as it expects, those beyond the plan end at once, and a plan beyond them (or one that does not fit
  * a word) is flagged for the host to take the pass again, looking at the plan (KTJ_DEVERR_CAREFUL). */
-#define SORTP_BITS 8
-__device__ __forceinline__ uint32_t sort_passes(const Scalars* sc) { return (sc->sort.key_bits + SORTP_BITS) / SORTP_BITS; } /* key and dropped bit */
-__device__ __forceinline__ bool sort_pass_idle(const Scalars* sc, uint32_t pass) { return sc->error != 0 || pass >= sort_passes(sc); }
-__device__ __forceinline__ bool sort_words_suffice(const Scalars* sc, uint32_t key_bits, uint32_t idx_bits, uint32_t passes_launched) {
-  return sc->error == 0 && key_bits <= 62u && (key_bits + 1u > SORTP_BITS ? key_bits + 1u - SORTP_BITS : 0u) + idx_bits <= 64u &&
-         (key_bits + SORTP_BITS) / SORTP_BITS <= passes_launched;
+/* Where the word has room for the whole key (low != 0) the passes leave the lowest bits out, and k_sortp_finish puts the rows
+ * that differ in these only into their order; otherwise the first pass's digit leaves the word. */
+struct SortRun { uint32_t low, passes; };
+__device__ __forceinline__ SortRun sort_run(const Scalars* sc, int finish) {
+  SortRun r;
+  r.low = finish ? sc->sort.low_bits : 0u;
+  const uint32_t bits = sc->sort.key_bits - r.low;
+  r.passes = bits ? (bits + SORTP_BITS - 1u) / SORTP_BITS : 1u;
+  return r;
 }
+__device__ __forceinline__ bool sort_pass_idle(const Scalars* sc, const SortRun& r, uint32_t pass) { return sc->error != 0 || pass >= r.passes; }
+__device__ __forceinline__ uint32_t sort_shift(const SortRun& r, uint32_t pass, uint32_t idx_bits) { return idx_bits + r.low + (r.low ? pass : pass - 1u) * SORTP_BITS; }
+__device__ __forceinline__ bool sort_words_suffice(const Scalars* sc, const SortRun& r, uint32_t key_bits, uint32_t idx_bits, uint32_t passes_launched) {
+  return sc->error == 0 && key_bits <= 62u && (r.low ? key_bits : key_bits > SORTP_BITS ? key_bits - SORTP_BITS : 0u) + idx_bits <= 64u &&
+         r.passes <= passes_launched;
+}
+__device__ __forceinline__ uint64_t sort_key(const SortPlan& p, uint64_t rank_dev, uint64_t rank_res, uint64_t rel) {
+  return (((rank_dev << p.res_bits) | rank_res) << p.ts_bits) | rel;
+}
+__device__ __forceinline__ uint64_t sort_key_dropped(const SortPlan& p) { return (uint64_t)p.n_dev << (p.res_bits + p.ts_bits); } /* behind everything */
 template <int BITS, int THREADS, int ITEMS_> struct SortP {
   static constexpr int NB = 1 << BITS;
   static constexpr int WAVES = THREADS / 64;
@@ -1581,11 +1609,12 @@ template <int BITS, int THREADS, int ITEMS_> struct SortP {
  * the first pass's, start from zero. */
 template <int BITS, int THREADS, int ITEMS, bool CHAIN>
 __global__ void __launch_bounds__(THREADS)
-k_sortp_make_keys(Columns c, uint64_t n, SortSets s, Scalars* sc, uint32_t idx_bits, uint32_t passes_launched, uint64_t* keys, uint32_t* hist,
+k_sortp_make_keys(Columns c, uint64_t n, SortSets s, Scalars* sc, uint32_t idx_bits, uint32_t passes_launched, int finish, uint64_t* keys, uint32_t* hist,
                   uint32_t n_blocks) {
   using P = SortP<BITS, THREADS, ITEMS>;
-  const uint32_t ts_bits = sc->sort.ts_bits, res_bits = sc->sort.res_bits, key_bits = sc->sort.key_bits;
-  if (!sort_words_suffice(sc, key_bits, idx_bits, passes_launched)) {
+  const SortPlan plan = sc->sort;
+  const SortRun run = sort_run(sc, finish);
+  if (!sort_words_suffice(sc, run, plan.key_bits, idx_bits, passes_launched)) {
     if (blockIdx.x == 0 && threadIdx.x == 0) flag_error(sc, KTJ_DEVERR_CAREFUL);
     return;
   }
@@ -1612,31 +1641,30 @@ k_sortp_make_keys(Columns c, uint64_t n, SortSets s, Scalars* sc, uint32_t idx_b
     for (int g = 0; g < G; ++g) {
       const uint64_t a = base + (uint64_t)(r0 + g) * THREADS + threadIdx.x;
       if (a >= n) continue;
-      uint64_t key = 1ULL << key_bits; /* dropped rows sort behind everything */
+      uint64_t key = sort_key_dropped(plan);
       if (meta[g] & KTJ_M_VALID) {
         const uint64_t rd = set_rank_memo(s.dev_keys, s.dev_rank, dev[g], memo_dev);
         const uint64_t rr = set_rank_memo(s.res_keys, s.res_rank, res[g], memo_res);
-        const uint64_t rel = (ts[g] ^ 0x8000000000000000ULL) - ts_min;
-        key = ((((rd << res_bits) | rr)) << ts_bits) | rel;
+        key = sort_key(plan, rd, rr, (ts[g] ^ 0x8000000000000000ULL) - ts_min);
       }
       keys[a] = key;
-      atomicAdd(&h[(uint32_t)key & (P::NB - 1u)], 1u);
+      atomicAdd(&h[(uint32_t)(key >> run.low) & (P::NB - 1u)], 1u);
     }
   }
   __syncthreads();
   if (CHAIN) {
-    const uint32_t passes = sort_passes(sc);
-    for (uint32_t k = threadIdx.x; k < passes * P::NB; k += THREADS)
+    for (uint32_t k = threadIdx.x; k < run.passes * P::NB; k += THREADS)
       hist[((uint64_t)(k / P::NB) * n_blocks + blockIdx.x) * P::NB + k % P::NB] = k < P::NB ? h[k] : 0u;
   } else if (hist != nullptr)
     for (int d = threadIdx.x; d < P::NB; d += THREADS) hist[(uint64_t)d * n_blocks + blockIdx.x] = h[d]; /* digit-major */
 }
 template <int BITS, int THREADS, int ITEMS>
 __global__ void __launch_bounds__(THREADS)
-k_sortp_hist(const uint64_t* words, uint64_t n, uint32_t pass, uint32_t idx_bits, const Scalars* sc, uint32_t* hist, uint32_t n_blocks) {
+k_sortp_hist(const uint64_t* words, uint64_t n, uint32_t pass, uint32_t idx_bits, int finish, const Scalars* sc, uint32_t* hist, uint32_t n_blocks) {
   using P = SortP<BITS, THREADS, ITEMS>;
-  if (sort_pass_idle(sc, pass)) return;
-  const uint32_t shift = idx_bits + (pass - 1u) * BITS;
+  const SortRun run = sort_run(sc, finish);
+  if (sort_pass_idle(sc, run, pass)) return;
+  const uint32_t shift = sort_shift(run, pass, idx_bits);
   __shared__ uint32_t h[P::NB];
   for (int d = threadIdx.x; d < P::NB; d += THREADS) h[d] = 0;
   __syncthreads();
@@ -1655,8 +1683,8 @@ k_sortp_hist(const uint64_t* words, uint64_t n, uint32_t pass, uint32_t idx_bits
  * over 256 totals) are left to every scatter workgroup. */
 template <int THREADS>
 __global__ void __launch_bounds__(THREADS)
-k_sortp_scan_digits(uint32_t* hist, uint32_t n_blocks, uint32_t* totals, uint32_t pass, const Scalars* sc) {
-  if (sort_pass_idle(sc, pass)) return;
+k_sortp_scan_digits(uint32_t* hist, uint32_t n_blocks, uint32_t* totals, uint32_t pass, int finish, const Scalars* sc) {
+  if (sort_pass_idle(sc, sort_run(sc, finish), pass)) return;
   __shared__ uint32_t wave_tot[THREADS / 64];
   uint32_t* row = hist + (uint64_t)blockIdx.x * n_blocks;
   const uint32_t per = (n_blocks + THREADS - 1) / THREADS;
@@ -1678,12 +1706,14 @@ k_sortp_scan_digits(uint32_t* hist, uint32_t n_blocks, uint32_t* totals, uint32_
 
 template <int BITS, int THREADS, int ITEMS, bool FROM_KEYS>
 __global__ void __launch_bounds__(THREADS)
-k_sortp_scatter(const uint64_t* in, uint64_t* words_out, uint32_t* perm_out, uint64_t n, uint32_t pass, uint32_t idx_bits, const Scalars* sc,
+k_sortp_scatter(const uint64_t* in, uint64_t* words_out, uint32_t* perm_out, uint64_t n, uint32_t pass, uint32_t idx_bits, int finish, const Scalars* sc,
                 const uint32_t* hist_scanned, const uint32_t* totals, uint32_t n_blocks) {
   using P = SortP<BITS, THREADS, ITEMS>;
-  if (sort_pass_idle(sc, pass)) return;
-  const bool TO_PERM = pass + 1u == sort_passes(sc);
-  const uint32_t shift = FROM_KEYS ? 0u : idx_bits + (pass - 1u) * BITS;
+  const SortRun run = sort_run(sc, finish);
+  if (sort_pass_idle(sc, run, pass)) return;
+  const bool TO_PERM = pass + 1u == run.passes && run.low == 0;
+  const uint32_t shift = FROM_KEYS ? run.low : sort_shift(run, pass, idx_bits);
+  const uint32_t gone = run.low ? 0u : (uint32_t)BITS; /* of the key, from the word */
   __shared__ uint64_t s_word[P::TILE];
   __shared__ uint16_t s_digit[FROM_KEYS ? P::TILE : 1]; /* the first pass's digit is no longer part of the word */
   __shared__ uint32_t wave_run[P::WAVES][P::NB]; /* count per (wavefront, digit), then its start inside the digit's run */
@@ -1741,12 +1771,8 @@ k_sortp_scatter(const uint64_t* in, uint64_t* words_out, uint32_t* perm_out, uin
     const uint64_t i = chunk + (uint64_t)r * 64u + lane;
     const bool valid = i < n;
     uint32_t digit;
-    if (FROM_KEYS) {
-      digit = (uint32_t)word[r] & (P::NB - 1u);
-      word[r] = (((word[r] >> BITS)) << idx_bits) | i;
-    } else {
-      digit = (uint32_t)(word[r] >> shift) & (P::NB - 1u);
-    }
+    digit = (uint32_t)(word[r] >> shift) & (P::NB - 1u);
+    if (FROM_KEYS) word[r] = ((word[r] >> gone) << idx_bits) | i;
     dig[r] = (uint16_t)digit;
     /* lanes of this wavefront holding the same digit */
     uint64_t peers = __ballot(valid ? 1 : 0);
@@ -1822,8 +1848,9 @@ template <int BITS, int THREADS, int ITEMS>
 __global__ void __launch_bounds__(THREADS)
 k_sortp_single(Columns c, uint32_t n, SortSets s, Scalars* sc, uint32_t* perm_out) {
   using P = SortP<BITS, THREADS, ITEMS>;
-  const uint32_t ts_bits = sc->sort.ts_bits, res_bits = sc->sort.res_bits, key_bits = sc->sort.key_bits;
-  if (!sort_words_suffice(sc, key_bits, 0u, 64u)) { /* key and index are kept apart here */
+  const SortPlan plan = sc->sort;
+  const uint32_t key_bits = plan.key_bits;
+  if (!sort_words_suffice(sc, sort_run(sc, 0), key_bits, 0u, 64u)) { /* key and index are kept apart here */
     if (threadIdx.x == 0) flag_error(sc, KTJ_DEVERR_CAREFUL);
     return;
   }
@@ -1847,17 +1874,16 @@ k_sortp_single(Columns c, uint32_t n, SortSets s, Scalars* sc, uint32_t* perm_ou
 #pragma unroll
   for (int r = 0; r < P::ITEMS; ++r) {
     const uint32_t a = chunk + (uint32_t)r * 64u + lane;
-    uint64_t k = 1ULL << key_bits; /* dropped rows sort behind everything */
+    uint64_t k = sort_key_dropped(plan);
     if (a < n && (c.meta[a] & KTJ_M_VALID)) {
       const uint64_t rd = set_rank(s.dev_keys, s.dev_rank, (uint64_t)c.dev[a]);
       const uint64_t rr = set_rank(s.res_keys, s.res_rank, (uint64_t)c.res[a]);
-      const uint64_t rel = ((uint64_t)c.ts[a] ^ 0x8000000000000000ULL) - ts_min;
-      k = ((((rd << res_bits) | rr)) << ts_bits) | rel;
+      k = sort_key(plan, rd, rr, ((uint64_t)c.ts[a] ^ 0x8000000000000000ULL) - ts_min);
     }
     key[r] = k;
     idx[r] = (uint16_t)a;
   }
-  const uint32_t passes = (key_bits + 1u + BITS - 1u) / BITS;
+  const uint32_t passes = key_bits ? (key_bits + BITS - 1u) / BITS : 1u;
   for (uint32_t pass = 0; pass < passes; ++pass) {
     const uint32_t shift = pass * BITS;
 #pragma unroll
@@ -1921,8 +1947,112 @@ k_sortp_single(Columns c, uint32_t n, SortSets s, Scalars* sc, uint32_t* perm_ou
   for (uint32_t p = threadIdx.x; p < n; p += THREADS) perm_out[p] = s_idx[p];
 }
 
+/* The words are in order but for their lowest bits (of the key; the index below them makes every word another).  Rows that differ
+ * in these only are neighbours, rows of a track within 65 us at most: a group.  They are in order of arrival, mostly that of their
+ * times; a row moves up by the rows in front of it that are larger and down by those behind it that are smaller.  A row is
+ * compared as 32 bits, the number of its group in the workgroup's rows and the lowest bits, so that rows of other groups need no
+ * look of their own.  Groups of more than FINISH_MOST rows must be in order already, or the whole order is made again with passes over all
+ * bits (KTJ_DEVERR_UNSORTED).  How long a group is, every workgroup that has a row of it sees alike: it loads that many rows in front
+ * of and behind its own.
+ *
+ * Takes the place of one or two of five passes (a count, a scan, a scatter each: 135 us for 22 million rows). */
+#define FINISH_MOST 256u
+#define CHAIN_MAX_N 98304ull /* of sort_packed_chain */
+template <int THREADS, int ITEMS>
+__global__ void __launch_bounds__(THREADS)
+k_sortp_finish(const uint64_t* buf_a, const uint64_t* buf_b, uint32_t* perm, uint64_t n, uint32_t idx_bits, Scalars* sc) {
+  constexpr uint32_t ROWS = ITEMS + 2, SPAN = THREADS * ROWS, CHUNKS = SPAN / 64u; /* the tile's rows, a turn in front of and one behind them */
+  static_assert(THREADS == FINISH_MOST && CHUNKS <= 128u && SPAN < 0x10000u, "chunks of a wavefront's lanes, numbers of groups");
+  __shared__ uint32_t s_val[SPAN];
+  __shared__ uint64_t s_edge[CHUNKS], s_start[CHUNKS]; /* a chunk's last word; a bit per row: first of its group */
+  const SortRun run = sort_run(sc, 1);
+  if (sc->error != 0 || run.low == 0) return; /* the last pass has written the permutation */
+  const uint64_t* in = run.passes & 1u ? buf_b : buf_a;
+  const uint32_t group_shift = idx_bits + run.low, lane = lane_id(), wave = threadIdx.x >> 6;
+  const uint64_t idx_mask = (1ULL << idx_bits) - 1ULL;
+  const uint64_t from = (uint64_t)blockIdx.x * (THREADS * ITEMS) - FINISH_MOST; /* (below 0: not loaded) */
+  uint64_t word[ROWS];
+#pragma unroll
+  for (uint32_t r = 0; r < ROWS; ++r) { /* (all loads in flight together) */
+    const uint64_t i = from + r * THREADS + threadIdx.x; /* row, or wrapped around */
+    word[r] = i < n ? in[i] : 0;
+  }
+#pragma unroll
+  for (uint32_t r = 0; r < ROWS; ++r) if (lane == 63u) s_edge[r * (THREADS / 64u) + wave] = word[r];
+  __syncthreads();
+  int turns = 0; /* rows smaller than the one in front of them, of the same group */
+#pragma unroll
+  for (uint32_t r = 0; r < ROWS; ++r) {
+    const uint64_t i = from + r * THREADS + threadIdx.x;
+    const uint32_t c = r * (THREADS / 64u) + wave;
+    uint64_t before = (uint64_t)__shfl_up((unsigned long long)word[r], 1);
+    if (lane == 0u) before = s_edge[c ? c - 1u : 0u];
+    /* (the first of the span begins a group whatever is in front of it: with a row of this tile that is one of too many) */
+    const bool same = (c != 0u || lane != 0u) && i < n && i != 0 && ((word[r] ^ before) >> group_shift) == 0;
+    const uint64_t starts = __ballot(!same);
+    if (lane == 0u) s_start[c] = starts;
+    turns |= same && word[r] < before ? 1 : 0;
+  }
+  turns = __syncthreads_or(turns);
+  if (!turns) {
+#pragma unroll
+    for (uint32_t r = 1; r <= ITEMS; ++r) {
+      const uint64_t i = from + r * THREADS + threadIdx.x;
+      if (i < n) perm[i] = (uint32_t)(word[r] & idx_mask);
+    }
+    return;
+  }
+  uint32_t upto0 = (uint32_t)__popcll(s_start[lane < CHUNKS ? lane : 0u]), upto1 = CHUNKS > 64u ? (uint32_t)__popcll(s_start[lane + 64u < CHUNKS ? lane + 64u : 0u]) : 0u;
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t x = __shfl_up(upto0, o), y = __shfl_up(upto1, o);
+    if (lane >= (uint32_t)o) { upto0 += x; upto1 += y; }
+  }
+  uint32_t val[ROWS];
+  const uint32_t low_mask = (1u << run.low) - 1u, all0 = __builtin_amdgcn_readlane(upto0, 63);
+#pragma unroll
+  for (uint32_t r = 0; r < ROWS; ++r) {
+    const uint32_t c = __builtin_amdgcn_readfirstlane(r * (THREADS / 64u) + wave);
+    const uint32_t groups = c == 0u ? 0u : c <= 64u ? __builtin_amdgcn_readlane(upto0, (c - 1u) & 63u) : all0 + __builtin_amdgcn_readlane(upto1, (c - 65u) & 63u);
+    const uint64_t starts = s_start[c] & (~0ULL >> (63u - lane));
+    val[r] = ((groups + (uint32_t)__popcll(starts)) << 16) | ((uint32_t)(word[r] >> idx_bits) & low_mask);
+    s_val[r * THREADS + threadIdx.x] = val[r];
+  }
+  __syncthreads();
+  bool unsorted = false;
+#pragma unroll
+  for (uint32_t r = 1; r <= ITEMS; ++r) {
+    const uint64_t i = from + r * THREADS + threadIdx.x;
+    const uint32_t k = r * THREADS + threadIdx.x, v = val[r];
+    uint32_t moves = 0, d = 1;
+    for (; d < FINISH_MOST; d += 2u) { /* as far as any lane's group reaches */
+      const uint32_t x0 = s_val[k + d], y0 = s_val[k - d], x1 = s_val[k + d + 1u], y1 = s_val[k - d - 1u];
+      moves += x0 < v ? 1u : 0u;
+      moves += x1 < v ? 1u : 0u;
+      moves -= y0 > v ? 1u : 0u;
+      moves -= y1 > v ? 1u : 0u;
+      const uint32_t x = x1 ^ v, y = y1 ^ v;
+      if (!__any((x < y ? x : y) < 0x10000u)) break;
+    }
+    if (d > FINISH_MOST / 2u) { /* a group that is too long?  (One of its two ends is farther than that from any of its rows.) */
+      uint32_t others = 0;
+      for (d = 1; d <= FINISH_MOST; ++d) others += ((s_val[k + d] ^ v) < 0x10000u ? 1u : 0u) + ((s_val[k - d] ^ v) < 0x10000u ? 1u : 0u);
+      if (others >= FINISH_MOST) { moves = 0; unsorted = unsorted || s_val[k - 1u] > v; }
+    }
+    if (i < n) perm[i + (uint64_t)(int64_t)(int32_t)moves] = (uint32_t)(word[r] & idx_mask);
+  }
+  if (unsorted) flag_error(sc, KTJ_DEVERR_UNSORTED);
+}
+static hipError_t sort_finish(const uint64_t* buf_a, const uint64_t* buf_b, uint32_t* perm, uint64_t n, uint32_t idx_bits, Scalars* sc, hipStream_t st) {
+  /* tiles that leave no CU without one; large ones where there are enough, as the rows around a tile are loaded twice */
+  auto launch = [&](auto kernel, uint64_t tile) { hipLaunchKernelGGL(kernel, dim3((unsigned)((n + tile - 1) / tile)), dim3(256), 0, st, buf_a, buf_b, perm, n, idx_bits, sc); };
+  if (n <= CHAIN_MAX_N) launch(k_sortp_finish<256, 1>, 256);
+  else if (n < 1ull << 20) launch(k_sortp_finish<256, 4>, 1024);
+  else launch(k_sortp_finish<256, 16>, 4096);
+  return KTJ_LAUNCH_CHECK();
+}
+
 template <int BITS, int THREADS, int ITEMS>
-static hipError_t sort_packed_t(Columns c, uint64_t n, SortSets s, Scalars* sc, uint32_t passes, uint32_t idx_bits, uint64_t* buf_a, uint64_t* buf_b,
+static hipError_t sort_packed_t(Columns c, uint64_t n, SortSets s, Scalars* sc, uint32_t passes, int finish, uint32_t idx_bits, uint64_t* buf_a, uint64_t* buf_b,
                                 uint32_t* perm, uint32_t* hist, hipStream_t st) {
   using P = SortP<BITS, THREADS, ITEMS>;
   const uint32_t n_blocks = (uint32_t)((n + P::TILE - 1) / P::TILE);
@@ -1933,20 +2063,21 @@ static hipError_t sort_packed_t(Columns c, uint64_t n, SortSets s, Scalars* sc, 
   /* the digits' totals live behind the counts (radix_tmp_elems leaves 256 spare entries) */
   uint32_t* totals = hist + (uint64_t)P::NB * n_blocks;
   static_assert(P::NB <= 256, "room for the totals behind the counts");
-  hipLaunchKernelGGL((k_sortp_make_keys<BITS, THREADS, ITEMS, false>), g, b, 0, st, c, n, s, sc, idx_bits, passes, buf_a, counts, n_blocks);
-  if (!single) hipLaunchKernelGGL((k_sortp_scan_digits<THREADS>), dim3(P::NB), b, 0, st, hist, n_blocks, totals, 0u, (const Scalars*)sc);
-  hipLaunchKernelGGL((k_sortp_scatter<BITS, THREADS, ITEMS, true>), g, b, 0, st, (const uint64_t*)buf_a, buf_b, perm, n, 0u, idx_bits,
+  hipLaunchKernelGGL((k_sortp_make_keys<BITS, THREADS, ITEMS, false>), g, b, 0, st, c, n, s, sc, idx_bits, passes, finish, buf_a, counts, n_blocks);
+  if (!single) hipLaunchKernelGGL((k_sortp_scan_digits<THREADS>), dim3(P::NB), b, 0, st, hist, n_blocks, totals, 0u, finish, (const Scalars*)sc);
+  hipLaunchKernelGGL((k_sortp_scatter<BITS, THREADS, ITEMS, true>), g, b, 0, st, (const uint64_t*)buf_a, buf_b, perm, n, 0u, idx_bits, finish,
                      (const Scalars*)sc, (const uint32_t*)counts, (const uint32_t*)totals, n_blocks);
   uint64_t* in = buf_b; uint64_t* out = buf_a;
   for (uint32_t p = 1; p < passes; ++p) {
     if (!single) {
-      hipLaunchKernelGGL((k_sortp_hist<BITS, THREADS, ITEMS>), g, b, 0, st, (const uint64_t*)in, n, p, idx_bits, (const Scalars*)sc, hist, n_blocks);
-      hipLaunchKernelGGL((k_sortp_scan_digits<THREADS>), dim3(P::NB), b, 0, st, hist, n_blocks, totals, p, (const Scalars*)sc);
+      hipLaunchKernelGGL((k_sortp_hist<BITS, THREADS, ITEMS>), g, b, 0, st, (const uint64_t*)in, n, p, idx_bits, finish, (const Scalars*)sc, hist, n_blocks);
+      hipLaunchKernelGGL((k_sortp_scan_digits<THREADS>), dim3(P::NB), b, 0, st, hist, n_blocks, totals, p, finish, (const Scalars*)sc);
     }
-    hipLaunchKernelGGL((k_sortp_scatter<BITS, THREADS, ITEMS, false>), g, b, 0, st, (const uint64_t*)in, out, perm, n, p, idx_bits,
+    hipLaunchKernelGGL((k_sortp_scatter<BITS, THREADS, ITEMS, false>), g, b, 0, st, (const uint64_t*)in, out, perm, n, p, idx_bits, finish,
                        (const Scalars*)sc, (const uint32_t*)counts, (const uint32_t*)totals, n_blocks);
     uint64_t* t = in; in = out; out = t;
   }
+  if (finish) return sort_finish(buf_a, buf_b, perm, n, idx_bits, sc, st);
   return KTJ_LAUNCH_CHECK();
 }
 
@@ -1962,17 +2093,17 @@ static hipError_t sort_packed_t(Columns c, uint64_t n, SortSets s, Scalars* sc, 
  * 4500 records 203 -> 177 us, 30 000 219 -> 202, 60 000 224 -> 216, 90 000 228 both, 120 000 229 -> 234; counts to
  * add up and cells to hand on grow with the tiles (at 733 000 keys a pass took 30 us instead of 25). */
 #define CHAIN_THREADS 1024
-#define CHAIN_MAX_N 98304ull
 template <int BITS, bool FROM_KEYS>
 __global__ void __launch_bounds__(CHAIN_THREADS)
-k_sortp_chain(const uint64_t* in, uint64_t* words_out, uint32_t* perm_out, uint32_t n, uint32_t pass, uint32_t idx_bits, const Scalars* sc,
+k_sortp_chain(const uint64_t* in, uint64_t* words_out, uint32_t* perm_out, uint32_t n, uint32_t pass, uint32_t idx_bits, int finish, const Scalars* sc,
               uint32_t* hist, uint32_t n_blocks) {
   using P = SortP<BITS, CHAIN_THREADS, 1>;
   constexpr uint32_t NB = P::NB, GROUPS = CHAIN_THREADS / NB;
-  if (sort_pass_idle(sc, pass)) return;
-  const bool TO_PERM = pass + 1u == sort_passes(sc);
-  const uint32_t shift = FROM_KEYS ? 0u : idx_bits + (pass - 1u) * BITS;
-  const uint32_t next_shift = FROM_KEYS ? idx_bits : shift + BITS;
+  const SortRun run = sort_run(sc, finish);
+  if (sort_pass_idle(sc, run, pass)) return;
+  const bool LAST = pass + 1u == run.passes, TO_PERM = LAST && run.low == 0;
+  const uint32_t shift = FROM_KEYS ? run.low : sort_shift(run, pass, idx_bits);
+  const uint32_t next_shift = sort_shift(run, pass + 1u, idx_bits);
   __shared__ uint32_t next[CHAIN_MAX_N / P::TILE * (NB / 2u)]; /* two cells a word */
   __shared__ uint32_t wave_run[P::WAVES][NB];
   __shared__ uint32_t part[2][GROUPS][NB]; /* counts before this tile, of all tiles */
@@ -1996,14 +2127,11 @@ k_sortp_chain(const uint64_t* in, uint64_t* words_out, uint32_t* perm_out, uint3
     part[1][group][d] = all;
   }
   for (uint32_t k = threadIdx.x; k < P::WAVES * NB; k += CHAIN_THREADS) (&wave_run[0][0])[k] = 0;
-  if (!TO_PERM)
+  if (!LAST)
     for (uint32_t k = threadIdx.x; k < n_blocks * (NB / 2u); k += CHAIN_THREADS) next[k] = 0;
   __syncthreads();
-  uint32_t digit;
-  if (FROM_KEYS) {
-    digit = (uint32_t)word & (NB - 1u);
-    word = ((word >> BITS) << idx_bits) | i;
-  } else digit = (uint32_t)(word >> shift) & (NB - 1u);
+  const uint32_t digit = (uint32_t)(word >> shift) & (NB - 1u);
+  if (FROM_KEYS) word = ((word >> (run.low ? 0u : (uint32_t)BITS)) << idx_bits) | i;
   uint64_t peers = __ballot(valid ? 1 : 0);
 #pragma unroll
   for (int b = 0; b < BITS; ++b) {
@@ -2038,11 +2166,12 @@ k_sortp_chain(const uint64_t* in, uint64_t* words_out, uint32_t* perm_out, uint3
     if (TO_PERM) perm_out[dst] = (uint32_t)(word & ((1ULL << idx_bits) - 1ULL));
     else {
       words_out[dst] = word;
+      if (LAST) return;
       const uint32_t cell = (dst / (uint32_t)P::TILE) * NB + ((uint32_t)(word >> next_shift) & (NB - 1u));
       atomicAdd(&next[cell >> 1], cell & 1u ? 0x10000u : 1u);
     }
   }
-  if (TO_PERM) return;
+  if (LAST) return;
   __syncthreads();
   uint32_t* next_hist = hist + (uint64_t)(pass + 1u) * n_blocks * NB;
   for (uint32_t k = threadIdx.x; k < n_blocks * (NB / 2u); k += CHAIN_THREADS) {
@@ -2052,20 +2181,21 @@ k_sortp_chain(const uint64_t* in, uint64_t* words_out, uint32_t* perm_out, uint3
   }
 }
 template <int BITS>
-static hipError_t sort_packed_chain(Columns c, uint64_t n, SortSets s, Scalars* sc, uint32_t passes, uint32_t idx_bits, uint64_t* buf_a,
+static hipError_t sort_packed_chain(Columns c, uint64_t n, SortSets s, Scalars* sc, uint32_t passes, int finish, uint32_t idx_bits, uint64_t* buf_a,
                                     uint64_t* buf_b, uint32_t* perm, uint32_t* hist, hipStream_t st) {
   using P = SortP<BITS, CHAIN_THREADS, 1>;
   const uint32_t n_blocks = (uint32_t)((n + P::TILE - 1) / P::TILE);
   const dim3 g(n_blocks), b(CHAIN_THREADS);
-  hipLaunchKernelGGL((k_sortp_make_keys<BITS, CHAIN_THREADS, 1, true>), g, b, 0, st, c, n, s, sc, idx_bits, passes, buf_a, hist, n_blocks);
-  hipLaunchKernelGGL((k_sortp_chain<BITS, true>), g, b, 0, st, (const uint64_t*)buf_a, buf_b, perm, (uint32_t)n, 0u, idx_bits,
+  hipLaunchKernelGGL((k_sortp_make_keys<BITS, CHAIN_THREADS, 1, true>), g, b, 0, st, c, n, s, sc, idx_bits, passes, finish, buf_a, hist, n_blocks);
+  hipLaunchKernelGGL((k_sortp_chain<BITS, true>), g, b, 0, st, (const uint64_t*)buf_a, buf_b, perm, (uint32_t)n, 0u, idx_bits, finish,
                      (const Scalars*)sc, hist, n_blocks);
   uint64_t* in = buf_b; uint64_t* out = buf_a;
   for (uint32_t p = 1; p < passes; ++p) {
-    hipLaunchKernelGGL((k_sortp_chain<BITS, false>), g, b, 0, st, (const uint64_t*)in, out, perm, (uint32_t)n, p, idx_bits,
+    hipLaunchKernelGGL((k_sortp_chain<BITS, false>), g, b, 0, st, (const uint64_t*)in, out, perm, (uint32_t)n, p, idx_bits, finish,
                        (const Scalars*)sc, hist, n_blocks);
     uint64_t* t = in; in = out; out = t;
   }
+  if (finish) return sort_finish(buf_a, buf_b, perm, n, idx_bits, sc, st);
   return KTJ_LAUNCH_CHECK();
 }
 #define SORTP_THREADS 256
@@ -2074,12 +2204,14 @@ static bool g_sortp_no_single = false;
 void sort_packed_force_passes(bool on) { g_sortp_no_single = on; }
 bool sort_packed_passes_forced() { return g_sortp_no_single; }
 static uint32_t sort_idx_bits(uint64_t n) { return (uint32_t)(64 - __builtin_clzll(n > 1 ? n - 1 : 1)); }
-bool sort_packed_fits(uint64_t n, uint32_t key_bits) {
-  const uint32_t total_bits = key_bits + 1u;
-  return (total_bits > SORTP_BITS ? total_bits - SORTP_BITS : 0u) + sort_idx_bits(n) <= 64u;
+bool sort_packed_fits(uint64_t n, const SortPlan& plan) {
+  return plan.key_bits <= 62u && (plan.key_bits > SORTP_BITS ? plan.key_bits - SORTP_BITS : 0u) + sort_idx_bits(n) <= 64u;
 }
-uint32_t sort_packed_passes(uint32_t key_bits) { return (key_bits + SORTP_BITS) / SORTP_BITS; }
-hipError_t sort_packed(Columns c, uint64_t n, SortSets s, Scalars* sc, uint32_t passes, uint64_t* buf_a, uint64_t* buf_b, uint32_t* perm,
+uint32_t sort_packed_passes(const SortPlan& plan, bool finish) {
+  const uint32_t bits = plan.key_bits - (finish ? plan.low_bits : 0u);
+  return bits ? (bits + SORTP_BITS - 1u) / SORTP_BITS : 1u;
+}
+hipError_t sort_packed(Columns c, uint64_t n, SortSets s, Scalars* sc, uint32_t passes, bool finish, uint64_t* buf_a, uint64_t* buf_b, uint32_t* perm,
                        uint32_t* hist, uint32_t* chain_hist, hipStream_t st) {
   if (n == 0) return hipSuccess;
   const uint32_t idx_bits = sort_idx_bits(n);
@@ -2092,10 +2224,10 @@ hipError_t sort_packed(Columns c, uint64_t n, SortSets s, Scalars* sc, uint32_t 
    * SORTP_SMALL_N keys, tiles of 512 spread over the GPU finish a pass sooner than the few 4096-key tiles
    * would (330 000 keys: 113 against 155 us; from a million keys on the large tiles win) */
   if (n > (uint64_t)SORTP_THREADS * 16u && n <= CHAIN_MAX_N && 256ull * passes * ((n + CHAIN_THREADS - 1) / CHAIN_THREADS) <= 2 * (n + 1))
-    return sort_packed_chain<SORTP_BITS>(c, n, s, sc, passes, idx_bits, buf_a, buf_b, perm, chain_hist, st);
+    return sort_packed_chain<SORTP_BITS>(c, n, s, sc, passes, finish, idx_bits, buf_a, buf_b, perm, chain_hist, st);
   if (n > (uint64_t)SORTP_THREADS * 16u && n < SORTP_SMALL_N)
-    return sort_packed_t<SORTP_BITS, SORTP_THREADS, 2>(c, n, s, sc, passes, idx_bits, buf_a, buf_b, perm, hist, st);
-  return sort_packed_t<SORTP_BITS, SORTP_THREADS, 16>(c, n, s, sc, passes, idx_bits, buf_a, buf_b, perm, hist, st);
+    return sort_packed_t<SORTP_BITS, SORTP_THREADS, 2>(c, n, s, sc, passes, finish, idx_bits, buf_a, buf_b, perm, hist, st);
+  return sort_packed_t<SORTP_BITS, SORTP_THREADS, 16>(c, n, s, sc, passes, finish, idx_bits, buf_a, buf_b, perm, hist, st);
 }
 
 /* ------------------------------------------------------------------------------------------ */

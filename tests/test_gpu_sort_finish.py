@@ -1,0 +1,96 @@
+"""The sort leaves the key's lowest bits out of its passes and puts rows that differ in these only, a group, into order behind them
+(k_sortp_finish): documents against the oracle with groups at the edges of a tile and of the longest that is put into order, in order
+of arrival and not, and with groups beyond it, whose order is made with passes over all bits."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import oracle_glue as og
+from kineto_amd import abi
+from kineto_amd.engine import TraceEngine
+from stream_builder import B, StreamBuilder
+
+pytestmark = pytest.mark.gpu
+
+
+def ops(ts, tid, window=None):
+    """CPU ops in this order of arrival; with a window: launches, of which it drops some."""
+    n = len(ts)
+    b = StreamBuilder(window=window or (B, B + 10**15), host_name="sort")
+    b.api(["hipLaunchKernel"], flow_start=[0])
+    names = [b.s("op%d" % k) for k in range(7)]
+    sp = b.build()
+    if window is None:
+        rec = np.zeros(n, dtype=np.dtype(abi.GenericRec))
+        rec["start_ns"], rec["end_ns"] = ts, ts + 5 + np.arange(n) % 900
+        rec["resource"], rec["device"], rec["id"] = tid, 4242, np.arange(n) + 1
+        rec["name_id"], rec["schema_id"] = np.array(names)[np.arange(n) % 7], abi.KTJ_NONE
+        held = (abi.GenericRec * n).from_buffer_copy(rec.tobytes())
+        sp.contents.generic, sp.contents.n_generic = C.cast(held, type(sp.contents.generic)), n
+    else:
+        rec = np.zeros(n, dtype=np.dtype(abi.RuntimeRec))
+        rec["begin"], rec["end"], rec["tid"], rec["pid"], rec["id"] = ts, ts + 5, tid, 4242, np.arange(n) + 1
+        held = (abi.RuntimeRec * n).from_buffer_copy(rec.tobytes())
+        sp.contents.runtime, sp.contents.n_runtime = C.cast(held, type(sp.contents.runtime)), n
+    sp._held = (held, b)
+    return sp
+
+
+def same_as_oracle(sp):
+    ora = og.OracleRun(sp)
+    want = ora.output()
+    with TraceEngine(sp.contents.trace_name.decode()) as eng:
+        eng.submit_stream(sp)
+        for turn in range(2):   # the second one knows how many passes there are
+            eng.process()
+            assert eng.output() == want, turn
+    ora.close()
+
+
+def groups(n, size, order, threads=3, seed=1):
+    """Rows in groups of `size` neighbours within 500 ns, groups a millisecond apart, each thread's rows of a group in this order."""
+    rng = np.random.default_rng(seed)
+    k = np.arange(n)
+    group, inside = k // (size * threads), k % (size * threads)
+    place = inside // threads
+    if order == "backwards":
+        place = size - 1 - place
+    elif order == "shuffled":
+        place = rng.permutation(size)[place]
+    elif order == "halves":   # one row only is smaller than the one before it
+        place = (place + size // 2) % size
+    ts = B + 10**6 + group * 2**20 + place * 500 // size   # (some at the same time: these stay as they came)
+    return ts, 5 + inside % threads
+
+
+@pytest.mark.parametrize("order", ("forwards", "backwards", "shuffled", "halves"))
+@pytest.mark.parametrize("size", (1, 2, 63, 64, 65, 255, 256, 257, 400, 700))
+def test_groups(size, order):
+    """257 rows and more, not in order: all bits by passes."""
+    print(size, order, flush=True)
+    same_as_oracle(ops(*groups(9001, size, order)))
+
+
+@pytest.mark.parametrize("n", (4097, 8191, 98304, 98305, 262144 + 7))
+def test_sizes(n):
+    """One launch a pass, tiles of 512 and tiles behind them, whole and with a few rows."""
+    print(n, flush=True)
+    same_as_oracle(ops(*groups(n, 256, "backwards", threads=2)))
+
+
+def test_large_tiles():
+    ts, tid = groups(1200001, 97, "shuffled", threads=5)
+    same_as_oracle(ops(ts, tid))
+
+
+def test_dropped_rows_and_random_order():
+    rng = np.random.default_rng(5)
+    for n in (5000, 20001):
+        ts = B + rng.integers(0, 10**9, n)
+        same_as_oracle(ops(ts, 5 + rng.integers(0, 4, n)))                                # any order
+        same_as_oracle(ops(ts, 5 + rng.integers(0, 4, n), (B + 10**8, B + 6 * 10**8)))    # half of them outside the window
+        same_as_oracle(ops(ts, 5 + rng.integers(0, 4, n), (B + 10**10, B + 10**11)))      # all of them
+        same_as_oracle(ops(np.full(n, B + 77), 5 + rng.integers(0, 4, n)))                # one time
+        far = np.where(np.arange(n) == n // 2, 1000, ts)                                  # a row at the clock's beginning
+        same_as_oracle(ops(far, 5 + rng.integers(0, 4, n)))
