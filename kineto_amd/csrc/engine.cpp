@@ -286,6 +286,8 @@ struct ktj_engine {
   bool small_last = false;   /* the last pass was a small one: it leaves no intermediate arrays for ktj_debug_fetch */
   bool no_small = false;     /* ktj_debug_fetch makes them */
   bool no_weave = false;     /* joined rows as they are: ktj_debug_fetch */
+  bool all_columns = false;  /* ktj_debug_fetch */
+  bool columns_are_all = true; /* of the last pass: Columns::all */
   bool no_room_for_text = false; /* and where these records' text rows do not fit into memory */
   hipError_t hip_error = hipSuccess; /* of the last call that failed */
   int64_t last_end_time = 0;
@@ -1296,6 +1298,7 @@ static Columns columns_of(const ktj_engine* e) {
   c.ts = e->c_ts.as<int64_t>(); c.dur = e->c_dur.as<int64_t>(); c.corr = e->c_corr.as<uint64_t>();
   c.dev = e->c_dev.as<int64_t>(); c.res = e->c_res.as<int64_t>(); c.meta = e->c_meta.as<uint32_t>();
   c.ext = e->c_ext.as<int32_t>();
+  c.all = e->columns_are_all;
   return c;
 }
 static hipError_t know_wall_clock(ktj_engine* e) {
@@ -1499,6 +1502,7 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
   const bool woven = n_coll == 0 && !e->noalloc && !e->no_weave && !e->no_room_for_text && !(e->flags & KTJ_CREATE_TILE_EMIT) && (e->not_woven == 0 || e->not_woven != ng + nr + nd);
   e->rows_are_text = woven;
   e->pass_info[0] = woven; e->pass_info[1] = e->pass_info[2] = e->pass_info[3] = 0;
+  e->columns_are_all = e->all_columns || max_spans != 0 || e->noalloc;
   const bool wide = woven && std::any_of(e->fields.begin(), e->fields.end(), [](const ktj_field& f) { return f.type == KTJ_F_F64; });
   e->pool_used = 0;
   size_t pass_bytes = 0;
@@ -1507,7 +1511,7 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
   e->pool_need = 0;
   NEED(e->d_entries, (ns + 1ull) * sizeof(DictEntry));
   NEED(e->d_name_blob, e->blob_bytes * 2 + KTJ_DICT_ROOM * (ns + 1ull)); NEED(e->d_arg_blob, e->blob_bytes + KTJ_DICT_ROOM * (ns + 1ull));
-  NEED(e->c_ts, Na * 8); NEED(e->c_dur, Na * 8); NEED(e->c_corr, Na * 8);
+  NEED(e->c_ts, Na * 8); NEED(e->c_dur, e->columns_are_all ? Na * 8 : 16); NEED(e->c_corr, Na * 8);
   NEED(e->c_dev, Na * 8); NEED(e->c_res, Na * 8); NEED(e->c_meta, Na * 4);
   NEED(e->c_ext, Na * 4);
   NEED(e->t_full, (cap_full + 1ull) * 8); NEED(e->t_narrow, (cap_narrow + 1ull) * 8);
@@ -1613,7 +1617,7 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
   /* only external-correlation records and user spans ask for the CPU ops' ids (5 M records without any: 58 us) */
   if (nx || max_spans) HIPCHK(build_cpu_ids(g_recs, ng, t_cpu, cpu_row, sc, st));
   HIPCHK(build_extcorr(x_recs, nx, tn, nc, t_cpu, cpu_row, g_recs, ctx, sc, st));
-  HIPCHK(join_runtime_rows(r_recs, nr, c, ng, api, tf, fc, tn, nc, e->slot_f.as<uint32_t>(), e->slot_n.as<uint32_t>(), ctx, rows,
+  HIPCHK(join_runtime_rows(r_recs, nr, c, ng, api, tf, fc, tn, nc, e->slot_f.as<uint32_t>(), e->slot_n.as<uint32_t>(), clock_of(e), ctx, rows,
                            e->len.as<uint32_t>(), sc, st));
   HIPCHK(republish_runtime_rows(r_recs, nr, c, ng, fc, nc, e->slot_f.as<uint32_t>(), e->slot_n.as<uint32_t>(), sc, st));
   unsigned long long* orphans = e->keys_a.as<unsigned long long>(); /* a bit per device row: the sort's words come later */
@@ -1672,7 +1676,7 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
     e->perm = e->vals_a.as<uint32_t>();
     e->sorted_keys = nullptr;
     HIPCHK(sort_packed(c, N, sets, sc, e->passes_to_launch(N), !e->sort_all_bits, e->keys_a.as<uint64_t>(), e->keys_b.as<uint64_t>(), e->perm, e->hist.as<uint32_t>(), e->offs.as<uint32_t>(), st));
-    HIPCHK(mat_rows(g_recs, ng, 0, nullptr, d_recs, nd, c, ng + nr, e->dev_link.as<DevLink>(), ctx, rows, e->len.as<uint32_t>(), sc, st));
+    HIPCHK(mat_rows(g_recs, ng, 0, nullptr, d_recs, nd, c, ng + nr, e->dev_link.as<DevLink>(), clock_of(e), ctx, rows, e->len.as<uint32_t>(), sc, st));
     for (;;) {
       text.out = e->out.as<char>(); text.out_cap = e->out.cap;
       HIPCHK(gather_offsets(e->perm, e->len.as<uint32_t>(), N, e->len_sorted.as<uint32_t>(), e->kind_sorted.as<uint8_t>(),
@@ -1786,8 +1790,8 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
                              e->sync_pos.as<uint32_t>(), e->sync_first.as<uint32_t>(), sc, st));
     sync_first = e->sync_first.as<uint32_t>();
   }
-  HIPCHK(mat_rows(g_recs, ng, 0, sync_first, d_recs, nd, c, ng + nr, e->dev_link.as<DevLink>(), ctx, rows, e->len.as<uint32_t>(), sc, st));
-  HIPCHK(mat_rows(e->synth_recs.as<ktj_generic_rec>(), e->n_spans, ng + nr + nd, nullptr, nullptr, 0, c, 0, nullptr, ctx, rows,
+  HIPCHK(mat_rows(g_recs, ng, 0, sync_first, d_recs, nd, c, ng + nr, e->dev_link.as<DevLink>(), clock_of(e), ctx, rows, e->len.as<uint32_t>(), sc, st));
+  HIPCHK(mat_rows(e->synth_recs.as<ktj_generic_rec>(), e->n_spans, ng + nr + nd, nullptr, nullptr, 0, c, 0, nullptr, clock_of(e), ctx, rows,
                   e->len.as<uint32_t>(), sc, st));
   if (n_coll) HIPCHK(collective_first(mat, e->perm, e->scalars.n_valid, n_coll, e->d_coll_first.as<uint32_t>(), st));
 
@@ -2206,11 +2210,13 @@ int ktj_debug_fetch(ktj_engine* e, int what, void* dst, uint64_t cap, uint64_t* 
     return KTJ_OK;
   }
   const bool as_text = what == KTJ_DBG_MAT && e->rows_are_text;
-  if (e->small_last || as_text) { /* a small pass keeps none of these: the launches of a large trace make them (and the same document) */
+  const bool not_kept = (what == KTJ_DBG_COL_DUR || what == KTJ_DBG_COL_EXT) && !e->columns_are_all;
+  if (e->small_last || as_text || not_kept) { /* a small pass keeps none of these: the launches of a large trace make them (and the same document) */
     e->no_small = true;
     e->no_weave = what == KTJ_DBG_MAT;
+    e->all_columns = true;
     const int rc = ktj_process(e, e->last_end_time);
-    e->no_small = e->no_weave = false;
+    e->no_small = e->no_weave = e->all_columns = false;
     if (rc != KTJ_OK) return rc;
   }
   const void* src = nullptr;

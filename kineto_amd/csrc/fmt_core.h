@@ -153,7 +153,7 @@ KTJ_HD KTJ_FI inline int64_t convert_timestamp(uint64_t t, uint64_t t0_approx, i
   if (!(ta > t0a)) return 0;
   const uint64_t dt = (uint64_t)(ta - t0a); /* > 0 */
   /* (double)dt: round to nearest even at 53 bits */
-  int lz = 0; { uint64_t x = dt; while (!(x >> 63)) { x <<= 1; ++lz; } }
+  const int lz = __builtin_clzll(dt);
   uint64_t m1 = dt << lz;             /* normalised, bit 63 set */
   int e1 = 63 - lz;                   /* dt = m1 * 2^(e1-63) */
   { const uint64_t low = m1 & 0x7FF; m1 >>= 11; /* 53 bits */

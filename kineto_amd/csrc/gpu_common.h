@@ -203,6 +203,12 @@ __device__ __forceinline__ RowCols cols_device(const ktj_device_rec& d, const Cl
 __device__ __forceinline__ void store_cols(const Columns& c, uint64_t a, const RowCols& r) {
   c.ts[a] = r.ts; c.dur[a] = r.dur; c.corr[a] = r.corr; c.dev[a] = r.dev; c.res[a] = r.res; c.meta[a] = r.meta; c.ext[a] = 0;
 }
+/* what the launches behind read; linked: device rows, which are joined without their records */
+__device__ __forceinline__ void store_cols(const Columns& c, uint64_t a, const RowCols& r, bool linked) {
+  c.ts[a] = r.ts; c.dev[a] = r.dev; c.res[a] = r.res; c.meta[a] = r.meta;
+  if (linked || c.all) c.corr[a] = r.corr;
+  if (c.all) { c.dur[a] = r.dur; c.ext[a] = 0; }
+}
 
 __device__ __forceinline__ bool is_async_op(uint32_t domain) { return domain != KTJ_DOM_MEMSET; }
 

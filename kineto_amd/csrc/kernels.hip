@@ -460,7 +460,7 @@ __global__ void __launch_bounds__(KTJ_BLOCK) k_decode(DecodeJob J, Columns c, Em
     if (has) {
       const RowCols r = cols_generic(l[threadIdx.x], ctx);
       left = J.text && (r.meta & KTJ_M_VALID) && (weave::left_generic(l[threadIdx.x], r.dev, ctx, J.schemas_not_taken) || weave::far_apart(l[threadIdx.x].start_ns, l[0].start_ns));
-      store_cols(c, J.first + b * KTJ_BLOCK + threadIdx.x, r);
+      store_cols(c, J.first + b * KTJ_BLOCK + threadIdx.x, r, false);
     }
     /* rows that may need a Stream Sync row of their own are rare: the extra passes run only if any */
     block_add_two(sc, KTJ_CNT_SYNC_TYPED, has && l[threadIdx.x].type == KTJ_TYPE_CUDA_SYNC, KTJ_CNT_NOT_TEXT, left);
@@ -478,7 +478,7 @@ __global__ void __launch_bounds__(KTJ_BLOCK) k_decode(DecodeJob J, Columns c, Em
       const RowCols r = cols_runtime(l[threadIdx.x], J.clk, J.win_start, J.win_end);
       oor = !(r.meta & KTJ_M_VALID);
       left = J.text && !oor && (weave::left_runtime(l[threadIdx.x], r.ts, r.dur, ctx, J.n_cids) || weave::far_apart(l[threadIdx.x].begin, l[0].begin));
-      store_cols(c, J.ng + b * KTJ_BLOCK + threadIdx.x, r);
+      store_cols(c, J.ng + b * KTJ_BLOCK + threadIdx.x, r, false);
     }
     block_add_two(sc, KTJ_CNT_OUT_OF_RANGE, oor, KTJ_CNT_NOT_TEXT, left);
     return;
@@ -495,7 +495,7 @@ __global__ void __launch_bounds__(KTJ_BLOCK) k_decode(DecodeJob J, Columns c, Em
       const RowCols r = cols_device(*d, J.clk, J.win_start, J.win_end);
       oor = !(r.meta & KTJ_M_VALID);
       left = J.text && !oor && (weave::left_device(*d, r.ts, r.dur, r.res, ctx) || weave::far_apart(d->begin, l[0].begin));
-      store_cols(c, J.ng + J.nr + i, r);
+      store_cols(c, J.ng + J.nr + i, r, true);
       DevBrief br;
       br.queue = d->queue; br.device = d->device; br.domain = device_row_domain(d->domain);
       J.brief[i] = br;
@@ -2463,7 +2463,7 @@ __device__ __forceinline__ bool bitmap_test_and_set(uint32_t* bitmap, uint32_t s
 #endif
 template <bool TEXT>
 __global__ void KX_JOIN_ATTR k_join_runtime(const ktj_runtime_rec* r, uint64_t n, Columns c, uint64_t first_runtime, ApiTable api, Table tf,
-                               FullCols fc, Table tn, NarrowCols nc, uint32_t* slot_f, uint32_t* slot_n, EmitCtx ctx, Rows rows,
+                               FullCols fc, Table tn, NarrowCols nc, uint32_t* slot_f, uint32_t* slot_n, ClockDev clk, EmitCtx ctx, Rows rows,
                                uint32_t* len, Scalars* sc, int rounds) {
   RowStats rs;
   uint32_t n_linked = 0;
@@ -2493,10 +2493,9 @@ __global__ void KX_JOIN_ATTR k_join_runtime(const ktj_runtime_rec* r, uint64_t n
     uint32_t meta = 0;
     int64_t ts = 0, dur = 0;
     if (i < n) {
-      id = load_once(&c.corr[a]);
+      id = rec.id;
       meta = load_once(&c.meta[a]);
       ts = load_once(&c.ts[a]);
-      dur = load_once(&c.dur[a]);
       sf = slot_insert(tf, id);
     }
     const uint32_t kind = (meta & KTJ_M_KIND_MASK) >> KTJ_M_KIND_SHIFT;
@@ -2535,7 +2534,8 @@ __global__ void KX_JOIN_ATTR k_join_runtime(const ktj_runtime_rec* r, uint64_t n
       }
       store_once(&slot_n[i], sn);
       if ((np_info & KTJ_NP_LINKED) && valid) ++n_linked;
-      store_once(&c.ext[a], ext);
+      if (c.all) store_once(&c.ext[a], ext);
+      dur = duration_from(clk, clk.runtime_mode, ts, rec.end);
       const bool known = rec.cid < api.n_cids;
       const uint32_t name = known ? api.cid_name_ids[rec.cid] : KTJ_NONE;
       const bool fstart = known && ((api.flow_start_bits[rec.cid >> 5] >> (rec.cid & 31u)) & 1u);
@@ -2628,8 +2628,8 @@ __global__ void k_republish_runtime(const ktj_runtime_rec* r, uint64_t n, Column
 }
 template <bool TEXT>
 __device__ __forceinline__ void mat_device_block(const ktj_device_rec* d, uint64_t n, const Columns& c, uint64_t first, const DevLink* link,
-                                                 const EmitCtx& ctx, Rows rows, uint32_t* len, Scalars* sc, uint64_t block, uint64_t blocks,
-                                                 uint4* stage) {
+                                                 const ClockDev& clk, const EmitCtx& ctx, Rows rows, uint32_t* len, Scalars* sc, uint64_t block,
+                                                 uint64_t blocks, uint4* stage) {
   RowStats rs;
   for (uint64_t base = block * KTJ_BLOCK; base < n; base += blocks * KTJ_BLOCK) {
     const uint32_t cnt = (uint32_t)(n - base < KTJ_BLOCK ? n - base : KTJ_BLOCK);
@@ -2649,7 +2649,8 @@ __device__ __forceinline__ void mat_device_block(const ktj_device_rec* d, uint64
         lv[0] = load_once(&src[0]);
         lv[1] = load_once(&src[1]);
       }
-      m = mat_device_v(rec, load_once(&c.ts[a]), load_once(&c.dur[a]), load_once(&c.res[a]),
+      const int64_t ts = load_once(&c.ts[a]);
+      m = mat_device_v(rec, ts, duration_from(clk, clk.device_mode, ts, rec.end), load_once(&c.res[a]),
                        (load_once(&c.meta[a]) & KTJ_M_VALID) != 0, load_once(&c.ext[a]),
                        (l.flags & KTJ_DL_HAS_GRID) != 0, l.p[0], l.p[1], l.p[2], (l.flags & KTJ_DL_HAS_SIZE) != 0, l.p[0], l.coll);
       count_row_stats(m, ctx, &rs);
@@ -2667,7 +2668,7 @@ __device__ __forceinline__ void mat_device_block(const ktj_device_rec* d, uint64
 template <bool GENERIC, bool DEVICE, bool TEXT>
 __global__ void __launch_bounds__(KTJ_BLOCK) __attribute__((amdgpu_waves_per_eu(4)))
 k_mat_rows(const ktj_generic_rec* g, uint64_t ng, uint64_t first_generic, const uint32_t* sync_first, uint32_t generic_blocks, const ktj_device_rec* d,
-           uint64_t nd, Columns c, uint64_t first_device, const DevLink* link, EmitCtx ctx, Rows rows, uint32_t* len, Scalars* sc, int clock) {
+           uint64_t nd, Columns c, uint64_t first_device, const DevLink* link, ClockDev clk, EmitCtx ctx, Rows rows, uint32_t* len, Scalars* sc, int clock) {
   static_assert(sizeof(MatRow) >= sizeof(ktj_generic_rec) && sizeof(MatRow) >= sizeof(ktj_device_rec), "the staging area holds the records, then the joined rows");
   __shared__ uint4 stage[KTJ_BLOCK * sizeof(typename RowOf<TEXT>::T) / 16];
   if (blockIdx.x == 0 && threadIdx.x == 0 && clock) stage_clock(sc, KTJ_CLOCK_SIZE);
@@ -2677,7 +2678,7 @@ k_mat_rows(const ktj_generic_rec* g, uint64_t ng, uint64_t first_generic, const 
   if (GENERIC && (!DEVICE || blockIdx.x < generic_blocks))
     mat_generic_block<TEXT>(g, ng, first_generic, ctx, sync_first, rows, len, sc, blockIdx.x, generic_blocks, stage);
   else if (DEVICE)
-    mat_device_block<TEXT>(d, nd, c, first_device, link, ctx, rows, len, sc, blockIdx.x - generic_blocks, gridDim.x - generic_blocks, stage);
+    mat_device_block<TEXT>(d, nd, c, first_device, link, clk, ctx, rows, len, sc, blockIdx.x - generic_blocks, gridDim.x - generic_blocks, stage);
 }
 /* Collective metadata: the first activity, in emission order, that prints each entry, per
  * backend (first[2k] nccl, first[2k + 1] hccl).  The host replays appendCollectiveMetadata's
@@ -2750,11 +2751,11 @@ k_gather_len(const uint32_t* perm, const uint32_t* len, uint64_t n, uint32_t* le
 
 #define MAT_ONE_LAUNCH_ROWS 262144u
 hipError_t mat_rows(const ktj_generic_rec* g, uint64_t ng, uint64_t first_generic, const uint32_t* sync_first, const ktj_device_rec* d, uint64_t nd,
-                    Columns c, uint64_t first_device, const DevLink* link, EmitCtx ctx, Rows rows, uint32_t* len, Scalars* sc, hipStream_t st) {
+                    Columns c, uint64_t first_device, const DevLink* link, const ClockDev& clk, EmitCtx ctx, Rows rows, uint32_t* len, Scalars* sc, hipStream_t st) {
   const unsigned gb = grid_stride_for(ng, KTJ_BLOCK), db = grid_stride_for(nd, KTJ_BLOCK);
   auto launch = [&](auto kernel, unsigned g_blocks, unsigned d_blocks, bool clock) {
     hipLaunchKernelGGL(kernel, dim3(g_blocks + d_blocks), dim3(KTJ_BLOCK), 0, st, g, ng, first_generic, sync_first, g_blocks, d, nd, c, first_device,
-                       link, ctx, rows, len, sc, clock ? 1 : 0);
+                       link, clk, ctx, rows, len, sc, clock ? 1 : 0);
   };
   const bool clock = first_generic == 0;
   if (gb && db && ng + nd < MAT_ONE_LAUNCH_ROWS) {
@@ -2767,7 +2768,7 @@ hipError_t mat_rows(const ktj_generic_rec* g, uint64_t ng, uint64_t first_generi
 }
 
 hipError_t join_runtime_rows(const ktj_runtime_rec* r, uint64_t n, Columns c, uint64_t first, ApiTable api, Table tf, FullCols fc,
-                             Table tn, NarrowCols nc, uint32_t* slot_f, uint32_t* slot_n, EmitCtx ctx, Rows rows,
+                             Table tn, NarrowCols nc, uint32_t* slot_f, uint32_t* slot_n, const ClockDev& clk, EmitCtx ctx, Rows rows,
                              uint32_t* len, Scalars* sc, hipStream_t st) {
   if (n == 0) return hipSuccess;
   /* As many groups per workgroup as let all workgroups run at a time (four per CU, by their registers and LDS), up to JOIN_ROWS:
@@ -2777,7 +2778,7 @@ hipError_t join_runtime_rows(const ktj_runtime_rec* r, uint64_t n, Columns c, ui
   const int rounds = groups <= at_once ? 1 : groups >= at_once * JOIN_ROWS ? JOIN_ROWS : (int)((groups + at_once - 1u) / at_once);
   auto launch = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3(grid_for(n, KTJ_BLOCK * rounds)), dim3(KTJ_BLOCK), 0, st, r, n, c, first, api, tf, fc, tn, nc,
-                       slot_f, slot_n, ctx, rows, len, sc, rounds);
+                       slot_f, slot_n, clk, ctx, rows, len, sc, rounds);
   };
   if (rows.schemas) launch(k_join_runtime<true>); else launch(k_join_runtime<false>);
   return KTJ_LAUNCH_CHECK();

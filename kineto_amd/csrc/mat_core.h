@@ -24,14 +24,17 @@ struct ClockDev {
 };
 
 /* RocprofActivityApi.cpp:166-175: begin and end are converted separately */
+KTJ_HD inline uint64_t convert_time(const ClockDev& c, uint32_t mode, uint64_t t) {
+  if (mode == KTJ_CLOCK_CONVERT) return (uint64_t)convert_timestamp(t, c.t0_approx, c.t0, c.scale_bits);
+  return mode == KTJ_CLOCK_OFFSET ? t + (uint64_t)c.async_offset : t;
+}
 KTJ_HD inline void convert_range(const ClockDev& c, uint32_t mode, uint64_t* begin, uint64_t* end) {
-  if (mode == KTJ_CLOCK_CONVERT) {
-    *begin = (uint64_t)convert_timestamp(*begin, c.t0_approx, c.t0, c.scale_bits);
-    *end = (uint64_t)convert_timestamp(*end, c.t0_approx, c.t0, c.scale_bits);
-  } else if (mode == KTJ_CLOCK_OFFSET) {
-    *begin += (uint64_t)c.async_offset;
-    *end += (uint64_t)c.async_offset;
-  }
+  *begin = convert_time(c, mode, *begin);
+  *end = convert_time(c, mode, *end);
+}
+/* duration() of a runtime or device row whose timestamp() is known: the converted end less that, for every kind (cols_runtime, device_times) */
+KTJ_HD inline int64_t duration_from(const ClockDev& c, uint32_t mode, int64_t ts, uint64_t end) {
+  return (int64_t)(convert_time(c, mode, end) - (uint64_t)ts);
 }
 
 /* The kind of a device row: the low 16 bits of `domain`; kinds this engine does not know are
