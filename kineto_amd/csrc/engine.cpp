@@ -234,7 +234,7 @@ struct ktj_engine {
   /* working buffers */
   DevBuf d_scalars, d_entries, d_name_blob, d_arg_blob;
   DevBuf c_ts, c_dur, c_corr, c_dev, c_res, c_meta, c_ext;
-  DevBuf t_full, t_narrow, t_cpu, f_has_runtime, f_first, f_stream_src, f_pay, n_ext_src, n_kern_src, n_copy_src, n_pay, slot_f, slot_n, dev_link, dev_brief, sync_keys, sync_pos, sync_first;
+  DevBuf t_full, t_narrow, t_cpu, f_has_runtime, f_first, f_stream_src, f_pay, n_ext_src, n_kern_src, n_copy_src, n_pay, slot_f, slot_n, dev_link, dev_queue, sync_keys, sync_pos, sync_first;
   DevBuf q_keys, q_stream, q_amb, dn_hash, dn_first, dn_dev, dn_key, dn_rank, dn_list;
   DevBuf s_dev_k, s_dev_r, s_dev_l, s_res_k, s_res_r, s_res_l;
   DevBuf keys_a, keys_b, vals_a, vals_b, hist, scan_tmp;
@@ -1523,7 +1523,7 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
   NEED(e->n_copy_src, (cap_narrow + 1ull) * 4); NEED(e->n_pay, (cap_narrow + 1ull) * sizeof(NarrowPay));
   NEED(e->slot_f, nr * 4 + 16); NEED(e->slot_n, nr * 4 + 16);
   NEED(e->dev_link, nd * sizeof(DevLink) + 16);
-  NEED(e->dev_brief, nd * sizeof(DevBrief) + 16);
+  NEED(e->dev_queue, nd * 8 + 16);
   NEED(e->q_keys, (KTJ_QUEUE_CAP + 1ull) * 8); NEED(e->q_stream, (KTJ_QUEUE_CAP + 1ull) * 8);
   NEED(e->q_amb, (KTJ_QUEUE_CAP + 1ull) * 4);
   NEED(e->dn_hash, (KTJ_DENSE_CAP + 1ull) * 8); NEED(e->dn_first, (KTJ_DENSE_CAP + 1ull) * 4);
@@ -1595,7 +1595,7 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
     job.whole_pass = true;
     job.text = woven;
     job.schemas_not_taken = e->schemas_not_taken; job.n_cids = (uint32_t)e->cid_names.size();
-    job.brief = e->dev_brief.as<DevBrief>();
+    job.queue = e->dev_queue.as<uint64_t>();
     job.clk = clock_of(e); job.win_start = e->win_start; job.win_end = e->win_end;
     HIPCHK(decode(job, c, ctx, sc, st));
   }
@@ -1622,7 +1622,7 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
   HIPCHK(republish_runtime_rows(r_recs, nr, c, ng, fc, nc, e->slot_f.as<uint32_t>(), e->slot_n.as<uint32_t>(), sc, st));
   unsigned long long* orphans = e->keys_a.as<unsigned long long>(); /* a bit per device row: the sort's words come later */
   HIPCHK(link_device_rows(nd, c, ng + nr, tf, fc, tn, nc, e->dev_link.as<DevLink>(), orphans, sc, st));
-  HIPCHK(backfill_streams(e->dev_brief.as<DevBrief>(), nd, c, ng + nr, tf, fc, orphans, stt, sc, st));
+  HIPCHK(backfill_streams(e->dev_queue.as<uint64_t>(), nd, max_spans != 0, c, ng + nr, tf, fc, orphans, stt, sc, st));
   if (max_spans) {
     const int rc = synthesise_user_spans(e, c, ctx, t_cpu, cpu_row, sc, N);
     if (rc != KTJ_OK) return rc;
@@ -1649,7 +1649,8 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
   }
   /* (settled here: collect_distinct flags what only a host that does not look would get wrong) */
   const bool straight = has_room && n_coll == 0 && max_spans == 0 && !e->stepwise && !(e->flags & KTJ_CREATE_TILE_EMIT) && e->sort_mode != 1;
-  HIPCHK(collect_distinct(c, N, nd, sets, sc, straight, ctx, book, st));
+  const Backfill fill{e->dev_queue.as<uint64_t>(), ng + nr, max_spans ? 0 : nd, stt};
+  HIPCHK(collect_distinct(c, N, nd, fill, sets, sc, straight, ctx, book, st));
   /* The document's activities, but for the tile variant: what the weaver prints, and at most n_left others. */
   auto put_activities = [&](uint64_t n_most, uint64_t n_left, uint64_t at, bool weave = true) -> int {
     if (woven && n_most && weave)

@@ -210,12 +210,13 @@ __device__ __forceinline__ void store_cols(const Columns& c, uint64_t a, const R
   if (c.all) { c.dur[a] = r.dur; c.ext[a] = 0; }
 }
 
+__device__ __forceinline__ uint32_t row_domain(uint32_t meta) { return (meta & KTJ_M_KIND_MASK) >> KTJ_M_KIND_SHIFT; }
 __device__ __forceinline__ bool is_async_op(uint32_t domain) { return domain != KTJ_DOM_MEMSET; }
 
-__device__ __forceinline__ bool dense_key(const DevBrief& d, uint64_t stream, uint64_t* key) {
-  if (!is_async_op(d.domain)) return false;
+__device__ __forceinline__ bool dense_key(uint32_t domain, uint64_t stream, uint64_t queue, uint64_t* key) {
+  if (!is_async_op(domain)) return false;
   if (stream != 0) *key = stream;
-  else if (d.queue != 0) *key = d.queue | (1ULL << 63);
+  else if (queue != 0) *key = queue | (1ULL << 63);
   else return false;
   return true;
 }

@@ -92,12 +92,6 @@ struct DevLink {
   uint32_t flags;          /* KTJ_DL_* */
   uint32_t coll;           /* 1 + index of the collective metadata of the linked CPU op (kernels) */
 };                         /* 32 bytes */
-/* the fields of a device row that the stream back-fill passes read */
-struct DevBrief {
-  uint64_t queue;
-  int32_t device;
-  uint32_t domain;
-};                         /* 16 bytes */
 #define KTJ_DL_HAS_SIZE 1u
 #define KTJ_DL_HAS_GRID 2u
 
@@ -257,7 +251,7 @@ struct DecodeJob {
   bool whole_pass;           /* false: generic records made during the pass, which are in no table */
   bool text;                 /* a pass that makes text rows: those that will be none are counted, as far as their records say so */
   uint32_t schemas_not_taken, n_cids;
-  DevBrief* brief;
+  uint64_t* queue;           /* of the device rows: what they have instead of a stream, and hardly ever read */
   ClockDev clk;
   int64_t win_start, win_end;
   uint32_t gb, rb, db;       /* set by decode() */
@@ -299,7 +293,7 @@ struct StreamTables {
   uint32_t* d_list;   /* KTJ_MAX_STREAM_PAIRS: slots of the pairs */
 };
 /* also checks the device rows whose id no runtime row has (tf, fc, link) */
-hipError_t backfill_streams(const DevBrief* d, uint64_t n, Columns c, uint64_t first_device, Table tf, FullCols fc, const unsigned long long* orphans,
+hipError_t backfill_streams(const uint64_t* queue, uint64_t n, bool assign, Columns c, uint64_t first_device, Table tf, FullCols fc, const unsigned long long* orphans,
                             StreamTables t, Scalars* sc, hipStream_t st);
 
 /* ---- GPU user annotations (GenericActivityProfiler.cpp:277-327, 423-433): one span per
@@ -330,6 +324,8 @@ hipError_t span_members(const ktj_extcorr_rec* u, uint64_t n_device, Columns c, 
                         SpanTables t, SpanMember* out, uint32_t cap_out, uint32_t* n_out, hipStream_t st);
 
 /* ---- stage 3: canonical order ---- */
+/* The device rows whose resourceId the sort still has to make of their streams and queues (k_dense_assign has, where n is 0) */
+struct Backfill { const uint64_t* queue; uint64_t first_device, n; StreamTables t; };
 struct SortSets {
   uint64_t* dev_keys;  /* KTJ_SET_CAP + 1, KTJ_EMPTY_KEY filled */
   uint32_t* dev_rank;
@@ -341,7 +337,7 @@ struct SortSets {
 /* distinct values and their ranks, and Scalars::sort; straight: the host will not look at anything before
  * the end of the pass, so what needs that is flagged (KTJ_DEVERR_CAREFUL).  book, if not null: what text_row and
  * weave_activities need to know of the schemas, from the dictionary views */
-hipError_t collect_distinct(Columns c, uint64_t n, uint64_t n_device, SortSets s, Scalars* sc, bool straight, const EmitCtx& ctx, weave::SchemaBook* book, hipStream_t st);
+hipError_t collect_distinct(Columns c, uint64_t n, uint64_t n_device, const Backfill& fill, SortSets s, Scalars* sc, bool straight, const EmitCtx& ctx, weave::SchemaBook* book, hipStream_t st);
 /* key = ((rank(dev) << res_bits | rank(res)) << ts_bits) | (ts - ts_min); dropped rows get 1 << key_bits */
 hipError_t make_keys(Columns c, uint64_t n, SortSets s, const Scalars* sc, uint32_t ts_bits, uint32_t res_bits,
                      uint32_t key_bits, uint64_t* keys, uint32_t* vals, hipStream_t st);

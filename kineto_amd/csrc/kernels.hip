@@ -496,9 +496,7 @@ __global__ void __launch_bounds__(KTJ_BLOCK) k_decode(DecodeJob J, Columns c, Em
       oor = !(r.meta & KTJ_M_VALID);
       left = J.text && !oor && (weave::left_device(*d, r.ts, r.dur, r.res, ctx) || weave::far_apart(d->begin, l[0].begin));
       store_cols(c, J.ng + J.nr + i, r, true);
-      DevBrief br;
-      br.queue = d->queue; br.device = d->device; br.domain = device_row_domain(d->domain);
-      J.brief[i] = br;
+      J.queue[i] = d->queue;
     }
     block_add_two(sc, KTJ_CNT_OUT_OF_RANGE, oor, KTJ_CNT_NOT_TEXT, left);
     return;
@@ -757,10 +755,10 @@ __global__ void k_link_device(uint64_t n, Columns c, uint64_t first_device, Tabl
  *    stream of the correlation-matched runtime row, is part of k_link_device): which stream every queue
  *    shows, ambiguous when one queue shows two different ones. */
 __global__ void k_after_link(uint64_t n, Columns c, uint64_t first_device, Table tf, FullCols fc, const unsigned long long* orphan_rows,
-                             const DevBrief* d, StreamTables t, Scalars* sc) {
-  const bool orphans = sc->n_device_orphans != 0, queues = sc->have_stream_src != 0 && sc->n_unresolved != 0;
+                             const uint64_t* queues, StreamTables t, Scalars* sc) {
+  const bool orphans = sc->n_device_orphans != 0, by_queue = sc->have_stream_src != 0 && sc->n_unresolved != 0;
   uint32_t n_bad = 0;
-  if (orphans || queues)
+  if (orphans || by_queue)
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) {
       const uint64_t a = first_device + i;
       if (orphans && (orphan_rows[i >> 6] >> (i & 63u) & 1ULL)) {
@@ -771,9 +769,9 @@ __global__ void k_after_link(uint64_t n, Columns c, uint64_t first_device, Table
           if (t2 != 0 && t1 > t2) ++n_bad;
         }
       }
-      if (queues) {
-        const uint64_t stream = (uint64_t)c.res[a], queue = d[i].queue;
-        if (is_async_op(d[i].domain) && stream != 0 && queue != 0) {
+      if (by_queue) {
+        const uint64_t stream = (uint64_t)c.res[a], queue = queues[i];
+        if (is_async_op(row_domain(c.meta[a])) && stream != 0 && queue != 0) {
           const uint32_t slot = table_insert_counted(t.q_keys, KTJ_QUEUE_CAP - 1u, queue, &sc->n_queues, KTJ_MAX_QUEUES);
           if (slot == KTJ_NOSLOT) flag_error(sc, KTJ_DEVERR_QUEUES);
           else {
@@ -976,7 +974,7 @@ __device__ __forceinline__ void dense_enter(StreamTables& t, uint64_t h, uint32_
   }
 }
 __global__ void __launch_bounds__(KTJ_BLOCK)
-k_dense_first(const DevBrief* d, uint64_t n, uint64_t per, Columns c, uint64_t first_device, StreamTables t, Scalars* sc) {
+k_dense_first(const uint64_t* queues, uint64_t n, uint64_t per, Columns c, uint64_t first_device, StreamTables t, Scalars* sc) {
   __shared__ unsigned long long l_key[DENSE_LOCAL_SLOTS];
   __shared__ unsigned long long l_pair_key[DENSE_LOCAL_SLOTS];
   __shared__ int32_t l_pair_dev[DENSE_LOCAL_SLOTS];
@@ -987,25 +985,32 @@ k_dense_first(const DevBrief* d, uint64_t n, uint64_t per, Columns c, uint64_t f
   __syncthreads();
   const uint64_t lo = blockIdx.x * per, hi = n < lo + per ? n : lo + per;
   for (uint64_t i0 = lo + threadIdx.x; i0 < hi; i0 += KTJ_BLOCK * DENSE_ROWS) {
-    DevBrief row[DENSE_ROWS];
-    uint64_t row_stream[DENSE_ROWS];
+    uint32_t row_meta[DENSE_ROWS];
+    int64_t row_dev[DENSE_ROWS];
+    uint64_t row_stream[DENSE_ROWS], row_queue[DENSE_ROWS];
 #pragma unroll
     for (uint32_t r = 0; r < DENSE_ROWS; ++r) { /* all loads of the group in flight together */
       const uint64_t i = i0 + r * KTJ_BLOCK;
-      if (i < hi) { row[r] = d[i]; row_stream[r] = (uint64_t)c.res[first_device + i]; }
+      if (i < hi) { row_meta[r] = c.meta[first_device + i]; row_dev[r] = c.dev[first_device + i]; row_stream[r] = (uint64_t)c.res[first_device + i]; }
+    }
+#pragma unroll
+    for (uint32_t r = 0; r < DENSE_ROWS; ++r) {
+      const uint64_t i = i0 + r * KTJ_BLOCK;
+      row_queue[r] = i < hi && row_stream[r] == 0 ? queues[i] : 0;
     }
 #pragma unroll
     for (uint32_t r = 0; r < DENSE_ROWS; ++r) {
       const uint64_t i = i0 + r * KTJ_BLOCK;
       if (i >= hi) break;
       uint64_t key, stream = row_stream[r];
-      const DevBrief b = row[r];
-      if (fill && stream == 0 && is_async_op(b.domain)) {
-        const uint32_t slot = table_find(t.q_keys, KTJ_QUEUE_CAP - 1u, b.queue);
+      const uint32_t domain = row_domain(row_meta[r]);
+      const int32_t device = (int32_t)row_dev[r];
+      if (fill && stream == 0 && is_async_op(domain)) {
+        const uint32_t slot = table_find(t.q_keys, KTJ_QUEUE_CAP - 1u, row_queue[r]);
         if (slot != KTJ_NOSLOT && t.q_amb[slot] == 0 && t.q_stream[slot] != 0) { stream = t.q_stream[slot]; c.res[first_device + i] = (int64_t)stream; }
       }
-      if (!dense_key(b, stream, &key)) continue;
-      const uint64_t h = dense_hash(b.device, key);
+      if (!dense_key(domain, stream, row_queue[r], &key)) continue;
+      const uint64_t h = dense_hash(device, key);
       uint32_t slot = (uint32_t)(h >> 20) & (DENSE_LOCAL_SLOTS - 1u);
       bool placed = false;
       for (uint32_t probe = 0; probe < 16 && !placed; ++probe) {
@@ -1013,12 +1018,12 @@ k_dense_first(const DevBrief* d, uint64_t n, uint64_t per, Columns c, uint64_t f
         if (cur == KTJ_EMPTY_KEY) {
           cur = atomicCAS(&l_key[slot], (unsigned long long)KTJ_EMPTY_KEY, (unsigned long long)h);
           /* the pair itself, for the table entry: every row of the pair would write the same two values */
-          if (cur == KTJ_EMPTY_KEY) { l_pair_dev[slot] = b.device; l_pair_key[slot] = key; }
+          if (cur == KTJ_EMPTY_KEY) { l_pair_dev[slot] = device; l_pair_key[slot] = key; }
         }
         if (cur == KTJ_EMPTY_KEY || cur == h) { if (l_min[slot] > (uint32_t)i) atomicMin(&l_min[slot], (uint32_t)i); placed = true; }
         else slot = (slot + 1u) & (DENSE_LOCAL_SLOTS - 1u);
       }
-      if (!placed) dense_enter(t, h, (uint32_t)i, b.device, key, sc); /* local table crowded: straight to the global one */
+      if (!placed) dense_enter(t, h, (uint32_t)i, device, key, sc); /* local table crowded: straight to the global one */
     }
   }
   __syncthreads();
@@ -1045,40 +1050,39 @@ k_dense_first(const DevBrief* d, uint64_t n, uint64_t per, Columns c, uint64_t f
     if (p < m) t.d_rank[s] = rank;
   }
 }
-/* pass 3c: resourceId() = stream != 0 ? stream : queue (RocprofActivity.h:100-102) */
-__global__ void k_dense_assign(const DevBrief* d, uint64_t n, Columns c, uint64_t first_device, StreamTables t,
+/* pass 3c: resourceId() = stream != 0 ? stream : queue (RocprofActivity.h:100-102).  Part of k_collect_distinct, which reads the same
+ * columns, but where the spans of user annotations ask for it before. */
+__device__ __forceinline__ uint32_t dense_number(const StreamTables& t, int32_t device, uint64_t key, Scalars* sc) {
+  const uint32_t slot = table_find(t.d_hash, KTJ_DENSE_CAP - 1u, dense_hash(device, key));
+  if (slot == KTJ_NOSLOT || t.d_dev[slot] != device || t.d_key[slot] != key) { flag_error(sc, KTJ_DEVERR_HASH_COLLISION); return 0; }
+  return t.d_rank[slot];
+}
+__global__ void k_dense_assign(const uint64_t* queues, uint64_t n, Columns c, uint64_t first_device, StreamTables t,
                                Scalars* sc) {
   const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const uint64_t a = first_device + i;
-  const DevBrief b = d[i];
-  if (!is_async_op(b.domain)) return;
-  uint64_t stream = (uint64_t)c.res[a];
-  if (sc->have_stream_src != 0) {
-    uint64_t key;
-    if (dense_key(b, stream, &key)) {
-      const uint32_t slot = table_find(t.d_hash, KTJ_DENSE_CAP - 1u, dense_hash(b.device, key));
-      if (slot == KTJ_NOSLOT || t.d_dev[slot] != b.device || t.d_key[slot] != key) {
-        flag_error(sc, KTJ_DEVERR_HASH_COLLISION);
-      } else stream = t.d_rank[slot];
-    }
-  }
-  c.res[a] = (int64_t)(stream != 0 ? stream : b.queue);
+  const uint32_t domain = row_domain(c.meta[a]);
+  if (!is_async_op(domain)) return;
+  uint64_t stream = (uint64_t)c.res[a], key;
+  const uint64_t queue = stream == 0 ? queues[i] : 0;
+  if (sc->have_stream_src != 0 && dense_key(domain, stream, queue, &key)) stream = dense_number(t, (int32_t)c.dev[a], key, sc);
+  c.res[a] = (int64_t)(stream != 0 ? stream : queue);
 }
 
-hipError_t backfill_streams(const DevBrief* d, uint64_t n, Columns c, uint64_t first_device, Table tf, FullCols fc, const unsigned long long* orphans,
+hipError_t backfill_streams(const uint64_t* queue, uint64_t n, bool assign, Columns c, uint64_t first_device, Table tf, FullCols fc, const unsigned long long* orphans,
                             StreamTables t, Scalars* sc, hipStream_t st) {
   if (n == 0) return hipSuccess;
   const dim3 g(grid_for(n, KTJ_BLOCK)), b(KTJ_BLOCK);
-  hipLaunchKernelGGL(k_after_link, dim3(grid_stride_for(n, KTJ_BLOCK)), b, 0, st, n, c, first_device, tf, fc, orphans, d, t, sc);
+  hipLaunchKernelGGL(k_after_link, dim3(grid_stride_for(n, KTJ_BLOCK)), b, 0, st, n, c, first_device, tf, fc, orphans, queue, t, sc);
   /* every workgroup pays for its local table and for each pair it has seen: 2048 rows each, fewer only while
    * that leaves CUs without a workgroup, and at most four workgroups per CU.  A workgroup's rows lie together, as buffers of a stream
    * mostly do: it sees few of the pairs then (rows a grid apart: 22 million records 85 us instead of 65, 3 million 37 instead of 32). */
   const unsigned few = grid_stride_for(n, KTJ_BLOCK * 2), many = grid_stride_for(n, KTJ_BLOCK * 8);
   const unsigned gd = many > 1024u ? 1024u : many > 256u ? many : few > 256u ? 256u : few;
   const uint64_t per = ((n + gd - 1) / gd + KTJ_BLOCK - 1) / KTJ_BLOCK * KTJ_BLOCK;
-  hipLaunchKernelGGL(k_dense_first, dim3((unsigned)((n + per - 1) / per)), b, 0, st, d, n, per, c, first_device, t, sc);
-  hipLaunchKernelGGL(k_dense_assign, g, b, 0, st, d, n, c, first_device, t, sc);
+  hipLaunchKernelGGL(k_dense_first, dim3((unsigned)((n + per - 1) / per)), b, 0, st, queue, n, per, c, first_device, t, sc);
+  if (assign) hipLaunchKernelGGL(k_dense_assign, g, b, 0, st, queue, n, c, first_device, t, sc);
   return KTJ_LAUNCH_CHECK();
 }
 
@@ -1210,9 +1214,34 @@ __device__ void lay_out_schemas(const EmitCtx& c, weave::SchemaBook* out, Schema
  * printed.  The workgroup that ends last ranks the values and plans the sort's keys.  With a book the first
  * workgroup lays out the schemas instead of taking rows: this is the longest launch before the size pass that
  * small passes have, too. */
-__global__ void __launch_bounds__(KTJ_BLOCK) k_collect_distinct(Columns c, uint64_t n, uint64_t per, uint64_t n_device, SortSets s, Scalars* sc, int straight, EmitCtx ctx, weave::SchemaBook* book) {
+/* Device rows take the number of their (device, stream) pair on the way, as their columns are read here anyway: a pass of its own
+ * read 24 bytes a row, of them 16 that were made for it only (11 million records 3655 -> 3603 us, 22 million 7850 -> 7806, 30 000
+ * 174 -> 171; 3 million 1169 -> 1161).
+ * What a workgroup has looked up of the numbers; a pair whose places are taken is looked up each time.  A number is
+ * stored behind the pair it belongs to (PAIR_CLAIMED: not yet). */
+#define PAIR_SLOTS 1024u
+#define PAIR_CLAIMED 0xFFFFFFFFu
+struct PairCache { unsigned long long key[PAIR_SLOTS]; int32_t dev[PAIR_SLOTS]; uint32_t number[PAIR_SLOTS]; };
+__device__ __forceinline__ uint32_t pair_number(PairCache& l, const StreamTables& t, int32_t device, uint64_t key, Scalars* sc) {
+  const uint32_t h = ((uint32_t)key ^ ((uint32_t)(key >> 32) * 0x9E3779B1u) ^ ((uint32_t)device * 0xC2B2AE35u)) * 0x85EBCA6Bu;
+  uint32_t slot = h >> 22, free = PAIR_SLOTS; /* 10 bits */
+  for (uint32_t probe = 0; probe < 4u; ++probe) {
+    const uint32_t x = __hip_atomic_load(&l.number[slot], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP);
+    if (x == 0) { free = slot; break; }
+    if (x != PAIR_CLAIMED && l.key[slot] == key && l.dev[slot] == device) return x;
+    slot = (slot + 1u) & (PAIR_SLOTS - 1u);
+  }
+  const uint32_t number = dense_number(t, device, key, sc);
+  if (free != PAIR_SLOTS && number != 0 && atomicCAS(&l.number[free], 0u, PAIR_CLAIMED) == 0u) {
+    l.key[free] = key; l.dev[free] = device;
+    __hip_atomic_store(&l.number[free], number, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+  }
+  return number;
+}
+__global__ void __launch_bounds__(KTJ_BLOCK) k_collect_distinct(Columns c, uint64_t n, uint64_t per, uint64_t n_device, Backfill fill, SortSets s, Scalars* sc, int straight, EmitCtx ctx, weave::SchemaBook* book) {
   __shared__ uint64_t red_min[KTJ_BLOCK >> 6], red_max[KTJ_BLOCK >> 6];
   __shared__ unsigned long long seen[2][LOCAL_SET_SLOTS + 1]; /* deviceId, resourceId values */
+  __shared__ PairCache pairs;
   static_assert(sizeof(SchemaLds) <= sizeof(seen), "laid out where the values would be");
   const uint32_t books = book ? 1u : 0u;
   const bool lays_out = blockIdx.x < books;
@@ -1220,9 +1249,14 @@ __global__ void __launch_bounds__(KTJ_BLOCK) k_collect_distinct(Columns c, uint6
   if (lays_out) {
     if (sc->no_text == 0) lay_out_schemas(ctx, book, reinterpret_cast<SchemaLds*>(seen));
   } else for (uint32_t k = threadIdx.x; k <= LOCAL_SET_SLOTS; k += blockDim.x) { seen[0][k] = KTJ_EMPTY_KEY; seen[1][k] = KTJ_EMPTY_KEY; }
+  for (uint32_t k = threadIdx.x; k < PAIR_SLOTS; k += blockDim.x) pairs.number[k] = 0;
   __syncthreads();
   uint64_t mn = ~0ULL, mx = 0ULL;
   uint64_t last_dev = 0, last_res = 0; /* of the thread's rows so far: most rows repeat them */
+  const bool numbered = sc->have_stream_src != 0;
+  uint64_t pair_key = 0; /* the thread's last pair; 0 is no key */
+  int32_t pair_dev = 0;
+  uint32_t pair_is = 0;
   bool any = false;
   uint32_t n_valid = 0;
   const uint64_t first = lays_out ? n : (blockIdx.x - books) * per, end = n < first + per ? n : first + per;
@@ -1237,6 +1271,39 @@ __global__ void __launch_bounds__(KTJ_BLOCK) k_collect_distinct(Columns c, uint6
       dev[r] = in ? (uint64_t)c.dev[a] : 0;
       res[r] = in ? (uint64_t)c.res[a] : 0;
       ts[r] = in ? (uint64_t)c.ts[a] : 0;
+    }
+    uint32_t ask = 0; /* device rows that take their pair's number: the key stands in res meanwhile */
+    uint64_t queue[COLLECT_ROWS];
+#pragma unroll
+    for (int r = 0; r < COLLECT_ROWS; ++r) {
+      const uint64_t a = a0 + (uint64_t)r * KTJ_BLOCK, i = a - fill.first_device; /* (wraps around in front of them) */
+      const bool device = a < end && a >= fill.first_device && i < fill.n && is_async_op(row_domain(meta[r]));
+      ask |= (device ? 1u : 0u) << r;
+      queue[r] = device && res[r] == 0 ? fill.queue[i] : 0;
+    }
+#pragma unroll
+    for (int r = 0; r < COLLECT_ROWS; ++r) {
+      if (!(ask >> r & 1u)) continue;
+      uint64_t key;
+      if (numbered && dense_key(row_domain(meta[r]), res[r], queue[r], &key)) res[r] = key;
+      else {
+        ask &= ~(1u << r);
+        if (res[r] == 0 && queue[r] != 0) { res[r] = queue[r]; c.res[a0 + (uint64_t)r * KTJ_BLOCK] = (int64_t)queue[r]; }
+      }
+    }
+    while (ask) {
+      const uint32_t at = (uint32_t)__builtin_ctz(ask);
+      ask &= ask - 1u;
+      uint64_t key = res[0], device = dev[0];
+#pragma unroll
+      for (uint32_t r = 1; r < COLLECT_ROWS; ++r) { key = at == r ? res[r] : key; device = at == r ? dev[r] : device; }
+      if (key != pair_key || (int32_t)device != pair_dev) {
+        pair_key = key; pair_dev = (int32_t)device;
+        pair_is = pair_number(pairs, fill.t, pair_dev, key, sc);
+      }
+#pragma unroll
+      for (uint32_t r = 0; r < COLLECT_ROWS; ++r) res[r] = at == r ? (uint64_t)pair_is : res[r];
+      c.res[a0 + (uint64_t)at * KTJ_BLOCK] = (int64_t)pair_is;
     }
     uint32_t todo = 0;
 #pragma unroll
@@ -1430,7 +1497,7 @@ hipError_t make_rank_keys(Columns c, const uint32_t* order, uint64_t n, SortSets
   return KTJ_LAUNCH_CHECK();
 }
 
-hipError_t collect_distinct(Columns c, uint64_t n, uint64_t n_device, SortSets s, Scalars* sc, bool straight, const EmitCtx& ctx, weave::SchemaBook* book, hipStream_t st) {
+hipError_t collect_distinct(Columns c, uint64_t n, uint64_t n_device, const Backfill& fill, SortSets s, Scalars* sc, bool straight, const EmitCtx& ctx, weave::SchemaBook* book, hipStream_t st) {
   if (n == 0) return hipSuccess;
   /* few, fat workgroups: each one pays for its own local set once (few rows: one group each) */
   /* at most four workgroups per CU: every workgroup pays for its local sets and its atomics at the
@@ -1440,7 +1507,7 @@ hipError_t collect_distinct(Columns c, uint64_t n, uint64_t n_device, SortSets s
   if (g > 1024u) g = 1024u;
   /* (a workgroup's rows lie together and have few values, as above: 733 000 records 34 -> 28 us, 22 million 151 -> 141) */
   const uint64_t per = ((n + g - 1) / g + KTJ_BLOCK - 1) / KTJ_BLOCK * KTJ_BLOCK;
-  hipLaunchKernelGGL(k_collect_distinct, dim3((unsigned)((n + per - 1) / per) + (book ? 1u : 0u)), dim3(KTJ_BLOCK), 0, st, c, n, per, n_device, s, sc, straight ? 1 : 0, ctx, book);
+  hipLaunchKernelGGL(k_collect_distinct, dim3((unsigned)((n + per - 1) / per) + (book ? 1u : 0u)), dim3(KTJ_BLOCK), 0, st, c, n, per, n_device, fill, s, sc, straight ? 1 : 0, ctx, book);
   return KTJ_LAUNCH_CHECK();
 }
 hipError_t make_keys(Columns c, uint64_t n, SortSets s, const Scalars* sc, uint32_t ts_bits, uint32_t res_bits,

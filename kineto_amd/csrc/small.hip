@@ -276,18 +276,17 @@ __global__ void __launch_bounds__(SMALL_JOIN_THREADS) k_small_join(SmallArgs A) 
       const uint32_t i = tid + k * SMALL_JOIN_THREADS;
       p_slot[k] = KTJ_NOSLOT;
       if (i >= nd) continue;
-      DevBrief b;
-      b.queue = A.d[i].queue; b.device = (int32_t)dv[k].dev; b.domain = (dv[k].meta & KTJ_M_KIND_MASK) >> KTJ_M_KIND_SHIFT;
+      const int32_t device = (int32_t)dv[k].dev;
       uint64_t key;
-      if (!dense_key(b, (uint64_t)dv[k].res, &key)) continue;
+      if (!dense_key((dv[k].meta & KTJ_M_KIND_MASK) >> KTJ_M_KIND_SHIFT, (uint64_t)dv[k].res, A.d[i].queue, &key)) continue;
       /* a pair is equal when device and key are: 0 and not the key tells a row of another device apart */
       auto same = [&](uint32_t e) -> uint64_t {
         const ktj_device_rec& o = A.d[e - 1u];
-        if (o.device != b.device) return ~key;
+        if (o.device != device) return ~key;
         const uint64_t res = (uint64_t)c.res[ng + nr + e - 1u];
         return res != 0 ? res : o.queue | (1ULL << 63);
       };
-      p_slot[k] = lds_insert(t_full, mask, pair_hash(b.device, key), key, i + 1u, same);
+      p_slot[k] = lds_insert(t_full, mask, pair_hash(device, key), key, i + 1u, same);
       atomicMin(&n_ext[p_slot[k]], i);
     }
     __syncthreads();
