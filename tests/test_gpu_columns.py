@@ -63,3 +63,17 @@ def test_clocks(runtime_mode, device_mode, spans):
         eng.process()
         assert eng.output() == want
     ora.close()
+
+
+@pytest.mark.parametrize("rows", (140000, 524288, 524289))
+def test_joined_rows_in_one_launch_and_in_two(rows):
+    """Generic and device records together below, at and behind the million up to which one launch makes both."""
+    print(rows, flush=True)
+    sp, release = abi.synth_stream(2, rows, host_name="columns")
+    ora = og.OracleRun(sp)
+    with TraceEngine(sp.contents.trace_name.decode()) as eng:
+        eng.submit_stream(sp)
+        eng.process()
+        assert eng.output() == ora.output()
+    ora.close()
+    release()
