@@ -1077,7 +1077,8 @@ hipError_t backfill_streams(const uint64_t* queue, uint64_t n, bool assign, Colu
   hipLaunchKernelGGL(k_after_link, dim3(grid_stride_for(n, KTJ_BLOCK)), b, 0, st, n, c, first_device, tf, fc, orphans, queue, t, sc);
   /* every workgroup pays for its local table and for each pair it has seen: 2048 rows each, fewer only while
    * that leaves CUs without a workgroup, and at most four workgroups per CU.  A workgroup's rows lie together, as buffers of a stream
-   * mostly do: it sees few of the pairs then (rows a grid apart: 22 million records 85 us instead of 65, 3 million 37 instead of 32). */
+   * mostly do: it sees few of the pairs then (rows a grid apart: 22 million records 85 us instead of 65, 3 million 37 instead of 32; 58 and 33 with
+   * columns of 20 bytes a row instead of 24). */
   const unsigned few = grid_stride_for(n, KTJ_BLOCK * 2), many = grid_stride_for(n, KTJ_BLOCK * 8);
   const unsigned gd = many > 1024u ? 1024u : many > 256u ? many : few > 256u ? 256u : few;
   const uint64_t per = ((n + gd - 1) / gd + KTJ_BLOCK - 1) / KTJ_BLOCK * KTJ_BLOCK;
@@ -1505,7 +1506,8 @@ hipError_t collect_distinct(Columns c, uint64_t n, uint64_t n_device, const Back
    * 1024: 0.17 ms) */
   unsigned g = grid_stride_for(n, n < (1u << 20) ? KTJ_BLOCK * COLLECT_ROWS : KTJ_BLOCK * 16);
   if (g > 1024u) g = 1024u;
-  /* (a workgroup's rows lie together and have few values, as above: 733 000 records 34 -> 28 us, 22 million 151 -> 141) */
+  /* (a workgroup's rows lie together and have few values, as above: 733 000 records 34 -> 28 us, 22 million 151 -> 141; 32 and 168 since
+   * device rows take their numbers here, 66 in a launch of its own for 22 million) */
   const uint64_t per = ((n + g - 1) / g + KTJ_BLOCK - 1) / KTJ_BLOCK * KTJ_BLOCK;
   hipLaunchKernelGGL(k_collect_distinct, dim3((unsigned)((n + per - 1) / per) + (book ? 1u : 0u)), dim3(KTJ_BLOCK), 0, st, c, n, per, n_device, fill, s, sc, straight ? 1 : 0, ctx, book);
   return KTJ_LAUNCH_CHECK();
