@@ -2052,7 +2052,9 @@ k_sortp_finish(const uint64_t* buf_a, const uint64_t* buf_b, uint32_t* perm, uin
   __shared__ uint32_t s_val[SPAN];
   __shared__ uint64_t s_edge[CHUNKS], s_start[CHUNKS]; /* a chunk's last word; a bit per row: first of its group */
   const SortRun run = sort_run(sc, 1);
-  if (sc->error != 0 || run.low == 0) return; /* the last pass has written the permutation */
+  /* (low of 0: the last pass has written the permutation.)  All wavefronts of a workgroup must see the same here, as they number
+   * groups and compare rows for each other: the one bit that this launch sets does not count. */
+  if ((sc->error & ~KTJ_DEVERR_UNSORTED) != 0 || run.low == 0) return;
   const uint64_t* in = run.passes & 1u ? buf_b : buf_a;
   const uint32_t group_shift = idx_bits + run.low, lane = lane_id(), wave = threadIdx.x >> 6;
   const uint64_t idx_mask = (1ULL << idx_bits) - 1ULL;

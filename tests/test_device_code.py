@@ -44,3 +44,15 @@ def test_document_parts_are_stored_before_they_are_announced(tmp_path):
             barriers += 1
             assert not waiting, "a barrier behind stores that nothing has waited for"
     assert barriers and stores
+
+
+@pytest.mark.parametrize("rows", (1, 4, 16))
+def test_the_bit_that_the_sorts_last_launch_sets_does_not_end_its_own_wavefronts(tmp_path, rows):
+    """Every wavefront of k_sortp_finish looks for itself whether the pass goes on, and moves rows for the others of its workgroup:
+    KTJ_DEVERR_UNSORTED, which workgroups of this very launch set, is taken out of the word that the wavefront has read."""
+    for text in instructions(tmp_path, "k_sortp_finishILi256ELi%dEE" % rows):
+        if text.startswith("s_barrier"):
+            pytest.fail("the word decides as it is")
+        if re.match(r"s_bitset0_b32 s\d+, 10$", text) or (re.match(r"[sv]_and_b32", text) and "0x%x" % (0xFFFFFFFF & ~1024) in text):
+            return
+    pytest.fail("neither the word nor a barrier")

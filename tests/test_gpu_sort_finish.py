@@ -94,3 +94,10 @@ def test_dropped_rows_and_random_order():
         same_as_oracle(ops(np.full(n, B + 77), 5 + rng.integers(0, 4, n)))                # one time
         far = np.where(np.arange(n) == n // 2, 1000, ts)                                  # a row at the clock's beginning
         same_as_oracle(ops(far, 5 + rng.integers(0, 4, n)))
+
+
+@pytest.mark.parametrize("n", (90001, 600011, 2400001))
+def test_long_groups_in_many_workgroups(n):
+    """Workgroups that start when others have found a group that is too long and not in order: tiles of every size."""
+    print(n, flush=True)
+    same_as_oracle(ops(*groups(n, 400, "shuffled")))
