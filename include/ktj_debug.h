@@ -28,8 +28,10 @@ enum {
   KTJ_DBG_NAME_OFF = 12,  /* uint64[n_strings+1]                                */
   KTJ_DBG_ARG_VIEW = 13,
   KTJ_DBG_ARG_OFF = 14,
-  KTJ_DBG_PASS = 15       /* uint64[4]  of the last pass that was no small one: it made text rows; none of them, as it left
+  KTJ_DBG_PASS = 15,      /* uint64[4]  of the last pass that was no small one: it made text rows; none of them, as it left
                              too many; activities that the weaver left; these had a wait of their own */
+  KTJ_DBG_SORT = 16       /* uint64[2]  of the last pass: bits of the key that the sort's passes left to the launch behind
+                             them; it found rows that it leaves, and the passes were made again over all bits */
 };
 
 /* Copies the array to dst (at most cap bytes) and reports its full size.  Valid after

@@ -242,6 +242,7 @@ struct ktj_engine {
   uint64_t not_woven = 0;                  /* number of these records with which a woven pass left too many activities (too_many_left) */
   int some_left = -1;                      /* the last woven pass had activities that the weaver leaves to emit_direct (1, 0; -1: there was none) */
   uint64_t pass_info[4] = {};              /* of the last pass (KTJ_DBG_PASS) */
+  uint64_t sort_info[2] = {};              /* and KTJ_DBG_SORT */
   DevBuf mat, schema_book, wide_text, len, len_sorted, kind_sorted, offs, out, tile_start;
   void* pinned_small = nullptr; size_t pinned_small_cap = 0;
   HostCtl* h_ctl = nullptr;                  /* pinned: what the device hands back during a pass */
@@ -1480,6 +1481,7 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
   }
   { const int rc = put_pending_pieces(e); if (rc != KTJ_OK) return rc; }
   e->last_end_time = end_time_ns;
+  e->sort_info[0] = e->sort_info[1] = 0;
   e->small_last = false;
   e->rows_are_text = false;
   if (!e->small_unfit && !e->no_small && nu == 0 && n_coll == 0 && small_fits(ng, nr, nd, nx) && !sort_packed_passes_forced() &&
@@ -1715,12 +1717,15 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
       HIPCHK(e->out.ensure(e->total_bytes + 64));
       HIPCHK(fill_u32(&sc->n_left, 0, 1, st)); /* the list is made anew */
     }
-    if (emitted) e->sort_passes = sort_packed_passes(e->scalars.sort, !e->sort_all_bits);
+    if (emitted) {
+      e->sort_passes = sort_packed_passes(e->scalars.sort, !e->sort_all_bits);
+      if (!e->sort_all_bits && !sort_packed_in_one_launch(N)) e->sort_info[0] = e->scalars.sort.low_bits;
+    }
     else if (e->scalars.error & ~(KTJ_DEVERR_CAREFUL | KTJ_DEVERR_UNSORTED | KTJ_DEVERR_DISTINCT_DEVICES | KTJ_DEVERR_DISTINCT_RESOURCES)) {
       e->last_error = limit_text(e->scalars.error);
       return KTJ_ERR_LIMIT;
     } else {
-      if (e->scalars.error == KTJ_DEVERR_UNSORTED) { e->sort_all_bits = true; e->sort_passes = sort_packed_passes(e->scalars.sort, false); }
+      if (e->scalars.error == KTJ_DEVERR_UNSORTED) { e->sort_all_bits = true; e->sort_info[1] = 1; e->sort_passes = sort_packed_passes(e->scalars.sort, false); }
       else e->stepwise = true;
       HIPCHK(clear_error_bits(sc, KTJ_DEVERR_CAREFUL | KTJ_DEVERR_UNSORTED, st));
     }
@@ -2205,9 +2210,10 @@ int ktj_debug_copy_reference(ktj_engine* e, uint64_t n_bytes, float* ms) {
 int ktj_debug_fetch(ktj_engine* e, int what, void* dst, uint64_t cap, uint64_t* n_bytes) {
   if (!e || !n_bytes) return KTJ_ERR_ARG;
   if (!e->processed) return KTJ_ERR_STATE;
-  if (what == KTJ_DBG_PASS) { /* (says what the last pass did: makes none) */
-    *n_bytes = sizeof e->pass_info;
-    if (dst) memcpy(dst, e->pass_info, std::min<uint64_t>(*n_bytes, cap));
+  if (what == KTJ_DBG_PASS || what == KTJ_DBG_SORT) { /* (say what the last pass did: make none) */
+    const void* info = what == KTJ_DBG_PASS ? e->pass_info : e->sort_info;
+    *n_bytes = what == KTJ_DBG_PASS ? sizeof e->pass_info : sizeof e->sort_info;
+    if (dst) memcpy(dst, info, std::min<uint64_t>(*n_bytes, cap));
     return KTJ_OK;
   }
   const bool as_text = what == KTJ_DBG_MAT && e->rows_are_text;

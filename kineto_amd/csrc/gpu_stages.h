@@ -353,6 +353,7 @@ hipError_t clear_error_bits(Scalars* sc, unsigned int bits, hipStream_t st);
  * arrival index per sorted position.  Usable when sort_packed_fits(n, plan). */
 bool sort_packed_fits(uint64_t n, const SortPlan& plan);
 bool sort_packed_passes_forced();
+bool sort_packed_in_one_launch(uint64_t n); /* which has no use for finish */
 void sort_packed_force_passes(bool on); /* tests: no one-launch sort of a single tile */
 uint32_t sort_packed_passes(const SortPlan& plan, bool finish); /* finish: the lowest bits are left to a launch behind the passes */
 /* key widths come from Scalars::sort; `passes` is how many are launched: those beyond the plan end at once, and

@@ -2291,6 +2291,7 @@ static hipError_t sort_packed_chain(Columns c, uint64_t n, SortSets s, Scalars* 
 static bool g_sortp_no_single = false;
 void sort_packed_force_passes(bool on) { g_sortp_no_single = on; }
 bool sort_packed_passes_forced() { return g_sortp_no_single; }
+bool sort_packed_in_one_launch(uint64_t n) { return n <= (uint64_t)SORTP_THREADS * 16u && !g_sortp_no_single; }
 static uint32_t sort_idx_bits(uint64_t n) { return (uint32_t)(64 - __builtin_clzll(n > 1 ? n - 1 : 1)); }
 bool sort_packed_fits(uint64_t n, const SortPlan& plan) {
   return plan.key_bits <= 62u && (plan.key_bits > SORTP_BITS ? plan.key_bits - SORTP_BITS : 0u) + sort_idx_bits(n) <= 64u;
@@ -2303,7 +2304,7 @@ hipError_t sort_packed(Columns c, uint64_t n, SortSets s, Scalars* sc, uint32_t 
                        uint32_t* hist, uint32_t* chain_hist, hipStream_t st) {
   if (n == 0) return hipSuccess;
   const uint32_t idx_bits = sort_idx_bits(n);
-  if (n <= (uint64_t)SORTP_THREADS * 16u && !g_sortp_no_single) {
+  if (sort_packed_in_one_launch(n)) {
     hipLaunchKernelGGL((k_sortp_single<SORTP_BITS, 1024, 4>), dim3(1), dim3(1024), 0, st, c, (uint32_t)n, s, sc, perm);
     return KTJ_LAUNCH_CHECK();
   }

@@ -11,10 +11,10 @@ import numpy as np
 from . import abi
 
 DBG = dict(ts=0, dur=1, dev=2, res=3, meta=4, ext=5, perm=6, len=7, offs=8, mat=9, sort_keys=10,
-           name_view=11, name_off=12, arg_view=13, arg_off=14, pass_info=15)
+           name_view=11, name_off=12, arg_view=13, arg_off=14, pass_info=15, sort_info=16)
 _DBG_DTYPE = dict(ts=np.int64, dur=np.int64, dev=np.int64, res=np.int64, meta=np.uint32, ext=np.int32,
                   perm=np.uint32, len=np.uint32, offs=np.uint64, mat=np.uint8, sort_keys=np.uint64,
-                  name_view=np.uint8, name_off=np.uint64, arg_view=np.uint8, arg_off=np.uint64, pass_info=np.uint64)
+                  name_view=np.uint8, name_off=np.uint64, arg_view=np.uint8, arg_off=np.uint64, pass_info=np.uint64, sort_info=np.uint64)
 
 
 _new_bytes = C.pythonapi.PyBytes_FromStringAndSize

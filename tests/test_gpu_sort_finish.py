@@ -38,14 +38,25 @@ def ops(ts, tid, window=None):
 
 
 def same_as_oracle(sp):
+    """What the passes say of the sort: bits left to the launch behind its passes, and whether these were made again (KTJ_DBG_SORT)."""
     ora = og.OracleRun(sp)
     want = ora.output()
+    info = []
     with TraceEngine(sp.contents.trace_name.decode()) as eng:
         eng.submit_stream(sp)
         for turn in range(2):   # the second one knows how many passes there are
             eng.process()
             assert eng.output() == want, turn
+            info.append([int(x) for x in eng.debug("sort_info")])
     ora.close()
+    return info
+
+
+def left_to_the_last_launch(info):
+    assert info[0][0] > 0 and info == 2 * [[info[0][0], 0]]
+
+
+ALL_BITS = [[0, 1], [0, 0]]   # in the second turn from the start
 
 
 def groups(n, size, order, threads=3, seed=1):
@@ -69,19 +80,35 @@ def groups(n, size, order, threads=3, seed=1):
 def test_groups(size, order):
     """257 rows and more, not in order: all bits by passes."""
     print(size, order, flush=True)
-    same_as_oracle(ops(*groups(9001, size, order)))
+    info = same_as_oracle(ops(*groups(9001, size, order)))
+    if size > 256 and order != "forwards":
+        assert info == ALL_BITS
+    else:
+        left_to_the_last_launch(info)
 
 
 @pytest.mark.parametrize("n", (4097, 8191, 98304, 98305, 262144 + 7))
 def test_sizes(n):
     """One launch a pass, tiles of 512 and tiles behind them, whole and with a few rows."""
     print(n, flush=True)
-    same_as_oracle(ops(*groups(n, 256, "backwards", threads=2)))
+    left_to_the_last_launch(same_as_oracle(ops(*groups(n, 256, "backwards", threads=2))))
 
 
 def test_large_tiles():
     ts, tid = groups(1200001, 97, "shuffled", threads=5)
-    same_as_oracle(ops(ts, tid))
+    left_to_the_last_launch(same_as_oracle(ops(ts, tid)))
+
+
+@pytest.mark.parametrize("size, order", ((255, "backwards"), (256, "shuffled"), (256, "halves"), (257, "forwards"), (257, "halves"), (257, "backwards")))
+@pytest.mark.parametrize("n", (98305, 1200001))
+def test_longest_groups_in_large_tiles(n, size, order):
+    """The longest groups that are put into order, and the shortest that are not, with tiles of 1024 rows and of 4096."""
+    print(n, size, order, flush=True)
+    info = same_as_oracle(ops(*groups(n, size, order)))
+    if size > 256 and order != "forwards":
+        assert info == ALL_BITS
+    else:
+        left_to_the_last_launch(info)
 
 
 def test_dropped_rows_and_random_order():
@@ -100,4 +127,4 @@ def test_dropped_rows_and_random_order():
 def test_long_groups_in_many_workgroups(n):
     """Workgroups that start when others have found a group that is too long and not in order: tiles of every size."""
     print(n, flush=True)
-    same_as_oracle(ops(*groups(n, 400, "shuffled")))
+    assert same_as_oracle(ops(*groups(n, 400, "shuffled"))) == ALL_BITS
