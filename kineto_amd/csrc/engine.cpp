@@ -273,17 +273,21 @@ struct ktj_engine {
 
   bool small_unfit = false;  /* these records need the launches of a large trace (Scalars::error of a small pass) */
   bool stepwise = false;     /* these records need a pass in which the host looks at the plan of the sort (KTJ_DEVERR_CAREFUL) */
-  bool sort_all_bits = false; /* by passes: their order of arrival is not that of their times where many are close together */
+  /* Not 0: all bits by passes, as the order of arrival is not that of the times where many are close together.  To find that out costs a
+   * second sort and a wait (KTJ_DEVERR_UNSORTED; 10 000 rows 160 instead of 100 us, 2 million 930 instead of 750), and the next records of a
+   * producer mostly come as these did: it is tried again for the 16th of them. */
+  uint32_t sort_all_bits = 0;
   uint32_t sort_passes = 0;  /* what these records took in the pass before, where there was one */
   uint32_t sort_passes_most = 0; /* of others before them */
   void other_records() {
-    small_unfit = stepwise = no_room_for_text = sort_all_bits = false; not_woven = 0;
+    small_unfit = stepwise = no_room_for_text = false; not_woven = 0;
+    if (sort_all_bits && sort_passes) --sort_all_bits; /* (there was a pass since) */
     sort_passes_most = std::max(sort_passes_most, sort_passes); sort_passes = 0;
   }
   /* Six passes sort the records of one capture: 2^38 ns, four and a half minutes, beside 9 bits of devices and rows; four
    * do where the lowest sixteen of these 48 bits need none, as the word has room for them beside the index and the rows lie far enough apart.  A
    * pass more than needed costs its three launches, a pass too few the launches behind the sort. */
-  uint32_t passes_to_launch(uint64_t n) const { return sort_passes ? sort_passes : std::max(sort_passes_most, n <= 65536u ? 4u : 6u); }
+  uint32_t passes_to_launch(uint64_t n) const { return sort_passes ? sort_passes : std::max(sort_passes_most, n <= 65536u && !sort_all_bits ? 4u : 6u); }
   bool small_last = false;   /* the last pass was a small one: it leaves no intermediate arrays for ktj_debug_fetch */
   bool no_small = false;     /* ktj_debug_fetch makes them */
   bool no_weave = false;     /* joined rows as they are: ktj_debug_fetch */
@@ -1678,7 +1682,8 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
     if (out_device) e->out.borrow(out_device, out_cap);
     e->perm = e->vals_a.as<uint32_t>();
     e->sorted_keys = nullptr;
-    HIPCHK(sort_packed(c, N, sets, sc, e->passes_to_launch(N), !e->sort_all_bits, e->keys_a.as<uint64_t>(), e->keys_b.as<uint64_t>(), e->perm, e->hist.as<uint32_t>(), e->offs.as<uint32_t>(), st));
+    auto sort = [&]() { return sort_packed(c, N, sets, sc, e->passes_to_launch(N), !e->sort_all_bits, e->keys_a.as<uint64_t>(), e->keys_b.as<uint64_t>(), e->perm, e->hist.as<uint32_t>(), e->offs.as<uint32_t>(), st); };
+    HIPCHK(sort());
     HIPCHK(mat_rows(g_recs, ng, 0, nullptr, d_recs, nd, c, ng + nr, e->dev_link.as<DevLink>(), clock_of(e), ctx, rows, e->len.as<uint32_t>(), sc, st));
     for (;;) {
       text.out = e->out.as<char>(); text.out_cap = e->out.cap;
@@ -1697,6 +1702,13 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
       HIPCHK(hipEventRecord(e->ev[EV_EMIT], st));
       HIPCHK(hipStreamSynchronize(st));
       e->scalars = e->h_ctl->scalars;
+      if (e->scalars.error == KTJ_DEVERR_UNSORTED) { /* the rows are made: what needs their order comes again, with passes over all bits */
+        e->sort_all_bits = 16; e->sort_info[1] = 1;
+        e->sort_passes = sort_packed_passes(e->scalars.sort, false);
+        HIPCHK(clear_error_bits(sc, KTJ_DEVERR_UNSORTED, st));
+        HIPCHK(sort());
+        continue;
+      }
       if (e->scalars.error) break;
       e->act_bytes = e->h_ctl->act_bytes;
       e->prefix_len = prefix.size();
@@ -1721,13 +1733,12 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
       e->sort_passes = sort_packed_passes(e->scalars.sort, !e->sort_all_bits);
       if (!e->sort_all_bits && !sort_packed_in_one_launch(N)) e->sort_info[0] = e->scalars.sort.low_bits;
     }
-    else if (e->scalars.error & ~(KTJ_DEVERR_CAREFUL | KTJ_DEVERR_UNSORTED | KTJ_DEVERR_DISTINCT_DEVICES | KTJ_DEVERR_DISTINCT_RESOURCES)) {
+    else if (e->scalars.error & ~(KTJ_DEVERR_CAREFUL | KTJ_DEVERR_DISTINCT_DEVICES | KTJ_DEVERR_DISTINCT_RESOURCES)) {
       e->last_error = limit_text(e->scalars.error);
       return KTJ_ERR_LIMIT;
     } else {
-      if (e->scalars.error == KTJ_DEVERR_UNSORTED) { e->sort_all_bits = true; e->sort_info[1] = 1; e->sort_passes = sort_packed_passes(e->scalars.sort, false); }
-      else e->stepwise = true;
-      HIPCHK(clear_error_bits(sc, KTJ_DEVERR_CAREFUL | KTJ_DEVERR_UNSORTED, st));
+      e->stepwise = true;
+      HIPCHK(clear_error_bits(sc, KTJ_DEVERR_CAREFUL, st));
     }
   }
   if (!emitted) { /* the stepwise rest */

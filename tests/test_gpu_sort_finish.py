@@ -128,3 +128,53 @@ def test_long_groups_in_many_workgroups(n):
     """Workgroups that start when others have found a group that is too long and not in order: tiles of every size."""
     print(n, flush=True)
     assert same_as_oracle(ops(*groups(n, 400, "shuffled"))) == ALL_BITS
+
+
+def test_long_groups_are_remembered_for_the_next_records():
+    """The passes are made twice for the first records of a producer, over all bits for the next fifteen, and the sixteenth are tried again."""
+    import torch
+    lib = abi.load_engine()
+    kinds = []
+    for order, size in (("shuffled", 400), ("forwards", 400), ("backwards", 300)):
+        for n in (9001, 30011):
+            sp = ops(*groups(n, size, order))
+            ora = og.OracleRun(sp)
+            records = torch.frombuffer(bytearray(C.string_at(sp.contents.generic, n * C.sizeof(abi.GenericRec))), dtype=torch.uint8).cuda()
+            kinds.append((sp, n, records, ora.output()))
+            ora.close()
+    torch.cuda.synchronize()
+    sp = kinds[0][0]
+    sp.contents.n_generic = 0
+    with TraceEngine(sp.contents.trace_name.decode()) as eng:
+        eng.submit_stream(sp)
+
+        def served(kind):
+            _, n, records, want = kinds[kind]
+            eng._chk(lib.ktj_submit_records_device(eng.h, abi.REC_GENERIC, records.data_ptr(), n), "ktj_submit_records_device")
+            eng.process()
+            assert eng.output() == want, kind
+            return [int(x) for x in eng.debug("sort_info")]
+
+        for kind in (3, 2):
+            low, again = served(kind)
+            assert low > 0 and again == 0
+        for bad, good in ((0, 3), (5, 2)):
+            assert served(bad) == [0, 1]
+            for turn in range(15):
+                assert served(turn % 6) == [0, 0], turn
+            low, again = served(good)
+            assert low > 0 and again == 0
+        assert served(1) == [0, 1]
+        served(2)
+
+
+def test_long_groups_and_rows_that_are_not_woven():
+    """The list of these is made with the order, the rows are made once: counters and list as if the first order had held."""
+    n = 300007
+    sp = ops(*groups(n, 400, "shuffled"))
+    rec = (abi.GenericRec * n).from_address(C.addressof(sp.contents.generic.contents))
+    for k in range(0, n, 5003):
+        rec[k].end_ns = rec[k].start_ns + 10**10
+    assert same_as_oracle(sp) == ALL_BITS
+    ts, tid = groups(20011, 400, "shuffled")
+    assert same_as_oracle(ops(ts, tid, (B + 10**6 + 2**20, B + 10**6 + 9 * 2**20))) == ALL_BITS   # launches, some of them dropped
