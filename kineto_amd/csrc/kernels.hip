@@ -2550,7 +2550,7 @@ __device__ __forceinline__ bool bitmap_test_and_set(uint32_t* bitmap, uint32_t s
   old = (uint32_t)__shfl((int)old, leader);
   return active && (twice || (old & bit) != 0);
 }
-#define JOIN_ROWS 4
+#define JOIN_ROWS 4u
 #ifndef KX_JOIN_ATTR
 #define KX_JOIN_ATTR
 #endif
@@ -2866,11 +2866,13 @@ hipError_t join_runtime_rows(const ktj_runtime_rec* r, uint64_t n, Columns c, ui
                              Table tn, NarrowCols nc, uint32_t* slot_f, uint32_t* slot_n, const ClockDev& clk, EmitCtx ctx, Rows rows,
                              uint32_t* len, Scalars* sc, hipStream_t st) {
   if (n == 0) return hipSuccess;
-  /* As many groups per workgroup as let all workgroups run at a time (four per CU, by their registers and LDS), up to JOIN_ROWS:
-   * with fewer the last ones run alone, with more CUs stand idle (333 000 rows, 1 / 2 / 4 groups: 56 / 50 / 66 us; a million
-   * 97 / 99 / 102; 10 million 1173 / 1160 / 1181). */
+  /* As many groups per workgroup as let all workgroups run at a time (four per CU, by their registers and LDS), as far as JOIN_ROWS do:
+   * with fewer the last ones run alone, with more CUs stand idle.  Behind that two, so that the last workgroups, which do not fill the
+   * GPU, are short ones.  1 / 2 / 3 / 4 groups, us: 333 000 rows 54 / 48 / 56 / 65, 500 000 50 / 48 / 54 / 63, 600 000 74 / 84 / 75 / 79,
+   * a million 103 / 106 / 120 / 107; 1.5 million 190 / 190 / 187 / 218, 2.5 million 302 / 301 / 324 / 332, 4 million 468 / 472 / 482 / 477,
+   * 10 million 1169 / 1151 / 1138 / 1148. */
   const uint64_t groups = grid_for(n, KTJ_BLOCK), at_once = 1024u;
-  const int rounds = groups <= at_once ? 1 : groups >= at_once * JOIN_ROWS ? JOIN_ROWS : (int)((groups + at_once - 1u) / at_once);
+  const int rounds = groups > at_once * JOIN_ROWS ? 2 : (int)((groups + at_once - 1u) / at_once);
   auto launch = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3(grid_for(n, KTJ_BLOCK * rounds)), dim3(KTJ_BLOCK), 0, st, r, n, c, first, api, tf, fc, tn, nc,
                        slot_f, slot_n, clk, ctx, rows, len, sc, rounds);
