@@ -2766,9 +2766,9 @@ __device__ __forceinline__ void mat_device_block(const ktj_device_rec* d, uint64
   flush_row_stats(rs, sc);
 }
 /* joined rows and lengths of the generic records (first workgroups) and of the device records (the others);
- * the runtime rows' are made in k_join_runtime.  Up to MAT_ONE_LAUNCH_ROWS both classes in one launch, as neither fills the GPU to its
- * end (400 000 rows 34 us, two launches 47; 700 000 57 and 70; a million 71 and 78).  Many: a launch for
- * each, as the code for both at once needs more registers (12 million: 690 against 575 us). */
+ * the runtime rows' are made in k_join_runtime.  Where there are both classes one launch makes them, as neither fills the GPU to its
+ * end (400 000 rows 34 us, two launches 47; a million 72 and 78; 2 million 140 and 150; 6 million 405 and 409; 12 million, of them 2 million
+ * generic, 698 and 701; 11 million and 20 000 generic 620 and 627). */
 template <bool GENERIC, bool DEVICE, bool TEXT>
 __global__ void __launch_bounds__(KTJ_BLOCK) __attribute__((amdgpu_waves_per_eu(4)))
 k_mat_rows(const ktj_generic_rec* g, uint64_t ng, uint64_t first_generic, const uint32_t* sync_first, uint32_t generic_blocks, const ktj_device_rec* d,
@@ -2854,7 +2854,6 @@ k_gather_len(const uint32_t* perm, const uint32_t* len, uint64_t n, uint32_t* le
     if ((v[k] >> 30) == KTJ_KIND_LEFT) left[at++] = (uint32_t)(base + (uint64_t)k * KTJ_BLOCK);
 }
 
-#define MAT_ONE_LAUNCH_ROWS 1048576u
 hipError_t mat_rows(const ktj_generic_rec* g, uint64_t ng, uint64_t first_generic, const uint32_t* sync_first, const ktj_device_rec* d, uint64_t nd,
                     Columns c, uint64_t first_device, const DevLink* link, const ClockDev& clk, EmitCtx ctx, Rows rows, uint32_t* len, Scalars* sc, hipStream_t st) {
   const unsigned gb = grid_stride_for(ng, KTJ_BLOCK), db = grid_stride_for(nd, KTJ_BLOCK);
@@ -2863,7 +2862,7 @@ hipError_t mat_rows(const ktj_generic_rec* g, uint64_t ng, uint64_t first_generi
                        link, clk, ctx, rows, len, sc, clock ? 1 : 0);
   };
   const bool clock = first_generic == 0;
-  if (gb && db && ng + nd < MAT_ONE_LAUNCH_ROWS) {
+  if (gb && db) {
     if (rows.schemas) launch(k_mat_rows<true, true, true>, gb, db, clock); else launch(k_mat_rows<true, true, false>, gb, db, clock);
   } else {
     if (gb) { if (rows.schemas) launch(k_mat_rows<true, false, true>, gb, 0, clock); else launch(k_mat_rows<true, false, false>, gb, 0, clock); }

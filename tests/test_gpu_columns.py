@@ -67,7 +67,7 @@ def test_clocks(runtime_mode, device_mode, spans):
 
 @pytest.mark.parametrize("rows", (140000, 524288, 524289))
 def test_joined_rows_in_one_launch_and_in_two(rows):
-    """Generic and device records together below, at and behind the million up to which one launch makes both."""
+    """Generic and device records together: one launch makes both, however many (behind a million there were two)."""
     print(rows, flush=True)
     sp, release = abi.synth_stream(2, rows, host_name="columns")
     ora = og.OracleRun(sp)
