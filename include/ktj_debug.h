@@ -35,8 +35,8 @@ enum {
 };
 
 /* Copies the array to dst (at most cap bytes) and reports its full size.  Valid after
- * ktj_process.  A trace of up to 2048 records keeps none of the arrays, and KTJ_DBG_MAT is not what
- * a larger one keeps mostly (rows as text): it is processed once more, with the launches of a large
+ * ktj_process.  A trace of up to 2048 records keeps none of the arrays, and KTJ_DBG_MAT, KTJ_DBG_COL_DUR and
+ * KTJ_DBG_COL_EXT are not what a larger one keeps mostly (rows as text, no columns that nothing reads): it is processed once more, with the launches of a large
  * trace and as ktj_process does it (the document is then in the engine's own buffer, also if
  * ktj_process_noalloc had put it into one of the caller's). */
 int ktj_debug_fetch(ktj_engine* e, int what, void* dst, uint64_t cap, uint64_t* n_bytes);

@@ -1211,15 +1211,8 @@ __device__ void lay_out_schemas(const EmitCtx& c, weave::SchemaBook* out, Schema
   __syncthreads();
   for (uint32_t j = k; j < weave::SCHEMA_TEXT * 4u; j += KTJ_BLOCK) out->text[j] = l->text[j];
 }
-/* Distinct deviceId and resourceId values, the range of the timestamps and the number of rows that are
- * printed.  The workgroup that ends last ranks the values and plans the sort's keys.  With a book the first
- * workgroup lays out the schemas instead of taking rows: this is the longest launch before the size pass that
- * small passes have, too. */
-/* Device rows take the number of their (device, stream) pair on the way, as their columns are read here anyway: a pass of its own
- * read 24 bytes a row, of them 16 that were made for it only (11 million records 3655 -> 3603 us, 22 million 7850 -> 7806, 30 000
- * 174 -> 171; 3 million 1169 -> 1161).
- * What a workgroup has looked up of the numbers; a pair whose places are taken is looked up each time.  A number is
- * stored behind the pair it belongs to (PAIR_CLAIMED: not yet). */
+/* What a workgroup of k_collect_distinct has looked up of the pairs' numbers; a pair whose places are taken is looked up each time.  A
+ * number is stored behind the pair it belongs to (PAIR_CLAIMED: not yet). */
 #define PAIR_SLOTS 1024u
 #define PAIR_CLAIMED 0xFFFFFFFFu
 struct PairCache { unsigned long long key[PAIR_SLOTS]; int32_t dev[PAIR_SLOTS]; uint32_t number[PAIR_SLOTS]; };
@@ -1239,6 +1232,13 @@ __device__ __forceinline__ uint32_t pair_number(PairCache& l, const StreamTables
   }
   return number;
 }
+/* Distinct deviceId and resourceId values, the range of the timestamps and the number of rows that are
+ * printed.  The workgroup that ends last ranks the values and plans the sort's keys.  With a book the first
+ * workgroup lays out the schemas instead of taking rows: this is the longest launch before the size pass that
+ * small passes have, too.
+ * Device rows take the number of their (device, stream) pair on the way, as their columns are read here anyway: a pass of its own
+ * read 24 bytes a row, of them 16 that were made for it only (11 million records 3655 -> 3603 us, 22 million 7850 -> 7806, 30 000
+ * 174 -> 171; 3 million 1169 -> 1161). */
 __global__ void __launch_bounds__(KTJ_BLOCK) k_collect_distinct(Columns c, uint64_t n, uint64_t per, uint64_t n_device, Backfill fill, SortSets s, Scalars* sc, int straight, EmitCtx ctx, weave::SchemaBook* book) {
   __shared__ uint64_t red_min[KTJ_BLOCK >> 6], red_max[KTJ_BLOCK >> 6];
   __shared__ unsigned long long seen[2][LOCAL_SET_SLOTS + 1]; /* deviceId, resourceId values */
@@ -1377,7 +1377,8 @@ __global__ void __launch_bounds__(KTJ_BLOCK) k_collect_distinct(Columns c, uint6
     p.res_bits = bits(mr ? mr - 1u : 0u);
     p.n_dev = md;
     p.key_bits = p.ts_bits + p.res_bits + bits(valid < n ? md : md ? md - 1u : 0u); /* rows that are dropped: a device behind the others */
-    /* The lowest bits that need no pass (k_sortp_finish): in 2^low ns, 65 us at most, a track has sixteen rows or fewer, were they
+    /* The lowest bits that need no pass (k_sortp_finish): in 2^low ns, 65 us at most, a track has thirty-two rows or fewer (sixteen where the
+     * trace takes all times of its bits, twice as many where it takes little more than half of them), were they
      * spread evenly over the trace and over the streams and threads; and no more bits than the passes that remain leave over.  (15
      * bits instead of 7 for 22 million, groups of 67 rows: a pass less, 135 us, but 220 us more behind the passes.) */
     const uint32_t pairs = sc->n_dense, threads = mr > pairs ? mr - pairs : 1u;
