@@ -178,3 +178,27 @@ def test_long_groups_and_rows_that_are_not_woven():
     assert same_as_oracle(sp) == ALL_BITS
     ts, tid = groups(20011, 400, "shuffled")
     assert same_as_oracle(ops(ts, tid, (B + 10**6 + 2**20, B + 10**6 + 9 * 2**20))) == ALL_BITS   # launches, some of them dropped
+
+
+def test_long_groups_in_a_buffer_of_the_callers():
+    """The second sort of ktj_process_noalloc, without room for the document and with it."""
+    import torch
+    for n in (9001, 40013):
+        sp = ops(*groups(n, 400, "shuffled"))
+        ora = og.OracleRun(sp)
+        want = ora.output()
+        ora.close()
+        for room in (len(want) // 2, len(want) + 64):
+            out = torch.full((len(want) + 4096,), 0xEE, dtype=torch.uint8, device="cuda:0")
+            torch.cuda.synchronize()
+            with TraceEngine(sp.contents.trace_name.decode()) as eng:
+                eng.submit_stream(sp)
+                for again in (1, 0):
+                    size = C.c_uint64()
+                    rc = eng.lib.ktj_process_noalloc(eng.h, eng.end_time_ns, out.data_ptr(), room, C.byref(size))
+                    got = bytes(out.cpu().numpy())
+                    if room < len(want):
+                        assert rc != 0 and size.value >= len(want) and got == b"\xEE" * len(got)
+                    else:
+                        assert rc == 0 and size.value == len(want) and got[:len(want)] == want and got[room:] == b"\xEE" * (len(got) - room)
+                        assert [int(x) for x in eng.debug("sort_info")] == [0, again]
