@@ -139,6 +139,14 @@ __device__ __forceinline__ uint64_t make_track(char* lds, uint32_t mine, uint64_
   return (uint64_t)(e2 | ((e5 - e2) << 8) | ((e8 - e5) << 16) | ((e10 - e8) << 24)) | ((uint64_t)(e12 - e10) << 32);
 }
 
+/* Documents of these many activities (250 MB at 480 bytes each) do not stay in the 256 MB last-level cache whichever way their lines
+ * are stored, but ordinary stores leave it and the L2s full of lines that are written back while the next kernels run: whole passes of
+ * 733 000 records 485 -> 465 us, of 3 million 1150 -> 1125 (k_decode of the next pass 94 -> 69 us), of 11 million 3590 -> 3560.  A smaller one
+ * is read back from there: sessions of 4000 operators with long strings (6 MB) 470 us with ordinary stores, 508 past the caches, files
+ * of 90 000 records 6430 and 6750. */
+#define WV_PAST_FROM (1u << 19)
+/* PAST: the document's whole lines are stored past the caches' replacement */
+template <bool PAST>
 __global__ void __launch_bounds__(WV_WAVES * 64u) __attribute__((amdgpu_waves_per_eu(4)))
 k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const uint8_t* kind_sorted, EmitCtx ctx, char* out, uint64_t prefix_len,
         const Scalars* sc, uint32_t rounds, const SchemaBook* schemas, const WideText* wide) {
@@ -421,13 +429,14 @@ k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const u
           if (lane < 8u) tb[nb + lane] = zero;
         }
       };
+      auto put_line = [](gptr p, v2u64 x) { if constexpr (PAST) __builtin_nontemporal_store(x, p); else *p = x; };
       auto store_lines = [&]() {
         if (nb) {
           const gptr dst = reinterpret_cast<gptr>((uintptr_t)doc);
           if (lane < 8u) reinterpret_cast<v2u64*>(tile)[lane] = rest;
-          if (lane < nb && lane >= own) dst[lane] = y0;
-          if (lane + 64u < nb) dst[lane + 64u] = y1;
-          if (lane + 128u < nb) dst[lane + 128u] = y2;
+          if (lane < nb && lane >= own) put_line(dst + lane, y0);
+          if (lane + 64u < nb) put_line(dst + lane + 64u, y1);
+          if (lane + 128u < nb) put_line(dst + lane + 128u, y2);
           wave_lds_order();
           doc += (uint64_t)nb * 16u;
           pend &= 127u;
@@ -495,7 +504,8 @@ hipError_t weave_activities(const TextRow* rows, const uint32_t* perm, const uin
    * records, whose turns make 12 for each: 136 us, with 4 141, with 8, one and a half times as many wavefronts as run, 150. */
   const uint64_t at_once = 256u * 16u, times = (turns + at_once * 24u - 1u) / (at_once * 24u);
   const uint32_t rounds = (uint32_t)((turns + at_once * times - 1u) / (at_once * times));
-  hipLaunchKernelGGL(k_weave, dim3(grid_for(turns, waves * rounds)), dim3(waves * 64u), WV_BOOK_BYTES + waves * WV_WAVE_BYTES, st, rows, perm, offs,
+  const auto kernel = n_most >= WV_PAST_FROM ? k_weave<true> : k_weave<false>;
+  hipLaunchKernelGGL(kernel, dim3(grid_for(turns, waves * rounds)), dim3(waves * 64u), WV_BOOK_BYTES + waves * WV_WAVE_BYTES, st, rows, perm, offs,
                      kind_sorted, ctx, out, prefix_len, sc, rounds, schemas, wide);
   return KTJ_LAUNCH_CHECK();
 }
