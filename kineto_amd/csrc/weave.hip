@@ -5,8 +5,8 @@
  * the lanes of a wavefront at different pieces, 168 registers for three wavefronts per SIMD, and no pass shorter than 38 us
  * as every wavefront runs through all of the formatter's code.  Here the text of 16 activities is laid out by the four
  * lanes that load each row, as a list of parts; then 64 segments at a time are fetched (a descriptor, up to 64 bytes of
- * text from LDS, a number of the row's), a prefix sum of their lengths gives their places, and they are OR-ed into a
- * zero-filled piece of the document in LDS, whose whole lines leave with lane-consecutive stores.  Numbers were made
+ * text from LDS, a number of the row's), a prefix sum of their lengths gives their places, and they are written into a
+ * piece of the document in LDS (put_segment), whose whole lines leave with lane-consecutive stores.  Numbers were made
  * into text in the size pass, which needs their lengths anyway; the texts with process and thread are made once per
  * track.  3730 vector and 740 LDS instructions for 64 activities (22 million records: kernels, runtime calls and operators),
  * four wavefronts per SIMD.
@@ -78,36 +78,64 @@ __device__ __forceinline__ void or_word(char* p, uint32_t v) {
 typedef unsigned long long v2u64 __attribute__((ext_vector_type(2)));
 typedef uint32_t v4u32 __attribute__((ext_vector_type(4)));
 
-__device__ __forceinline__ void or_text(char* q, uint32_t sh, const v4u32& x, uint32_t before) { /* four words of a text: those at q on */
-  or_word(q, __builtin_amdgcn_alignbyte(x.x, before, sh)); or_word(q + 4, __builtin_amdgcn_alignbyte(x.y, x.x, sh));
-  or_word(q + 8, __builtin_amdgcn_alignbyte(x.z, x.y, sh)); or_word(q + 12, __builtin_amdgcn_alignbyte(x.w, x.z, sh));
-}
-/* a segment (zeros behind its text and its number) to byte p of a zero-filled buffer */
-__device__ __forceinline__ void or_segment(char* buf, uint32_t p, uint32_t len, const v4u32& a, const v4u32& b, const v4u32& c, const v4u32& d,
-                                           uint32_t n_num, const v4u32& num) {
-  const uint32_t sh = 0u - p;                                   /* bits 0 and 1 count */
-  char* q = buf + (int32_t)(((int32_t)p - 1) & ~3);             /* the word of the byte before */
-  or_text(q, sh, a, 0u);
-  or_word(q + 16, __builtin_amdgcn_alignbyte(b.x, a.w, sh));
-  if (n_num) {
-    const uint32_t p2 = p + len, sh2 = 0u - p2;
-    char* q2 = buf + (int32_t)(((int32_t)p2 - 1) & ~3);
-    or_word(q2, __builtin_amdgcn_alignbyte(num.x, 0u, sh2)); or_word(q2 + 4, __builtin_amdgcn_alignbyte(num.y, num.x, sh2));
-    or_word(q2 + 8, __builtin_amdgcn_alignbyte(num.z, num.y, sh2));
-    if (n_num > 8u) { or_word(q2 + 12, __builtin_amdgcn_alignbyte(num.w, num.z, sh2)); or_word(q2 + 16, __builtin_amdgcn_alignbyte(0u, num.w, sh2)); }
+#define WV_WORD(hi, lo) __builtin_amdgcn_alignbyte(hi, lo, sh)
+/* a segment of up to 32 bytes of text (zeros behind its text and its number) to byte p of a zero-filled buffer */
+__device__ __forceinline__ void or_segment(char* buf, uint32_t p, uint32_t len, const v4u32& a, const v4u32& b, uint32_t n_num, const v4u32& num) {
+  {
+    const uint32_t sh = 0u - p;                                   /* bits 0 and 1 count */
+    char* q = buf + (int32_t)(((int32_t)p - 1) & ~3);             /* the word of the byte before */
+    or_word(q, WV_WORD(a.x, 0u)); or_word(q + 4, WV_WORD(a.y, a.x)); or_word(q + 8, WV_WORD(a.z, a.y)); or_word(q + 12, WV_WORD(a.w, a.z));
+    or_word(q + 16, WV_WORD(b.x, a.w)); or_word(q + 20, WV_WORD(b.y, b.x)); or_word(q + 24, WV_WORD(b.z, b.y)); or_word(q + 28, WV_WORD(b.w, b.z));
+    or_word(q + 32, WV_WORD(0u, b.w));
   }
-  if (len > 16u) {
-    or_word(q + 20, __builtin_amdgcn_alignbyte(b.y, b.x, sh)); or_word(q + 24, __builtin_amdgcn_alignbyte(b.z, b.y, sh));
-    or_word(q + 28, __builtin_amdgcn_alignbyte(b.w, b.z, sh)); or_word(q + 32, __builtin_amdgcn_alignbyte(c.x, b.w, sh));
-    if (len > 32u) {
-      or_word(q + 36, __builtin_amdgcn_alignbyte(c.y, c.x, sh)); or_word(q + 40, __builtin_amdgcn_alignbyte(c.z, c.y, sh));
-      or_word(q + 44, __builtin_amdgcn_alignbyte(c.w, c.z, sh)); or_word(q + 48, __builtin_amdgcn_alignbyte(d.x, c.w, sh));
-      if (len > 48u) {
-        or_word(q + 52, __builtin_amdgcn_alignbyte(d.y, d.x, sh)); or_word(q + 56, __builtin_amdgcn_alignbyte(d.z, d.y, sh));
-        or_word(q + 60, __builtin_amdgcn_alignbyte(d.w, d.z, sh)); or_word(q + 64, __builtin_amdgcn_alignbyte(0u, d.w, sh));
+  if (n_num) {
+    const uint32_t p2 = p + len, sh = 0u - p2;
+    char* q = buf + (int32_t)(((int32_t)p2 - 1) & ~3);
+    or_word(q, WV_WORD(num.x, 0u)); or_word(q + 4, WV_WORD(num.y, num.x)); or_word(q + 8, WV_WORD(num.z, num.y));
+    or_word(q + 12, WV_WORD(num.w, num.z)); or_word(q + 16, WV_WORD(0u, num.w));
+  }
+}
+typedef volatile __attribute__((address_space(3))) uint32_t* lds_word; /* (volatile: these accesses stay in their order) */
+__device__ __forceinline__ void put_word(char* p, uint32_t v) { *(lds_word)p = v; }
+__device__ __forceinline__ void or_shared_word(char* p, uint32_t v) { __hip_atomic_fetch_or((lds_word)p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT); }
+/* Segments one behind the other, a lane's behind that of the lane before it, to byte p and the following of a buffer that holds
+ * anything.  A word belongs to the segment that has its first byte, is written whole and OR-ed by whoever has the others.  A text's words are
+ * written up to the end of its sixteen bytes, whatever it has of them: the words too many are zeros in words of lanes behind, and these lanes
+ * write there later, as the last word of a text goes first, everybody's, and a word of a lane behind is an earlier one of its text.  Then come
+ * the numbers, which write their own words only, then the words that are shared.  A wavefront's LDS accesses are carried out in
+ * their order.  (All of them OR-ed to a buffer of zeros, whole lines cleared when they left: a 64-lane store of 16 bytes each takes
+ * the LDS pipe 14 cycles, three of them of the 290 that 64 segments take.  22 million records 3.42 -> 3.30 ms, 11 million kernels
+ * 1.68 -> 1.65, 733 000 records 141 -> 136 us.) */
+__device__ __forceinline__ void put_segment(char* buf, uint32_t p, uint32_t len, const v4u32& a, const v4u32& b, const v4u32& c, const v4u32& d,
+                                            uint32_t n_num, const v4u32& num) {
+  char* const q = buf + (int32_t)(((int32_t)p - 1) & ~3);       /* the word of the byte before: shared, if anything of the text is in it */
+  const uint32_t sh = 0u - p;                                   /* bits 0 and 1 count */
+  if (len + n_num + ((p - 1u) & 3u) > 3u) {                     /* (all in the first word: the lane behind has the same words) */
+    if (len > 16u) {
+      if (len > 32u) {
+        if (len > 48u) { put_word(q + 64, WV_WORD(0u, d.w)); put_word(q + 60, WV_WORD(d.w, d.z)); put_word(q + 56, WV_WORD(d.z, d.y)); put_word(q + 52, WV_WORD(d.y, d.x)); }
+        put_word(q + 48, WV_WORD(d.x, c.w)); put_word(q + 44, WV_WORD(c.w, c.z)); put_word(q + 40, WV_WORD(c.z, c.y)); put_word(q + 36, WV_WORD(c.y, c.x));
+      }
+      put_word(q + 32, WV_WORD(c.x, b.w)); put_word(q + 28, WV_WORD(b.w, b.z)); put_word(q + 24, WV_WORD(b.z, b.y)); put_word(q + 20, WV_WORD(b.y, b.x));
+    }
+    put_word(q + 16, WV_WORD(b.x, a.w)); put_word(q + 12, WV_WORD(a.w, a.z)); put_word(q + 8, WV_WORD(a.z, a.y)); put_word(q + 4, WV_WORD(a.y, a.x));
+  }
+  if (n_num) {
+    const uint32_t p2 = p + len, sh = 0u - p2, upto = n_num + ((p2 - 1u) & 3u) + 1u; /* bytes from q2 on */
+    char* const q2 = buf + (int32_t)(((int32_t)p2 - 1) & ~3);
+    if (upto > 4u) {
+      put_word(q2 + 4, WV_WORD(num.y, num.x));
+      if (upto > 8u) {
+        put_word(q2 + 8, WV_WORD(num.z, num.y));
+        if (upto > 12u) {
+          put_word(q2 + 12, WV_WORD(num.w, num.z));
+          if (upto > 16u) put_word(q2 + 16, WV_WORD(0u, num.w));
+        }
       }
     }
+    or_shared_word(q2, WV_WORD(num.x, 0u));
   }
+  or_shared_word(q, WV_WORD(a.x, 0u));
 }
 extern __shared__ __attribute__((aligned(16))) char wv_lds[];
 /* the track's texts, with the lead of its times; their lengths, a byte each */
@@ -135,7 +163,7 @@ __device__ __forceinline__ uint64_t make_track(char* lds, uint32_t mine, uint64_
                  e10 = __builtin_amdgcn_readlane(end, 10), e12 = __builtin_amdgcn_readlane(end, 12);
   const uint32_t start = which == 0 ? 0u : which == 1 ? e2 : which == 2 ? e5 : which == 3 ? e8 : e10;
   wave_lds_order();
-  if (lane < N_PIECES) or_segment(track, which * KTJ_WEAVE_LIT + (end - len - n_num - start), len, a, b, zero, zero, n_num, num);
+  if (lane < N_PIECES) or_segment(track, which * KTJ_WEAVE_LIT + (end - len - n_num - start), len, a, b, n_num, num);
   return (uint64_t)(e2 | ((e5 - e2) << 8) | ((e8 - e5) << 16) | ((e10 - e8) << 24)) | ((uint64_t)(e12 - e10) << 32);
 }
 
@@ -162,7 +190,6 @@ k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const u
   const uint32_t* const refs = reinterpret_cast<const uint32_t*>(wv_lds + WV_BOOK_REF);
   uint32_t* const parts = reinterpret_cast<uint32_t*>(wv_lds + mine + WV_PARTS_AT);
   char* const tile = wv_lds + mine + WV_TILE_AT;
-  for (uint32_t k = lane; k < WV_TILE_ROOM / 16u; k += 64u) reinterpret_cast<uint4*>(tile)[k] = make_uint4(0, 0, 0, 0);
   __syncthreads();
   const uint64_t n_rows = sc->emit_rows;
   typedef __attribute__((address_space(1))) v2u64* gptr;
@@ -199,21 +226,17 @@ k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const u
       uint64_t* t = reinterpret_cast<uint64_t*>(tile + at);
       uint64_t* w = reinterpret_cast<uint64_t*>(doc + at);
       if (i_next == n_rows) {
-        if (fill < 8) { const uint64_t k = (1ull << (8 * fill)) - 1ull; t[0] |= w[0] & ~k; t[1] = w[1]; }
-        else if (fill > 8) { const uint64_t k = (1ull << (8 * (fill - 8))) - 1ull; t[1] |= w[1] & ~k; }
-        else t[1] = w[1];
+        if (fill < 8) { const uint64_t k = (1ull << (8 * fill)) - 1ull; t[0] = (t[0] & k) | (w[0] & ~k); t[1] = w[1]; }
+        else { const uint64_t k = (1ull << (8 * (fill - 8))) - 1ull; t[1] = (t[1] & k) | (w[1] & ~k); }
       } else if (fill >= 8) { /* the successor's first bytes complete it */
-        const uint32_t n = 16u - fill;
-        const uint64_t hb = BlockWriter::head_bytes() & (n == 8 ? ~0ull : (1ull << (8 * n)) - 1ull);
-        t[1] |= hb << (8 * (fill - 8));
+        const uint32_t s = 8 * (fill - 8);
+        t[1] = (t[1] & ((1ull << s) - 1ull)) | (BlockWriter::head_bytes() << s);
       }
     }
     wave_lds_order();
     const uint32_t blocks = (pend >> 4) + (fill >= 8 || (fill && i_next == n_rows) ? 1u : 0u);
     if (lane <= 8u) {
-      v2u64* tb = reinterpret_cast<v2u64*>(tile);
-      const v2u64 x = tb[lane];
-      tb[lane] = (v2u64){0, 0};
+      const v2u64 x = reinterpret_cast<v2u64*>(tile)[lane];
       if (lane >= own && lane < blocks) reinterpret_cast<gptr>((uintptr_t)doc)[lane] = x;
     }
     wave_lds_order();
@@ -417,16 +440,11 @@ k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const u
         nb = (pend >> 7) * 8u;
         if (nb) {
           v2u64* tb = reinterpret_cast<v2u64*>(tile);
-          const v2u64 zero = {0, 0};
-          /* (three turns reach the end of the tile; read first, all of them, then cleared) */
+          /* (three turns reach the end of the tile) */
           if (lane < nb) y0 = tb[lane];
           if (lane + 64u < nb) y1 = tb[lane + 64u];
           if (lane + 128u < nb) y2 = tb[lane + 128u];
           if (lane < 8u) rest = tb[nb + lane];
-          if (lane < nb) tb[lane] = zero;
-          if (lane + 64u < nb) tb[lane + 64u] = zero;
-          if (lane + 128u < nb) tb[lane + 128u] = zero;
-          if (lane < 8u) tb[nb + lane] = zero;
         }
       };
       auto put_line = [](gptr p, v2u64 x) { if constexpr (PAST) __builtin_nontemporal_store(x, p); else *p = x; };
@@ -474,7 +492,7 @@ k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const u
         const uint32_t end = dpp_add(mine_len);
         const bool now = valid && end + pend <= WV_TILE;
         const uint32_t n = (uint32_t)__popcll(__ballot(now)); /* (never 0: a segment is shorter than the tile) */
-        if (now) or_segment(tile, pend + (end - mine_len), len, x.a, b, c, d, n_num, x.num);
+        if (now) put_segment(tile, pend + (end - mine_len), len, x.a, b, c, d, n_num, x.num);
         pend += __builtin_amdgcn_readlane(end, n - 1u);
         wave_lds_order();
         take_lines();

@@ -420,6 +420,41 @@ def test_many_turns_with_few_rows_left(n, left_known, long_names):
     assert first[3] == 0 or not left_known
 
 
+def short_stream(n):
+    """n CPU ops whose texts are laid out in segments of a few bytes (names and strings of 0 to 9, of 58 to 70 and of 120 to 136
+    characters, one word and less among them), at every alignment."""
+    import numpy as np
+    rng = np.random.default_rng(n)
+    b = StreamBuilder(window=(B, B + 10**15), host_name="short")
+    lengths = [*range(10), *range(58, 71), *range(120, 137)]
+    names = np.array([b.s(_text(k, k)) for k in lengths])
+    text = b.schema([("s", abi.F_STR, 1), ("y", abi.F_I64, 1)])
+    raw = b.schema([(None, abi.F_RAW, 1)])
+    values = rng.integers(0, 10**6, 512)
+    values[::2] = names[rng.integers(0, len(names), 256)]
+    b.arg_slots([int(v) for v in values])
+    sp = b.build()
+    rec = np.zeros(n, dtype=np.dtype(abi.GenericRec))
+    k = np.arange(n)
+    rec["start_ns"] = B + 10 * k
+    rec["end_ns"] = rec["start_ns"] + rng.integers(0, 10**rng.integers(0, 7, n))
+    rec["resource"], rec["device"], rec["id"] = 5 + k // 41 % 3, 42, k + 1
+    rec["name_id"] = names[np.where(rng.integers(0, 3, n), rng.integers(0, 10, n), rng.integers(0, len(names), n))]
+    rec["schema_id"] = np.array([abi.KTJ_NONE, text, raw], dtype=np.uint32)[rng.integers(0, 3, n)]
+    rec["args_off"] = 2 * rng.integers(0, 256, n)
+    held = (abi.GenericRec * n).from_buffer_copy(rec.tobytes())
+    sp.contents.generic, sp.contents.n_generic = C.cast(held, type(sp.contents.generic)), n
+    sp.held = held
+    return sp
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", (1, 2, 17, 1000, 30007, 524321))
+def test_segments_of_a_few_bytes(n):
+    """Several in one word of the document, and (the last) lines stored past the caches."""
+    assert _gpu_vs_oracle(short_stream(n), passes=2)[1][0] == 1
+
+
 @pytest.mark.gpu
 def test_rows_left_that_no_pass_before_had():
     """Behind a wait of their own: the engine's last pass had none."""
