@@ -8,20 +8,23 @@
  * text from LDS, a number of the row's), a prefix sum of their lengths gives their places, and they are written into a
  * piece of the document in LDS (put_segment), whose whole lines leave with lane-consecutive stores.  Numbers were made
  * into text in the size pass, which needs their lengths anyway; the texts with process and thread are made once per
- * track.  3730 vector and 740 LDS instructions for 64 activities (22 million records: kernels, runtime calls and operators),
- * four wavefronts per SIMD.
+ * track.
  *
- * What bounds it: memory (22 million records 13.6 GB in 3.44 ms, 0.89 of what a plain copy reaches; 11 million kernels 0.95),
- * with the vector units busy for 2.1 and the LDS pipes for 1.9 of the 3.44 ms, a third of that bank conflicts.
- * Measured against k_emit_direct: 10 000 x 3 records 38.7 -> 15.5 us, 4000 operators with long strings
- * 71 -> 24 us, 733 000 records 176 -> 136 us, 3 million 795 -> 451 us, 11 million kernels 2.06 -> 1.70 ms, 22 million
- * records 4.59 -> 3.44 ms, 5 million operators with long strings (1.4 KB each: strings beyond 128 bytes are fetched from
- * memory piece by piece) 3.20 -> 2.67 ms; the size pass has become up to 18 % longer for the numbers' text.
+ * What bounds it: latency, the LDS pipe and the vector units before memory (22 million records 2.97 ms, 13.6 GB, of which 2.6 ms are
+ * what a copy of two parts read and seven written takes; without its stores the kernel takes some 2.5, without words written
+ * to LDS either 2.0), so it is the wavefronts in flight that count: five per SIMD, which five workgroups of
+ * four make (of five or of ten wavefronts three and one fit into a CU: 4.2 and 4.5 ms).  That takes 96 registers and
+ * 32000 bytes of LDS per workgroup: texts that begin alike are there once, and names and the piece of the document share their room
+ * (2944 bytes of document and 1280 of names would not fit; 2304 and 768 are short of most groups of 64 segments: 11 million
+ * kernels 1.88 ms).  Four -> five wavefronts: 733 000 records 136 -> 121 us, 3 million 443 -> 402, 22 million 3.30 -> 2.97 ms,
+ * 5 million operators with long strings 2.64 -> 2.45, 11 million kernels, at the memory's rate, 1.65 -> 1.62; three: 2.48, two 2.83.
+ *
+ * Measured against k_emit_direct (lane per activity): 10 000 x 3 records 38.7 -> 15 us, 4000 operators with long strings
+ * 71 -> 23 us, 733 000 records 176 -> 121 us, 3 million 795 -> 402 us, 11 million kernels 2.06 -> 1.62 ms, 22 million
+ * records 4.59 -> 2.97 ms, 5 million operators with long strings (1.4 KB each: strings beyond 128 bytes are fetched from
+ * memory piece by piece) 3.20 -> 2.45 ms; the size pass has become up to 18 % longer for the numbers' text.
  * (Long strings' whole lines from the dictionary to the document past the tile, the loads of four strings at a time in
- * front of any store: 2.70 ms, and 26 instead of 24 us for 4000 of them.)
- * Fewer wavefronts cost: three per SIMD 2.48 ms for the kernels, two 2.83.  Five (96 registers, 2048 bytes of tile, 512
- * of names) gave 2.22, 2048 bytes being short of most groups of 64 segments; with the tile as it is 96 registers alone
- * 1.97.  Workgroups of four wavefronts: eight, with the book in LDS twice per CU instead of four times, 1.74.
+ * front of any store: no gain.)
  */
 #include "gpu_common.h"
 #include "weave_core.h"
@@ -36,20 +39,22 @@ using namespace weave;
 #define WV_PARTS (WV_ROWS * 7u)
 #define WV_VAL_BYTES (S_RUN * 16u)                    /* S_A and the following; an odd number of sixteens: the same slot of neighbours lies in other banks */
 #define WV_VAL(slot) (((slot) - 1u) * 16u)
-#define WV_NAMES 1280u                                /* bytes of strings that wait in LDS */
+#define WV_NAMES 1280u                                /* bytes of strings that wait in LDS, at most */
 #define WV_NAME_MOST 128u
-#define WV_TILE 2944u                                 /* bytes of document that wait in LDS */
-#define WV_TILE_ROOM (WV_TILE + 128u)                 /* a line behind it, and what texts write beyond their end */
 /* of a wavefront: */
-#define WV_NAMES_AT (WV_ROWS * WV_VAL_BYTES)
-#define WV_TRACK_AT (WV_NAMES_AT + WV_NAMES)
+#define WV_TRACK_AT (WV_ROWS * WV_VAL_BYTES)
 #define WV_PARTS_AT (WV_TRACK_AT + T_COUNT * KTJ_WEAVE_LIT)
 #define WV_TILE_AT (WV_PARTS_AT + WV_PARTS * 4u + 32u)
-#define WV_WAVE_BYTES (WV_TILE_AT + WV_TILE_ROOM)
-/* of the workgroup, in front of them: the texts, the book's and the schemas'; the schemas' plans; where the parts are; descriptors */
-#define WV_BOOK_PLANS ((MAX_TEXT + SCHEMA_TEXT) * 16u)
-#define WV_BOOK_REF (WV_BOOK_PLANS + MAX_SCHEMAS * (uint32_t)sizeof(SchemaPlan))
-#define WV_BOOK_DESC (WV_BOOK_REF + R_COUNT * 4u)
+/* the bytes of the document that wait in LDS, from the front on, and the strings, from the end on: between them what texts write beyond
+ * their end, behind the former at least a line */
+#define WV_SPACE 3600u
+#define WV_GAP 32u
+#define WV_TILE_MOST 3072u                            /* whole lines leave in three turns at most */
+#define WV_WAVE_BYTES (WV_TILE_AT + WV_SPACE)
+/* of the workgroup, in front of them: the texts, the book's and the schemas'; where the parts are, the schemas' behind the book's; descriptors */
+#define WV_BOOK_REF ((LDS_BOOK.n_text + SCHEMA_TEXT) * 16u)
+#define WV_BOOK_PLANS (WV_BOOK_REF + (R_COUNT + 1u) / 2u * 4u)
+#define WV_BOOK_DESC (WV_BOOK_PLANS + MAX_SCHEMAS * 4u)
 #define WV_BOOK_BYTES ((WV_BOOK_DESC + (MAX_DESC + SCHEMA_DESC) * 4u + 15u) / 16u * 16u)
 
 /* a part: first segment | kind << 15 (text, or one of the strings of S_RUN) | first descriptor << 17 | activity << 26 */
@@ -58,7 +63,48 @@ using namespace weave;
 #define WV_PART_DESC(x) (((x) >> 17) & 0x1FFu)
 #define WV_PART_ACT(x) ((x) >> 26)
 
-static __device__ constexpr Book g_book = BOOK;
+/* The book as it lies in LDS.  A text's first 32 bytes and the others are at places of their own (in 27 heads of events the former are
+ * the same), a part is named by sixteen bits. */
+#define WV_WD_LEN(x) ((x) & 0x7Fu)
+#define WV_WD_TRACK (1u << 7)
+#define WV_WD_SLOT(x) (((x) >> 8) & 0xFu)
+#define WV_WD_UNIT(x) (((x) >> 12) & 0x1FFu)
+#define WV_WD_UNIT2(x) (((x) >> 21) & 0x1FFu)       /* (bits 30 and 31: WV_FAR) */
+#define WV_WD(len, slot, unit, unit2) ((len) | ((slot) << 8) | ((unit) << 12) | ((unit2) << 21))
+#define WV_REF(base, count) ((base) | ((count) << 9))
+#define WV_REF_BASE(r) ((r) & 0x1FFu)
+#define WV_REF_COUNT(r) ((r) >> 9)
+struct LdsBook {
+  uint32_t text[MAX_TEXT * 4], desc[MAX_DESC], n_text;
+  uint16_t ref[R_COUNT + 1u];
+};
+constexpr LdsBook make_lds_book() {
+  LdsBook l{};
+  auto place = [&](const uint32_t* w, uint32_t units) { /* the same bytes somewhere already? */
+    uint32_t at = 0;
+    for (; at + units <= l.n_text; ++at) {
+      bool same = true;
+      for (uint32_t i = 0; i < units * 4; ++i) same = same && l.text[at * 4 + i] == w[i];
+      if (same) break;
+    }
+    if (at + units > l.n_text) {
+      at = l.n_text;
+      for (uint32_t i = 0; i < units * 4; ++i) l.text[at * 4 + i] = w[i];
+      l.n_text += units;
+    }
+    return at;
+  };
+  for (uint32_t k = 0; k < BOOK.n_desc; ++k) {
+    const uint32_t d = BOOK.desc[k], len = KTJ_WD_LEN(d), unit = KTJ_WD_UNIT(d), units = (len + 15) / 16;
+    if (d & KTJ_WD_TRACK) l.desc[k] = WV_WD(len, KTJ_WD_SLOT(d), unit, unit + 2) | WV_WD_TRACK;
+    else l.desc[k] = WV_WD(len, KTJ_WD_SLOT(d), place(BOOK.text + unit * 4, units < 2 ? units : 2), units > 2 ? place(BOOK.text + (unit + 2) * 4, units - 2) : 0);
+  }
+  for (uint32_t r = 0; r < R_COUNT; ++r) l.ref[r] = (uint16_t)WV_REF(KTJ_WREF_BASE(BOOK.ref[r]), KTJ_WREF_COUNT(BOOK.ref[r]));
+  return l;
+}
+constexpr LdsBook LDS_BOOK = make_lds_book();
+static_assert(MAX_DESC + SCHEMA_DESC <= 512u && SCHEMA_DESC < 128u && LDS_BOOK.n_text + SCHEMA_TEXT + 2u <= 512u, "nine bits each, seven for a count");
+static __device__ constexpr LdsBook g_book = LDS_BOOK;
 
 __device__ __forceinline__ uint32_t dpp_add(uint32_t v) { /* inclusive sum over the wavefront */
 #define WV_DPP(ctrl, rows) v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, rows, 0xF, false)
@@ -146,11 +192,11 @@ __device__ __forceinline__ uint64_t make_track(char* lds, uint32_t mine, uint64_
   const Text pid = text_of(dev), tid = text_of(thread);
   Text time = text_of(lead);
   if (lead == 0) { time.lo = 0; time.n = 0; }
-  const uint32_t desc = lane < N_PIECES ? *reinterpret_cast<const uint32_t*>(lds + WV_BOOK_DESC + (KTJ_WREF_BASE(g_book.ref[R_PIECES]) + lane) * 4u) : 0u;
-  const uint32_t len = KTJ_WD_LEN(desc), slot = KTJ_WD_SLOT(desc), n_num = slot == S_PID ? pid.n : slot == S_TID ? tid.n : slot == S_LEAD ? time.n : 0u;
+  const uint32_t desc = lane < N_PIECES ? *reinterpret_cast<const uint32_t*>(lds + WV_BOOK_DESC + (WV_REF_BASE(LDS_BOOK.ref[R_PIECES]) + lane) * 4u) : 0u;
+  const uint32_t len = WV_WD_LEN(desc), slot = WV_WD_SLOT(desc), n_num = slot == S_PID ? pid.n : slot == S_TID ? tid.n : slot == S_LEAD ? time.n : 0u;
   const v4u32 zero = {0, 0, 0, 0};
   v4u32 a = zero, b = zero, num = zero;
-  const v4u32* t = reinterpret_cast<const v4u32*>(lds) + KTJ_WD_UNIT(desc);
+  const v4u32* t = reinterpret_cast<const v4u32*>(lds) + WV_WD_UNIT(desc);
   if (len) a = t[0];
   if (len > 16u) b = t[1];
   if (slot == S_PID) { num.x = (uint32_t)pid.lo; num.y = (uint32_t)(pid.lo >> 32); num.z = (uint32_t)pid.hi; num.w = (uint32_t)(pid.hi >> 32); }
@@ -175,19 +221,29 @@ __device__ __forceinline__ uint64_t make_track(char* lds, uint32_t mine, uint64_
 #define WV_PAST_FROM (1u << 19)
 /* PAST: the document's whole lines are stored past the caches' replacement */
 template <bool PAST>
-__global__ void __launch_bounds__(WV_WAVES * 64u) __attribute__((amdgpu_waves_per_eu(4)))
+__global__ void __launch_bounds__(WV_WAVES * 64u) __attribute__((amdgpu_waves_per_eu(5)))
 k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const uint8_t* kind_sorted, EmitCtx ctx, char* out, uint64_t prefix_len,
         const Scalars* sc, uint32_t rounds, const SchemaBook* schemas, const WideText* wide) {
   if (sc->no_text) return;
   const uint32_t lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  static_assert(WV_BOOK_PLANS % 16u == 0 && sizeof(SchemaPlan) % 16u == 0, "in sixteens");
-  for (uint32_t k = threadIdx.x; k < MAX_TEXT; k += blockDim.x) reinterpret_cast<uint4*>(wv_lds)[k] = reinterpret_cast<const uint4*>(g_book.text)[k];
-  for (uint32_t k = threadIdx.x; k < (WV_BOOK_REF - MAX_TEXT * 16u) / 16u; k += blockDim.x) /* the schemas' texts and plans */
-    reinterpret_cast<uint4*>(wv_lds)[MAX_TEXT + k] = reinterpret_cast<const uint4*>(schemas)[k];
-  for (uint32_t k = threadIdx.x; k < R_COUNT + MAX_DESC + SCHEMA_DESC; k += blockDim.x)
-    reinterpret_cast<uint32_t*>(wv_lds + WV_BOOK_REF)[k] = k < R_COUNT ? g_book.ref[k] : k < R_COUNT + MAX_DESC ? g_book.desc[k - R_COUNT] : schemas->desc[k - R_COUNT - MAX_DESC];
+  for (uint32_t k = threadIdx.x; k < LDS_BOOK.n_text + SCHEMA_TEXT; k += blockDim.x)
+    reinterpret_cast<uint4*>(wv_lds)[k] = k < LDS_BOOK.n_text ? reinterpret_cast<const uint4*>(g_book.text)[k] : reinterpret_cast<const uint4*>(schemas->text)[k - LDS_BOOK.n_text];
+  for (uint32_t k = threadIdx.x; k < R_COUNT; k += blockDim.x) reinterpret_cast<uint16_t*>(wv_lds + WV_BOOK_REF)[k] = g_book.ref[k];
+  if (threadIdx.x < MAX_SCHEMAS) {
+    const uint32_t a = schemas->plan[threadIdx.x].args, b = schemas->plan[threadIdx.x].args2;
+    reinterpret_cast<uint32_t*>(wv_lds + WV_BOOK_PLANS)[threadIdx.x] = WV_REF(KTJ_WREF_BASE(a), KTJ_WREF_COUNT(a)) | (WV_REF(KTJ_WREF_BASE(b), KTJ_WREF_COUNT(b)) << 16);
+  }
+  for (uint32_t k = threadIdx.x; k < MAX_DESC + SCHEMA_DESC; k += blockDim.x) {
+    uint32_t d;
+    if (k < MAX_DESC) d = g_book.desc[k];
+    else {
+      const uint32_t x = schemas->desc[k - MAX_DESC], unit = (KTJ_WD_UNIT(x) - SCHEMA_UNIT + LDS_BOOK.n_text) & 0x1FFu;
+      d = WV_WD(KTJ_WD_LEN(x), KTJ_WD_SLOT(x), unit, (unit + 2u) & 0x1FFu);
+    }
+    reinterpret_cast<uint32_t*>(wv_lds + WV_BOOK_DESC)[k] = d;
+  }
   const uint32_t mine = WV_BOOK_BYTES + wave * WV_WAVE_BYTES; /* this wavefront's LDS */
-  const uint32_t* const refs = reinterpret_cast<const uint32_t*>(wv_lds + WV_BOOK_REF);
+  const uint16_t* const refs = reinterpret_cast<const uint16_t*>(wv_lds + WV_BOOK_REF);
   uint32_t* const parts = reinterpret_cast<uint32_t*>(wv_lds + mine + WV_PARTS_AT);
   char* const tile = wv_lds + mine + WV_TILE_AT;
   __syncthreads();
@@ -282,15 +338,15 @@ k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const u
       const uint32_t a = KTJ_TR_ARGS(plan);
       if (a >= KTJ_TR_SCHEMA) {
         if (a != KTJ_TR_NO_ARGS) {
-          const SchemaPlan* p = reinterpret_cast<const SchemaPlan*>(wv_lds + WV_BOOK_PLANS) + (a - KTJ_TR_SCHEMA);
-          args_ref = p->args; args2_ref = p->args2;
+          const uint32_t both = reinterpret_cast<const uint32_t*>(wv_lds + WV_BOOK_PLANS)[a - KTJ_TR_SCHEMA];
+          args_ref = both & 0xFFFFu; args2_ref = both >> 16;
         }
       } else { args_ref = refs[R_ARGS + a]; args2_ref = refs[R_ARGS2 + a]; }
-      const uint32_t name = KTJ_TR_NAMED(plan) != KTJ_TR_NAME_RUN ? KTJ_WREF_COUNT(refs[KTJ_TR_NAMED(plan)]) : (len0 + KTJ_WEAVE_LIT - 1u) / KTJ_WEAVE_LIT;
+      const uint32_t name = KTJ_TR_NAMED(plan) != KTJ_TR_NAME_RUN ? WV_REF_COUNT(refs[KTJ_TR_NAMED(plan)]) : (len0 + KTJ_WEAVE_LIT - 1u) / KTJ_WEAVE_LIT;
       const uint32_t runs = (len1 + KTJ_WEAVE_LIT - 1u) / KTJ_WEAVE_LIT;
-      const uint32_t head = KTJ_WREF_COUNT(refs[R_HEAD + KTJ_TR_TYPE(plan)]), body = KTJ_WREF_COUNT(refs[R_BODY_NONE + KTJ_TR_BODY(plan)]);
-      const uint32_t tail = KTJ_WREF_COUNT(refs[R_TAIL + KTJ_TR_TAIL(plan)]);
-      const uint32_t args = KTJ_WREF_COUNT(args_ref), args2 = KTJ_WREF_COUNT(args2_ref);
+      const uint32_t head = WV_REF_COUNT(refs[R_HEAD + KTJ_TR_TYPE(plan)]), body = WV_REF_COUNT(refs[R_BODY_NONE + KTJ_TR_BODY(plan)]);
+      const uint32_t tail = WV_REF_COUNT(refs[R_TAIL + KTJ_TR_TAIL(plan)]);
+      const uint32_t args = WV_REF_COUNT(args_ref), args2 = WV_REF_COUNT(args2_ref);
       counts = ((2u + (name ? 1u : 0u) + (args ? 1u : 0u) + (runs ? 1u : 0u) + (args2 ? 1u : 0u) + (tail ? 1u : 0u)) << 16) |
                (head + name + body + args + runs + args2 + tail);
       units = (len0 <= WV_NAME_MOST ? (len0 + 15u) / 16u : 0u) | (KTJ_TR_BETWEEN(plan) == 3u ? 2u << 16 : 0u);
@@ -298,17 +354,18 @@ k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const u
     const uint32_t upto = dpp_add(counts), before = upto - counts; /* of the first lane of each */
     /* the strings in LDS: wide texts, two units each, and names as far as there is room */
     static_assert(WV_ROWS * sizeof(WideText) <= WV_NAMES && sizeof(WideText) == 32, "the wide texts have room");
-    const uint32_t units_upto = dpp_add(units), double_at = WV_NAMES_AT + ((units_upto - units) >> 16) * 16u;
-    const uint32_t name_upto = (units_upto & 0xFFFFu) + (__builtin_amdgcn_readlane(units_upto, 63) >> 16);
+    const uint32_t units_upto = dpp_add(units), double_at = WV_WAVE_BYTES - (units_upto >> 16) * 16u;
+    const uint32_t wide_units = __builtin_amdgcn_readlane(units_upto, 63) >> 16, name_upto = (units_upto & 0xFFFFu) + wide_units;
     units &= 0xFFFFu;
     const bool near = units != 0 && name_upto <= WV_NAMES / 16u;
-    const uint32_t name_at = WV_NAMES_AT + (name_upto - units) * 16u;
-    v4u32 nx, ny, wx, wy;
-    const bool wide_text = counts != 0 && KTJ_TR_BETWEEN(plan) == 3u;
-    if (wide_text) {
-      const gsrc src = reinterpret_cast<gsrc>((uint64_t)(uintptr_t)wide + (uint64_t)more * sizeof(WideText));
-      wx = src[0]; wy = src[1];
-    }
+    const uint32_t name_at = WV_WAVE_BYTES - name_upto * 16u;
+    /* what they leave of the space (the last of the names that are there says it) */
+    const uint64_t near_ones = __ballot(near);
+    const uint32_t taken = (near_ones ? __builtin_amdgcn_readlane(name_upto, 63u - (uint32_t)__clzll((long long)near_ones)) : wide_units) * 16u + WV_GAP;
+    const uint32_t room = WV_SPACE - taken < WV_TILE_MOST ? WV_SPACE - taken : WV_TILE_MOST;
+    v4u32 nx, ny, wx;
+    const uint32_t wide_at = WV_QUAD(counts != 0 && KTJ_TR_BETWEEN(plan) == 3u ? mine + double_at : 0u, 0);
+    if (h < 2u && wide_at) wx = reinterpret_cast<gsrc>((uint64_t)(uintptr_t)wide + (uint64_t)more * sizeof(WideText))[h];
     const uint32_t q_units = WV_QUAD(near ? units : 0u, 0), q_at = mine + WV_QUAD(name_at, 0);
     {
       const gsrc src = reinterpret_cast<gsrc>((uint64_t)(uintptr_t)ctx.dict.name_blob + (uint64_t)name_off * 16u);
@@ -318,7 +375,7 @@ k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const u
     if (counts) {
       uint32_t* w = parts + (before >> 16);
       uint32_t seg = (before & 0x7FFFu) | (act << 26); /* (segments stay below their 15 bits) */
-      auto put_part = [&](uint32_t ref) { const uint32_t n = KTJ_WREF_COUNT(ref); if (n) { *w++ = seg | (KTJ_WREF_BASE(ref) << 17); seg += n; } };
+      auto put_part = [&](uint32_t ref) { const uint32_t n = WV_REF_COUNT(ref); if (n) { *w++ = seg | (WV_REF_BASE(ref) << 17); seg += n; } };
       put_part(refs[R_HEAD + KTJ_TR_TYPE(plan)]);
       if (KTJ_TR_NAMED(plan) != KTJ_TR_NAME_RUN) put_part(refs[KTJ_TR_NAMED(plan)]);
       else if (len0) { *w++ = seg | (1u << 15); seg += (len0 + KTJ_WEAVE_LIT - 1u) / KTJ_WEAVE_LIT; }
@@ -337,10 +394,7 @@ k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const u
     }
     const uint32_t totals = __builtin_amdgcn_readlane(upto, 63);
     if (lane == 0) parts[totals >> 16] = totals & 0x7FFFu;
-    if (wide_text) {
-      *reinterpret_cast<v4u32*>(wv_lds + mine + double_at) = wx;
-      *reinterpret_cast<v4u32*>(wv_lds + mine + double_at + 16u) = wy;
-    }
+    if (h < 2u && wide_at) *reinterpret_cast<v4u32*>(wv_lds + wide_at + h * 16u) = wx;
     if (h < q_units) {
       *reinterpret_cast<v4u32*>(wv_lds + q_at + h * 16u) = nx;
       if (h + 4u < q_units) *reinterpret_cast<v4u32*>(wv_lds + q_at + (h + 4u) * 16u) = ny;
@@ -394,7 +448,7 @@ k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const u
       }
       wave_lds_order();
       /* 64 segments at a time: what the next ones are made of is read before these are put together */
-      struct Piece { v4u32 a, num; uint32_t desc, at, part; }; /* at: in LDS; WV_FAR: place in the string's blob, in units of sixteen bytes */
+      struct Piece { v4u32 a, num; uint32_t desc, at, at2, part; }; /* at: in LDS; WV_FAR: place in the string's blob, in units of sixteen bytes */
 #define WV_FAR (1u << 30)
 #define WV_FAR_ARG (1u << 31)
       uint32_t part_after = 0;
@@ -414,19 +468,22 @@ k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const u
         const uint32_t kind = WV_PART_KIND(pr), vrow = mine + WV_PART_ACT(pr) * WV_VAL_BYTES;
         const uint32_t idx = kind == 0 && valid ? WV_PART_DESC(pr) + seg : 0u;
         x.desc = *reinterpret_cast<const uint32_t*>(wv_lds + WV_BOOK_DESC + idx * 4u);
-        x.at = KTJ_WD_UNIT(x.desc) * 16u;
-        if (x.desc & KTJ_WD_TRACK) {
-          x.desc |= (uint32_t)(track_lens >> (KTJ_WD_UNIT(x.desc) * 2u)) & 0x7Fu; /* (four units to a text) */
+        x.at = WV_WD_UNIT(x.desc) * 16u;
+        x.at2 = WV_WD_UNIT2(x.desc) * 16u;
+        if (x.desc & WV_WD_TRACK) {
+          x.desc |= (uint32_t)(track_lens >> (WV_WD_UNIT(x.desc) * 2u)) & 0x7Fu; /* (four units to a text) */
           x.at += mine + WV_TRACK_AT;
+          x.at2 += mine + WV_TRACK_AT;
         }
         if (kind != 0) {
           const uint64_t r = *reinterpret_cast<const uint64_t*>(wv_lds + vrow + WV_VAL(S_RUN) + (2u - kind) * 8u);
           const uint32_t rest = ((uint32_t)(r >> 32) & 0xFFFFu) - seg * KTJ_WEAVE_LIT, near = (uint32_t)(r >> 48);
           x.at = near ? mine + near + seg * KTJ_WEAVE_LIT : (uint32_t)r + seg * (KTJ_WEAVE_LIT / 16u);
-          x.desc = KTJ_WD(rest < KTJ_WEAVE_LIT ? rest : KTJ_WEAVE_LIT, S_NONE, 0u) | (near ? 0u : kind == 1u ? WV_FAR : WV_FAR | WV_FAR_ARG);
+          x.at2 = x.at + 32u;
+          x.desc = WV_WD(rest < KTJ_WEAVE_LIT ? rest : KTJ_WEAVE_LIT, S_NONE, 0u, 0u) | (near ? 0u : kind == 1u ? WV_FAR : WV_FAR | WV_FAR_ARG);
         }
         x.a = *reinterpret_cast<const v4u32*>(wv_lds + (x.desc & WV_FAR ? 0u : x.at));
-        const uint32_t slot = KTJ_WD_SLOT(x.desc);
+        const uint32_t slot = WV_WD_SLOT(x.desc);
         x.num = *reinterpret_cast<const v4u32*>(wv_lds + vrow + (slot == S_K ? WV_VAL(S_RUN) : WV_VAL(slot))); /* (S_NONE: what lies there, which does not count) */
         if (slot == S_K) { x.num.w = x.num.y; x.num.y = 0; x.num.z = 0; }
         if (slot == S_NONE) x.num.w = 0;
@@ -465,14 +522,14 @@ k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const u
       /* As many of them as the tile has room for; the others are fetched again.  (All of them, in two turns over the tile:
        * 5 % more for 11 million kernels.) */
       auto put = [&](Piece& x) {
-        const uint32_t len = KTJ_WD_LEN(x.desc);
+        const uint32_t len = WV_WD_LEN(x.desc);
         const bool far = (x.desc & WV_FAR) != 0;
         v4u32 b = {0, 0, 0, 0}, c = b, d = b;
         if (len > 16u && !far) {
           b = *reinterpret_cast<const v4u32*>(wv_lds + x.at + 16u);
           if (len > 32u) {
-            c = *reinterpret_cast<const v4u32*>(wv_lds + x.at + 32u);
-            if (len > 48u) d = *reinterpret_cast<const v4u32*>(wv_lds + x.at + 48u);
+            c = *reinterpret_cast<const v4u32*>(wv_lds + x.at2);
+            if (len > 48u) d = *reinterpret_cast<const v4u32*>(wv_lds + x.at2 + 16u);
           }
         }
         if (__any(far)) {
@@ -490,7 +547,7 @@ k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const u
         const bool valid = g + lane < g_end;
         const uint32_t mine_len = valid ? len + n_num : 0u;
         const uint32_t end = dpp_add(mine_len);
-        const bool now = valid && end + pend <= WV_TILE;
+        const bool now = valid && end + pend <= room;
         const uint32_t n = (uint32_t)__popcll(__ballot(now)); /* (never 0: a segment is shorter than the tile) */
         if (now) put_segment(tile, pend + (end - mine_len), len, x.a, b, c, d, n_num, x.num);
         pend += __builtin_amdgcn_readlane(end, n - 1u);
@@ -514,13 +571,15 @@ k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const u
 hipError_t weave_activities(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const uint8_t* kind_sorted, uint64_t n_most, EmitCtx ctx, char* out,
                  uint64_t prefix_len, const Scalars* sc, const SchemaBook* schemas, const WideText* wide, hipStream_t st) {
   if (n_most == 0) return hipSuccess;
-  static_assert(WV_TILE_ROOM / 16u <= 3u * 64u, "the tile leaves in three turns at most");
+  static_assert(WV_TILE_MOST / 16u <= 3u * 64u && WV_TILE_MOST + 128u <= WV_SPACE, "three turns, and a line behind them");
+  static_assert(WV_BOOK_BYTES + WV_WAVES * WV_WAVE_BYTES <= 32000u, "five workgroups per CU: 160 KB in pieces of 1280 bytes");
   const uint64_t turns = (n_most + WV_ROWS - 1) / WV_ROWS;
   const uint32_t waves = turns >= 256u * WV_WAVES ? WV_WAVES : turns <= 256u ? 1u : (uint32_t)((turns + 255u) / 256u);
-  /* Turns of a wavefront: all that run at a time end together, up to about 24 (fewer: the book is copied more often, 22 million
-   * records 3.62 ms with 6, 3.47 with 16, 3.42 with 24; more: the last are late, 3 million 460 us with 24, 529 with 32).  733 000
-   * records, whose turns make 12 for each: 136 us, with 4 141, with 8, one and a half times as many wavefronts as run, 150. */
-  const uint64_t at_once = 256u * 16u, times = (turns + at_once * 24u - 1u) / (at_once * 24u);
+  /* Turns of a wavefront: those of a pass that all wavefronts at once can take with up to forty each are dealt out to them (3 million
+   * records 37 each 400 us, 19 and twice as many wavefronts 407).  Of longer passes each takes about twelve: the fewer, the closer
+   * together lie the pieces of the document that are written at a time, but each copies the book (22 million records with 8, 12, 16,
+   * 24, 40: 3.09, 2.97, 3.00, 3.04, 3.04 ms; 5 million operators with long strings 2.45, 2.44, 2.52, 2.50, 2.51). */
+  const uint64_t at_once = 256u * 20u, times = turns <= at_once * 40u ? 1u : (turns + at_once * 12u - 1u) / (at_once * 12u);
   const uint32_t rounds = (uint32_t)((turns + at_once * times - 1u) / (at_once * times));
   const auto kernel = n_most >= WV_PAST_FROM ? k_weave<true> : k_weave<false>;
   hipLaunchKernelGGL(kernel, dim3(grid_for(turns, waves * rounds)), dim3(waves * 64u), WV_BOOK_BYTES + waves * WV_WAVE_BYTES, st, rows, perm, offs,
