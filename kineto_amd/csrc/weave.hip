@@ -267,9 +267,12 @@ k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const u
     q0 = r[h];                           /* S_Z, S_EXT, S_FLOW, S_DUR and plan, name, lens, more */
     q1 = r[4u + h];                      /* S_A and the track, S_TS, S_X, S_Y */
   };
-  uint32_t row = i_begin + act < i_end ? perm[i_begin + act] : 0u;
+  auto row_at = [&](uint64_t i) { return perm[i < i_end ? i : i_end - 1]; }; /* (with a condition on the load the next turn's rows were waited for as
+   * soon as they were asked for, where a register that the other way leaves as it is meets the one that is loaded: 22 million records 2.99 ms,
+   * now 2.85, 11 million kernels 1.62 and 1.52) */
+  uint32_t row = row_at(i_begin + act);
   load_row(row);
-  row = i_begin + WV_ROWS + act < i_end ? perm[i_begin + WV_ROWS + act] : 0u;
+  row = row_at(i_begin + WV_ROWS + act);
 
   uint32_t part = 0, pend = 0, own = 0;
   char* doc = nullptr;
@@ -400,10 +403,8 @@ k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const u
       if (h + 4u < q_units) *reinterpret_cast<v4u32*>(wv_lds + q_at + (h + 4u) * 16u) = ny;
     }
     /* the next turn's rows */
-    if (i0 + WV_ROWS < i_end) {
-      load_row(row);
-      row = i0 + 2u * WV_ROWS + act < i_end ? perm[i0 + 2u * WV_ROWS + act] : 0u;
-    }
+    load_row(row);
+    row = row_at(i0 + 2u * WV_ROWS + act);
 
     /* ---- neighbouring activities of a track ---- */
     if (open && !(ok_mask & 1u)) close_document(i0);
@@ -561,6 +562,7 @@ k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const u
         store_lines();
         put(x);
       }
+      asm volatile("" : "+v"(q0), "+v"(q1), "+v"(row)); /* the next turn's rows are waited for here, and not behind these lines' stores */
       store_lines();
       if (next_lane != 64u && !(todo & (1ull << next_lane))) close_document(i0 + (next_lane >> 2));
     }
