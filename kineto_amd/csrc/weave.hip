@@ -51,10 +51,14 @@ using namespace weave;
 #define WV_GAP 32u
 #define WV_TILE_MOST 3072u                            /* whole lines leave in three turns at most */
 #define WV_WAVE_BYTES (WV_TILE_AT + WV_SPACE)
-/* of the workgroup, in front of them: the texts, the book's and the schemas'; where the parts are, the schemas' behind the book's; descriptors */
+/* of the workgroup, in front of them: the texts, the book's and the schemas'; where the parts are: the book's, those of the schemas' args and
+ * an empty one, those of their args2 and an empty one; descriptors */
 #define WV_BOOK_REF ((LDS_BOOK.n_text + SCHEMA_TEXT) * 16u)
-#define WV_BOOK_PLANS (WV_BOOK_REF + (R_COUNT + 1u) / 2u * 4u)
-#define WV_BOOK_DESC (WV_BOOK_PLANS + MAX_SCHEMAS * 4u)
+#define WV_REF_SCHEMA R_COUNT
+#define WV_REF_SCHEMA2 (WV_REF_SCHEMA + MAX_SCHEMAS + 1u)
+#define WV_REF_EMPTY (WV_REF_SCHEMA + MAX_SCHEMAS)
+#define WV_REFS (WV_REF_SCHEMA2 + MAX_SCHEMAS + 1u)
+#define WV_BOOK_DESC (WV_BOOK_REF + (WV_REFS + 1u) / 2u * 4u)
 #define WV_BOOK_BYTES ((WV_BOOK_DESC + (MAX_DESC + SCHEMA_DESC) * 4u + 15u) / 16u * 16u)
 
 /* a part: first segment | kind << 15 (text, or one of the strings of S_RUN) | first descriptor << 17 | activity << 26 */
@@ -76,7 +80,7 @@ using namespace weave;
 #define WV_REF_COUNT(r) ((r) >> 9)
 struct LdsBook {
   uint32_t text[MAX_TEXT * 4], desc[MAX_DESC], n_text;
-  uint16_t ref[R_COUNT + 1u];
+  uint16_t ref[R_COUNT];
 };
 constexpr LdsBook make_lds_book() {
   LdsBook l{};
@@ -111,6 +115,14 @@ __device__ __forceinline__ uint32_t dpp_add(uint32_t v) { /* inclusive sum over 
   WV_DPP(0x111, 0xF); WV_DPP(0x112, 0xF); WV_DPP(0x114, 0xF); WV_DPP(0x118, 0xF);
   WV_DPP(0x142, 0xA); WV_DPP(0x143, 0xC);
 #undef WV_DPP
+  return v;
+}
+/* inclusive sum over the activities, four lanes to each that have the same */
+__device__ __forceinline__ uint32_t quad_add(uint32_t v) {
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xF, 0xF, false);
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xF, 0xF, false);
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xA, 0xF, false);
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xC, 0xF, false);
   return v;
 }
 __device__ __forceinline__ void wave_lds_order() {
@@ -160,11 +172,11 @@ __device__ __forceinline__ void put_segment(char* buf, uint32_t p, uint32_t len,
     if (len > 16u) {
       if (len > 32u) {
         if (len > 48u) { put_word(q + 64, WV_WORD(0u, d.w)); put_word(q + 60, WV_WORD(d.w, d.z)); put_word(q + 56, WV_WORD(d.z, d.y)); put_word(q + 52, WV_WORD(d.y, d.x)); }
-        put_word(q + 48, WV_WORD(d.x, c.w)); put_word(q + 44, WV_WORD(c.w, c.z)); put_word(q + 40, WV_WORD(c.z, c.y)); put_word(q + 36, WV_WORD(c.y, c.x));
+        put_word(q + 48, WV_WORD(len > 48u ? d.x : 0u, c.w)); put_word(q + 44, WV_WORD(c.w, c.z)); put_word(q + 40, WV_WORD(c.z, c.y)); put_word(q + 36, WV_WORD(c.y, c.x));
       }
-      put_word(q + 32, WV_WORD(c.x, b.w)); put_word(q + 28, WV_WORD(b.w, b.z)); put_word(q + 24, WV_WORD(b.z, b.y)); put_word(q + 20, WV_WORD(b.y, b.x));
+      put_word(q + 32, WV_WORD(len > 32u ? c.x : 0u, b.w)); put_word(q + 28, WV_WORD(b.w, b.z)); put_word(q + 24, WV_WORD(b.z, b.y)); put_word(q + 20, WV_WORD(b.y, b.x));
     }
-    put_word(q + 16, WV_WORD(b.x, a.w)); put_word(q + 12, WV_WORD(a.w, a.z)); put_word(q + 8, WV_WORD(a.z, a.y)); put_word(q + 4, WV_WORD(a.y, a.x));
+    put_word(q + 16, WV_WORD(len > 16u ? b.x : 0u, a.w)); put_word(q + 12, WV_WORD(a.w, a.z)); put_word(q + 8, WV_WORD(a.z, a.y)); put_word(q + 4, WV_WORD(a.y, a.x));
   }
   if (n_num) {
     const uint32_t p2 = p + len, sh = 0u - p2, upto = n_num + ((p2 - 1u) & 3u) + 1u; /* bytes from q2 on */
@@ -183,7 +195,8 @@ __device__ __forceinline__ void put_segment(char* buf, uint32_t p, uint32_t len,
   }
   or_shared_word(q, WV_WORD(a.x, 0u));
 }
-extern __shared__ __attribute__((aligned(16))) char wv_lds[];
+/* (of a fixed size, also where a workgroup has fewer wavefronts: its address is then a constant that the compiler folds) */
+#define WV_LDS_BYTES (WV_BOOK_BYTES + WV_WAVES * WV_WAVE_BYTES)
 /* the track's texts, with the lead of its times; their lengths, a byte each */
 __device__ __forceinline__ uint64_t make_track(char* lds, uint32_t mine, uint64_t dev, uint64_t thread, uint32_t lead) {
   const uint32_t lane = lane_id();
@@ -224,14 +237,18 @@ template <bool PAST>
 __global__ void __launch_bounds__(WV_WAVES * 64u) __attribute__((amdgpu_waves_per_eu(5)))
 k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const uint8_t* kind_sorted, EmitCtx ctx, char* out, uint64_t prefix_len,
         const Scalars* sc, uint32_t rounds, const SchemaBook* schemas, const WideText* wide) {
+  __shared__ __attribute__((aligned(16))) char wv_lds[WV_LDS_BYTES];
   if (sc->no_text) return;
   const uint32_t lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   for (uint32_t k = threadIdx.x; k < LDS_BOOK.n_text + SCHEMA_TEXT; k += blockDim.x)
     reinterpret_cast<uint4*>(wv_lds)[k] = k < LDS_BOOK.n_text ? reinterpret_cast<const uint4*>(g_book.text)[k] : reinterpret_cast<const uint4*>(schemas->text)[k - LDS_BOOK.n_text];
-  for (uint32_t k = threadIdx.x; k < R_COUNT; k += blockDim.x) reinterpret_cast<uint16_t*>(wv_lds + WV_BOOK_REF)[k] = g_book.ref[k];
-  if (threadIdx.x < MAX_SCHEMAS) {
-    const uint32_t a = schemas->plan[threadIdx.x].args, b = schemas->plan[threadIdx.x].args2;
-    reinterpret_cast<uint32_t*>(wv_lds + WV_BOOK_PLANS)[threadIdx.x] = WV_REF(KTJ_WREF_BASE(a), KTJ_WREF_COUNT(a)) | (WV_REF(KTJ_WREF_BASE(b), KTJ_WREF_COUNT(b)) << 16);
+  uint16_t* const refs = reinterpret_cast<uint16_t*>(wv_lds + WV_BOOK_REF);
+  for (uint32_t k = threadIdx.x; k < R_COUNT; k += blockDim.x) refs[k] = g_book.ref[k];
+  if (threadIdx.x <= MAX_SCHEMAS) {
+    const SchemaPlan* const p = schemas->plan + threadIdx.x;
+    const uint32_t a = threadIdx.x < MAX_SCHEMAS ? p->args : 0u, b = threadIdx.x < MAX_SCHEMAS ? p->args2 : 0u;
+    refs[WV_REF_SCHEMA + threadIdx.x] = (uint16_t)WV_REF(KTJ_WREF_BASE(a), KTJ_WREF_COUNT(a));
+    refs[WV_REF_SCHEMA2 + threadIdx.x] = (uint16_t)WV_REF(KTJ_WREF_BASE(b), KTJ_WREF_COUNT(b));
   }
   for (uint32_t k = threadIdx.x; k < MAX_DESC + SCHEMA_DESC; k += blockDim.x) {
     uint32_t d;
@@ -243,7 +260,6 @@ k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const u
     reinterpret_cast<uint32_t*>(wv_lds + WV_BOOK_DESC)[k] = d;
   }
   const uint32_t mine = WV_BOOK_BYTES + wave * WV_WAVE_BYTES; /* this wavefront's LDS */
-  const uint16_t* const refs = reinterpret_cast<const uint16_t*>(wv_lds + WV_BOOK_REF);
   uint32_t* const parts = reinterpret_cast<uint32_t*>(wv_lds + mine + WV_PARTS_AT);
   char* const tile = wv_lds + mine + WV_TILE_AT;
   __syncthreads();
@@ -252,6 +268,12 @@ k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const u
   typedef const __attribute__((address_space(1))) v4u32* gsrc;
 
   const uint32_t h = lane & 3u, act = lane >> 2;
+  /* which of an activity's parts the lane names, and where the plan says which they are: head, name, body and args, then the string between
+   * them, args2 and tail */
+  const uint32_t shift_a = h == 0u ? 0u : h == 1u ? 5u : h == 2u ? 12u : 14u, width_a = h == 0u ? 5u : h == 2u ? 2u : 7u;
+  const uint32_t base_a = h == 0u ? (uint32_t)R_HEAD : h == 1u ? 0u : h == 2u ? (uint32_t)R_BODY_NONE : (uint32_t)R_ARGS;
+  const uint32_t shift_b = h == 1u ? 14u : 21u, width_b = h == 1u ? 7u : h == 2u ? 4u : 0u;
+  const uint32_t base_b = h == 1u ? (uint32_t)R_ARGS2 : h == 2u ? (uint32_t)R_TAIL : (uint32_t)WV_REF_EMPTY;
   v2u64* const vals = reinterpret_cast<v2u64*>(wv_lds + mine + act * WV_VAL_BYTES);
   uint64_t track_made = ~0ull; /* what the track's texts are made of */
   uint32_t track_made_high = ~0u;
@@ -269,7 +291,7 @@ k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const u
   };
   auto row_at = [&](uint64_t i) { return perm[i < i_end ? i : i_end - 1]; }; /* (with a condition on the load the next turn's rows were waited for as
    * soon as they were asked for, where a register that the other way leaves as it is meets the one that is loaded: 22 million records 2.99 ms,
-   * now 2.85, 11 million kernels 1.62 and 1.52) */
+   * then 2.85, 11 million kernels 1.62 and 1.52) */
   uint32_t row = row_at(i_begin + act);
   load_row(row);
   row = row_at(i_begin + WV_ROWS + act);
@@ -304,16 +326,15 @@ k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const u
   for (uint64_t i0 = i_begin; i0 < i_end; i0 += WV_ROWS) {
     const bool active = i0 + act < i_end;
     /* rows that format_activity prints are another kernel's */
-    const uint64_t left_of = __ballot(!active || (h == 3u && (q1.w >> 24) == KTJ_ROW_LEFT));
+    const uint64_t left_of = __builtin_amdgcn_ballot_w64(!active || (h == 3u && (q1.w >> 24) == KTJ_ROW_LEFT));
     const uint64_t ok_mask = ~(left_of | (left_of >> 3)) & 0x1111111111111111ull; /* a bit at the first lane of each of the others */
     const bool mine_ok = (ok_mask >> (lane & ~3u)) & 1u;
 #define WV_QUAD(x, k) ((uint32_t)__builtin_amdgcn_mov_dpp((int)(x), (k) * 0x55, 0xF, 0xF, true)) /* the k-th lane's, for all four */
-    /* (the first lane's:) */
-    const uint32_t plan = q0.w, name_off = WV_QUAD(q0.w, KTJ_TR_NAME), lens = WV_QUAD(q0.w, KTJ_TR_LENS), more = WV_QUAD(q0.w, KTJ_TR_MORE);
-    const uint64_t track = (uint64_t)q1.z | ((uint64_t)q1.w << 32);
+    const uint32_t plan = WV_QUAD(q0.w, KTJ_TR_PLAN), name_off = WV_QUAD(q0.w, KTJ_TR_NAME), lens = WV_QUAD(q0.w, KTJ_TR_LENS), more = WV_QUAD(q0.w, KTJ_TR_MORE);
+    const uint32_t track_low = WV_QUAD(q1.z, 0), track_mid = WV_QUAD(q1.w, 0);
     /* the times' lead and the thread's upper bits */
     uint32_t track_high = KTJ_TR_TID_HIGH(plan);
-    if (__any((lens & KTJ_TR_HAS_LEAD) != 0)) {
+    if (__builtin_amdgcn_ballot_w64((lens & KTJ_TR_HAS_LEAD) != 0)) {
       uint32_t lead = KTJ_TR_LEAD_NIBBLE(q0.z) << (4u * h);
       lead |= (uint32_t)__builtin_amdgcn_mov_dpp((int)lead, 0xB1, 0xF, 0xF, true); /* the quad's: its lanes 1 0 3 2, then 2 3 0 1 */
       lead |= (uint32_t)__builtin_amdgcn_mov_dpp((int)lead, 0x4E, 0xF, 0xF, true);
@@ -322,72 +343,70 @@ k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const u
     /* activities whose track or lead is not that of the one before: a bit at the first lane of each */
     uint64_t new_track;
     {
-      uint64_t before = __shfl_up((unsigned long long)track, 4);
-      uint32_t before_high = __shfl_up(track_high, 4);
-      if (lane == 0u) { before = track_made; before_high = track_made_high; }
-      new_track = __ballot(h == 0u && (track != before || track_high != before_high));
+      /* the lane four before: the last of the row before for the first lanes of a row of sixteen, the wavefront's last activity's for the first of all */
+#define WV_BEFORE(x, first) ((uint32_t)__builtin_amdgcn_update_dpp(__builtin_amdgcn_update_dpp((int)(first), (int)(x), 0x142, 0xE, 0xF, false), (int)(x), 0x114, 0xF, 0xF, false))
+      const uint32_t low = WV_BEFORE(track_low, (uint32_t)track_made), mid = WV_BEFORE(track_mid, (uint32_t)(track_made >> 32)), high = WV_BEFORE(track_high, track_made_high);
+#undef WV_BEFORE
+      new_track = __builtin_amdgcn_ballot_w64(((track_low ^ low) | (track_mid ^ mid) | (track_high ^ high)) != 0u) & 0x1111111111111111ull;
     }
-    const v4u32 z = {q0.x, q0.y, q0.z & 0xFFFFFFu, KTJ_TR_COUNT(q0.z) << 24};
+    const v4u32 z = {q0.x, q0.y, q0.z & 0xFFFFFFu, q0.z & 0xF000000u};
     vals[S_Z - 1u + h] = __builtin_bit_cast(v2u64, z);
     {
       const uint32_t on = (q1.y >> 24) > KTJ_TR_A_NEAR ? more : 0u; /* (of the first lane) */
       const v4u32 a = {q1.x, (q1.y & 0xFFFFFFu) | (on << 24), on >> 8, q1.y & 0xFF000000u}, x = h == 0u ? a : q1;
       vals[S_A - 1u + h] = __builtin_bit_cast(v2u64, x);
     }
-    /* how many segments and parts, and the room for the name (the first lane) */
-    uint32_t counts = 0, units = 0, args_ref = 0, args2_ref = 0;
-    const uint32_t len0 = lens & 0xFFFFu, len1 = KTJ_TR_LEN1(lens);
-    if (h == 0u && mine_ok) {
-      const uint32_t a = KTJ_TR_ARGS(plan);
-      if (a >= KTJ_TR_SCHEMA) {
-        if (a != KTJ_TR_NO_ARGS) {
-          const uint32_t both = reinterpret_cast<const uint32_t*>(wv_lds + WV_BOOK_PLANS)[a - KTJ_TR_SCHEMA];
-          args_ref = both & 0xFFFFu; args2_ref = both >> 16;
-        }
-      } else { args_ref = refs[R_ARGS + a]; args2_ref = refs[R_ARGS2 + a]; }
-      const uint32_t name = KTJ_TR_NAMED(plan) != KTJ_TR_NAME_RUN ? WV_REF_COUNT(refs[KTJ_TR_NAMED(plan)]) : (len0 + KTJ_WEAVE_LIT - 1u) / KTJ_WEAVE_LIT;
-      const uint32_t runs = (len1 + KTJ_WEAVE_LIT - 1u) / KTJ_WEAVE_LIT;
-      const uint32_t head = WV_REF_COUNT(refs[R_HEAD + KTJ_TR_TYPE(plan)]), body = WV_REF_COUNT(refs[R_BODY_NONE + KTJ_TR_BODY(plan)]);
-      const uint32_t tail = WV_REF_COUNT(refs[R_TAIL + KTJ_TR_TAIL(plan)]);
-      const uint32_t args = WV_REF_COUNT(args_ref), args2 = WV_REF_COUNT(args2_ref);
-      counts = ((2u + (name ? 1u : 0u) + (args ? 1u : 0u) + (runs ? 1u : 0u) + (args2 ? 1u : 0u) + (tail ? 1u : 0u)) << 16) |
-               (head + name + body + args + runs + args2 + tail);
-      units = (len0 <= WV_NAME_MOST ? (len0 + 15u) / 16u : 0u) | (KTJ_TR_BETWEEN(plan) == 3u ? 2u << 16 : 0u);
+    const uint32_t len0 = lens & 0xFFFFu, len1 = KTJ_TR_LEN1(lens), between = KTJ_TR_BETWEEN(plan);
+    /* The parts: four lanes name an activity's, two each.  Sums over its lanes in front (segments and parts of the first four, of the others),
+     * then over the activities.  (By one lane of the four, one part after the other, each behind its own access to LDS, and a dozen
+     * instructions more per 64 segments: 22 million records 2.86 ms, now 2.82, 11 million kernels 1.53 and 1.49.) */
+    uint32_t before, upto;
+    {
+      uint32_t ref_a = __builtin_amdgcn_ubfe(plan, shift_a, width_a) + base_a, ref_b = __builtin_amdgcn_ubfe(plan, shift_b, width_b) + base_b;
+      const uint32_t args = KTJ_TR_ARGS(plan), schema = args - KTJ_TR_SCHEMA < MAX_SCHEMAS ? args - KTJ_TR_SCHEMA : MAX_SCHEMAS;
+      if (args >= KTJ_TR_SCHEMA && h == 3u) ref_a = WV_REF_SCHEMA + schema;
+      if (args >= KTJ_TR_SCHEMA && h == 1u) ref_b = WV_REF_SCHEMA2 + schema;
+      const uint32_t a = refs[ref_a], b = refs[ref_b];
+      uint32_t n_a = WV_REF_COUNT(a), n_b = WV_REF_COUNT(b), part_a = (WV_REF_BASE(a) << 17) | (act << 26), part_b = (WV_REF_BASE(b) << 17) | (act << 26);
+      if (h == 1u && KTJ_TR_NAMED(plan) == KTJ_TR_NAME_RUN) { n_a = (len0 + KTJ_WEAVE_LIT - 1u) / KTJ_WEAVE_LIT; part_a = (1u << 15) | (act << 26); }
+      if (h == 0u) { n_b = (len1 + KTJ_WEAVE_LIT - 1u) / KTJ_WEAVE_LIT; part_b = (2u << 15) | (act << 26); }
+      n_a = mine_ok ? n_a : 0u; n_b = mine_ok ? n_b : 0u;
+      static_assert((KTJ_WEAVE_MAX_RUN + KTJ_WEAVE_LIT - 1u) / KTJ_WEAVE_LIT + 127u * 2u < 1024u, "ten bits for an activity's segments on either side");
+      const uint32_t c = n_a | ((n_a ? 1u : 0u) << 10) | (n_b << 13) | ((n_b ? 1u : 0u) << 23);
+      uint32_t in_front = (uint32_t)__builtin_amdgcn_mov_dpp((int)c, 0x90, 0xF, 0xF, true);              /* lanes 0 0 1 2 */
+      in_front = h >= 1u ? in_front : 0u;
+      const uint32_t two = in_front + (uint32_t)__builtin_amdgcn_mov_dpp((int)in_front, 0x90, 0xF, 0xF, true);
+      in_front += (uint32_t)__builtin_amdgcn_mov_dpp((int)two, 0x90, 0xF, 0xF, true);                  /* of the lanes before: none, one, two, three */
+      const uint32_t all = WV_QUAD(in_front + c, 3);
+      const uint32_t first_segs = all & 0x3FFu, first_parts = (all >> 10) & 7u;
+      const uint32_t total = (first_segs + ((all >> 13) & 0x3FFu)) | ((first_parts + (all >> 23)) << 16);
+      upto = quad_add(total);
+      before = upto - total;
+      const uint32_t segs = before & 0xFFFFu, n_parts = before >> 16;
+      if (n_a) parts[n_parts + ((in_front >> 10) & 7u)] = part_a | (segs + (in_front & 0x3FFu)); /* (segments stay below their 15 bits) */
+      if (n_b) parts[n_parts + first_parts + (in_front >> 23)] = part_b | (segs + first_segs + ((in_front >> 13) & 0x3FFu));
     }
-    const uint32_t upto = dpp_add(counts), before = upto - counts; /* of the first lane of each */
     /* the strings in LDS: wide texts, two units each, and names as far as there is room */
     static_assert(WV_ROWS * sizeof(WideText) <= WV_NAMES && sizeof(WideText) == 32, "the wide texts have room");
-    const uint32_t units_upto = dpp_add(units), double_at = WV_WAVE_BYTES - (units_upto >> 16) * 16u;
+    const bool is_wide = mine_ok && between == 3u;
+    const uint32_t name_units = mine_ok && len0 <= WV_NAME_MOST ? (len0 + 15u) / 16u : 0u;
+    const uint32_t units_upto = quad_add(name_units | (is_wide ? 2u << 16 : 0u));
     const uint32_t wide_units = __builtin_amdgcn_readlane(units_upto, 63) >> 16, name_upto = (units_upto & 0xFFFFu) + wide_units;
-    units &= 0xFFFFu;
-    const bool near = units != 0 && name_upto <= WV_NAMES / 16u;
-    const uint32_t name_at = WV_WAVE_BYTES - name_upto * 16u;
+    const bool near = name_units != 0 && name_upto <= WV_NAMES / 16u;
+    const uint32_t double_at = WV_WAVE_BYTES - (units_upto >> 16) * 16u, name_at = WV_WAVE_BYTES - name_upto * 16u;
     /* what they leave of the space (the last of the names that are there says it) */
-    const uint64_t near_ones = __ballot(near);
-    const uint32_t taken = (near_ones ? __builtin_amdgcn_readlane(name_upto, 63u - (uint32_t)__clzll((long long)near_ones)) : wide_units) * 16u + WV_GAP;
+    const uint64_t near_ones = __builtin_amdgcn_ballot_w64(near);
+    const uint32_t taken = (near_ones ? __builtin_amdgcn_readlane(name_upto, 63u - (uint32_t)__builtin_clzll(near_ones)) : wide_units) * 16u + WV_GAP;
     const uint32_t room = WV_SPACE - taken < WV_TILE_MOST ? WV_SPACE - taken : WV_TILE_MOST;
     v4u32 nx, ny, wx;
-    const uint32_t wide_at = WV_QUAD(counts != 0 && KTJ_TR_BETWEEN(plan) == 3u ? mine + double_at : 0u, 0);
-    if (h < 2u && wide_at) wx = reinterpret_cast<gsrc>((uint64_t)(uintptr_t)wide + (uint64_t)more * sizeof(WideText))[h];
-    const uint32_t q_units = WV_QUAD(near ? units : 0u, 0), q_at = mine + WV_QUAD(name_at, 0);
+    const bool load_wide = is_wide && h < 2u, load_x = near && h < name_units, load_y = near && h + 4u < name_units;
+    if (load_wide) wx = reinterpret_cast<gsrc>((uint64_t)(uintptr_t)wide + (uint64_t)more * sizeof(WideText))[h];
     {
       const gsrc src = reinterpret_cast<gsrc>((uint64_t)(uintptr_t)ctx.dict.name_blob + (uint64_t)name_off * 16u);
-      if (h < q_units) { nx = src[h]; if (h + 4u < q_units) ny = src[h + 4u]; }
+      if (load_x) { nx = src[h]; if (load_y) ny = src[h + 4u]; }
     }
 #undef WV_QUAD
-    if (counts) {
-      uint32_t* w = parts + (before >> 16);
-      uint32_t seg = (before & 0x7FFFu) | (act << 26); /* (segments stay below their 15 bits) */
-      auto put_part = [&](uint32_t ref) { const uint32_t n = WV_REF_COUNT(ref); if (n) { *w++ = seg | (WV_REF_BASE(ref) << 17); seg += n; } };
-      put_part(refs[R_HEAD + KTJ_TR_TYPE(plan)]);
-      if (KTJ_TR_NAMED(plan) != KTJ_TR_NAME_RUN) put_part(refs[KTJ_TR_NAMED(plan)]);
-      else if (len0) { *w++ = seg | (1u << 15); seg += (len0 + KTJ_WEAVE_LIT - 1u) / KTJ_WEAVE_LIT; }
-      put_part(refs[R_BODY_NONE + KTJ_TR_BODY(plan)]);
-      put_part(args_ref);
-      if (len1) { *w++ = seg | (2u << 15); seg += (len1 + KTJ_WEAVE_LIT - 1u) / KTJ_WEAVE_LIT; }
-      put_part(args2_ref);
-      put_part(refs[R_TAIL + KTJ_TR_TAIL(plan)]);
-      const uint32_t between = KTJ_TR_BETWEEN(plan);
+    if (h == 0u && mine_ok) {
       const uint32_t at = between < 2u ? 0u : between == 2u ? act * WV_VAL_BYTES + WV_VAL(S_Y) : double_at;
       v4u32 runs;
       runs.x = more; runs.y = len1 | (at << 16);
@@ -395,12 +414,11 @@ k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const u
       runs.z = name_off; runs.w = len0 | ((near ? name_at : 0u) << 16);
       vals[S_RUN - 1u] = __builtin_bit_cast(v2u64, runs);
     }
-    const uint32_t totals = __builtin_amdgcn_readlane(upto, 63);
-    if (lane == 0) parts[totals >> 16] = totals & 0x7FFFu;
-    if (h < 2u && wide_at) *reinterpret_cast<v4u32*>(wv_lds + wide_at + h * 16u) = wx;
-    if (h < q_units) {
-      *reinterpret_cast<v4u32*>(wv_lds + q_at + h * 16u) = nx;
-      if (h + 4u < q_units) *reinterpret_cast<v4u32*>(wv_lds + q_at + (h + 4u) * 16u) = ny;
+    const uint32_t n_parts = __builtin_amdgcn_readlane(upto, 63) >> 16;
+    if (load_wide) *reinterpret_cast<v4u32*>(wv_lds + mine + double_at + h * 16u) = wx;
+    if (load_x) {
+      *reinterpret_cast<v4u32*>(wv_lds + mine + name_at + h * 16u) = nx;
+      if (load_y) *reinterpret_cast<v4u32*>(wv_lds + mine + name_at + (h + 4u) * 16u) = ny;
     }
     /* the next turn's rows */
     load_row(row);
@@ -420,7 +438,7 @@ k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const u
       part = __builtin_amdgcn_readlane(before, first) >> 16;
       const uint64_t upto_first = first >= 60u ? ~0ull : (1ull << (first + 4u)) - 1ull;
       if (new_track & upto_first & ~track_seen) {
-        const uint32_t low = __builtin_amdgcn_readlane((uint32_t)track, first), high = __builtin_amdgcn_readlane((uint32_t)(track >> 32), first);
+        const uint32_t low = __builtin_amdgcn_readlane(track_low, first), high = __builtin_amdgcn_readlane(track_mid, first);
         track_made_high = (uint32_t)__builtin_amdgcn_readlane(track_high, first);
         track_made = (uint64_t)low | ((uint64_t)high << 32);
         track_lens = make_track(wv_lds, mine, low & ((1u << KTJ_TR_DEV_BITS) - 1u), (track_made >> KTJ_TR_DEV_BITS) | ((uint64_t)(track_made_high & 31u) << 42), track_made_high >> 5);
@@ -455,15 +473,16 @@ k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const u
       uint32_t part_after = 0;
       auto fetch = [&]() {
         Piece x;
-        /* which part each segment belongs to: a part's first segment is marked, the marks counted */
-        const uint32_t rel = WV_PART_START(parts[part + lane]) - g; /* (behind the last part: what lies there, which does not count) */
-        const bool inside = part + lane <= (totals >> 16) && rel - 1u < 64u;
-        const uint64_t marks = __ballot(__builtin_amdgcn_ds_permute((int)(inside && rel < 64u ? rel * 4u : 0u), 1) != 0);
+        /* which part each segment belongs to: the first segments of the parts behind this one are marked, the marks counted (one that
+         * is 64 behind marks the first, which does not count, like the sixty-fifth it is) */
+        const uint32_t rel = WV_PART_START(parts[part + 1u + lane]) - g;
+        const bool follows = lane < n_parts - 1u - part && rel <= 64u;
+        const uint64_t marks = __builtin_amdgcn_ballot_w64(__builtin_amdgcn_ds_permute((int)(follows ? rel * 4u : 0u), 1) != 0);
         const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(marks >> 33), __builtin_amdgcn_mbcnt_lo((uint32_t)(marks >> 1), 0u));
         x.part = part + rank;
         uint32_t pr = parts[x.part];
-        part_after = part + (uint32_t)__popcll(__ballot(inside && rel <= g_end - g)); /* (the next activities' are theirs) */
-        const bool valid = g + lane < g_end;
+        part_after = part + (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(follows));
+        const bool valid = lane < g_end - g;
         const uint32_t seg = g + lane - WV_PART_START(pr);
         if (!valid) pr = 0;
         const uint32_t kind = WV_PART_KIND(pr), vrow = mine + WV_PART_ACT(pr) * WV_VAL_BYTES;
@@ -479,14 +498,17 @@ k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const u
         if (kind != 0) {
           const uint64_t r = *reinterpret_cast<const uint64_t*>(wv_lds + vrow + WV_VAL(S_RUN) + (2u - kind) * 8u);
           const uint32_t rest = ((uint32_t)(r >> 32) & 0xFFFFu) - seg * KTJ_WEAVE_LIT, near = (uint32_t)(r >> 48);
-          x.at = near ? mine + near + seg * KTJ_WEAVE_LIT : (uint32_t)r + seg * (KTJ_WEAVE_LIT / 16u);
+          x.at = (near ? mine + near : (uint32_t)r) + (seg << (near ? 6u : 2u));
           x.at2 = x.at + 32u;
           x.desc = WV_WD(rest < KTJ_WEAVE_LIT ? rest : KTJ_WEAVE_LIT, S_NONE, 0u, 0u) | (near ? 0u : kind == 1u ? WV_FAR : WV_FAR | WV_FAR_ARG);
         }
         x.a = *reinterpret_cast<const v4u32*>(wv_lds + (x.desc & WV_FAR ? 0u : x.at));
         const uint32_t slot = WV_WD_SLOT(x.desc);
-        x.num = *reinterpret_cast<const v4u32*>(wv_lds + vrow + (slot == S_K ? WV_VAL(S_RUN) : WV_VAL(slot))); /* (S_NONE: what lies there, which does not count) */
-        if (slot == S_K) { x.num.w = x.num.y; x.num.y = 0; x.num.z = 0; }
+        x.num = *reinterpret_cast<const v4u32*>(wv_lds + vrow + slot * 16u - 16u); /* (S_NONE: what lies there, which does not count) */
+        if (__builtin_amdgcn_ballot_w64(slot == S_K) && slot == S_K) { /* in the place of S_RUN */
+          x.num = *reinterpret_cast<const v4u32*>(wv_lds + vrow + WV_VAL(S_RUN));
+          x.num.w = x.num.y; x.num.y = 0; x.num.z = 0;
+        }
         if (slot == S_NONE) x.num.w = 0;
         return x;
       };
@@ -525,7 +547,7 @@ k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const u
       auto put = [&](Piece& x) {
         const uint32_t len = WV_WD_LEN(x.desc);
         const bool far = (x.desc & WV_FAR) != 0;
-        v4u32 b = {0, 0, 0, 0}, c = b, d = b;
+        v4u32 b, c, d; /* (what a text does not reach does not count) */
         if (len > 16u && !far) {
           b = *reinterpret_cast<const v4u32*>(wv_lds + x.at + 16u);
           if (len > 32u) {
@@ -533,7 +555,7 @@ k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const u
             if (len > 48u) d = *reinterpret_cast<const v4u32*>(wv_lds + x.at2 + 16u);
           }
         }
-        if (__any(far)) {
+        if (__builtin_amdgcn_ballot_w64(far)) {
           if (far) {
             const gsrc src = reinterpret_cast<gsrc>((uint64_t)(uintptr_t)(x.desc & WV_FAR_ARG ? ctx.dict.arg_blob : ctx.dict.name_blob)) + x.at;
             x.a = src[0];
@@ -545,11 +567,11 @@ k_weave(const TextRow* rows, const uint32_t* perm, const uint64_t* offs, const u
         }
         const uint32_t n_num = x.num.w >> 24;
         x.num.w &= 0xFFFFFFu;
-        const bool valid = g + lane < g_end;
+        const bool valid = lane < g_end - g;
         const uint32_t mine_len = valid ? len + n_num : 0u;
         const uint32_t end = dpp_add(mine_len);
         const bool now = valid && end + pend <= room;
-        const uint32_t n = (uint32_t)__popcll(__ballot(now)); /* (never 0: a segment is shorter than the tile) */
+        const uint32_t n = (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(now)); /* (never 0: a segment is shorter than the tile) */
         if (now) put_segment(tile, pend + (end - mine_len), len, x.a, b, c, d, n_num, x.num);
         pend += __builtin_amdgcn_readlane(end, n - 1u);
         wave_lds_order();
@@ -574,7 +596,7 @@ hipError_t weave_activities(const TextRow* rows, const uint32_t* perm, const uin
                  uint64_t prefix_len, const Scalars* sc, const SchemaBook* schemas, const WideText* wide, hipStream_t st) {
   if (n_most == 0) return hipSuccess;
   static_assert(WV_TILE_MOST / 16u <= 3u * 64u && WV_TILE_MOST + 128u <= WV_SPACE, "three turns, and a line behind them");
-  static_assert(WV_BOOK_BYTES + WV_WAVES * WV_WAVE_BYTES <= 32000u, "five workgroups per CU: 160 KB in pieces of 1280 bytes");
+  static_assert(WV_LDS_BYTES <= 32000u, "five workgroups per CU: 160 KB in pieces of 1280 bytes");
   const uint64_t turns = (n_most + WV_ROWS - 1) / WV_ROWS;
   const uint32_t waves = turns >= 256u * WV_WAVES ? WV_WAVES : turns <= 256u ? 1u : (uint32_t)((turns + 255u) / 256u);
   /* Turns of a wavefront: those of a pass that all wavefronts at once can take with up to forty each are dealt out to them (3 million
@@ -584,7 +606,7 @@ hipError_t weave_activities(const TextRow* rows, const uint32_t* perm, const uin
   const uint64_t at_once = 256u * 20u, times = turns <= at_once * 40u ? 1u : (turns + at_once * 12u - 1u) / (at_once * 12u);
   const uint32_t rounds = (uint32_t)((turns + at_once * times - 1u) / (at_once * times));
   const auto kernel = n_most >= WV_PAST_FROM ? k_weave<true> : k_weave<false>;
-  hipLaunchKernelGGL(kernel, dim3(grid_for(turns, waves * rounds)), dim3(waves * 64u), WV_BOOK_BYTES + waves * WV_WAVE_BYTES, st, rows, perm, offs,
+  hipLaunchKernelGGL(kernel, dim3(grid_for(turns, waves * rounds)), dim3(waves * 64u), 0, st, rows, perm, offs,
                      kind_sorted, ctx, out, prefix_len, sc, rounds, schemas, wide);
   return KTJ_LAUNCH_CHECK();
 }
