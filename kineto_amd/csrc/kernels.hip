@@ -93,14 +93,17 @@ struct ProbeSeq {
   __device__ __forceinline__ uint32_t slot(uint32_t mask) const { return ((run << 4) | low) & mask; }
   __device__ __forceinline__ void next() { run += step; }
 };
+/* A table as its plan has it, read once: the stores of a pass over rows would have it read again for each (11 million kernels: links 388 -> 373 us). */
+struct TableView { uint64_t* keys; uint32_t mask, keyed_direct, direct; uint64_t base, span; };
+__device__ __forceinline__ TableView view(const Table& t) { return TableView{t.keys, t.mask, t.keyed_direct, t.ctl->direct, t.ctl->base, t.ctl->span}; }
 /* Returns the slot of `key`, inserting it if absent; KTJ_NOSLOT when the table is full (hash
  * mode) or the key lies outside the planned range (direct mode; cannot happen for keys that were
  * part of the range computation). */
-__device__ uint32_t slot_insert(const Table& t, uint64_t key) {
-  if (t.ctl->direct) {
+__device__ uint32_t slot_insert(const TableView& t, uint64_t key) {
+  if (t.direct) {
     if (t.keyed_direct && key == KTJ_EMPTY_KEY) { t.keys[t.mask + 1u] = 0; return t.mask + 1u; }
-    const uint64_t idx = key - t.ctl->base;
-    if (idx > t.ctl->span) return KTJ_NOSLOT;
+    const uint64_t idx = key - t.base;
+    if (idx > t.span) return KTJ_NOSLOT;
     if (t.keyed_direct && t.keys[idx] != key) t.keys[idx] = key; /* every writer stores the same value */
     return (uint32_t)idx;
   }
@@ -120,11 +123,11 @@ __device__ uint32_t slot_insert(const Table& t, uint64_t key) {
 }
 /* In direct mode without stored keys every id inside the range has a slot; one that was never
  * inserted reads as empty per-slot values. */
-__device__ uint32_t slot_find(const Table& t, uint64_t key) {
-  if (t.ctl->direct) {
+__device__ uint32_t slot_find(const TableView& t, uint64_t key) {
+  if (t.direct) {
     if (t.keyed_direct && key == KTJ_EMPTY_KEY) return t.keys[t.mask + 1u] == 0 ? t.mask + 1u : KTJ_NOSLOT;
-    const uint64_t idx = key - t.ctl->base;
-    if (idx > t.ctl->span) return KTJ_NOSLOT;
+    const uint64_t idx = key - t.base;
+    if (idx > t.span) return KTJ_NOSLOT;
     if (t.keyed_direct && t.keys[idx] != key) return KTJ_NOSLOT;
     return (uint32_t)idx;
   }
@@ -138,6 +141,9 @@ __device__ uint32_t slot_find(const Table& t, uint64_t key) {
   }
   return KTJ_NOSLOT;
 }
+
+__device__ __forceinline__ uint32_t slot_insert(const Table& t, uint64_t key) { return slot_insert(view(t), key); }
+__device__ __forceinline__ uint32_t slot_find(const Table& t, uint64_t key) { return slot_find(view(t), key); }
 
 /* Sums a per-thread count over the workgroup and adds it to a global counter with one atomic per
  * workgroup (a single hot address serialises atomics in L2, so they must be rare).  Must be
@@ -421,7 +427,12 @@ __device__ __forceinline__ const Rec* stage_records(const Rec* recs, uint64_t ba
   constexpr uint32_t U = sizeof(Rec) / 16;
   const uint32_t cnt = (uint32_t)((n - base) < KTJ_BLOCK ? (n - base) : KTJ_BLOCK);
   const uint4* g = reinterpret_cast<const uint4*>(recs + base);
-  for (uint32_t i = threadIdx.x; i < cnt * U; i += KTJ_BLOCK) stage[i] = g[i];
+  const uint32_t last = cnt * U - 1u;
+  uint4 x[U];
+#pragma unroll
+  for (uint32_t k = 0; k < U; ++k) { const uint32_t i = threadIdx.x + k * KTJ_BLOCK; x[k] = g[i < last ? i : last]; }
+#pragma unroll
+  for (uint32_t k = 0; k < U; ++k) { const uint32_t i = threadIdx.x + k * KTJ_BLOCK; stage[i < last ? i : last] = x[k]; }
   __syncthreads();
   *n_here = cnt;
   return reinterpret_cast<const Rec*>(stage);
@@ -619,8 +630,9 @@ __device__ __forceinline__ void resolved_external(uint64_t ext_id, const Table& 
  * records share a correlation id, which the returning atomicMax tells; only otherwise
  * k_resolve_external lets the winners write again.  The CPU-op ids are in their table already, the
  * table was cleared, and the runtime rows come later. */
-__global__ void k_build_extcorr(const ktj_extcorr_rec* e, uint64_t n, Table tn, NarrowCols nc, Table cpu, const uint32_t* cpu_row,
+__global__ void k_build_extcorr(const ktj_extcorr_rec* e, uint64_t n, Table tn_planned, NarrowCols nc, Table cpu, const uint32_t* cpu_row,
                                 const ktj_generic_rec* g, EmitCtx ctx, Scalars* sc) {
+  const TableView tn = view(tn_planned);
   const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   bool repeats = false;
   if (i < n) {
@@ -643,7 +655,8 @@ __global__ void k_build_extcorr(const ktj_extcorr_rec* e, uint64_t n, Table tn, 
 /* activityMap_[act->correlationId()] = act: GenericActivityProfiler.cpp:262 */
 /* cpu_row (optional): per slot, 1 + index of the last record with that id, for the traces whose
  * CPU ops hand collective metadata to the kernels linked to them */
-__global__ void k_build_cpu_ids(const ktj_generic_rec* g, uint64_t n, Table cpu, uint32_t* cpu_row, Scalars* sc) {
+__global__ void k_build_cpu_ids(const ktj_generic_rec* g, uint64_t n, Table cpu_planned, uint32_t* cpu_row, Scalars* sc) {
+  const TableView cpu = view(cpu_planned);
   const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const uint32_t slot = slot_insert(cpu, (uint64_t)(int64_t)load_once(&g[i].id));
@@ -676,8 +689,9 @@ __global__ void k_resolve_external(const ktj_extcorr_rec* e, uint64_t n, Table t
  * array of first rows is only touched for ids that no runtime row has: in-window device rows take part in "first seen" there and are
  * checked afterwards by k_after_link.  Rows outside the window still take a stream from the
  * slot (slots with a stream come from runtime rows and exist already). */
-__global__ void k_link_device(uint64_t n, Columns c, uint64_t first_device, Table tf, FullCols fc, Table tn, NarrowCols nc,
+__global__ void k_link_device(uint64_t n, Columns c, uint64_t first_device, Table tf_planned, FullCols fc, Table tn_planned, NarrowCols nc,
                               DevLink* link, unsigned long long* orphans, Scalars* sc) {
+  const TableView tf = view(tf_planned), tn = view(tn_planned);
   uint32_t n_linked = 0, n_bad = 0, n_unresolved = 0, n_orphans = 0;
   const bool have_stream_src = sc->have_stream_src != 0;
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) {
@@ -2363,21 +2377,31 @@ __device__ __forceinline__ void store_row(MatRow* dst, const MatRow& m) {
  * row touches a cache line (or two) of its own with every 16-byte access, 64 lines per
  * instruction; moved by the workgroup with lane-consecutive 16-byte accesses the same bytes are
  * whole lines.  `rows` is the workgroup's first row, `cnt` its number of rows; the callers put
- * the barriers.  Records are read once and joined rows written once: both go past the L2's usual
- * replacement (config 3: join stage 2.51 -> 2.26 ms). */
+ * the barriers (workgroups of KTJ_BLOCK).  Records are read once and joined rows written once: both go past the L2's usual
+ * replacement (config 3: join stage 2.51 -> 2.26 ms).
+ * All loads of a group are asked for before any is waited for, those behind the last row again for its last block: in a loop of a
+ * length that the compiler does not know each was waited for and stored before the next, six trips to memory one after the other for the
+ * largest records (22 million records: rows 697 -> 600 us, join 1970 -> 1880, decode 486 -> 466; 5 million operators: rows 462 -> 397). */
 template <typename T>
 __device__ __forceinline__ void rows_global_to_lds(const T* rows, uint32_t cnt, uint4* lds) {
   typedef unsigned int v4u __attribute__((ext_vector_type(4)));
   const v4u* g = reinterpret_cast<const v4u*>(rows);
   v4u* l = reinterpret_cast<v4u*>(lds);
-  for (uint32_t k = threadIdx.x; k < cnt * (uint32_t)(sizeof(T) / 16); k += blockDim.x) l[k] = load_once(&g[k]);
+  constexpr uint32_t U = sizeof(T) / 16;
+  const uint32_t last = cnt * U - 1u;
+  v4u x[U];
+#pragma unroll
+  for (uint32_t k = 0; k < U; ++k) { const uint32_t i = threadIdx.x + k * KTJ_BLOCK; x[k] = load_once(&g[i < last ? i : last]); }
+#pragma unroll
+  for (uint32_t k = 0; k < U; ++k) { const uint32_t i = threadIdx.x + k * KTJ_BLOCK; l[i < last ? i : last] = x[k]; }
 }
 template <typename T>
 __device__ __forceinline__ void rows_lds_to_global(T* rows, uint32_t cnt, const uint4* lds) {
   typedef unsigned int v4u __attribute__((ext_vector_type(4)));
   v4u* g = reinterpret_cast<v4u*>(rows);
   const v4u* l = reinterpret_cast<const v4u*>(lds);
-  for (uint32_t k = threadIdx.x; k < cnt * (uint32_t)(sizeof(T) / 16); k += blockDim.x) store_once(&g[k], l[k]);
+#pragma unroll
+  for (uint32_t u = 0; u < (uint32_t)(sizeof(T) / 16); ++u) { const uint32_t k = threadIdx.x + u * KTJ_BLOCK; if (k < cnt * (uint32_t)(sizeof(T) / 16)) store_once(&g[k], l[k]); }
 }
 /* rows that are a line of eight blocks, block b of row r at b ^ (r & 7): neighbouring lanes write theirs to other banks */
 template <>
@@ -2385,7 +2409,8 @@ __device__ __forceinline__ void rows_lds_to_global(weave::TextRow* rows, uint32_
   typedef unsigned int v4u __attribute__((ext_vector_type(4)));
   v4u* g = reinterpret_cast<v4u*>(rows);
   const v4u* l = reinterpret_cast<const v4u*>(lds);
-  for (uint32_t k = threadIdx.x; k < cnt * 8u; k += blockDim.x) store_once(&g[k], l[k ^ ((k >> 3) & 7u)]);
+#pragma unroll
+  for (uint32_t u = 0; u < 8u; ++u) { const uint32_t k = threadIdx.x + u * KTJ_BLOCK; if (k < cnt * 8u) store_once(&g[k], l[k ^ ((k >> 3) & 7u)]); }
 }
 template <typename T>
 __device__ __forceinline__ T row_from_lds(const uint4* lds) {
@@ -2566,9 +2591,10 @@ __device__ __forceinline__ bool bitmap_test_and_set(uint32_t* bitmap, uint32_t s
 #define KX_JOIN_ATTR
 #endif
 template <bool TEXT>
-__global__ void KX_JOIN_ATTR k_join_runtime(const ktj_runtime_rec* r, uint64_t n, Columns c, uint64_t first_runtime, ApiTable api, Table tf,
-                               FullCols fc, Table tn, NarrowCols nc, uint32_t* slot_f, uint32_t* slot_n, ClockDev clk, EmitCtx ctx, Rows rows,
+__global__ void KX_JOIN_ATTR k_join_runtime(const ktj_runtime_rec* r, uint64_t n, Columns c, uint64_t first_runtime, ApiTable api, Table tf_planned,
+                               FullCols fc, Table tn_planned, NarrowCols nc, uint32_t* slot_f, uint32_t* slot_n, ClockDev clk, EmitCtx ctx, Rows rows,
                                uint32_t* len, Scalars* sc, int rounds) {
+  const TableView tf = view(tf_planned), tn = view(tn_planned);
   RowStats rs;
   uint32_t n_linked = 0;
   bool any_carries_stream = false, any_repeats = false;
@@ -2580,9 +2606,6 @@ __global__ void KX_JOIN_ATTR k_join_runtime(const ktj_runtime_rec* r, uint64_t n
     const uint64_t base = ((uint64_t)blockIdx.x * rounds + round) * blockDim.x;
     if (base >= n) break;
     const uint32_t cnt = (uint32_t)(n - base < blockDim.x ? n - base : blockDim.x);
-    __syncthreads(); /* the previous round's rows have left the staging area */
-    rows_global_to_lds(r + base, cnt, stage);
-    __syncthreads();
     const uint64_t i = base + threadIdx.x;
     bool carries_stream = false;
     uint32_t sf = KTJ_NOSLOT;
@@ -2590,6 +2613,11 @@ __global__ void KX_JOIN_ATTR k_join_runtime(const ktj_runtime_rec* r, uint64_t n
     /* everything the row reads from its own record and columns is requested up front, so that the
      * table accesses below (each a round trip of its own) overlap with it */
     const uint64_t a = first_runtime + (i < n ? i : 0);
+    const uint32_t meta_of = load_once(&c.meta[a]);
+    const int64_t ts_of = load_once(&c.ts[a]);
+    __syncthreads(); /* the previous round's rows have left the staging area */
+    rows_global_to_lds(r + base, cnt, stage);
+    __syncthreads();
     /* the lane's record stays in LDS and is read field by field; the joined row takes its place */
     uint4* my_slot = &stage[threadIdx.x * (sizeof(ktj_runtime_rec) / 16)];
     const ktj_runtime_rec& rec = *reinterpret_cast<const ktj_runtime_rec*>(my_slot);
@@ -2598,8 +2626,8 @@ __global__ void KX_JOIN_ATTR k_join_runtime(const ktj_runtime_rec* r, uint64_t n
     int64_t ts = 0, dur = 0;
     if (i < n) {
       id = rec.id;
-      meta = load_once(&c.meta[a]);
-      ts = load_once(&c.ts[a]);
+      meta = meta_of;
+      ts = ts_of;
       sf = slot_insert(tf, id);
     }
     const uint32_t kind = (meta & KTJ_M_KIND_MASK) >> KTJ_M_KIND_SHIFT;
@@ -2737,25 +2765,27 @@ __device__ __forceinline__ void mat_device_block(const ktj_device_rec* d, uint64
   RowStats rs;
   for (uint64_t base = block * KTJ_BLOCK; base < n; base += blocks * KTJ_BLOCK) {
     const uint32_t cnt = (uint32_t)(n - base < KTJ_BLOCK ? n - base : KTJ_BLOCK);
+    const uint64_t i = base + (threadIdx.x < cnt ? threadIdx.x : 0u), a = first + i;
+    const bool active = threadIdx.x < cnt;
+    MatRow m;
+    DevLink l; /* (the columns and the link are on their way with the records) */
+    {
+      typedef unsigned int v4u __attribute__((ext_vector_type(4)));
+      const v4u* src = reinterpret_cast<const v4u*>(&link[i]);
+      v4u* lv = reinterpret_cast<v4u*>(&l);
+      lv[0] = load_once(&src[0]);
+      lv[1] = load_once(&src[1]);
+    }
+    const int64_t ts = load_once(&c.ts[a]), res = load_once(&c.res[a]);
+    const uint32_t meta = load_once(&c.meta[a]);
+    const int32_t ext = load_once(&c.ext[a]);
     __syncthreads(); /* the previous round's rows have left the staging area */
     rows_global_to_lds(d + base, cnt, stage);
     __syncthreads();
-    const uint64_t i = base + threadIdx.x, a = first + i;
-    const bool active = threadIdx.x < cnt;
-    MatRow m;
     if (active) {
       const ktj_device_rec rec = row_from_lds<ktj_device_rec>(stage);
-      DevLink l;
-      {
-        typedef unsigned int v4u __attribute__((ext_vector_type(4)));
-        const v4u* src = reinterpret_cast<const v4u*>(&link[i]);
-        v4u* lv = reinterpret_cast<v4u*>(&l);
-        lv[0] = load_once(&src[0]);
-        lv[1] = load_once(&src[1]);
-      }
-      const int64_t ts = load_once(&c.ts[a]);
-      m = mat_device_v(rec, ts, duration_from(clk, clk.device_mode, ts, rec.end), load_once(&c.res[a]),
-                       (load_once(&c.meta[a]) & KTJ_M_VALID) != 0, load_once(&c.ext[a]),
+      m = mat_device_v(rec, ts, duration_from(clk, clk.device_mode, ts, rec.end), res,
+                       (meta & KTJ_M_VALID) != 0, ext,
                        (l.flags & KTJ_DL_HAS_GRID) != 0, l.p[0], l.p[1], l.p[2], (l.flags & KTJ_DL_HAS_SIZE) != 0, l.p[0], l.coll);
       count_row_stats(m, ctx, &rs);
     }
