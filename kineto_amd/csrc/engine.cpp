@@ -234,7 +234,7 @@ struct ktj_engine {
   /* working buffers */
   DevBuf d_scalars, d_entries, d_name_blob, d_arg_blob;
   DevBuf c_ts, c_dur, c_corr, c_dev, c_res, c_meta, c_ext;
-  DevBuf t_full, t_narrow, t_cpu, f_has_runtime, f_first, f_stream_src, f_pay, n_ext_src, n_kern_src, n_copy_src, n_pay, slot_f, slot_n, dev_link, dev_queue, sync_keys, sync_pos, sync_first;
+  DevBuf t_full, t_narrow, t_cpu, f_has_runtime, f_first, f_stream_src, f_pay, n_ext_src, n_kern_src, n_copy_src, n_pay, n_head, slot_f, slot_n, dev_link, dev_queue, sync_keys, sync_pos, sync_first;
   DevBuf q_keys, q_stream, q_amb, dn_hash, dn_first, dn_dev, dn_key, dn_rank, dn_list;
   DevBuf s_dev_k, s_dev_r, s_dev_l, s_res_k, s_res_r, s_res_l;
   DevBuf keys_a, keys_b, vals_a, vals_b, hist, scan_tmp;
@@ -1527,6 +1527,7 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
   NEED(e->f_has_runtime, (cap_full / 32 + 2ull) * 4);
   NEED(e->n_ext_src, (cap_narrow + 1ull) * 4); NEED(e->n_kern_src, (cap_narrow + 1ull) * 4);
   NEED(e->n_copy_src, (cap_narrow + 1ull) * 4); NEED(e->n_pay, (cap_narrow + 1ull) * sizeof(NarrowPay));
+  if (!e->noalloc) NEED(e->n_head, (cap_narrow + 1ull) * sizeof(NarrowHead)); /* (the scratch array has as many records without) */
   NEED(e->slot_f, nr * 4 + 16); NEED(e->slot_n, nr * 4 + 16);
   NEED(e->dev_link, nd * sizeof(DevLink) + 16);
   NEED(e->dev_queue, nd * 8 + 16);
@@ -1611,7 +1612,8 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
   Table tn{e->t_narrow.as<uint64_t>(), cap_narrow - 1, 0u, &sc->plan.ctl[KTJ_TBL_NARROW]};
   Table t_cpu{e->t_cpu.as<uint64_t>(), cap_cpu - 1, 1u, &sc->plan.ctl[KTJ_TBL_CPU]};
   FullCols fc{e->f_has_runtime.as<uint32_t>(), e->f_first.as<uint32_t>(), e->f_stream_src.as<uint32_t>(), e->f_pay.as<FullPay>()};
-  NarrowCols nc{e->n_ext_src.as<uint32_t>(), e->n_kern_src.as<uint32_t>(), e->n_copy_src.as<uint32_t>(), e->n_pay.as<NarrowPay>()};
+  NarrowCols nc{e->n_ext_src.as<uint32_t>(), e->n_kern_src.as<uint32_t>(), e->n_copy_src.as<uint32_t>(), e->n_pay.as<NarrowPay>(),
+                e->noalloc ? nullptr : e->n_head.as<NarrowHead>()};
   e->h_ctl->weave = KTJ_WEAVE_UNKNOWN;
   HIPCHK(plan_tables(tf, fc, tn, nc, t_cpu, (e->flags & KTJ_CREATE_HASH_JOIN) != 0, woven ? ng + nr + nd : 0u, &e->h_ctl_dev->weave, sc, st));
   ApiTable api{e->d_cid_names.as<uint32_t>(), (uint32_t)e->cid_names.size(), e->d_flow_bits.as<uint32_t>(), e->malloc_cid};

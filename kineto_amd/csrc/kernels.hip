@@ -94,8 +94,8 @@ struct ProbeSeq {
   __device__ __forceinline__ void next() { run += step; }
 };
 /* A table as its plan has it, read once: the stores of a pass over rows would have it read again for each (11 million kernels: links 388 -> 373 us). */
-struct TableView { uint64_t* keys; uint32_t mask, keyed_direct, direct; uint64_t base, span; };
-__device__ __forceinline__ TableView view(const Table& t) { return TableView{t.keys, t.mask, t.keyed_direct, t.ctl->direct, t.ctl->base, t.ctl->span}; }
+struct TableView { uint64_t* keys; uint32_t mask, keyed_direct, direct, no_heads; uint64_t base, span; };
+__device__ __forceinline__ TableView view(const Table& t) { return TableView{t.keys, t.mask, t.keyed_direct, t.ctl->direct, t.ctl->no_heads, t.ctl->base, t.ctl->span}; }
 /* Returns the slot of `key`, inserting it if absent; KTJ_NOSLOT when the table is full (hash
  * mode) or the key lies outside the planned range (direct mode; cannot happen for keys that were
  * part of the range computation). */
@@ -551,6 +551,8 @@ k_plan_clear(Scalars* sc, Table tf, FullCols fc, Table tn, NarrowCols nc, Table 
   __shared__ TableCtl ctl[3];
   if (blockIdx.x == 0 && threadIdx.x == 0) stage_clock(sc, KTJ_CLOCK_JOIN);
   if (threadIdx.x < 64) {
+    bool beyond_31_bits = false;
+    static_assert(KTJ_TBL_FULL == 0 && KTJ_TBL_NARROW == 1, "the full table's range comes first");
     for (int k = 0; k < 3; ++k) {
       unsigned long long lo = sc->range_shard[threadIdx.x][2 * k], hi = sc->range_shard[threadIdx.x][2 * k + 1];
       for (int o = 32; o > 0; o >>= 1) {
@@ -560,7 +562,10 @@ k_plan_clear(Scalars* sc, Table tf, FullCols fc, Table tn, NarrowCols nc, Table 
       }
       const uint64_t cap = (uint64_t)(k == KTJ_TBL_FULL ? tf.mask : k == KTJ_TBL_NARROW ? tn.mask : cpu.mask) + 1u;
       TableCtl x;
-      x.base = 0; x.span = 0; x.direct = 0; x.pad = 0;
+      x.base = 0; x.span = 0; x.direct = 0; x.no_heads = 0;
+      /* (KTJ_TBL_FULL, whose range has the ids of all runtime and device rows, comes first) */
+      if (k == KTJ_TBL_FULL) beyond_31_bits = lo <= hi && hi >= 0x80000000ULL;
+      if (k == KTJ_TBL_NARROW) x.no_heads = beyond_31_bits || !nc.head ? 1u : 0u;
       /* the reserved key never takes part in direct addressing (it has its own slot) */
       if (!force_hash && lo <= hi && hi - lo < cap) { x.base = lo; x.span = hi - lo; x.direct = 1; }
       if (threadIdx.x == 0) {
@@ -593,11 +598,13 @@ k_plan_clear(Scalars* sc, Table tf, FullCols fc, Table tn, NarrowCols nc, Table 
   }
   const uint64_t words = (sf.n + 31) / 32; /* the bitmap: whole words up to the extent, and the word of the reserved slot */
   for (uint64_t i = at; i <= words; i += step) fc.has_runtime[i < words ? i : (tf.mask + 1ull) / 32] = 0;
+  const bool no_heads = ctl[KTJ_TBL_NARROW].no_heads != 0;
   NarrowPay z;
   z.ext_val = 0; z.info = 0; z.pay[0] = z.pay[1] = z.pay[2] = 0;
   for (uint64_t i = at; i <= sn.n; i += step) {
     const uint64_t k = i < sn.n ? i : tn.mask + 1ull;
-    nc.ext_src[k] = 0; nc.kern_src[k] = 0; nc.copy_src[k] = 0; nc.pay[k] = z;
+    nc.ext_src[k] = 0; nc.kern_src[k] = 0; nc.copy_src[k] = 0;
+    if (no_heads) nc.pay[k] = z; else nc.head[k] = NarrowHead{0, 0};
   }
 }
 hipError_t plan_tables(Table tf, FullCols fc, Table tn, NarrowCols nc, Table cpu, bool force_hash, uint64_t n_rows, uint32_t* h_weave, Scalars* sc, hipStream_t st) {
@@ -624,6 +631,10 @@ __device__ __forceinline__ void resolved_external(uint64_t ext_id, const Table& 
     if (row) *info |= collective_for_linked(g[row - 1], ctx) << KTJ_NP_COLL_SHIFT;
   }
 }
+__device__ __forceinline__ void leave_external(const TableView& tn, const NarrowCols& nc, uint32_t slot, int32_t ext_val, uint32_t info) {
+  if (tn.no_heads) { nc.pay[slot].ext_val = ext_val; nc.pay[slot].info = info; }
+  else nc.head[slot] = NarrowHead{ext_val, info};
+}
 /* cpuCorrelationMap_[correlation] = externalId: RocmActivityProfiler.cpp:135-148.  The last record of
  * a correlation id stays (atomicMax over the record index).  Every record resolves its external id
  * against the CPU-op ids at once and writes the result into the slot: that is final when no two
@@ -646,7 +657,7 @@ __global__ void k_build_extcorr(const ktj_extcorr_rec* e, uint64_t n, Table tn_p
       int32_t ext_val;
       uint32_t info;
       resolved_external(rec.external_id, cpu, cpu_row, g, ctx, &ext_val, &info);
-      if (info != 0) { nc.pay[slot].ext_val = ext_val; nc.pay[slot].info = info; }
+      if (info != 0) leave_external(tn, nc, slot, ext_val, info);
     }
   }
   /* one store per workgroup at most: every lane storing the same flag would queue up in L2 */
@@ -668,15 +679,15 @@ __global__ void k_build_cpu_ids(const ktj_generic_rec* g, uint64_t n, Table cpu_
 __global__ void k_resolve_external(const ktj_extcorr_rec* e, uint64_t n, Table tn, NarrowCols nc, Table cpu,
                                    const uint32_t* cpu_row, const ktj_generic_rec* g, EmitCtx ctx, const Scalars* sc) {
   if (sc->ext_ids_repeat == 0) return;
+  const TableView table = view(tn);
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) {
     const ktj_extcorr_rec rec = e[i];
-    const uint32_t slot = slot_find(tn, rec.correlation);
+    const uint32_t slot = slot_find(table, rec.correlation);
     if (slot == KTJ_NOSLOT || nc.ext_src[slot] != (uint32_t)i + 1u) continue;
     int32_t ext_val;
     uint32_t info;
     resolved_external(rec.external_id, cpu, cpu_row, g, ctx, &ext_val, &info);
-    nc.pay[slot].ext_val = ext_val;
-    nc.pay[slot].info = info;
+    leave_external(table, nc, slot, ext_val, info);
   }
 }
 /* One pass over the device rows with one slot of each table:
@@ -716,6 +727,10 @@ __global__ void k_link_device(uint64_t n, Columns c, uint64_t first_device, Tabl
       fp = fc.pay[sf];
       runtime_bits = fc.has_runtime[sf >> 5];
       if (!((runtime_bits >> (sf & 31u)) & 1u)) { fp.first_ts = 0; fp.stream = 0; } /* no runtime row wrote this slot in this pass */
+    }
+    if (sn != KTJ_NOSLOT && !tn.no_heads && !((runtime_bits >> (sf & 31u)) & 1u)) { /* nor that one */
+      const NarrowHead head = nc.head[sn];
+      np.ext_val = head.ext_val; np.info = head.info; np.pay[0] = np.pay[1] = np.pay[2] = 0;
     }
     DevLink l;
     l.p[0] = l.p[1] = l.p[2] = 0; l.flags = 0; l.coll = 0;
@@ -2638,7 +2653,10 @@ __global__ void KX_JOIN_ATTR k_join_runtime(const ktj_runtime_rec* r, uint64_t n
     if (i < n) sn = publishes ? slot_insert(tn, narrow_corr_key(id)) : slot_find(tn, narrow_corr_key(id));
     int32_t ext = 0;
     uint32_t np_info = 0;
-    if (sn != KTJ_NOSLOT) { ext = nc.pay[sn].ext_val; np_info = nc.pay[sn].info; }
+    if (sn != KTJ_NOSLOT) {
+      const NarrowHead head = tn.no_heads ? NarrowHead{nc.pay[sn].ext_val, nc.pay[sn].info} : nc.head[sn];
+      ext = head.ext_val; np_info = head.info;
+    }
     const bool repeats = bitmap_test_and_set(fc.has_runtime, sf, sf != KTJ_NOSLOT);
     if (i < n) {
       carries_stream = (meta & KTJ_M_HAS_STREAM) != 0;
@@ -2651,18 +2669,20 @@ __global__ void KX_JOIN_ATTR k_join_runtime(const ktj_runtime_rec* r, uint64_t n
         if (carries_stream) fp.stream = rec.kind == KTJ_RT_KERNEL ? rec.u.kernel.stream : rec.u.copy.stream;
         fc.pay[sf] = fp;
       }
-      if (publishes) {
-        if (sn == KTJ_NOSLOT) flag_error(sc, KTJ_DEVERR_TABLE_FULL);
-        else {
-          NarrowPay* np = &nc.pay[sn];
-          if (kind == KTJ_RT_KERNEL) {
-            pack_grid(rec, np->pay);
-            np->info = (np_info & ~KTJ_NP_KIND_MASK) | KTJ_DL_HAS_GRID;
-          } else {
-            np->pay[0] = rec.kind == KTJ_RT_COPY ? rec.u.copy.size : rec.u.malloc_.size;
-            np->info = (np_info & ~KTJ_NP_KIND_MASK) | KTJ_DL_HAS_SIZE;
-          }
+      if (publishes && sn == KTJ_NOSLOT) flag_error(sc, KTJ_DEVERR_TABLE_FULL);
+      if (sn != KTJ_NOSLOT && (publishes || !tn.no_heads)) { /* (with heads there is nothing there that another row's would be) */
+        NarrowPay np;
+        np.ext_val = ext; np.info = np_info & ~KTJ_NP_KIND_MASK;
+        np.pay[0] = np.pay[1] = np.pay[2] = 0;
+        if (publishes) {
+          if (kind == KTJ_RT_KERNEL) pack_grid(rec, np.pay);
+          else np.pay[0] = rec.kind == KTJ_RT_COPY ? rec.u.copy.size : rec.u.malloc_.size;
+          np.info |= kind == KTJ_RT_KERNEL ? KTJ_DL_HAS_GRID : KTJ_DL_HAS_SIZE;
         }
+        typedef unsigned int v4u __attribute__((ext_vector_type(4)));
+        v4u* const dst = reinterpret_cast<v4u*>(&nc.pay[sn]);
+        dst[0] = reinterpret_cast<const v4u*>(&np)[0];
+        dst[1] = reinterpret_cast<const v4u*>(&np)[1];
       }
       store_once(&slot_n[i], sn);
       if ((np_info & KTJ_NP_LINKED) && valid) ++n_linked;

@@ -1,0 +1,58 @@
+"""What the external-correlation records leave for the runtime and device rows has a place of its own where all ids fit 31 bits
+(NarrowHead): documents and counters against the oracle, in memory that a pass over other records has just left, for ids that only
+some classes of records have, rows that hand nothing over, ids that several rows have, and ids beyond 31 bits that coincide after narrowing."""
+import pytest
+
+import oracle_glue as og
+from kineto_amd import abi
+from kineto_amd.engine import TraceEngine
+from stream_builder import B, StreamBuilder
+
+pytestmark = pytest.mark.gpu
+N = 1200
+
+
+def stream(first_id, step, full, beyond, repeated):
+    """full: every id has a record of each class, and all of it is handed over.  Otherwise ids lack one class or two, rows lie outside the
+    capture window or are of no kind, and (repeated) share ids."""
+    b = StreamBuilder(window=(B + 10**6, B + 10**9), host_name="heads")
+    b.api(["hipLaunchKernel", "hipMemcpyAsync", "hipMalloc", "hipDeviceSynchronize"], flow_start=[0, 1], malloc_cid=2)
+    for k in range(0, N, 4):
+        b.add_generic("op%d" % (k % 7), 0, B + 2 * 10**6 + k, B + 2 * 10**6 + k + 9, 4242, 5, id=k + 1)
+    for k in range(N):
+        id = first_id + k * step + ((1 << 32) * (k % 3) if beyond else 0)
+        of = lambda m: full or k % m != m - 1   # noqa: E731
+        if of(3):
+            b.add_extcorr(id, k // 4 * 4 + 1 if full or k % 7 else 10**6)   # (some name no CPU op)
+            if repeated and k % 11 == 0:
+                b.add_extcorr(id, k // 8 * 8 + 1)
+        at = B + 2 * 10**6 + 10 * k if full or k % 6 else B + 100   # (some in front of the window)
+        kind = 1 if full else k % 4
+        if of(5):
+            for again in range(2 if repeated and k % 9 == 0 else 1):
+                b.add_runtime(id, at + again, at + 5, kind, 4242, 5 + k % 3, kind=(kind + again) % 4, grid=(k + 1, 2, again + 1), workgroup=(64, 1, 1), stream=k % 3, size=k * 8)
+        if of(4):
+            b.add_device(id, at + 900, at + 950, domain=0 if kind == 1 else 1, op=1 + k % 4, device=k % 2, name="kernel%d" % (k % 9), stream=k % 3, queue=7 + k % 2)
+    return b.build()
+
+
+@pytest.mark.parametrize("hashed", (False, True))
+@pytest.mark.parametrize("beyond, repeated, step", ((False, False, 1), (False, True, 3), (False, False, 977), (True, False, 1), (True, True, 2)))
+def test_rows_that_lack_one_class_or_another(beyond, repeated, step, hashed):
+    lib = abi.load_engine()
+    lib.ktj_debug_force_sort_passes(1)
+    try:
+        # the first leaves its rows' values in the memory that the second then takes
+        for sp in (stream(5, step, True, False, False), stream(5, step, False, beyond, repeated)):
+            o = og.OracleRun(sp)
+            want, counters = o.output(), o.counters()
+            o.close()
+            with TraceEngine(sp.contents.trace_name.decode(), base_time_ns=sp.contents.base_time_ns, hash_join=hashed) as e:
+                e.submit_stream(sp)
+                for _ in range(2):
+                    e.process()
+                    assert e.output() == want
+                    got = e.stats()
+                    assert [got.n_linked, got.gpu_and_cpu_op_out_of_order, got.out_of_range_events] == [counters[k] for k in ("n_linked", "out_of_order", "out_of_range")]
+    finally:
+        lib.ktj_debug_force_sort_passes(0)
