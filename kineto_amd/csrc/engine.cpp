@@ -1629,7 +1629,7 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
                            e->len.as<uint32_t>(), sc, st));
   HIPCHK(republish_runtime_rows(r_recs, nr, c, ng, fc, nc, e->slot_f.as<uint32_t>(), e->slot_n.as<uint32_t>(), sc, st));
   unsigned long long* orphans = e->keys_a.as<unsigned long long>(); /* a bit per device row: the sort's words come later */
-  HIPCHK(link_device_rows(nd, c, ng + nr, tf, fc, tn, nc, e->dev_link.as<DevLink>(), orphans, sc, st));
+  HIPCHK(link_device_rows(nd, c, ng + nr, tf, fc, tn, nc, links_in(e->dev_link.p, nd), orphans, sc, st));
   HIPCHK(backfill_streams(e->dev_queue.as<uint64_t>(), nd, max_spans != 0, c, ng + nr, tf, fc, orphans, stt, sc, st));
   if (max_spans) {
     const int rc = synthesise_user_spans(e, c, ctx, t_cpu, cpu_row, sc, N);
@@ -1686,7 +1686,7 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
     e->sorted_keys = nullptr;
     auto sort = [&]() { return sort_packed(c, N, sets, sc, e->passes_to_launch(N), !e->sort_all_bits, e->keys_a.as<uint64_t>(), e->keys_b.as<uint64_t>(), e->perm, e->hist.as<uint32_t>(), e->offs.as<uint32_t>(), st); };
     HIPCHK(sort());
-    HIPCHK(mat_rows(g_recs, ng, 0, nullptr, d_recs, nd, c, ng + nr, e->dev_link.as<DevLink>(), clock_of(e), ctx, rows, e->len.as<uint32_t>(), sc, st));
+    HIPCHK(mat_rows(g_recs, ng, 0, nullptr, d_recs, nd, c, ng + nr, links_in(e->dev_link.p, nd), clock_of(e), ctx, rows, e->len.as<uint32_t>(), sc, st));
     for (;;) {
       text.out = e->out.as<char>(); text.out_cap = e->out.cap;
       HIPCHK(gather_offsets(e->perm, e->len.as<uint32_t>(), N, e->len_sorted.as<uint32_t>(), e->kind_sorted.as<uint8_t>(),
@@ -1809,8 +1809,8 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
                              e->sync_pos.as<uint32_t>(), e->sync_first.as<uint32_t>(), sc, st));
     sync_first = e->sync_first.as<uint32_t>();
   }
-  HIPCHK(mat_rows(g_recs, ng, 0, sync_first, d_recs, nd, c, ng + nr, e->dev_link.as<DevLink>(), clock_of(e), ctx, rows, e->len.as<uint32_t>(), sc, st));
-  HIPCHK(mat_rows(e->synth_recs.as<ktj_generic_rec>(), e->n_spans, ng + nr + nd, nullptr, nullptr, 0, c, 0, nullptr, clock_of(e), ctx, rows,
+  HIPCHK(mat_rows(g_recs, ng, 0, sync_first, d_recs, nd, c, ng + nr, links_in(e->dev_link.p, nd), clock_of(e), ctx, rows, e->len.as<uint32_t>(), sc, st));
+  HIPCHK(mat_rows(e->synth_recs.as<ktj_generic_rec>(), e->n_spans, ng + nr + nd, nullptr, nullptr, 0, c, 0, Links{}, clock_of(e), ctx, rows,
                   e->len.as<uint32_t>(), sc, st));
   if (n_coll) HIPCHK(collective_first(mat, e->perm, e->scalars.n_valid, n_coll, e->d_coll_first.as<uint32_t>(), st));
 

@@ -102,6 +102,17 @@ struct DevLink {
 };                         /* 32 bytes */
 #define KTJ_DL_HAS_SIZE 1u
 #define KTJ_DL_HAS_GRID 2u
+/* The same for many rows, each value by itself: most rows of graph launches take nothing over, and the values that a wavefront's rows
+ * have none of are neither stored nor loaded (11 million kernels of graphs: k_link_device 227 -> 167 us, k_mat_rows 558 -> 505; where all rows
+ * have a grid 4 bytes a row less). */
+struct Links {
+  uint64_t* p[3];          /* [0] where KTJ_DL_HAS_SIZE or KTJ_DL_HAS_GRID, the others where KTJ_DL_HAS_GRID */
+  uint32_t* info;          /* KTJ_DL_* | coll << KTJ_NP_COLL_SHIFT */
+};
+inline Links links_in(void* memory /* n DevLinks */, uint64_t n) {
+  uint64_t* const w = static_cast<uint64_t*>(memory);
+  return Links{{w, w + n, w + 2 * n}, reinterpret_cast<uint32_t*>(w + 3 * n)};
+}
 
 /* Columns in arrival order: generic rows, then runtime rows, then device rows.  Where a row's record is read again anyway, for its
  * joined row, duration and correlation id come from there, and nothing reads the "External id" of rows that are no device rows
@@ -287,7 +298,7 @@ hipError_t collective_first(const MatRow* mat, const uint32_t* perm, uint64_t n_
 /* per device row: "External id", timestamp-order check, stream of the launching row, and the
  * size / grid hand-over (into link[]) */
 hipError_t link_device_rows(uint64_t n, Columns c, uint64_t first_device, Table tf, FullCols fc, Table tn, NarrowCols nc,
-                            DevLink* link, unsigned long long* orphans /* a bit per row */, Scalars* sc, hipStream_t st);
+                            Links link, unsigned long long* orphans /* a bit per row */, Scalars* sc, hipStream_t st);
 /* stream back-fill: queue table (keys/vals/ambiguous) and dense table are caller-provided, zeroed */
 struct StreamTables {
   uint64_t* q_keys;   /* KTJ_QUEUE_CAP + 1, filled with KTJ_EMPTY_KEY */
@@ -394,7 +405,7 @@ hipError_t stream_sync_first(const uint32_t* perm, uint64_t n_sorted, const ktj_
 /* joined rows and lengths of generic records (arrival index first_generic on; sync_first: per record, from
  * stream_sync_first, or null when there are no such rows) and of device records */
 hipError_t mat_rows(const ktj_generic_rec* g, uint64_t ng, uint64_t first_generic, const uint32_t* sync_first, const ktj_device_rec* d, uint64_t nd,
-                    Columns c, uint64_t first_device, const DevLink* link, const ClockDev& clk, EmitCtx ctx, Rows rows, uint32_t* len, Scalars* sc, hipStream_t st);
+                    Columns c, uint64_t first_device, Links link, const ClockDev& clk, EmitCtx ctx, Rows rows, uint32_t* len, Scalars* sc, hipStream_t st);
 /* the pass over the runtime rows: publishes what device rows take over (first timestamp, stream, grid,
  * size) into the tables, reads the "External id", makes the joined rows and their lengths; runs
  * after build_extcorr and before link_device_rows */

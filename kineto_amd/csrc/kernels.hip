@@ -701,7 +701,7 @@ __global__ void k_resolve_external(const ktj_extcorr_rec* e, uint64_t n, Table t
  * checked afterwards by k_after_link.  Rows outside the window still take a stream from the
  * slot (slots with a stream come from runtime rows and exist already). */
 __global__ void k_link_device(uint64_t n, Columns c, uint64_t first_device, Table tf_planned, FullCols fc, Table tn_planned, NarrowCols nc,
-                              DevLink* link, unsigned long long* orphans, Scalars* sc) {
+                              Links link, unsigned long long* orphans, Scalars* sc) {
   const TableView tf = view(tf_planned), tn = view(tn_planned);
   uint32_t n_linked = 0, n_bad = 0, n_unresolved = 0, n_orphans = 0;
   const bool have_stream_src = sc->have_stream_src != 0;
@@ -732,15 +732,10 @@ __global__ void k_link_device(uint64_t n, Columns c, uint64_t first_device, Tabl
       const NarrowHead head = nc.head[sn];
       np.ext_val = head.ext_val; np.info = head.info; np.pay[0] = np.pay[1] = np.pay[2] = 0;
     }
-    DevLink l;
-    l.p[0] = l.p[1] = l.p[2] = 0; l.flags = 0; l.coll = 0;
+    uint32_t info = 0; /* for the joined row */
     if (sn != KTJ_NOSLOT) {
       if ((np.info & KTJ_NP_LINKED) && valid) ++n_linked;
-      if (domain != KTJ_DOM_MEMSET && (np.info & KTJ_NP_KIND_MASK) != 0) {
-        l.flags = np.info & KTJ_NP_KIND_MASK;
-        l.p[0] = np.pay[0]; l.p[1] = np.pay[1]; l.p[2] = np.pay[2];
-      }
-      l.coll = np.info >> KTJ_NP_COLL_SHIFT;
+      info = np.info & ~(KTJ_NP_LINKED | (domain != KTJ_DOM_MEMSET ? 0u : KTJ_NP_KIND_MASK));
     }
     bool orphan = false;
     store_once(&c.ext[a], np.ext_val);
@@ -758,14 +753,10 @@ __global__ void k_link_device(uint64_t n, Columns c, uint64_t first_device, Tabl
       }
       if (have_stream_src && is_async_op(domain) && res == 0 && fp.stream != 0) { res = (int64_t)fp.stream; c.res[a] = res; }
     }
-    {
-      typedef unsigned int v4u __attribute__((ext_vector_type(4)));
-      static_assert(sizeof(DevLink) == 32, "two 16-byte stores");
-      const v4u* lv = reinterpret_cast<const v4u*>(&l);
-      v4u* dst = reinterpret_cast<v4u*>(&link[i]);
-      store_once(&dst[0], lv[0]);
-      store_once(&dst[1], lv[1]);
-    }
+    /* (whole lines or none: what a row does not have is not read) */
+    store_once(&link.info[i], info);
+    if (__any((info & KTJ_NP_KIND_MASK) != 0)) store_once(&link.p[0][i], np.pay[0]);
+    if (__any((info & KTJ_DL_HAS_GRID) != 0)) { store_once(&link.p[1][i], np.pay[1]); store_once(&link.p[2][i], np.pay[2]); }
     if (is_async_op(domain) && res == 0) ++n_unresolved;
     /* a bit per row, for k_after_link: with the flag in the 32-byte link it read 352 MB to find the few of 11 M
      * rows (127 us, now 25); a wavefront's rows are 64 in a row */
@@ -829,7 +820,7 @@ hipError_t build_extcorr(const ktj_extcorr_rec* e, uint64_t n, Table tn, NarrowC
   return KTJ_LAUNCH_CHECK();
 }
 hipError_t link_device_rows(uint64_t n, Columns c, uint64_t first_device, Table tf, FullCols fc, Table tn, NarrowCols nc,
-                            DevLink* link, unsigned long long* orphans, Scalars* sc, hipStream_t st) {
+                            Links link, unsigned long long* orphans, Scalars* sc, hipStream_t st) {
   if (n == 0) return hipSuccess;
   hipLaunchKernelGGL(k_link_device, dim3(grid_stride_for(n, KTJ_BLOCK)), dim3(KTJ_BLOCK), 0, st, n, c, first_device, tf, fc, tn,
                      nc, link, orphans, sc);
@@ -2779,23 +2770,23 @@ __global__ void k_republish_runtime(const ktj_runtime_rec* r, uint64_t n, Column
   block_add(sc, KTJ_CNT_OUT_OF_ORDER, n_bad);
 }
 template <bool TEXT>
-__device__ __forceinline__ void mat_device_block(const ktj_device_rec* d, uint64_t n, const Columns& c, uint64_t first, const DevLink* link,
+__device__ __forceinline__ void mat_device_block(const ktj_device_rec* d, uint64_t n, const Columns& c, uint64_t first, const Links& link,
                                                  const ClockDev& clk, const EmitCtx& ctx, Rows rows, uint32_t* len, Scalars* sc, uint64_t block,
                                                  uint64_t blocks, uint4* stage) {
   RowStats rs;
+  /* which values of its link a row has is asked for a group ahead */
+  const auto info_at = [&](uint64_t i) { return load_once(&link.info[i < n ? i : n - 1]); };
+  uint32_t next_info = info_at(block * KTJ_BLOCK + threadIdx.x);
   for (uint64_t base = block * KTJ_BLOCK; base < n; base += blocks * KTJ_BLOCK) {
     const uint32_t cnt = (uint32_t)(n - base < KTJ_BLOCK ? n - base : KTJ_BLOCK);
+    const uint32_t info = next_info;
+    next_info = info_at(base + blocks * KTJ_BLOCK + threadIdx.x);
     const uint64_t i = base + (threadIdx.x < cnt ? threadIdx.x : 0u), a = first + i;
     const bool active = threadIdx.x < cnt;
     MatRow m;
-    DevLink l; /* (the columns and the link are on their way with the records) */
-    {
-      typedef unsigned int v4u __attribute__((ext_vector_type(4)));
-      const v4u* src = reinterpret_cast<const v4u*>(&link[i]);
-      v4u* lv = reinterpret_cast<v4u*>(&l);
-      lv[0] = load_once(&src[0]);
-      lv[1] = load_once(&src[1]);
-    }
+    uint64_t p0 = 0, p1 = 0, p2 = 0; /* (the columns and the link are on their way with the records) */
+    if (info & KTJ_NP_KIND_MASK) p0 = load_once(&link.p[0][i]);
+    if (info & KTJ_DL_HAS_GRID) { p1 = load_once(&link.p[1][i]); p2 = load_once(&link.p[2][i]); }
     const int64_t ts = load_once(&c.ts[a]), res = load_once(&c.res[a]);
     const uint32_t meta = load_once(&c.meta[a]);
     const int32_t ext = load_once(&c.ext[a]);
@@ -2806,7 +2797,7 @@ __device__ __forceinline__ void mat_device_block(const ktj_device_rec* d, uint64
       const ktj_device_rec rec = row_from_lds<ktj_device_rec>(stage);
       m = mat_device_v(rec, ts, duration_from(clk, clk.device_mode, ts, rec.end), res,
                        (meta & KTJ_M_VALID) != 0, ext,
-                       (l.flags & KTJ_DL_HAS_GRID) != 0, l.p[0], l.p[1], l.p[2], (l.flags & KTJ_DL_HAS_SIZE) != 0, l.p[0], l.coll);
+                       (info & KTJ_DL_HAS_GRID) != 0, p0, p1, p2, (info & KTJ_DL_HAS_SIZE) != 0, p0, info >> KTJ_NP_COLL_SHIFT);
       count_row_stats(m, ctx, &rs);
     }
     __syncthreads(); /* every lane has taken its record */
@@ -2823,7 +2814,7 @@ __device__ __forceinline__ void mat_device_block(const ktj_device_rec* d, uint64
 template <bool GENERIC, bool DEVICE, bool TEXT>
 __global__ void __launch_bounds__(KTJ_BLOCK) __attribute__((amdgpu_waves_per_eu(4)))
 k_mat_rows(const ktj_generic_rec* g, uint64_t ng, uint64_t first_generic, const uint32_t* sync_first, uint32_t generic_blocks, const ktj_device_rec* d,
-           uint64_t nd, Columns c, uint64_t first_device, const DevLink* link, ClockDev clk, EmitCtx ctx, Rows rows, uint32_t* len, Scalars* sc, int clock) {
+           uint64_t nd, Columns c, uint64_t first_device, Links link, ClockDev clk, EmitCtx ctx, Rows rows, uint32_t* len, Scalars* sc, int clock) {
   static_assert(sizeof(MatRow) >= sizeof(ktj_generic_rec) && sizeof(MatRow) >= sizeof(ktj_device_rec), "the staging area holds the records, then the joined rows");
   __shared__ uint4 stage[KTJ_BLOCK * sizeof(typename RowOf<TEXT>::T) / 16];
   if (blockIdx.x == 0 && threadIdx.x == 0 && clock) stage_clock(sc, KTJ_CLOCK_SIZE);
@@ -2906,7 +2897,7 @@ k_gather_len(const uint32_t* perm, const uint32_t* len, uint64_t n, uint32_t* le
 }
 
 hipError_t mat_rows(const ktj_generic_rec* g, uint64_t ng, uint64_t first_generic, const uint32_t* sync_first, const ktj_device_rec* d, uint64_t nd,
-                    Columns c, uint64_t first_device, const DevLink* link, const ClockDev& clk, EmitCtx ctx, Rows rows, uint32_t* len, Scalars* sc, hipStream_t st) {
+                    Columns c, uint64_t first_device, Links link, const ClockDev& clk, EmitCtx ctx, Rows rows, uint32_t* len, Scalars* sc, hipStream_t st) {
   const unsigned gb = grid_stride_for(ng, KTJ_BLOCK), db = grid_stride_for(nd, KTJ_BLOCK);
   auto launch = [&](auto kernel, unsigned g_blocks, unsigned d_blocks, bool clock) {
     hipLaunchKernelGGL(kernel, dim3(g_blocks + d_blocks), dim3(KTJ_BLOCK), 0, st, g, ng, first_generic, sync_first, g_blocks, d, nd, c, first_device,
