@@ -150,7 +150,7 @@ __device__ __forceinline__ uint32_t slot_find(const Table& t, uint64_t key) { re
  * reached by every thread of the workgroup.  block_add_to: a counter of its own address, for counts
  * that are zero in nearly every workgroup; block_add: one of the sharded counters of Scalars. */
 __device__ __forceinline__ uint32_t block_sum(uint32_t mine) { /* the sum, in thread 0 */
-  __shared__ uint32_t partial[KTJ_BLOCK >> 6];
+  __shared__ uint32_t partial[16]; /* of up to 1024 threads */
   const uint32_t w = wave_sum_u32(mine);
   __syncthreads();
   if (lane_id() == 0) partial[threadIdx.x >> 6] = w;
@@ -983,6 +983,8 @@ __device__ __forceinline__ uint64_t dense_hash(int32_t device, uint64_t key) {
  * and touches the global table once per pair.  The workgroup that ends last gives every pair its number:
  * 1 + number of pairs of the same device seen earlier. */
 #define DENSE_LOCAL_SLOTS 1024u
+/* (every workgroup enters each pair that it has: 489 of 256 threads instead of 123 of 1024 for a million device rows 34 us, now 22) */
+#define DENSE_THREADS 1024u
 #define DENSE_ROWS 4u
 #define KTJ_DENSE_MAX KTJ_MAX_STREAM_PAIRS
 __device__ __forceinline__ void dense_enter(StreamTables& t, uint64_t h, uint32_t first, int32_t dev, uint64_t key, Scalars* sc) {
@@ -997,7 +999,7 @@ __device__ __forceinline__ void dense_enter(StreamTables& t, uint64_t h, uint32_
     if (k < KTJ_DENSE_MAX) agent_store(&t.d_list[k], g); else flag_error(sc, KTJ_DEVERR_STREAMS);
   }
 }
-__global__ void __launch_bounds__(KTJ_BLOCK)
+__global__ void __launch_bounds__(DENSE_THREADS)
 k_dense_first(const uint64_t* queues, uint64_t n, uint64_t per, Columns c, uint64_t first_device, StreamTables t, Scalars* sc) {
   __shared__ unsigned long long l_key[DENSE_LOCAL_SLOTS];
   __shared__ unsigned long long l_pair_key[DENSE_LOCAL_SLOTS];
@@ -1008,23 +1010,23 @@ k_dense_first(const uint64_t* queues, uint64_t n, uint64_t per, Columns c, uint6
   for (uint32_t k = threadIdx.x; k < DENSE_LOCAL_SLOTS; k += blockDim.x) { l_key[k] = KTJ_EMPTY_KEY; l_min[k] = 0xFFFFFFFFu; }
   __syncthreads();
   const uint64_t lo = blockIdx.x * per, hi = n < lo + per ? n : lo + per;
-  for (uint64_t i0 = lo + threadIdx.x; i0 < hi; i0 += KTJ_BLOCK * DENSE_ROWS) {
+  for (uint64_t i0 = lo + threadIdx.x; i0 < hi; i0 += DENSE_THREADS * DENSE_ROWS) {
     uint32_t row_meta[DENSE_ROWS];
     int64_t row_dev[DENSE_ROWS];
     uint64_t row_stream[DENSE_ROWS], row_queue[DENSE_ROWS];
 #pragma unroll
     for (uint32_t r = 0; r < DENSE_ROWS; ++r) { /* all loads of the group in flight together */
-      const uint64_t i = i0 + r * KTJ_BLOCK, a = first_device + (i < hi ? i : hi - 1);
+      const uint64_t i = i0 + r * DENSE_THREADS, a = first_device + (i < hi ? i : hi - 1);
       row_meta[r] = c.meta[a]; row_dev[r] = c.dev[a]; row_stream[r] = (uint64_t)c.res[a];
     }
 #pragma unroll
     for (uint32_t r = 0; r < DENSE_ROWS; ++r) {
-      const uint64_t i = i0 + r * KTJ_BLOCK;
+      const uint64_t i = i0 + r * DENSE_THREADS;
       row_queue[r] = i < hi && row_stream[r] == 0 ? queues[i] : 0;
     }
 #pragma unroll
     for (uint32_t r = 0; r < DENSE_ROWS; ++r) {
-      const uint64_t i = i0 + r * KTJ_BLOCK;
+      const uint64_t i = i0 + r * DENSE_THREADS;
       if (i >= hi) break;
       uint64_t key, stream = row_stream[r];
       const uint32_t domain = row_domain(row_meta[r]);
@@ -1056,7 +1058,7 @@ k_dense_first(const uint64_t* queues, uint64_t n, uint64_t per, Columns c, uint6
   if (!last_workgroup(&sc->done[KTJ_DONE_DENSE])) return;
   const uint32_t n_pairs = agent_load(&sc->n_dense), m = n_pairs < KTJ_DENSE_MAX ? n_pairs : KTJ_DENSE_MAX;
   unsigned long long* l_pair = l_key; /* device and first row of a chunk of the pairs */
-  for (uint32_t p0 = 0; p0 < m; p0 += KTJ_BLOCK) { /* every thread one pair of this round, against all of them */
+  for (uint32_t p0 = 0; p0 < m; p0 += DENSE_THREADS) { /* every thread one pair of this round, against all of them */
     const uint32_t p = p0 + threadIdx.x;
     const uint32_t s = p < m ? agent_load(&t.d_list[p]) : 0u;
     const uint32_t dev = p < m ? (uint32_t)agent_load(&t.d_dev[s]) : 0u, first = p < m ? agent_load(&t.d_first[s]) : 0u;
@@ -1064,7 +1066,7 @@ k_dense_first(const uint64_t* queues, uint64_t n, uint64_t per, Columns c, uint6
     for (uint32_t q0 = 0; q0 < m; q0 += DENSE_LOCAL_SLOTS) {
       const uint32_t here = m - q0 < DENSE_LOCAL_SLOTS ? m - q0 : DENSE_LOCAL_SLOTS;
       __syncthreads();
-      for (uint32_t q = threadIdx.x; q < here; q += KTJ_BLOCK) {
+      for (uint32_t q = threadIdx.x; q < here; q += DENSE_THREADS) {
         const uint32_t o = agent_load(&t.d_list[q0 + q]);
         l_pair[q] = ((unsigned long long)(uint32_t)agent_load(&t.d_dev[o]) << 32) | agent_load(&t.d_first[o]);
       }
@@ -1103,10 +1105,11 @@ hipError_t backfill_streams(const uint64_t* queue, uint64_t n, bool assign, Colu
    * that leaves CUs without a workgroup, and at most four workgroups per CU.  A workgroup's rows lie together, as buffers of a stream
    * mostly do: it sees few of the pairs then (rows a grid apart: 22 million records 85 us instead of 65, 3 million 37 instead of 32; 58 and 33 with
    * columns of 20 bytes a row instead of 24). */
-  const unsigned few = grid_stride_for(n, KTJ_BLOCK * 2), many = grid_stride_for(n, KTJ_BLOCK * 8);
-  const unsigned gd = many > 1024u ? 1024u : many > 256u ? many : few > 256u ? 256u : few;
-  const uint64_t per = ((n + gd - 1) / gd + KTJ_BLOCK - 1) / KTJ_BLOCK * KTJ_BLOCK;
-  hipLaunchKernelGGL(k_dense_first, dim3((unsigned)((n + per - 1) / per)), b, 0, st, queue, n, per, c, first_device, t, sc);
+  const unsigned few = grid_stride_for(n, DENSE_THREADS * 2), many = grid_stride_for(n, DENSE_THREADS * 8);
+  const unsigned most = 1024u * 256u / DENSE_THREADS;
+  const unsigned gd = many > most ? most : many > 256u ? many : few > 256u ? 256u : few;
+  const uint64_t per = ((n + gd - 1) / gd + DENSE_THREADS - 1) / DENSE_THREADS * DENSE_THREADS;
+  hipLaunchKernelGGL(k_dense_first, dim3((unsigned)((n + per - 1) / per)), dim3(DENSE_THREADS), 0, st, queue, n, per, c, first_device, t, sc);
   if (assign) hipLaunchKernelGGL(k_dense_assign, g, b, 0, st, queue, n, c, first_device, t, sc);
   return KTJ_LAUNCH_CHECK();
 }
@@ -1136,6 +1139,9 @@ __device__ __forceinline__ bool local_set_first(unsigned long long* lds /* LOCAL
   return true;
 }
 #define COLLECT_ROWS 4
+/* (of 256 threads, twice as many enter their values: 733 000 records 3 us longer, 3 million 8, 5 million 9; of 1024: the same, and 30 000
+ * records 2 us longer) */
+#define COLLECT_THREADS 512u
 #define SORTP_BITS 8 /* of a digit of the one-word sort */
 __device__ __forceinline__ void set_enter(uint64_t* keys, uint32_t* list, unsigned int* count, uint64_t v, Scalars* sc, unsigned too_many) {
   bool fresh;
@@ -1149,7 +1155,7 @@ __device__ __forceinline__ void set_enter(uint64_t* keys, uint32_t* list, unsign
 /* by one workgroup: rank of each distinct value = number of smaller values (signed) */
 __device__ void rank_values(const uint64_t* keys, const uint32_t* list, uint32_t* rank, uint32_t m, int64_t* lds /* LOCAL_SET_SLOTS */) {
   auto value = [&](uint32_t slot) { return slot < KTJ_SET_CAP ? (int64_t)agent_load(&keys[slot]) : (int64_t)-1; };
-  for (uint32_t p0 = 0; p0 < m; p0 += KTJ_BLOCK) {
+  for (uint32_t p0 = 0; p0 < m; p0 += COLLECT_THREADS) {
     const uint32_t p = p0 + threadIdx.x;
     const uint32_t s = p < m ? agent_load(&list[p]) : 0u;
     const int64_t v = p < m ? value(s) : 0;
@@ -1157,7 +1163,7 @@ __device__ void rank_values(const uint64_t* keys, const uint32_t* list, uint32_t
     for (uint32_t q0 = 0; q0 < m; q0 += LOCAL_SET_SLOTS) {
       const uint32_t here = m - q0 < LOCAL_SET_SLOTS ? m - q0 : LOCAL_SET_SLOTS;
       __syncthreads();
-      for (uint32_t q = threadIdx.x; q < here; q += KTJ_BLOCK) lds[q] = value(agent_load(&list[q0 + q]));
+      for (uint32_t q = threadIdx.x; q < here; q += COLLECT_THREADS) lds[q] = value(agent_load(&list[q0 + q]));
       __syncthreads();
       for (uint32_t q = 0; q < here; ++q) r += lds[q] < v ? 1u : 0u;
     }
@@ -1223,7 +1229,7 @@ __device__ void lay_out_schemas(const EmitCtx& c, weave::SchemaBook* out, Schema
   }
   __syncthreads();
   {
-    const uint32_t schema = k >> 4, size = l->size[schema], upto = l->upto[schema];
+    const uint32_t schema = (k >> 4) & (weave::MAX_SCHEMAS - 1u), size = l->size[schema], upto = k < KTJ_BLOCK ? l->upto[schema] : 0u;
     if (upto) {
       const uint32_t before = upto - size;
       for (uint32_t j = k & 15u; j < (size & 0xFFFFu); j += 16u) out->desc[(before & 0xFFFFu) + j] = KTJ_WD_MOVED(l->desc[schema][j], before >> 16);
@@ -1263,8 +1269,8 @@ __device__ __forceinline__ uint32_t pair_number(PairCache& l, const StreamTables
  * Device rows take the number of their (device, stream) pair on the way, as their columns are read here anyway: a pass of its own
  * read 24 bytes a row, of them 16 that were made for it only (11 million records 3655 -> 3603 us, 22 million 7850 -> 7806, 30 000
  * 174 -> 171; 3 million 1169 -> 1161). */
-__global__ void __launch_bounds__(KTJ_BLOCK) k_collect_distinct(Columns c, uint64_t n, uint64_t per, uint64_t n_device, Backfill fill, SortSets s, Scalars* sc, int straight, EmitCtx ctx, weave::SchemaBook* book) {
-  __shared__ uint64_t red_min[KTJ_BLOCK >> 6], red_max[KTJ_BLOCK >> 6];
+__global__ void __launch_bounds__(COLLECT_THREADS) k_collect_distinct(Columns c, uint64_t n, uint64_t per, uint64_t n_device, Backfill fill, SortSets s, Scalars* sc, int straight, EmitCtx ctx, weave::SchemaBook* book) {
+  __shared__ uint64_t red_min[COLLECT_THREADS >> 6], red_max[COLLECT_THREADS >> 6];
   __shared__ unsigned long long seen[2][LOCAL_SET_SLOTS + 1]; /* deviceId, resourceId values */
   __shared__ PairCache pairs;
   static_assert(sizeof(SchemaLds) <= sizeof(seen), "laid out where the values would be");
@@ -1285,24 +1291,24 @@ __global__ void __launch_bounds__(KTJ_BLOCK) k_collect_distinct(Columns c, uint6
   bool any = false;
   uint32_t n_valid = 0;
   const uint64_t first = lays_out ? n : (blockIdx.x - books) * per, end = n < first + per ? n : first + per;
-  for (uint64_t a0 = first + threadIdx.x; a0 < end; a0 += KTJ_BLOCK * COLLECT_ROWS) {
+  for (uint64_t a0 = first + threadIdx.x; a0 < end; a0 += COLLECT_THREADS * COLLECT_ROWS) {
     uint32_t meta[COLLECT_ROWS];
     uint64_t dev[COLLECT_ROWS], res[COLLECT_ROWS], ts[COLLECT_ROWS];
 #pragma unroll
     for (int r = 0; r < COLLECT_ROWS; ++r) { /* all loads of the group in flight together */
-      const uint64_t at = a0 + (uint64_t)r * KTJ_BLOCK, a = at < end ? at : end - 1;
+      const uint64_t at = a0 + (uint64_t)r * COLLECT_THREADS, a = at < end ? at : end - 1;
       meta[r] = c.meta[a];
       dev[r] = (uint64_t)c.dev[a];
       res[r] = (uint64_t)c.res[a];
       ts[r] = (uint64_t)c.ts[a];
     }
 #pragma unroll
-    for (int r = 0; r < COLLECT_ROWS; ++r) meta[r] = a0 + (uint64_t)r * KTJ_BLOCK < end ? meta[r] : 0u; /* (not a row) */
+    for (int r = 0; r < COLLECT_ROWS; ++r) meta[r] = a0 + (uint64_t)r * COLLECT_THREADS < end ? meta[r] : 0u; /* (not a row) */
     uint32_t ask = 0; /* device rows that take their pair's number: the key stands in res meanwhile */
     uint64_t queue[COLLECT_ROWS];
 #pragma unroll
     for (int r = 0; r < COLLECT_ROWS; ++r) {
-      const uint64_t a = a0 + (uint64_t)r * KTJ_BLOCK, i = a - fill.first_device; /* (wraps around in front of them) */
+      const uint64_t a = a0 + (uint64_t)r * COLLECT_THREADS, i = a - fill.first_device; /* (wraps around in front of them) */
       const bool device = a < end && a >= fill.first_device && i < fill.n && is_async_op(row_domain(meta[r]));
       ask |= (device ? 1u : 0u) << r;
       queue[r] = device && res[r] == 0 ? fill.queue[i] : 0;
@@ -1314,7 +1320,7 @@ __global__ void __launch_bounds__(KTJ_BLOCK) k_collect_distinct(Columns c, uint6
       if (numbered && dense_key(row_domain(meta[r]), res[r], queue[r], &key)) res[r] = key;
       else {
         ask &= ~(1u << r);
-        if (res[r] == 0 && queue[r] != 0) { res[r] = queue[r]; c.res[a0 + (uint64_t)r * KTJ_BLOCK] = (int64_t)queue[r]; }
+        if (res[r] == 0 && queue[r] != 0) { res[r] = queue[r]; c.res[a0 + (uint64_t)r * COLLECT_THREADS] = (int64_t)queue[r]; }
       }
     }
     while (ask) {
@@ -1329,7 +1335,7 @@ __global__ void __launch_bounds__(KTJ_BLOCK) k_collect_distinct(Columns c, uint6
       }
 #pragma unroll
       for (uint32_t r = 0; r < COLLECT_ROWS; ++r) res[r] = at == r ? (uint64_t)pair_is : res[r];
-      c.res[a0 + (uint64_t)at * KTJ_BLOCK] = (int64_t)pair_is;
+      c.res[a0 + (uint64_t)at * COLLECT_THREADS] = (int64_t)pair_is;
     }
     uint32_t todo = 0;
 #pragma unroll
@@ -1530,12 +1536,12 @@ hipError_t collect_distinct(Columns c, uint64_t n, uint64_t n_device, const Back
   /* at most four workgroups per CU: every workgroup pays for its local sets and its atomics at the
    * end once, and a thousand of them keep enough loads in flight (4096: 0.23 ms for 22 M rows,
    * 1024: 0.17 ms) */
-  unsigned g = grid_stride_for(n, n < (1u << 20) ? KTJ_BLOCK * COLLECT_ROWS : KTJ_BLOCK * 16);
-  if (g > 1024u) g = 1024u;
+  unsigned g = grid_stride_for(n, n < (1u << 20) ? COLLECT_THREADS * COLLECT_ROWS : COLLECT_THREADS * 16);
+  if (g > 1024u * 256u / COLLECT_THREADS) g = 1024u * 256u / COLLECT_THREADS;
   /* (a workgroup's rows lie together and have few values, as above: 733 000 records 34 -> 28 us, 22 million 151 -> 141; 32 and 168 since
    * device rows take their numbers here, 66 in a launch of its own for 22 million) */
-  const uint64_t per = ((n + g - 1) / g + KTJ_BLOCK - 1) / KTJ_BLOCK * KTJ_BLOCK;
-  hipLaunchKernelGGL(k_collect_distinct, dim3((unsigned)((n + per - 1) / per) + (book ? 1u : 0u)), dim3(KTJ_BLOCK), 0, st, c, n, per, n_device, fill, s, sc, straight ? 1 : 0, ctx, book);
+  const uint64_t per = ((n + g - 1) / g + COLLECT_THREADS - 1) / COLLECT_THREADS * COLLECT_THREADS;
+  hipLaunchKernelGGL(k_collect_distinct, dim3((unsigned)((n + per - 1) / per) + (book ? 1u : 0u)), dim3(COLLECT_THREADS), 0, st, c, n, per, n_device, fill, s, sc, straight ? 1 : 0, ctx, book);
   return KTJ_LAUNCH_CHECK();
 }
 hipError_t make_keys(Columns c, uint64_t n, SortSets s, const Scalars* sc, uint32_t ts_bits, uint32_t res_bits,
