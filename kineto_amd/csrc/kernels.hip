@@ -809,6 +809,9 @@ __global__ void k_after_link(uint64_t n, Columns c, uint64_t first_device, Table
   block_add(sc, KTJ_CNT_OUT_OF_ORDER, n_bad);
 }
 
+/* Launches that find nothing to do in most passes: every workgroup looks that up, and 4096 of them take 4.6 us for it, 1024 three (where there
+ * is something to do they take as long: ids that pairs of a million launches share, join 520 -> 410 us, rows without a launch 344 and 345). */
+static unsigned grid_rarely(uint64_t n) { const unsigned g = grid_stride_for(n, KTJ_BLOCK); return g < 1024u ? g : 1024u; }
 hipError_t build_cpu_ids(const ktj_generic_rec* g, uint64_t n, Table cpu, uint32_t* cpu_row, Scalars* sc, hipStream_t st) {
   if (n == 0) return hipSuccess;
   hipLaunchKernelGGL(k_build_cpu_ids, dim3(grid_for(n, KTJ_BLOCK)), dim3(KTJ_BLOCK), 0, st, g, n, cpu, cpu_row, sc);
@@ -819,7 +822,7 @@ hipError_t build_extcorr(const ktj_extcorr_rec* e, uint64_t n, Table tn, NarrowC
                          const ktj_generic_rec* g, EmitCtx ctx, Scalars* sc, hipStream_t st) {
   if (n == 0) return hipSuccess;
   hipLaunchKernelGGL(k_build_extcorr, dim3(grid_for(n, KTJ_BLOCK)), dim3(KTJ_BLOCK), 0, st, e, n, tn, nc, cpu, cpu_row, g, ctx, sc);
-  hipLaunchKernelGGL(k_resolve_external, dim3(grid_stride_for(n, KTJ_BLOCK)), dim3(KTJ_BLOCK), 0, st, e, n, tn, nc, cpu, cpu_row, g,
+  hipLaunchKernelGGL(k_resolve_external, dim3(grid_rarely(n)), dim3(KTJ_BLOCK), 0, st, e, n, tn, nc, cpu, cpu_row, g,
                      ctx, (const Scalars*)sc);
   return KTJ_LAUNCH_CHECK();
 }
@@ -1100,7 +1103,7 @@ hipError_t backfill_streams(const uint64_t* queue, uint64_t n, bool assign, Colu
                             StreamTables t, Scalars* sc, hipStream_t st) {
   if (n == 0) return hipSuccess;
   const dim3 g(grid_for(n, KTJ_BLOCK)), b(KTJ_BLOCK);
-  hipLaunchKernelGGL(k_after_link, dim3(grid_stride_for(n, KTJ_BLOCK)), b, 0, st, n, c, first_device, tf, fc, orphans, queue, t, sc);
+  hipLaunchKernelGGL(k_after_link, dim3(grid_rarely(n)), b, 0, st, n, c, first_device, tf, fc, orphans, queue, t, sc);
   /* every workgroup pays for its local table and for each pair it has seen: 2048 rows each, fewer only while
    * that leaves CUs without a workgroup, and at most four workgroups per CU.  A workgroup's rows lie together, as buffers of a stream
    * mostly do: it sees few of the pairs then (rows a grid apart: 22 million records 85 us instead of 65, 3 million 37 instead of 32; 58 and 33 with
@@ -2965,9 +2968,9 @@ hipError_t join_runtime_rows(const ktj_runtime_rec* r, uint64_t n, Columns c, ui
 hipError_t republish_runtime_rows(const ktj_runtime_rec* r, uint64_t n, Columns c, uint64_t first, FullCols fc, NarrowCols nc,
                                   const uint32_t* slot_f, const uint32_t* slot_n, Scalars* sc, hipStream_t st) {
   if (n == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_runtime_winners, dim3(grid_stride_for(n, KTJ_BLOCK)), dim3(KTJ_BLOCK), 0, st, n, c, first, fc, nc, slot_f,
+  hipLaunchKernelGGL(k_runtime_winners, dim3(grid_rarely(n)), dim3(KTJ_BLOCK), 0, st, n, c, first, fc, nc, slot_f,
                      slot_n, (const Scalars*)sc);
-  hipLaunchKernelGGL(k_republish_runtime, dim3(grid_stride_for(n, KTJ_BLOCK)), dim3(KTJ_BLOCK), 0, st, r, n, c, first, fc, nc,
+  hipLaunchKernelGGL(k_republish_runtime, dim3(grid_rarely(n)), dim3(KTJ_BLOCK), 0, st, r, n, c, first, fc, nc,
                      slot_f, slot_n, sc);
   return KTJ_LAUNCH_CHECK();
 }
