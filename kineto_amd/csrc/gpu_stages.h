@@ -39,7 +39,8 @@ struct TableCtl {
 };
 struct Table {
   uint64_t* keys;          /* cap + 1 */
-  uint32_t mask;           /* cap - 1, cap a power of two >= 16 */
+  uint32_t mask;           /* cap - 1, cap a power of two >= 16: slots that direct mode can have; the one behind them is the reserved key's */
+  uint32_t runs;           /* hash mode: runs of sixteen slots that are used, a power of two or a prime, all below cap */
   uint32_t keyed_direct;   /* 1: a plain set, membership is told by the stored key in both modes */
   const TableCtl* ctl;
 };

@@ -83,19 +83,20 @@ __device__ uint32_t table_find(const uint64_t* keys, uint32_t mask, uint64_t key
  * consecutive ids therefore share one run, while strided or clustered ids still spread like under
  * a full hash and a collision costs one probe in another run rather than a walk through a full one. */
 struct ProbeSeq {
-  uint32_t run, step, low;
-  __device__ __forceinline__ ProbeSeq(uint64_t key) {
+  uint32_t run, step, low, runs;
+  __device__ __forceinline__ ProbeSeq(uint64_t key, uint32_t n_runs) {
     const uint64_t h = hash64(key >> 4);
-    run = (uint32_t)h;
-    step = (uint32_t)(h >> 32) | 1u; /* odd: visits every run of a power-of-two table */
+    runs = n_runs;
+    run = __umulhi((uint32_t)h, runs);
+    step = 1u + 2u * __umulhi((uint32_t)(h >> 32), runs >> 1); /* odd and below `runs`: visits every run, whose number is a power of two or a prime */
     low = ((uint32_t)key + (uint32_t)((h * 0x9E3779B97F4A7C15ULL) >> 60)) & 15u; /* ids sharing low bits still use all positions */
   }
-  __device__ __forceinline__ uint32_t slot(uint32_t mask) const { return ((run << 4) | low) & mask; }
-  __device__ __forceinline__ void next() { run += step; }
+  __device__ __forceinline__ uint32_t slot() const { return (run << 4) | low; }
+  __device__ __forceinline__ void next() { run += step; run = run >= runs ? run - runs : run; }
 };
 /* A table as its plan has it, read once: the stores of a pass over rows would have it read again for each (11 million kernels: links 388 -> 373 us). */
-struct TableView { uint64_t* keys; uint32_t mask, keyed_direct, direct, no_heads; uint64_t base, span; };
-__device__ __forceinline__ TableView view(const Table& t) { return TableView{t.keys, t.mask, t.keyed_direct, t.ctl->direct, t.ctl->no_heads, t.ctl->base, t.ctl->span}; }
+struct TableView { uint64_t* keys; uint32_t mask, runs, keyed_direct, direct, no_heads; uint64_t base, span; };
+__device__ __forceinline__ TableView view(const Table& t) { return TableView{t.keys, t.mask, t.runs, t.keyed_direct, t.ctl->direct, t.ctl->no_heads, t.ctl->base, t.ctl->span}; }
 /* Returns the slot of `key`, inserting it if absent; KTJ_NOSLOT when the table is full (hash
  * mode) or the key lies outside the planned range (direct mode; cannot happen for keys that were
  * part of the range computation). */
@@ -108,9 +109,9 @@ __device__ uint32_t slot_insert(const TableView& t, uint64_t key) {
     return (uint32_t)idx;
   }
   if (key == KTJ_EMPTY_KEY) { t.keys[t.mask + 1u] = 0; return t.mask + 1u; }
-  ProbeSeq p(key);
-  for (uint32_t probe = 0; probe <= (t.mask >> 4); ++probe, p.next()) {
-    const uint32_t slot = p.slot(t.mask);
+  ProbeSeq p(key, t.runs);
+  for (uint32_t probe = 0; probe < t.runs; ++probe, p.next()) {
+    const uint32_t slot = p.slot();
     uint64_t cur = t.keys[slot];
     if (cur == key) return slot;
     if (cur == KTJ_EMPTY_KEY) {
@@ -132,9 +133,9 @@ __device__ uint32_t slot_find(const TableView& t, uint64_t key) {
     return (uint32_t)idx;
   }
   if (key == KTJ_EMPTY_KEY) return t.keys[t.mask + 1u] == 0 ? t.mask + 1u : KTJ_NOSLOT;
-  ProbeSeq p(key);
-  for (uint32_t probe = 0; probe <= (t.mask >> 4); ++probe, p.next()) {
-    const uint32_t slot = p.slot(t.mask);
+  ProbeSeq p(key, t.runs);
+  for (uint32_t probe = 0; probe < t.runs; ++probe, p.next()) {
+    const uint32_t slot = p.slot();
     uint64_t cur = t.keys[slot];
     if (cur == key) return slot;
     if (cur == KTJ_EMPTY_KEY) return KTJ_NOSLOT;
@@ -589,7 +590,7 @@ k_plan_clear(Scalars* sc, Table tf, FullCols fc, Table tn, NarrowCols nc, Table 
   }
   __syncthreads();
   const uint64_t at = (uint64_t)blockIdx.x * KTJ_BLOCK + threadIdx.x, step = (uint64_t)gridDim.x * KTJ_BLOCK;
-  auto span = [&](int k, const Table& t) { TableSpan s; s.direct = ctl[k].direct != 0; s.n = s.direct ? ctl[k].span + 1ull : (uint64_t)t.mask + 1ull; return s; };
+  auto span = [&](int k, const Table& t) { TableSpan s; s.direct = ctl[k].direct != 0; s.n = s.direct ? ctl[k].span + 1ull : (uint64_t)t.runs * 16u; return s; };
   const TableSpan sf = span(KTJ_TBL_FULL, tf), sn = span(KTJ_TBL_NARROW, tn), scpu = span(KTJ_TBL_CPU, cpu);
   clear_keys(tf, sf, at, step);
   clear_keys(tn, sn, at, step);

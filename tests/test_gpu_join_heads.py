@@ -56,3 +56,28 @@ def test_rows_that_lack_one_class_or_another(beyond, repeated, step, hashed):
                     assert [got.n_linked, got.gpu_and_cpu_op_out_of_order, got.out_of_range_events] == [counters[k] for k in ("n_linked", "out_of_order", "out_of_range")]
     finally:
         lib.ktj_debug_force_sort_passes(0)
+
+
+@pytest.mark.parametrize("ops", (349525, 349526, 420001))
+def test_tables_of_a_prime_number_of_runs(ops):
+    """Ids too far apart for slots of their own, some without a runtime row: the last table of a power of two runs, and tables of as many
+    as the records ask for."""
+    print(ops, flush=True)
+    sp, release = abi.synth_stream(2, ops, host_name="heads")
+    s = sp.contents
+    assert (s.n_runtime, s.n_device) == (ops, ops)
+    for k in range(ops):
+        s.runtime[k].id = s.runtime[k].id * 977 + (k % 5 == 4)
+        s.device[k].id *= 977
+    for k in range(s.n_extcorr):
+        s.extcorr[k].correlation *= 977
+    o = og.OracleRun(sp)
+    want, counters = o.output(), o.counters()
+    o.close()
+    with TraceEngine(s.trace_name.decode(), base_time_ns=s.base_time_ns) as e:
+        e.submit_stream(sp)
+        for _ in range(2):
+            e.process()
+            assert e.output() == want
+            assert e.stats().n_linked == counters["n_linked"]
+    release()
