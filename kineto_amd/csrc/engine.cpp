@@ -1698,9 +1698,10 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
     if (out_device) e->out.borrow(out_device, out_cap);
     e->perm = e->vals_a.as<uint32_t>();
     e->sorted_keys = nullptr;
-    auto sort = [&]() { return sort_packed(c, N, sets, sc, e->passes_to_launch(N), !e->sort_all_bits, e->keys_a.as<uint64_t>(), e->keys_b.as<uint64_t>(), e->perm, e->hist.as<uint32_t>(), e->offs.as<uint32_t>(), st); };
-    HIPCHK(sort());
-    HIPCHK(mat_rows(g_recs, ng, 0, nullptr, d_recs, nd, c, ng + nr, links_in(e->dev_link.p, nd), clock_of(e), ctx, rows, e->len.as<uint32_t>(), sc, st));
+    auto sort = [&](RowsJob* job) { return sort_packed(c, N, sets, sc, e->passes_to_launch(N), !e->sort_all_bits, e->keys_a.as<uint64_t>(), e->keys_b.as<uint64_t>(), e->perm, e->hist.as<uint32_t>(), e->offs.as<uint32_t>(), job, st); };
+    RowsJob job{g_recs, ng, d_recs, nd, c, ng + nr, links_in(e->dev_link.p, nd), clock_of(e), ctx, rows, e->len.as<uint32_t>(), false};
+    HIPCHK(sort(&job));
+    if (!job.made) HIPCHK(mat_rows(g_recs, ng, 0, nullptr, d_recs, nd, c, ng + nr, links_in(e->dev_link.p, nd), clock_of(e), ctx, rows, e->len.as<uint32_t>(), sc, st));
     for (;;) {
       text.out = e->out.as<char>(); text.out_cap = e->out.cap;
       HIPCHK(gather_offsets(e->perm, e->len.as<uint32_t>(), N, e->len_sorted.as<uint32_t>(), e->kind_sorted.as<uint8_t>(),
@@ -1722,7 +1723,7 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
         e->sort_all_bits = 16; e->sort_info[1] = 1;
         e->sort_passes = sort_packed_passes(e->scalars.sort, false);
         HIPCHK(clear_error_bits(sc, KTJ_DEVERR_UNSORTED, st));
-        HIPCHK(sort());
+        HIPCHK(sort(nullptr));
         continue;
       }
       if (e->scalars.error) break;
@@ -1797,7 +1798,7 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
       if (rc == KTJ_OK) rc = sort_again([&](const uint32_t* o, uint64_t* k, uint32_t* v) { return make_column_keys(c.dev, c.meta, o, N, 1, k, v, st); }, 1);
       if (rc != KTJ_OK) return rc;
     } else if (e->sort_mode != 1 && sort_packed_fits(N, e->scalars.sort)) {
-      HIPCHK(sort_packed(c, N, sets, sc, sort_packed_passes(e->scalars.sort, false), false, ka, kb, va, hist, e->offs.as<uint32_t>(), st));
+      HIPCHK(sort_packed(c, N, sets, sc, sort_packed_passes(e->scalars.sort, false), false, ka, kb, va, hist, e->offs.as<uint32_t>(), nullptr, st));
       e->perm = va;
       e->sorted_keys = nullptr;
     } else if (key_bits <= 62) {

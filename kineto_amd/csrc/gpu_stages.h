@@ -369,6 +369,28 @@ hipError_t make_ts_keys(Columns c, uint64_t n, const Scalars* sc, uint64_t* keys
 hipError_t make_column_keys(const int64_t* column, const uint32_t* meta, const uint32_t* order, uint64_t n, int validity,
                             uint64_t* keys, uint32_t* vals, hipStream_t st);
 hipError_t clear_error_bits(Scalars* sc, unsigned int bits, hipStream_t st);
+/* With schemas set the rows are TextRows (those that the weaver does not print MatRows in the same places, marked:
+ * KTJ_ROW_LEFT, and tail kind KTJ_KIND_LEFT beside their lengths but where Scalars::no_text leaves all); otherwise all are MatRows. */
+struct Rows {
+  void* p;
+  const weave::SchemaBook* schemas;
+  weave::WideText* wide; /* of the generic records */
+};
+/* What mat_rows takes, for the sort: rows of both classes are made in its last launch where it has one that they may come with (made). */
+struct RowsJob {
+  const ktj_generic_rec* g;
+  uint64_t ng;
+  const ktj_device_rec* d;
+  uint64_t nd;
+  Columns c;
+  uint64_t first_device;
+  Links link;
+  ClockDev clk;
+  EmitCtx ctx;
+  Rows rows;
+  uint32_t* len;
+  bool made;
+};
 /* The composite-key sort on single 64-bit words (key above the arrival index); perm receives the
  * arrival index per sorted position.  Usable when sort_packed_fits(n, plan). */
 bool sort_packed_fits(uint64_t n, const SortPlan& plan);
@@ -379,7 +401,7 @@ uint32_t sort_packed_passes(const SortPlan& plan, bool finish); /* finish: the l
 /* key widths come from Scalars::sort; `passes` is how many are launched: those beyond the plan end at once, and
  * a plan that needs more (or does not fit a word) sets KTJ_DEVERR_CAREFUL in Scalars::error */
 hipError_t sort_packed(Columns c, uint64_t n, SortSets s, Scalars* sc, uint32_t passes, bool finish, uint64_t* buf_a, uint64_t* buf_b, uint32_t* perm,
-                       uint32_t* hist, uint32_t* chain_hist /* 8 bytes per row */, hipStream_t st);
+                       uint32_t* hist, uint32_t* chain_hist /* 8 bytes per row */, RowsJob* job /* or none */, hipStream_t st);
 hipError_t make_rank_keys(Columns c, const uint32_t* order, uint64_t n, SortSets s, uint32_t res_bits, uint32_t rank_bits,
                           uint64_t* keys, uint32_t* vals, hipStream_t st);
 /* stable LSD radix sort of (key, val) pairs on the low `bits` bits; result ends in keys_out/vals_out
@@ -390,13 +412,6 @@ hipError_t radix_sort(uint64_t* keys_a, uint32_t* vals_a, uint64_t* keys_b, uint
                       uint64_t** res_keys, uint32_t** res_vals, hipStream_t st);
 
 /* ---- stage 4a: joined rows + exact byte length (arrival order) ---- */
-/* With schemas set the rows are TextRows (those that the weaver does not print MatRows in the same places, marked:
- * KTJ_ROW_LEFT, and tail kind KTJ_KIND_LEFT beside their lengths but where Scalars::no_text leaves all); otherwise all are MatRows. */
-struct Rows {
-  void* p;
-  const weave::SchemaBook* schemas;
-  weave::WideText* wide; /* of the generic records */
-};
 #define KTJ_KIND_LEFT 3u
 /* keys: KTJ_SYNC_CAP + 1, first_pos: KTJ_SYNC_CAP + 1, is_first: n_generic (all caller-provided);
  * dev: the deviceId column */

@@ -2095,21 +2095,28 @@ k_sortp_single(Columns c, uint32_t n, SortSets s, Scalars* sc, uint32_t* perm_ou
  * Takes the place of one or two of five passes (a count, a scan, a scatter each: 135 us for 22 million rows). */
 #define FINISH_MOST 256u
 #define CHAIN_MAX_N 98304ull /* of sort_packed_chain */
-template <int THREADS, int ITEMS>
-__global__ void __launch_bounds__(THREADS)
-k_sortp_finish(const uint64_t* buf_a, const uint64_t* buf_b, uint32_t* perm, uint64_t n, uint32_t idx_bits, Scalars* sc) {
-  constexpr uint32_t ROWS = ITEMS + 2, SPAN = THREADS * ROWS, CHUNKS = SPAN / 64u; /* the tile's rows, a turn in front of and one behind them */
+template <int THREADS, int ITEMS> struct FinishLds {
+  static constexpr uint32_t ROWS = ITEMS + 2, SPAN = THREADS * ROWS, CHUNKS = SPAN / 64u; /* the tile's rows, a turn in front of and one behind them */
   static_assert(THREADS == FINISH_MOST && CHUNKS <= 128u && SPAN < 0x10000u, "chunks of a wavefront's lanes, numbers of groups");
-  __shared__ uint32_t s_val[SPAN];
-  __shared__ uint64_t s_edge[CHUNKS], s_start[CHUNKS]; /* a chunk's last word; a bit per row: first of its group */
+  uint64_t edge[CHUNKS], start[CHUNKS]; /* a chunk's last word; a bit per row: first of its group */
+  uint32_t val[SPAN];
+};
+/* own_bits: those of Scalars::error that the launch sets */
+template <int THREADS, int ITEMS>
+__device__ __forceinline__ void finish_tile(const uint64_t* buf_a, const uint64_t* buf_b, uint32_t* perm, uint64_t n, uint32_t idx_bits, Scalars* sc,
+                                            unsigned int own_bits, uint64_t tile, FinishLds<THREADS, ITEMS>& lds) {
+  constexpr uint32_t ROWS = FinishLds<THREADS, ITEMS>::ROWS, SPAN = FinishLds<THREADS, ITEMS>::SPAN, CHUNKS = FinishLds<THREADS, ITEMS>::CHUNKS;
+  uint32_t* const s_val = lds.val;
+  uint64_t* const s_edge = lds.edge;
+  uint64_t* const s_start = lds.start;
   const SortRun run = sort_run(sc, 1);
   /* (low of 0: the last pass has written the permutation.)  All wavefronts of a workgroup must see the same here, as they number
-   * groups and compare rows for each other: the one bit that this launch sets does not count. */
-  if ((sc->error & ~KTJ_DEVERR_UNSORTED) != 0 || run.low == 0) return;
+   * groups and compare rows for each other: what this launch sets does not count. */
+  if ((sc->error & ~own_bits) != 0 || run.low == 0) return;
   const uint64_t* in = run.passes & 1u ? buf_b : buf_a;
   const uint32_t group_shift = idx_bits + run.low, lane = lane_id(), wave = threadIdx.x >> 6;
   const uint64_t idx_mask = (1ULL << idx_bits) - 1ULL;
-  const uint64_t from = (uint64_t)blockIdx.x * (THREADS * ITEMS) - FINISH_MOST; /* (below 0: not loaded) */
+  const uint64_t from = tile * (THREADS * ITEMS) - FINISH_MOST; /* (below 0: not loaded) */
   uint64_t word[ROWS];
   /* All loads in flight together.  Many words go past the caches, as in the scatter: left there they push out what k_gather_len reads behind
    * the joined rows (22 million rows: 94 us there instead of 84, 61 and 60 here.  11 million and less: the same). */
@@ -2212,9 +2219,20 @@ k_sortp_finish(const uint64_t* buf_a, const uint64_t* buf_b, uint32_t* perm, uin
     if (i < n) perm[i + (uint64_t)(int64_t)(int32_t)moves] = (uint32_t)(word[r] & idx_mask);
   }
 }
-static hipError_t sort_finish(const uint64_t* buf_a, const uint64_t* buf_b, uint32_t* perm, uint64_t n, uint32_t idx_bits, Scalars* sc, hipStream_t st) {
+template <int THREADS, int ITEMS>
+__global__ void __launch_bounds__(THREADS)
+k_sortp_finish(const uint64_t* buf_a, const uint64_t* buf_b, uint32_t* perm, uint64_t n, uint32_t idx_bits, Scalars* sc) {
+  __shared__ FinishLds<THREADS, ITEMS> lds;
+  finish_tile<THREADS, ITEMS>(buf_a, buf_b, perm, n, idx_bits, sc, KTJ_DEVERR_UNSORTED, blockIdx.x, lds);
+}
+static bool finish_and_rows(const uint64_t* buf_a, const uint64_t* buf_b, uint32_t* perm, uint64_t n, uint32_t idx_bits, uint64_t tile, Scalars* sc,
+                            RowsJob* job, hipStream_t st);
+static hipError_t sort_finish(const uint64_t* buf_a, const uint64_t* buf_b, uint32_t* perm, uint64_t n, uint32_t idx_bits, Scalars* sc, RowsJob* job, hipStream_t st) {
   /* tiles that leave no CU without one; large ones where there are enough, as the rows around a tile are loaded twice */
-  auto launch = [&](auto kernel, uint64_t tile) { hipLaunchKernelGGL(kernel, dim3((unsigned)((n + tile - 1) / tile)), dim3(256), 0, st, buf_a, buf_b, perm, n, idx_bits, sc); };
+  auto launch = [&](auto kernel, uint64_t tile) {
+    if (finish_and_rows(buf_a, buf_b, perm, n, idx_bits, tile, sc, job, st)) return;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)((n + tile - 1) / tile)), dim3(256), 0, st, buf_a, buf_b, perm, n, idx_bits, sc);
+  };
   if (n <= CHAIN_MAX_N) launch(k_sortp_finish<256, 1>, 256);
   else if (n < 1ull << 20) launch(k_sortp_finish<256, 4>, 1024);
   else launch(k_sortp_finish<256, 16>, 4096);
@@ -2223,7 +2241,7 @@ static hipError_t sort_finish(const uint64_t* buf_a, const uint64_t* buf_b, uint
 
 template <int BITS, int THREADS, int ITEMS>
 static hipError_t sort_packed_t(Columns c, uint64_t n, SortSets s, Scalars* sc, uint32_t passes, int finish, uint32_t idx_bits, uint64_t* buf_a, uint64_t* buf_b,
-                                uint32_t* perm, uint32_t* hist, hipStream_t st) {
+                                uint32_t* perm, uint32_t* hist, RowsJob* job, hipStream_t st) {
   using P = SortP<BITS, THREADS, ITEMS>;
   const uint32_t n_blocks = (uint32_t)((n + P::TILE - 1) / P::TILE);
   const dim3 g(n_blocks), b(THREADS);
@@ -2247,7 +2265,7 @@ static hipError_t sort_packed_t(Columns c, uint64_t n, SortSets s, Scalars* sc, 
                        (const Scalars*)sc, (const uint32_t*)counts, (const uint32_t*)totals, n_blocks);
     uint64_t* t = in; in = out; out = t;
   }
-  if (finish) return sort_finish(buf_a, buf_b, perm, n, idx_bits, sc, st);
+  if (finish) return sort_finish(buf_a, buf_b, perm, n, idx_bits, sc, job, st);
   return KTJ_LAUNCH_CHECK();
 }
 
@@ -2352,7 +2370,7 @@ k_sortp_chain(const uint64_t* in, uint64_t* words_out, uint32_t* perm_out, uint3
 }
 template <int BITS>
 static hipError_t sort_packed_chain(Columns c, uint64_t n, SortSets s, Scalars* sc, uint32_t passes, int finish, uint32_t idx_bits, uint64_t* buf_a,
-                                    uint64_t* buf_b, uint32_t* perm, uint32_t* hist, hipStream_t st) {
+                                    uint64_t* buf_b, uint32_t* perm, uint32_t* hist, RowsJob* job, hipStream_t st) {
   using P = SortP<BITS, CHAIN_THREADS, 1>;
   const uint32_t n_blocks = (uint32_t)((n + P::TILE - 1) / P::TILE);
   const dim3 g(n_blocks), b(CHAIN_THREADS);
@@ -2365,7 +2383,7 @@ static hipError_t sort_packed_chain(Columns c, uint64_t n, SortSets s, Scalars* 
                        (const Scalars*)sc, hist, n_blocks);
     uint64_t* t = in; in = out; out = t;
   }
-  if (finish) return sort_finish(buf_a, buf_b, perm, n, idx_bits, sc, st);
+  if (finish) return sort_finish(buf_a, buf_b, perm, n, idx_bits, sc, job, st);
   return KTJ_LAUNCH_CHECK();
 }
 #define SORTP_THREADS 256
@@ -2383,7 +2401,7 @@ uint32_t sort_packed_passes(const SortPlan& plan, bool finish) {
   return bits ? (bits + SORTP_BITS - 1u) / SORTP_BITS : 1u;
 }
 hipError_t sort_packed(Columns c, uint64_t n, SortSets s, Scalars* sc, uint32_t passes, bool finish, uint64_t* buf_a, uint64_t* buf_b, uint32_t* perm,
-                       uint32_t* hist, uint32_t* chain_hist, hipStream_t st) {
+                       uint32_t* hist, uint32_t* chain_hist, RowsJob* job, hipStream_t st) {
   if (n == 0) return hipSuccess;
   const uint32_t idx_bits = sort_idx_bits(n);
   if (sort_packed_in_one_launch(n)) {
@@ -2395,10 +2413,10 @@ hipError_t sort_packed(Columns c, uint64_t n, SortSets s, Scalars* sc, uint32_t 
    * SORTP_SMALL_N keys, tiles of 512 spread over the GPU finish a pass sooner than the few 4096-key tiles
    * would (330 000 keys: 113 against 155 us; from a million keys on the large tiles win) */
   if (n > (uint64_t)SORTP_THREADS * 16u && n <= CHAIN_MAX_N && 256ull * passes * ((n + CHAIN_THREADS - 1) / CHAIN_THREADS) <= 2 * (n + 1))
-    return sort_packed_chain<SORTP_BITS>(c, n, s, sc, passes, finish, idx_bits, buf_a, buf_b, perm, chain_hist, st);
+    return sort_packed_chain<SORTP_BITS>(c, n, s, sc, passes, finish, idx_bits, buf_a, buf_b, perm, chain_hist, job, st);
   if (n > (uint64_t)SORTP_THREADS * 16u && n < SORTP_SMALL_N)
-    return sort_packed_t<SORTP_BITS, SORTP_THREADS, 2>(c, n, s, sc, passes, finish, idx_bits, buf_a, buf_b, perm, hist, st);
-  return sort_packed_t<SORTP_BITS, SORTP_THREADS, 16>(c, n, s, sc, passes, finish, idx_bits, buf_a, buf_b, perm, hist, st);
+    return sort_packed_t<SORTP_BITS, SORTP_THREADS, 2>(c, n, s, sc, passes, finish, idx_bits, buf_a, buf_b, perm, hist, job, st);
+  return sort_packed_t<SORTP_BITS, SORTP_THREADS, 16>(c, n, s, sc, passes, finish, idx_bits, buf_a, buf_b, perm, hist, job, st);
 }
 
 /* ------------------------------------------------------------------------------------------ */
@@ -2857,6 +2875,28 @@ k_mat_rows(const ktj_generic_rec* g, uint64_t ng, uint64_t first_generic, const 
   else if (DEVICE)
     mat_device_block<TEXT>(d, nd, c, first_device, link, clk, ctx, rows, len, sc, blockIdx.x - generic_blocks, gridDim.x - generic_blocks, stage);
 }
+/* The sort's last launch (first workgroups) and the rows of both classes in one: neither needs anything of the other, and the former is a
+ * chain of loads and LDS accesses that leaves the memory idle, with fewer workgroups than the GPU holds up to a few million rows.  Passes,
+ * one after the other and now, us: 30 000 records 172 -> 168, 180 000 220 -> 213, 733 000 413 -> 407, 3 million 985 -> 972; 11 and 22 million, where both are
+ * at the memory's rate by themselves, 3153 and 3146, 6838 and 6841. */
+template <int ITEMS>
+__global__ void __launch_bounds__(KTJ_BLOCK) __attribute__((amdgpu_waves_per_eu(4)))
+k_finish_and_rows(const uint64_t* buf_a, const uint64_t* buf_b, uint32_t* perm, uint64_t n, uint32_t idx_bits, uint32_t finish_blocks, const ktj_generic_rec* g,
+                  uint64_t ng, uint32_t generic_blocks, const ktj_device_rec* d, uint64_t nd, Columns c, uint64_t first_device, Links link, ClockDev clk,
+                  EmitCtx ctx, Rows rows, uint32_t* len, Scalars* sc) {
+  using Lds = FinishLds<KTJ_BLOCK, ITEMS>;
+  __shared__ union { uint4 stage[KTJ_BLOCK * sizeof(typename RowOf<true>::T) / 16]; Lds finish; } lds;
+  if (blockIdx.x == 0 && threadIdx.x == 0) stage_clock(sc, KTJ_CLOCK_SIZE);
+  constexpr unsigned int own_bits = KTJ_DEVERR_RECORD_TOO_LONG | KTJ_DEVERR_UNSORTED;
+  if (blockIdx.x < finish_blocks) {
+    finish_tile<KTJ_BLOCK, ITEMS>(buf_a, buf_b, perm, n, idx_bits, sc, own_bits, blockIdx.x, lds.finish);
+    return;
+  }
+  if (sc->error & ~own_bits) return; /* (as in k_mat_rows) */
+  const uint32_t block = blockIdx.x - finish_blocks;
+  if (block < generic_blocks) mat_generic_block<true>(g, ng, 0, ctx, nullptr, rows, len, sc, block, generic_blocks, lds.stage);
+  else mat_device_block<true>(d, nd, c, first_device, link, clk, ctx, rows, len, sc, block - generic_blocks, gridDim.x - finish_blocks - generic_blocks, lds.stage);
+}
 /* Collective metadata: the first activity, in emission order, that prints each entry, per
  * backend (first[2k] nccl, first[2k + 1] hccl).  The host replays appendCollectiveMetadata's
  * bookkeeping (output_json.cpp:799-835) over these.  Runs only for traces that carry any. */
@@ -2946,6 +2986,21 @@ hipError_t mat_rows(const ktj_generic_rec* g, uint64_t ng, uint64_t first_generi
     if (db) { if (rows.schemas) launch(k_mat_rows<false, true, true>, 0, db, clock && !gb); else launch(k_mat_rows<false, true, false>, 0, db, clock && !gb); }
   }
   return KTJ_LAUNCH_CHECK();
+}
+
+static bool finish_and_rows(const uint64_t* buf_a, const uint64_t* buf_b, uint32_t* perm, uint64_t n, uint32_t idx_bits, uint64_t tile, Scalars* sc,
+                            RowsJob* job, hipStream_t st) {
+  if (!job || !job->ng || !job->nd || !job->rows.schemas) return false;
+  const unsigned fb = (unsigned)((n + tile - 1) / tile), gb = grid_stride_for(job->ng, KTJ_BLOCK), db = grid_stride_for(job->nd, KTJ_BLOCK);
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(fb + gb + db), dim3(KTJ_BLOCK), 0, st, buf_a, buf_b, perm, n, idx_bits, fb, job->g, job->ng, gb, job->d, job->nd, job->c,
+                       job->first_device, job->link, job->clk, job->ctx, job->rows, job->len, sc);
+  };
+  if (tile == 1u * KTJ_BLOCK) launch(k_finish_and_rows<1>);
+  else if (tile == 4u * KTJ_BLOCK) launch(k_finish_and_rows<4>);
+  else launch(k_finish_and_rows<16>);
+  job->made = true;
+  return true;
 }
 
 hipError_t join_runtime_rows(const ktj_runtime_rec* r, uint64_t n, Columns c, uint64_t first, ApiTable api, Table tf, FullCols fc,

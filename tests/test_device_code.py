@@ -56,3 +56,14 @@ def test_the_bit_that_the_sorts_last_launch_sets_does_not_end_its_own_wavefronts
         if re.match(r"s_bitset0_b32 s\d+, 10$", text) or (re.match(r"[sv]_and_b32", text) and "0x%x" % (0xFFFFFFFF & ~1024) in text):
             return
     pytest.fail("neither the word nor a barrier")
+
+
+@pytest.mark.parametrize("rows", (1, 4, 16))
+def test_neither_do_those_of_the_launch_that_makes_rows_as_well(tmp_path, rows):
+    """k_finish_and_rows sets KTJ_DEVERR_RECORD_TOO_LONG too, and its workgroups look for either."""
+    for text in instructions(tmp_path, "k_finish_and_rowsILi%dEE" % rows):
+        if text.startswith("s_barrier"):
+            pytest.fail("the word decides as it is")
+        if re.match(r"[sv]_and_b32", text) and "0x%x" % (0xFFFFFFFF & ~(1024 | 8)) in text:
+            return
+    pytest.fail("neither the word nor a barrier")

@@ -1,0 +1,36 @@
+"""The sort's last launch makes the rows of CPU ops and kernels as well (k_finish_and_rows): documents against the oracle where its
+workgroups are of every kind, with groups that are put into order there and with one that has the order made again."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from kineto_amd import abi
+from stream_builder import B
+from test_gpu_sort_finish import ALL_BITS, groups, left_to_the_last_launch, ops, same_as_oracle
+
+pytestmark = pytest.mark.gpu
+
+
+def ops_and_kernels(n_ops, n_kernels, size, order):
+    """The groups' rows on three threads, and kernels on three streams in groups of their own."""
+    sp = ops(*groups(n_ops, size, order))
+    ts, stream = groups(n_kernels, size, order, seed=2)
+    rec = np.zeros(n_kernels, dtype=np.dtype(abi.DeviceRec))
+    rec["begin"], rec["end"], rec["stream"], rec["id"] = ts, ts + 3 + np.arange(n_kernels) % 700, stream, np.arange(n_kernels) + 10**6
+    rec["name_id"], rec["queue"] = np.arange(n_kernels) % 7, 1
+    held = (abi.DeviceRec * n_kernels).from_buffer_copy(rec.tobytes())
+    sp.contents.device, sp.contents.n_device = C.cast(held, type(sp.contents.device)), n_kernels
+    sp._held += (held,)
+    return sp
+
+
+@pytest.mark.parametrize("size, order", ((1, "forwards"), (256, "backwards"), (257, "halves")))
+@pytest.mark.parametrize("n_ops, n_kernels", ((4096, 1), (1, 4500), (257, 98304 - 257), (98304, 1), (40000, 70001), (600000, 500000)))
+def test_rows_come_with_the_sorts_last_launch(n_ops, n_kernels, size, order):
+    print(n_ops, n_kernels, size, order, flush=True)
+    info = same_as_oracle(ops_and_kernels(n_ops, n_kernels, size, order))
+    if size > 256:
+        assert info == ALL_BITS
+    else:
+        left_to_the_last_launch(info)
