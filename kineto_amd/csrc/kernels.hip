@@ -1658,11 +1658,24 @@ k_radix_scatter(const uint64_t* keys_in, const uint32_t* vals_in, uint64_t* keys
   }
 }
 
-/* counts per (digit, tile) plus the digits' totals; below SORTP_SMALL_N keys the packed sort's tiles are 512 keys */
-#define SORTP_SMALL_N (1ull << 19)
 #define SORTP_STREAM_N (1ull << 24)
+/* Keys per thread of the packed sort's tiles, 256 threads to each: as few as leave no CU without a tile, as many as keep the counts, a
+ * launch of 256 workgroups per pass to add up, short.  2 / 4 / 8 / 16, passes in us: 240 000 keys 219 / 221 / 228 / 243, 396 000 287 / 286 / 289 / 304,
+ * 600 000 321 / 317 / 321 / 332, 733 000 386 / 380 / 383 / 394, 900 000 406 / 398 / 399 / 408, 1.5 million 591 / 564 / 560 / 574, 3 million 1039 / 986 / 965 / 962,
+ * 4.4 million 1622 / 1519 / 1470 / 1472. */
+static const uint64_t sort_items_end[] = {3ull << 17, 1ull << 20, 1ull << 21};
+static uint32_t sort_items(uint64_t n) {
+  uint32_t items = 2;
+  for (const uint64_t end : sort_items_end) items *= n >= end ? 2u : 1u;
+  return items;
+}
+/* counts per (digit, tile) plus the digits' totals, of up to n keys: fewer may have more tiles */
 uint64_t radix_tmp_elems(uint64_t n) {
-  const uint64_t tiles = n < SORTP_SMALL_N ? (n + 511) / 512 : (n + RADIX_TILE - 1) / RADIX_TILE;
+  uint64_t tiles = (n + RADIX_TILE - 1) / RADIX_TILE;
+  for (const uint64_t end : sort_items_end) {
+    const uint64_t m = n < end ? n : end - 1u, tile = 256ull * sort_items(m), t = (m + tile - 1) / tile;
+    tiles = t > tiles ? t : tiles;
+  }
   return 256ull * tiles + 256;
 }
 
@@ -1721,7 +1734,7 @@ __device__ __forceinline__ uint64_t sort_key_dropped(const SortPlan& p) { return
 template <int BITS, int THREADS, int ITEMS_> struct SortP {
   static constexpr int NB = 1 << BITS;
   static constexpr int WAVES = THREADS / 64;
-  static constexpr int ITEMS = ITEMS_; /* keys per thread: 16, or 2 where a trace has too few keys to fill the GPU with tiles of 4096 */
+  static constexpr int ITEMS = ITEMS_; /* keys per thread (sort_items) */
   static constexpr int TILE = THREADS * ITEMS;
   static constexpr int WAVE_KEYS = 64 * ITEMS;
   static_assert(NB % THREADS == 0 || THREADS % NB == 0, "digits and threads must divide");
@@ -2409,14 +2422,13 @@ hipError_t sort_packed(Columns c, uint64_t n, SortSets s, Scalars* sc, uint32_t 
     return KTJ_LAUNCH_CHECK();
   }
   /* a few thousand keys are one tile; then one launch a pass, where the counts of all passes (1 KiB per pass and
-   * tile) fit the 8 bytes per row of chain_hist: eight passes of an odd few thousand keys do not.  Up to
-   * SORTP_SMALL_N keys, tiles of 512 spread over the GPU finish a pass sooner than the few 4096-key tiles
-   * would (330 000 keys: 113 against 155 us; from a million keys on the large tiles win) */
+   * tile) fit the 8 bytes per row of chain_hist: eight passes of an odd few thousand keys do not.  Behind that tiles by sort_items */
   if (n > (uint64_t)SORTP_THREADS * 16u && n <= CHAIN_MAX_N && 256ull * passes * ((n + CHAIN_THREADS - 1) / CHAIN_THREADS) <= 2 * (n + 1))
     return sort_packed_chain<SORTP_BITS>(c, n, s, sc, passes, finish, idx_bits, buf_a, buf_b, perm, chain_hist, job, st);
-  if (n > (uint64_t)SORTP_THREADS * 16u && n < SORTP_SMALL_N)
-    return sort_packed_t<SORTP_BITS, SORTP_THREADS, 2>(c, n, s, sc, passes, finish, idx_bits, buf_a, buf_b, perm, hist, job, st);
-  return sort_packed_t<SORTP_BITS, SORTP_THREADS, 16>(c, n, s, sc, passes, finish, idx_bits, buf_a, buf_b, perm, hist, job, st);
+  const uint32_t items = n > (uint64_t)SORTP_THREADS * 16u ? sort_items(n) : 16u;
+  const auto tiles = [&](auto sort) { return sort(c, n, s, sc, passes, finish, idx_bits, buf_a, buf_b, perm, hist, job, st); };
+  return items == 2u ? tiles(sort_packed_t<SORTP_BITS, SORTP_THREADS, 2>) : items == 4u ? tiles(sort_packed_t<SORTP_BITS, SORTP_THREADS, 4>)
+       : items == 8u ? tiles(sort_packed_t<SORTP_BITS, SORTP_THREADS, 8>) : tiles(sort_packed_t<SORTP_BITS, SORTP_THREADS, 16>);
 }
 
 /* ------------------------------------------------------------------------------------------ */

@@ -34,3 +34,10 @@ def test_rows_come_with_the_sorts_last_launch(n_ops, n_kernels, size, order):
         assert info == ALL_BITS
     else:
         left_to_the_last_launch(info)
+
+
+@pytest.mark.parametrize("n", (393215, 393216, 2**20 - 1, 2**20, 2**21 - 1, 2**21))
+def test_tiles_of_each_size(n):
+    """The fewest and the most keys of tiles of 512, 1024, 2048 and 4096 each."""
+    print(n, flush=True)
+    left_to_the_last_launch(same_as_oracle(ops(*groups(n, 97, "shuffled", threads=5))))
