@@ -113,8 +113,8 @@ def summarize_hbm(fetch_dir, write_dir, stats_csv, config, copy_bytes=1 << 30):
         print("%-36s %8d %10.1f %10.1f %9s %7.0f %7.3f" % (k[:36], n, fb / 1e6, wb / 1e6, "%.1f" % a if a else "-", gbs,
                                                           gbs / HBM_PEAK_GBS))
     for k, n, fb, wb, a in rows:
-        if k == DOMINANT_KERNEL:
-            print("traffic_json: " + json.dumps({"kernel": k, "config": config, "fetch_bytes_per_launch": round(fb),
+        if k.split("<")[0] == DOMINANT_KERNEL:
+            print("traffic_json: " + json.dumps({"kernel": DOMINANT_KERNEL, "config": config, "fetch_bytes_per_launch": round(fb),
                                                  "write_bytes_per_launch": round(wb), "hbm_bytes_per_launch": round(fb + wb)}))
 
 

@@ -10,8 +10,8 @@
  * into text in the size pass, which needs their lengths anyway; the texts with process and thread are made once per
  * track.
  *
- * What bounds it: latency, the LDS pipe and the vector units before memory (22 million records 2.97 ms, 13.6 GB, of which 2.6 ms are
- * what a copy of two parts read and seven written takes; without its stores the kernel takes some 2.5, without words written
+ * What bounds it: latency, the LDS pipe and the vector units before memory (22 million records 2.97 ms when it came to five wavefronts
+ * per SIMD, 2.83 now, 13.4 GB, of which 2.6 ms are what a copy of two parts read and seven written takes; without its stores the kernel takes some 2.5, without words written
  * to LDS either 2.0), so it is the wavefronts in flight that count: five per SIMD, which five workgroups of
  * four make (of five or of ten wavefronts three and one fit into a CU: 4.2 and 4.5 ms).  That takes 96 registers and
  * 32000 bytes of LDS per workgroup: texts that begin alike are there once, and names and the piece of the document share their room
@@ -20,11 +20,12 @@
  * 5 million operators with long strings 2.64 -> 2.45, 11 million kernels, at the memory's rate, 1.65 -> 1.62; three: 2.48, two 2.83.
  *
  * Measured against k_emit_direct (lane per activity): 10 000 x 3 records 38.7 -> 15 us, 4000 operators with long strings
- * 71 -> 23 us, 733 000 records 176 -> 121 us, 3 million 795 -> 402 us, 11 million kernels 2.06 -> 1.62 ms, 22 million
- * records 4.59 -> 2.97 ms, 5 million operators with long strings (1.4 KB each: strings beyond 128 bytes are fetched from
- * memory piece by piece) 3.20 -> 2.45 ms; the size pass has become up to 18 % longer for the numbers' text.
+ * 71 -> 23 us, 733 000 records 176 -> 105 us, 3 million 795 -> 367 us, 11 million kernels 2.06 -> 1.52 ms, 22 million
+ * records 4.59 -> 2.83 ms, 5 million operators with long strings (1.4 KB each: strings beyond 128 bytes are fetched from
+ * memory piece by piece) 3.20 -> 2.44 ms; the size pass has become up to 18 % longer for the numbers' text.
  * (Long strings' whole lines from the dictionary to the document past the tile, the loads of four strings at a time in
- * front of any store: no gain.)
+ * front of any store: no gain.  Strings waited for in front of the last lines' stores, with these lines read from LDS a second time: passes 0.6 to
+ * 1.5 % longer.)
  */
 #include "gpu_common.h"
 #include "weave_core.h"
