@@ -376,7 +376,7 @@ struct Rows {
   const weave::SchemaBook* schemas;
   weave::WideText* wide; /* of the generic records */
 };
-/* What mat_rows takes, for the sort: rows of both classes are made in its last launch where it has one that they may come with (made). */
+/* What mat_rows takes, for the sort: the rows are made in its last launch where it has one that they may come with (made). */
 struct RowsJob {
   const ktj_generic_rec* g;
   uint64_t ng;

@@ -2887,10 +2887,11 @@ k_mat_rows(const ktj_generic_rec* g, uint64_t ng, uint64_t first_generic, const 
   else if (DEVICE)
     mat_device_block<TEXT>(d, nd, c, first_device, link, clk, ctx, rows, len, sc, blockIdx.x - generic_blocks, gridDim.x - generic_blocks, stage);
 }
-/* The sort's last launch (first workgroups) and the rows of both classes in one: neither needs anything of the other, and the former is a
+/* The sort's last launch (first workgroups) and the rows of either class in one: neither needs anything of the other, and the former is a
  * chain of loads and LDS accesses that leaves the memory idle, with fewer workgroups than the GPU holds up to a few million rows.  Passes,
  * one after the other and now, us: 30 000 records 172 -> 168, 180 000 220 -> 213, 733 000 413 -> 407, 3 million 985 -> 972; 11 and 22 million, where both are
- * at the memory's rate by themselves, 3153 and 3146, 6838 and 6841. */
+ * at the memory's rate by themselves, 3153 and 3146, 6838 and 6841.  CPU ops or kernels alone: 20 000 records 140 -> 138, 150 000 220 -> 215, a million
+ * 771 -> 766, 3 million 2058 -> 2048. */
 template <int ITEMS>
 __global__ void __launch_bounds__(KTJ_BLOCK) __attribute__((amdgpu_waves_per_eu(4)))
 k_finish_and_rows(const uint64_t* buf_a, const uint64_t* buf_b, uint32_t* perm, uint64_t n, uint32_t idx_bits, uint32_t finish_blocks, const ktj_generic_rec* g,
@@ -3002,8 +3003,8 @@ hipError_t mat_rows(const ktj_generic_rec* g, uint64_t ng, uint64_t first_generi
 
 static bool finish_and_rows(const uint64_t* buf_a, const uint64_t* buf_b, uint32_t* perm, uint64_t n, uint32_t idx_bits, uint64_t tile, Scalars* sc,
                             RowsJob* job, hipStream_t st) {
-  if (!job || !job->ng || !job->nd || !job->rows.schemas) return false;
-  const unsigned fb = (unsigned)((n + tile - 1) / tile), gb = grid_stride_for(job->ng, KTJ_BLOCK), db = grid_stride_for(job->nd, KTJ_BLOCK);
+  if (!job || job->ng + job->nd == 0 || !job->rows.schemas) return false;
+  const unsigned fb = (unsigned)((n + tile - 1) / tile), gb = job->ng ? grid_stride_for(job->ng, KTJ_BLOCK) : 0u, db = job->nd ? grid_stride_for(job->nd, KTJ_BLOCK) : 0u;
   auto launch = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3(fb + gb + db), dim3(KTJ_BLOCK), 0, st, buf_a, buf_b, perm, n, idx_bits, fb, job->g, job->ng, gb, job->d, job->nd, job->c,
                        job->first_device, job->link, job->clk, job->ctx, job->rows, job->len, sc);

@@ -14,7 +14,8 @@ pytestmark = pytest.mark.gpu
 
 def ops_and_kernels(n_ops, n_kernels, size, order):
     """The groups' rows on three threads, and kernels on three streams in groups of their own."""
-    sp = ops(*groups(n_ops, size, order))
+    sp = ops(*groups(max(n_ops, 1), size, order))
+    sp.contents.n_generic = n_ops
     ts, stream = groups(n_kernels, size, order, seed=2)
     rec = np.zeros(n_kernels, dtype=np.dtype(abi.DeviceRec))
     rec["begin"], rec["end"], rec["stream"], rec["id"] = ts, ts + 3 + np.arange(n_kernels) % 700, stream, np.arange(n_kernels) + 10**6
@@ -26,7 +27,7 @@ def ops_and_kernels(n_ops, n_kernels, size, order):
 
 
 @pytest.mark.parametrize("size, order", ((1, "forwards"), (256, "backwards"), (257, "halves")))
-@pytest.mark.parametrize("n_ops, n_kernels", ((4096, 1), (1, 4500), (257, 98304 - 257), (98304, 1), (40000, 70001), (600000, 500000)))
+@pytest.mark.parametrize("n_ops, n_kernels", ((4096, 1), (1, 4500), (0, 4097), (257, 98304 - 257), (98304, 1), (40000, 70001), (600000, 500000)))
 def test_rows_come_with_the_sorts_last_launch(n_ops, n_kernels, size, order):
     print(n_ops, n_kernels, size, order, flush=True)
     info = same_as_oracle(ops_and_kernels(n_ops, n_kernels, size, order))
