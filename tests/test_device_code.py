@@ -124,3 +124,22 @@ def test_neither_do_those_of_the_launch_that_makes_rows_as_well(tmp_path, rows):
     def masked(text):
         return re.match(r"[sv]_and_b32", text) and "0x%x" % (0xFFFFFFFF & ~(1024 | 8)) in text
     assert not error_word_unmasked(code, masked) and not barrier_without(code, masked)
+
+
+@pytest.mark.parametrize("past", (0, 1))
+def test_segments_go_to_the_document_statement_by_statement(tmp_path, past):
+    """What put_segment writes too much is written over by lanes behind, whose word there is an earlier one of their text: all lanes'
+    stores of one statement stand before any lane's of the next.  So the stores to the tile are in the code once each, in the order of the
+    source (a text's words from the last one on, the number's, then the words that segments share), and the wavefront passes them forwards
+    only, whichever of its lanes skip some."""
+    code = instructions(tmp_path, "k_weaveILb%dEE" % past, addresses=True)
+    store = re.compile(r"ds_(write|or)_b32 v\d+, v\d+(?: offset:(\d+))?$")
+    stores = [(k, m[1], int(m[2] or 0)) for k, (_, text) in enumerate(code) for m in [store.match(text)] if m]
+    tile = max(offset for _, _, offset in stores) - 64  # (of the last of sixteen words)
+    here = [(k, kind, offset - tile) for k, kind, offset in stores if offset >= tile]
+    assert [x[1:] for x in here] == ([("write", 4 * w) for w in range(16, 0, -1)] + [("write", 4 * w) for w in range(1, 5)] + [("or", 0)] * 2)
+    first, last = here[0][0], here[-1][0]
+    for k, after in enumerate(successors(code)):
+        for n in after:
+            assert n > k or not (first < n <= last or first <= k <= last), "a branch back to one of them, or from among them"
+    assert not [t for _, t in code[first:last] if re.match(r"ds_(?!read)", t) and not store.match(t)]
