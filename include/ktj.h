@@ -437,8 +437,8 @@ enum {
   KTJ_STAGE_DECODE = 1,   /* raw records → columns                                             */
   KTJ_STAGE_CONVERT = 2,  /* clock conversion + window filter: part of KTJ_STAGE_DECODE, always 0     */
   KTJ_STAGE_JOIN = 3,     /* hash build + probe (ext-corr, runtime↔device, streams)            */
-  KTJ_STAGE_SORT = 4,     /* key build + stable radix sort                                     */
-  KTJ_STAGE_SIZE = 5,     /* exact byte length per record                                      */
+  KTJ_STAGE_SORT = 4,     /* key build + stable radix sort; its last launch is part of         */
+  KTJ_STAGE_SIZE = 5,     /* .. this where it makes rows as well; exact byte length per record */
   KTJ_STAGE_SCAN = 6,     /* device-wide exclusive scan                                        */
   KTJ_STAGE_EMIT = 7,     /* JSON formatting into the output buffer                            */
   KTJ_STAGE_D2H = 8,      /* device → pinned host copy (file sink: time spent waiting for it)  */

@@ -239,6 +239,7 @@ struct ktj_engine {
   DevBuf s_dev_k, s_dev_r, s_dev_l, s_res_k, s_res_r, s_res_l;
   DevBuf keys_a, keys_b, vals_a, vals_b, hist, scan_tmp;
   bool rows_are_text = false;              /* of the last pass: TextRows in mat */
+  bool rows_with_sort = false;             /* likewise: the sort's last launch made rows as well */
   uint64_t not_woven = 0;                  /* number of these records with which a woven pass left too many activities (too_many_left) */
   int some_left = -1;                      /* the last woven pass had activities that the weaver leaves to emit_direct (1, 0; -1: there was none) */
   uint64_t pass_info[4] = {};              /* of the last pass (KTJ_DBG_PASS) */
@@ -1347,8 +1348,9 @@ static void count_stats(ktj_engine* e, uint64_t N) {
   s.stage_bytes[KTJ_STAGE_CONVERT] = 0;
   s.stage_bytes[KTJ_STAGE_JOIN] = nx * 12 + ng * 12 + nr * 12 + (nr + nd) * 12 * 2 +
                                    nr * (sizeof(ktj_runtime_rec) + 48 + sizeof(MatRow) + 4); /* incl. the runtime rows' joined rows */
-  s.stage_bytes[KTJ_STAGE_SORT] = N * 56;
-  s.stage_bytes[KTJ_STAGE_SIZE] = (ng * sizeof(ktj_generic_rec) + nd * sizeof(ktj_device_rec)) + (ng + nd) * 48 +
+  const uint64_t last_launch = e->rows_with_sort ? N * 12 : 0; /* a word in, an index out: counted where its time is */
+  s.stage_bytes[KTJ_STAGE_SORT] = N * 56 - last_launch;
+  s.stage_bytes[KTJ_STAGE_SIZE] = last_launch + (ng * sizeof(ktj_generic_rec) + nd * sizeof(ktj_device_rec)) + (ng + nd) * 48 +
                                    (ng + nd) * (sizeof(MatRow) + 4) + N * 8;
   s.stage_bytes[KTJ_STAGE_SCAN] = N * 12;
   s.stage_bytes[KTJ_STAGE_EMIT] = e->scalars.n_valid * (sizeof(MatRow) + 12) + e->act_bytes;
@@ -1501,7 +1503,7 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
   e->last_end_time = end_time_ns;
   e->sort_info[0] = e->sort_info[1] = 0;
   e->small_last = false;
-  e->rows_are_text = false;
+  e->rows_are_text = e->rows_with_sort = false;
   if (!e->small_unfit && !e->no_small && nu == 0 && n_coll == 0 && small_fits(ng, nr, nd, nx) && !sort_packed_passes_forced() &&
       !(e->flags & (KTJ_CREATE_TILE_EMIT | KTJ_CREATE_HASH_JOIN | KTJ_CREATE_PAIR_SORT))) {
     bool done = false;
@@ -1701,6 +1703,7 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
     auto sort = [&](RowsJob* job) { return sort_packed(c, N, sets, sc, e->passes_to_launch(N), !e->sort_all_bits, e->keys_a.as<uint64_t>(), e->keys_b.as<uint64_t>(), e->perm, e->hist.as<uint32_t>(), e->offs.as<uint32_t>(), job, st); };
     RowsJob job{g_recs, ng, d_recs, nd, c, ng + nr, links_in(e->dev_link.p, nd), clock_of(e), ctx, rows, e->len.as<uint32_t>(), false};
     HIPCHK(sort(&job));
+    e->rows_with_sort = job.made;
     if (!job.made) HIPCHK(mat_rows(g_recs, ng, 0, nullptr, d_recs, nd, c, ng + nr, links_in(e->dev_link.p, nd), clock_of(e), ctx, rows, e->len.as<uint32_t>(), sc, st));
     for (;;) {
       text.out = e->out.as<char>(); text.out_cap = e->out.cap;
@@ -1724,6 +1727,7 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
         e->sort_passes = sort_packed_passes(e->scalars.sort, false);
         HIPCHK(clear_error_bits(sc, KTJ_DEVERR_UNSORTED, st));
         HIPCHK(sort(nullptr));
+        e->rows_with_sort = false;
         continue;
       }
       if (e->scalars.error) break;
@@ -1759,6 +1763,7 @@ static int process_pass(ktj_engine* e, int64_t end_time_ns, void* out_device, ui
     }
   }
   if (!emitted) { /* the stepwise rest */
+  e->rows_with_sort = false;
   HIPCHK(publish(sc, nullptr, nullptr, 0, &e->h_ctl_dev->scalars, nullptr, nullptr, st));
   HIPCHK(hipStreamSynchronize(st));
   e->scalars = e->h_ctl->scalars;

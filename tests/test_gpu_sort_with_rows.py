@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 
 from kineto_amd import abi
+from kineto_amd.engine import TraceEngine
 from stream_builder import B
 from test_gpu_sort_finish import ALL_BITS, groups, left_to_the_last_launch, ops, same_as_oracle
 
@@ -42,3 +43,16 @@ def test_tiles_of_each_size(n):
     """The fewest and the most keys of tiles of 512, 1024, 2048 and 4096 each."""
     print(n, flush=True)
     left_to_the_last_launch(same_as_oracle(ops(*groups(n, 97, "shuffled", threads=5))))
+
+
+def test_the_last_launchs_bytes_are_counted_with_its_time():
+    """12 bytes a row, under the rows' stage where they are made there, and under the sort's otherwise."""
+    sp = ops_and_kernels(4096, 4096, 3, "backwards")
+    counted = []
+    for as_tiles in (False, True):
+        with TraceEngine(sp.contents.trace_name.decode(), tile_emit=as_tiles) as e:
+            e.submit_stream(sp)
+            e.process()
+            counted.append([int(e.stats().stage_bytes[abi.STAGE_NAMES.index(k)]) for k in ("sort", "size")])
+    assert counted[1][0] == 56 * 8192 and counted[0][0] == 44 * 8192
+    assert sum(counted[0]) == sum(counted[1])
