@@ -987,7 +987,8 @@ __device__ __forceinline__ uint64_t dense_hash(int32_t device, uint64_t key) {
  * and touches the global table once per pair.  The workgroup that ends last gives every pair its number:
  * 1 + number of pairs of the same device seen earlier. */
 #define DENSE_LOCAL_SLOTS 1024u
-/* (every workgroup enters each pair that it has: 489 of 256 threads instead of 123 of 1024 for a million device rows 34 us, now 22) */
+/* (every workgroup enters each pair that it has: a million device rows 32 us with 489 workgroups of 256 threads, 21 with 245 of 1024; ten million 58 and 55
+ * with 1002 and 251) */
 #define DENSE_THREADS 1024u
 #define DENSE_ROWS 4u
 #define KTJ_DENSE_MAX KTJ_MAX_STREAM_PAIRS
@@ -1105,13 +1106,11 @@ hipError_t backfill_streams(const uint64_t* queue, uint64_t n, bool assign, Colu
   if (n == 0) return hipSuccess;
   const dim3 g(grid_for(n, KTJ_BLOCK)), b(KTJ_BLOCK);
   hipLaunchKernelGGL(k_after_link, dim3(grid_rarely(n)), b, 0, st, n, c, first_device, tf, fc, orphans, queue, t, sc);
-  /* every workgroup pays for its local table and for each pair it has seen: 2048 rows each, fewer only while
-   * that leaves CUs without a workgroup, and at most four workgroups per CU.  A workgroup's rows lie together, as buffers of a stream
-   * mostly do: it sees few of the pairs then (rows a grid apart: 22 million records 85 us instead of 65, 3 million 37 instead of 32; 58 and 33 with
+  /* Every workgroup pays for its local table and for each pair it has seen: 2048 rows each, and from 524 288 rows on, where that would be more than a
+   * workgroup per CU, as many as make 256 of them.  A workgroup's rows lie together, as buffers of a stream mostly do: it sees few of the pairs then
+   * (measured with up to 1024 workgroups of 256 threads; rows a grid apart: 22 million records 85 us instead of 65, 3 million 37 instead of 32; 58 and 33 with
    * columns of 20 bytes a row instead of 24). */
-  const unsigned few = grid_stride_for(n, DENSE_THREADS * 2), many = grid_stride_for(n, DENSE_THREADS * 8);
-  const unsigned most = 1024u * 256u / DENSE_THREADS;
-  const unsigned gd = many > most ? most : many > 256u ? many : few > 256u ? 256u : few;
+  const unsigned few = grid_stride_for(n, DENSE_THREADS * 2), gd = few < 256u ? few : 256u;
   const uint64_t per = ((n + gd - 1) / gd + DENSE_THREADS - 1) / DENSE_THREADS * DENSE_THREADS;
   hipLaunchKernelGGL(k_dense_first, dim3((unsigned)((n + per - 1) / per)), dim3(DENSE_THREADS), 0, st, queue, n, per, c, first_device, t, sc);
   if (assign) hipLaunchKernelGGL(k_dense_assign, g, b, 0, st, queue, n, c, first_device, t, sc);
@@ -1536,10 +1535,9 @@ hipError_t make_rank_keys(Columns c, const uint32_t* order, uint64_t n, SortSets
 
 hipError_t collect_distinct(Columns c, uint64_t n, uint64_t n_device, const Backfill& fill, SortSets s, Scalars* sc, bool straight, const EmitCtx& ctx, weave::SchemaBook* book, hipStream_t st) {
   if (n == 0) return hipSuccess;
-  /* few, fat workgroups: each one pays for its own local set once (few rows: one group each) */
-  /* at most four workgroups per CU: every workgroup pays for its local sets and its atomics at the
-   * end once, and a thousand of them keep enough loads in flight (4096: 0.23 ms for 22 M rows,
-   * 1024: 0.17 ms) */
+  /* Few, fat workgroups: every one pays for its local sets and its atomics at the end once.  Up to a million rows four rows a
+   * thread, then sixteen and, from 4.2 million on, more: at most 512 workgroups, two per CU, keep enough loads in flight (of 256 threads, when the numbers of
+   * streams were another launch's: 4096 of them 230 us for 22 million rows, 1024 170). */
   unsigned g = grid_stride_for(n, n < (1u << 20) ? COLLECT_THREADS * COLLECT_ROWS : COLLECT_THREADS * 16);
   if (g > 1024u * 256u / COLLECT_THREADS) g = 1024u * 256u / COLLECT_THREADS;
   /* (a workgroup's rows lie together and have few values, as above: 733 000 records 34 -> 28 us, 22 million 151 -> 141; 32 and 168 since
