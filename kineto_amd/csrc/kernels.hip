@@ -2887,7 +2887,7 @@ k_mat_rows(const ktj_generic_rec* g, uint64_t ng, uint64_t first_generic, const 
 }
 /* The sort's last launch (first workgroups) and the rows of either class in one: neither needs anything of the other, and the former is a
  * chain of loads and LDS accesses that leaves the memory idle, with fewer workgroups than the GPU holds up to a few million rows.  Passes,
- * one after the other and now, us: 30 000 records 172 -> 168, 180 000 220 -> 213, 733 000 413 -> 407, 3 million 985 -> 972; 11 and 22 million, where both are
+ * one after the other and now, us: 30 000 records 172 -> 168 (no more than runs differ), 180 000 220 -> 213, 733 000 413 -> 407, 3 million 985 -> 972; 11 and 22 million, where both are
  * at the memory's rate by themselves, 3153 and 3146, 6838 and 6841.  CPU ops or kernels alone: 20 000 records 140 -> 138, 150 000 220 -> 215, a million
  * 771 -> 766, 3 million 2058 -> 2048. */
 template <int ITEMS>

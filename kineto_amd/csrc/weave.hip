@@ -227,11 +227,15 @@ __device__ __forceinline__ uint64_t make_track(char* lds, uint32_t mine, uint64_
   return (uint64_t)(e2 | ((e5 - e2) << 8) | ((e8 - e5) << 16) | ((e10 - e8) << 24)) | ((uint64_t)(e12 - e10) << 32);
 }
 
-/* Documents of these many activities (250 MB at 480 bytes each) do not stay in the 256 MB last-level cache whichever way their lines
- * are stored, but ordinary stores leave it and the L2s full of lines that are written back while the next kernels run: whole passes of
- * 733 000 records 485 -> 465 us, of 3 million 1150 -> 1125 (k_decode of the next pass 94 -> 69 us), of 11 million 3590 -> 3560.  A smaller one
+/* A document that does not stay in the 256 MB last-level cache leaves it and the L2s, when stored in the ordinary way, full of lines that are
+ * written back while the next kernels run: whole passes of
+ * 733 000 records 485 -> 465 us, of 3 million 1150 -> 1125 (k_decode of the next pass 94 -> 69 us), of 11 million 3590 -> 3560.  A small one
  * is read back from there: sessions of 4000 operators with long strings (6 MB) 470 us with ordinary stores, 508 past the caches, files
- * of 90 000 records 6430 and 6750. */
+ * of 90 000 records (37 MB) 6430 and 6750.  The host knows the activities at this point and not their bytes, so the line is at as many as make 250 MB
+ * of 480 bytes each.  On either side of it, passes with ordinary stores and past the caches, us, sessions to the host's memory with both the same within
+ * their spread of 3 %: above, 600 000 plain operators (167 MB) 239 and 226, 555 000 records (224 MB) 302 and 291; below, 286 000 records (127 MB) 257 and 256,
+ * 440 000 (196 MB) 299 and 293, 504 000 kernels of graphs (229 MB) 318 and 314, operators with strings of a kilobyte 264 and 255 (200 000, 276 MB), 393 and 372
+ * (400 000, 552 MB): short activities lose nothing by it, and long ones leave some unused. */
 #define WV_PAST_FROM (1u << 19)
 /* PAST: the document's whole lines are stored past the caches' replacement */
 template <bool PAST>
@@ -603,7 +607,9 @@ hipError_t weave_activities(const TextRow* rows, const uint32_t* perm, const uin
   /* Turns of a wavefront: those of a pass that all wavefronts at once can take with up to forty each are dealt out to them (3 million
    * records 37 each 400 us, 19 and twice as many wavefronts 407).  Of longer passes each takes about twelve: the fewer, the closer
    * together lie the pieces of the document that are written at a time, but each copies the book (22 million records with 8, 12, 16,
-   * 24, 40: 3.09, 2.97, 3.00, 3.04, 3.04 ms; 5 million operators with long strings 2.45, 2.44, 2.52, 2.50, 2.51). */
+   * 24, 40: 3.09, 2.97, 3.00, 3.04, 3.04 ms; 5 million operators with long strings 2.45, 2.44, 2.52, 2.50, 2.51).  Around the line, which is at 3.28 million rows,
+   * whole passes dealt out and with about twelve turns each: 2.55 million records 855 and 863 us, 3.33 million 1070 and 1077, 3.9 million 1212 and 1220, 3.16 million
+   * kernels 1020 and 1016, operators with long strings 3 million 2050 and 2026, 3.5 million 2382 and 2360. */
   const uint64_t at_once = 256u * 20u, times = turns <= at_once * 40u ? 1u : (turns + at_once * 12u - 1u) / (at_once * 12u);
   const uint32_t rounds = (uint32_t)((turns + at_once * times - 1u) / (at_once * times));
   const auto kernel = n_most >= WV_PAST_FROM ? k_weave<true> : k_weave<false>;
